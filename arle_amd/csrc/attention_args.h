@@ -31,6 +31,10 @@ struct AttnArgs {
   const float* sink;   // [q heads] or null: exp(sink_h) joins the softmax's denominator, with no value behind it
   float out_scale;     // a factor on the output, in 32 bits
   int splits;
+  int segments;        // PREP with splits: how many segments share the segments * splits waves of a kv head
+  int* ws_plan;        // PREP with splits: [segments][2] a segment's first wave and its number of waves, then
+                       // [segments * splits][8] every wave's DecodeShare
+  int plan_made;       // the plan is there already (an earlier layer of the same step made it); 0: this launch makes it
   int ws_rows;   // token rows that the split-KV workspace holds for a segment
   int portion_splits;  // parts into which the LDS kernel cuts the keys of a row block (1: whole; it writes out)
   float* pws_o;        // [token row][q head][part][D]   (portion_splits > 1)
@@ -67,6 +71,88 @@ __device__ __forceinline__ bf16x8 zero_bf16x8() {
 __device__ __forceinline__ float row_factor(const float* sink, float out_scale, int head, float m, float l) {
   if (sink) l += exp2f(sink[head] * 1.4426950408889634f - m);
   return l > 0.f ? out_scale / l : 0.f;
+}
+
+// Inclusive sum (or maximum) over the lanes 0 .. lane of a wave of 64, of values that are not negative: shifts inside
+// the rows of 16, then a row's total handed on to the next ones; lane 63 holds the whole wave's.
+#define ARLE_PREFIX(NAME, JOIN)                                                                              \
+  __device__ __forceinline__ int NAME(int v) {                                                               \
+    int u;                                                                                                   \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false), v = JOIN; /* row_shr 1, 2, 4, 8 */        \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false), v = JOIN;                                 \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false), v = JOIN;                                 \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false), v = JOIN;                                 \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false), v = JOIN; /* lane 15 of a row to the next */ \
+    u = __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false), v = JOIN; /* lane 31 to the upper half */ \
+    return v;                                                                                                \
+  }
+ARLE_PREFIX(wave_prefix_sum, v + u)
+ARLE_PREFIX(wave_prefix_max, max(v, u))
+#undef ARLE_PREFIX
+
+// How the blocks of 32 keys of a step of single decoded tokens are shared out over the `waves` waves that a kv head
+// gets: every wave takes up to `per` blocks of one segment, per being the smallest number with which all segments'
+// waves are no more than there are and no segment has more than 64 (which is what the merge takes).  Equal contexts
+// get what an even split of each would give them.  waves is at least the number of segments.
+struct DecodeShare {
+  int seg, split, count;   // the wave's segment (-1: none), its place among the segment's waves, how many those are
+  int first;               // the segment's first wave
+  int per;
+  int start, slot;         // the segment's position and its row of the block table
+  int unused;
+};
+static_assert(sizeof(DecodeShare) == 8 * sizeof(int), "a plan keeps eight numbers a wave");
+__device__ __forceinline__ int decode_blocks(int start, int window) {   // blocks of 32 that hold a key which the token sees
+  const int lo = window > 0 ? max(0, start - window + 1) : 0;
+  return start / 32 + 1 - lo / 32;
+}
+__device__ __forceinline__ DecodeShare decode_share(const int* seg_start, const int* seg_slot, int segments, int window, int waves,
+                                                    int wave) {
+  const int lane = threadIdx.x & (kWave - 1);
+  // segment `at + lane`: up to 64 of them are one load, kept; further ones are read again where they are needed
+  const int start0 = seg_start[min(lane, segments - 1)], slot0 = seg_slot[min(lane, segments - 1)];
+  const int blocks0 = lane < segments ? decode_blocks(start0, window) : 0;
+  auto blocks_at = [&](int at) {
+    const int got = seg_start[min(at + lane, segments - 1)];
+    return at + lane < segments ? decode_blocks(got, window) : 0;
+  };
+  auto last = [](int v) { return __builtin_amdgcn_readlane(v, kWave - 1); };
+  int total = last(wave_prefix_sum(blocks0)), most = last(wave_prefix_max(blocks0));
+  for (int at = kWave; at < segments; at += kWave) {
+    const int b = blocks_at(at);
+    total += last(wave_prefix_sum(b));
+    most = max(most, last(wave_prefix_max(b)));
+  }
+  DecodeShare s;
+  s.per = max(max((total + waves - 1) / waves, (most + kWave - 1) / kWave), 1);
+  int mine0, incl0;
+  for (;; ++s.per) {   // ends: with per = most a segment is one wave
+    mine0 = (blocks0 + s.per - 1) / s.per;
+    incl0 = wave_prefix_sum(mine0);
+    int need = last(incl0);
+    for (int at = kWave; at < segments; at += kWave) need += last(wave_prefix_sum((blocks_at(at) + s.per - 1) / s.per));
+    if (need <= waves || s.per >= most) break;
+  }
+  s.seg = -1;
+  s.split = s.count = s.first = s.start = s.slot = s.unused = 0;
+  int before = 0;
+  for (int at = 0; at < segments; at += kWave) {
+    const int mine = at == 0 ? mine0 : (blocks_at(at) + s.per - 1) / s.per;
+    const int incl = at == 0 ? incl0 : wave_prefix_sum(mine);
+    const unsigned long long past = __ballot(before + incl > wave);
+    if (past != 0) {   // the first segment whose waves reach beyond this one
+      const int l = __builtin_ctzll(past);
+      s.seg = at + l;
+      s.count = __builtin_amdgcn_readlane(mine, l);
+      s.first = before + __builtin_amdgcn_readlane(incl, l) - s.count;
+      s.split = wave - s.first;
+      s.start = at == 0 ? __builtin_amdgcn_readlane(start0, l) : seg_start[s.seg];
+      s.slot = at == 0 ? __builtin_amdgcn_readlane(slot0, l) : seg_slot[s.seg];
+      return s;
+    }
+    before += last(incl);
+  }
+  return s;
 }
 
 __device__ __forceinline__ float group_max4(float v) {  // over the 4 lanes i, i+16, i+32, i+48

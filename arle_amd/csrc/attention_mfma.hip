@@ -305,6 +305,9 @@ static AttnArgs make_args(const void* q, long long q_stride, void* out, long lon
   a.sink = nullptr;
   a.out_scale = 1.0f;
   a.splits = splits;
+  a.segments = 0;
+  a.ws_plan = nullptr;
+  a.plan_made = 0;
   a.ws_rows = arle_attn_ws_rows(max_qlen, nq, nkv);
   a.portion_splits = 1;
   a.plan_token = 0;
@@ -386,7 +389,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
       side_rc = launch_attn<1>(b, dim3(1, nkv, static_cast<unsigned>(z)), side->stream);
       if (side_rc == 0 && splits > 1) {
         attn_merge_kernel<<<dim3(segments * b.ws_rows, nq), kMergeWaves * kWave, 0, side->stream>>>(
-            ws_o, ws_ml, b.out, o_stride, seg_row0, b.ws_rows, b.rows_max, nq, nkv, D, splits, a.sink, a.out_scale);
+            ws_o, ws_ml, b.out, o_stride, seg_row0, b.ws_rows, b.rows_max, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
         side_rc = launch_status();
       }
     }
@@ -423,7 +426,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
     rc = launch_attn<1>(a, dim3(1, nkv, static_cast<unsigned>(z)), s);
     if (rc != 0 || splits == 1) return rc;
     attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
-        ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, a.rows_max, nq, nkv, D, splits, a.sink, a.out_scale);
+        ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, a.rows_max, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
     return launch_status();
   }
   if (max_rows > 16 && splits > 1) return static_cast<int>(hipErrorInvalidValue);  // two row tiles: no split
@@ -433,7 +436,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
   rc = nt == 1 ? launch_attn<1>(a, grid, s) : launch_attn<2>(a, grid, s);
   if (rc != 0 || splits == 1) return rc;
   attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
-      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale);
+      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
   return launch_status();
 }
 
@@ -457,7 +460,11 @@ static int compute_units() {
 // 16-byte aligned), added in order; or, with parts_bf16, the projection itself in bfloat16 (n_parts 1).  q_w / k_w: per-head norm weights [D] (both or neither; float32 if w_f32, else
 // bfloat16; 16-byte aligned), eps inside the root.  cos / sin: float32 [positions][rot / 2], rot 0 (no rotation) or a
 // multiple of 64 up to D.  The new token's key and value are written to its slot of the pages (which the block table
-// must already hold) and take part in the attention from registers.  D 64 or 128, nq / nkv <= 16; everything else
+// must already hold) and take part in the attention from registers.  With splits > 1 there are `waves` waves a
+// kv head (at least one a segment; 0: segments * splits, or splits a segment in a workgroup of its own), over which the
+// segments' keys are shared out (ws_o [waves][nq][D], ws_ml [waves][nq][2]; ws_plan int32 [2 segments + 8 waves],
+// 8-byte aligned, is written by a call with plan_made 0 and read by later calls of the same step, segments, window and
+// waves with plan_made 1).  D 64 or 128, nq / nkv <= 16; everything else
 // as arle_attn_paged_mfma with max_qlen 1.  The same results as arle_qk_prep followed by arle_attn_paged_mfma but
 // for the order in which a head's squares are added for its norm.
 extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_parts, long long part_stride, long long row_stride,
@@ -465,18 +472,21 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
                                      int rot, float eps, void* out, long long o_stride, void* k_pages, void* v_pages,
                                      const int* block_table, int table_stride, const int* seg_row0, const int* seg_slot,
                                      const int* seg_start, int segments, int nq, int nkv, int D, int page_size,
-                                     float scale, int window, int splits, float* ws_o, float* ws_ml, void* stream) {
+                                     float scale, int window, int splits, float* ws_o, float* ws_ml, int waves, int* ws_plan,
+                                     int plan_made, void* stream) {
   if (segments == 0) return 0;
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if ((D != 64 && D != 128) || page_size < 4 || (page_size & (page_size - 1)) != 0 || nkv <= 0 || nq % nkv != 0 ||
-      nq / nkv > 16 || splits < 1 || splits > 64 || (splits > 1 && (ws_o == nullptr || ws_ml == nullptr)) ||
-      parts == nullptr || n_parts < 1 || (parts_bf16 && n_parts != 1) || part_stride % 8 != 0 || row_stride % 8 != 0 ||
+      nq / nkv > 16 || splits < 1 || splits > 64 || (splits > 1 && (ws_o == nullptr || ws_ml == nullptr || ws_plan == nullptr)) ||
+      reinterpret_cast<uintptr_t>(ws_plan) % 8 != 0 || parts == nullptr || n_parts < 1 || (parts_bf16 && n_parts != 1) || part_stride % 8 != 0 || row_stride % 8 != 0 ||
       !aligned(parts) ||
       (q_w == nullptr) != (k_w == nullptr) || !aligned(q_w) || !aligned(k_w) || rot < 0 || rot > D || rot % 64 != 0 ||
       (rot > 0 && (cos_t == nullptr || sin_t == nullptr || !aligned(cos_t) || !aligned(sin_t))) ||
       k_pages == nullptr || v_pages == nullptr || !aligned(k_pages))
     return static_cast<int>(hipErrorInvalidValue);
-  const long long z = static_cast<long long>(segments) * splits;
+  if (waves < 0 || (waves > 0 && (waves < segments || splits <= 1))) return static_cast<int>(hipErrorInvalidValue);
+  const bool spread = waves > 0;   // the caller wants the keys shared out, whatever the number of splits
+  const long long z = spread ? waves : static_cast<long long>(segments) * splits;
   if (nkv > 65535 || z > 65535) return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
   AttnArgs a = make_args(nullptr, 0, out, o_stride, k_pages, v_pages, block_table, table_stride, seg_row0, seg_slot,
@@ -497,7 +507,7 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
   a.prep_v_pages = static_cast<uint16_t*>(v_pages);
   // two to four splits and a workgroup for every compute unit even so: the splits of a (segment, kv head) share a
   // workgroup and merge in LDS (measured on MI355X at the Qwen3-4B widths, 64 requests at 2,048 tokens in two splits)
-  if (splits > 1 && splits <= kInWgWavesMax && g_decode_inwg != 0 &&
+  if (!spread && splits > 1 && splits <= kInWgWavesMax && g_decode_inwg != 0 &&
       (g_decode_inwg > 0 || static_cast<long long>(segments) * nkv >= compute_units())) {
     const dim3 grid(1, nkv, static_cast<unsigned>(segments));
     if (D == 128 && parts_bf16)
@@ -510,6 +520,9 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
       attn_mfma_kernel<1, 64, true, true, true, false><<<grid, splits * kWave, 0, s>>>(a);
     return launch_status();
   }
+  a.segments = segments;
+  a.ws_plan = splits > 1 ? ws_plan : nullptr;
+  a.plan_made = plan_made;
   const dim3 grid(1, nkv, static_cast<unsigned>(z));
   if (D == 128 && parts_bf16)
     attn_mfma_kernel<1, 128, true, true, false, true><<<grid, kWave, 0, s>>>(a);
@@ -522,7 +535,7 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
   const int rc = launch_status();
   if (rc != 0 || splits == 1) return rc;
   attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
-      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale);
+      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
   return launch_status();
 }
 
@@ -605,6 +618,6 @@ extern "C" int arle_attn_decode_static(const void* q, long long q_stride, void* 
   int rc = launch_attn<1>(a, dim3(1, nkv, static_cast<unsigned>(z)), s);
   if (rc != 0 || splits == 1) return rc;
   attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
-      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale);
+      ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, 0, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
   return launch_status();
 }

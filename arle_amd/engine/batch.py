@@ -62,6 +62,7 @@ class StepBatch:
     kv_splits: int | None = None  # split-KV factor fixed by the caller (a captured graph), else chosen per call
     plan_token: int = 0          # names one pass over the layers (set by the model): what parts plan once a pass
     max_portion_kv: int = 0      # longest context (cached + new) among the segments of more than one token; 0: none
+    total_context: int = 0       # the contexts (cached + new) of all segments together
     carry: dict = field(default_factory=dict)   # what a layer hands to later layers of the same pass (emptied by the model at the start of a pass)
 
 
@@ -159,6 +160,7 @@ def build_step_batch(entries, slot_of, length_of, vocab_size: int, device, into=
     return StepBatch(num_tokens=row, segments=segments, max_position=meta[2], max_qlen=meta[3], min_qlen=meta[4],
                      single_segments=meta[5],
                      max_portion_kv=max((s.start + s.length for s in segments if s.length > 1), default=0),
+                     total_context=sum(s.start + s.length for s in segments),
                      host=host, **dev)
 
 

@@ -141,6 +141,7 @@ class Engine:
         self.max_graph_logits_bytes = 64 << 20
         self._graph_pool = None
         self.graph_replays = 0
+        self._warm_total = None       # the contexts' total that a step of `warm_up` stands for
 
     # -- construction -----------------------------------------------------------------
     @classmethod
@@ -217,8 +218,7 @@ class Engine:
             # A step that is replayed from its graph runs no Python between its kernels, so nothing can fail half way.
             if decode_only:
                 rows_now = len(entries)
-                replayed = (rows_now, self.model.decode_launch_class(
-                    rows_now, max(before[e.request] for e in entries) + 1)) in self._graphs
+                replayed = (rows_now, self._decode_class(entries, before)) in self._graphs
             else:
                 replayed = shape_key is not None and shape_key in self._graphs
             if not replayed:
@@ -241,6 +241,11 @@ class Engine:
         return logits
 
     # -- captured decode steps ----------------------------------------------------------------
+    def _decode_class(self, entries, before) -> tuple:
+        """What the launches of a step of single decoded tokens depend on beside the number of rows."""
+        contexts = [before[e.request] + 1 for e in entries]
+        return self.model.decode_launch_class(len(entries), max(contexts), self._warm_total or sum(contexts))
+
     def _decode_step_graphed(self, entries, before, borrow: bool = False) -> torch.Tensor:
         """A step of single decoded tokens through a HIP graph captured for its number of rows.
 
@@ -252,8 +257,7 @@ class Engine:
         attention, which follows the longest context).
         """
         rows = len(entries)
-        max_kv = max(before[e.request] for e in entries) + 1
-        key = (rows, self.model.decode_launch_class(rows, max_kv))
+        key = (rows, self._decode_class(entries, before))
         all_rows = [StepEntry(e.request, e.tokens, [0]) for e in entries]
         length_before = before.__getitem__
         rec = self._graphs.pop(key, None)
@@ -262,6 +266,7 @@ class Engine:
             batch = build_step_batch(all_rows, self.cache.slot_of.__getitem__, length_before,
                                      self.spec.vocab_size, self.device, into=static)
             batch.kv_splits = None
+            batch.total_context = self._warm_total or batch.total_context
             logits = self.model.forward(batch, self.cache)   # this step's result, and the warm-up
             torch.cuda.synchronize()
             graph = torch.cuda.CUDAGraph()
@@ -302,22 +307,25 @@ class Engine:
         wanted = {}
         for rows in sizes:
             for context in contexts:
-                wanted.setdefault((rows, self.model.decode_launch_class(rows, context)), context)
-        todo = [(key, context) for key, context in wanted.items() if key not in self._graphs]
+                for total in (rows * context, rows - 1 + context):      # contexts all alike, and one long among short ones
+                    wanted.setdefault((rows, self.model.decode_launch_class(rows, context, total)), (context, total))
+        todo = [(key, *shape) for key, shape in wanted.items() if key not in self._graphs]
         self.max_graphs = max(self.max_graphs, len(self._graphs) + len(todo) + 16)
         captured = 0
-        for (rows, _), context in todo:
+        for (rows, _), context, total in todo:
             names = [("__warm_up__", i) for i in range(rows)]
             try:
                 for name in names:
                     self.add_request(name)
                 if context > 1:
                     self.cache.append([(names[0], context - 1)])    # bookkeeping only: the keys are whatever the pages hold
+                self._warm_total = total
                 self.step([StepEntry(name, [0], [0]) for name in names])
                 captured += 1
             except OutOfPages:
                 pass        # the pool does not hold this context beside the other rows: serving will not see it either
             finally:
+                self._warm_total = None
                 for name in names:
                     if self.cache.is_live(name):
                         self.end_request(name)

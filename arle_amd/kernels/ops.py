@@ -340,6 +340,34 @@ def decode_splits(segments: int, num_kv_heads: int, max_kv_len: int) -> int:
     return max(1, min(-(-_MFMA_TARGET_WAVES // (segments * num_kv_heads)), decode_split_cap(max_kv_len)))
 
 
+_DECODE_WAVES = 1024        # waves of the kernel that prepares q, k and v itself that run at a time: one a SIMD by its registers
+_DECODE_SPREAD = 0.8        # contexts that fill less than this of their longest count as ragged
+_DECODE_INSIDE_PAIRS = 256  # (request, kv head) pairs from which equal contexts are split inside a workgroup
+
+
+def decode_share(segments: int, num_kv_heads: int, max_kv_len: int, total_kv_len: int | None = None) -> tuple:
+    """(splits, waves) of attn_decode_prep for a step of single decoded tokens whose contexts are max_kv_len keys at most
+    and total_kv_len together (None: all alike).
+
+    waves > 0: so many waves a kv head, over which the keys of all requests are shared out.  One wave a SIMD is what the
+    kernel's registers let run at a time, and a wave more than that costs a second turn (batch 8 at 2,048 tokens, whole
+    steps of the Qwen3-4B shape: 2.86 ms at 1,024 waves, 2.89 at 768, 2.98 at 512, 3.14 at 1,280).  waves 0: with a pair of
+    request and kv head for every compute unit and equal contexts the splits of a pair are waves of one workgroup, which
+    spares the merge (or there is one split); ragged contexts are shared out there too.  Whole steps of the Qwen3-4B shape, one
+    or half of the requests at 2,048 tokens and the others so much shorter that all fill a part of what the longest would,
+    inside / shared out, ms: 32 requests full 4.38 / 4.63, nine tenths 4.42 / 4.40, 0.8 4.34 / 4.23, half 4.18 / 3.74; 64
+    requests full 6.61 / 6.73, 0.8 6.21 / 6.22, 0.7 6.10 / 6.02, 0.3 5.59 / 4.85."""
+    pairs = segments * num_kv_heads
+    cap = decode_split_cap(max_kv_len)
+    ragged = total_kv_len is not None and total_kv_len < _DECODE_SPREAD * segments * max_kv_len
+    if pairs >= _DECODE_INSIDE_PAIRS and not ragged:
+        return decode_splits(segments, num_kv_heads, max_kv_len), 0
+    waves = min(max(_DECODE_WAVES // num_kv_heads, 2 * segments if ragged else segments), segments * cap, _GRID_Y_MAX)
+    if waves <= segments or (waves < 2 * segments and not ragged):     # equal contexts take a wave each or two each
+        return 1, 0
+    return 2, waves     # two or more: the number that counts is the waves'
+
+
 _PORTION_SPLITS_MAX = 8         # parts into which the keys of a portion's row block may be cut
 _PORTION_ROWS = 128             # rows of a row block of the portions kernel
 _PORTION_LIST_MAX = 16384       # (row block, segment) pairs that its work list holds
@@ -463,12 +491,16 @@ def attn_decode_prep_supported(dtype, head_dim: int, page_size: int, group: int,
 def attn_decode_prep(parts, out, k_pages, v_pages, block_table, seg_row0, seg_slot, seg_start, *, max_kv_len: int,
                      num_q_heads: int, num_kv_heads: int, head_dim: int, page_size: int, scale: float, eps: float,
                      q_weight=None, k_weight=None, cos=None, sin=None, rotary_dim: int = 0, window: int = 0,
-                     splits: int | None = None):
+                     splits: int | None = None, total_kv_len: int | None = None, carry: dict | None = None):
     """A step of single decoded tokens (segment s is token row s) from the float32 stack of partial products
     [S, T, (nq + 2 nkv) D] of its fused q|k|v projection, or from the projection itself in bfloat16 [T, (nq + 2 nkv) D]:
     what qk_prep and attn_paged_mfma do one after the other, in the attention's own kernel.  Every wave sums, norms and rotates its q heads itself; the wave whose keys end
     with the new token's does the same for the k head, writes key and value into the cache and uses them from its
-    registers.  out: bfloat16 [T, nq*D]."""
+    registers.  out: bfloat16 [T, nq*D].
+    total_kv_len: the contexts' lengths together, by which ragged ones are told from equal ones (decode_share).
+    carry: a dictionary that lives for one pass over the layers.  Where the requests' keys are shared out over all waves of
+    a kv head, the first layer works out how, and the later ones of the pass with as many waves and the same window find
+    it there."""
     _gpu(parts, out, k_pages, v_pages, block_table, seg_row0, seg_slot, seg_start, q_weight, k_weight, cos, sin)
     group = num_q_heads // max(num_kv_heads, 1)
     width = (num_q_heads + 2 * num_kv_heads) * head_dim
@@ -509,19 +541,29 @@ def attn_decode_prep(parts, out, k_pages, v_pages, block_table, seg_row0, seg_sl
               and cos.dim() == 2 and cos.shape == sin.shape and cos.shape[1] == rotary_dim // 2 and cos.is_contiguous()
               and sin.is_contiguous() and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0,
               "cos/sin must be contiguous 16-byte aligned float32 [positions, rotary_dim/2]")
+    waves = 0
     if splits is None:
-        splits = decode_splits(segments, num_kv_heads, max_kv_len)
+        splits, waves = decode_share(segments, num_kv_heads, max_kv_len, None if window else total_kv_len)
     _need(1 <= splits <= 64, "splits must be 1..64")
-    _need(segments * splits <= _GRID_Y_MAX and num_kv_heads <= _GRID_Y_MAX, "too many segments for one launch")
-    ws_o = ws_ml = None
+    held = waves or segments * splits
+    _need(held <= _GRID_Y_MAX and num_kv_heads <= _GRID_Y_MAX, "too many segments for one launch")
+    ws_o = ws_ml = plan = None
+    plan_made = False
     if splits > 1:
-        ws_o = torch.empty((segments, num_q_heads, splits, head_dim), dtype=torch.float32, device=out.device)
-        ws_ml = torch.empty((segments, num_q_heads, splits, 2), dtype=torch.float32, device=out.device)
+        ws_o = torch.empty((held, num_q_heads, head_dim), dtype=torch.float32, device=out.device)
+        ws_ml = torch.empty((held, num_q_heads, 2), dtype=torch.float32, device=out.device)
+        key = ("decode_share", segments, int(held), int(window))
+        plan = carry.get(key) if carry is not None else None
+        plan_made = plan is not None
+        if not plan_made:
+            plan = torch.empty((2 * segments + 8 * held,), dtype=torch.int32, device=out.device)
+            if carry is not None:
+                carry[key] = plan
     lib.call("arle_attn_decode_prep", parts.data_ptr(), int(whole), n_parts, part_stride, row_stride, _ptr(q_weight),
              _ptr(k_weight), w_f32, _ptr(cos), _ptr(sin), int(rotary_dim), float(eps), out.data_ptr(), out.stride(0),
              k_pages.data_ptr(), v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], seg_row0.data_ptr(),
              seg_slot.data_ptr(), seg_start.data_ptr(), segments, num_q_heads, num_kv_heads, head_dim, page_size,
-             float(scale), int(window), int(splits), _ptr(ws_o), _ptr(ws_ml), _stream())
+             float(scale), int(window), int(splits), _ptr(ws_o), _ptr(ws_ml), int(waves), _ptr(plan), int(plan_made), _stream())
     return out
 
 

@@ -133,15 +133,19 @@ class DecoderModel:
             if prepare is not None:
                 prepare(max_positions)
 
-    def decode_launch_class(self, rows: int, max_context: int) -> tuple:
+    def decode_launch_class(self, rows: int, max_context: int, total_context: int | None = None) -> tuple:
         """What the launches of a step of `rows` single decoded tokens depend on beyond `rows`, over all parts (the
-        distinct answers of `Part.decode_launch_class`, in a fixed order)."""
+        distinct answers of `Part.decode_launch_class` and, with the contexts' total (default: all are max_context long), of
+        `Part.decode_spread_class`, in a fixed order)."""
+        if total_context is None:
+            total_context = rows * max_context
         found = set()
         for part in self.parts:
-            ask = getattr(part, "decode_launch_class", None)
-            answer = ask(rows, max_context) if ask is not None else None
-            if answer is not None:
-                found.add(answer)
+            for name, args in (("decode_launch_class", (rows, max_context)), ("decode_spread_class", (rows, max_context, total_context))):
+                ask = getattr(part, name, None)
+                answer = ask(*args) if ask is not None else None
+                if answer is not None:
+                    found.add((name, answer))
         return tuple(sorted(found, key=repr))
 
     def cache_needs(self):

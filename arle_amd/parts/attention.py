@@ -99,7 +99,12 @@ class PagedAttention(Part):
         # the split-KV factor of the matrix-core kernel is the one launch dimension that follows the context
         if self.rt.is_f32 or self.D % 16 or self.D > ops.MFMA_MAX_HEAD_DIM:
             return None
-        return ops.decode_splits(rows, self.nkv, max_context)
+        return ops.decode_splits(rows, self.nkv, max_context), ops.decode_share(rows, self.nkv, max_context)
+
+    def decode_spread_class(self, rows, max_context, total_context):
+        if self.rt.is_f32 or not self.folds_preparation or self.window:
+            return None
+        return ops.decode_share(rows, self.nkv, max_context, total_context)
 
     def forward(self, x, batch, cache):
         """x [T, H] -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear)."""
@@ -125,7 +130,8 @@ class PagedAttention(Part):
                                  batch.seg_slot, batch.seg_start, max_kv_len=batch.max_position + 1,
                                  num_q_heads=self.nq, num_kv_heads=self.nkv, head_dim=self.D, page_size=cache.page_size,
                                  scale=self.scale, eps=self.eps, q_weight=self.q_norm, k_weight=self.k_norm, cos=cos,
-                                 sin=sin, rotary_dim=rot, window=self.window or 0, splits=getattr(batch, "kv_splits", None))
+                                 sin=sin, rotary_dim=rot, window=self.window or 0, splits=getattr(batch, "kv_splits", None),
+                                 total_kv_len=getattr(batch, "total_context", 0) or None, carry=getattr(batch, "carry", None))
             return self.o(out, partials_ok=True)
         if projected.dim() == 3:
             q = torch.empty((x.shape[0], Q), dtype=x.dtype, device=x.device)

@@ -132,6 +132,13 @@ class Part:
         serves both."""
         return None
 
+    def decode_spread_class(self, rows: int, max_context: int, total_context: int):
+        """As decode_launch_class, for what the launches depend on beyond it when the contexts of the rows are
+        `total_context` tokens together.  The default asks the parts nested in this one."""
+        found = tuple(child.decode_spread_class(rows, max_context, total_context)
+                      for child in getattr(self, "child_parts", {}).values() if hasattr(child, "decode_spread_class"))
+        return None if all(f is None for f in found) else found
+
     def prepare(self, max_positions: int) -> None:
         """Called by the engine once the longest request is known, before any step runs or is captured: whatever
         a part keeps that grows with the position (a table of angles, slopes, a window of taps) is made for

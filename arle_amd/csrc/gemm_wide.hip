@@ -1,0 +1,359 @@
+// bfloat16 matrix product for prompt portions:  C[M,N] = X[M,K] . W[N,K]^T, both row-major, K a multiple of 64.
+//
+// A workgroup owns BM rows x BN columns (128 to 256 x 64 to 320) and walks K in stages of 64: the stage's rows of X and W, 128
+// bytes each, go from memory straight into LDS (global_load_lds, no registers on the way), two stages deep, and every wave
+// feeds v_mfma_f32_32x32x16_bf16 from there.  What bounds it, and what was done about that (MI355X, gate|up of the Qwen3-4B
+// shape, N 19,456, K 2,560, weights cold):
+//
+//   * The matrix cores, at the clock that the chip holds when all 256 compute units multiply real data (1.75 to 1.84 PFLOP/s):
+//     the loop alone runs at 1.53, a whole launch of 8,192 rows at 1.30 (628 us; the library's product and the activation
+//     kernel 771, gemm_tiles 793).
+//   * Turns: a launch lasts as many turns of its workgroups as they fill the compute units.  gate|up at 2,048 rows is 608
+//     tiles of 256 x 256, three turns for 2.4; 256 x 320 is 488, two turns for 1.9: 167 us against gemm_tiles' 200.  So there are
+//     twelve shapes, and the caller's plan takes the one whose turns are shortest (ops.wide_plan).
+//   * Latency of what comes from memory: with two stages a fetch has one stage's time (1.2 to 1.8 us), which a miss of the L2
+//     under load does not keep to.  Every wave therefore touches, four stages ahead, a few of the 128-byte lines that its
+//     XCD's workgroups will fetch (a dword a line, into a corner of LDS that nobody reads): 2,048 rows 223 -> 186 us, 8,192
+//     rows 679 -> 600.  More stages of 32 k instead (rows of 64 bytes) were 6 to 8 % slower: half lines cost the fetch path
+//     twice the requests.
+//   * The step's operand reads (4 cycles of LDS each) and loads are pinned between its products (sched_barrier): the next
+//     step's operands are read while this step multiplies, the barrier of a stage stands in its last step, behind which
+//     the first operands of the next stage are read and the place of this one is filled again.
+//   * The activation: expf and the divide of 40 thousand pairs took 9 of a workgroup's 85 us; with the vector unit's own
+//     exponential and reciprocal 4.
+//
+// Four waves (one a SIMD) or eight, measured alike in the loop; eight hold the accumulators of 256 x 320 in 256 registers each.
+#include "common.h"
+
+#include <type_traits>
+
+namespace arle {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kWdXcds = 8;
+constexpr int kWdXcdPlaces = 32;   // workgroups that an XCD runs at a time: one a compute unit
+constexpr int kWdK = 64;           // k of a stage: rows of 128 bytes
+constexpr int kEpiNone = 0, kEpiSiluMul = 1;
+
+struct WideArgs {
+  const uint16_t* x;
+  int64_t ldx;
+  const uint16_t* w;
+  int64_t ldw;
+  void* out;
+  int64_t ldo;
+  int M, N, K;
+  int m_blocks, n_blocks;
+  int patch_rows, patch_cols;
+  int stages_per_split;
+  int64_t split_stride;
+};
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register: naming it as clobbered is the point
+// 16 bytes a lane from base + lane_bytes to lds_at + 16 lane.  As assembly, because behind the builtin every LDS read is
+// made to wait for all loads in flight.
+__device__ __forceinline__ void wide_load(const uint16_t* base, uint32_t lane_bytes, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_at), "v"(lane_bytes), "s"(base)
+               : "memory", "m0");
+}
+// A dword of each lane's line, to a place in LDS that nobody reads: it brings the line into the L2.
+__device__ __forceinline__ void wide_touch(const uint16_t* from, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_at), "v"(from) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// x / (1 + exp(-x)) with the exponential and the reciprocal of the vector unit (each within an ulp or two of float32; the
+// result is rounded to bfloat16 behind it)
+__device__ __forceinline__ float silu(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
+
+template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
+__global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(const WideArgs a) {
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, kWaves = WM * WN;
+  constexpr int kRowsALoad = 8 * kWaves;                        // rows that one load of every wave brings
+  static_assert(BM % kRowsALoad == 0 && BN % kRowsALoad == 0, "whole loads");
+  constexpr int LX = BM / kRowsALoad, LA = (BM + BN) / kRowsALoad;
+  constexpr int kStage = (BM + BN) * 128;
+  constexpr int kProducts = TM * TN, kReads = TM + TN, kReadsASlot = (kReads + kProducts - 2) / (kProducts - 1);
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, h = lane >> 5;
+  const int wm = wave / WN, wn = wave % WN;
+
+  const int xcd = blockIdx.x % kWdXcds, q = blockIdx.x / kWdXcds;
+  const int patch = a.patch_rows * a.patch_cols, in_patch = q % patch, p = q / patch;
+  const int row_groups = (a.m_blocks + a.patch_rows - 1) / a.patch_rows;
+  const int mb = __builtin_amdgcn_readfirstlane((p % row_groups) * a.patch_rows + in_patch % a.patch_rows);
+  const int nb = __builtin_amdgcn_readfirstlane(((p / row_groups) * a.patch_cols + in_patch / a.patch_rows) * kWdXcds + xcd);
+  if (mb >= a.m_blocks || nb >= a.n_blocks) return;  // the whole workgroup
+  const int m0 = mb * BM, n0 = nb * BN;
+  const int M = a.M, N = a.N;
+  const int all_stages = a.K / kWdK;
+  const int st0 = blockIdx.y * a.stages_per_split;
+  const int n_st = min(a.stages_per_split, all_stages - st0);
+  const uint16_t* xb = a.x + static_cast<int64_t>(m0) * a.ldx + static_cast<int64_t>(st0) * kWdK;
+  const uint16_t* wb = a.w + static_cast<int64_t>(n0) * a.ldw + static_cast<int64_t>(st0) * kWdK;
+
+  // a load brings 8 rows of 128 bytes; piece lane % 8 of an LDS row holds the row's k piece (lane % 8) ^ (row / 2 % 8),
+  // so that sixteen lanes of an operand read never share a bank
+  const int lr = 8 * wave + (lane >> 3);
+  const int piece = (lane & 7) ^ ((lr >> 1) & 7);
+  uint32_t off[LA];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const bool of_x = i < LX;
+    const int row = kRowsALoad * (of_x ? i : i - LX) + lr;
+    off[i] = static_cast<uint32_t>(min(row, of_x ? M - 1 - m0 : N - 1 - n0)) * static_cast<uint32_t>((of_x ? a.ldx : a.ldw) * 2) + piece * 16;
+  }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + 1024u * wave);
+  auto load = [&](int i, uint32_t buf, const uint16_t* xs, const uint16_t* ws) {   // i is a constant where this is called
+    wide_load(i < LX ? xs : ws, off[i], lds0 + buf + 1024u * kWaves * i);
+  };
+  // What comes from memory and not from the L2 comes late: every stage a wave touches a few of the 128-byte lines that the
+  // stage kAhead later will fetch (the workgroups that share a column block's weights or a row block's x on an XCD
+  // share out its lines), so that the fetch itself meets the L2.
+  constexpr int kAhead = 4;
+  const int x_share = max(1, kWdXcdPlaces / a.patch_rows);
+  const int w_lines = (BN + a.patch_rows * kWaves - 1) / (a.patch_rows * kWaves), x_lines = (BM + x_share * kWaves - 1) / (x_share * kWaves);
+  const uint16_t* touch_from;
+  if (lane < w_lines)
+    touch_from = wb + static_cast<int64_t>(min(((mb % a.patch_rows) * kWaves + wave) * w_lines + lane, N - 1 - n0)) * a.ldw;
+  else
+    touch_from = xb + static_cast<int64_t>(min((((nb / kWdXcds) % x_share) * kWaves + wave) * x_lines + min(lane - w_lines, x_lines - 1), M - 1 - m0)) * a.ldx;
+  const bool touches = lane < w_lines + x_lines;
+  const uint32_t touch_at = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + 2 * kStage + 256u * wave);
+  auto touch = [&](int stages) {
+    if (touches) wide_touch(touch_from + stages * kWdK, touch_at);
+  };
+  uint32_t at[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) at[kk] = j * 128 + (((2 * kk + h) ^ ((j >> 1) & 7)) * 16);
+  const uint32_t x_at = wm * TM * 4096, w_at = BM * 128 + wn * TN * 4096;
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int t = 0; t < TM; ++t)
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][tn][r] = 0.f;
+  bf16x8 fx[2][TM], fw[2][TN];
+  auto read_one = [&](int i, int set, int kk, uint32_t buf) {
+    if (i < TM)
+      fx[set][i] = *reinterpret_cast<const bf16x8*>(lds + buf + x_at + at[kk] + 4096 * i);
+    else
+      fw[set][i - TM] = *reinterpret_cast<const bf16x8*>(lds + buf + w_at + at[kk] + 4096 * (i - TM));
+  };
+
+  constexpr int kEarly = (LA + 1) / 2;   // loads of a stage that go out in the step that frees its place; the others in the step after it
+#pragma unroll
+  for (int i = 0; i < LA; ++i) load(i, 0, xb, wb);
+  if (n_st > 1) {
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) load(i, kStage, xb + kWdK, wb + kWdK);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kEarly) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  if (n_st > 3) touch(2), touch(3);
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < kReads; ++i) read_one(i, 0, 0, 0);
+
+  // One stage: four steps of 16 k.  NEXT: what is still to be fetched (2: the rest of stage s + 1 and the first part of
+  // s + 2; 1: the former only; 0: nothing, and no stage follows)
+  auto stage = [&](auto next_tag, uint32_t buf) {
+    constexpr int NEXT = decltype(next_tag)::value;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int set = kk & 1;
+#pragma unroll
+      for (int m = 0; m < kProducts; ++m) {
+        if (kk == 3 && m == 1 && NEXT > 0) {
+          // every wave has its operands of this stage, and its pieces of the next one have landed
+          // (a line that was touched for later may still be on its way)
+          if (NEXT == 3) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const int t = m % TM, tn = m / TM;
+        acc[t][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][tn], fx[set][t], acc[t][tn], 0, 0, 0);
+        // the next step's operands behind the products 1, 2, ...
+#pragma unroll
+        for (int r = (m - 1) * kReadsASlot; m > 0 && r < m * kReadsASlot && r < kReads; ++r) {
+          if (kk < 3) read_one(r, set ^ 1, kk + 1, buf);
+          else if (NEXT > 0) read_one(r, set ^ 1, 0, kStage - buf);
+        }
+        if (kk == 3 && NEXT > 1 && m >= 1) {
+#pragma unroll
+          for (int i = 0; i < kEarly; ++i)
+            if (1 + i * (kProducts - 1) / kEarly == m) load(i, buf, xb + 2 * kWdK, wb + 2 * kWdK);
+        }
+        if (kk == 0 && NEXT > 0) {
+#pragma unroll
+          for (int i = kEarly; i < LA; ++i)
+            if ((i - kEarly) * kProducts / (LA - kEarly) == m) load(i, kStage - buf, xb + kWdK, wb + kWdK);
+        }
+        if (kk == 1 && NEXT == 3 && m == 1) touch(kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  uint32_t buf = 0;
+  int s = 0;
+  for (; s + kAhead < n_st; ++s) {
+    stage(std::integral_constant<int, 3>{}, buf);
+    buf = kStage - buf;
+    xb += kWdK, wb += kWdK, touch_from += kWdK;
+  }
+  for (; s + 2 < n_st; ++s) {
+    stage(std::integral_constant<int, 2>{}, buf);
+    buf = kStage - buf;
+    xb += kWdK, wb += kWdK;
+  }
+  if (s + 1 < n_st) {
+    stage(std::integral_constant<int, 1>{}, buf);
+    buf = kStage - buf;
+  }
+  stage(std::integral_constant<int, 0>{}, buf);
+
+  // acc[t][tn][r] = C[m0 + 32 (TM wm + t) + j][n0 + 32 (TN wn + tn) + 8 (r / 4) + 4 h + r % 4]; row tiles go through a
+  // part of LDS of the wave's own (float32 ones a column tile at a time) and leave as whole rows
+  constexpr int kElt = static_cast<int>(sizeof(TOut));
+  constexpr int kTile = EPI == kEpiSiluMul ? 16 : 32;                // output columns of a column tile
+  constexpr int kGroup = kElt == 2 ? TN : 1;                         // column tiles that leave together
+  constexpr int kPitch = kTile * kGroup * kElt + 16;
+  constexpr int kPieces = kTile * kGroup * kElt / 16;
+  static_assert(kWaves * 32 * kPitch <= 2 * kStage, "the epilogue's rows fit the stages");
+  TOut* out = static_cast<TOut*>(a.out) + static_cast<int64_t>(blockIdx.y) * a.split_stride;
+  const int n_out = EPI == kEpiSiluMul ? N / 2 : N;
+  const int c0 = (EPI == kEpiSiluMul ? n0 / 2 : n0) + kTile * TN * wn;
+  const int r0 = m0 + 32 * TM * wm;
+  __syncthreads();
+  unsigned char* mine = lds + wave * (32 * kPitch);
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+#pragma unroll
+    for (int g = 0; g < TN; g += kGroup) {
+#pragma unroll
+      for (int tn = g; tn < g + kGroup; ++tn) {
+#pragma unroll
+        for (int q4 = 0; q4 < kTile / 8; ++q4) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = acc[t][tn][4 * q4 + e];
+            if constexpr (EPI == kEpiSiluMul) v[e] = silu(v[e]) * acc[t][tn][4 * q4 + e + 8];
+          }
+          unsigned char* to = mine + j * kPitch + (kTile * (tn - g) + 8 * q4 + 4 * h) * kElt;
+          if constexpr (kElt == 2)
+            *reinterpret_cast<uint2*>(to) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          else
+            *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int i = 0; i < kPieces / 2; ++i) {
+        const int idx = 64 * i + lane, rr = idx / kPieces, pc = idx % kPieces;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + rr * kPitch + pc * 16);
+        const int row = r0 + 32 * t + rr, col = c0 + kTile * g + pc * (16 / kElt);
+        if (row < M && col < n_out) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * a.ldo + col) = v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+}
+
+static int g_wide_rows = 8, g_wide_cols = 4;
+
+template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
+int launch_wide(WideArgs a, int splits, hipStream_t s) {
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+  constexpr size_t lds = 2 * (BM + BN) * 128 + 256 * WM * WN;
+  static_assert(lds <= 160 * 1024, "two stages fit the LDS");
+  static bool asked = false;   // more than 64 KiB of LDS has to be asked for, once
+  if (!asked) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, EPI, TOut>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return static_cast<int>(e);
+    }
+    asked = true;
+  }
+  a.m_blocks = (a.M + BM - 1) / BM;
+  a.n_blocks = (a.N + BN - 1) / BN;
+  a.patch_rows = a.m_blocks < g_wide_rows ? a.m_blocks : g_wide_rows;
+  a.patch_cols = a.m_blocks > a.patch_rows ? g_wide_cols : 1;
+  const long long cols_an_xcd = (a.n_blocks + kWdXcds - 1) / kWdXcds;
+  const long long row_groups = (a.m_blocks + a.patch_rows - 1) / a.patch_rows;
+  const long long col_groups = (cols_an_xcd + a.patch_cols - 1) / a.patch_cols;
+  const long long grid = row_groups * col_groups * a.patch_rows * a.patch_cols * kWdXcds;
+  if (grid > 0x7fffffffLL) return static_cast<int>(hipErrorInvalidValue);
+  gemm_wide_kernel<WM, WN, TM, TN, EPI, TOut><<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(splits)), WM * WN * kWave, lds, s>>>(a);
+  return launch_status();
+}
+
+template <int WM, int WN, int TM, int TN>
+int dispatch_wide(const WideArgs& a, int splits, int out_dtype, int epilogue, hipStream_t s) {
+  if (epilogue) return launch_wide<WM, WN, TM, TN, kEpiSiluMul, bf16>(a, splits, s);
+  return out_dtype == kF32 ? launch_wide<WM, WN, TM, TN, kEpiNone, float>(a, splits, s) : launch_wide<WM, WN, TM, TN, kEpiNone, bf16>(a, splits, s);
+}
+
+}  // namespace arle
+
+using namespace arle;
+
+extern "C" void arle_gemm_wide_patch(int rows, int cols) {
+  if (rows >= 1 && cols >= 1) g_wide_rows = rows, g_wide_cols = cols;
+}
+
+// x [M, K], w [N, K] bfloat16 with 16-byte aligned rows, K % 64 == 0, N % 32 == 0.  out [M, N] (bfloat16 or float32), or
+// with epilogue 1 [M, N/2] bfloat16 (gate and up rows of w interleaved in blocks of 16): silu(gate) * up.
+extern "C" int arle_gemm_wide(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int out_dtype,
+                              int M, int N, int K, int epilogue, int row_tiles, int col_tiles, int splits, int stages_per_split,
+                              long long split_stride, void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const int per16 = out_dtype == kF32 ? 4 : 8;
+  if (K <= 0 || K % kWdK != 0 || N % 32 != 0 || ldx % 8 != 0 || ldw % 8 != 0 || ldx >= (1 << 20) || ldw >= (1 << 20) ||
+      !aligned(x) || !aligned(w) || !aligned(out) || ldo % per16 != 0 || split_stride % per16 != 0 ||
+      (epilogue != kEpiNone && epilogue != kEpiSiluMul) || (epilogue == kEpiSiluMul && out_dtype == kF32) || splits < 1 ||
+      splits > 65535 || stages_per_split < 1 || (splits > 1 && (out_dtype != kF32 || epilogue != kEpiNone)))
+    return static_cast<int>(hipErrorInvalidValue);
+  const int stages = K / kWdK;
+  if (static_cast<long long>(splits - 1) * stages_per_split >= stages || static_cast<long long>(splits) * stages_per_split < stages)
+    return static_cast<int>(hipErrorInvalidValue);
+  const WideArgs a{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(w), ldw, out, ldo, M, N, K,
+                   0, 0, 0, 0, stages_per_split, split_stride};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (1000 * row_tiles + col_tiles) {   // rows and columns of a workgroup
+    case 256320: return dispatch_wide<4, 2, 2, 5>(a, splits, out_dtype, epilogue, s);
+    case 256256: return dispatch_wide<4, 2, 2, 4>(a, splits, out_dtype, epilogue, s);
+    case 256192: return dispatch_wide<4, 2, 2, 3>(a, splits, out_dtype, epilogue, s);
+    case 128064: return dispatch_wide<2, 2, 2, 1>(a, splits, out_dtype, epilogue, s);
+    case 128096: return dispatch_wide<4, 1, 1, 3>(a, splits, out_dtype, epilogue, s);
+    case 128128: return dispatch_wide<2, 2, 2, 2>(a, splits, out_dtype, epilogue, s);
+    case 128160: return dispatch_wide<4, 1, 1, 5>(a, splits, out_dtype, epilogue, s);
+    case 256160: return dispatch_wide<4, 1, 2, 5>(a, splits, out_dtype, epilogue, s);
+    case 128256: return dispatch_wide<2, 2, 2, 4>(a, splits, out_dtype, epilogue, s);
+    case 128192: return dispatch_wide<2, 2, 2, 3>(a, splits, out_dtype, epilogue, s);
+    case 128320: return dispatch_wide<2, 2, 2, 5>(a, splits, out_dtype, epilogue, s);
+    case 192320: return dispatch_wide<2, 2, 3, 5>(a, splits, out_dtype, epilogue, s);
+  }
+  return static_cast<int>(hipErrorInvalidValue);
+}

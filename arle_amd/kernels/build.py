@@ -29,6 +29,7 @@ SOURCES = {
     "gemm_f32": "gemm_f32.hip",
     "gemm_rows": "gemm_rows.hip",
     "gemm_tiles": "gemm_tiles.hip",
+    "gemm_wide": "gemm_wide.hip",
     "rope_kv": "rope_kv.hip",
     "attention_simt": "attention_simt.hip",
     "attention_mfma": "attention_mfma.hip",

@@ -1038,6 +1038,72 @@ def gemm_tiles(x, tiles, n: int, out_dtype=torch.bfloat16, epilogue: int = EPI_N
     return out
 
 
+# Workgroup shapes (rows x columns) of gemm_wide and what one of them takes for a stage of 64 k when every compute unit has
+# one, in us, activation or not (MI355X, weights cold, from products of 65 to 8,192 rows at K 2,560 and 4,096; beside the
+# stages a workgroup takes 4 us for its first loads and its results).  A launch takes as many turns as its workgroups fill
+# the compute units; wide_plan picks the shape (and the parts of K) whose turns take least.
+WIDE_STAGE_US = {(128, 64): 0.62, (128, 96): 0.80, (128, 128): 0.87, (128, 160): 0.89, (128, 192): 0.92, (128, 256): 1.04,
+                 (128, 320): 1.15, (256, 160): 1.16, (256, 192): 1.32, (256, 256): 1.52, (192, 320): 1.52, (256, 320): 1.85}
+_WIDE_FIXED_US = 4.0
+_WIDE_MAX_PARTS = 8
+_WIDE_K = 64            # K comes in whole stages
+
+
+def gemm_wide_supported(n: int, k: int, x_stride: int, w_stride: int | None = None) -> bool:
+    """Whether gemm_wide takes a product of these sizes: K in stages of 64, columns in blocks of 32, rows of x and W on the
+    16-byte grid."""
+    w_stride = k if w_stride is None else w_stride
+    return (k > 0 and k % _WIDE_K == 0 and n > 0 and n % 32 == 0 and x_stride % 8 == 0 and w_stride % 8 == 0
+            and max(x_stride, w_stride) < 1 << 20)
+
+
+@functools.lru_cache(maxsize=4096)
+def wide_plan(rows: int, n: int, k: int, parts: int = 1, units: int = 256) -> tuple:
+    """((rows, columns) of a workgroup, estimated us) of gemm_wide for a product in `parts` parts of K on `units` compute
+    units."""
+    stages = -(-(k // _WIDE_K) // parts)
+    best = None
+    for (bm, bn), stage_us in WIDE_STAGE_US.items():
+        workgroups = -(-rows // bm) * -(-n // bn) * parts
+        us = -(-workgroups // units) * (_WIDE_FIXED_US + stages * stage_us)
+        if best is None or us < best[1]:
+            best = ((bm, bn), us)
+    return best
+
+
+def gemm_wide(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, shape=None, splits: int = 1):
+    """x [M, K] . W^T for prompt portions, W [N, K] as it is stored: workgroups of `shape` rows x columns (default:
+    wide_plan's), both operands through LDS.  EPI_SILU_MUL: gate and up rows of W interleaved in blocks of 16; returns
+    [M, N/2].  splits > 1: K cut into that many parts of whole stages of 64; returns the float32 stack [splits, M, N]."""
+    _gpu(x, w)
+    _rows(x, "x")
+    _rows(w, "w")
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_wide takes bfloat16 operands")
+    (M, K), N = x.shape, w.shape[0]
+    _need(w.shape[1] == K, "x and W differ in K")
+    _need(gemm_wide_supported(N, K, x.stride(0), w.stride(0)) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0,
+          "gemm_wide: K in stages of 64, N in blocks of 32, 16-byte aligned rows")
+    fused = epilogue == EPI_SILU_MUL
+    _need(out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and not fused), "gemm_wide writes bfloat16, or float32 without an epilogue")
+    stages = K // _WIDE_K
+    _need(1 <= splits <= min(stages, 65535), f"gemm_wide cannot cut {stages} stages of K into {splits} parts")
+    per = -(-stages // splits)
+    splits = -(-stages // per)      # parts of `per` stages cover K; the last one may be shorter
+    if shape is None:
+        shape = wide_plan(M, N, K, splits, _compute_units(x.device.index or 0))[0]
+    _need(tuple(shape) in WIDE_STAGE_US, f"gemm_wide has no workgroups of {shape}")
+    if splits > 1:
+        _need(not fused and out_dtype == torch.float32, "parts of K come back as a float32 stack without an epilogue")
+        out = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
+        ldo, stride = out.stride(1), out.stride(0)
+    else:
+        out = torch.empty((M, N // 2 if fused else N), dtype=out_dtype, device=x.device)
+        ldo, stride = out.stride(0), 0
+    lib.call("arle_gemm_wide", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), ldo, _CODES[out_dtype], M, N, K,
+             int(epilogue), int(shape[0]), int(shape[1]), splits, per, stride, _stream())
+    return out
+
+
 SUM_ACTS = {None: 0, "squared_relu": 1}      # what a sum of partial products passes through: nothing, or max(z, 0)^2
 
 
@@ -1248,7 +1314,22 @@ class ProductChoice:
     splits: int = 0        # parts of K; 0: the kernel's own plan
 
 
-PRODUCT_KERNELS = ("rows", "stream", "rounds", "tiles", "tiles_parts", "library", "library_parts")
+PRODUCT_KERNELS = ("rows", "stream", "rounds", "tiles", "tiles_parts", "wide", "library", "library_parts")
+
+# gate|up with its activation by gemm_wide from 65 rows on where K is at most _WIDE_MAX_K, and up to _WIDE_MID_ROWS rows
+# beyond.  MI355X, cold weights, us, the library's product and the activation kernel / gemm_tiles / gemm_wide: Qwen3-4B
+# (N 19,456, K 2,560) 97 rows 40.5 / 49.5 / 32.3, 256 51.7 / 51.0 / 35.8, 512 64.3 / 83.4 / 48.6, 1,024 115 / 120 / 84,
+# 2,048 217 / 200 / 167, 4,096 440 / 393 / 327, 8,192 772 / 793 / 648; Qwen3-8B (N 24,576, K 4,096) 256 70.2 / 78.1 / 59.4,
+# 544 133.7 / 121.0 / 98.2, 768 152.7 / 179.7 / 125.4, 1,536 264 / 298 / 248, 2,048 309 / 372 / 318, 8,192 1,218 / 1,475 / 1,249.
+_WIDE_MIN_ROWS = 65
+_WIDE_MAX_K = 3072
+_WIDE_MID_ROWS = 1792
+
+
+def gemm_wide_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
+    """Whether gate|up with its activation runs in gemm_wide (the rule for widths that no table names)."""
+    return (rows >= _WIDE_MIN_ROWS and n >= _TILES_MIN_N and gemm_wide_supported(n, k, x_stride)
+            and (k <= _WIDE_MAX_K or rows <= _WIDE_MID_ROWS))
 _PRODUCT_TABLE: dict = {}
 
 
@@ -1261,6 +1342,8 @@ def product_by_rules(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, f
             return ProductChoice("rows", (_fused_variant(rows),), 1)
         if rows and aligned and tiled and gemm_rows_rounds_preferred(rows, n, k, x_stride):
             return ProductChoice("rounds")
+        if aligned and gemm_wide_preferred(rows, n, k, x_stride):
+            return ProductChoice("wide")
         if aligned and tiled and gemm_tiles_preferred(rows, n, k, x_stride, fused=True):
             return ProductChoice("tiles", (8, 144) if rows >= _TILES_BIG_ROWS else (4, 44))
         return ProductChoice("library")
@@ -1305,6 +1388,8 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                         found.append(ProductChoice("rounds", (round_steps,)))
         if tiled and eight and n % 32 == 0 and rows > ROWS_KERNEL_MAX:
             found += [ProductChoice("tiles", v) for v in ((4, 44), (8, 144))]
+        if rows > ROWS_KERNEL_MAX and gemm_wide_supported(n, k, x_stride):
+            found.append(ProductChoice("wide"))
         return found
     if few:
         for variant in range(ROWS_VARIANTS):
@@ -1319,6 +1404,9 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                     found.append(ProductChoice("stream", (variant,), parts))
                     if parts in (2, 4, 8):      # and with two workgroups for every compute unit
                         found.append(ProductChoice("stream", (variant, 2 * _STREAM_TARGET_WORKGROUPS // parts), parts))
+    if rows > ROWS_KERNEL_MAX and gemm_wide_supported(n, k, x_stride):
+        found.append(ProductChoice("wide", (), 1))
+        found += [ProductChoice("wide", (), parts) for parts in range(2, _WIDE_MAX_PARTS + 1) if k >= 256 * parts and small(parts / 3)]
     if rows > ROWS_KERNEL_MAX // 2:
         for parts in (2, 4, 8):
             if k % (32 * parts) == 0 and small(parts):
@@ -1376,6 +1464,8 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
             return gemm_rows_rounds(x, w, x.dtype, tiles=tiles, round_steps=choice.variant[0] if choice.variant else None)
         if kernel == "tiles":
             return gemm_tiles(x, tiles, w.shape[0], x.dtype, EPI_SILU_MUL, variant=choice.variant or None)
+        if kernel == "wide":
+            return gemm_wide(x, w, x.dtype, EPI_SILU_MUL, shape=choice.variant or None)
         return silu_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), 16)
     if kernel == "rows":
         out = gemm_rows(x, w, out_dtype, variant=choice.variant[0] if choice.variant else None,
@@ -1389,6 +1479,9 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
                          splits=choice.splits)
     elif kernel == "tiles":
         out = gemm_tiles(x, tiles, w.shape[0], out_dtype, variant=choice.variant or None)
+    elif kernel == "wide":
+        parts = max(choice.splits, 1)
+        out = gemm_wide(x, w, torch.float32 if parts > 1 else out_dtype, shape=choice.variant or None, splits=parts)
     elif kernel == "library_parts":
         out = _library_mm_split_k(x, w, choice.splits)
         if out is None:

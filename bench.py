@@ -67,7 +67,7 @@ def prefill_flops(c, tokens: int) -> float:
 
 # ---- where a step's time goes: kernels of a profiled step, sorted into the parts of a layer -------------------------
 
-GEMM_NAMES = ("gemm_rows", "gemm_stream", "gemm_tiles", "gemm_f32", "Cijk_", "sum_partials", "silu_mul")
+GEMM_NAMES = ("gemm_rows", "gemm_stream", "gemm_tiles", "gemm_wide", "gemm_f32", "Cijk_", "sum_partials", "silu_mul")
 PARTS = ("qkv", "o", "gate_up", "down", "head", "attention", "qk_prep", "norm", "other")
 
 
@@ -77,7 +77,8 @@ def _template_args(name: str) -> list:
 
 def _completes_gate_up(name: str) -> bool:
     """Whether this kernel leaves gate|up complete: a product with the activation fused (gemm_rows_kernel<MT, WN,
-    WK, PD, XD, EPI, out> / gemm_tiles_kernel<MT, TN, PD, PX, PIPE, EPI, out> with EPI = 1), or the activation kernel
+    WK, PD, XD, EPI, out> / gemm_tiles_kernel<MT, TN, PD, PX, PIPE, EPI, out> / gemm_wide_kernel<WM, WN, TM, TN, EPI, out>
+    with EPI = 1), or the activation kernel
     behind a plain product."""
     if "silu_mul" in name:
         return True
@@ -86,6 +87,8 @@ def _completes_gate_up(name: str) -> bool:
         return len(args) > 5 and args[5] == "1"
     if "gemm_tiles_kernel" in name:
         return len(args) > 5 and args[5] == "1"
+    if "gemm_wide_kernel" in name:
+        return len(args) > 4 and args[4] == "1"
     return False
 
 

@@ -1,0 +1,79 @@
+"""The product for prompt portions with both operands through LDS (`ops.gemm_wide`): every workgroup shape at one row and
+column block and over their edges, strided rows, one to more stages of K than the LDS holds, parts of K, both output types,
+the activation; against the float64 product.  bfloat16 operands are exact in float32, a sum of K terms in float32 is off
+by at most K 2^-24 of the terms' absolute sum (1e-5 in relative norm here), a bfloat16 result by 2^-9 more."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+SHAPES = [(128, 64), (128, 96), (128, 128), (128, 160), (128, 192), (128, 256), (128, 320), (256, 160), (256, 192), (256, 256),
+          (192, 320), (256, 320)]
+
+
+def _operands(M, N, K, seed, pad_x=0, pad_w=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    make = lambda r, c, pad: torch.randn(r, c + pad, generator=gen, device="cuda").bfloat16()[:, :c]
+    return make(M, K, pad_x), make(N, K, pad_w)
+
+
+def _rel(got, want):
+    assert torch.isfinite(got.float()).all()
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("M,N,K,pad_x,pad_w", [(1, 32, 64, 0, 0), (33, 96, 128, 8, 0), (127, 352, 192, 0, 64), (256, 320, 256, 0, 0),
+                                                (257, 672, 320, 24, 8), (300, 1952, 1088, 0, 0)])
+def test_every_shape_over_its_edges(shape, M, N, K, pad_x, pad_w):
+    from arle_amd.kernels import ops
+
+    x, w = _operands(M, N, K, M + N, pad_x, pad_w)
+    want = x.double() @ w.double().T
+    assert _rel(ops.gemm_wide(x, w, torch.float32, shape=shape), want) < 1e-5
+    assert _rel(ops.gemm_wide(x, w, shape=shape), want) < 2.0 ** -8
+    gate_up = want.view(M, -1, 2, 16)
+    act = (torch.nn.functional.silu(gate_up[:, :, 0]) * gate_up[:, :, 1]).reshape(M, -1)
+    assert _rel(ops.gemm_wide(x, w, epilogue=ops.EPI_SILU_MUL, shape=shape), act) < 2.0 ** -8
+    for parts in (2, 3, 5):
+        if parts <= K // 64:
+            stack = ops.gemm_wide(x, w, torch.float32, shape=shape, splits=parts)
+            assert stack.dim() == 3 and _rel(stack.sum(0), want) < 1e-5
+
+
+def test_the_activation_at_the_ends_of_its_range():
+    """Gates far below and above zero: silu goes to -0 and to the gate itself, and no product with an infinity inside."""
+    from arle_amd.kernels import ops
+
+    gates = torch.tensor([-300.0, -100.0, -88.0, -20.0, -1.0, -0.0, 0.0, 1e-20, 1.0, 20.0, 90.0, 300.0, 3e4, -3e4, 5.0, -5.0])
+    x = torch.zeros(1, 64, dtype=torch.bfloat16, device="cuda")
+    x[0, 0] = 1.0
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device="cuda")
+    w[:16, 0], w[16:, 0] = gates.bfloat16().cuda(), 2.0
+    got = ops.gemm_wide(x, w, epilogue=ops.EPI_SILU_MUL)[0].double().cpu()
+    want = (torch.nn.functional.silu(gates.bfloat16().double()) * 2).bfloat16().double()
+    assert torch.isfinite(got).all() and torch.allclose(got, want, rtol=2.0 ** -8, atol=1e-30)
+
+
+@pytest.mark.parametrize("rows", [65, 97, 300, 1153, 2048])
+def test_gate_up_takes_it_by_the_rule_and_the_plan_fits(rows):
+    from arle_amd.kernels import ops
+
+    n, k = 6144, 512
+    x, w = _operands(rows, n, k, rows)
+    assert ops.choose_product(rows, n, k, k, tiled=False, fused=True, partials_ok=False).kernel == "wide"
+    want = (x.double() @ w.double().T).view(rows, -1, 2, 16)
+    want = (torch.nn.functional.silu(want[:, :, 0]) * want[:, :, 1]).reshape(rows, -1)
+    assert _rel(ops.gate_up_act(x, w), want) < 2.0 ** -8
+
+
+def test_what_it_does_not_take_goes_elsewhere():
+    from arle_amd.kernels import ops
+
+    for n, k, x_stride in ((6144, 544, 544), (6144 + 16, 512, 512), (6144, 512, 516)):
+        assert not ops.gemm_wide_supported(n, k, x_stride)
+    x, w = _operands(100, 6144, 544, 1)
+    with pytest.raises(ops.ShapeError):
+        ops.gemm_wide(x, w)
+    want = (x.double() @ w.double().T).view(100, -1, 2, 16)
+    want = (torch.nn.functional.silu(want[:, :, 0]) * want[:, :, 1]).reshape(100, -1)
+    assert _rel(ops.gate_up_act(x, w), want) < 2e-2

@@ -39,6 +39,7 @@ SOURCES = {
     "short_conv": "short_conv.hip",
     "polynorm": "polynorm.hip",
     "mlstm": "mlstm.hip",
+    "mlstm_chunks": "mlstm_chunks.hip",
     "attention_softcap": "attention_softcap.hip",
     "post_norm": "post_norm.hip",
     "latent": "latent.hip",

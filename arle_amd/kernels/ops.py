@@ -1704,6 +1704,53 @@ def mlstm_scan(q, k, v, gates, bias_i, bias_f, cap: float, s_state, n_state, m_s
     return num, nq, coefs
 
 
+# Rows of the longest segment from which a step's rows go through the matrix memory in chunks of 64.  A layer of the Gufasun
+# design at the Qwen3-4B widths (20 heads of 128 x 128) on MI355X, us, token by token / in chunks: one prompt
+# of 64 rows 45 / 32, 96 53 / 35, 128 66 / 35, 512 225 / 55, 2,048 860 / 155; 128 rows beside 16 single ones 97 / 69.
+MLSTM_CHUNK_MIN_ROWS = 96
+
+
+def mlstm_chunks_supported(longest: int, key_dim: int, value_dim: int) -> bool:
+    """Whether mlstm_chunks takes heads of these sizes, and pays for segments of up to `longest` rows."""
+    return (longest >= MLSTM_CHUNK_MIN_ROWS and key_dim % 32 == 0 and value_dim % 32 == 0 and 32 <= key_dim <= 128
+            and 32 <= value_dim <= 128)
+
+
+def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_state, seg_row0, seg_slot, weight, eps: float,
+                 out_dtype, *, heads: int, key_dim: int, value_dim: int):
+    """mlstm_scan and mlstm_output over chunks of 64 rows, the products on the 32-bit matrix instructions.  qkvg float32
+    [T, 2 H D + 2 H Dv]: q, k, v and the output gate side by side.  Returns [T, H * Dv]."""
+    _gpu(qkvg, gates, bias_i, bias_f, s_state, n_state, m_state, seg_row0, seg_slot, weight)
+    H, D, Dv = heads, key_dim, value_dim
+    _rows(qkvg, "qkvg")
+    tokens, width = qkvg.shape[0], H * Dv
+    _need(qkvg.dtype == torch.float32 and qkvg.shape[1] == 2 * H * (D + Dv) and qkvg.stride(0) % 4 == 0 and qkvg.data_ptr() % 16 == 0,
+          "qkvg must be float32 [T, 2 H (D + Dv)] with 16-byte aligned rows")
+    _need(mlstm_chunks_supported(MLSTM_CHUNK_MIN_ROWS, D, Dv), "mlstm_chunks takes heads of multiples of 32 up to 128")
+    _rows(gates, "gates")
+    _need(gates.dtype == torch.float32 and gates.shape == (tokens, 2 * H), "gates must be float32 [T, 2 * heads]")
+    _need(bias_i.shape == (H,) and bias_f.shape == (H,) and bias_i.dtype == bias_f.dtype == torch.float32
+          and bias_i.is_contiguous() and bias_f.is_contiguous(), "gate biases must be float32 [heads]")
+    slots = s_state.shape[0]
+    _need(s_state.shape == (slots, H, D, Dv) and n_state.shape == (slots, H, D) and m_state.shape == (slots, H)
+          and all(t.dtype == torch.float32 and t.is_contiguous() for t in (s_state, n_state, m_state)),
+          "mLSTM states are float32 [slots, H, D, Dv], [slots, H, D] and [slots, H]")
+    segments = seg_slot.numel()
+    _i32(seg_slot, "seg_slot")
+    _i32(seg_row0, "seg_row0", segments + 1)
+    _need(weight.shape == (width,) and weight.is_contiguous() and weight.dtype in _CODES, "the norm weight must be [H * Dv]")
+    out = torch.empty((tokens, width), dtype=out_dtype, device=qkvg.device)
+    items = _chunk_items(tokens, segments)
+    scratch = torch.empty(lib.function_raw("arle_mlstm_chunks_bytes", ctypes.c_longlong, "mlstm_chunks", (ctypes.c_int,) * 4)(
+        items, H, D, Dv), dtype=torch.uint8, device=qkvg.device)
+    at = lambda column: qkvg.data_ptr() + 4 * column
+    lib.call("arle_mlstm_chunks", at(0), at(H * D), at(2 * H * D), at(2 * H * D + width), qkvg.stride(0), gates.data_ptr(),
+             gates.stride(0), bias_i.data_ptr(), bias_f.data_ptr(), float(cap), s_state.data_ptr(), n_state.data_ptr(),
+             m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), segments, items, H, D, Dv, scratch.data_ptr(),
+             weight.data_ptr(), _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
+    return out
+
+
 def mlstm_output(num, nq, coefs, gate, weight, eps: float, out_dtype, *, heads: int, value_dim: int):
     """o = num / (max(|nq|, exp(-m)) + 1e-6); then each head's o divided by its root mean square, times `weight`
     [heads * value_dim], times sigmoid(gate)."""

@@ -7,14 +7,15 @@
 // top-k -> renormalise -> top-p -> renormalise -> inverse CDF with a uniform u
 // drawn on the host); penalties infer/src/sampler.rs:100-140.
 //
-// Differences kept on purpose: the top-k and top-p thresholds are found exactly, eight
-// bits of the bit pattern of the (non-negative) probabilities at a time, from 256-bin
+// Differences kept on purpose: the top-k and top-p thresholds are found exactly, ten or
+// eleven bits of the bit pattern of the (non-negative) probabilities at a time, from
 // histograms filled with integer atomics, instead of 32 halvings of a float interval;
 // each thread owns a contiguous run of the vocabulary so the inverse CDF walks tokens
 // in index order; one launch serves many rows with per-row parameters; and the
 // log-probability of a chosen token (the reference has it for greedy rows only,
 // sampling.cu:252-317) is a kernel of its own that serves greedy and sampled rows.
 #include "common.h"
+#include <type_traits>
 
 namespace arle {
 
@@ -148,29 +149,55 @@ __global__ __launch_bounds__(kWave) void argmax_merge_kernel(const ArgMax* __res
 //   min_p:  e >= min_p                       (the largest e is exp(0) = 1)
 //   top_k:  e >= the k-th largest e           (ties of the k-th stay)
 //   top_p:  e >= the largest t whose kept mass reaches top_p of the mass kept so far
-// The k-th largest value and the mass threshold are found digit by digit, eight bits at a time: a pass over
-// the row fills a histogram of 256 bins with the next digit of the elements that match the digits found so
-// far; scanning the bins from the top gives the digit in which the count (the mass) is reached.  Counts are
-// integers and masses are summed as 64-bit fixed-point numbers (e * 2^40), so the histograms do not depend
-// on the order in which workgroups add to them, and every workgroup that reads them finds the same digits.
-// The token is then drawn by the inverse CDF in token order: u * (kept mass) falls into a chunk, and inside
-// the chunk into a token.
+// The k-th largest value and the mass threshold are found digit by digit, 11 + 11 + 10 bits: a pass over the
+// row fills a histogram with the next digit of the elements that match the digits found so far; scanning the bins
+// from the top gives the digit in which the count (the mass) is reached.  Counts are integers and masses are summed as
+// 64-bit fixed-point numbers (e * 2^40), so the histograms do not depend on the order in which workgroups add to
+// them, and every workgroup that reads them finds the same digits.  The token is then drawn by the inverse CDF in
+// token order: u * (kept mass) falls into a chunk, and inside the chunk into a token.
+//
+// What bounds a call of few rows is the chain of kernels, of many rows reading e once a pass.  So:
+//   - the pass that makes e also fills the first histogram, of top_k, or of top_p where the row has no top_k;
+//   - it leaves the largest e of every 64 tokens; the later passes read only groups that reach the threshold's known
+//     digits (of 50 kept tokens in 151,936 at most 50 groups of 2,374);
+//   - every workgroup finds the next digit by itself, with all its threads, from one histogram: the digits before it
+//     and what is left to reach stand in the row's slot of the pass before.
+// 64 rows of 151,936 logits, kernels back to back: with top_k 50 and top_p 0.9 184 us -> 98 us, top_p alone 136 -> 83,
+// top_k alone 84 -> 71; one row 142 -> 80 (before: digits of eight bits, every pass read the whole row and scanned all
+// digits before its own with one wave, and one thread added up 256 bins).
 constexpr int kSelThreads = kChunkThreads;
 constexpr int kSelWaves = kSelThreads / kWave;
+constexpr int kGroup = kWave;                   // tokens that share a largest e
 constexpr float kMassScale = 1099511627776.0f;  // 2^40
+constexpr int kBins0 = 1024, kBins1 = 2048, kBins2 = 1024;   // a non-negative float has no bit 31: ten bits lead
+constexpr int kRowBins = kBins0 + kBins1 + kBins2;
+
+// What a pass has found of a row's threshold.
+struct Slot {
+  unsigned long long rest;   // rank (mass) still to reach inside the bin of the last digit
+  unsigned int prefix;       // the digits so far
+  unsigned int floor;        // what min_p (and, once it is known, top_k) asks of e
+  unsigned int open;         // 1: the row does not reach the rank (the mass): everything above the floor stays
+  unsigned int unused;
+};
+// The passes, in order.  FIRST, SECOND: digits 0 and 1 of top_k, or of top_p for a row without top_k.  FLOOR: the last
+// digit of top_k, and top_p's first histogram.  THIRD, FOURTH: digits 0 and 1 of top_p for a row with top_k.
+enum Pass { kFirst = 0, kSecond = 1, kFloor = 2, kThird = 3, kFourth = 4, kPasses = 5 };
 
 struct SampleArgs {
   const float* logits;
   float* e;  // [rows, vocab]
-  int vocab, chunk_len, chunks;
+  int vocab, chunk_len, chunks, groups;   // groups of kGroup tokens in a chunk
   const float* temperature;
   const int* top_k;
   const float* top_p;
   const float* min_p;
   const float* u;
   const ArgMax* part_max;          // [rows, chunks]
-  unsigned int* hist_k;            // [rows, 4, 256] counts
-  unsigned long long* hist_p;      // [rows, 4, 256] masses
+  unsigned int* hist_k;            // [rows, kRowBins] counts
+  unsigned long long* hist_p;      // [rows, kRowBins] masses
+  Slot* slots;                     // [rows, kPasses]
+  float* group_max;                // [rows, chunks, groups]
   float* chunk_mass;               // [rows, chunks]
   unsigned int* threshold;         // [rows] bits of the final threshold
   int use_top_k, use_top_p;        // 0: no row of this call uses the filter (its passes are not launched)
@@ -197,102 +224,111 @@ __device__ __forceinline__ RowParams row_params(const SampleArgs& a, int row) {
   return r;
 }
 
-__device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int src) {
+__device__ __forceinline__ unsigned int min_p_bits(const RowParams& r) {
+  return r.min_p > 0.f ? __float_as_uint(r.min_p) : 0u;
+}
+
+__device__ __forceinline__ unsigned int shfl_any(unsigned int v, int src) { return __shfl(v, src, kWave); }
+__device__ __forceinline__ unsigned long long shfl_any(unsigned long long v, int src) {
   const unsigned int lo = __shfl(static_cast<unsigned int>(v), src, kWave);
   const unsigned int hi = __shfl(static_cast<unsigned int>(v >> 32), src, kWave);
   return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
-__device__ __forceinline__ unsigned int shfl_any(unsigned int v, int src) { return __shfl(v, src, kWave); }
-__device__ __forceinline__ unsigned long long shfl_any(unsigned long long v, int src) { return shfl_u64(v, src); }
-
-// Digits of the threshold, most significant first, from `levels` histograms [levels][256] (level l holds the
-// elements that match the digits of the levels before it).  need: the rank (the mass) to reach, counted from
-// the top, at least 1.  Every thread of the workgroup calls this; bins is LDS [levels * 256], result LDS [4].
-// Returns false when the whole row does not reach `need` (then everything is kept).  prefix: the digits found,
-// rest: what is left to reach inside the bin of the last digit.
-template <typename T>
-__device__ bool select_digits(const T* __restrict__ hist, int levels, T need, T* bins, unsigned long long* result,
-                              unsigned int& prefix, T& rest) {
-  for (int l = 0; l < levels; ++l) bins[l * 256 + threadIdx.x] = hist[l * 256 + threadIdx.x];
-  __syncthreads();
-  if (threadIdx.x < kWave) {
-    const int lane = threadIdx.x;
-    unsigned int digits = 0;
-    bool ok = true;
-    for (int l = 0; l < levels && ok; ++l) {
-      T m[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) m[j] = bins[l * 256 + 4 * lane + j];
-      const T own = m[0] + m[1] + m[2] + m[3];
-      T suffix = own;  // sum over the bins of this lane and of the lanes above it
-#pragma unroll
-      for (int off = 1; off < kWave; off <<= 1) {
-        const T other = shfl_any(suffix, min(lane + off, kWave - 1));
-        if (lane + off < kWave) suffix += other;
-      }
-      const T above_lane = suffix - own;
-      const bool here = above_lane < need && suffix >= need;
-      unsigned int digit = 0;
-      T left = 0;
-      if (here) {
-        T above = above_lane;
-#pragma unroll
-        for (int j = 3; j >= 0; --j) {
-          if (left == 0 && above + m[j] >= need) {
-            digit = 4 * lane + j;
-            left = need - above;  // >= 1
-          }
-          above += m[j];
-        }
-      }
-      const unsigned long long votes = __ballot(here);
-      if (votes == 0ull) {
-        ok = false;
-      } else {
-        const int src = __ffsll(static_cast<long long>(votes)) - 1;
-        digits = (digits << 8) | shfl_any(digit, src);
-        need = shfl_any(left, src);
-      }
-    }
-    if (lane == 0) {
-      result[0] = ok ? 1ull : 0ull;
-      result[1] = digits;
-      result[2] = static_cast<unsigned long long>(need);
-    }
-  }
-  __syncthreads();
-  prefix = static_cast<unsigned int>(result[1]);
-  rest = static_cast<T>(result[2]);
-  const bool ok = result[0] != 0ull;
-  __syncthreads();  // bins and result may be used again
-  return ok;
-}
 
 struct SelectLds {
-  unsigned long long bins[4 * 256];
-  unsigned long long result[4];
+  unsigned long long wave_total[kSelWaves];
+  unsigned long long rest;
+  unsigned int digit, ok;
 };
-
-// Bits of the top-k threshold of a row (0: keep everything), from the four count histograms.
-__device__ unsigned int top_k_bits(const SampleArgs& a, int row, const RowParams& r, SelectLds& lds) {
-  if (!r.k_active) return 0u;  // the same for every thread
-  unsigned int prefix, rest;
-  const bool ok = select_digits<unsigned int>(a.hist_k + static_cast<int64_t>(row) * 1024, 4,
-                                              static_cast<unsigned int>(r.k),
-                                              reinterpret_cast<unsigned int*>(lds.bins), lds.result, prefix, rest);
-  return ok ? prefix : 0u;
-}
-
-// The threshold below which min_p and top_k drop a token.
-__device__ unsigned int floor_bits(const SampleArgs& a, int row, const RowParams& r, SelectLds& lds) {
-  const unsigned int mp = r.min_p > 0.f ? __float_as_uint(r.min_p) : 0u;
-  return max(mp, top_k_bits(a, row, r, lds));
-}
 
 // What top_p asks of the kept mass, as a fixed-point number (at least 1).
 __device__ __forceinline__ unsigned long long top_p_need(float top_p, unsigned long long total) {
   const unsigned long long need = static_cast<unsigned long long>(static_cast<double>(top_p) * static_cast<double>(total));
   return need < 1ull ? 1ull : need;
+}
+
+// The digit in which a histogram of BINS bins, counted from the top, reaches need(total) >= 1, and what is left to reach
+// inside that bin.  False when the whole histogram does not.  Every thread of the workgroup calls it.
+template <int BINS, typename T, typename Need>
+__device__ __forceinline__ bool select_digit(const T* __restrict__ hist, Need need_of, SelectLds& lds, unsigned int& digit, T& rest) {
+  constexpr int kPer = BINS / kSelThreads;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  T m[kPer];
+  T own = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    m[j] = hist[kPer * threadIdx.x + j];
+    own += m[j];
+  }
+  T suffix = own;  // over the bins of this thread and of the wave's threads above it
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const T other = shfl_any(suffix, min(lane + off, kWave - 1));
+    if (lane + off < kWave) suffix += other;
+  }
+  if (lane == 0) lds.wave_total[wave] = static_cast<unsigned long long>(suffix);
+  if (threadIdx.x == 0) lds.ok = 0u;
+  __syncthreads();
+  T above = suffix - own, total = 0;
+#pragma unroll
+  for (int w = 0; w < kSelWaves; ++w) {
+    const T t = static_cast<T>(lds.wave_total[w]);
+    total += t;
+    if (w > wave) above += t;
+  }
+  const T need = need_of(total);
+  if (above < need && above + own >= need) {   // one thread: the sums grow from thread to thread downwards
+    unsigned int at = 0u;
+    T left = 0;
+#pragma unroll
+    for (int j = kPer - 1; j >= 0; --j) {
+      if (left == 0 && above + m[j] >= need) {
+        at = kPer * threadIdx.x + j;
+        left = need - above;  // >= 1
+      }
+      above += m[j];
+    }
+    lds.digit = at;
+    lds.rest = static_cast<unsigned long long>(left);
+    lds.ok = 1u;
+  }
+  __syncthreads();
+  const bool ok = lds.ok != 0u;
+  digit = lds.digit;
+  rest = static_cast<T>(lds.rest);
+  __syncthreads();  // lds may be used again
+  return ok;
+}
+
+// Digit LEVEL of a threshold, from its histogram (the row's kRowBins bins) and what the pass before found.
+template <int LEVEL, typename T, typename Need>
+__device__ __forceinline__ Slot next_digit(const T* __restrict__ row_bins, Need first_need, Slot s, SelectLds& lds) {
+  constexpr int kBins = LEVEL == 0 ? kBins0 : LEVEL == 1 ? kBins1 : kBins2;
+  constexpr int kAt = LEVEL == 0 ? 0 : LEVEL == 1 ? kBins0 : kBins0 + kBins1;
+  constexpr int kBits = LEVEL == 0 ? 10 : LEVEL == 1 ? 11 : 10;
+  if (s.open) return s;  // the same for every thread
+  unsigned int digit;
+  T rest;
+  const T left = static_cast<T>(s.rest);
+  const bool ok = select_digit<kBins, T>(row_bins + kAt, [&](T total) { return LEVEL == 0 ? first_need(total) : left; }, lds,
+                                         digit, rest);
+  if (!ok) {
+    s.open = 1u;
+  } else {
+    s.prefix = LEVEL == 0 ? digit : (s.prefix << kBits) | digit;
+    s.rest = static_cast<unsigned long long>(rest);
+  }
+  return s;
+}
+template <int LEVEL>
+__device__ __forceinline__ Slot next_k(const SampleArgs& a, int row, const RowParams& r, const Slot& s, SelectLds& lds) {
+  return next_digit<LEVEL, unsigned int>(a.hist_k + static_cast<int64_t>(row) * kRowBins,
+                                         [&](unsigned int) { return static_cast<unsigned int>(r.k); }, s, lds);
+}
+template <int LEVEL>
+__device__ __forceinline__ Slot next_p(const SampleArgs& a, int row, const RowParams& r, const Slot& s, SelectLds& lds) {
+  return next_digit<LEVEL, unsigned long long>(a.hist_p + static_cast<int64_t>(row) * kRowBins,
+                                               [&](unsigned long long total) { return top_p_need(r.top_p, total); }, s, lds);
 }
 
 __device__ __forceinline__ float merged_max(const SampleArgs& a, int row, float* lds /* [kSelWaves] */) {
@@ -302,98 +338,186 @@ __device__ __forceinline__ float merged_max(const SampleArgs& a, int row, float*
   return block_max<kSelWaves>(v, lds);
 }
 
-// e = exp(x / T - max) for the chunk, and the first digit's histogram of top_k.
+// Calls take(e) for the tokens of a chunk whose group of 64 reaches `lower` (bits); wave w has the groups w, w + 4, ..,
+// in this order, a token a lane: a thread meets the tokens threadIdx.x, threadIdx.x + 256, .. of the chunk.
+template <typename Take>
+__device__ __forceinline__ void walk_chunk(const SampleArgs& a, int row, int chunk, unsigned int lower, Take take) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int begin = chunk * a.chunk_len, len = min(a.vocab - begin, a.chunk_len);
+  const float* e = a.e + static_cast<int64_t>(row) * a.vocab + begin;
+  const float* gm = a.group_max + (static_cast<int64_t>(row) * a.chunks + chunk) * a.groups;
+  const int have = (max(len, 0) + kGroup - 1) / kGroup;
+  for (int base = wave; base < have; base += kSelWaves * kWave) {
+    const int g = base + kSelWaves * lane;
+    const bool live = g < have && __float_as_uint(gm[min(g, have - 1)]) >= lower;
+    unsigned long long mask = __ballot(live);
+    while (mask != 0ull) {
+      float v[4];
+      bool in[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = mask != 0ull ? __builtin_ctzll(mask) : 0;
+        const int i = (base + kSelWaves * at) * kGroup + lane;
+        in[j] = mask != 0ull && i < len;
+        mask &= mask - 1ull;   // 0 stays 0
+        v[j] = in[j] ? e[i] : -1.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (in[j]) take(v[j]);
+    }
+  }
+}
+
+// Adds digit LEVEL of the chunk's tokens that match the slot's digits and reach its floor to the row's histogram.
+template <int LEVEL, bool MASS>
+__device__ __forceinline__ void fill_bins(const SampleArgs& a, int row, int chunk, const Slot& s, void* lds_bins) {
+  using T = std::conditional_t<MASS, unsigned long long, unsigned int>;
+  constexpr int kBins = LEVEL == 0 ? kBins0 : LEVEL == 1 ? kBins1 : kBins2;
+  constexpr int kAt = LEVEL == 0 ? 0 : LEVEL == 1 ? kBins0 : kBins0 + kBins1;
+  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 0 ? 21 : LEVEL == 1 ? 10 : 0;
+  T* bins = static_cast<T*>(lds_bins);
+#pragma unroll
+  for (int j = 0; j < kBins / kSelThreads; ++j) bins[j * kSelThreads + threadIdx.x] = 0;
+  __syncthreads();
+  const unsigned int prefix = s.prefix, floor = s.floor;
+  walk_chunk(a, row, chunk, LEVEL == 0 ? floor : max(floor, prefix << kHigh), [&](float v) {
+    const unsigned int bits = __float_as_uint(v);
+    if (!(v >= 0.f && bits >= floor && (LEVEL == 0 || (bits >> kHigh) == prefix))) return;
+    const T n = MASS ? static_cast<T>(v * kMassScale) : static_cast<T>(1);
+    if (n) atomicAdd(&bins[(bits >> kLow) & (kBins - 1)], n);
+  });
+  __syncthreads();
+  T* to = (MASS ? reinterpret_cast<T*>(a.hist_p) : reinterpret_cast<T*>(a.hist_k)) + static_cast<int64_t>(row) * kRowBins + kAt;
+#pragma unroll
+  for (int j = 0; j < kBins / kSelThreads; ++j) {
+    const T n = bins[j * kSelThreads + threadIdx.x];
+    if (n) atomicAdd(to + j * kSelThreads + threadIdx.x, n);
+  }
+}
+
+__device__ __forceinline__ float row16_max(float v) {   // over the 16 lanes of a row, into all of them
+#define ARLE_ROR_MAX(n) \
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n, 0xf, 0xf, true)));
+  ARLE_ROR_MAX(8) ARLE_ROR_MAX(4) ARLE_ROR_MAX(2) ARLE_ROR_MAX(1)
+#undef ARLE_ROR_MAX
+  return v;
+}
+
+// e = exp(x / T - max) for the chunk, the largest e of its groups, and the first histogram: top_k's, or top_p's for a row
+// without top_k.  A thread takes four tokens at a time.  Neighbouring tokens fall into the same few bins, so the workgroup
+// keeps several copies of the histogram, lane by lane in turn, and adds them up at its end.
 __global__ __launch_bounds__(kSelThreads) void sample_exp_kernel(const SampleArgs a) {
+  constexpr int kCopiesK = 4, kCopiesP = 2;
   __shared__ float red[kSelWaves];
-  __shared__ unsigned int hist[256];
+  __shared__ unsigned long long bins[kCopiesP * kBins0];
+  static_assert(sizeof(bins) == kCopiesK * kBins0 * sizeof(unsigned int), "both histograms fill the same LDS");
   const int row = blockIdx.y, chunk = blockIdx.x;
   const RowParams r = row_params(a, row);
   if (r.greedy) return;
-  hist[threadIdx.x] = 0u;
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool by_mass = r.p_active && !r.k_active, any = r.k_active || r.p_active;
+  const int begin = chunk * a.chunk_len, len = min(a.vocab - begin, a.chunk_len);
+  const float* x = a.logits + static_cast<int64_t>(row) * a.vocab + begin;
+  float* e = a.e + static_cast<int64_t>(row) * a.vocab + begin;
+  float* gm = a.group_max + (static_cast<int64_t>(row) * a.chunks + chunk) * a.groups;
+  const bool wide = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(e) % 16 == 0;
+  auto load = [&](int at) {
+    float4 v = {0.f, 0.f, 0.f, 0.f};
+    if (wide && at + 4 <= len) return *reinterpret_cast<const float4*>(x + at);
+    if (at < len) v.x = x[at];
+    if (at + 1 < len) v.y = x[at + 1];
+    if (at + 2 < len) v.z = x[at + 2];
+    if (at + 3 < len) v.w = x[at + 3];
+    return v;
+  };
+  float4 next = load(4 * static_cast<int>(threadIdx.x));
+  if (any)
+#pragma unroll
+    for (int j = 0; j < kCopiesP * kBins0 / kSelThreads; ++j) bins[j * kSelThreads + threadIdx.x] = 0ull;
   const float mx = merged_max(a, row, red) * r.inv_t;  // the block reduction also orders the LDS writes above
-  const float* x = a.logits + static_cast<int64_t>(row) * a.vocab;
-  float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
-  const unsigned int mp = r.min_p > 0.f ? __float_as_uint(r.min_p) : 0u;
-  for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads) {
-    const float v = expf(x[i] * r.inv_t - mx);
-    e[i] = v;
-    const unsigned int bits = __float_as_uint(v);
-    if (r.k_active && v >= 0.f && bits >= mp) atomicAdd(&hist[bits >> 24], 1u);
-  }
-  if (!r.k_active) return;
-  __syncthreads();
-  const unsigned int n = hist[threadIdx.x];
-  if (n) atomicAdd(a.hist_k + static_cast<int64_t>(row) * 1024 + threadIdx.x, n);
-}
-
-// Digit `level` (1..3) of the top_k threshold.
-__global__ __launch_bounds__(kSelThreads) void sample_top_k_kernel(const SampleArgs a, int level) {
-  __shared__ SelectLds sel;
-  __shared__ unsigned int hist[256];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  const RowParams r = row_params(a, row);
-  if (r.greedy || !r.k_active) return;
-  unsigned int prefix, rest;
-  const bool ok = select_digits<unsigned int>(a.hist_k + static_cast<int64_t>(row) * 1024, level,
-                                              static_cast<unsigned int>(r.k),
-                                              reinterpret_cast<unsigned int*>(sel.bins), sel.result, prefix, rest);
-  if (!ok) return;  // fewer than k tokens are left: all of them stay
-  hist[threadIdx.x] = 0u;
-  __syncthreads();
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
-  const unsigned int mp = r.min_p > 0.f ? __float_as_uint(r.min_p) : 0u;
-  const int high = 32 - 8 * level, low = 24 - 8 * level;
-  for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads) {
-    const float v = e[i];
-    const unsigned int bits = __float_as_uint(v);
-    if (v >= 0.f && bits >= mp && (bits >> high) == prefix) atomicAdd(&hist[(bits >> low) & 255u], 1u);
-  }
-  __syncthreads();
-  const unsigned int n = hist[threadIdx.x];
-  if (n) atomicAdd(a.hist_k + static_cast<int64_t>(row) * 1024 + level * 256 + threadIdx.x, n);
-}
-
-// Digit `level` (0..3) of the top_p threshold, over what min_p and top_k have kept.
-__global__ __launch_bounds__(kSelThreads) void sample_top_p_kernel(const SampleArgs a, int level) {
-  __shared__ SelectLds sel;
-  __shared__ unsigned long long hist[256];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  const RowParams r = row_params(a, row);
-  if (r.greedy || !r.p_active) return;
-  const unsigned int floor = floor_bits(a, row, r, sel);
-  const unsigned long long* hp = a.hist_p + static_cast<int64_t>(row) * 1024;
-  unsigned int prefix = 0u;
-  if (level > 0) {
-    // the whole kept mass is the sum of the first histogram
-    sel.bins[threadIdx.x] = hp[threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long total = 0ull;
-      for (int b = 0; b < 256; ++b) total += sel.bins[b];
-      sel.result[3] = total;
+  const unsigned int mp = min_p_bits(r);
+  unsigned int* counts = reinterpret_cast<unsigned int*>(bins);
+  for (int base = 0; base < len; base += 4 * kSelThreads) {
+    const int at = base + 4 * static_cast<int>(threadIdx.x);
+    const float4 in = next;
+    next = load(at + 4 * kSelThreads);
+    const float v[4] = {expf(in.x * r.inv_t - mx), expf(in.y * r.inv_t - mx), expf(in.z * r.inv_t - mx),
+                        expf(in.w * r.inv_t - mx)};
+    float most = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (at + j < len) most = fmaxf(most, v[j]);
+    if (wide && at + 4 <= len) {
+      *reinterpret_cast<float4*>(e + at) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (at + j < len) e[at + j] = v[j];
     }
-    __syncthreads();
-    const unsigned long long need = top_p_need(r.top_p, sel.result[3]);
-    __syncthreads();
-    unsigned long long rest;
-    if (!select_digits<unsigned long long>(hp, level, need, sel.bins, sel.result, prefix, rest)) return;
+    if (any) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const unsigned int bits = __float_as_uint(v[j]);
+        if (!(at + j < len && v[j] >= 0.f && bits >= mp)) continue;
+        const unsigned int bin = (bits >> 21) & (kBins0 - 1);
+        if (by_mass) {
+          const unsigned long long n = static_cast<unsigned long long>(v[j] * kMassScale);
+          if (n) atomicAdd(&bins[bin * kCopiesP + (lane & (kCopiesP - 1))], n);
+        } else {
+          atomicAdd(&counts[bin * kCopiesK + (lane & (kCopiesK - 1))], 1u);
+        }
+      }
+    }
+    most = row16_max(most);
+    if ((lane & 15) == 0 && at < len) gm[at / kGroup] = most;
   }
-  hist[threadIdx.x] = 0ull;
+  if (!any) return;
   __syncthreads();
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
-  const int high = 32 - 8 * level, low = 24 - 8 * level;
-  for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads) {
-    const float v = e[i];
-    const unsigned int bits = __float_as_uint(v);
-    if (v >= 0.f && bits >= floor && (level == 0 || (bits >> high) == prefix))
-      atomicAdd(&hist[(bits >> low) & 255u], static_cast<unsigned long long>(v * kMassScale));
+  for (int bin = threadIdx.x; bin < kBins0; bin += kSelThreads) {
+    if (by_mass) {
+      unsigned long long n = 0ull;
+#pragma unroll
+      for (int c = 0; c < kCopiesP; ++c) n += bins[bin * kCopiesP + c];
+      if (n) atomicAdd(a.hist_p + static_cast<int64_t>(row) * kRowBins + bin, n);
+    } else {
+      unsigned int n = 0u;
+#pragma unroll
+      for (int c = 0; c < kCopiesK; ++c) n += counts[bin * kCopiesK + c];
+      if (n) atomicAdd(a.hist_k + static_cast<int64_t>(row) * kRowBins + bin, n);
+    }
   }
-  __syncthreads();
-  const unsigned long long n = hist[threadIdx.x];
-  if (n) atomicAdd(const_cast<unsigned long long*>(hp) + level * 256 + threadIdx.x, n);
+}
+
+// One pass: the next digit of the row's threshold, and the histogram of the one after it.
+template <int PASS>
+__global__ __launch_bounds__(kSelThreads) void sample_pass_kernel(const SampleArgs a) {
+  __shared__ unsigned long long bins[kBins1];
+  __shared__ SelectLds sel;
+  const int row = blockIdx.y, chunk = blockIdx.x;
+  const RowParams r = row_params(a, row);
+  if (r.greedy) return;
+  if (PASS >= kFloor ? !(r.k_active && r.p_active) : !(r.k_active || r.p_active)) return;
+  Slot* slots = a.slots + static_cast<int64_t>(row) * kPasses;
+  Slot s = {0ull, 0u, min_p_bits(r), 0u, 0u};
+  if constexpr (PASS > 0) s = slots[PASS - 1];
+  if constexpr (PASS == kFirst) s = r.k_active ? next_k<0>(a, row, r, s, sel) : next_p<0>(a, row, r, s, sel);
+  if constexpr (PASS == kSecond) s = r.k_active ? next_k<1>(a, row, r, s, sel) : next_p<1>(a, row, r, s, sel);
+  if constexpr (PASS == kFloor) {
+    s = next_k<2>(a, row, r, s, sel);
+    const unsigned int floor = s.open ? s.floor : max(s.floor, s.prefix);
+    s = Slot{0ull, 0u, floor, 0u, 0u};
+  }
+  if constexpr (PASS == kThird) s = next_p<0>(a, row, r, s, sel);
+  if constexpr (PASS == kFourth) s = next_p<1>(a, row, r, s, sel);
+  if (chunk == 0 && threadIdx.x == 0) slots[PASS] = s;
+  if (s.open) return;
+  if constexpr (PASS == kFirst || PASS == kSecond) {
+    if (r.k_active) fill_bins<PASS == kFirst ? 1 : 2, false>(a, row, chunk, s, bins);
+    else fill_bins<PASS == kFirst ? 1 : 2, true>(a, row, chunk, s, bins);
+  } else {
+    fill_bins<PASS - kFloor, true>(a, row, chunk, s, bins);
+  }
 }
 
 // The final threshold of the row and the kept mass of every chunk.
@@ -403,39 +527,29 @@ __global__ __launch_bounds__(kSelThreads) void sample_mass_kernel(const SampleAr
   const int row = blockIdx.y, chunk = blockIdx.x;
   const RowParams r = row_params(a, row);
   if (r.greedy) return;
-  unsigned int thr = floor_bits(a, row, r, sel);
-  if (r.p_active) {
-    const unsigned long long* hp = a.hist_p + static_cast<int64_t>(row) * 1024;
-    sel.bins[threadIdx.x] = hp[threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long total = 0ull;
-      for (int b = 0; b < 256; ++b) total += sel.bins[b];
-      sel.result[3] = total;
-    }
-    __syncthreads();
-    const unsigned long long need = top_p_need(r.top_p, sel.result[3]);
-    __syncthreads();
-    unsigned int prefix;
-    unsigned long long rest;
-    if (select_digits<unsigned long long>(hp, 4, need, sel.bins, sel.result, prefix, rest)) thr = max(thr, prefix);
+  unsigned int thr = min_p_bits(r);
+  if (r.k_active || r.p_active) {
+    Slot s = a.slots[static_cast<int64_t>(row) * kPasses + (r.k_active && r.p_active ? kFourth : kSecond)];
+    s = r.p_active ? next_p<2>(a, row, r, s, sel) : next_k<2>(a, row, r, s, sel);
+    thr = s.open ? s.floor : max(s.floor, s.prefix);
   }
   if (chunk == 0 && threadIdx.x == 0) a.threshold[row] = thr;
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
   float mass = 0.f;
-  for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads) {
-    const float v = e[i];
+  walk_chunk(a, row, chunk, thr, [&](float v) {
     if (v >= 0.f && __float_as_uint(v) >= thr) mass += v;
-  }
+  });
   mass = block_sum<kSelWaves>(mass, red);
   if (threadIdx.x == 0) a.chunk_mass[static_cast<int64_t>(row) * a.chunks + chunk] = mass;
+}
+
+__device__ __forceinline__ float lane_value(float v, int lane /* the same in every lane */) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // The token: greedy rows take the first maximum; the others the inverse CDF in token order.
 __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleArgs a) {
   __shared__ ArgMax best[kSelWaves];
-  __shared__ float part[kSelThreads];
+  __shared__ alignas(16) float part[kSelThreads];
   __shared__ float chunk_start;
   __shared__ int chunk_of_target, chosen;
   const int row = blockIdx.x;
@@ -464,29 +578,44 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
   }
   const unsigned int thr = a.threshold[row];
   const float* masses = a.chunk_mass + static_cast<int64_t>(row) * a.chunks;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < kWave) {   // wave 0: lane l has the masses 4 l .. 4 l + 3; lanes without any add nothing
+    const int lane = threadIdx.x;
+    float m[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m[j] = 4 * lane + j < a.chunks ? masses[4 * lane + j] : 0.f;
+    const unsigned long long some = __ballot(m[0] > 0.f || m[1] > 0.f || m[2] > 0.f || m[3] > 0.f);
     float total = 0.f;
-    for (int c = 0; c < a.chunks; ++c) total += masses[c];
+    for (unsigned long long left = some; left != 0ull; left &= left - 1ull) {
+      const int l = __builtin_ctzll(left);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) total += lane_value(m[j], l);
+    }
     const float target = a.u[row] * total;
     float run = 0.f;
     int at = -1, last = 0;
     float start = 0.f, last_start = 0.f;
-    for (int c = 0; c < a.chunks; ++c) {
-      const float m = masses[c];
-      if (m > 0.f) {
-        last = c;
-        last_start = run;
+    for (unsigned long long left = some; left != 0ull && at < 0; left &= left - 1ull) {
+      const int l = __builtin_ctzll(left);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float mass = lane_value(m[j], l);
+        if (mass > 0.f) {
+          last = 4 * l + j;
+          last_start = run;
+          if (at < 0 && target < run + mass) {
+            at = last;
+            start = run;
+          }
+        }
+        run += mass;
       }
-      if (at < 0 && target < run + m) {
-        at = c;
-        start = run;
-      }
-      run += m;
     }
-    chunk_of_target = at >= 0 ? at : last;  // u at or past the whole mass (rounding): the last chunk that holds any
-    chunk_start = at >= 0 ? start : last_start;
-    part[0] = target;
-    chosen = -1;
+    if (lane == 0) {
+      chunk_of_target = at >= 0 ? at : last;  // u at or past the whole mass (rounding): the last chunk that holds any
+      chunk_start = at >= 0 ? start : last_start;
+      part[0] = target;
+      chosen = -1;
+    }
   }
   __syncthreads();
   const int chunk = chunk_of_target;
@@ -502,17 +631,32 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
     const float v = e[i];
     return (v >= 0.f && __float_as_uint(v) >= thr) ? v : 0.f;
   };
+  const float* gm = a.group_max + (static_cast<int64_t>(row) * a.chunks + chunk) * a.groups;
+  bool live = false;   // a group that the thread's tokens lie in reaches the threshold
+  if (lo < hi)
+    for (int g = (lo - begin) / kGroup; g <= (hi - 1 - begin) / kGroup; ++g) live |= __float_as_uint(gm[g]) >= thr;
   float mine = 0.f;
-  for (int i = lo; i < hi; ++i) mine += kept(i);
+  if (live)
+#pragma unroll 4
+    for (int i = lo; i < hi; ++i) mine += kept(i);
   part[threadIdx.x] = mine;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float run = before;  // exclusive prefix, serial
-    for (int t = 0; t < kSelThreads; ++t) {
-      const float c = part[t];
-      part[t] = run;
-      run += c;
+  if (threadIdx.x < kWave) {   // exclusive prefix in the threads' order: wave 0, four threads a lane; lanes without mass add nothing
+    const int lane = threadIdx.x;
+    const float4 c = *reinterpret_cast<const float4*>(&part[4 * lane]);
+    float run = before;
+    float4 own = {before, before, before, before};
+    for (unsigned long long left = __ballot(c.x > 0.f || c.y > 0.f || c.z > 0.f || c.w > 0.f); left != 0ull; left &= left - 1ull) {
+      const int l = __builtin_ctzll(left);
+      float4 p;
+      p.x = run;
+      p.y = p.x + lane_value(c.x, l);
+      p.z = p.y + lane_value(c.y, l);
+      p.w = p.z + lane_value(c.z, l);
+      run = p.w + lane_value(c.w, l);
+      if (lane == l) own = p;
     }
+    *reinterpret_cast<float4*>(&part[4 * lane]) = own;
   }
   __syncthreads();
   const float start = part[threadIdx.x];
@@ -603,13 +747,18 @@ extern "C" int arle_argmax_rows(const float* logits, int rows, int vocab, int* o
 }
 
 // Scratch of a sampling call, in bytes: the histograms (which the caller hands over filled with zeros: the whole
-// scratch may simply be zeroed), the chunk maxima and masses, and the thresholds.
-static inline size_t sample_hist_p_bytes(int rows) { return static_cast<size_t>(rows) * 1024 * sizeof(unsigned long long); }
-static inline size_t sample_hist_k_bytes(int rows) { return static_cast<size_t>(rows) * 1024 * sizeof(unsigned int); }
+// scratch may simply be zeroed), the passes' slots, the chunk maxima and masses, the groups' maxima and the thresholds.
+static inline int sample_chunk_len(int vocab, int chunks) { return (((vocab + chunks - 1) / chunks) + 3) & ~3; }
+static inline int sample_groups(int vocab, int chunks) { return (sample_chunk_len(vocab, chunks) + kGroup - 1) / kGroup; }
+static inline size_t sample_hist_p_bytes(int rows) { return static_cast<size_t>(rows) * kRowBins * sizeof(unsigned long long); }
+static inline size_t sample_hist_k_bytes(int rows) { return static_cast<size_t>(rows) * kRowBins * sizeof(unsigned int); }
 extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
-  const size_t chunks = static_cast<size_t>(arle_argmax_chunks(rows, vocab));
-  return static_cast<long long>(sample_hist_p_bytes(rows) + sample_hist_k_bytes(rows) +
-                                rows * chunks * (sizeof(ArgMax) + sizeof(float)) + rows * sizeof(unsigned int));
+  const int chunks = arle_argmax_chunks(rows, vocab);
+  return static_cast<long long>(sample_hist_p_bytes(rows) + static_cast<size_t>(rows) * kPasses * sizeof(Slot) +
+                                sample_hist_k_bytes(rows) +
+                                static_cast<size_t>(rows) * chunks *
+                                    (sizeof(ArgMax) + sizeof(float) + sample_groups(vocab, chunks) * sizeof(float)) +
+                                rows * sizeof(unsigned int));
 }
 
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
@@ -628,7 +777,8 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.e = probs;
   a.vocab = vocab;
   a.chunks = arle_argmax_chunks(rows, vocab);
-  a.chunk_len = (((vocab + a.chunks - 1) / a.chunks) + 3) & ~3;
+  a.chunk_len = sample_chunk_len(vocab, a.chunks);
+  a.groups = sample_groups(vocab, a.chunks);
   a.temperature = temperature;
   a.top_k = top_k;
   a.top_p = top_p;
@@ -637,6 +787,8 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   unsigned char* at = static_cast<unsigned char*>(scratch);
   a.hist_p = reinterpret_cast<unsigned long long*>(at);
   at += sample_hist_p_bytes(rows);
+  a.slots = reinterpret_cast<Slot*>(at);
+  at += static_cast<size_t>(rows) * kPasses * sizeof(Slot);
   a.hist_k = reinterpret_cast<unsigned int*>(at);
   at += sample_hist_k_bytes(rows);
   ArgMax* part_max = reinterpret_cast<ArgMax*>(at);
@@ -644,6 +796,8 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   at += static_cast<size_t>(rows) * a.chunks * sizeof(ArgMax);
   a.chunk_mass = reinterpret_cast<float*>(at);
   at += static_cast<size_t>(rows) * a.chunks * sizeof(float);
+  a.group_max = reinterpret_cast<float*>(at);
+  at += static_cast<size_t>(rows) * a.chunks * a.groups * sizeof(float);
   a.threshold = reinterpret_cast<unsigned int*>(at);
   a.use_top_k = use_top_k;
   a.use_top_p = use_top_p;
@@ -651,10 +805,15 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   const dim3 grid(a.chunks, rows);
   argmax_chunks_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, part_max);
   sample_exp_kernel<<<grid, kSelThreads, 0, s>>>(a);
-  if (use_top_k)
-    for (int level = 1; level < 4; ++level) sample_top_k_kernel<<<grid, kSelThreads, 0, s>>>(a, level);
-  if (use_top_p)
-    for (int level = 0; level < 4; ++level) sample_top_p_kernel<<<grid, kSelThreads, 0, s>>>(a, level);
+  if (use_top_k || use_top_p) {
+    sample_pass_kernel<kFirst><<<grid, kSelThreads, 0, s>>>(a);
+    sample_pass_kernel<kSecond><<<grid, kSelThreads, 0, s>>>(a);
+  }
+  if (use_top_k && use_top_p) {
+    sample_pass_kernel<kFloor><<<grid, kSelThreads, 0, s>>>(a);
+    sample_pass_kernel<kThird><<<grid, kSelThreads, 0, s>>>(a);
+    sample_pass_kernel<kFourth><<<grid, kSelThreads, 0, s>>>(a);
+  }
   sample_mass_kernel<<<grid, kSelThreads, 0, s>>>(a);
   sample_pick_kernel<<<rows, kSelThreads, 0, s>>>(a);
   return launch_status();

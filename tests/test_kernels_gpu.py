@@ -435,6 +435,30 @@ def test_sampling_of_long_rows_cut_into_chunks(rows, vocab):
         assert got[r] == plain.sample_token(logits[r], p["temperature"], 0.44, -1, 1.0, p.get("min_p", 0.0)), (r, p)
 
 
+@pytest.mark.parametrize("vocab", [63, 64, 65, 1025, 8191, 8193, 16449])
+def test_sampling_at_the_edges_of_groups_and_chunks(vocab):
+    """Kept tokens at the ends of a row, ties of the k-th that fill other groups of 64, rows without any spread, and
+    every combination of filters (each takes its own passes) in one call and in calls of their own."""
+    g = _g(62)
+    base = torch.randn(4, vocab, generator=g).mul_(2.0)
+    base[0, [0, vocab - 1]] = 9.0                                   # a row's first and last token hold nearly all mass
+    base[1] = 0.25                                                  # all alike: the k-th's ties are the whole row
+    base[2] = torch.where(torch.arange(vocab) % 61 == 0, 3.0, -30.0)  # ties, one to a group or none
+    filters = [dict(top_k=5), dict(top_p=0.7), dict(top_k=5, top_p=0.7), dict(min_p=0.2, top_p=0.7), dict(min_p=0.2), dict()]
+    pars = [p for p in filters for _ in range(4)]
+    logits = base.repeat(len(filters), 1).contiguous()
+    for u in (0.02, 0.497, 0.98):
+        want = [plain.sample_token(row, 0.9, u, p.get("top_k", -1), p.get("top_p", 1.0), p.get("min_p", 0.0))
+                for row, p in zip(logits, pars)]
+        column = lambda key, default, dtype: torch.tensor([p.get(key, default) for p in pars], dtype=dtype, device=DEV)
+        full = lambda v: torch.full((len(pars),), v, dtype=torch.float32, device=DEV)
+        got = ops.sample_rows(logits.to(DEV), full(0.9), column("top_k", -1, torch.int32), column("top_p", 1.0, torch.float32),
+                              column("min_p", 0.0, torch.float32), full(u)).tolist()
+        assert got == want, u
+        for n, p in enumerate(filters):
+            assert _sample(base, 0.9, u, **p) == want[4 * n:4 * n + 4], (u, p)
+
+
 def test_penalties():
     logits = torch.tensor([[2.0, -2.0, 1.0, 0.5], [1.0, 1.0, 1.0, 1.0]])
     d = logits.to(DEV)

@@ -297,3 +297,13 @@ def test_attention_of_chosen_rows_equals_those_rows_of_the_whole():
     assert torch.allclose(some[[0, 4, 10]], whole[[0, 4, 10]], rtol=0, atol=1e-14) and float(some[[1, 2, 3, 5]].abs().max()) == 0.0
     windowed = plain.causal_attention(q, k, v, 2, window=3)
     assert torch.allclose(plain.causal_attention(q, k, v, 2, window=3, rows=[7])[7], windowed[7], rtol=0, atol=1e-14)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 64])
+def test_uniform_numbers_of_many_rows_are_those_of_single_rows(rows):
+    from arle_amd.sampling.sampler import uniform, uniforms
+
+    seeds = [(-7, 3, 2 ** 64 - 1, 2 ** 70 + 5)[i % 4] + 1000 * i for i in range(rows)]
+    indices = [i * i if i % 3 else 2 ** 40 + i for i in range(rows)]
+    got = uniforms(seeds, indices)
+    assert got.dtype.name == "float32" and got.tolist() == [uniform(s, i) for s, i in zip(seeds, indices)]

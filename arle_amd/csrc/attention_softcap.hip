@@ -384,15 +384,14 @@ extern "C" int arle_wide_norm_store(void* q, long long q_stride, const void* k, 
 }
 
 // ---- matrix-core kernel (bfloat16) ------------------------------------------------------------
-// One wave a work item of sixteen queries that share a kv head: sixteen consecutive rows of one request for one
+// One wave a work item of queries that share a kv head: sixteen or 32 consecutive rows of one request for one
 // q head (prompt portions), or one decoded row for the up to sixteen q heads of a kv head.  The scores are
-// computed transposed, S^T[key][query] = K . Q^T with `v_mfma_f32_16x16x32_bf16`, so that a lane holds, for its
-// query (lane % 16), the keys 4g..4g+3 (g = lane / 16) of each sixteen-key half of a tile of 32 keys: the cap, the
-// penalty, the mask and the running softmax are per-lane arithmetic plus two lane exchanges, and the eight
-// probabilities of a lane are, as they lie, the B operand of the second product O^T += V^T . P^T once the keys of
-// the tile are taken in the order (4g..4g+3 of the first half, 4g..4g+3 of the second) on the V side too, which is
-// two 8-byte loads from the d-major value pages.  A half tile is sixteen slots of one page (page sizes are
-// multiples of 16).  Pages that a window has passed (entry -1) and slots beyond the newest key are never visible;
+// computed transposed, S^T[key][query] = K . Q^T with `v_mfma_f32_16x16x32_bf16`, of a tile of 32 keys in two halves:
+// row r of half h is key 8 (r / 4) + 4 h + r % 4, so that a lane holds, for its query (lane % 16), the keys 8g..8g+7
+// (g = lane / 16): the cap, the penalty, the mask and the running softmax are per-lane arithmetic plus two lane
+// exchanges, and the eight probabilities of a lane are, as they lie, the B operand of the second product
+// O^T += V^T . P^T with one 16-byte load from the d-major value pages on the V side.  Sixteen keys in a row are slots of
+// one page (page sizes are multiples of 16).  Pages that a window has passed (entry -1) and slots beyond the newest key are never visible;
 // their keys are masked by a select and their values replaced by zeros, so that stale bits cannot reach a sum.
 namespace arle {
 
@@ -400,15 +399,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-
-// tanh through one exponential and the hardware's reciprocal (a division in full would be a dozen instructions a score)
-__device__ __forceinline__ float fast_tanh(float x) {
-  return fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __expf(2.0f * x)), 1.0f);
-}
-
-// Portions do not fetch a tile ahead: with thousands of waves, more of them a SIMD hide the loads better than a second
-// set of registers (2,048 rows behind a window of 1,024: 213 us a layer without, 288 with).
-constexpr bool kCapRowsAhead = false;
 
 struct CapArgs {
   const bf16* q; long long q_stride;
@@ -429,26 +419,32 @@ struct CapArgs {
 
 // KC: chunks of 32 of the key size held (Dk <= 32 KC); VC: chunks of 16 of the value size (Dv <= 16 VC).
 // HEADS: a work item is one row (a segment of one row) and the q heads of a kv head, and the WAVES waves of the
-// workgroup take its tiles of keys in turn and add their sums through LDS; else an item is sixteen rows of one q head,
+// workgroup take its tiles of keys in turn and add their sums through LDS; else an item is 16 QB rows of one q head,
 // and the waves of a workgroup are WAVES q heads of one kv head on the same rows, so that they fetch the same tiles.
-// (Portions of heads up to 128 are asked to fit three waves a SIMD: the kernel waits for its loads, and 163 registers
-// hold what 202 held; with larger heads, or four waves, the compiler would spill.)
-template <int KC, int VC, bool HEADS, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(!HEADS && KC <= 4 && VC <= 8 ? 3 : 1)))
+//
+// What bounds portions: every wave fetches its tiles by itself, 16 KB for 32 keys of 128, through its compute unit's
+// cache, and a score costs three quarter-rate instructions (two exponentials and a reciprocal).  So two blocks of sixteen
+// rows share a tile (QB 2, where there are waves enough), values come in pieces of 16 bytes, keys of the next tile are
+// fetched while this one's probabilities are made and values while its scores are, masks are worked out in the tiles at
+// the ends only, sums are rescaled only where a maximum moved, and the lanes' sums meet once at the end.  A layer of 2,048
+// rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 85 now; 256 rows 25 -> 16; eight decoded rows
+// behind 2,048 keys 21 -> 17.  (Portions of heads up to 128 are held to the registers of two waves a SIMD.)
+template <int KC, int VC, bool HEADS, int WAVES, int QB>
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(!HEADS && KC <= 4 && VC <= 8 ? 2 : 1)))
 void attn_softcap_mfma_kernel(const CapArgs a) {
   extern __shared__ float merge_lds[];   // HEADS: [WAVES][n_vc][64 lanes][4], then m [WAVES][16], l [WAVES][16]; then page ids
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, n = lane % 16, g = lane / 16;
   const int group = a.nq / a.nkv;
-  int seg, row, head, kvh, first_row, last_row;
-  bool live;
+  int seg, head, kvh, first_row, last_row, row[QB];
+  bool live[QB];
   if (HEADS) {
     // a kv head with more than sixteen q heads is taken by several workgroups, sixteen q heads each
     const int parts = (group + 15) / 16, part = blockIdx.y % parts;
     seg = blockIdx.x;
     kvh = blockIdx.y / parts;
-    row = first_row = last_row = a.seg_row0[seg];
+    row[0] = first_row = last_row = a.seg_row0[seg];
     head = kvh * group + min(16 * part + n, group - 1);
-    live = 16 * part + n < group;
+    live[0] = 16 * part + n < group;
   } else {
     // Workgroups go to the chip's eight dies in turn (the launch order is blockIdx.x fastest), and every die has a
     // level-two cache of its own: with the head groups a multiple of eight, die i takes the head groups i, i + 8, ...
@@ -459,10 +455,10 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
       by = die + 8 * (within / gridDim.x);
       bx = within % gridDim.x;
     }
-    // the bx-th block of sixteen rows, counted through the segments
+    // the bx-th block of rows, counted through the segments
     int left = bx, found = -1;
     for (int s = 0; s < a.segments; ++s) {
-      const int blocks = (a.seg_row0[s + 1] - a.seg_row0[s] + 15) / 16;
+      const int blocks = (a.seg_row0[s + 1] - a.seg_row0[s] + 16 * QB - 1) / (16 * QB);
       if (left < blocks) {
         found = s;
         break;
@@ -474,23 +470,26 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
     head = by * WAVES + wave;
     kvh = head / group;
     const int end = a.seg_row0[seg + 1];
-    first_row = a.seg_row0[seg] + left * 16;
-    last_row = min(first_row + 15, end - 1);
-    live = first_row + n < end;
-    row = min(first_row + n, end - 1);
+    first_row = a.seg_row0[seg] + left * (16 * QB);
+    last_row = min(first_row + 16 * QB - 1, end - 1);
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      live[b] = first_row + 16 * b + n < end;
+      row[b] = min(first_row + 16 * b + n, end - 1);
+    }
   }
   const int seg_first = a.seg_row0[seg];
-  const int pos = a.seg_start[seg] + (row - seg_first);
+  const int start = a.seg_start[seg];
   // keys that any query of the item sees: from the first row's window to the last row's own position
-  const int pos_lo = a.seg_start[seg] + (first_row - seg_first);
-  const int pos_hi = a.seg_start[seg] + (last_row - seg_first);
+  const int pos_lo = start + (first_row - seg_first);
+  const int pos_hi = start + (last_row - seg_first);
   auto first_seen = [&](int p) {
     int lo = a.window > 0 ? max(0, p - a.window + 1) : 0;
     if (a.chunk > 0) lo = max(lo, p / a.chunk * a.chunk);
     return lo;
   };
   const int key_lo = first_seen(pos_lo);
-  const int my_lo = first_seen(pos);
+  const int all_lo = first_seen(pos_hi);   // every row sees the keys from here to pos_lo
   // The request's first `keep` keys stay visible to rows whose window has passed them.  Their tiles of 32 keys that
   // lie wholly in front of the first tile of the windows are `head_tiles` tiles of their own, walked first; the walk
   // counts tiles through both parts (`walk` 0 .. walk_last), and `tile_of` gives the tile of keys behind a count.
@@ -498,25 +497,36 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
   const int head_tiles = min((keep + 31) / 32, key_lo / 32);
   const int main_first = key_lo / 32;
   auto tile_of = [&](int walk) { return walk < head_tiles ? walk : walk - head_tiles + main_first; };
-  const float sink = a.sink ? load_as_float(a.sink, a.sink_dtype, head) : -INFINITY;
+  // Scores are kept in units of ln 2, so that every exponential is one of base 2.
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float sink = a.sink ? load_as_float(a.sink, a.sink_dtype, head) * kLog2e : -INFINITY;
   const int* table = a.block_table + static_cast<int64_t>(a.seg_slot[seg]) * a.table_stride;
   const float pen1 = a.r1 ? load_as_float(a.r1, a.r_dtype, head) : 0.f;
   const float pen2 = a.r1 ? load_as_float(a.r2, a.r_dtype, head) : 0.f;
-  const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  // cap tanh(x / cap) = cap - 2 cap / (1 + exp(2 x / cap)), x = scale * product
+  const float to_exp = a.cap > 0.f ? 2.0f * kLog2e * a.scale / a.cap : 0.f, cap2 = a.cap * kLog2e, scale2 = a.scale * kLog2e;
   const int n_kc = (a.Dk + 31) / 32, n_vc = a.Dv / 16;
 
   // Q^T operand: for chunk c, Q[row][32 c + 8 g .. + 7]
-  bf16x8_t qreg[KC];
-  const bf16* qr = a.q + static_cast<int64_t>(row) * a.q_stride + head * a.Dk;
+  bf16x8_t qreg[QB][KC];
 #pragma unroll
-  for (int c = 0; c < KC; ++c) {
-    const u32x4_t raw = *reinterpret_cast<const u32x4_t*>(qr + min(32 * c + 8 * g, a.Dk - 8));
-    qreg[c] = __builtin_bit_cast(bf16x8_t, 32 * c + 8 * g < a.Dk ? raw : u32x4_t{0, 0, 0, 0});
+  for (int b = 0; b < QB; ++b) {
+    const bf16* qr = a.q + static_cast<int64_t>(row[b]) * a.q_stride + head * a.Dk;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const u32x4_t raw = *reinterpret_cast<const u32x4_t*>(qr + min(32 * c + 8 * g, a.Dk - 8));
+      qreg[b][c] = __builtin_bit_cast(bf16x8_t, 32 * c + 8 * g < a.Dk ? raw : u32x4_t{0, 0, 0, 0});
+    }
   }
-  f32x4_t acc[VC];
+  f32x4_t acc[QB][VC];
+  float m_run[QB], l_run[QB];   // a row's largest score so far (the same in its four lanes), and this lane's part of its sum
 #pragma unroll
-  for (int c = 0; c < VC; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  for (int b = 0; b < QB; ++b) {
+    m_run[b] = -INFINITY;
+    l_run[b] = 0.f;
+#pragma unroll
+    for (int c = 0; c < VC; ++c) acc[b][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
 
   const int64_t k_page = static_cast<int64_t>(a.nkv) * a.page_size * a.Dk, v_page = static_cast<int64_t>(a.nkv) * a.page_size * a.Dv;
   const int64_t k_head = static_cast<int64_t>(kvh) * a.page_size * a.Dk, v_head = static_cast<int64_t>(kvh) * a.page_size * a.Dv;
@@ -524,8 +534,6 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
   const int tile_first = HEADS ? wave : 0;                                   // counts of the walk
   const int tile_last = head_tiles + pos_hi / 32 - main_first, last_entry = a.table_stride - 1;
 
-  // Every load of a tile (K rows, V columns, after the two page ids) is sent a tile ahead, while the tile before it
-  // is worked through; a tile past the last is the last one again, fetched and dropped.
   // The ids of the pages that the item sees are put into LDS once: a tile's loads then follow no load of a page id,
   // and the reads of LDS are counted apart from the loads from memory, so they disturb no wait for those.
   const int page_first = (key_lo / 32 * 32) / a.page_size;   // the page of the first tile's first key, which may lie in front of key_lo's
@@ -537,116 +545,179 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
   for (int i = threadIdx.x; i <= (pos_hi / 32 * 32 + 31) / a.page_size - page_first; i += WAVES * kWave)
     page_lds[i] = table[min(page_first + i, last_entry)];
   __syncthreads();
-  auto load_tile = [&](int walk, u32x4_t (&kraw)[2][KC], u32x4_t (&vraw)[VC]) {
-    const int at = min(walk, tile_last);
+  // A tile past the last is the last one again, fetched and dropped.  No load stands under a condition (one would make
+  // every later wait a wait for all loads in flight): a piece past the head's size is the head's last piece again, zeroed
+  // or left unused afterwards.
+  // the page (clamped) and the slot in it of key key0 + 16 * high, high given a lane
+  auto place = [&](int at, bool high, int64_t& page, int& in_page) {
     const int key0 = tile_of(at) * 32;
+    const int p0 = key0 / a.page_size, p1 = (key0 + 16) / a.page_size;
+    const int p = high ? p1 : p0;
+    in_page = (high ? key0 + 16 - p1 * a.page_size : key0 - p0 * a.page_size);
+    page = max(at < head_tiles ? head_lds[p] : page_lds[max(p - page_first, 0)], 0);
+  };
+  // Row r of half h of a tile is key 8 (r / 4) + 4 h + r % 4: a lane's scores 4 g .. 4 g + 3 of both halves are then the
+  // keys 8 g .. 8 g + 7, which the value pages hold in one piece of 16 bytes.
+  auto load_keys = [&](int walk, u32x4_t (&kraw)[2][KC]) {
+    int64_t page;
+    int in_page;
+    place(min(walk, tile_last), n >= 8, page, in_page);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const int kb = key0 + 16 * half;
-      const int64_t page = max(at < head_tiles ? head_lds[kb / a.page_size] : page_lds[max(kb / a.page_size - page_first, 0)], 0);
-      const int in_page = kb % a.page_size;
-      const bf16* kr = a.k_pages + page * k_page + k_head + static_cast<int64_t>(in_page + n) * a.Dk;
-      // no load stands under a condition (one would make every later wait a wait for all loads in flight): a piece
-      // past the head's size is the head's last piece again, zeroed or left unused afterwards
+      const bf16* kr = a.k_pages + page * k_page + k_head +
+                       static_cast<int64_t>(in_page + 8 * (n / 4 % 2) + 4 * half + n % 4) * a.Dk;
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         const u32x4_t raw = *reinterpret_cast<const u32x4_t*>(kr + min(32 * c + 8 * g, a.Dk - 8));
         kraw[half][c] = 32 * c + 8 * g < a.Dk ? raw : u32x4_t{0, 0, 0, 0};
       }
+    }
+  };
+  auto load_values = [&](int walk, u32x4_t (&vraw)[VC]) {
+    int64_t page;
+    int in_page;
+    place(min(walk, tile_last), g >= 2, page, in_page);
+    const bf16* vp = a.v_pages + page * v_page + v_head + in_page + 8 * (g % 2);
 #pragma unroll
-      for (int c = 0; c < VC; ++c) {
-        const bf16* vr = a.v_pages + page * v_page + v_head + static_cast<int64_t>(min(16 * c + n, a.Dv - 1)) * a.page_size +
-                         in_page + 4 * g;
-        const u32x2_t two = *reinterpret_cast<const u32x2_t*>(vr);
-        vraw[c][2 * half] = two[0];
-        vraw[c][2 * half + 1] = two[1];
+    for (int c = 0; c < VC; ++c)
+      vraw[c] = *reinterpret_cast<const u32x4_t*>(vp + static_cast<int64_t>(min(16 * c + n, a.Dv - 1)) * a.page_size);
+  };
+
+  // the scores of a tile, capped, penalised and masked: s[b][4 half + i] is key 8 g + 4 half + i of it
+  auto score = [&](int walk, const u32x4_t (&kraw)[2][KC], float (&s)[QB][8]) {
+    const int key0 = tile_of(walk) * 32 + 8 * g;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        // S^T half tile: A = K[the half's sixteen keys][32 c + 8 g ..], B = Q^T
+        f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+          if (c < n_kc) z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kraw[half][c]), qreg[b][c], z, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[b][4 * half + i] = z[i];
+      }
+    }
+    const bool whole = key0 - 8 * g >= all_lo && key0 - 8 * g + 31 <= pos_lo;   // every row sees every key
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      if (a.cap > 0.f) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          s[b][i] = fmaf(-2.0f * cap2, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[b][i] * to_exp)), cap2);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[b][i] *= scale2;
+      }
+      const int pos = start + (row[b] - seg_first);
+      if (a.r1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          s[b][i] -= pen1 * __builtin_amdgcn_logf(1.0f + pen2 * static_cast<float>(pos - key0 - i));
+      }
+      if (!whole) {
+        const int my_lo = first_seen(pos);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          s[b][i] = ((key0 + i >= my_lo || key0 + i < keep) && key0 + i <= pos) ? s[b][i] : -INFINITY;
       }
     }
   };
-
-  auto work_tile = [&](int walk, const u32x4_t (&kraw)[2][KC], const u32x4_t (&vraw)[VC]) {
-    const int key0 = tile_of(walk) * 32;
-    float s[8];
+  // the running maximum and sums, and O^T += V^T . P^T
+  auto gather = [&](int walk, float (&s)[QB][8], const u32x4_t (&vraw)[VC]) {
+    const int key0 = tile_of(walk) * 32 + 8 * g;
+    bf16x8_t pop[QB];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      // S^T half tile: A = K[key kb + n][32 c + 8 g ..], B = Q^T
-      f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < QB; ++b) {
+      float m_new = m_run[b];
 #pragma unroll
-      for (int c = 0; c < KC; ++c)
-        if (c < n_kc) z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kraw[half][c]), qreg[c], z, 0, 0, 0);
+      for (int i = 0; i < 8; ++i) m_new = fmaxf(m_new, s[b][i]);
+      m_new = fmaxf(m_new, __shfl_xor(m_new, 16, kWave));
+      m_new = fmaxf(m_new, __shfl_xor(m_new, 32, kWave));
+      // a query whose window begins behind this tile has seen nothing yet: keep its sums at zero without 0 * inf
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      if (__any(m_new != m_run[b])) {   // later tiles seldom hold a larger score for any of the rows
+        const float alpha = __builtin_amdgcn_exp2f(m_run[b] - m_safe);
+        l_run[b] *= alpha;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = key0 + 16 * half + 4 * g + i;
-        float v = z[i] * a.scale;
-        if (a.cap > 0.f) v = a.cap * fast_tanh(v * inv_cap);
-        if (a.r1) v -= pen1 * __logf(1.0f + pen2 * static_cast<float>(pos - key));
-        s[4 * half + i] = ((key >= my_lo || key < keep) && key <= pos) ? v : -INFINITY;
+        for (int c = 0; c < VC; ++c) {
+          acc[b][c][0] *= alpha; acc[b][c][1] *= alpha; acc[b][c][2] *= alpha; acc[b][c][3] *= alpha;
+        }
+        m_run[b] = m_new;
       }
-    }
-    float m_new = m_run;
+      float p[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) m_new = fmaxf(m_new, s[i]);
-    m_new = fmaxf(m_new, __shfl_xor(m_new, 16, kWave));
-    m_new = fmaxf(m_new, __shfl_xor(m_new, 32, kWave));
-    // a query whose window begins behind this tile has seen nothing yet: keep its sums at zero without 0 * inf
-    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __expf(m_run - m_safe);
-    float p[8], sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      p[i] = __expf(s[i] - m_safe);
-      sum += p[i];
+      for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(s[b][i] - m_safe);
+      l_run[b] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+      u32x4_t pb;
+      pb[0] = pack_bf16x2(p[0], p[1]);
+      pb[1] = pack_bf16x2(p[2], p[3]);
+      pb[2] = pack_bf16x2(p[4], p[5]);
+      pb[3] = pack_bf16x2(p[6], p[7]);
+      pop[b] = __builtin_bit_cast(bf16x8_t, pb);
     }
-    sum += __shfl_xor(sum, 16, kWave);
-    sum += __shfl_xor(sum, 32, kWave);
-    l_run = l_run * alpha + sum;
-    m_run = m_new;
-    u32x4_t pb;
-    pb[0] = pack_bf16x2(p[0], p[1]);
-    pb[1] = pack_bf16x2(p[2], p[3]);
-    pb[2] = pack_bf16x2(p[4], p[5]);
-    pb[3] = pack_bf16x2(p[6], p[7]);
-    const bf16x8_t pop = __builtin_bit_cast(bf16x8_t, pb);
     // which of this lane's eight key slots hold written keys (those between the item's first and last key, and the
     // kept first ones)
-    const bool edge = key0 < key_lo || key0 + 31 > pos_hi;
+    const bool edge = key0 - 8 * g < key_lo || key0 - 8 * g + 31 > pos_hi;
+    u32x4_t written = {~0u, ~0u, ~0u, ~0u};
+    if (edge) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = key0 + j;
+        if ((key < key_lo && key >= keep) || key > pos_hi) written[j / 2] &= (j % 2) ? 0x0000ffffu : 0xffff0000u;
+      }
+    }
 #pragma unroll
     for (int c = 0; c < VC; ++c) {
       if (c < n_vc) {
         u32x4_t vr = vraw[c];
-        if (edge) {
+        if (edge) vr &= written;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int key = key0 + 16 * (j / 4) + 4 * g + j % 4;
-            if ((key < key_lo && key >= keep) || key > pos_hi) vr[j / 2] &= (j % 2) ? 0x0000ffffu : 0xffff0000u;
-          }
-        }
-        f32x4_t o = acc[c];
-        o[0] *= alpha; o[1] *= alpha; o[2] *= alpha; o[3] *= alpha;
-        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vr), pop, o, 0, 0, 0);
+        for (int b = 0; b < QB; ++b)
+          acc[b][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vr), pop[b], acc[b][c], 0, 0, 0);
       }
     }
   };
 
   // (with keys of more than 128 and values of more than 128 a second set of tile registers no longer fits a wave's
   // registers: a decoded row behind 1,024 keys of 256 took 144 us with it)
-  if ((HEADS || kCapRowsAhead) && 2 * KC + VC <= 24) {
+  float sc[QB][8];
+  if (HEADS && 2 * KC + VC <= 24) {
     // a decoded row's waves are few and each walks a chain of tiles: the next tile's loads fly while this one is worked
     u32x4_t k_even[2][KC], v_even[VC], k_odd[2][KC], v_odd[VC];
-    if (tile_first <= tile_last) load_tile(tile_first, k_even, v_even);
+    if (tile_first <= tile_last) {
+      load_keys(tile_first, k_even);
+      load_values(tile_first, v_even);
+    }
     for (int tile = tile_first; tile <= tile_last; tile += 2 * tile_step) {
-      load_tile(tile + tile_step, k_odd, v_odd);
-      work_tile(tile, k_even, v_even);
+      load_keys(tile + tile_step, k_odd);
+      load_values(tile + tile_step, v_odd);
+      score(tile, k_even, sc);
+      gather(tile, sc, v_even);
       if (tile + tile_step > tile_last) break;
-      load_tile(tile + 2 * tile_step, k_even, v_even);
-      work_tile(tile + tile_step, k_odd, v_odd);
+      load_keys(tile + 2 * tile_step, k_even);
+      load_values(tile + 2 * tile_step, v_even);
+      score(tile + tile_step, k_odd, sc);
+      gather(tile + tile_step, sc, v_odd);
     }
-  } else {
+  } else if (tile_first <= tile_last) {
+    // the keys' registers are free once the scores are there, the values' once they are added: each then takes the next
+    // tile's, which fly while the other half of the work is done
     u32x4_t k_now[2][KC], v_now[VC];
+    load_keys(tile_first, k_now);
+    load_values(tile_first, v_now);
     for (int tile = tile_first; tile <= tile_last; tile += tile_step) {
-      load_tile(tile, k_now, v_now);
-      work_tile(tile, k_now, v_now);
+      score(tile, k_now, sc);
+      load_keys(tile + tile_step, k_now);
+      gather(tile, sc, v_now);
+      load_values(tile + tile_step, v_now);
     }
+  }
+#pragma unroll
+  for (int b = 0; b < QB; ++b) {   // a row's sum: its four lanes' parts
+    l_run[b] += __shfl_xor(l_run[b], 16, kWave);
+    l_run[b] += __shfl_xor(l_run[b], 32, kWave);
   }
 
   if (HEADS && WAVES > 1) {
@@ -656,24 +727,24 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
     float* part_l = part_m + WAVES * 16;
 #pragma unroll
     for (int c = 0; c < VC; ++c)
-      if (c < n_vc) part[(wave * n_vc + c) * kWave + lane] = acc[c];
+      if (c < n_vc) part[(wave * n_vc + c) * kWave + lane] = acc[0][c];
     if (g == 0) {
-      part_m[wave * 16 + n] = m_run;
-      part_l[wave * 16 + n] = l_run;
+      part_m[wave * 16 + n] = m_run[0];
+      part_l[wave * 16 + n] = l_run[0];
     }
     __syncthreads();
     float m_all = sink;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) m_all = fmaxf(m_all, part_m[w * 16 + n]);
-    float l_all = a.sink ? __expf(sink - m_all) : 0.f, f[WAVES];
+    float l_all = a.sink ? __builtin_amdgcn_exp2f(sink - m_all) : 0.f, f[WAVES];
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      f[w] = __expf(part_m[w * 16 + n] - m_all);
+      f[w] = __builtin_amdgcn_exp2f(part_m[w * 16 + n] - m_all);
       l_all += part_l[w * 16 + n] * f[w];
     }
-    if (!live) return;
+    if (!live[0]) return;
     const float inv_l = a.out_scale / l_all;
-    bf16* orow = a.out + static_cast<int64_t>(row) * a.o_stride + head * a.Dv;
+    bf16* orow = a.out + static_cast<int64_t>(row[0]) * a.o_stride + head * a.Dv;
     for (int c = wave; c < n_vc; c += WAVES) {
       f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -688,24 +759,31 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
     }
     return;
   }
-  if (!live) return;
-  float inv_l = a.out_scale / l_run;
-  if (a.sink) {
-    const float m_all = fmaxf(m_run, sink), keep = __expf(m_run - m_all);
-    inv_l = keep / (l_run * keep + __expf(sink - m_all)) * a.out_scale;
-  }
-  bf16* orow = a.out + static_cast<int64_t>(row) * a.o_stride + head * a.Dv;
 #pragma unroll
-  for (int c = 0; c < VC; ++c) {
-    if (c < n_vc) {
-      u32x2_t packed;
-      packed[0] = pack_bf16x2(acc[c][0] * inv_l, acc[c][1] * inv_l);
-      packed[1] = pack_bf16x2(acc[c][2] * inv_l, acc[c][3] * inv_l);
-      *reinterpret_cast<u32x2_t*>(orow + 16 * c + 4 * g) = packed;
+  for (int b = 0; b < QB; ++b) {
+    if (!live[b]) continue;
+    float inv_l = a.out_scale / l_run[b];
+    if (a.sink) {
+      const float m_all = fmaxf(m_run[b], sink), kept = __builtin_amdgcn_exp2f(m_run[b] - m_all);
+      inv_l = kept / (l_run[b] * kept + __builtin_amdgcn_exp2f(sink - m_all)) * a.out_scale;
+    }
+    bf16* orow = a.out + static_cast<int64_t>(row[b]) * a.o_stride + head * a.Dv;
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      if (c < n_vc) {
+        u32x2_t packed;
+        packed[0] = pack_bf16x2(acc[b][c][0] * inv_l, acc[b][c][1] * inv_l);
+        packed[1] = pack_bf16x2(acc[b][c][2] * inv_l, acc[b][c][3] * inv_l);
+        *reinterpret_cast<u32x2_t*>(orow + 16 * c + 4 * g) = packed;
+      }
     }
   }
 }
 
+// Waves of 32 rows from which a prompt portion takes them rather than waves of 16: with fewer, more waves fill the chip
+// better than fewer loads help (32 q heads of 128, window 1,024, 16 against 32 rows a wave: 512 rows, 544 such waves, 25
+// and 34 us; 1,024 rows, 1,056 waves, 62 and 59; four portions of 300 rows 33 and 31; 2,048 rows 136 and 85).
+constexpr long long kCapTwoBlocks = 1024;
 constexpr int kCapSplitWaves = 8;   // waves that share the keys of a decoded row
 constexpr int kCapLdsMost = 160 * 1024;   // LDS of a gfx950 compute unit: no workgroup can ask for more
 
@@ -761,6 +839,19 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
   const int head_waves = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);   // q heads of one kv head that share a workgroup
   const size_t merge_bytes = static_cast<size_t>(kCapSplitWaves) * ((Dv / 16) * kWave * 4 + 32) * sizeof(float) + page_bytes;
   if (heads_mode && merge_bytes > static_cast<size_t>(cap_lds_limit())) return static_cast<int>(hipErrorInvalidValue);
+  const int wide_blocks = (row_blocks - segments) / 2 + segments;   // as row_blocks, of 32 rows
+  const bool two = Dk <= 128 && Dv <= 128 && static_cast<long long>(wide_blocks) * nq >= kCapTwoBlocks &&
+                   page_bytes + 2 * sizeof(int) <= 48 * 1024;
+#define ARLE_CAP_ROWS(KC, VC, QB, BLOCKS, BYTES)                                                                   \
+  do {                                                                                                             \
+    constexpr int kQb = KC <= 4 && VC <= 8 ? QB : 1;                                                               \
+    if (head_waves == 4)                                                                                           \
+      attn_softcap_mfma_kernel<KC, VC, false, 4, kQb><<<dim3(BLOCKS, nq / 4), 4 * kWave, BYTES, s>>>(a);           \
+    else if (head_waves == 2)                                                                                      \
+      attn_softcap_mfma_kernel<KC, VC, false, 2, kQb><<<dim3(BLOCKS, nq / 2), 2 * kWave, BYTES, s>>>(a);           \
+    else                                                                                                           \
+      attn_softcap_mfma_kernel<KC, VC, false, 1, kQb><<<dim3(BLOCKS, nq), kWave, BYTES, s>>>(a);                   \
+  } while (0)
 #define ARLE_CAP(KC, VC)                                                                                           \
   do {                                                                                                             \
     if (heads_mode) {                                                                                              \
@@ -768,20 +859,18 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
       if (!raised && merge_bytes > 48 * 1024) {                                                                    \
         const int most = kCapSplitWaves * (VC * kWave * 4 + 32) * 4 + 48 * 1024;                                   \
         const hipError_t e = hipFuncSetAttribute(                                                                  \
-            reinterpret_cast<const void*>(&attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves>),                \
+            reinterpret_cast<const void*>(&attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves, 1>),                \
             hipFuncAttributeMaxDynamicSharedMemorySize, most < cap_lds_limit() ? most : cap_lds_limit());              \
         if (e != hipSuccess) return static_cast<int>(e);                                                           \
         raised = true;                                                                                             \
       }                                                                                                            \
-      attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves>                                                       \
+      attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves, 1>                                                    \
           <<<dim3(segments, nkv * ((group + 15) / 16)), kCapSplitWaves * kWave, merge_bytes, s>>>(a);                                    \
     }                                                                                                              \
-    else if (head_waves == 4)                                                                                      \
-      attn_softcap_mfma_kernel<KC, VC, false, 4><<<dim3(row_blocks, nq / 4), 4 * kWave, page_bytes, s>>>(a);                \
-    else if (head_waves == 2)                                                                                      \
-      attn_softcap_mfma_kernel<KC, VC, false, 2><<<dim3(row_blocks, nq / 2), 2 * kWave, page_bytes, s>>>(a);                \
+    else if (two)                                                                                                  \
+      ARLE_CAP_ROWS(KC, VC, 2, wide_blocks, page_bytes + 2 * sizeof(int));                                         \
     else                                                                                                           \
-      attn_softcap_mfma_kernel<KC, VC, false, 1><<<dim3(row_blocks, nq), kWave, page_bytes, s>>>(a);                        \
+      ARLE_CAP_ROWS(KC, VC, 1, row_blocks, page_bytes);                                                            \
   } while (0)
   if (size <= 64) {
     ARLE_CAP(4, 4);
@@ -795,5 +884,6 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
     ARLE_CAP(8, 16);
   }
 #undef ARLE_CAP
+#undef ARLE_CAP_ROWS
   return launch_status();
 }

@@ -1899,7 +1899,7 @@ def attn_softcap_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot,
                       num_q_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, page_size: int, scale: float,
                       softcap: float = 0.0, r1=None, r2=None, window: int = 0, chunk: int = 0, sink=None,
                       keep_first: int = 0, out_scale: float = 1.0):
-    """`attn_softcap_simt` on the matrix cores, bfloat16: sixteen rows of a segment a wave, or (when every segment is
+    """`attn_softcap_simt` on the matrix cores, bfloat16: sixteen or 32 rows of a segment a wave, or (when every segment is
     one decoded row) one row's q heads of a kv head, sixteen at a time, a wave.  keep_first (with a window and no
     chunks): the request's first so many keys stay visible to rows whose window has passed them."""
     _need(keep_first >= 0 and (keep_first == 0 or (window > 0 and chunk == 0)),

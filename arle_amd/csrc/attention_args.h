@@ -31,9 +31,9 @@ struct AttnArgs {
   const float* sink;   // [q heads] or null: exp(sink_h) joins the softmax's denominator, with no value behind it
   float out_scale;     // a factor on the output, in 32 bits
   int splits;
-  int segments;        // PREP with splits: how many segments share the segments * splits waves of a kv head
+  int segments;        // PREP with splits: how many segments share the waves of a kv head (gridDim.z of them)
   int* ws_plan;        // PREP with splits: [segments][2] a segment's first wave and its number of waves, then
-                       // [segments * splits][8] every wave's DecodeShare
+                       // [waves][8] every wave's DecodeShare
   int plan_made;       // the plan is there already (an earlier layer of the same step made it); 0: this launch makes it
   int ws_rows;   // token rows that the split-KV workspace holds for a segment
   int portion_splits;  // parts into which the LDS kernel cuts the keys of a row block (1: whole; it writes out)

@@ -463,8 +463,8 @@ static int compute_units() {
 // must already hold) and take part in the attention from registers.  With splits > 1 there are `waves` waves a
 // kv head (at least one a segment; 0: segments * splits, or splits a segment in a workgroup of its own), over which the
 // segments' keys are shared out (ws_o [waves][nq][D], ws_ml [waves][nq][2]; ws_plan int32 [2 segments + 8 waves],
-// 8-byte aligned, is written by a call with plan_made 0 and read by later calls of the same step, segments, window and
-// waves with plan_made 1).  D 64 or 128, nq / nkv <= 16; everything else
+// 8-byte aligned, is written by a call with waves > 0 and plan_made 0 and read by later calls of the same step, segments,
+// window and waves with plan_made 1; without `waves` it is scratch of the call, which may leave it unwritten).  D 64 or 128, nq / nkv <= 16; everything else
 // as arle_attn_paged_mfma with max_qlen 1.  The same results as arle_qk_prep followed by arle_attn_paged_mfma but
 // for the order in which a head's squares are added for its norm.
 extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_parts, long long part_stride, long long row_stride,
@@ -522,7 +522,7 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
   }
   a.segments = segments;
   a.ws_plan = splits > 1 ? ws_plan : nullptr;
-  a.plan_made = plan_made;
+  a.plan_made = spread && plan_made;
   const dim3 grid(1, nkv, static_cast<unsigned>(z));
   if (D == 128 && parts_bf16)
     attn_mfma_kernel<1, 128, true, true, false, true><<<grid, kWave, 0, s>>>(a);

@@ -498,9 +498,9 @@ def attn_decode_prep(parts, out, k_pages, v_pages, block_table, seg_row0, seg_sl
     with the new token's does the same for the k head, writes key and value into the cache and uses them from its
     registers.  out: bfloat16 [T, nq*D].
     total_kv_len: the contexts' lengths together, by which ragged ones are told from equal ones (decode_share).
-    carry: a dictionary that lives for one pass over the layers.  Where the requests' keys are shared out over all waves of
-    a kv head, the first layer works out how, and the later ones of the pass with as many waves and the same window find
-    it there."""
+    carry: a dictionary that lives for one pass over the layers.  Where decode_share has the requests' keys shared out over all
+    waves of a kv head, the first layer works out how, and the later ones of the pass with as many waves and the same
+    window find it there."""
     _gpu(parts, out, k_pages, v_pages, block_table, seg_row0, seg_slot, seg_start, q_weight, k_weight, cos, sin)
     group = num_q_heads // max(num_kv_heads, 1)
     width = (num_q_heads + 2 * num_kv_heads) * head_dim
@@ -552,13 +552,14 @@ def attn_decode_prep(parts, out, k_pages, v_pages, block_table, seg_row0, seg_sl
     if splits > 1:
         ws_o = torch.empty((held, num_q_heads, head_dim), dtype=torch.float32, device=out.device)
         ws_ml = torch.empty((held, num_q_heads, 2), dtype=torch.float32, device=out.device)
-        key = ("decode_share", segments, int(held), int(window))
-        plan = carry.get(key) if carry is not None else None
-        plan_made = plan is not None
+        # Only a launch that is given its number of waves is sure to write the plan (one with splits of its own may keep them
+        # inside a workgroup), so only such launches leave theirs to the pass.
+        kept = carry if waves and carry is not None else {}
+        key = ("decode_share", segments, int(waves), int(window))
+        plan_made = key in kept
         if not plan_made:
-            plan = torch.empty((2 * segments + 8 * held,), dtype=torch.int32, device=out.device)
-            if carry is not None:
-                carry[key] = plan
+            kept[key] = torch.empty((2 * segments + 8 * held,), dtype=torch.int32, device=out.device)
+        plan = kept[key]
     lib.call("arle_attn_decode_prep", parts.data_ptr(), int(whole), n_parts, part_stride, row_stride, _ptr(q_weight),
              _ptr(k_weight), w_f32, _ptr(cos), _ptr(sin), int(rotary_dim), float(eps), out.data_ptr(), out.stride(0),
              k_pages.data_ptr(), v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], seg_row0.data_ptr(),

@@ -19,7 +19,9 @@
 //
 // Measured on MI355X, 2,048 rows, 20 heads, D = Dv = 128, us a layer: 5 + 86 + 61 where the token-by-token kernels take 125
 // (gates) + 708 (memory) + 18 (output); the error of a layer's output against 64 bits is the same (2e-7 to 6e-6 either way).
-// A NaN or an infinity in a row's v reaches the earlier rows of its own chunk too (a weight of zero times it).
+// A NaN or an infinity in a row's v spoils that row and the later ones, as token by token (where an infinity meets a
+// state's column with both signs).  The second product would carry it to the chunk's earlier rows too, as a weight of zero
+// times it: it takes zeros for such values, and the rows from the first one on are made NaN behind it.
 #include "chunks.h"
 #include "common.h"
 
@@ -317,11 +319,26 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[t][r] *= inter[32 * t + 8 * (r / 4) + 4 * half + r % 4];
     const float* p0 = k_lds + i * kPPitch + half;
+    float check = 0.f;        // NaN as soon as a value is no finite number
+#pragma unroll
+    for (int j = 0; j < 32; ++j) check = fmaf(vr[j], 0.f, check);
+    int spoilt = kChunkRows;  // the first row of this column that holds such a value
+    if (__any(check != 0.f)) {
+#pragma unroll
+      for (int j = 31; j >= 0; --j)
+        if (!__builtin_isfinite(vr[j])) spoilt = 2 * j + half, vr[j] = 0.f;
+      spoilt = min(spoilt, __shfl_xor(spoilt, 32, kWave));
+    }
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
       if (j < 16) acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(p0[2 * j], vr[j], acc[0], 0, 0, 0);
       acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(p0[32 * kPPitch + 2 * j], vr[j], acc[1], 0, 0, 0);
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * t + 8 * (r / 4) + 4 * half + r % 4 >= spoilt) acc[t][r] = __builtin_nanf("");
   }
   __syncthreads();   // q has been read
   if (has_cols) {

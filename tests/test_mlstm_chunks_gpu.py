@@ -65,3 +65,29 @@ def test_chunks_give_the_recurrence(lengths, H, D, Dv, gate_std):
                                     15.0, *plain, c["row0"], c["slot"], heads=H, key_dim=D, value_dim=Dv)
     by_row = ops.mlstm_output(num, nq, coefs, c["qkvg"][:, 2 * a + b:], c["weight"], 1e-6, torch.float32, heads=H, value_dim=Dv)
     assert _rel(by_row, want) < 2e-5
+
+
+@pytest.mark.parametrize("lengths,D,Dv,bad", [([64], 128, 128, 63), ([130], 64, 96, 31), ([100, 70], 32, 64, 99), ([100, 70], 96, 32, 133),
+                                              ([129], 128, 128, 128)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+def test_a_value_that_is_no_number_reaches_its_row_and_later_ones_only(lengths, D, Dv, bad, value):
+    """One entry of one head's v: the rows in front of it, the other requests and the other heads keep their bits, and the
+    rows from it on hold no number where the token-by-token kernels hold none."""
+    from arle_amd.kernels import ops
+
+    H, T = 2, sum(lengths)
+    c = _case(lengths, H, D, Dv, 1.0, 3 + bad)
+    qk, vw = H * D, H * Dv
+    spoilt = c["qkvg"].clone()
+    spoilt[bad, 2 * qk + Dv + Dv // 2 + 1] = value       # head 1
+    chunks = lambda p: ops.mlstm_chunks(p, c["gates"], c["bi"], c["bf"], 15.0, *[t.clone() for t in c["state"]], c["row0"], c["slot"],
+                                        c["weight"], 1e-6, torch.float32, heads=H, key_dim=D, value_dim=Dv)
+    clean, got = chunks(c["qkvg"]), chunks(spoilt)
+    num, nq, coefs = ops.mlstm_scan(spoilt[:, :qk], spoilt[:, qk:2 * qk], spoilt[:, 2 * qk:2 * qk + vw], c["gates"], c["bi"], c["bf"], 15.0,
+                                    *[t.clone() for t in c["state"]], c["row0"], c["slot"], heads=H, key_dim=D, value_dim=Dv)
+    by_row = ops.mlstm_output(num, nq, coefs, spoilt[:, 2 * qk + vw:], c["weight"], 1e-6, torch.float32, heads=H, value_dim=Dv)
+    end = next(int(e) for e in c["row0"].tolist()[1:] if e > bad)
+    reached = torch.zeros(T, vw, dtype=torch.bool, device="cuda")
+    reached[bad:end, Dv:] = True
+    assert torch.equal(got[~reached], clean[~reached]) and torch.isfinite(clean).all()
+    assert torch.equal(torch.isfinite(by_row), torch.isfinite(got))

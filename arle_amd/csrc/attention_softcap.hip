@@ -427,7 +427,7 @@ struct CapArgs {
 // rows share a tile (QB 2, where there are waves enough), values come in pieces of 16 bytes, keys of the next tile are
 // fetched while this one's probabilities are made and values while its scores are, masks are worked out in the tiles at
 // the ends only, sums are rescaled only where a maximum moved, and the lanes' sums meet once at the end.  A layer of 2,048
-// rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 85 now; 256 rows 25 -> 16; eight decoded rows
+// rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 89 now; 256 rows 25 -> 16; eight decoded rows
 // behind 2,048 keys 21 -> 17.  (Portions of heads up to 128 are held to the registers of two waves a SIMD.)
 template <int KC, int VC, bool HEADS, int WAVES, int QB>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(!HEADS && KC <= 4 && VC <= 8 ? 2 : 1)))
@@ -657,25 +657,28 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
       pb[3] = pack_bf16x2(p[6], p[7]);
       pop[b] = __builtin_bit_cast(bf16x8_t, pb);
     }
-    // which of this lane's eight key slots hold written keys (those between the item's first and last key, and the
-    // kept first ones)
-    const bool edge = key0 - 8 * g < key_lo || key0 - 8 * g + 31 > pos_hi;
-    u32x4_t written = {~0u, ~0u, ~0u, ~0u};
-    if (edge) {
+    // In the tiles at the ends, which of this lane's eight key slots hold keys that a block of sixteen rows sees (those
+    // between its first row's first and its last row's last key, and the kept first ones): the values of the others enter
+    // its sums as zeros, so that what is in a slot never written, or a NaN that only the other block sees, stays out of them.
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = key0 + j;
-        if ((key < key_lo && key >= keep) || key > pos_hi) written[j / 2] &= (j % 2) ? 0x0000ffffu : 0xffff0000u;
+    for (int b = 0; b < QB; ++b) {
+      const int lo = b == 0 ? key_lo : first_seen(pos_lo + 16 * b), hi = QB == 1 ? pos_hi : min(pos_lo + 16 * b + 15, pos_hi);
+      const bool edge = key0 - 8 * g < lo || key0 - 8 * g + 31 > hi;
+      u32x4_t seen = {~0u, ~0u, ~0u, ~0u};
+      if (edge) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = key0 + j;
+          if ((key < lo && key >= keep) || key > hi) seen[j / 2] &= (j % 2) ? 0x0000ffffu : 0xffff0000u;
+        }
       }
-    }
 #pragma unroll
-    for (int c = 0; c < VC; ++c) {
-      if (c < n_vc) {
-        u32x4_t vr = vraw[c];
-        if (edge) vr &= written;
-#pragma unroll
-        for (int b = 0; b < QB; ++b)
+      for (int c = 0; c < VC; ++c) {
+        if (c < n_vc) {
+          u32x4_t vr = vraw[c];
+          if (edge) vr &= seen;
           acc[b][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vr), pop[b], acc[b][c], 0, 0, 0);
+        }
       }
     }
   };
@@ -781,8 +784,9 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
 }
 
 // Waves of 32 rows from which a prompt portion takes them rather than waves of 16: with fewer, more waves fill the chip
-// better than fewer loads help (32 q heads of 128, window 1,024, 16 against 32 rows a wave: 512 rows, 544 such waves, 25
-// and 34 us; 1,024 rows, 1,056 waves, 62 and 59; four portions of 300 rows 33 and 31; 2,048 rows 136 and 85).
+// better than fewer loads help (32 q heads of 128, window 1,024, 16 against 32 rows a wave: 640 rows, 672 such waves, 36
+// and 45 us; 1,024 rows, 1,056 waves, 62 and 64; 1,150 rows 72 and 73; 1,250 rows 81 and 74; four portions of 300 rows 33
+// and 32; 2,048 rows 136 and 89).
 constexpr long long kCapTwoBlocks = 1024;
 constexpr int kCapSplitWaves = 8;   // waves that share the keys of a decoded row
 constexpr int kCapLdsMost = 160 * 1024;   // LDS of a gfx950 compute unit: no workgroup can ask for more

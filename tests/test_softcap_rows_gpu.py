@@ -88,3 +88,38 @@ def test_rows_in_blocks_of_32_match_64_bit_attention(case):
             # bits, so half a unit of the last is up to 2^-8 of the number; 32-bit scores (errors of 1e-5) add less than a tenth
             bound = 2.0 ** -8 * 1.1 * (of_abs + want.abs()) + 1e-6
             assert ((got[rows, h] - want).abs() <= bound).all(), (i, h)
+
+
+@pytest.mark.parametrize("rows,context,window,keep,nq,bad", [(96, 20, 0, 0, 512, 20 + 17), (96, 20, 40, 0, 512, 20 + 47), (96, 20, 40, 0, 512, 3),
+                                                             (70, 0, 33, 0, 512, 31), (96, 70, 40, 5, 512, 3), (96, 20, 40, 0, 8, 20 + 47)])
+def test_a_value_that_is_no_number_stays_in_the_blocks_of_sixteen_rows_that_see_it(rows, context, window, keep, nq, bad):
+    """The key's blocks of sixteen rows (counted from the portion's first) may all become NaN; every other block keeps its bits,
+    with 32 rows a wave (the first five cases) as with sixteen."""
+    from arle_amd.kernels import ops
+
+    nkv, D, page = 8, 32, 16
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    pages = -(-(rows + context) // page)
+    q, k, v = rnd(rows, nq * D), rnd(pages, nkv, page, D), rnd(pages, nkv, D, page)
+    i32 = lambda values: torch.tensor(values, dtype=torch.int32, device=DEV)
+
+    def run(v_pages):
+        out = torch.empty(rows, nq * D, dtype=torch.bfloat16, device=DEV)
+        ops.attn_softcap_mfma(q, out, k, v_pages, i32([list(range(pages))]), i32([0, rows]), i32([0]), i32([context]), max_qlen=rows,
+                              num_q_heads=nq, num_kv_heads=nkv, key_dim=D, value_dim=D, page_size=page, scale=D ** -0.5, softcap=30.0,
+                              window=window, keep_first=keep)
+        return out
+
+    spoilt = v.clone()
+    spoilt[bad // page, :, :, bad % page] = float("nan")
+    clean, got = run(v), run(spoilt)
+    assert torch.isfinite(clean).all()
+    for first in range(0, rows, 16):
+        at = range(context + first, context + min(first + 16, rows))
+        sees = any(bad <= p and (not window or p - bad < window or bad < keep) for p in at)
+        block = slice(first, first + 16)
+        assert torch.equal(got[block], clean[block]) or sees, first
+        for p in at:
+            if bad <= p and (not window or p - bad < window or bad < keep):
+                assert torch.isnan(got[p - context]).all(), p

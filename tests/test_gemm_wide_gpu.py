@@ -77,3 +77,44 @@ def test_what_it_does_not_take_goes_elsewhere():
     want = (x.double() @ w.double().T).view(100, -1, 2, 16)
     want = (torch.nn.functional.silu(want[:, :, 0]) * want[:, :, 1]).reshape(100, -1)
     assert _rel(ops.gate_up_act(x, w), want) < 2e-2
+
+
+@pytest.mark.parametrize("base,shape", [(-76, (128, 64)), (-50, (256, 320)), (-24, (128, 192)), (-9, (128, 320)), (2, (192, 320))])
+def test_the_activation_keeps_the_error_of_a_whole_exponential_and_division(base, shape):
+    """Gates that a float holds exactly, base + i / 1,024 up to base + 15.8, and ups of 1: the result is silu rounded to
+    bfloat16, and it rounds the other way than the 64-bit silu where that lies within the 32-bit error of a middle between
+    two bfloat16 numbers.  An error of e ulp in the mean does so for a share of e 2^-16 to 2 e 2^-16 of the values; expf and
+    a division have 0.3 to 0.45 (1.4e-5 at most), the exponential and the reciprocal of the vector unit 3 to 15 below -5."""
+    from arle_amd.kernels import ops
+
+    rows, n = 128, 8192
+    x = torch.zeros(rows, 64, device="cuda")
+    x[:, 0], x[:, 1] = 1.0, torch.arange(rows, device="cuda") % 128
+    w = torch.zeros(n // 32, 2, 16, 64, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(4)
+    w[:, 0, :, 0] = base
+    w[:, 0, :, 1] = torch.randint(0, 128, (n // 32, 16), device="cuda", generator=g) / 1024
+    w[:, 1, :, 0] = 1.0
+    x, w = x.bfloat16(), w.reshape(n, 64).bfloat16()
+    gate = (x.double() @ w.view(n // 32, 2, 16, 64)[:, 0].reshape(-1, 64).double().T)
+    want = (gate / (1 + torch.exp(-gate))).bfloat16()
+    got = ops.gemm_wide(x, w, epilogue=ops.EPI_SILU_MUL, shape=shape)
+    assert float((got != want).double().mean()) < 4e-5
+
+
+def test_the_activation_below_where_the_reciprocal_leaves_the_floats():
+    """exp(-x) from 2^126 on: the reciprocal of 1 + exp(-x) is no normal number, the result is one."""
+    from arle_amd.kernels import ops
+
+    gates = torch.tensor([-79.5, -80.0, -80.5, -87.0, -87.5, -88.0, -88.5, -100.0, 79.5, 80.0, 88.5, 3e38, float("inf"), float("nan"), 1.0, -1.0])
+    x = torch.zeros(3, 64, dtype=torch.bfloat16, device="cuda")
+    x[:, 0] = 1.0
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device="cuda")
+    w[:16, 0], w[16:, 0] = gates.bfloat16().cuda(), 2.0
+    got = ops.gemm_wide(x, w, epilogue=ops.EPI_SILU_MUL).float().cpu()
+    exact = gates.bfloat16().double()
+    want = (exact / (1 + torch.exp(-exact)) * 2).float()
+    for row in got:
+        assert torch.isnan(row[13]) and float(row[12]) == float("inf")
+        keep = [i for i in range(16) if i not in (11, 12, 13)]
+        assert torch.allclose(row[keep], want[keep], rtol=2.0 ** -8, atol=1e-38) and float(row[11]) == float("inf")

@@ -1705,16 +1705,34 @@ def mlstm_scan(q, k, v, gates, bias_i, bias_f, cap: float, s_state, n_state, m_s
     return num, nq, coefs
 
 
-# Rows of the longest segment from which a step's rows go through the matrix memory in chunks of 64.  A layer of the Gufasun
-# design at the Qwen3-4B widths (20 heads of 128 x 128) on MI355X, us, token by token / in chunks: one prompt
-# of 64 rows 45 / 32, 96 53 / 35, 128 66 / 35, 512 225 / 55, 2,048 860 / 155; 128 rows beside 16 single ones 97 / 69.
+# Rows of the longest segment from which a step's rows may go through the matrix memory in chunks of 64.  A layer of the
+# Gufasun design at the Qwen3-4B widths (20 heads of 128 x 128) on MI355X, us, token by token / in chunks: one prompt
+# of 64 rows 45 / 32, 96 53 / 35, 128 66 / 35, 512 225 / 55, 2,048 860 / 155.
 MLSTM_CHUNK_MIN_ROWS = 96
 
 
-def mlstm_chunks_supported(longest: int, key_dim: int, value_dim: int) -> bool:
-    """Whether mlstm_chunks takes heads of these sizes, and pays for segments of up to `longest` rows."""
-    return (longest >= MLSTM_CHUNK_MIN_ROWS and key_dim % 32 == 0 and value_dim % 32 == 0 and 32 <= key_dim <= 128
-            and 32 <= value_dim <= 128)
+def mlstm_chunks_supported(key_dim: int, value_dim: int) -> bool:
+    """Whether mlstm_chunks takes heads of these sizes."""
+    return key_dim % 32 == 0 and value_dim % 32 == 0 and 32 <= key_dim <= 128 and 32 <= value_dim <= 128
+
+
+def mlstm_chunks_preferred(longest: int, tokens: int, segments: int, heads: int, key_dim: int, value_dim: int) -> bool:
+    """Whether a step's rows go in chunks: where the estimate of their time is below that of the token-by-token kernels.
+
+    Token by token a step lasts as long as its longest segment's chain of rows or as all rows' arithmetic, and every
+    segment's state is read and written once; in chunks the longest segment's chain is short, but every segment, a decoded
+    row too, is a chunk of its own whose state is written and read once more, and every workgroup counts through the
+    segments.  The figures are a layer's on MI355X, heads of 20 x 128 x 128, 8 x 64 x 64 and 4 x 128 x 128.  One portion
+    beside decoded rows, 20 heads of 128, us, token by token / in chunks: 96 rows and 16 84 / 69, and 32 112 / 126,
+    and 256 502 / 1,331; 512 and 64 352 / 252, and 128 468 / 557; 2,048 and 128 1,168 / 679, and 256 1,452 / 1,521; 64
+    portions of 100 rows 1,078 / 412."""
+    if longest < MLSTM_CHUNK_MIN_ROWS or not mlstm_chunks_supported(key_dim, value_dim):
+        return False
+    size = heads * key_dim * value_dim / (20 * 128 * 128)      # of a state, against the one that the figures are for
+    by_rows = 10 + max(0.41 * longest, 0.165 * size * tokens) + 1.7 * size * segments
+    by_chunks = (30 + 0.058 * longest + max(2.1 * size, 0.3) * _chunk_items(tokens, segments)
+                 + (0.002 + 0.009 * size) * segments * segments)
+    return by_chunks < by_rows
 
 
 def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_state, seg_row0, seg_slot, weight, eps: float,
@@ -1727,7 +1745,7 @@ def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_st
     tokens, width = qkvg.shape[0], H * Dv
     _need(qkvg.dtype == torch.float32 and qkvg.shape[1] == 2 * H * (D + Dv) and qkvg.stride(0) % 4 == 0 and qkvg.data_ptr() % 16 == 0,
           "qkvg must be float32 [T, 2 H (D + Dv)] with 16-byte aligned rows")
-    _need(mlstm_chunks_supported(MLSTM_CHUNK_MIN_ROWS, D, Dv), "mlstm_chunks takes heads of multiples of 32 up to 128")
+    _need(mlstm_chunks_supported(D, Dv), "mlstm_chunks takes heads of multiples of 32 up to 128")
     _rows(gates, "gates")
     _need(gates.dtype == torch.float32 and gates.shape == (tokens, 2 * H), "gates must be float32 [T, 2 * heads]")
     _need(bias_i.shape == (H,) and bias_f.shape == (H,) and bias_i.dtype == bias_f.dtype == torch.float32

@@ -12,8 +12,9 @@ Per token, with h the mixer's input, H heads, key size D, value size Dv:
 S, n and m start at zero and live in 32-bit state slots `[H, D, Dv]`, `[H, D]`, `[H]` of the request; the gates'
 projections, the gates, the recurrence and the head norm are 32-bit in every mode.  q, k, v and the output gate
 come from one fused product that hands over its 32-bit sums; the two gate projections are a product of their own.
-In float32 mode, and for steps of short segments, the rows go one by one, so that a row's bits do not depend on how its
-request was cut; in bfloat16 mode portions go in chunks of 64 rows, in 32-bit products all the same.
+In float32 mode the rows go one by one, so that a row's bits do not depend on how its request was cut; in bfloat16 mode
+the rows of steps with a long portion go in chunks of 64 where that is faster (`ops.mlstm_chunks_preferred`), in 32-bit
+products all the same.
 """
 from __future__ import annotations
 
@@ -86,7 +87,7 @@ class MLSTMMixer(Part):
         # on a single one), and what rounding them to bfloat16 costs there is ten times a usual row's error
         p = self.qkvg(x, out_dtype=torch.float32)
         gates = self.gates(x, out_dtype=torch.float32)[:, :2 * self.H]
-        if not self.rt.is_f32 and ops.mlstm_chunks_supported(batch.max_qlen, self.D, self.Dv):
+        if not self.rt.is_f32 and ops.mlstm_chunks_preferred(batch.max_qlen, x.shape[0], batch.seg_slot.numel(), self.H, self.D, self.Dv):
             y = ops.mlstm_chunks(p, gates, self.i_bias, self.f_bias, self.cap, cache["S"].state, cache["n"].state, cache["m"].state,
                                  batch.seg_row0, batch.seg_slot, self.norm, self.eps, self.rt.act_dtype, heads=self.H,
                                  key_dim=self.D, value_dim=self.Dv)

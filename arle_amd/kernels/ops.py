@@ -1728,6 +1728,8 @@ def mlstm_chunks_preferred(longest: int, tokens: int, segments: int, heads: int,
     portions of 100 rows 1,078 / 412."""
     if longest < MLSTM_CHUNK_MIN_ROWS or not mlstm_chunks_supported(key_dim, value_dim):
         return False
+    if _chunk_items(tokens, segments) * heads * key_dim * value_dim * 4 > _DECAY_WORK_BYTES:
+        return False        # the state in front of every chunk is kept; token by token a step needs less memory
     size = heads * key_dim * value_dim / (20 * 128 * 128)      # of a state, against the one that the figures are for
     by_rows = 10 + max(0.41 * longest, 0.165 * size * tokens) + 1.7 * size * segments
     by_chunks = (30 + 0.058 * longest + max(2.1 * size, 0.3) * _chunk_items(tokens, segments)

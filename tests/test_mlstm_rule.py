@@ -34,3 +34,10 @@ def test_decoded_rows_and_other_head_sizes_go_row_by_row():
     assert not ops.mlstm_chunks_preferred(95, 95, 1, 20, 128, 128)
     for sizes in ((48, 64), (64, 160), (130, 70)):
         assert not ops.mlstm_chunks_preferred(2048, 2048, 1, 20, *sizes)
+
+
+def test_a_step_whose_chunks_would_not_fit_the_workspace_goes_row_by_row():
+    """20 heads of 128 x 128: a state of 1.31 MB a chunk, so 4 GiB are 3,276 of them."""
+    assert ops.mlstm_chunks_preferred(40960, 40960, 1, 20, 128, 128)
+    assert not ops.mlstm_chunks_preferred(220000, 220000, 1, 20, 128, 128)
+    assert not ops.mlstm_chunks_preferred(60000, 60000, 1, 96, 128, 128)

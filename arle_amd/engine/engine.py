@@ -217,15 +217,15 @@ class Engine:
             # a mixer with state of its own overwrites it while the step runs: keep what a failed step must leave.
             # A step that is replayed from its graph runs no Python between its kernels, so nothing can fail half way.
             if decode_only:
-                rows_now = len(entries)
-                replayed = (rows_now, self._decode_class(entries, before)) in self._graphs
+                decode_key = self._decode_key(entries, before)
+                replayed = decode_key in self._graphs
             else:
                 replayed = shape_key is not None and shape_key in self._graphs
             if not replayed:
                 saved_state = self.cache.snapshot_state([e.request for e in entries])
             self.cache.sync_tables()
             if decode_only:
-                logits = self._decode_step_graphed(entries, before, borrow_logits)
+                logits = self._decode_step_graphed(decode_key, entries, before, borrow_logits)
             elif shape_key is not None:
                 logits = self._step_graphed(shape_key, entries, before, borrow_logits)
             else:
@@ -241,12 +241,12 @@ class Engine:
         return logits
 
     # -- captured decode steps ----------------------------------------------------------------
-    def _decode_class(self, entries, before) -> tuple:
-        """What the launches of a step of single decoded tokens depend on beside the number of rows."""
+    def _decode_key(self, entries, before) -> tuple:
+        """What the launches of a step of single decoded tokens depend on: the number of rows and the parts' answers."""
         contexts = [before[e.request] + 1 for e in entries]
-        return self.model.decode_launch_class(len(entries), max(contexts), self._warm_total or sum(contexts))
+        return len(entries), self.model.decode_launch_class(len(entries), max(contexts), self._warm_total or sum(contexts))
 
-    def _decode_step_graphed(self, entries, before, borrow: bool = False) -> torch.Tensor:
+    def _decode_step_graphed(self, key, entries, before, borrow: bool = False) -> torch.Tensor:
         """A step of single decoded tokens through a HIP graph captured for its number of rows.
 
         The graph computes the logits of every row; the wanted ones are picked afterwards.  What
@@ -257,7 +257,6 @@ class Engine:
         attention, which follows the longest context).
         """
         rows = len(entries)
-        key = (rows, self._decode_class(entries, before))
         all_rows = [StepEntry(e.request, e.tokens, [0]) for e in entries]
         length_before = before.__getitem__
         rec = self._graphs.pop(key, None)

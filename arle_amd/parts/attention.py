@@ -106,6 +106,9 @@ class PagedAttention(Part):
             return None
         return ops.decode_share(rows, self.nkv, max_context, total_context)
 
+    def decode_class_sizes(self):
+        return self.rt.is_f32, self.D, self.nkv, self.window, self.folds_preparation
+
     def forward(self, x, batch, cache):
         """x [T, H] -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear)."""
         Q, KV = self.q_width, self.kv_width

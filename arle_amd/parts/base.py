@@ -81,6 +81,12 @@ class Pending(list):
     """What a block leaves for the next norm to add into the residual: [(addend, bias or None), ...]."""
 
 
+def nested_class_sizes(parts):
+    """`Part.decode_class_sizes` of a part that answers what these parts nested in it do."""
+    found = tuple((type(p), p.decode_class_sizes()) for p in parts if hasattr(p, "decode_class_sizes"))
+    return None if all(sizes is None for _, sizes in found) else found
+
+
 class Part:
     role = ""
     kind = ""
@@ -138,6 +144,15 @@ class Part:
         found = tuple(child.decode_spread_class(rows, max_context, total_context)
                       for child in getattr(self, "child_parts", {}).values() if hasattr(child, "decode_spread_class"))
         return None if all(f is None for f in found) else found
+
+    def decode_class_sizes(self):
+        """What of this part its answers to decode_launch_class and decode_spread_class hang on (a hashable value; None: it
+        never answers): of the parts of a kind with equal sizes a model asks one, once a step.  A part that answers and
+        says nothing of its sizes counts for itself; the default speaks for the parts nested in this one."""
+        kind = type(self)
+        if kind.decode_launch_class is not Part.decode_launch_class or kind.decode_spread_class is not Part.decode_spread_class:
+            return self
+        return nested_class_sizes(getattr(self, "child_parts", {}).values())
 
     def prepare(self, max_positions: int) -> None:
         """Called by the engine once the longest request is known, before any step runs or is captured: whatever

@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import ops
-from .base import Part, WeightDecl, lookup, register
+from .base import Part, WeightDecl, lookup, nested_class_sizes, register
 from .linear import Linear
 
 
@@ -48,6 +48,9 @@ class _TwoMixers(Part):
     def decode_launch_class(self, rows, max_context):
         found = tuple(m.decode_launch_class(rows, max_context) for m in (self.left, self.right))
         return None if all(f is None for f in found) else found
+
+    def decode_class_sizes(self):
+        return nested_class_sizes((self.left, self.right))
 
 
 @register("mixer", "mixer_pair")

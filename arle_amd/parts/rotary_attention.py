@@ -172,6 +172,9 @@ class RotaryAttention(Part):
             return None
         return ops.decode_splits(rows, self.nkv, self._keys_seen(max_context))
 
+    def decode_class_sizes(self):
+        return self.rt.is_f32, self.softcap, self.Dk, self.Dv, self.nkv, self.window
+
     def takes_sums(self, x, batch) -> bool:
         """Whether this step is one of decoded rows that `heads_of_sums` takes."""
         rotary_dim, interleaved = 0, False

@@ -11,7 +11,7 @@ from __future__ import annotations
 
 from ..cache.manager import StateNeed
 from ..kernels import ops
-from .base import Part, WeightDecl, register
+from .base import Part, WeightDecl, nested_class_sizes, register
 
 
 class ShortConv:
@@ -88,6 +88,9 @@ class InputConvMixer(Part):
 
     def decode_launch_class(self, rows, max_context):
         return self.inner.decode_launch_class(rows, max_context)
+
+    def decode_class_sizes(self):
+        return nested_class_sizes((self.inner,))
 
     def forward(self, x, batch, cache):
         cache = cache or {}

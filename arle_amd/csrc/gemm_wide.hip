@@ -306,7 +306,7 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   }
 }
 
-static int g_wide_rows = 8, g_wide_cols = 4;
+constexpr int kWdPatchRows = 8, kWdPatchCols = 4;   // row and column blocks that an XCD's workgroups take together
 
 template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
 int launch_wide(WideArgs a, int splits, hipStream_t s) {
@@ -325,8 +325,8 @@ int launch_wide(WideArgs a, int splits, hipStream_t s) {
   }
   a.m_blocks = (a.M + BM - 1) / BM;
   a.n_blocks = (a.N + BN - 1) / BN;
-  a.patch_rows = a.m_blocks < g_wide_rows ? a.m_blocks : g_wide_rows;
-  a.patch_cols = a.m_blocks > a.patch_rows ? g_wide_cols : 1;
+  a.patch_rows = a.m_blocks < kWdPatchRows ? a.m_blocks : kWdPatchRows;
+  a.patch_cols = a.m_blocks > a.patch_rows ? kWdPatchCols : 1;
   const long long cols_an_xcd = (a.n_blocks + kWdXcds - 1) / kWdXcds;
   const long long row_groups = (a.m_blocks + a.patch_rows - 1) / a.patch_rows;
   const long long col_groups = (cols_an_xcd + a.patch_cols - 1) / a.patch_cols;
@@ -345,10 +345,6 @@ int dispatch_wide(const WideArgs& a, int splits, int out_dtype, int epilogue, hi
 }  // namespace arle
 
 using namespace arle;
-
-extern "C" void arle_gemm_wide_patch(int rows, int cols) {
-  if (rows >= 1 && cols >= 1) g_wide_rows = rows, g_wide_cols = cols;
-}
 
 // x [M, K], w [N, K] bfloat16 with 16-byte aligned rows, K % 64 == 0, N % 32 == 0.  out [M, N] (bfloat16 or float32), or
 // with epilogue 1 [M, N/2] bfloat16 (gate and up rows of w interleaved in blocks of 16): silu(gate) * up.

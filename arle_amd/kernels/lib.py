@@ -33,7 +33,6 @@ SIGNATURES = {
     "arle_gemm_rows_lds": ("gemm_rows", [_i, _i, _i]),
     "arle_gemm_tiles": ("gemm_tiles", [_p, _ll, _p, _p, _ll, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _ll, _p]),
     "arle_gemm_wide": ("gemm_wide", [_p, _ll, _p, _ll, _p, _ll, _i, _i, _i, _i, _i, _i, _i, _i, _i, _ll, _p]),
-    "arle_gemm_wide_patch": ("gemm_wide", [_i, _i]),
     "arle_gemm_tiles_patch": ("gemm_tiles", [_i, _i]),
     "arle_gemm_rows_lds_max": ("gemm_rows", []),
     "arle_gemm_f32": ("gemm_f32", [_p, _ll, _p, _ll, _p, _ll, _i, _i, _i, _p]),

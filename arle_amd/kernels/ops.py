@@ -1046,6 +1046,7 @@ def gemm_tiles(x, tiles, n: int, out_dtype=torch.bfloat16, epilogue: int = EPI_N
 WIDE_STAGE_US = {(128, 64): 0.62, (128, 96): 0.80, (128, 128): 0.87, (128, 160): 0.89, (128, 192): 0.92, (128, 256): 1.04,
                  (128, 320): 1.15, (256, 160): 1.16, (256, 192): 1.32, (256, 256): 1.52, (192, 320): 1.52, (256, 320): 1.85}
 _WIDE_FIXED_US = 4.0
+_XCDS = 8
 _WIDE_MAX_PARTS = 8
 _WIDE_K = 64            # K comes in whole stages
 
@@ -1065,8 +1066,9 @@ def wide_plan(rows: int, n: int, k: int, parts: int = 1, units: int = 256) -> tu
     stages = -(-(k // _WIDE_K) // parts)
     best = None
     for (bm, bn), stage_us in WIDE_STAGE_US.items():
-        workgroups = -(-rows // bm) * -(-n // bn) * parts
-        us = -(-workgroups // units) * (_WIDE_FIXED_US + stages * stage_us)
+        # column blocks go to the XCDs in turn: the one with most of them is the last to be done
+        workgroups = -(-rows // bm) * -(-(-(-n // bn)) // _XCDS) * parts
+        us = -(-workgroups * _XCDS // units) * (_WIDE_FIXED_US + stages * stage_us)
         if best is None or us < best[1]:
             best = ((bm, bn), us)
     return best

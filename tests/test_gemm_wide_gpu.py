@@ -118,3 +118,18 @@ def test_the_activation_below_where_the_reciprocal_leaves_the_floats():
         assert torch.isnan(row[13]) and float(row[12]) == float("inf")
         keep = [i for i in range(16) if i not in (11, 12, 13)]
         assert torch.allclose(row[keep], want[keep], rtol=2.0 ** -8, atol=1e-38) and float(row[11]) == float("inf")
+
+
+@pytest.mark.parametrize("shape,row_blocks,col_blocks", [((128, 64), 9, 8), ((128, 64), 10, 22), ((128, 96), 13, 33), ((128, 320), 17, 3),
+                                                         ((256, 160), 10, 9), ((256, 256), 16, 41), ((192, 320), 11, 10), ((256, 320), 9, 40)])
+def test_blocks_of_several_patches(shape, row_blocks, col_blocks):
+    """More row blocks than a patch has, in numbers that eight does not divide, and column blocks to match: every block is
+    somebody's, the last ones in part."""
+    from arle_amd.kernels import ops
+
+    M, N = shape[0] * row_blocks - 37, shape[1] * col_blocks - 32
+    x, w = _operands(M, N, 128, row_blocks)
+    want = x.double() @ w.double().T
+    assert _rel(ops.gemm_wide(x, w, shape=shape), want) < 2.0 ** -8
+    stack = ops.gemm_wide(x, w, torch.float32, shape=shape, splits=2)
+    assert _rel(stack.sum(0), want) < 1e-5

@@ -1319,20 +1319,31 @@ class ProductChoice:
 
 PRODUCT_KERNELS = ("rows", "stream", "rounds", "tiles", "tiles_parts", "wide", "library", "library_parts")
 
-# gate|up with its activation by gemm_wide from 65 rows on where K is at most _WIDE_MAX_K, and up to _WIDE_MID_ROWS rows
-# beyond.  MI355X, cold weights, us, the library's product and the activation kernel / gemm_tiles / gemm_wide: Qwen3-4B
-# (N 19,456, K 2,560) 97 rows 40.5 / 49.5 / 32.3, 256 51.7 / 51.0 / 35.8, 512 64.3 / 83.4 / 48.6, 1,024 115 / 120 / 84,
-# 2,048 217 / 200 / 167, 4,096 440 / 393 / 327, 8,192 772 / 793 / 648; Qwen3-8B (N 24,576, K 4,096) 256 70.2 / 78.1 / 59.4,
-# 544 133.7 / 121.0 / 98.2, 768 152.7 / 179.7 / 125.4, 1,536 264 / 298 / 248, 2,048 309 / 372 / 318, 8,192 1,218 / 1,475 / 1,249.
-_WIDE_MIN_ROWS = 65
-_WIDE_MAX_K = 3072
+# gate|up with its activation by gemm_wide, for widths that no table names.  MI355X, launches from a captured graph, cold
+# weights, us, what the other rules take (the library's product and the activation kernel, or gemm_tiles) / gemm_wide:
+#   K <= 1,024, from 65 rows on: N 6,144, K 1,024 97 rows 13.4 / 10.4, 256 17.5 / 10.8, 1,024 24.7 / 17.3, 4,096 75.7 / 55.3.
+#   K <= 2,560, from 129 on: N 12,288, K 2,048 97 rows 22.0 / 22.7, 160 29.3 / 24.2, 512 41.8 / 34.4, 2,560 128.7 / 113.5; N
+#     4,096, K 2,048 97 rows 13.7 / 16.4, 160 18.3 / 16.5 (and 256, where the library is at its best, 16.0 / 17.1).
+#   K <= 6,144, 193 to 256 rows and from 512 on, beyond K 3,072 up to 1,792: with little of a turn filled the long walk over
+#     K is not paid for.  N 28,672, K 5,120 128 rows 76.5 / 85.3, 192 90.5 / 96.3, 256 101.8 / 99.3, 384 122.1 / 135.2, 512
+#     162.0 / 140.8, 1,024 302 / 257; N 20,480, K 6,144 128 rows 76.5 / 83.3, 256 109.4 / 89.6, 512 144.5 / 123.9; N 16,384,
+#     K 3,072 128 rows 35.6 / 37.1, 256 48.1 / 41.1, 640 72.3 / 79.1, 1,024 100.9 / 88.6.
+#   K 8,192, N 57,344: 128 rows 228 / 259, 512 440 / 443, 1,536 1,101 / 1,216.
+# Of 261 such products taken from 65 to 8,192 rows six were slower by 3 % and more (10 % at most), all of them 17 % faster.
+_WIDE_BY_K = ((1024, 65), (2560, 129), (6144, 512))     # (K up to, rows from)
+_WIDE_TWO_BLOCKS = (193, 256)                           # and these rows, two row blocks of 128 that are all but full
+_WIDE_ANY_ROWS_K = 3072
 _WIDE_MID_ROWS = 1792
 
 
 def gemm_wide_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
     """Whether gate|up with its activation runs in gemm_wide (the rule for widths that no table names)."""
-    return (rows >= _WIDE_MIN_ROWS and n >= _TILES_MIN_N and gemm_wide_supported(n, k, x_stride)
-            and (k <= _WIDE_MAX_K or rows <= _WIDE_MID_ROWS))
+    if n < _TILES_MIN_N or not gemm_wide_supported(n, k, x_stride) or (k > _WIDE_ANY_ROWS_K and rows > _WIDE_MID_ROWS):
+        return False
+    least = next((least for most_k, least in _WIDE_BY_K if k <= most_k), None)
+    return least is not None and (rows >= least or _WIDE_TWO_BLOCKS[0] <= rows <= _WIDE_TWO_BLOCKS[1])
+
+
 _PRODUCT_TABLE: dict = {}
 
 

@@ -3,6 +3,25 @@ import pytest
 
 from arle_amd.kernels import ops
 
+# (rows, N, K) of gate|up and which was faster by 3 % and more: gemm_wide, or what the other rules take (us on MI355X)
+MEASURED = [
+    ((65, 6144, 1024), True), ((256, 6144, 1024), True), ((3072, 6144, 1024), True), ((8192, 12288, 1024), True),     # 13.1 / 10.3, 17.5 / 10.8, 51.9 / 47.2, 221.9 / 200.1
+    ((65, 4096, 2048), False), ((97, 8192, 3072), False), ((128, 8192, 3072), False), ((80, 16384, 3072), False),     # 13.4 / 16.3, 25.0 / 30.1, 26.6 / 32.1, 32.4 / 36.0
+    ((160, 12288, 2048), True), ((512, 12288, 2048), True), ((2560, 12288, 2048), True), ((256, 16384, 3072), True),  # 29.3 / 24.2, 41.8 / 34.4, 130.3 / 115.2, 48.1 / 41.1
+    ((65, 28672, 5120), False), ((160, 28672, 5120), False), ((192, 28672, 5120), False), ((384, 28672, 5120), False),  # 72.1 / 83.0, 82.5 / 97.0, 90.5 / 96.3, 122.1 / 135.2
+    ((512, 28672, 5120), True), ((1792, 28672, 5120), True), ((256, 20480, 6144), True), ((128, 20480, 6144), False),  # 162.0 / 140.8, 549.4 / 446.4, 109.4 / 89.6, 76.5 / 83.3
+    ((65, 22016, 4096), False), ((128, 28672, 4096), False), ((320, 28672, 4096), False), ((1280, 28672, 4096), True),  # 52.0 / 56.8, 63.6 / 71.7, 94.7 / 105.2, 302.4 / 260.3
+    ((128, 57344, 8192), False), ((320, 57344, 8192), False), ((1536, 57344, 8192), False), ((320, 28672, 8192), False),  # 228 / 259, 336 / 415, 1,101 / 1,216, 171 / 209
+]
+
+
+@pytest.mark.parametrize("size,wide", MEASURED)
+def test_the_faster_kernel_is_taken(size, wide):
+    rows, n, k = size
+    choice = ops.product_by_rules(rows, n, k, k, tiled=True, fused=True, partials_ok=False)
+    assert (choice.kernel == "wide") == wide
+
+
 # (rows, N, K), workgroups that were slower and faster ones (us): what an XCD gets of the column blocks decides, not their sum
 PLANS = [
     (3072, 6144, 1024, (256, 320), (256, 160)),      # 67.5 / 47.2: 240 workgroups, but 36 on some XCDs of 32 places

@@ -59,3 +59,27 @@ def test_every_block_has_one_workgroup_and_no_row_is_empty(row_blocks, col_block
     inside = [p for p in taken if p[1] < col_blocks]
     assert len(inside) == len(set(inside)) == row_blocks * col_blocks
     assert len(taken) - len(inside) < 8 * row_blocks       # only the last column blocks' XCDs have places left
+
+
+@pytest.mark.parametrize("rows,n,k,fused,kernel", [
+    (1000, 2560, 4096, False, "library_parts"),      # 29.5 us / gemm_wide's two parts 30.9
+    (6272, 2560, 4096, False, "library"), (6400, 2560, 9728, False, "library"),     # 95.8 / 120.5, 208 / 261
+    (6272, 5120, 8192, False, "library"), (6400, 5120, 25600, False, "library"),    # 341 / 449, 1,086 / 1,417
+    (6410, 2560, 4096, False, "wide"), (6410, 2560, 9728, False, "wide"),           # 117.7 / 118.2, 267 / 262
+    (6410, 5120, 8192, False, "wide"), (6410, 5120, 25600, False, "wide"),          # 578 / 423, 1,830 / 1,363
+    (6400, 19456, 2560, True, "wide"), (6500, 19456, 2560, True, "library"), (6657, 19456, 2560, True, "wide"),   # 611 / 531, 540 / 558
+    (6272, 24576, 4096, True, "library"), (6410, 24576, 4096, True, "wide"),        # 979 / 1,003, 1,135 / 1,026
+])
+def test_the_shipped_tables_have_their_lines_where_the_kernels_cross(rows, n, k, fused, kernel):
+    """The library's 256 x 256 workgroups fill a last turn up to 6,400 rows (25 row blocks) of these widths."""
+    import glob
+    import os
+
+    keep = dict(ops._PRODUCT_TABLE)
+    try:
+        for path in glob.glob(os.path.join(ops.PRODUCT_TABLE_DIR, "*.json")):
+            ops.load_product_table(path)
+        assert ops.choose_product(rows, n, k, k, tiled=True, fused=fused, partials_ok=True).kernel == kernel
+    finally:
+        ops._PRODUCT_TABLE.clear()
+        ops._PRODUCT_TABLE.update(keep)

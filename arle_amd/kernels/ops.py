@@ -1143,7 +1143,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.b
     _need(out_dtype in (torch.bfloat16, torch.float32), "gemm_bf16 writes bfloat16 or float32")
     rows, n, k = x.shape[0], w.shape[0], x.shape[1]
     choice = choose_product(rows, n, k, x.stride(0), tiled=tiles is not None, fused=False, partials_ok=partials_ok,
-                            aligned=x.data_ptr() % 16 == 0)
+                            aligned=x.data_ptr() % 16 == 0, w_aligned=w.data_ptr() % 16 == 0)
     return run_product(choice, x, w, tiles, out_dtype, partials_ok)
 
 
@@ -1348,15 +1348,16 @@ _PRODUCT_TABLE: dict = {}
 
 
 def product_by_rules(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, fused: bool, partials_ok: bool,
-                     aligned: bool = True) -> ProductChoice:
+                     aligned: bool = True, w_aligned: bool = True) -> ProductChoice:
     """The kernel for x[rows, k] . w[n, k]^T by the measured thresholds.  fused: gate|up with SiLU·mul (w holds
-    gate and up rows interleaved in blocks of 16), whose result is the activation [rows, n/2]."""
+    gate and up rows interleaved in blocks of 16), whose result is the activation [rows, n/2].  aligned, w_aligned: x and
+    w begin on the 16-byte grid (w as it lies, contiguous, which gemm_wide reads; its tiles always do)."""
     if fused:
         if rows and aligned and gemm_rows_preferred(rows, n, k, x_stride, fused=True):
             return ProductChoice("rows", (_fused_variant(rows),), 1)
         if rows and aligned and tiled and gemm_rows_rounds_preferred(rows, n, k, x_stride):
             return ProductChoice("rounds")
-        if aligned and gemm_wide_preferred(rows, n, k, x_stride):
+        if aligned and w_aligned and gemm_wide_preferred(rows, n, k, x_stride):
             return ProductChoice("wide")
         if aligned and tiled and gemm_tiles_preferred(rows, n, k, x_stride, fused=True):
             return ProductChoice("tiles", (8, 144) if rows >= _TILES_BIG_ROWS else (4, 44))
@@ -1454,16 +1455,17 @@ def clear_product_table() -> None:
 
 
 def choose_product(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, fused: bool, partials_ok: bool,
-                   aligned: bool = True) -> ProductChoice:
+                   aligned: bool = True, w_aligned: bool = True) -> ProductChoice:
     """The table's entry for these widths and this many rows if there is one (the tables were measured with operands
-    on the 16-byte grid: others go by the rules), else `product_by_rules`."""
+    on the 16-byte grid: others go by the rules, as do those that gemm_wide does not take), else `product_by_rules`."""
     on_grid = aligned and k % 8 == 0 and x_stride % 8 == 0
     entries = _PRODUCT_TABLE.get((n, k, fused, tiled)) if on_grid and _PRODUCT_TABLE else None
     if entries:
-        for most_rows, choice in entries:
-            if rows <= most_rows:
-                return choice
-    return product_by_rules(rows, n, k, x_stride, tiled=tiled, fused=fused, partials_ok=partials_ok, aligned=aligned)
+        choice = next((c for most_rows, c in entries if rows <= most_rows), None)
+        if choice is not None and (choice.kernel != "wide" or (w_aligned and gemm_wide_supported(n, k, x_stride))):
+            return choice
+    return product_by_rules(rows, n, k, x_stride, tiled=tiled, fused=fused, partials_ok=partials_ok, aligned=aligned,
+                            w_aligned=w_aligned)
 
 
 def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool, fused: bool = False):
@@ -1521,7 +1523,7 @@ def gate_up_act(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor | None = N
     if act != 0:     # the products that apply the activation themselves know silu only
         return act_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), act, 16)
     choice = choose_product(rows, n, k, x.stride(0), tiled=tiles is not None, fused=True, partials_ok=False,
-                            aligned=x.data_ptr() % 16 == 0)
+                            aligned=x.data_ptr() % 16 == 0, w_aligned=w.is_contiguous() and w.data_ptr() % 16 == 0)
     return run_product(choice, x, w, tiles, x.dtype, False, fused=True)
 
 

@@ -83,3 +83,43 @@ def test_the_shipped_tables_have_their_lines_where_the_kernels_cross(rows, n, k,
     finally:
         ops._PRODUCT_TABLE.clear()
         ops._PRODUCT_TABLE.update(keep)
+
+
+def test_operands_off_its_grid_do_not_go_to_it():
+    """Weights that begin between two multiples of 16 bytes, or rows of x too far apart: the rules without gemm_wide."""
+    widths = (6144, 1024)
+    table = {"6144,1024,1,1": [[4096, "wide", [], 0]], "6144,1024,0,1": [[4096, "wide", [], 2]]}
+    keep = dict(ops._PRODUCT_TABLE)
+    try:
+        for fused in (True, False):
+            ops._PRODUCT_TABLE.clear()
+            by_rules = ops.choose_product(300, *widths, 1024, tiled=True, fused=fused, partials_ok=True, w_aligned=False).kernel
+            ops.load_product_table(table)
+            on_grid = dict(tiled=True, fused=fused, partials_ok=True)
+            assert ops.choose_product(300, *widths, 1024, **on_grid).kernel == "wide" != by_rules
+            assert ops.choose_product(300, *widths, 1024, w_aligned=False, **on_grid).kernel == by_rules
+            assert ops.choose_product(300, *widths, 1 << 20, **on_grid).kernel != "wide"
+    finally:
+        ops._PRODUCT_TABLE.clear()
+        ops._PRODUCT_TABLE.update(keep)
+
+
+def test_calls_look_where_their_weights_lie(monkeypatch):
+    """gate_up_act and gemm_bf16 with a contiguous view that begins two bytes into its storage, and gate_up_act with rows of
+    w further apart than K: none of them goes to gemm_wide (the last is then refused, as it was)."""
+    import torch
+
+    chosen = []
+    monkeypatch.setattr(ops, "_gpu", lambda *tensors: None)
+    monkeypatch.setattr(ops, "run_product", lambda choice, *args, **kw: chosen.append(choice.kernel))
+    monkeypatch.setattr(ops, "_PRODUCT_TABLE", {(4096, 512, False, False): [(4096, ops.ProductChoice("wide", (), 1))]})
+    x = torch.zeros(200, 512, dtype=torch.bfloat16)
+    store = torch.zeros(4096 * 520 + 16, dtype=torch.bfloat16)
+    first = next(i for i in range(8) if store[i:].data_ptr() % 16 == 0)
+    straight, shifted = (store[first + i:first + i + 4096 * 512].view(4096, 512) for i in (0, 1))
+    apart = store[first:first + 4096 * 520].view(4096, 520)[:, :512]
+    for w in (straight, shifted, apart):
+        ops.gate_up_act(x, w)
+    for w in (straight, shifted):
+        ops.gemm_bf16(x, w)
+    assert chosen[0] == chosen[3] == "wide" and "wide" not in (chosen[1], chosen[2], chosen[4])

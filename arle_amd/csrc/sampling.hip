@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kWave) void argmax_merge_kernel(const ArgMax* __res
 //   min_p:  e >= min_p                       (the largest e is exp(0) = 1)
 //   top_k:  e >= the k-th largest e           (ties of the k-th stay)
 //   top_p:  e >= the largest t whose kept mass reaches top_p of the mass kept so far
-// The k-th largest value and the mass threshold are found digit by digit, 11 + 11 + 10 bits: a pass over the
+// The k-th largest value and the mass threshold are found digit by digit, 10 + 11 + 10 bits: a pass over the
 // row fills a histogram with the next digit of the elements that match the digits found so far; scanning the bins
 // from the top gives the digit in which the count (the mass) is reached.  Counts are integers and masses are summed as
 // 64-bit fixed-point numbers (e * 2^40), so the histograms do not depend on the order in which workgroups add to
@@ -746,23 +746,24 @@ extern "C" int arle_argmax_rows(const float* logits, int rows, int vocab, int* o
   return launch_status();
 }
 
-// Scratch of a sampling call, in bytes: the histograms (which the caller hands over filled with zeros: the whole
-// scratch may simply be zeroed), the passes' slots, the chunk maxima and masses, the groups' maxima and the thresholds.
+// Scratch of a sampling call, in bytes: the histograms of top_k and of top_p, the passes' slots, the chunk maxima and masses,
+// the groups' maxima and the thresholds.
 static inline int sample_chunk_len(int vocab, int chunks) { return (((vocab + chunks - 1) / chunks) + 3) & ~3; }
 static inline int sample_groups(int vocab, int chunks) { return (sample_chunk_len(vocab, chunks) + kGroup - 1) / kGroup; }
-static inline size_t sample_hist_p_bytes(int rows) { return static_cast<size_t>(rows) * kRowBins * sizeof(unsigned long long); }
-static inline size_t sample_hist_k_bytes(int rows) { return static_cast<size_t>(rows) * kRowBins * sizeof(unsigned int); }
+extern "C" long long arle_sample_hist_k_bytes(int rows) { return static_cast<long long>(rows) * kRowBins * sizeof(unsigned int); }
+extern "C" long long arle_sample_hist_p_bytes(int rows) { return static_cast<long long>(rows) * kRowBins * sizeof(unsigned long long); }
 extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
   const int chunks = arle_argmax_chunks(rows, vocab);
-  return static_cast<long long>(sample_hist_p_bytes(rows) + static_cast<size_t>(rows) * kPasses * sizeof(Slot) +
-                                sample_hist_k_bytes(rows) +
+  return arle_sample_hist_k_bytes(rows) + arle_sample_hist_p_bytes(rows) +
+         static_cast<long long>(static_cast<size_t>(rows) * kPasses * sizeof(Slot) +
                                 static_cast<size_t>(rows) * chunks *
                                     (sizeof(ArgMax) + sizeof(float) + sample_groups(vocab, chunks) * sizeof(float)) +
                                 rows * sizeof(unsigned int));
 }
 
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
-// arle_sample_scratch_bytes(rows, vocab) zeroed bytes, 8-byte aligned.  use_top_k / use_top_p == 0 promise that
+// arle_sample_scratch_bytes(rows, vocab) bytes, 8-byte aligned, of which the caller zeroes the first
+// arle_sample_hist_k_bytes(rows) with use_top_k and the arle_sample_hist_p_bytes(rows) behind those with use_top_p.  use_top_k / use_top_p == 0 promise that
 // no row of the call has the filter switched on (top_k in 1..vocab-1, top_p < 1); its passes are then left out.
 extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float* probs,
                                 const float* temperature, const int* top_k, const float* top_p,
@@ -785,12 +786,12 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.min_p = min_p;
   a.u = u;
   unsigned char* at = static_cast<unsigned char*>(scratch);
+  a.hist_k = reinterpret_cast<unsigned int*>(at);
+  at += arle_sample_hist_k_bytes(rows);
   a.hist_p = reinterpret_cast<unsigned long long*>(at);
-  at += sample_hist_p_bytes(rows);
+  at += arle_sample_hist_p_bytes(rows);
   a.slots = reinterpret_cast<Slot*>(at);
   at += static_cast<size_t>(rows) * kPasses * sizeof(Slot);
-  a.hist_k = reinterpret_cast<unsigned int*>(at);
-  at += sample_hist_k_bytes(rows);
   ArgMax* part_max = reinterpret_cast<ArgMax*>(at);
   a.part_max = part_max;
   at += static_cast<size_t>(rows) * a.chunks * sizeof(ArgMax);

@@ -459,6 +459,27 @@ def test_sampling_at_the_edges_of_groups_and_chunks(vocab):
             assert _sample(base, 0.9, u, **p) == want[4 * n:4 * n + 4], (u, p)
 
 
+@pytest.mark.parametrize("rows,vocab", [(5, 200), (3, 9000), (2, 40000)])
+def test_sampling_asks_no_more_of_its_scratch_than_zeroed_histograms(rows, vocab, monkeypatch):
+    """With every new buffer full of ones, rows with and without each filter, greedy ones among them, choose the same tokens
+    as in a call with both filters' passes and zeros throughout."""
+    g = _g(9)
+    logits = torch.randn(rows, vocab, generator=g).mul_(2.0).to(DEV)
+    column = lambda values, dtype=torch.float32: torch.tensor([values[r % len(values)] for r in range(rows)], dtype=dtype, device=DEV)
+    u, empty = column([0.3, 0.9]), torch.empty
+    zeros = lambda *a, **k: empty(*a, **k).zero_()
+    ones = lambda *a, **k: empty(*a, **k).view(torch.uint8).fill_(0xff).view(k["dtype"])
+    for ks, ps, ms in (([-1], [1.0], [0.0]), ([-1], [1.0], [0.1]), ([40, -1], [1.0], [0.0]), ([-1], [0.7, 1.0], [0.0]), ([40, -1], [0.7, 0.9, 1.0], [0.0])):
+        for temps in ([0.9], [0.9, 0.0]):
+            args = column(temps), column(ks, torch.int32), column(ps), column(ms), u
+            monkeypatch.setattr(torch, "empty", zeros)
+            want = ops.sample_rows(logits, *args).tolist()
+            monkeypatch.setattr(torch, "empty", ones)
+            got = ops.sample_rows(logits, *args, use_top_k=max(ks) > 0, use_top_p=min(ps) < 1).tolist()
+            monkeypatch.setattr(torch, "empty", empty)
+            assert got == want, (ks, ps, ms, temps)
+
+
 def test_penalties():
     logits = torch.tensor([[2.0, -2.0, 1.0, 0.5], [1.0, 1.0, 1.0, 1.0]])
     d = logits.to(DEV)

@@ -183,6 +183,50 @@ def test_mlstm_in_every_cut_and_over_a_long_sequence(dtype, m):
             assert torch.equal(got, first), f"cuts {cuts} change the bits"
 
 
+@pytest.mark.parametrize("m", [mlstm(2, 64, 96), mlstm(1, 128, 128, cap=3.0), mlstm(3, 32, 32)])
+def test_mlstm_portions_in_chunks_hand_over_to_single_rows_and_back(m, monkeypatch):
+    """bfloat16 mode, heads that the chunks take: portions of 96 rows and more go in chunks, shorter ones and single rows
+    row by row, on one state; alone, and beside another request that decodes."""
+    from arle_amd.kernels import ops
+
+    longest, whole = [], ops.mlstm_chunks
+    monkeypatch.setattr(ops, "mlstm_chunks", lambda qkvg, *a, **k: longest.append(qkvg.shape[0]) or whole(qkvg, *a, **k))
+    width, T = 48, 150
+    t = mlstm_tensors(width, m, 31, gate_std=0.05)
+    x = rnd((T, width), 41)
+    x[4] *= 1.5
+    params = {"hidden_size": width, "heads": m["heads"], "key_dim": m["dim"], "value_dim": m["vdim"],
+              "gate_cap": m["gate_cap"], "eps": 1e-5}
+    part = make_part("mixer", "mlstm", params, t, BF16)
+    want = plain.mlstm_mixer(x.double(), plain_names(t), m, 1e-5)
+    for cuts, chunked in (((150,), [150]), ((100, 1, 49), [100]), ((64, 86), []), ((149, 1), [149]), ((1, 99, 50), [99]), ((7, 1, 130, 1, 11), [130])):
+        longest.clear()
+        close(run_mixer(part, x, cuts, dtype=BF16), want, BF16, f"mlstm {m}, cuts {cuts}")
+        assert longest == chunked, cuts
+    # r's portions beside s, which has 40 rows and decodes on
+    lengths = {"s": 0, "r": 0}
+    rows = {"s": rnd((44, width), 43), "r": x}
+    cache = CacheManager([part.cache_need()], page_size=4, num_pages=60, max_slots=3, max_request_tokens=160, device=torch.device(DEV),
+                         dtype=BF16)
+    for key in lengths:
+        cache.admit(key)
+    longest.clear()
+    outs = {"s": [], "r": []}
+    for step in ({"s": 40}, {"r": 100, "s": 1}, {"s": 1, "r": 1}, {"r": 48, "s": 1}, {"r": 1, "s": 1}):
+        cache.append(list(step.items()))
+        cache.sync_tables()
+        batch = build_step_batch([StepEntry(k, [0] * n, []) for k, n in step.items()], cache.slot_of.__getitem__, lengths.__getitem__, 10, DEV)
+        part_rows = torch.cat([rows[k][lengths[k]:lengths[k] + n] for k, n in step.items()]).to(DEV, BF16).contiguous()
+        y = part.forward(part_rows, batch, cache.view(0))
+        y = (y.float().sum(0) if y.dim() == 3 else y.float()).cpu()
+        for k, piece in zip(step, y.split(list(step.values()))):
+            outs[k].append(piece)
+            lengths[k] += step[k]
+    assert longest == [101]
+    for k in outs:
+        close(torch.cat(outs[k]), plain.mlstm_mixer(rows[k].double(), plain_names(t), m, 1e-5), BF16, f"mlstm {m}, {k} of a mixed step")
+
+
 def attention_tensors(width, m, seed, shares=False):
     H, G, D, Dv, taps = m["heads"], m["kv_heads"], m["dim"], m["vdim"], m["conv"]
     t = {"q": rnd((H * D, width), seed, 0.3), "q_bias": rnd((H * D,), seed + 1, 0.3), "q_norm": 1 + rnd((D,), seed + 2, 0.1),

@@ -68,31 +68,20 @@ __device__ __forceinline__ void wide_touch(const uint16_t* from, uint32_t lds_at
 #pragma clang diagnostic pop
 
 // x / (1 + exp(-x)) to the error of expf and a whole divide, for |x| < kSiluNear, where nothing leaves the range of a
-// float: exp(-x) = 2^n 2^f with n + f = -x log2(e) in two parts, and the quotient from the reciprocal with one correction.
-// Against 64 bits over [-80, 80]: at most 2.71 ulp, 0.44 to 0.65 in the root mean square, for both forms alike (the vector
-// unit's exponential of the rounded -x log2(e) and its reciprocal, as they come: up to 63 ulp, 21).
+// float: exp(-x) = 2^t (1 + r), t = -x log2(e) rounded and r = -x - t ln 2, ln 2 in two parts; the quotient by 1 + 2^t from the
+// reciprocal, corrected by what is left of x behind it and behind its share of 2^t r.  Against 64 bits over [-80, 80]: at most
+// 2.71 ulp, 0.44 to 0.65 in the root mean square, for both forms alike (the vector unit's exponential of t alone and its
+// reciprocal, as they come: up to 63 ulp, 21).
 constexpr float kSiluNear = 80.0f;
 __device__ __forceinline__ float silu_near(float x) {
-#pragma clang fp contract(off)   // t - n is exact as it stands
-  constexpr float kHi = -1.44269502162933349609375f, kLo = -1.92596299112661746e-8f;   // -log2(e)
-  const float t = x * kHi, n = __builtin_rintf(t);
-  const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f((t - n) + fmaf(x, kLo, fmaf(x, kHi, -t))), static_cast<int>(n));
+#pragma clang fp contract(off)
+  constexpr float kLog2e = 1.44269502162933349609375f, kLn2Hi = 0.693147182464599609375f, kLn2Lo = -1.904654212125933550e-9f;
+  const float t = x * -kLog2e, r = fmaf(t, -kLn2Lo, fmaf(t, -kLn2Hi, -x));
+  const float e = __builtin_amdgcn_exp2f(t), d = 1.0f + e;
   const float inv = __builtin_amdgcn_rcpf(d), q = x * inv;
-  return fmaf(fmaf(-d, q, x), inv, q);
+  return fmaf(fmaf(-(e * r), q, fmaf(-d, q, x)), inv, q);
 }
-// gate[0 .. 7] *= sigmoid of themselves
-__device__ __forceinline__ void silu8(float (&gate)[8]) {
-  float most = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(gate[e]));   // a NaN may pass: it stays one either way
-  if (!__any(most >= kSiluNear)) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) gate[e] = silu_near(gate[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) gate[e] = gate[e] / (1.0f + expf(-gate[e]));
-  }
-}
+__device__ __forceinline__ float silu_whole(float x) { return x / (1.0f + expf(-x)); }
 
 template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
 __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(const WideArgs a) {
@@ -148,7 +137,9 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   };
   // What comes from memory and not from the L2 comes late: every stage a wave touches a few of the 128-byte lines that the
   // stage kAhead later will fetch (the workgroups that share a column block's weights or a row block's x in a patch
-  // share out its lines), so that the fetch itself meets the L2.
+  // share out its lines), so that the fetch itself meets the L2.  A lane touches one line a stage, so a wave 64 of them: where a
+  // patch has a single row block, the four waves of 256 and 320 columns have 64 and 80 lines of W each and no lane for x
+  // (which the column blocks' workgroups of the XCD then fetch from the L2 behind whichever of them comes first).
   constexpr int kAhead = 4;
   const int x_share = a.m_blocks > kWdPatchRows ? kWdPatchCols : kWdXcdPlaces / rows_here;
   const int w_lines = (BN + rows_here * kWaves - 1) / (rows_here * kWaves), x_lines = (BM + x_share * kWaves - 1) / (x_share * kWaves);
@@ -270,48 +261,58 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   const int r0 = m0 + 32 * TM * wm;
   __syncthreads();
   unsigned char* mine = lds + wave * (32 * kPitch);
+  // FAR: a gate of the wave is beyond kSiluNear.  That copy stands behind the other one: inside it, tile by tile, it took the
+  // kernel from 20 to 47 KB, and between a model's other kernels a launch waits for its code.
+  auto leave = [&](auto far_tag) {
+    constexpr bool FAR = decltype(far_tag)::value;
 #pragma unroll
-  for (int t = 0; t < TM; ++t) {
+    for (int t = 0; t < TM; ++t) {
 #pragma unroll
-    for (int g = 0; g < TN; g += kGroup) {
+      for (int g = 0; g < TN; g += kGroup) {
 #pragma unroll
-      for (int tn = g; tn < g + kGroup; ++tn) {
-        [[maybe_unused]] float gate[8];
-        if constexpr (EPI == kEpiSiluMul) {
+        for (int tn = g; tn < g + kGroup; ++tn) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) gate[e] = acc[t][tn][e];
-          silu8(gate);
-        }
+          for (int q4 = 0; q4 < kTile / 8; ++q4) {
+            float v[4];
 #pragma unroll
-        for (int q4 = 0; q4 < kTile / 8; ++q4) {
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if constexpr (EPI == kEpiSiluMul) v[e] = gate[4 * q4 + e] * acc[t][tn][4 * q4 + e + 8];
-            else v[e] = acc[t][tn][4 * q4 + e];
+            for (int e = 0; e < 4; ++e) {
+              v[e] = acc[t][tn][4 * q4 + e];
+              if constexpr (EPI == kEpiSiluMul) v[e] = (FAR ? silu_whole(v[e]) : silu_near(v[e])) * acc[t][tn][4 * q4 + e + 8];
+            }
+            unsigned char* to = mine + j * kPitch + (kTile * (tn - g) + 8 * q4 + 4 * h) * kElt;
+            if constexpr (kElt == 2)
+              *reinterpret_cast<uint2*>(to) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            else
+              *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
           }
-          unsigned char* to = mine + j * kPitch + (kTile * (tn - g) + 8 * q4 + 4 * h) * kElt;
-          if constexpr (kElt == 2)
-            *reinterpret_cast<uint2*>(to) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          else
-            *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
         }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-      for (int i = 0; i < kPieces / 2; ++i) {
-        const int idx = 64 * i + lane, rr = idx / kPieces, pc = idx % kPieces;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + rr * kPitch + pc * 16);
-        const int row = r0 + 32 * t + rr, col = c0 + kTile * g + pc * (16 / kElt);
-        if (row < M && col < n_out) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * a.ldo + col) = v;
+        for (int i = 0; i < kPieces / 2; ++i) {
+          const int idx = 64 * i + lane, rr = idx / kPieces, pc = idx % kPieces;
+          const u32x4 v = *reinterpret_cast<const u32x4*>(mine + rr * kPitch + pc * 16);
+          const int row = r0 + 32 * t + rr, col = c0 + kTile * g + pc * (16 / kElt);
+          if (row < M && col < n_out) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * a.ldo + col) = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+  };
+  float most = 0.f;
+  if constexpr (EPI == kEpiSiluMul) {
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(acc[t][tn][e]));   // a NaN may pass: it stays one either way
   }
+  if (__builtin_expect(EPI != kEpiSiluMul || !__any(most >= kSiluNear), 1)) leave(std::false_type{});
+  else if constexpr (EPI == kEpiSiluMul) leave(std::true_type{});
 }
 
 template <int WM, int WN, int TM, int TN, int EPI, typename TOut>

@@ -427,8 +427,9 @@ struct CapArgs {
 // rows share a tile (QB 2, where there are waves enough), values come in pieces of 16 bytes, keys of the next tile are
 // fetched while this one's probabilities are made and values while its scores are, masks are worked out in the tiles at
 // the ends only, sums are rescaled only where a maximum moved, and the lanes' sums meet once at the end.  A layer of 2,048
-// rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 89 now; 256 rows 25 -> 16; eight decoded rows
-// behind 2,048 keys 21 -> 17.  (Portions of heads up to 128 are held to the registers of two waves a SIMD.)
+// rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 89 now (184 and 110 between the other kernels of a
+// prompt; the masks that each block of sixteen rows has of its own are 4 and 8 of these); 256 rows 25 -> 16; eight decoded
+// rows behind 2,048 keys 21 -> 17.  (Portions of heads up to 128 are held to the registers of two waves a SIMD.)
 template <int KC, int VC, bool HEADS, int WAVES, int QB>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(!HEADS && KC <= 4 && VC <= 8 ? 2 : 1)))
 void attn_softcap_mfma_kernel(const CapArgs a) {

@@ -6,22 +6,22 @@
 // shape, N 19,456, K 2,560, weights cold):
 //
 //   * The matrix cores, at the clock that the chip holds when all 256 compute units multiply real data (1.75 to 1.84 PFLOP/s):
-//     the loop alone runs at 1.53, a whole launch of 8,192 rows at 1.30 (628 us; the library's product and the activation
-//     kernel 771, gemm_tiles 793).
+//     the loop alone runs at 1.53, a whole launch of 8,192 rows at 1.25 (652 us; the library's product and the activation
+//     kernel 763, gemm_tiles 760; cards differ by 7 %).
 //   * Turns: a launch lasts as many turns of its workgroups as they fill the compute units.  gate|up at 2,048 rows is 608
-//     tiles of 256 x 256, three turns for 2.4; 256 x 320 is 488, two turns for 1.9: 167 us against gemm_tiles' 200.  So there are
+//     tiles of 256 x 256, three turns for 2.4; 256 x 320 is 488, two turns for 1.9: 172 us against gemm_tiles' 222.  So there are
 //     twelve shapes, and the caller's plan takes the one whose turns are shortest (ops.wide_plan).
 //   * Latency of what comes from memory: with two stages a fetch has one stage's time (1.2 to 1.8 us), which a miss of the L2
 //     under load does not keep to.  Every wave therefore touches, four stages ahead, a few of the 128-byte lines that its
 //     XCD's workgroups will fetch (a dword a line, into a corner of LDS that nobody reads): 2,048 rows 223 -> 186 us, 8,192
-//     rows 679 -> 600.  More stages of 32 k instead (rows of 64 bytes) were 6 to 8 % slower: half lines cost the fetch path
+//     rows 679 -> 600 in the form that the kernel had then.  More stages of 32 k instead (rows of 64 bytes) were 6 to 8 % slower: half lines cost the fetch path
 //     twice the requests.
 //   * The step's operand reads (4 cycles of LDS each) and loads are pinned between its products (sched_barrier): the next
 //     step's operands are read while this step multiplies, the barrier of a stage stands in its last step, behind which
 //     the first operands of the next stage are read and the place of this one is filled again.
 //   * The activation of a workgroup's 40 thousand pairs: the same error as expf and a divide without their cases for what
-//     leaves the floats, 172 instead of 178 us at 2,048 rows in one run (the bare exponential and reciprocal of the vector
-//     unit would be 167, with errors up to 63 ulp below zero).
+//     leaves the floats, 167 us at 2,048 rows where the bare exponential and reciprocal of the vector unit (errors up to 63
+//     ulp below zero) take 163 in the same run.
 //
 // Four waves (one a SIMD) or eight, measured alike in the loop; eight hold the accumulators of 256 x 320 in 256 registers each.
 #include "common.h"

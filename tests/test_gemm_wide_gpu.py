@@ -133,3 +133,25 @@ def test_blocks_of_several_patches(shape, row_blocks, col_blocks):
     assert _rel(ops.gemm_wide(x, w, shape=shape), want) < 2.0 ** -8
     stack = ops.gemm_wide(x, w, torch.float32, shape=shape, splits=2)
     assert _rel(stack.sum(0), want) < 1e-5
+
+
+@pytest.mark.parametrize("shape", [(128, 64), (192, 320), (256, 320)])
+@pytest.mark.parametrize("scale", [79.875, 80.0, 300.0])
+def test_one_wave_with_gates_beyond_the_short_form(shape, scale):
+    """Gates of two rows reach `scale` with either sign, all others stay within 1: their waves take the whole exponential and
+    division from 80 on, beside waves that do not.  Both forms are off by 3 ulp of a float at most, so every result is the
+    64-bit one rounded to bfloat16, or its neighbour where that lies at a middle.  exp(-x) of a float is infinite from 2^128
+    (x below -88.72) on, where the result is -0 instead of x / (1 + exp(-x)), 89 2^-128 at most."""
+    from arle_amd.kernels import ops
+
+    M, n = 300, 640
+    x = torch.zeros(M, 64, dtype=torch.bfloat16, device="cuda")
+    x[:, 0] = torch.linspace(-1, 1, M, device="cuda").bfloat16()
+    x[37, 0], x[290, 0] = scale, -scale
+    w = torch.zeros(n // 32, 2, 16, 64, dtype=torch.bfloat16, device="cuda")
+    w[:, 0, :, 0] = torch.linspace(0.0625, 1, n // 2, device="cuda").bfloat16().view(n // 32, 16)
+    x[:, 1], w[:, 1, :, 1] = 1.0, 1.0
+    gate = x[:, :1].double() @ w[:, 0, :, 0].reshape(1, -1).double()
+    want = gate / (1 + torch.exp(-gate))
+    got = ops.gemm_wide(x, w.reshape(n, 64), epilogue=ops.EPI_SILU_MUL, shape=shape).double()
+    assert torch.allclose(got, want, rtol=2.0 ** -8 * (1 + 2.0 ** -10), atol=89 * 2.0 ** -128)

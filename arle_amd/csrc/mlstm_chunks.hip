@@ -14,16 +14,20 @@
 //   mlstm_chunk_gates   a wave a (chunk, head): gates, b, e and the running maximum of e by scans over the lanes
 //   mlstm_chunk_carry   a workgroup a (request, head, 32 columns of Dv) walks the request's chunks with its part of S in
 //                       accumulators, leaves S_0, n_0 and m_0 of every chunk; the next chunk's k and v are fetched meanwhile
+//   mlstm_chunk_sums,   the same for longer requests in two kernels without a chain of products: see there
+//   mlstm_chunk_scan
 //   mlstm_chunk_out     a workgroup a (chunk, head): scores, weights, both products, the denominator, the head norm, the
 //                       norm weight and the output gate
 //
-// Measured on MI355X, 2,048 rows, 20 heads, D = Dv = 128, us a layer: 5 + 86 + 61 where the token-by-token kernels take 125
-// (gates) + 708 (memory) + 18 (output); the error of a layer's output against 64 bits is the same (2e-7 to 6e-6 either way).
+// Measured on MI355X, 2,048 rows, 20 heads, D = Dv = 128, us a layer: 5 + 42 + 61 (5 + 86 + 61 with the walk) where the
+// token-by-token kernels take 125 (gates) + 708 (memory) + 18 (output); the error of a layer's output against 64 bits is the same (2e-7 to 6e-6 either way).
 // A NaN or an infinity in a row's v spoils that row and the later ones, as token by token (where an infinity meets a
 // state's column with both signs).  The second product would carry it to the chunk's earlier rows too, as a weight of zero
 // times it: it takes zeros for such values, and the rows from the first one on are made NaN behind it.
 #include "chunks.h"
 #include "common.h"
+
+#include <type_traits>
 
 namespace arle {
 
@@ -198,6 +202,135 @@ __global__ __launch_bounds__(KD* kWave) void mlstm_chunk_carry_kernel(const Mlst
 #pragma unroll
   for (int r = 0; r < 16; ++r) s_state[static_cast<int64_t>(d_of(r)) * Dv + i] = S[r];
   if (z == 0 && half == 0) n_state[i] = n;      // m goes back in the last kernel: other workgroups of the head may still read it here
+}
+
+// The same walk for requests of several chunks, in two kernels: the chunks' own sums side by side, then the states in front
+// of them.  With top_c the largest e of chunk c, U_c = sum_s exp(e_s - top_c) k_s v_s^T needs nothing of the chunks before it,
+// and S_(c+1) = exp(m_c + b_c - m_(c+1)) S_c + exp(top_c + b_c - m_(c+1)) U_c is element by element.
+//
+// The sums: a workgroup a (chunk, head), a wave 32 rows (d) of U, 32 columns after another.  The products of a chunk and head
+// are 2 MFLOP; what bounds it is the fetch of k and v, and U on its way out.
+template <int KD>
+__global__ __launch_bounds__(KD* kWave) void mlstm_chunk_sums_kernel(const MlstmChunkArgs a) {
+  constexpr int D = 32 * KD;
+  __shared__ float weights[KD][kChunkRows];
+  const int item = blockIdx.x, h = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, i = lane & 31, half = lane >> 5;
+  const ChunkAt c = find_chunk(a.seg_row0, a.segments, item);
+  if (c.rows == 0) return;                    // the whole workgroup
+  const int Dv = a.Dv, H = a.H;
+  const int64_t at = static_cast<int64_t>(item) * H + h;
+  // rows that are not there have e = -inf and weigh 0
+  const float2 e = *reinterpret_cast<const float2*>(a.rows + at * kChunkRows + lane);
+  const double top = a.ends[at].top;
+  const float* kp = a.k + static_cast<int64_t>(h) * D + 32 * wave + i;
+  const float* vp = a.v + static_cast<int64_t>(h) * Dv + i;
+  float k[32], v[2][32];
+  auto row = [&](int j) { return static_cast<int64_t>(c.row0 + min(j + 32 * half, c.rows - 1)) * a.row_stride; };
+#pragma unroll
+  for (int j = 0; j < 32; ++j) k[j] = kp[row(j)];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) v[0][j] = vp[row(j)];
+  weights[wave][lane] = expf(static_cast<float>(static_cast<double>(e.x) + static_cast<double>(e.y) - top));
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float n_sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    k[j] *= weights[wave][j + 32 * half];
+    n_sum += k[j];
+  }
+  n_sum += __shfl_xor(n_sum, 32, kWave);
+  if (half == 0) a.n0[at * D + 32 * wave + i] = n_sum;
+  float* u = a.s0 + (at * D + 32 * wave) * Dv + i;
+#pragma unroll
+  for (int z = 0; z < 4; ++z) {
+    if (32 * z < Dv) {
+      if (32 * z + 32 < Dv) {
+#pragma unroll
+        for (int j = 0; j < 32; ++j) v[(z + 1) & 1][j] = vp[row(j) + 32 * z + 32];
+      }
+      f32x16 U;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) U[r] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) U = __builtin_amdgcn_mfma_f32_32x32x2f32(k[j], v[z & 1][j], U, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) u[static_cast<int64_t>(8 * (r / 4) + 4 * half + r % 4) * Dv + 32 * z] = U[r];
+    }
+  }
+}
+
+// The states: a thread four elements of a (request, head)'s S through all its chunks, whose sums it fetches kScanAhead chunks
+// ahead and whose places take S_0 (the last blockIdx.z: n, an element a thread).  Bound by reading U and writing S_0, 84 MB
+// a layer at 2,048 rows of 20 heads.
+constexpr int kScanThreads = 256, kScanAhead = 8;
+// Rows of the longest request from which on sums and scan take the walk's place.  MI355X, all kernels of a layer, us, walk /
+// sums and scan: 20 heads of 128 one request of 256 rows 41.8 / 43.3, 320 44.9 / 44.9, 512 54.7 / 48.6, 1,024 84.7 / 67.8, 2,048
+// 149.8 / 108.1, 8,192 546 / 392, eight of 512 182 / 184; 8 heads of 64 256 rows 30.1 / 26.7, 2,048 108 / 43; 4 heads of
+// 128 256 rows 38.0 / 37.9, 2,048 115 / 52, eight of 256 43.8 / 48.6.
+constexpr int kSumsMinRows = 384;
+
+__global__ __launch_bounds__(kScanThreads) void mlstm_chunk_scan_kernel(const MlstmChunkArgs a, int D) {
+  const int seg = blockIdx.x, h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
+  const int Dv = a.Dv, H = a.H;
+  const int row0 = a.seg_row0[seg], rows = a.seg_row0[seg + 1] - row0;
+  if (rows <= 0) return;
+  int item = 0;
+  for (int s = 0; s < seg; ++s) item += (a.seg_row0[s + 1] - a.seg_row0[s] + kChunkRows - 1) / kChunkRows;
+  const int chunks = (rows + kChunkRows - 1) / kChunkRows;
+  const int64_t slot = a.seg_slot[seg], first = static_cast<int64_t>(item) * H + h;
+  float m = a.m_state[slot * H + h];      // it goes back in the last kernel: other workgroups of the head may still read it here
+  auto walk = [&](auto* state, auto* sums, int64_t a_chunk, bool tells, auto scaled) {
+    using T = std::remove_reference_t<decltype(*state)>;
+    T S = *state, ahead[kScanAhead];
+    ChunkEnd ends[kScanAhead];
+#pragma unroll
+    for (int j = 0; j < kScanAhead; ++j) {
+      const int c = min(j, chunks - 1);
+      ahead[j] = sums[c * a_chunk];
+      ends[j] = a.ends[first + static_cast<int64_t>(c) * H];
+    }
+    for (int c0 = 0; c0 < chunks; c0 += kScanAhead) {
+#pragma unroll
+      for (int j = 0; j < kScanAhead; ++j) {
+        const int c = c0 + j;
+        if (c < chunks) {
+          const T u = ahead[j];
+          const ChunkEnd end = ends[j];
+          const int next = min(c + kScanAhead, chunks - 1);      // past the end: the last one again, whose place nobody has written yet
+          if (c + kScanAhead < chunks) {
+            ahead[j] = sums[next * a_chunk];
+            ends[j] = a.ends[first + static_cast<int64_t>(next) * H];
+          }
+          const float m_end = static_cast<float>(end.b + fmax(static_cast<double>(m), end.top));
+          const float keep = expf(static_cast<float>(static_cast<double>(m) + end.b - static_cast<double>(m_end)));
+          const float take = expf(static_cast<float>(end.top + end.b - static_cast<double>(m_end)));
+          sums[c * a_chunk] = S;
+          if (tells) {
+            const int64_t at = first + static_cast<int64_t>(c) * H;
+            a.m0[at * 2] = m;
+            a.m0[at * 2 + 1] = m_end;
+          }
+          S = scaled(S, keep, u, take);
+          m = m_end;
+        }
+      }
+    }
+    *state = S;
+  };
+  if (z + 1 < static_cast<int>(gridDim.z)) {
+    const int e = z * kScanThreads + tid;
+    if (e >= D * Dv / 4) return;
+    walk(reinterpret_cast<float4*>(a.s_state + (slot * H + h) * D * Dv) + e, reinterpret_cast<float4*>(a.s0 + first * D * Dv) + e,
+         static_cast<int64_t>(H) * D * Dv / 4, z == 0 && tid == 0, [](float4 S, float keep, float4 u, float take) {
+           return float4{fmaf(S.x, keep, u.x * take), fmaf(S.y, keep, u.y * take), fmaf(S.z, keep, u.z * take), fmaf(S.w, keep, u.w * take)};
+         });
+  } else if (tid < D) {
+    walk(a.n_state + (slot * H + h) * D + tid, a.n0 + first * D + tid, static_cast<int64_t>(H) * D, false,
+         [](float S, float keep, float u, float take) { return fmaf(S, keep, u * take); });
+  }
 }
 
 constexpr int kOutWaves = 4;
@@ -389,9 +522,15 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
 }
 
 template <int KD>
-int launch_chunks(const MlstmChunkArgs& a, hipStream_t s) {
+int launch_chunks(const MlstmChunkArgs& a, int longest, hipStream_t s) {
   mlstm_chunk_gates_kernel<<<dim3(a.items, a.H), kWave, 0, s>>>(a);
-  mlstm_chunk_carry_kernel<KD><<<dim3(a.segments, a.H, a.Dv / 32), KD * kWave, 0, s>>>(a);
+  if (longest >= kSumsMinRows) {
+    constexpr int D = 32 * KD;
+    mlstm_chunk_sums_kernel<KD><<<dim3(a.items, a.H), KD * kWave, 0, s>>>(a);
+    mlstm_chunk_scan_kernel<<<dim3(a.segments, a.H, (D * a.Dv / 4 + kScanThreads - 1) / kScanThreads + 1), kScanThreads, 0, s>>>(a, D);
+  } else {
+    mlstm_chunk_carry_kernel<KD><<<dim3(a.segments, a.H, a.Dv / 32), KD * kWave, 0, s>>>(a);
+  }
   mlstm_chunk_out_kernel<KD><<<dim3(a.items, a.H), kOutWaves * kWave, 0, s>>>(a);
   return launch_status();
 }
@@ -414,7 +553,7 @@ extern "C" long long arle_mlstm_chunks_bytes(int items, int H, int D, int Dv) {
 extern "C" int arle_mlstm_chunks(const float* q, const float* k, const float* v, const float* gate, long long row_stride,
                                  const float* gates, long long gates_stride, const float* bias_i, const float* bias_f, float cap,
                                  float* s_state, float* n_state, float* m_state, const int* seg_row0, const int* seg_slot,
-                                 int segments, int items, int H, int D, int Dv, void* workspace, const void* weight, int w_dtype,
+                                 int segments, int items, int longest, int H, int D, int Dv, void* workspace, const void* weight, int w_dtype,
                                  void* out, int out_dtype, float eps, void* stream) {
   if (segments == 0 || items == 0) return 0;
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
@@ -432,10 +571,11 @@ extern "C" int arle_mlstm_chunks(const float* q, const float* k, const float* v,
   a.rows = reinterpret_cast<ChunkRow*>(at), at += pairs * kChunkRows * sizeof(ChunkRow);
   a.m0 = reinterpret_cast<float*>(at);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!aligned(s_state)) longest = 0;      // the states' kernel reads four elements at a time
   switch (D / 32) {
-    case 1: return launch_chunks<1>(a, s);
-    case 2: return launch_chunks<2>(a, s);
-    case 3: return launch_chunks<3>(a, s);
-    default: return launch_chunks<4>(a, s);
+    case 1: return launch_chunks<1>(a, longest, s);
+    case 2: return launch_chunks<2>(a, longest, s);
+    case 3: return launch_chunks<3>(a, longest, s);
+    default: return launch_chunks<4>(a, longest, s);
   }
 }

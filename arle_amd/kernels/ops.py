@@ -1762,9 +1762,10 @@ def mlstm_chunks_preferred(longest: int, tokens: int, segments: int, heads: int,
 
 
 def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_state, seg_row0, seg_slot, weight, eps: float,
-                 out_dtype, *, heads: int, key_dim: int, value_dim: int):
+                 out_dtype, *, heads: int, key_dim: int, value_dim: int, longest: int | None = None):
     """mlstm_scan and mlstm_output over chunks of 64 rows, the products on the 32-bit matrix instructions.  qkvg float32
-    [T, 2 H D + 2 H Dv]: q, k, v and the output gate side by side.  Returns [T, H * Dv]."""
+    [T, 2 H D + 2 H Dv]: q, k, v and the output gate side by side; longest: rows of the longest segment, where the caller
+    knows them (any step is right with any value; short ones are faster with theirs).  Returns [T, H * Dv]."""
     _gpu(qkvg, gates, bias_i, bias_f, s_state, n_state, m_state, seg_row0, seg_slot, weight)
     H, D, Dv = heads, key_dim, value_dim
     _rows(qkvg, "qkvg")
@@ -1791,8 +1792,8 @@ def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_st
     at = lambda column: qkvg.data_ptr() + 4 * column
     lib.call("arle_mlstm_chunks", at(0), at(H * D), at(2 * H * D), at(2 * H * D + width), qkvg.stride(0), gates.data_ptr(),
              gates.stride(0), bias_i.data_ptr(), bias_f.data_ptr(), float(cap), s_state.data_ptr(), n_state.data_ptr(),
-             m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), segments, items, H, D, Dv, scratch.data_ptr(),
-             weight.data_ptr(), _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
+             m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), segments, items, tokens if longest is None else int(longest), H, D, Dv,
+             scratch.data_ptr(), weight.data_ptr(), _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
     return out
 
 

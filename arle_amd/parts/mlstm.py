@@ -90,7 +90,7 @@ class MLSTMMixer(Part):
         if not self.rt.is_f32 and ops.mlstm_chunks_preferred(batch.max_qlen, x.shape[0], batch.seg_slot.numel(), self.H, self.D, self.Dv):
             y = ops.mlstm_chunks(p, gates, self.i_bias, self.f_bias, self.cap, cache["S"].state, cache["n"].state, cache["m"].state,
                                  batch.seg_row0, batch.seg_slot, self.norm, self.eps, self.rt.act_dtype, heads=self.H,
-                                 key_dim=self.D, value_dim=self.Dv)
+                                 key_dim=self.D, value_dim=self.Dv, longest=batch.max_qlen)
             return self.o(y, out_dtype=torch.float32, partials_ok=True)
         q, k, v, g = p[:, :qk], p[:, qk:2 * qk], p[:, 2 * qk:2 * qk + vw], p[:, 2 * qk + vw:]
         num, nq, coefs = ops.mlstm_scan(q, k, v, gates, self.i_bias, self.f_bias, self.cap, cache["S"].state,

@@ -1,18 +1,23 @@
 // bfloat16 matrix product for prompt portions:  C[M,N] = X[M,K] . W[N,K]^T, both row-major, K a multiple of 64.
 //
-// A workgroup owns BM rows x BN columns (128 to 256 x 64 to 320) and walks K in stages of 64: the stage's rows of X and W, 128
-// bytes each, go from memory straight into LDS (global_load_lds, no registers on the way), two stages deep, and every wave
-// feeds v_mfma_f32_32x32x16_bf16 from there.  What bounds it, and what was done about that (MI355X, gate|up of the Qwen3-4B
-// shape, N 19,456, K 2,560, weights cold):
+// A workgroup owns BM rows x BN columns (64 to 256 x 64 to 320) and walks K in stages of 64: the stage's rows of X and W, 128
+// bytes each, go from memory straight into LDS (global_load_lds, no registers on the way), two to five stages deep, and every
+// wave feeds v_mfma_f32_32x32x16_bf16 from there.  What bounds it, and what was done about that (MI355X, gate|up of the
+// Qwen3-4B shape, N 19,456, K 2,560, weights cold):
 //
 //   * The matrix cores, at the clock that the chip holds when all 256 compute units multiply real data (1.75 to 1.84 PFLOP/s):
 //     the loop alone runs at 1.53, a whole launch of 8,192 rows at 1.25 (652 us; the library's product and the activation
 //     kernel 763, gemm_tiles 760; cards differ by 7 %).
 //   * Turns: a launch lasts as many turns of its workgroups as they fill the compute units.  gate|up at 2,048 rows is 608
 //     tiles of 256 x 256, three turns for 2.4; 256 x 320 is 488, two turns for 1.9: 172 us against gemm_tiles' 222.  So there are
-//     twelve shapes, and the caller's plan takes the one whose turns are shortest (ops.wide_plan).
-//   * Latency of what comes from memory: with two stages a fetch has one stage's time (1.2 to 1.8 us), which a miss of the L2
-//     under load does not keep to.  Every wave therefore touches, four stages ahead, a few of the 128-byte lines that its
+//     nineteen shapes, and the caller's plan takes the one whose turns are shortest (ops.wide_plan).
+//   * Few rows: W streams at what the workgroups have in flight.  Shapes whose stages are small keep three to five of them in the
+//     LDS (80 to 150 KB): a stage's fetch has two to four stages' time.  9 to 256 rows are then W at 4 to 4.6 TB/s: 64 rows 26.3 us
+//     with two stages and lines touched ahead 32.7 (128 x 96, 97 rows: 30.6 / 34.9; 128 x 160, 160 rows 33.4 / 37.7); a sixth stage and
+//     more change nothing.  From operand tiles, whose kilobytes lie whole in memory where rows are 128 bytes each 5 KB apart,
+//     64 rows take 23.7 us for 26.8, 128 rows 29.5 for 32.7, 256 rows 35.0 for 38.7; from 544 rows on the two are level.
+//   * Latency of what comes from memory in the large shapes: with two stages a fetch has one stage's time (1.2 to 1.8 us), which
+//     a miss of the L2 under load does not keep to.  There every wave touches, four stages ahead, a few of the 128-byte lines that its
 //     XCD's workgroups will fetch (a dword a line, into a corner of LDS that nobody reads): 2,048 rows 223 -> 186 us, 8,192
 //     rows 679 -> 600 in the form that the kernel had then.  More stages of 32 k instead (rows of 64 bytes) were 6 to 8 % slower: half lines cost the fetch path
 //     twice the requests.
@@ -51,6 +56,7 @@ struct WideArgs {
   int m_blocks, n_blocks;
   int stages_per_split;
   int64_t split_stride;
+  int tiled;               // w holds operand tiles (see below) instead of rows
 };
 
 #pragma clang diagnostic push
@@ -83,14 +89,16 @@ __device__ __forceinline__ float silu_near(float x) {
 }
 __device__ __forceinline__ float silu_whole(float x) { return x / (1.0f + expf(-x)); }
 
-template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
-__global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(const WideArgs a) {
+template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut>
+__global__ __launch_bounds__(WM* WN* kWave, (WM * WN + 3) / 4) void gemm_wide_kernel(const WideArgs a) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, kWaves = WM * WN;
   constexpr int kRowsALoad = 8 * kWaves;                        // rows that one load of every wave brings
-  static_assert(BM % kRowsALoad == 0 && BN % kRowsALoad == 0, "whole loads");
+  static_assert(BM % kRowsALoad == 0 && BN % kRowsALoad == 0 && kRowsALoad % 16 == 0, "whole loads, of whole rounds of the pieces' order");
   constexpr int LX = BM / kRowsALoad, LA = (BM + BN) / kRowsALoad;
   constexpr int kStage = (BM + BN) * 128;
-  constexpr int kProducts = TM * TN, kReads = TM + TN, kReadsASlot = (kReads + kProducts - 2) / (kProducts - 1);
+  constexpr int kProducts = TM * TN, kReads = TM + TN;
+  constexpr int kSlots = kProducts > 1 ? kProducts - 1 : 1, kReadsASlot = (kReads + kSlots - 1) / kSlots;   // reads go behind the products 1, 2, ... (behind the only one)
+  constexpr bool kTouch = NS == 2;
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -117,7 +125,11 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   const int st0 = blockIdx.y * a.stages_per_split;
   const int n_st = min(a.stages_per_split, all_stages - st0);
   const uint16_t* xb = a.x + static_cast<int64_t>(m0) * a.ldx + static_cast<int64_t>(st0) * kWdK;
-  const uint16_t* wb = a.w + static_cast<int64_t>(n0) * a.ldw + static_cast<int64_t>(st0) * kWdK;
+  // a tile of W: 16 columns x 32 k, 1 KB; a stage's k of 16 columns are two of them side by side
+  const int tile_row = a.K / 32 * 512;     // elements between the tiles of neighbouring sixteens of columns
+  const int w_step = a.tiled ? 1024 : kWdK;
+  const uint16_t* wb = a.tiled ? a.w + static_cast<int64_t>(n0 / 16) * tile_row + static_cast<int64_t>(st0) * w_step
+                               : a.w + static_cast<int64_t>(n0) * a.ldw + static_cast<int64_t>(st0) * kWdK;
 
   // a load brings 8 rows of 128 bytes; piece lane % 8 of an LDS row holds the row's k piece (lane % 8) ^ (row / 2 % 8),
   // so that sixteen lanes of an operand read never share a bank
@@ -129,6 +141,10 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
     const bool of_x = i < LX;
     const int row = kRowsALoad * (of_x ? i : i - LX) + lr;
     off[i] = static_cast<uint32_t>(min(row, of_x ? M - 1 - m0 : N - 1 - n0)) * static_cast<uint32_t>((of_x ? a.ldx : a.ldw) * 2) + piece * 16;
+    if (!of_x && a.tiled) {      // a wave's load is a tile
+      const int tile = (i - LX) * kWaves + wave;
+      off[i] = static_cast<uint32_t>(min(tile / 2, (N - n0) / 16 - 1)) * static_cast<uint32_t>(tile_row * 2) + (tile % 2) * 1024 + lane * 16;
+    }
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + 1024u * wave);
@@ -140,23 +156,30 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   // share out its lines), so that the fetch itself meets the L2.  A lane touches one line a stage, so a wave 64 of them: where a
   // patch has a single row block, the four waves of 256 and 320 columns have 64 and 80 lines of W each and no lane for x
   // (which the column blocks' workgroups of the XCD then fetch from the L2 behind whichever of them comes first).
-  constexpr int kAhead = 4;
+  constexpr int kAhead = 4;      // with two stages only: three and more bring what comes late themselves
   const int x_share = a.m_blocks > kWdPatchRows ? kWdPatchCols : kWdXcdPlaces / rows_here;
   const int w_lines = (BN + rows_here * kWaves - 1) / (rows_here * kWaves), x_lines = (BM + x_share * kWaves - 1) / (x_share * kWaves);
   const uint16_t* touch_from;
-  if (lane < w_lines)
-    touch_from = wb + static_cast<int64_t>(min((patch_row * kWaves + wave) * w_lines + lane, N - 1 - n0)) * a.ldw;
-  else
+  int touch_step = kWdK;
+  if (lane < w_lines) {
+    const int line = min((patch_row * kWaves + wave) * w_lines + lane, N - 1 - n0);
+    touch_from = wb + (a.tiled ? static_cast<int64_t>(line / 16) * tile_row + line % 16 * 64 : static_cast<int64_t>(line) * a.ldw);
+    touch_step = w_step;
+  } else {
     touch_from = xb + static_cast<int64_t>(min((((nb / kWdXcds) % x_share) * kWaves + wave) * x_lines + min(lane - w_lines, x_lines - 1), M - 1 - m0)) * a.ldx;
+  }
   const bool touches = lane < w_lines + x_lines;
   const uint32_t touch_at = __builtin_amdgcn_readfirstlane(
-      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + 2 * kStage + 256u * wave);
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + NS * kStage + 256u * wave);
   auto touch = [&](int stages) {
-    if (touches) wide_touch(touch_from + stages * kWdK, touch_at);
+    if (touches) wide_touch(touch_from + stages * touch_step, touch_at);
   };
-  uint32_t at[4];
+  uint32_t at[4], w_piece[4];
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) at[kk] = j * 128 + (((2 * kk + h) ^ ((j >> 1) & 7)) * 16);
+  for (int kk = 0; kk < 4; ++kk) {
+    at[kk] = j * 128 + (((2 * kk + h) ^ ((j >> 1) & 7)) * 16);
+    w_piece[kk] = a.tiled ? (j >> 4) * 2048 + kk * 512 + h * 256 + (j & 15) * 16 : at[kk];   // 16 lanes read 256 bytes side by side
+  }
   const uint32_t x_at = wm * TM * 4096, w_at = BM * 128 + wn * TN * 4096;
 
   f32x16 acc[TM][TN];
@@ -171,81 +194,92 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
     if (i < TM)
       fx[set][i] = *reinterpret_cast<const bf16x8*>(lds + buf + x_at + at[kk] + 4096 * i);
     else
-      fw[set][i - TM] = *reinterpret_cast<const bf16x8*>(lds + buf + w_at + at[kk] + 4096 * (i - TM));
+      fw[set][i - TM] = *reinterpret_cast<const bf16x8*>(lds + buf + w_at + w_piece[kk] + 4096 * (i - TM));
   };
 
   constexpr int kEarly = (LA + 1) / 2;   // loads of a stage that go out in the step that frees its place; the others in the step after it
+  static_assert((NS - 2) * LA + kEarly < 64, "the loads in flight fit the counter");
 #pragma unroll
-  for (int i = 0; i < LA; ++i) load(i, 0, xb, wb);
-  if (n_st > 1) {
+  for (int st = 0; st < NS - 1; ++st) {
+    if (st < n_st) {
 #pragma unroll
-    for (int i = 0; i < kEarly; ++i) load(i, kStage, xb + kWdK, wb + kWdK);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kEarly) : "memory");
+      for (int i = 0; i < LA; ++i) load(i, st * kStage, xb + st * kWdK, wb + st * w_step);
+    }
+  }
+  if (n_st >= NS) {
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) load(i, (NS - 1) * kStage, xb + (NS - 1) * kWdK, wb + (NS - 1) * w_step);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * LA + kEarly) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  if (n_st > 3) touch(2), touch(3);
+  if (kTouch && n_st > 3) touch(2), touch(3);
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int i = 0; i < kReads; ++i) read_one(i, 0, 0, 0);
 
-  // One stage: four steps of 16 k.  NEXT: what is still to be fetched (2: the rest of stage s + 1 and the first part of
-  // s + 2; 1: the former only; 0: nothing, and no stage follows)
-  auto stage = [&](auto next_tag, uint32_t buf) {
-    constexpr int NEXT = decltype(next_tag)::value;
+  // One stage, four steps of 16 k, and what it sends for later: the rest of stage s + NS - 1 in its first step, to the place
+  // of the stage before it, and the first part of s + NS in its last, to its own.  LEFT: the stages that follow it, up to NS.
+  // TOUCH: it touches the lines of stage s + kAhead.
+  uint32_t before = (NS - 1) * kStage, buf = 0, next = kStage;
+  auto stage = [&](auto left_tag, auto touch_tag) {
+    constexpr int LEFT = decltype(left_tag)::value;
+    constexpr bool TOUCH = decltype(touch_tag)::value;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int set = kk & 1;
 #pragma unroll
       for (int m = 0; m < kProducts; ++m) {
-        if (kk == 3 && m == 1 && NEXT > 0) {
-          // every wave has its operands of this stage, and its pieces of the next one have landed
-          // (a line that was touched for later may still be on its way)
-          if (NEXT == 3) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)" ::: "memory");
-          else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        if (kk == 3 && m == (kProducts > 1 ? 1 : 0) && LEFT > 0) {
+          // every wave has its operands of this stage, and its pieces of the next one have landed: what was sent behind those
+          // may still be on its way
+          constexpr int kFlying = (LEFT - 1 < NS - 2 ? LEFT - 1 : NS - 2) * LA + (TOUCH ? 1 : 0);
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT > 0 ? kFlying : 0) : "memory");
           __builtin_amdgcn_s_barrier();
           __builtin_amdgcn_sched_barrier(0);
         }
         const int t = m % TM, tn = m / TM;
         acc[t][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][tn], fx[set][t], acc[t][tn], 0, 0, 0);
-        // the next step's operands behind the products 1, 2, ...
+        // the next step's operands
+        const int slot = kProducts > 1 ? m - 1 : 0;
 #pragma unroll
-        for (int r = (m - 1) * kReadsASlot; m > 0 && r < m * kReadsASlot && r < kReads; ++r) {
+        for (int r = slot * kReadsASlot; slot >= 0 && r < (slot + 1) * kReadsASlot && r < kReads; ++r) {
           if (kk < 3) read_one(r, set ^ 1, kk + 1, buf);
-          else if (NEXT > 0) read_one(r, set ^ 1, 0, kStage - buf);
+          else if (LEFT > 0) read_one(r, set ^ 1, 0, next);
         }
-        if (kk == 3 && NEXT > 1 && m >= 1) {
+        if (kk == 3 && LEFT >= NS && slot >= 0) {
 #pragma unroll
           for (int i = 0; i < kEarly; ++i)
-            if (1 + i * (kProducts - 1) / kEarly == m) load(i, buf, xb + 2 * kWdK, wb + 2 * kWdK);
+            if (i * kSlots / kEarly == slot) load(i, buf, xb + NS * kWdK, wb + NS * w_step);
         }
-        if (kk == 0 && NEXT > 0) {
+        if (kk == 0 && LEFT >= NS - 1) {
 #pragma unroll
           for (int i = kEarly; i < LA; ++i)
-            if ((i - kEarly) * kProducts / (LA - kEarly) == m) load(i, kStage - buf, xb + kWdK, wb + kWdK);
+            if ((i - kEarly) * kProducts / (LA - kEarly) == m) load(i, before, xb + (NS - 1) * kWdK, wb + (NS - 1) * w_step);
         }
-        if (kk == 1 && NEXT == 3 && m == 1) touch(kAhead);
+        if (kk == 1 && TOUCH && slot == 0) touch(kAhead);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    before = buf, buf = next, next = next + kStage == NS * kStage ? 0 : next + kStage;
+    xb += kWdK, wb += w_step;
   };
-  uint32_t buf = 0;
+  constexpr std::false_type plain{};
   int s = 0;
-  for (; s + kAhead < n_st; ++s) {
-    stage(std::integral_constant<int, 3>{}, buf);
-    buf = kStage - buf;
-    xb += kWdK, wb += kWdK, touch_from += kWdK;
+  if constexpr (kTouch) {
+    for (; s + kAhead < n_st; ++s) {
+      stage(std::integral_constant<int, NS>{}, std::true_type{});
+      touch_from += touch_step;
+    }
   }
-  for (; s + 2 < n_st; ++s) {
-    stage(std::integral_constant<int, 2>{}, buf);
-    buf = kStage - buf;
-    xb += kWdK, wb += kWdK;
-  }
-  if (s + 1 < n_st) {
-    stage(std::integral_constant<int, 1>{}, buf);
-    buf = kStage - buf;
-  }
-  stage(std::integral_constant<int, 0>{}, buf);
+  for (; s + NS < n_st; ++s) stage(std::integral_constant<int, NS>{}, plain);
+  const int left = n_st - 1 - s;
+  static_assert(NS <= 5, "the last stages are written out");
+  if constexpr (NS > 4) { if (left >= 4) stage(std::integral_constant<int, 4>{}, plain); }
+  if constexpr (NS > 3) { if (left >= 3) stage(std::integral_constant<int, 3>{}, plain); }
+  if constexpr (NS > 2) { if (left >= 2) stage(std::integral_constant<int, 2>{}, plain); }
+  if (left >= 1) stage(std::integral_constant<int, 1>{}, plain);
+  stage(std::integral_constant<int, 0>{}, plain);
 
   // acc[t][tn][r] = C[m0 + 32 (TM wm + t) + j][n0 + 32 (TN wn + tn) + 8 (r / 4) + 4 h + r % 4]; row tiles go through a
   // part of LDS of the wave's own (float32 ones a column tile at a time) and leave as whole rows
@@ -254,7 +288,7 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   constexpr int kGroup = kElt == 2 ? TN : 1;                         // column tiles that leave together
   constexpr int kPitch = kTile * kGroup * kElt + 16;
   constexpr int kPieces = kTile * kGroup * kElt / 16;
-  static_assert(kWaves * 32 * kPitch <= 2 * kStage, "the epilogue's rows fit the stages");
+  static_assert(kWaves * 32 * kPitch <= NS * kStage, "the epilogue's rows fit the stages");
   TOut* out = static_cast<TOut*>(a.out) + static_cast<int64_t>(blockIdx.y) * a.split_stride;
   const int n_out = EPI == kEpiSiluMul ? N / 2 : N;
   const int c0 = (EPI == kEpiSiluMul ? n0 / 2 : n0) + kTile * TN * wn;
@@ -315,14 +349,14 @@ __global__ __launch_bounds__(WM* WN* kWave, WM* WN / 4) void gemm_wide_kernel(co
   else if constexpr (EPI == kEpiSiluMul) leave(std::true_type{});
 }
 
-template <int WM, int WN, int TM, int TN, int EPI, typename TOut>
+template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut>
 int launch_wide(WideArgs a, int splits, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-  constexpr size_t lds = 2 * (BM + BN) * 128 + 256 * WM * WN;
-  static_assert(lds <= 160 * 1024, "two stages fit the LDS");
+  constexpr size_t lds = NS * (BM + BN) * 128 + (NS == 2 ? 256 * WM * WN : 0);
+  static_assert(lds <= 160 * 1024, "the stages fit the LDS");
   static bool asked = false;   // more than 64 KiB of LDS has to be asked for, once
   if (!asked) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, EPI, TOut>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) {
       (void)hipGetLastError();
@@ -334,14 +368,14 @@ int launch_wide(WideArgs a, int splits, hipStream_t s) {
   a.n_blocks = (a.N + BN - 1) / BN;
   const long long grid = static_cast<long long>(a.m_blocks) * ((a.n_blocks + kWdXcds - 1) / kWdXcds) * kWdXcds;
   if (grid > 0x7fffffffLL) return static_cast<int>(hipErrorInvalidValue);
-  gemm_wide_kernel<WM, WN, TM, TN, EPI, TOut><<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(splits)), WM * WN * kWave, lds, s>>>(a);
+  gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut><<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(splits)), WM * WN * kWave, lds, s>>>(a);
   return launch_status();
 }
 
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, int NS>
 int dispatch_wide(const WideArgs& a, int splits, int out_dtype, int epilogue, hipStream_t s) {
-  if (epilogue) return launch_wide<WM, WN, TM, TN, kEpiSiluMul, bf16>(a, splits, s);
-  return out_dtype == kF32 ? launch_wide<WM, WN, TM, TN, kEpiNone, float>(a, splits, s) : launch_wide<WM, WN, TM, TN, kEpiNone, bf16>(a, splits, s);
+  if (epilogue) return launch_wide<WM, WN, TM, TN, NS, kEpiSiluMul, bf16>(a, splits, s);
+  return out_dtype == kF32 ? launch_wide<WM, WN, TM, TN, NS, kEpiNone, float>(a, splits, s) : launch_wide<WM, WN, TM, TN, NS, kEpiNone, bf16>(a, splits, s);
 }
 
 }  // namespace arle
@@ -349,10 +383,11 @@ int dispatch_wide(const WideArgs& a, int splits, int out_dtype, int epilogue, hi
 using namespace arle;
 
 // x [M, K], w [N, K] bfloat16 with 16-byte aligned rows, K % 64 == 0, N % 32 == 0.  out [M, N] (bfloat16 or float32), or
-// with epilogue 1 [M, N/2] bfloat16 (gate and up rows of w interleaved in blocks of 16): silu(gate) * up.
+// with epilogue 1 [M, N/2] bfloat16 (gate and up rows of w interleaved in blocks of 16): silu(gate) * up.  tiled: w is the
+// operand tiles of [N, K], [N/16][K/32][64 lanes][8], lane 16 g + i = W[16 t + i][32 s + 8 g .. +7] (ldw is not looked at).
 extern "C" int arle_gemm_wide(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int out_dtype,
                               int M, int N, int K, int epilogue, int row_tiles, int col_tiles, int splits, int stages_per_split,
-                              long long split_stride, void* stream) {
+                              long long split_stride, int tiled, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const int per16 = out_dtype == kF32 ? 4 : 8;
@@ -365,21 +400,28 @@ extern "C" int arle_gemm_wide(const void* x, long long ldx, const void* w, long 
   if (static_cast<long long>(splits - 1) * stages_per_split >= stages || static_cast<long long>(splits) * stages_per_split < stages)
     return static_cast<int>(hipErrorInvalidValue);
   const WideArgs a{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(w), ldw, out, ldo, M, N, K,
-                   0, 0, stages_per_split, split_stride};
+                   0, 0, stages_per_split, split_stride, tiled};
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (1000 * row_tiles + col_tiles) {   // rows and columns of a workgroup
-    case 256320: return dispatch_wide<4, 2, 2, 5>(a, splits, out_dtype, epilogue, s);
-    case 256256: return dispatch_wide<4, 2, 2, 4>(a, splits, out_dtype, epilogue, s);
-    case 256192: return dispatch_wide<4, 2, 2, 3>(a, splits, out_dtype, epilogue, s);
-    case 128064: return dispatch_wide<2, 2, 2, 1>(a, splits, out_dtype, epilogue, s);
-    case 128096: return dispatch_wide<4, 1, 1, 3>(a, splits, out_dtype, epilogue, s);
-    case 128128: return dispatch_wide<2, 2, 2, 2>(a, splits, out_dtype, epilogue, s);
-    case 128160: return dispatch_wide<4, 1, 1, 5>(a, splits, out_dtype, epilogue, s);
-    case 256160: return dispatch_wide<4, 1, 2, 5>(a, splits, out_dtype, epilogue, s);
-    case 128256: return dispatch_wide<2, 2, 2, 4>(a, splits, out_dtype, epilogue, s);
-    case 128192: return dispatch_wide<2, 2, 2, 3>(a, splits, out_dtype, epilogue, s);
-    case 128320: return dispatch_wide<2, 2, 2, 5>(a, splits, out_dtype, epilogue, s);
-    case 192320: return dispatch_wide<2, 2, 3, 5>(a, splits, out_dtype, epilogue, s);
+    case 64064: return dispatch_wide<2, 2, 1, 1, 5>(a, splits, out_dtype, epilogue, s);
+    case 64096: return dispatch_wide<2, 1, 1, 3, 4>(a, splits, out_dtype, epilogue, s);
+    case 64128: return dispatch_wide<2, 2, 1, 2, 4>(a, splits, out_dtype, epilogue, s);
+    case 128064: return dispatch_wide<2, 2, 2, 1, 4>(a, splits, out_dtype, epilogue, s);
+    case 128096: return dispatch_wide<4, 1, 1, 3, 4>(a, splits, out_dtype, epilogue, s);
+    case 128128: return dispatch_wide<2, 2, 2, 2, 4>(a, splits, out_dtype, epilogue, s);
+    case 128160: return dispatch_wide<4, 1, 1, 5, 3>(a, splits, out_dtype, epilogue, s);
+    case 128192: return dispatch_wide<2, 2, 2, 3, 3>(a, splits, out_dtype, epilogue, s);
+    case 128256: return dispatch_wide<2, 2, 2, 4, 3>(a, splits, out_dtype, epilogue, s);
+    case 128320: return dispatch_wide<2, 2, 2, 5, 2>(a, splits, out_dtype, epilogue, s);
+    case 192128: return dispatch_wide<2, 2, 3, 2, 3>(a, splits, out_dtype, epilogue, s);
+    case 192192: return dispatch_wide<2, 2, 3, 3, 3>(a, splits, out_dtype, epilogue, s);
+    case 192256: return dispatch_wide<2, 2, 3, 4, 2>(a, splits, out_dtype, epilogue, s);
+    case 192320: return dispatch_wide<2, 2, 3, 5, 2>(a, splits, out_dtype, epilogue, s);
+    case 256128: return dispatch_wide<4, 2, 2, 2, 3>(a, splits, out_dtype, epilogue, s);
+    case 256160: return dispatch_wide<4, 1, 2, 5, 3>(a, splits, out_dtype, epilogue, s);
+    case 256192: return dispatch_wide<4, 2, 2, 3, 2>(a, splits, out_dtype, epilogue, s);
+    case 256256: return dispatch_wide<4, 2, 2, 4, 2>(a, splits, out_dtype, epilogue, s);
+    case 256320: return dispatch_wide<4, 2, 2, 5, 2>(a, splits, out_dtype, epilogue, s);
   }
   return static_cast<int>(hipErrorInvalidValue);
 }

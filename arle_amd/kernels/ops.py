@@ -788,9 +788,9 @@ def pack_weight_tiles(w: torch.Tensor) -> torch.Tensor:
 
 
 def _check_tiles(tiles, N: int, K: int) -> None:
-    _need(tiles.dtype == torch.bfloat16 and tiles.is_contiguous() and tiles.dim() == 3 and tiles.shape[1:] == (-(-K // 32), 512)
-          and tiles.shape[0] >= -(-N // 16) and tiles.data_ptr() % 16 == 0,
-          f"operand tiles of a [{N}, {K}] matrix have the shape [{-(-N // 16)}, {-(-K // 32)}, 512], got {tuple(tiles.shape)}")
+    if not (tiles.dtype == torch.bfloat16 and tiles.is_contiguous() and tiles.dim() == 3 and tiles.shape[1:] == (-(-K // 32), 512)
+            and tiles.shape[0] >= -(-N // 16) and tiles.data_ptr() % 16 == 0):
+        raise ShapeError(f"operand tiles of a [{N}, {K}] matrix have the shape [{-(-N // 16)}, {-(-K // 32)}, 512], got {tuple(tiles.shape)}")
 
 
 def gemm_rows(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, variant: int | None = None,
@@ -1052,11 +1052,17 @@ def gemm_tiles(x, tiles, n: int, out_dtype=torch.bfloat16, epilogue: int = EPI_N
 # one, in us, activation or not (MI355X, weights cold, from products of 65 to 8,192 rows at K 2,560 and 4,096; beside the
 # stages a workgroup takes 4 us for its first loads and its results).  A launch takes as many turns as its workgroups fill
 # the compute units; wide_plan picks the shape (and the parts of K) whose turns take least.
-WIDE_STAGE_US = {(128, 64): 0.62, (128, 96): 0.80, (128, 128): 0.87, (128, 160): 0.89, (128, 192): 0.92, (128, 256): 1.04,
-                 (128, 320): 1.15, (256, 160): 1.16, (256, 192): 1.32, (256, 256): 1.52, (192, 320): 1.52, (256, 320): 1.85}
+WIDE_STAGE_US = {(64, 64): 0.22, (64, 96): 0.32, (64, 128): 0.44, (128, 64): 0.35, (128, 96): 0.46, (128, 128): 0.54, (128, 160): 0.64,
+                 (128, 192): 0.73, (128, 256): 0.88, (128, 320): 1.06, (192, 128): 0.69, (192, 192): 0.90, (192, 256): 1.15,
+                 (256, 128): 0.83, (256, 160): 1.03, (256, 192): 1.25, (256, 256): 1.48, (192, 320): 1.43, (256, 320): 1.73}
+# Shapes that are for steps of so many rows at most: beyond them the taller ones are level or ahead (the estimate, which
+# knows one time a stage for all row counts, would take them).
+_WIDE_MOST_ROWS = {(64, 64): 256, (64, 96): 256, (64, 128): 256, (192, 128): 1024, (192, 192): 1024, (192, 256): 1024}
 _WIDE_FIXED_US = 4.0
 _XCDS = 8
 _WIDE_MAX_PARTS = 8
+_WIDE_FROM_ROWS = 9             # fewer rows stay with the kernels that stream W through registers
+_WIDE_CANDIDATE_SHAPES = 3      # shapes that a tuner tries for a number of parts
 _WIDE_K = 64            # K comes in whole stages
 
 
@@ -1069,25 +1075,32 @@ def gemm_wide_supported(n: int, k: int, x_stride: int, w_stride: int | None = No
 
 
 @functools.lru_cache(maxsize=4096)
-def wide_plan(rows: int, n: int, k: int, parts: int = 1, units: int = 256) -> tuple:
-    """((rows, columns) of a workgroup, estimated us) of gemm_wide for a product in `parts` parts of K on `units` compute
-    units."""
+def wide_shapes(rows: int, n: int, k: int, parts: int = 1, units: int = 256) -> tuple:
+    """((rows, columns) of a workgroup, estimated us) of every shape that gemm_wide has, for a product in `parts` parts of K on
+    `units` compute units, the fastest first."""
     stages = -(-(k // _WIDE_K) // parts)
-    best = None
+    found = []
     for (bm, bn), stage_us in WIDE_STAGE_US.items():
+        if rows > _WIDE_MOST_ROWS.get((bm, bn), rows):
+            continue
         # column blocks go to the XCDs in turn: the one with most of them is the last to be done
         workgroups = -(-rows // bm) * -(-(-(-n // bn)) // _XCDS) * parts
         us = -(-workgroups * _XCDS // units) * (_WIDE_FIXED_US + stages * stage_us)
-        if best is None or us < best[1]:
-            best = ((bm, bn), us)
-    return best
+        found.append(((bm, bn), us))
+    return tuple(sorted(found, key=lambda f: f[1]))
 
 
-def gemm_wide(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, shape=None, splits: int = 1):
+def wide_plan(rows: int, n: int, k: int, parts: int = 1, units: int = 256) -> tuple:
+    """The first of wide_shapes."""
+    return wide_shapes(rows, n, k, parts, units)[0]
+
+
+def gemm_wide(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, shape=None, splits: int = 1, tiles: torch.Tensor | None = None):
     """x [M, K] . W^T for prompt portions, W [N, K] as it is stored: workgroups of `shape` rows x columns (default:
     wide_plan's), both operands through LDS.  EPI_SILU_MUL: gate and up rows of W interleaved in blocks of 16; returns
-    [M, N/2].  splits > 1: K cut into that many parts of whole stages of 64; returns the float32 stack [splits, M, N]."""
-    _gpu(x, w)
+    [M, N/2].  splits > 1: K cut into that many parts of whole stages of 64; returns the float32 stack [splits, M, N].
+    tiles: pack_weight_tiles(w), to be read instead of w."""
+    _gpu(x, w, tiles)
     _rows(x, "x")
     _rows(w, "w")
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_wide takes bfloat16 operands")
@@ -1095,6 +1108,8 @@ def gemm_wide(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, shape
     _need(w.shape[1] == K, "x and W differ in K")
     _need(gemm_wide_supported(N, K, x.stride(0), w.stride(0)) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0,
           "gemm_wide: K in stages of 64, N in blocks of 32, 16-byte aligned rows")
+    if tiles is not None:
+        _check_tiles(tiles, N, K)
     fused = epilogue == EPI_SILU_MUL
     _need(out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and not fused), "gemm_wide writes bfloat16, or float32 without an epilogue")
     stages = K // _WIDE_K
@@ -1111,8 +1126,8 @@ def gemm_wide(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, shape
     else:
         out = torch.empty((M, N // 2 if fused else N), dtype=out_dtype, device=x.device)
         ldo, stride = out.stride(0), 0
-    lib.call("arle_gemm_wide", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), ldo, _CODES[out_dtype], M, N, K,
-             int(epilogue), int(shape[0]), int(shape[1]), splits, per, stride, _stream())
+    lib.call("arle_gemm_wide", x.data_ptr(), x.stride(0), (w if tiles is None else tiles).data_ptr(), w.stride(0), out.data_ptr(), ldo, _CODES[out_dtype], M, N, K,
+             int(epilogue), int(shape[0]), int(shape[1]), splits, per, stride, int(tiles is not None), _stream())
     return out
 
 
@@ -1353,6 +1368,28 @@ def gemm_wide_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
     return least is not None and (rows >= least or _WIDE_TWO_BLOCKS[0] <= rows <= _WIDE_TWO_BLOCKS[1])
 
 
+# Plain products by gemm_wide, for widths that no table names: outputs of 5,120 columns and more, whole sums (where a stack
+# of partial sums is welcome, the kernels of few rows keep theirs).  MI355X, cold weights, us, the other rules / gemm_wide:
+#   up to 1,024 rows: N 9,728, K 2,560 9 rows 15.2 / 14.8, 32 16.6 / 14.5, 64 19.5 / 17.3, 128 24.7 / 20.1, 256 38.4 / 26.3, 512
+#     37.7 / 32.5, 1,024 56.1 / 47.7; N 5,120, K 5,120 192 rows 43.7 / 27.3, 512 49.3 / 42.0, 1,024 63.8 / 56.1; N 16,384, K 5,120
+#     16 rows 45.8 / 30.2, 64 36.7 / 32.4, 256 66.8 / 56.1; narrower ones go either way (N 4,096, K 2,560 9 rows 10.2 / 12.1,
+#     112 12.4 / 13.7, 256 and beyond within 6 %).
+#   beyond: where the plan's workgroups are the largest, 256 x 320, they fill their turns: N 9,728, K 2,560 1,792 rows 119 / 81,
+#     2,048 108 / 88, 4,096 191 / 170; N 12,288, K 3,072 1,536 rows 123 / 99, 6,144 457 / 381; N 10,240, K 2,560 6,144 rows
+#     243 / 252 is the worst of it.  With the other shapes the library is level or ahead (N 9,728, K 2,560 1,536 rows 63 / 69,
+#     3,072 125 / 132; N 8,192, K 2,048 2,048 rows 55 / 62).
+_WIDE_PLAIN_MIN_N = 5120
+_WIDE_PLAIN_MAX_K = 5120
+_WIDE_PLAIN_ANY_SHAPE_ROWS = 1024
+
+
+def gemm_wide_plain_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
+    """Whether a plain product runs whole in gemm_wide (the rule for widths that no table names)."""
+    if rows < _WIDE_FROM_ROWS or n < _WIDE_PLAIN_MIN_N or k > _WIDE_PLAIN_MAX_K or not gemm_wide_supported(n, k, x_stride):
+        return False
+    return rows <= _WIDE_PLAIN_ANY_SHAPE_ROWS or wide_plan(rows, n, k)[0] == (256, 320)
+
+
 _PRODUCT_TABLE: dict = {}
 
 
@@ -1372,7 +1409,10 @@ def product_by_rules(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, f
             return ProductChoice("tiles", (8, 144) if rows >= _TILES_BIG_ROWS else (4, 44))
         return ProductChoice("library")
     staying = aligned and gemm_stream_preferred(rows, n, k, x_stride, tiled=tiled)
-    if not staying and aligned and gemm_rows_preferred(rows, n, k, x_stride):
+    few = staying or (aligned and gemm_rows_preferred(rows, n, k, x_stride))
+    if not (few and partials_ok) and aligned and w_aligned and gemm_wide_plain_preferred(rows, n, k, x_stride):
+        return ProductChoice("wide", (), 1)
+    if few and not staying:
         return ProductChoice("rows")
     if staying:
         variant, splits = _stream_plan(rows, n, k, tiled)
@@ -1412,8 +1452,8 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                         found.append(ProductChoice("rounds", (round_steps,)))
         if tiled and eight and n % 32 == 0 and rows > ROWS_KERNEL_MAX:
             found += [ProductChoice("tiles", v) for v in ((4, 44), (8, 144))]
-        if rows > ROWS_KERNEL_MAX and gemm_wide_supported(n, k, x_stride):
-            found.append(ProductChoice("wide"))
+        if rows >= _WIDE_FROM_ROWS and gemm_wide_supported(n, k, x_stride):
+            found += [ProductChoice("wide", shape, 0) for shape, _ in wide_shapes(rows, n, k)[:_WIDE_CANDIDATE_SHAPES]]
         return found
     if few:
         for variant in range(ROWS_VARIANTS):
@@ -1428,9 +1468,10 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                     found.append(ProductChoice("stream", (variant,), parts))
                     if parts in (2, 4, 8):      # and with two workgroups for every compute unit
                         found.append(ProductChoice("stream", (variant, 2 * _STREAM_TARGET_WORKGROUPS // parts), parts))
-    if rows > ROWS_KERNEL_MAX and gemm_wide_supported(n, k, x_stride):
-        found.append(ProductChoice("wide", (), 1))
-        found += [ProductChoice("wide", (), parts) for parts in range(2, _WIDE_MAX_PARTS + 1) if k >= 256 * parts and small(parts / 3)]
+    if rows >= _WIDE_FROM_ROWS and gemm_wide_supported(n, k, x_stride):
+        for parts in range(1, _WIDE_MAX_PARTS + 1):
+            if parts == 1 or (k >= 256 * parts and small(parts / 3)):
+                found += [ProductChoice("wide", shape, parts) for shape, _ in wide_shapes(rows, n, k, parts)[:_WIDE_CANDIDATE_SHAPES]]
     if rows > ROWS_KERNEL_MAX // 2:
         for parts in (2, 4, 8):
             if k % (32 * parts) == 0 and small(parts):
@@ -1490,7 +1531,7 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
         if kernel == "tiles":
             return gemm_tiles(x, tiles, w.shape[0], x.dtype, EPI_SILU_MUL, variant=choice.variant or None)
         if kernel == "wide":
-            return gemm_wide(x, w, x.dtype, EPI_SILU_MUL, shape=choice.variant or None)
+            return gemm_wide(x, w, x.dtype, EPI_SILU_MUL, shape=choice.variant or None, tiles=tiles)
         return silu_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), 16)
     if kernel == "rows":
         out = gemm_rows(x, w, out_dtype, variant=choice.variant[0] if choice.variant else None,
@@ -1506,7 +1547,7 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
         out = gemm_tiles(x, tiles, w.shape[0], out_dtype, variant=choice.variant or None)
     elif kernel == "wide":
         parts = max(choice.splits, 1)
-        out = gemm_wide(x, w, torch.float32 if parts > 1 else out_dtype, shape=choice.variant or None, splits=parts)
+        out = gemm_wide(x, w, torch.float32 if parts > 1 else out_dtype, shape=choice.variant or None, splits=parts, tiles=tiles)
     elif kernel == "library_parts":
         out = _library_mm_split_k(x, w, choice.splits)
         if out is None:

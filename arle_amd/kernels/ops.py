@@ -1838,6 +1838,40 @@ def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_st
     return out
 
 
+def mlstm_decode_supported(key_dim: int, value_dim: int, s_state) -> bool:
+    """Whether mlstm_decode takes heads of these sizes."""
+    return 0 < key_dim <= 128 and value_dim in (32, 64, 128) and s_state.data_ptr() % 16 == 0
+
+
+def mlstm_decode(y, gates, bias_i, bias_f, cap: float, s_state, n_state, m_state, seg_row0, seg_slot, weight, eps: float, out_dtype, *,
+                 heads: int, key_dim: int, value_dim: int):
+    """mlstm_scan and mlstm_output for a step of single rows, one a request (no slot comes twice), in one kernel.  y float32
+    [T, 2 H D + 2 H Dv] (q, k, v and the output gate side by side), gates float32 [T, >= 2 H]; either may be a contiguous stack
+    [S, T, ...] of partial sums, added in order.  Returns [T, H * Dv]."""
+    _gpu(y, gates, bias_i, bias_f, s_state, n_state, m_state, seg_row0, seg_slot, weight)
+    H, D, Dv = heads, key_dim, value_dim
+    tokens, width = y.shape[-2], H * Dv
+    for name, t, least in (("y", y, 2 * H * (D + Dv)), ("gates", gates, 2 * H)):
+        _need(t.dtype == torch.float32 and t.dim() in (2, 3) and t.shape[-2] == tokens and t.shape[-1] >= least and t.stride(-1) == 1
+              and (t.dim() == 2 or t.is_contiguous()), f"{name} must be float32 rows of the heads' values, or a contiguous stack")
+    _need(mlstm_decode_supported(D, Dv, s_state), "mlstm_decode takes heads of up to 128 x 32, 64 or 128")
+    _need(bias_i.shape == (H,) and bias_f.shape == (H,) and bias_i.dtype == bias_f.dtype == torch.float32
+          and bias_i.is_contiguous() and bias_f.is_contiguous(), "gate biases must be float32 [heads]")
+    slots = s_state.shape[0]
+    _need(s_state.shape == (slots, H, D, Dv) and n_state.shape == (slots, H, D) and m_state.shape == (slots, H)
+          and all(t.dtype == torch.float32 and t.is_contiguous() for t in (s_state, n_state, m_state)),
+          "mLSTM states are float32 [slots, H, D, Dv], [slots, H, D] and [slots, H]")
+    _i32(seg_slot, "seg_slot", tokens)
+    _i32(seg_row0, "seg_row0", tokens + 1)
+    _need(weight.shape == (width,) and weight.is_contiguous() and weight.dtype in _CODES, "the norm weight must be [H * Dv]")
+    out = torch.empty((tokens, width), dtype=out_dtype, device=y.device)
+    stack = lambda t: (t.data_ptr(), t.stride(0), t.stride(1), t.shape[0]) if t.dim() == 3 else (t.data_ptr(), 0, t.stride(0), 1)
+    lib.call("arle_mlstm_decode", *stack(y), *stack(gates), bias_i.data_ptr(), bias_f.data_ptr(), float(cap), s_state.data_ptr(),
+             n_state.data_ptr(), m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), tokens, H, D, Dv, weight.data_ptr(),
+             _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
+    return out
+
+
 def mlstm_output(num, nq, coefs, gate, weight, eps: float, out_dtype, *, heads: int, value_dim: int):
     """o = num / (max(|nq|, exp(-m)) + 1e-6); then each head's o divided by its root mean square, times `weight`
     [heads * value_dim], times sigmoid(gate)."""

@@ -85,16 +85,22 @@ class MLSTMMixer(Part):
         qk, vw = self.H * self.D, self.H * self.Dv
         # 32-bit sums out of the product: q and k meet in dot products whose terms cancel (a request's first rows hang
         # on a single one), and what rounding them to bfloat16 costs there is ten times a usual row's error
+        S, n, m = cache["S"].state, cache["n"].state, cache["m"].state
+        if not self.rt.is_f32 and batch.max_qlen == 1 and ops.mlstm_decode_supported(self.D, self.Dv, S):
+            y = ops.mlstm_decode(self.qkvg(x, out_dtype=torch.float32, partials_ok=True),
+                                 self.gates(x, out_dtype=torch.float32, partials_ok=True), self.i_bias, self.f_bias, self.cap, S, n, m,
+                                 batch.seg_row0, batch.seg_slot, self.norm, self.eps, self.rt.act_dtype, heads=self.H,
+                                 key_dim=self.D, value_dim=self.Dv)
+            return self.o(y, out_dtype=torch.float32, partials_ok=True)
         p = self.qkvg(x, out_dtype=torch.float32)
         gates = self.gates(x, out_dtype=torch.float32)[:, :2 * self.H]
         if not self.rt.is_f32 and ops.mlstm_chunks_preferred(batch.max_qlen, x.shape[0], batch.seg_slot.numel(), self.H, self.D, self.Dv):
-            y = ops.mlstm_chunks(p, gates, self.i_bias, self.f_bias, self.cap, cache["S"].state, cache["n"].state, cache["m"].state,
+            y = ops.mlstm_chunks(p, gates, self.i_bias, self.f_bias, self.cap, S, n, m,
                                  batch.seg_row0, batch.seg_slot, self.norm, self.eps, self.rt.act_dtype, heads=self.H,
                                  key_dim=self.D, value_dim=self.Dv, longest=batch.max_qlen)
             return self.o(y, out_dtype=torch.float32, partials_ok=True)
         q, k, v, g = p[:, :qk], p[:, qk:2 * qk], p[:, 2 * qk:2 * qk + vw], p[:, 2 * qk + vw:]
-        num, nq, coefs = ops.mlstm_scan(q, k, v, gates, self.i_bias, self.f_bias, self.cap, cache["S"].state,
-                                        cache["n"].state, cache["m"].state, batch.seg_row0, batch.seg_slot,
+        num, nq, coefs = ops.mlstm_scan(q, k, v, gates, self.i_bias, self.f_bias, self.cap, S, n, m, batch.seg_row0, batch.seg_slot,
                                         heads=self.H, key_dim=self.D, value_dim=self.Dv)
         y = ops.mlstm_output(num, nq, coefs, g, self.norm, self.eps, self.rt.act_dtype, heads=self.H, value_dim=self.Dv)
         return self.o(y, out_dtype=torch.float32, partials_ok=True)   # it goes into the 32-bit residual unrounded

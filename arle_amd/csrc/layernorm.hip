@@ -87,24 +87,24 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_kernel(
 // The same for the usual types: terms that are float32 (a projection's 32-bit output or its stack of partial
 // products), biases, weights and outputs of one type TA, a width that is a multiple of 4.  Four elements a lane and
 // access, every load of a row issued without a condition on data, before anything is stored.
-template <typename TA, int PER4>
-__global__ __launch_bounds__(kLnThreads) void add_layernorm_vec_kernel(
+template <typename TA, int NT, int PER4>
+__global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     float* __restrict__ residual, const float* __restrict__ t0, int n0, long long s0, const TA* __restrict__ b0,
     const float* __restrict__ t1, int n1, long long s1, const TA* __restrict__ b1, const TA* __restrict__ wa,
     const TA* __restrict__ wb, TA* __restrict__ out_a, TA* __restrict__ out_b, const int* __restrict__ rows, int width,
     float eps, const TA* __restrict__ ca, const TA* __restrict__ cb) {
-  __shared__ float lds[kLnWaves];
+  __shared__ float lds[(NT / kWave)];
   const int r = blockIdx.x;
   const int64_t src = rows ? rows[r] : r;
   const int64_t base = src * width;
   const int last = width - 4, tid = threadIdx.x;
   float4 x[PER4];
 #pragma unroll
-  for (int k = 0; k < PER4; ++k) x[k] = ld4<float>(residual + base + min((tid + k * kLnThreads) * 4, last));
+  for (int k = 0; k < PER4; ++k) x[k] = ld4<float>(residual + base + min((tid + k * NT) * 4, last));
   auto add_term = [&](const float* t, int n, long long stride, const TA* bias) {
     float4 d[PER4];
 #pragma unroll
-    for (int k = 0; k < PER4; ++k) d[k] = ld4<float>(t + base + min((tid + k * kLnThreads) * 4, last));
+    for (int k = 0; k < PER4; ++k) d[k] = ld4<float>(t + base + min((tid + k * NT) * 4, last));
     // the parts of a stack are fetched several at a time (eight for rows up to 4,096 wide) without a condition (a part past the last is the last one
     // again, fetched and dropped), so that their loads are in flight together; they are added in the stack's order
     constexpr int G = PER4 <= 4 ? 8 : (PER4 <= 8 ? 4 : 2);
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_vec_kernel(
       for (int j = 0; j < G; ++j) {
         const long long at = min(s0 + j, n - 1) * stride + base;
 #pragma unroll
-        for (int k = 0; k < PER4; ++k) e[j][k] = ld4<float>(t + at + min((tid + k * kLnThreads) * 4, last));
+        for (int k = 0; k < PER4; ++k) e[j][k] = ld4<float>(t + at + min((tid + k * NT) * 4, last));
       }
 #pragma unroll
       for (int j = 0; j < G; ++j) {
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_vec_kernel(
 #pragma unroll
     for (int k = 0; k < PER4; ++k) {
       if (bias) {
-        const float4 e = ld4<TA>(bias + min((tid + k * kLnThreads) * 4, last));
+        const float4 e = ld4<TA>(bias + min((tid + k * NT) * 4, last));
         d[k].x += e.x; d[k].y += e.y; d[k].z += e.z; d[k].w += e.w;
       }
       x[k].x += d[k].x; x[k].y += d[k].y; x[k].z += d[k].z; x[k].w += d[k].w;
@@ -139,11 +139,11 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_vec_kernel(
   float4 w_a[PER4], w_b[PER4], c_a[PER4], c_b[PER4];
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
-    w_a[k] = ld4<TA>(wa + min((tid + k * kLnThreads) * 4, last));
-    w_b[k] = ld4<TA>((wb ? wb : wa) + min((tid + k * kLnThreads) * 4, last));
+    w_a[k] = ld4<TA>(wa + min((tid + k * NT) * 4, last));
+    w_b[k] = ld4<TA>((wb ? wb : wa) + min((tid + k * NT) * 4, last));
     // (a bias that is absent is the weight again, fetched and dropped)
-    c_a[k] = ld4<TA>((ca ? ca : wa) + min((tid + k * kLnThreads) * 4, last));
-    c_b[k] = ld4<TA>((cb ? cb : wa) + min((tid + k * kLnThreads) * 4, last));
+    c_a[k] = ld4<TA>((ca ? ca : wa) + min((tid + k * NT) * 4, last));
+    c_b[k] = ld4<TA>((cb ? cb : wa) + min((tid + k * NT) * 4, last));
     if (!ca) c_a[k] = float4{0.f, 0.f, 0.f, 0.f};
     if (!cb) c_b[k] = float4{0.f, 0.f, 0.f, 0.f};
   }
@@ -152,25 +152,25 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_vec_kernel(
   float sum = 0.f;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
-    const int i = (tid + k * kLnThreads) * 4;
+    const int i = (tid + k * NT) * 4;
     if (i < width) {
       if (!rows && (t0 || t1)) st4<float>(residual + base + i, x[k]);
       sum += (x[k].x + x[k].y) + (x[k].z + x[k].w);
     }
   }
-  const float mu = block_sum<kLnWaves>(sum, lds) / static_cast<float>(width);
+  const float mu = block_sum<(NT / kWave)>(sum, lds) / static_cast<float>(width);
   float sq = 0.f;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
-    const int i = (tid + k * kLnThreads) * 4;
+    const int i = (tid + k * NT) * 4;
     x[k].x -= mu; x[k].y -= mu; x[k].z -= mu; x[k].w -= mu;
     if (i < width) sq += (x[k].x * x[k].x + x[k].y * x[k].y) + (x[k].z * x[k].z + x[k].w * x[k].w);
   }
-  const float inv = 1.0f / sqrtf(block_sum<kLnWaves>(sq, lds) / static_cast<float>(width) + eps);
+  const float inv = 1.0f / sqrtf(block_sum<(NT / kWave)>(sq, lds) / static_cast<float>(width) + eps);
   const int64_t o = static_cast<int64_t>(r) * width;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
-    const int i = (tid + k * kLnThreads) * 4;
+    const int i = (tid + k * NT) * 4;
     if (i < width) {
       const float4 w = w_a[k], c = c_a[k];
       st4<TA>(out_a + o + i, float4{fmaf(x[k].x * inv, w.x, c.x), fmaf(x[k].y * inv, w.y, c.y), fmaf(x[k].z * inv, w.z, c.z),
@@ -188,22 +188,33 @@ template <typename TA>
 static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, const void* wa, const void* wb, void* out_a,
                          void* out_b, const int* rows, int n_rows, int width, float eps, const void* ca, const void* cb,
                          hipStream_t s) {
-#define ARLE_LNV(PER4)                                                                                              \
-  add_layernorm_vec_kernel<TA, PER4><<<n_rows, kLnThreads, 0, s>>>(                                                  \
+#define ARLE_LNV(NT, PER4)                                                                                          \
+  add_layernorm_vec_kernel<TA, NT, PER4><<<n_rows, NT, 0, s>>>(                                                  \
       residual, static_cast<const float*>(t0.data), t0.n_stack, t0.stack_stride, static_cast<const TA*>(t0.bias),  \
       static_cast<const float*>(t1.data), t1.n_stack, t1.stack_stride, static_cast<const TA*>(t1.bias),            \
       static_cast<const TA*>(wa), static_cast<const TA*>(wb), static_cast<TA*>(out_a), static_cast<TA*>(out_b), rows, \
       width, eps, static_cast<const TA*>(ca), static_cast<const TA*>(cb))
-  if (width <= kLnThreads * 4) {
-    ARLE_LNV(1);
-  } else if (width <= kLnThreads * 8) {
-    ARLE_LNV(2);
-  } else if (width <= kLnThreads * 16) {
-    ARLE_LNV(4);
-  } else if (width <= kLnThreads * 32) {
-    ARLE_LNV(8);
+  // Workgroups as wide as the row where that is more than 2,048 elements: nearly every load of a row is then on its way at once
+  // and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
+  // 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
+  // wide 8.2 / 6.2, 2,048 rows 68.7 / 60.8.  Narrower rows need several a compute unit (1,536 wide, 2,048 rows 20.0 / 27.1), and
+  // so do many rows of 8,192 (8 rows 8.7 / 7.9, 2,048 86.2 / 89.8).
+  if (width <= 1024) {
+    ARLE_LNV(256, 1);
+  } else if (width <= 2048) {
+    ARLE_LNV(256, 2);
+  } else if (width <= 2560) {
+    ARLE_LNV(640, 1);
+  } else if (width <= 4096) {
+    ARLE_LNV(1024, 1);
+  } else if (width <= 5120) {
+    ARLE_LNV(640, 2);
+  } else if (width <= 8192 && n_rows < 1024) {
+    ARLE_LNV(1024, 2);
+  } else if (width <= 8192) {
+    ARLE_LNV(256, 8);
   } else {
-    ARLE_LNV(16);
+    ARLE_LNV(256, 16);
   }
 #undef ARLE_LNV
   return launch_status();

@@ -177,6 +177,59 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
   }
 }
 
+// A step of single rows, one a request: a lane's four channels of the state belong to nobody else in the step, so it
+// writes them back moved on by its row, and no second kernel has to wait for this one (decode steps of the Gufasun design have
+// twelve of these pairs, 4.4 + 3.9 us each at 8 requests; together 4.6).  PARTS: the input is a stack of float32 partial sums, added in order and
+// rounded to T as the kernel that adds such stacks does.
+template <typename T, int TAPS, bool PARTS>
+__global__ void conv_step_kernel(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,
+                                 const T* __restrict__ bias, const T* __restrict__ out_bias, const T* __restrict__ w,
+                                 T* __restrict__ state, const int* __restrict__ slot_of_token, T* __restrict__ out,
+                                 long long out_stride, int channels, int flags) {
+  const int64_t t = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (c >= channels) return;
+  T* mine = state + static_cast<int64_t>(slot_of_token[t]) * (TAPS - 1) * channels + c;
+  float4 in[TAPS];     // in[back]: the input `back` rows before this one
+#pragma unroll
+  for (int back = 1; back < TAPS; ++back) in[back] = ld4<T>(mine + static_cast<int64_t>(TAPS - 1 - back) * channels);
+  if constexpr (PARTS) {
+    const float* at = static_cast<const float*>(u) + t * u_stride + c;
+    float4 v = ld4<float>(at);
+    for (int s = 1; s < parts; ++s) {
+      const float4 e = ld4<float>(at + s * part_stride);
+      v = float4{v.x + e.x, v.y + e.y, v.z + e.z, v.w + e.w};
+    }
+    in[0] = float4{to_float(from_float<T>(v.x)), to_float(from_float<T>(v.y)), to_float(from_float<T>(v.z)), to_float(from_float<T>(v.w))};
+  } else {
+    in[0] = ld4<T>(static_cast<const T*>(u) + t * u_stride + c);
+  }
+  const float4 b = bias ? ld4<T>(bias + c) : float4{0.f, 0.f, 0.f, 0.f};
+  in[0] = float4{in[0].x + b.x, in[0].y + b.y, in[0].z + b.z, in[0].w + b.w};
+  float wt[4][TAPS];   // four channels' taps are 4 * TAPS consecutive elements
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) {
+    const float4 v = ld4<T>(w + static_cast<int64_t>(c) * TAPS + 4 * j);
+    const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wt[(4 * j + i) / TAPS][(4 * j + i) % TAPS] = e[i];
+  }
+  const float4 ob = out_bias ? ld4<T>(out_bias + c) : float4{0.f, 0.f, 0.f, 0.f};
+  float acc[4] = {ob.x, ob.y, ob.z, ob.w};
+  const float now[4] = {in[0].x, in[0].y, in[0].z, in[0].w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt[i][TAPS - 1], now[i], ((flags & kConvAdd) ? now[i] : 0.f) + acc[i]);
+#pragma unroll
+  for (int back = 1; back < TAPS; ++back) {
+    const float v[4] = {in[back].x, in[back].y, in[back].z, in[back].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt[i][TAPS - 1 - back], v[i], acc[i]);
+  }
+#pragma unroll
+  for (int back = 0; back < TAPS - 1; ++back) st4<T>(mine + static_cast<int64_t>(TAPS - 2 - back) * channels, in[back]);
+  st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], flags), conv_out(acc[1], flags), conv_out(acc[2], flags), conv_out(acc[3], flags)});
+}
+
 // One thread a (segment, channel): the new state is the last taps-1 of (old state, this step's inputs).
 __global__ void conv_state_update_kernel(const void* __restrict__ u, long long u_stride, int u_dtype,
                                          const void* __restrict__ bias, int bias_dtype, void* __restrict__ state,
@@ -265,5 +318,38 @@ extern "C" int arle_conv_state_update(const void* u, long long u_stride, int u_d
   dim3 grid(segments, (channels + 255) / 256);
   conv_state_update_kernel<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(
       u, u_stride, u_dtype, bias, bias_dtype, state, state_dtype, seg_row0, seg_slot, channels, taps);
+  return launch_status();
+}
+
+// A step of single rows, no slot twice: the convolution of each and its request's state moved on.  u [T, channels] of `dtype`
+// with rows u_stride apart, or, with parts > 0, a stack of so many float32 [T, channels] part_stride apart (u_stride its rows').
+// bias, out_bias [channels] or null, w [channels, taps], state [slots, taps - 1, channels] and out [T, channels] of `dtype`;
+// taps 2 to 4, channels % 4 == 0, everything on the 16-byte grid.
+extern "C" int arle_conv_step(const void* u, long long u_stride, int parts, long long part_stride, int dtype, const void* bias,
+                              const void* out_bias, const void* w, void* state, const int* slot_of_token, void* out,
+                              long long out_stride, int tokens, int channels, int taps, int flags, void* stream) {
+  if (tokens == 0 || channels == 0) return 0;
+  const auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (taps < 2 || taps > 4 || channels % 4 != 0 || u_stride % 4 != 0 || part_stride % 4 != 0 || out_stride % 4 != 0 || parts < 0 ||
+      !at16(u) || !at16(out) || !at16(state) || !at16(w) || !at16(bias) || !at16(out_bias))
+    return static_cast<int>(hipErrorInvalidValue);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid(tokens, (channels / 4 + 255) / 256);
+#define ARLE_CONV_STEP(T, TAPS, PARTS)                                                                                       \
+  conv_step_kernel<T, TAPS, PARTS><<<grid, 256, 0, s>>>(u, u_stride, parts, part_stride, static_cast<const T*>(bias),        \
+                                                        static_cast<const T*>(out_bias), static_cast<const T*>(w),           \
+                                                        static_cast<T*>(state), slot_of_token, static_cast<T*>(out),         \
+                                                        out_stride, channels, flags)
+#define ARLE_CONV_STEP_TAPS(T, PARTS)                                                                                        \
+  do {                                                                                                                       \
+    if (taps == 2) ARLE_CONV_STEP(T, 2, PARTS); else if (taps == 3) ARLE_CONV_STEP(T, 3, PARTS); else ARLE_CONV_STEP(T, 4, PARTS); \
+  } while (0)
+  if (dtype == kF32) {
+    if (parts > 0) ARLE_CONV_STEP_TAPS(float, true); else ARLE_CONV_STEP_TAPS(float, false);
+  } else {
+    if (parts > 0) ARLE_CONV_STEP_TAPS(bf16, true); else ARLE_CONV_STEP_TAPS(bf16, false);
+  }
+#undef ARLE_CONV_STEP_TAPS
+#undef ARLE_CONV_STEP
   return launch_status();
 }

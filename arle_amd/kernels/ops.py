@@ -1697,6 +1697,39 @@ def causal_conv(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, 
     return out
 
 
+def conv_step_supported(weight, state, *, bias=None, out_bias=None) -> bool:
+    """Whether conv_step takes a convolution of this weight and state: one type throughout, 2 to 4 taps, channels in whole groups
+    of four, on the 16-byte grid."""
+    if weight is None or state is None:
+        return False
+    aligned = lambda t: t is None or (t.dtype == weight.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0)
+    return (weight.dtype in _CODES and 2 <= weight.shape[1] <= 4 and weight.shape[0] % 4 == 0
+            and aligned(weight) and aligned(state) and aligned(bias) and aligned(out_bias))
+
+
+def conv_step(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, bias=None, add_input: bool = False, silu: bool = False,
+              out_bias=None):
+    """causal_conv and conv_state_update for a step of single rows, one a request (no slot comes twice): every row's
+    convolution, and its request's state moved on.  u [T, C] of the weight's type, or a float32 stack [S, T, C], added in order
+    and rounded to that type."""
+    _gpu(u, weight, state, slot_of_token, bias, out_bias)
+    parts = u.shape[0] if u.dim() == 3 else 0
+    tokens, channels = u.shape[-2:]
+    _i32(slot_of_token, "slot_of_token", tokens)
+    _need(weight.shape[0] == channels and tuple(state.shape[1:]) == (weight.shape[1] - 1, channels)
+          and conv_step_supported(weight, state, bias=bias, out_bias=out_bias), "conv_step does not take this convolution")
+    _need((u.dtype == torch.float32 and u.is_contiguous()) if parts else (u.dtype == weight.dtype and u.stride(1) == 1),
+          "conv_step takes rows of the weight's type, or a contiguous float32 stack")
+    _need(u.stride(-2) % 4 == 0 and u.data_ptr() % 16 == 0, "conv_step takes rows on the 16-byte grid")
+    for b in (bias, out_bias):
+        _need(b is None or b.shape == (channels,), "a convolution's bias must be [channels]")
+    out = torch.empty((tokens, channels), dtype=weight.dtype, device=u.device)
+    lib.call("arle_conv_step", u.data_ptr(), u.stride(-2), parts, u.stride(0) if parts else 0, _code(weight), _ptr(bias), _ptr(out_bias),
+             weight.data_ptr(), state.data_ptr(), slot_of_token.data_ptr(), out.data_ptr(), out.stride(0), tokens, channels,
+             weight.shape[1], (1 if add_input else 0) | (2 if silu else 0), _stream())
+    return out
+
+
 def conv_state_update(u: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor, *, bias=None):
     """state[slot] <- the last taps-1 rows of (state[slot], the request's rows of u (+ bias)), for every segment."""
     _gpu(u, state, seg_row0, seg_slot, bias)
@@ -1715,17 +1748,31 @@ def conv_state_update(u: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tens
 # ------------------------------------------------------------------------ PolyNorm activation
 
 
+def polynorm_parts_supported(width: int, dtype: torch.dtype, coef, bias) -> bool:
+    """Whether PolyNorm adds a stack itself: one type, rows of whole groups of four."""
+    return width % 4 == 0 and coef.dtype == dtype and (bias is None or bias.dtype == dtype)
+
+
 def polynorm(u: torch.Tensor, coef: torch.Tensor, eps: float, *, bias=None, out_dtype: torch.dtype | None = None):
     """a N(z) + b N(z^2) + c N(z^3) + e over rows of z = u + bias; N divides a row by its root mean square;
-    coef = (a, b, c, e) on the GPU."""
+    coef = (a, b, c, e) on the GPU.  u may be a float32 stack [S, T, width], added in order and rounded to out_dtype (then the
+    type of coef and bias too)."""
     _gpu(u, coef, bias)
-    _rows(u, "u")
-    tokens, width = u.shape
+    tokens, width = u.shape[-2:]
     _need(coef.shape == (4,) and coef.is_contiguous() and coef.dtype in _CODES, "PolyNorm takes four coefficients")
     _need(0 < width <= 24576, "PolyNorm takes rows of up to 24,576 values")
     if bias is not None:
         _need(bias.shape == (width,) and bias.is_contiguous() and bias.dtype in _CODES, "the bias must be [width]")
     out = torch.empty((tokens, width), dtype=out_dtype or u.dtype, device=u.device)
+    if u.dim() == 3:
+        if not polynorm_parts_supported(width, out.dtype, coef, bias):
+            u = sum_partials(u, out.dtype)
+        else:
+            _need(u.dtype == torch.float32 and u.is_contiguous(), "a stack of partial sums is contiguous float32")
+            lib.call("arle_polynorm_parts", u.data_ptr(), u.shape[0], _ptr(bias), coef.data_ptr(), out.data_ptr(), _code(out), tokens,
+                     width, float(eps), _stream())
+            return out
+    _rows(u, "u")
     lib.call("arle_polynorm", u.data_ptr(), u.stride(0), _code(u), _ptr(bias), _code(bias) if bias is not None else 0,
              coef.data_ptr(), _code(coef), out.data_ptr(), _code(out), tokens, width, float(eps), _stream())
     return out

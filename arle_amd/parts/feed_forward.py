@@ -126,6 +126,8 @@ class PolyNormFeedForward(Part):
 
     def forward(self, x):
         """x [T, H] -> (delta, bias of the down projection): the block's next norm adds both."""
-        act = ops.polynorm(self.up(x), self.coef, self.eps, bias=self.up_bias)
+        # the parts that the products of few rows leave are added by the activation, which rounds their sum to x's type
+        few = x.shape[0] <= ops.ROWS_KERNEL_MAX and ops.polynorm_parts_supported(self.up.out_features, x.dtype, self.coef, self.up_bias)
+        act = ops.polynorm(self.up(x, partials_ok=few), self.coef, self.eps, bias=self.up_bias, out_dtype=x.dtype)
         # float32 out: the sum goes into the 32-bit residual unrounded
         return self.down(act, out_dtype=torch.float32, partials_ok=True), self.down_bias

@@ -29,9 +29,19 @@ class ShortConv:
         """The state of a convolution of `taps` taps: its last taps - 1 inputs, in the activation type."""
         return StateNeed((taps - 1, channels), None) if taps > 1 else None
 
+    def takes_parts(self, batch, state_view) -> bool:
+        """Whether the step is one of single rows whose convolution and state are one kernel, which adds a stack itself."""
+        return (batch.max_qlen == 1 and state_view is not None and self.taps > 1
+                and ops.conv_step_supported(self.weight, state_view.state, bias=self.bias, out_bias=self.out_bias))
+
     def __call__(self, u, batch, state_view, add_input: bool = False, silu: bool = False):
-        """The convolution of the step's rows (with `silu`, its silu); the requests' states move on by the rows they brought."""
+        """The convolution of the step's rows (with `silu`, its silu); the requests' states move on by the rows they brought.
+        u may be a float32 stack of partial sums where `takes_parts` says so."""
         state = state_view.state if (state_view is not None and self.taps > 1) else None
+        if u.dim() == 3 or (u.dtype == getattr(self.weight, "dtype", None) and u.stride(0) % 4 == 0 and u.data_ptr() % 16 == 0
+                            and self.takes_parts(batch, state_view)):
+            return ops.conv_step(u, self.weight, state, batch.slot_of_token, bias=self.bias, add_input=add_input, silu=silu,
+                                 out_bias=self.out_bias)
         y = ops.causal_conv(u, self.weight, state, batch.slot_of_token, bias=self.bias, add_input=add_input, silu=silu,
                             out_bias=self.out_bias)
         if state is not None:

@@ -128,7 +128,9 @@ class SoftcapAttention(Part):
         kv = cache["kv"]
         if kv.writes == self.shares_kv:
             raise ValueError("a layer that shares keys and values must read another entry's pages, and only such a layer")
-        y = self.conv(self.proj(x), batch, cache.get("conv"))
+        conv = cache.get("conv")
+        few = x.shape[0] <= ops.ROWS_KERNEL_MAX and self.conv.takes_parts(batch, conv) and self.conv.weight.dtype == x.dtype
+        y = self.conv(self.proj(x, partials_ok=few), batch, conv)
         Q = self.widths[0]
         q = y[:, :Q]
         if self.shares_kv:

@@ -1,0 +1,87 @@
+"""Kernels of steps in which every request brings one row: the convolution with its state (`ops.conv_step`) and PolyNorm of a
+stack against the kernels that they stand for, bit for bit (the same sums in the same order, stacks rounded as the kernel that
+adds them does); the mLSTM in one kernel (`ops.mlstm_decode`) against the 64-bit recurrence (bounds as in
+test_mlstm_chunks_gpu); the layer norm at the edges of its workgroups' widths (two 32-bit passes: 1e-5)."""
+import pytest
+import torch
+
+from test_mlstm_chunks_gpu import _case, _recurrence, _rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps,channels,rows", [(2, 4, 1), (3, 1020, 3), (4, 1028, 8), (4, 2560, 70)])
+@pytest.mark.parametrize("biased,flags", [(False, {}), (True, dict(add_input=True)), (True, dict(silu=True))])
+def test_the_convolution_and_its_state(dtype, taps, channels, rows, biased, flags):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(taps + channels)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
+    u, w, state = rand(rows, channels + 8)[:, :channels], rand(channels, taps), rand(rows + 2, taps - 1, channels)
+    bias, out_bias = (rand(channels), rand(channels)) if biased else (None, None)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    slots = i32([rows + 1 - r for r in range(rows)])
+    stack = torch.randn(3, rows, channels, generator=gen, device="cuda")
+    for given, parts in ((u, None), (ops.sum_partials(stack, dtype), stack)):
+        want_state, got_state = state.clone(), state.clone()
+        want = ops.causal_conv(given, w, want_state, slots, bias=bias, out_bias=out_bias, **flags)
+        ops.conv_state_update(given, want_state, i32(list(range(rows + 1))), slots, bias=bias)
+        got = ops.conv_step(given if parts is None else parts, w, got_state, slots, bias=bias, out_bias=out_bias, **flags)
+        assert torch.equal(got, want) and torch.equal(got_state, want_state)
+    assert not ops.conv_step_supported(rand(channels, 5), state) and not ops.conv_step_supported(rand(6, 4), state)
+    with pytest.raises(ops.ShapeError):
+        ops.conv_step(u, w, state[:, :, :-4], slots)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4, 2044, 2048, 2052, 4100, 9728, 10244, 14340, 24576])
+def test_polynorm_of_a_stack(dtype, width):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    stack = torch.randn(3, 5, width, generator=gen, device="cuda")
+    coef, bias = torch.randn(4, generator=gen, device="cuda").to(dtype), torch.randn(width, generator=gen, device="cuda").to(dtype)
+    whole = ops.sum_partials(stack, dtype)
+    for b in (None, bias):
+        got = ops.polynorm(stack, coef, 1e-6, bias=b, out_dtype=dtype)
+        assert torch.equal(got, ops.polynorm(whole, coef, 1e-6, bias=b))
+        z = whole.double() + (0 if b is None else b.double())
+        n = lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-6)
+        c = coef.double()
+        want = c[0] * n(z) + c[1] * n(z ** 2) + c[2] * n(z ** 3) + c[3]
+        assert _rel(got, want) < (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("rows,H,D,Dv,gate_std", [(1, 2, 128, 128, 1.0), (5, 3, 100, 64, 3.0), (9, 1, 32, 32, 20.0), (3, 2, 128, 32, 1.0), (2, 2, 7, 128, 1.0)])
+def test_the_memory_in_one_kernel(rows, H, D, Dv, gate_std):
+    from arle_amd.kernels import ops
+
+    c = _case([1] * rows, H, D, Dv, gate_std, 7 + rows)
+    want, states = _recurrence(c, H, D, Dv, 15.0)
+    noise = torch.randn_like(c["qkvg"]) * 0.5
+    wide = torch.cat([c["gates"], torch.zeros(rows, 16, device="cuda")], 1).contiguous()
+    forms = [(c["qkvg"], c["gates"]), (torch.stack([c["qkvg"] - noise, noise]), torch.stack([wide * 0.25, wide * 0.5, wide * 0.25]))]
+    for y, gates in forms:
+        mine = [t.clone() for t in c["state"]]
+        got = ops.mlstm_decode(y, gates, c["bi"], c["bf"], 15.0, *mine, c["row0"], c["slot"], c["weight"], 1e-6, torch.float32, heads=H,
+                               key_dim=D, value_dim=Dv)
+        assert _rel(got, want) < 2e-5
+        for state, ref, before in zip(mine, states, c["state"]):
+            assert _rel(state, ref) < 1e-6 and torch.equal(state[0], before[0])     # slot 0 belongs to nobody
+    assert not ops.mlstm_decode_supported(160, 128, c["state"][0]) and not ops.mlstm_decode_supported(128, 96, c["state"][0])
+
+
+@pytest.mark.parametrize("width", [1024, 1028, 2556, 2560, 2564, 4096, 4100, 5120, 5124, 8192, 8196, 16384])
+@pytest.mark.parametrize("rows", [1, 300])
+def test_layer_norm_at_the_edges_of_its_workgroups(width, rows):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    residual, stack, weight, bias = rand(rows, width) + 3, rand(3, rows, width), rand(width), rand(width)
+    want = residual.double() + stack.double().sum(0) + bias.double()
+    got = ops.add_layernorm(residual, [(stack, bias)], weight, 1e-6, torch.float32)
+    assert _rel(residual, want) < 1e-6
+    d = want - want.mean(-1, keepdim=True)
+    assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5

@@ -78,10 +78,21 @@ __global__ __launch_bounds__(kSampThreads) void argmax_rows_kernel(const float* 
 // (value, index) of its chunk in parts[row][chunk], and argmax_merge_kernel picks among them by the same rule.
 constexpr int kChunkThreads = 256;
 
+// clear_a, clear_b (null: nothing): so many 16-byte pieces a row that a sampling call wants zeroed, a row's chunks in turn.
+struct ClearRows {
+  uint4* a;
+  uint4* b;
+  int a_pieces, a_stride, b_pieces, b_stride;   // to clear, and from row to row
+};
+
 __global__ __launch_bounds__(kChunkThreads) void argmax_chunks_kernel(const float* __restrict__ logits, int vocab,
-                                                                     int chunk_len, ArgMax* __restrict__ parts) {
+                                                                     int chunk_len, ArgMax* __restrict__ parts, const ClearRows clear) {
   __shared__ ArgMax lds[kChunkThreads / kWave];
   const int row = blockIdx.y, chunk = blockIdx.x;
+  for (int i = chunk * kChunkThreads + static_cast<int>(threadIdx.x); i < clear.a_pieces; i += gridDim.x * kChunkThreads)
+    clear.a[static_cast<int64_t>(row) * clear.a_stride + i] = uint4{0u, 0u, 0u, 0u};
+  for (int i = chunk * kChunkThreads + static_cast<int>(threadIdx.x); i < clear.b_pieces; i += gridDim.x * kChunkThreads)
+    clear.b[static_cast<int64_t>(row) * clear.b_stride + i] = uint4{0u, 0u, 0u, 0u};
   const float* x = logits + static_cast<int64_t>(row) * vocab;
   const int begin = chunk * chunk_len, end = min(vocab, begin + chunk_len);
   ArgMax a;
@@ -546,38 +557,38 @@ __device__ __forceinline__ float lane_value(float v, int lane /* the same in eve
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// The token: greedy rows take the first maximum; the others the inverse CDF in token order.
-__global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleArgs a) {
-  __shared__ ArgMax best[kSelWaves];
-  __shared__ alignas(16) float part[kSelThreads];
-  __shared__ float chunk_start;
-  __shared__ int chunk_of_target, chosen;
-  const int row = blockIdx.x;
-  const RowParams r = row_params(a, row);
-  if (r.greedy) {
-    ArgMax m;
-    m.v = -INFINITY;
-    m.i = 0x7fffffff;
-    for (int c = threadIdx.x; c < a.chunks; c += kSelThreads)
-      m = better(m, a.part_max[static_cast<int64_t>(row) * a.chunks + c]);
+struct PickLds {
+  ArgMax best[kSelWaves];
+  alignas(16) float part[kSelThreads];
+  float chunk_start, target;
+  int chunk_of_target, chosen;
+};
+
+// A greedy row's token: the first maximum.
+__device__ __forceinline__ void pick_greedy(const SampleArgs& a, int row, PickLds& l) {
+  ArgMax m;
+  m.v = -INFINITY;
+  m.i = 0x7fffffff;
+  for (int c = threadIdx.x; c < a.chunks; c += kSelThreads)
+    m = better(m, a.part_max[static_cast<int64_t>(row) * a.chunks + c]);
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      ArgMax o;
-      o.v = __shfl_xor(m.v, off, kWave);
-      o.i = __shfl_xor(m.i, off, kWave);
-      m = better(m, o);
-    }
-    if (threadIdx.x % kWave == 0) best[threadIdx.x / kWave] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      ArgMax t = best[0];
-      for (int w = 1; w < kSelWaves; ++w) t = better(t, best[w]);
-      a.out[row] = t.i == 0x7fffffff ? 0 : t.i;
-    }
-    return;
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    ArgMax o;
+    o.v = __shfl_xor(m.v, off, kWave);
+    o.i = __shfl_xor(m.i, off, kWave);
+    m = better(m, o);
   }
-  const unsigned int thr = a.threshold[row];
-  const float* masses = a.chunk_mass + static_cast<int64_t>(row) * a.chunks;
+  if (threadIdx.x % kWave == 0) l.best[threadIdx.x / kWave] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    ArgMax t = l.best[0];
+    for (int w = 1; w < kSelWaves; ++w) t = better(t, l.best[w]);
+    a.out[row] = t.i == 0x7fffffff ? 0 : t.i;
+  }
+}
+
+// The chunk that u * (kept mass) falls into, and the mass in front of it.
+__device__ __forceinline__ void find_target(const SampleArgs& a, float u, const float* masses, PickLds& l) {
   if (threadIdx.x < kWave) {   // wave 0: lane l has the masses 4 l .. 4 l + 3; lanes without any add nothing
     const int lane = threadIdx.x;
     float m[4];
@@ -586,21 +597,21 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
     const unsigned long long some = __ballot(m[0] > 0.f || m[1] > 0.f || m[2] > 0.f || m[3] > 0.f);
     float total = 0.f;
     for (unsigned long long left = some; left != 0ull; left &= left - 1ull) {
-      const int l = __builtin_ctzll(left);
+      const int at = __builtin_ctzll(left);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) total += lane_value(m[j], l);
+      for (int j = 0; j < 4; ++j) total += lane_value(m[j], at);
     }
-    const float target = a.u[row] * total;
+    const float target = u * total;
     float run = 0.f;
     int at = -1, last = 0;
     float start = 0.f, last_start = 0.f;
     for (unsigned long long left = some; left != 0ull && at < 0; left &= left - 1ull) {
-      const int l = __builtin_ctzll(left);
+      const int from = __builtin_ctzll(left);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float mass = lane_value(m[j], l);
+        const float mass = lane_value(m[j], from);
         if (mass > 0.f) {
-          last = 4 * l + j;
+          last = 4 * from + j;
           last_start = run;
           if (at < 0 && target < run + mass) {
             at = last;
@@ -611,17 +622,43 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
       }
     }
     if (lane == 0) {
-      chunk_of_target = at >= 0 ? at : last;  // u at or past the whole mass (rounding): the last chunk that holds any
-      chunk_start = at >= 0 ? start : last_start;
-      part[0] = target;
-      chosen = -1;
+      l.chunk_of_target = at >= 0 ? at : last;  // u at or past the whole mass (rounding): the last chunk that holds any
+      l.chunk_start = at >= 0 ? start : last_start;
+      l.target = target;
+      l.chosen = -1;
     }
   }
   __syncthreads();
-  const int chunk = chunk_of_target;
-  const float target = part[0];
-  const float before = chunk_start;
+}
+
+// part[t], what thread t's tokens of the chunk weigh, becomes the mass in front of them (in the threads' order).
+__device__ __forceinline__ void add_up_parts(PickLds& l, float before) {
   __syncthreads();
+  if (threadIdx.x < kWave) {   // wave 0, four threads a lane; lanes without mass add nothing
+    const int lane = threadIdx.x;
+    const float4 c = *reinterpret_cast<const float4*>(&l.part[4 * lane]);
+    float run = before;
+    float4 own = {before, before, before, before};
+    for (unsigned long long left = __ballot(c.x > 0.f || c.y > 0.f || c.z > 0.f || c.w > 0.f); left != 0ull; left &= left - 1ull) {
+      const int from = __builtin_ctzll(left);
+      float4 p;
+      p.x = run;
+      p.y = p.x + lane_value(c.x, from);
+      p.z = p.y + lane_value(c.y, from);
+      p.w = p.z + lane_value(c.z, from);
+      run = p.w + lane_value(c.w, from);
+      if (lane == from) own = p;
+    }
+    *reinterpret_cast<float4*>(&l.part[4 * lane]) = own;
+  }
+  __syncthreads();
+}
+
+// The token by the inverse CDF in token order, from e, the threshold and the chunks' kept masses.
+__device__ __forceinline__ void pick_token(const SampleArgs& a, int row, unsigned int thr, const float* masses, PickLds& l) {
+  find_target(a, a.u[row], masses, l);
+  const int chunk = l.chunk_of_target;
+  const float target = l.target, before = l.chunk_start;
   const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
   const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
   // thread t owns the tokens [lo, hi) of the chunk, in token order
@@ -639,27 +676,9 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
   if (live)
 #pragma unroll 4
     for (int i = lo; i < hi; ++i) mine += kept(i);
-  part[threadIdx.x] = mine;
-  __syncthreads();
-  if (threadIdx.x < kWave) {   // exclusive prefix in the threads' order: wave 0, four threads a lane; lanes without mass add nothing
-    const int lane = threadIdx.x;
-    const float4 c = *reinterpret_cast<const float4*>(&part[4 * lane]);
-    float run = before;
-    float4 own = {before, before, before, before};
-    for (unsigned long long left = __ballot(c.x > 0.f || c.y > 0.f || c.z > 0.f || c.w > 0.f); left != 0ull; left &= left - 1ull) {
-      const int l = __builtin_ctzll(left);
-      float4 p;
-      p.x = run;
-      p.y = p.x + lane_value(c.x, l);
-      p.z = p.y + lane_value(c.y, l);
-      p.w = p.z + lane_value(c.z, l);
-      run = p.w + lane_value(c.w, l);
-      if (lane == l) own = p;
-    }
-    *reinterpret_cast<float4*>(&part[4 * lane]) = own;
-  }
-  __syncthreads();
-  const float start = part[threadIdx.x];
+  l.part[threadIdx.x] = mine;
+  add_up_parts(l, before);
+  const float start = l.part[threadIdx.x];
   if (target >= start && target < start + mine && hi > lo) {
     float run = start;
     int pick = -1;
@@ -677,25 +696,385 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
           break;
         }
     }
-    if (pick >= 0) atomicMax(&chosen, pick);
+    if (pick >= 0) atomicMax(&l.chosen, pick);
   }
   __syncthreads();
-  if (chosen < 0) {
+  if (l.chosen < 0) {
     // the target lies outside what the threads found (rounding between the two ways of adding): the last kept
     // token of the chunk, or of the row when the chunk holds none
     int last = -1;
     for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads)
       if (kept(i) > 0.f) last = max(last, i);
-    if (last >= 0) atomicMax(&chosen, last);
+    __syncthreads();   // everybody has looked at `chosen`
+    if (last >= 0) atomicMax(&l.chosen, last);
     __syncthreads();
-    if (chosen < 0) {
+    if (l.chosen < 0) {
       for (int i = threadIdx.x; i < a.vocab; i += kSelThreads)
         if (kept(i) > 0.f) last = max(last, i);
-      if (last >= 0) atomicMax(&chosen, last);
+      __syncthreads();
+      if (last >= 0) atomicMax(&l.chosen, last);
       __syncthreads();
     }
   }
-  if (threadIdx.x == 0) a.out[row] = max(chosen, 0);
+  if (threadIdx.x == 0) a.out[row] = max(l.chosen, 0);
+}
+
+// The token: greedy rows take the first maximum; the others the inverse CDF in token order.
+__global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleArgs a) {
+  __shared__ PickLds l;
+  const int row = blockIdx.x;
+  if (row_params(a, row).greedy) pick_greedy(a, row, l);
+  else pick_token(a, row, a.threshold[row], a.chunk_mass + static_cast<int64_t>(row) * a.chunks, l);
+}
+
+// Rows with a small top_k: everything behind the first histogram in one kernel, a workgroup a row.  The first digit leaves few
+// tokens that may be kept (of 151,936 with top_k 50 some seventy), whose groups' largest e tell where they are: they are
+// gathered into LDS, put into token order, and the threshold of top_k, that of top_p, the chunks' masses and the token come out
+// of comparisons of each with each.  The thresholds are the same values (exact, counts and fixed-point masses); a chunk's mass
+// is added in the order of sample_mass_kernel's threads and waves, a thread's in pick_token's, where what is not kept adds
+// nothing: the same bits, the same token.  A row with more than kFinishMost such tokens (ties) is
+// read once a digit by its workgroup (rows of 151,936 equal logits: 270 to 300 us a call, with the passes of many workgroups 86
+// for one and 256 for 64).
+// 64 rows of 151,936 logits, top_k 50 and top_p 0.9: seven kernels
+// 45 us (5.7 to 8.6 each), this one 15.5; what it is is four trips through memory and steps in LDS.
+constexpr int kFinishMost = 1024, kFinishThreads = 1024;
+
+struct FinishLds {
+  PickLds pick;
+  int count, n_live;
+  unsigned int threshold, ok, digit, rest;
+  unsigned long long left, wave_sum[kFinishThreads / kWave];
+  unsigned int wave_total[kFinishThreads / kWave];
+  float masses[256];
+  int first[256], behind[256];            // of a chunk: its first token in the list, and the one behind its last
+  union {
+    struct {
+      uint2 raw[kFinishMost];               // bits and token, as gathered
+      unsigned int bits[kFinishMost];       // in token order
+      int token[kFinishMost];
+      unsigned long long mass[kFinishMost];
+      int live[kFinishMost];                // groups that hold them
+    } list;
+    struct {
+      unsigned long long bins[kBins1];
+      float wave_mass[256][kSelWaves];
+    };
+  };
+};
+
+// One digit of a threshold of a row by one workgroup: the histogram of digit LEVEL of the tokens that reach `floor` and match the
+// digits so far (counts, or with MASS fixed-point masses) in LDS, and the bin in which, from the top, need(total) is reached.
+// Equal values of a wave are added as one.  False when the whole histogram does not reach it.
+template <int LEVEL, bool MASS, typename Need>
+__device__ __forceinline__ bool row_digit(const float* __restrict__ e, int vocab, unsigned int floor, unsigned int& prefix,
+                                          unsigned long long& rest, Need need_of, FinishLds& l) {
+  constexpr int kBins = LEVEL == 0 ? kBins0 : LEVEL == 1 ? kBins1 : kBins2;
+  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 0 ? 21 : LEVEL == 1 ? 10 : 0, kBits = LEVEL == 1 ? 11 : 10;
+  constexpr int kPer = kBins / kFinishThreads, kAhead = 8;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) l.bins[j * kFinishThreads + tid] = 0ull;
+  if (tid == 0) l.ok = 0u;
+  __syncthreads();
+  for (int base = 0; base < vocab; base += kAhead * kFinishThreads) {
+    float v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = e[min(base + j * kFinishThreads + tid, vocab - 1)];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const unsigned int bits = __float_as_uint(v[j]);
+      const unsigned long long n = MASS ? static_cast<unsigned long long>(v[j] * kMassScale) : 1ull;
+      const bool in = base + j * kFinishThreads + tid < vocab && v[j] >= 0.f && bits >= floor && (LEVEL == 0 || (bits >> kHigh) == prefix) && n != 0ull;
+      const unsigned long long some = __ballot(in);
+      if (some == 0ull) continue;
+      const int lead = __builtin_ctzll(some);
+      const bool like = in && bits == static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(bits), lead));
+      const unsigned long long alike = __ballot(like);
+      if (like ? lane == lead : in)
+        atomicAdd(&l.bins[(bits >> kLow) & (kBins - 1)], like ? n * static_cast<unsigned long long>(__builtin_popcountll(alike)) : n);
+    }
+  }
+  __syncthreads();
+  unsigned long long m[kPer], own = 0ull;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) own += m[j] = l.bins[kPer * tid + j];
+  unsigned long long suffix = own;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned long long other = shfl_any(suffix, min(lane + off, kWave - 1));
+    if (lane + off < kWave) suffix += other;
+  }
+  if (lane == 0) l.wave_sum[wave] = suffix;
+  __syncthreads();
+  unsigned long long above = suffix - own, total = 0ull;
+#pragma unroll
+  for (int w = 0; w < kFinishThreads / kWave; ++w) {
+    total += l.wave_sum[w];
+    if (w > wave) above += l.wave_sum[w];
+  }
+  const unsigned long long need = need_of(total);
+  if (above < need && above + own >= need) {
+#pragma unroll
+    for (int j = kPer - 1; j >= 0; --j) {
+      if (above < need && above + m[j] >= need) l.ok = 1u, l.digit = kPer * tid + j, l.left = need - above;
+      above += m[j];
+    }
+  }
+  __syncthreads();
+  const bool ok = l.ok != 0u;
+  prefix = (LEVEL == 0 ? 0u : prefix << kBits) | l.digit;
+  rest = l.left;
+  __syncthreads();
+  return ok;
+}
+
+// A row that the list does not hold, by the workgroup alone; `s`: what the first histogram gave.
+__device__ __forceinline__ void finish_by_passes(const SampleArgs& a, int row, const RowParams& r, const Slot& s, FinishLds& l) {
+  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  unsigned int thr = s.floor, prefix = s.prefix;
+  unsigned long long rest = s.rest;
+  auto left = [&](unsigned long long) { return rest; };
+  if (!s.open && row_digit<1, false>(e, a.vocab, s.floor, prefix, rest, left, l) && row_digit<2, false>(e, a.vocab, s.floor, prefix, rest, left, l))
+    thr = max(thr, prefix);
+  if (r.p_active) {
+    auto first = [&](unsigned long long total) { return top_p_need(r.top_p, total); };
+    const unsigned int floor = thr;
+    if (row_digit<0, true>(e, a.vocab, floor, prefix, rest, first, l) && row_digit<1, true>(e, a.vocab, floor, prefix, rest, left, l) &&
+        row_digit<2, true>(e, a.vocab, floor, prefix, rest, left, l))
+      thr = max(floor, prefix);
+  }
+  // 256 threads a chunk, as sample_mass_kernel's workgroups
+  const int t = threadIdx.x % kSelThreads, lane = threadIdx.x & (kWave - 1), wave = t / kWave;
+  for (int c = threadIdx.x / kSelThreads; c < a.chunks; c += kFinishThreads / kSelThreads) {
+    const int begin = c * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
+    float mass = 0.f;
+#pragma unroll 8
+    for (int i = begin + t; i < end; i += kSelThreads) {
+      const float v = e[i];
+      if (v >= 0.f && __float_as_uint(v) >= thr) mass += v;
+    }
+    mass = wave_sum(mass);
+    if (lane == 0) l.wave_mass[c][wave] = mass;
+  }
+  __syncthreads();
+  if (threadIdx.x >= kSelThreads) return;      // whole waves: the others' barriers do without them
+  if (static_cast<int>(threadIdx.x) < a.chunks) {
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSelWaves; ++w) total += l.wave_mass[threadIdx.x][w];
+    l.masses[threadIdx.x] = total;
+  }
+  __syncthreads();
+  pick_token(a, row, thr, l.masses, l.pick);
+}
+
+__global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const SampleArgs a) {
+  __shared__ FinishLds l;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  // what is wanted of the row and does not hang on anything else: all on its way at once
+  constexpr int kAhead = 4;
+  const float* gm = a.group_max + static_cast<int64_t>(row) * a.chunks * a.groups;
+  const int groups = a.chunks * a.groups;
+  float most[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) most[j] = gm[min(j * kFinishThreads + tid, groups - 1)];
+  const unsigned int own = a.hist_k[static_cast<int64_t>(row) * kRowBins + tid];
+  const float u = a.u[row];
+  const RowParams r = row_params(a, row);
+  if (r.greedy) {
+    if (tid >= kSelThreads) return;      // whole waves: the others' barriers do without them
+    pick_greedy(a, row, l.pick);
+    return;
+  }
+  const unsigned int mp = min_p_bits(r);
+  if (tid == 0) l.count = l.n_live = 0, l.ok = 0u, l.threshold = mp;
+  for (int c = tid; c < 256; c += kFinishThreads) l.first[c] = l.behind[c] = 0, l.masses[c] = 0.f;
+  // the first digit, a bin a thread
+  static_assert(kFinishThreads == kBins0, "a bin a thread");
+  unsigned int suffix = own;   // over the wave's bins from this one up
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned int other = __shfl(suffix, min(lane + off, kWave - 1), kWave);
+    if (lane + off < kWave) suffix += other;
+  }
+  if (lane == 0) l.wave_total[wave] = suffix;
+  __syncthreads();
+  unsigned int above_bin = suffix - own;
+#pragma unroll
+  for (int w = 0; w < kFinishThreads / kWave; ++w)
+    if (w > wave) above_bin += l.wave_total[w];
+  const unsigned int k = static_cast<unsigned int>(r.k);
+  if (above_bin < k && above_bin + own >= k) l.ok = 1u, l.digit = tid, l.rest = k - above_bin;
+  __syncthreads();
+  const bool open = l.ok == 0u;      // the row does not reach the rank: everything above min_p's floor stays
+  const Slot s{open ? 0ull : static_cast<unsigned long long>(l.rest), open ? 0u : l.digit, mp, open ? 1u : 0u, 0u};
+  // tokens that may be kept, in the groups whose largest e may be.  An e of zero weighs nothing and is never drawn: where the
+  // rank is only reached among those (most logits -inf, say), the others all stay, which is what the list then gives.
+  const unsigned int lower = max(open ? mp : max(mp, s.prefix << 21), 1u);
+  for (int base = 0; base < groups; base += kAhead * kFinishThreads) {
+    if (base > 0) {
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) most[j] = gm[min(base + j * kFinishThreads + tid, groups - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int g = base + j * kFinishThreads + tid;
+      const int chunk = g / a.groups, in_chunk = g - chunk * a.groups;
+      // (a chunk's last groups may lie past its end, and nobody has written those)
+      if (g < groups && in_chunk * kGroup < min(a.chunk_len, a.vocab - chunk * a.chunk_len) && __float_as_uint(most[j]) >= lower) {
+        const int at = atomicAdd(&l.n_live, 1);
+        if (at < kFinishMost) l.list.live[at] = g;
+      }
+    }
+  }
+  __syncthreads();
+  const int n_live = l.n_live;
+  if (n_live <= kFinishMost) {
+    const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+    constexpr int kEach = 8;
+    for (int base = kEach * wave; base < n_live; base += kEach * kFinishThreads / kWave) {
+      float v[kEach];
+      int token[kEach];
+#pragma unroll
+      for (int j = 0; j < kEach; ++j) {
+        const int g = l.list.live[min(base + j, n_live - 1)], chunk = g / a.groups;
+        const int in_chunk = (g - chunk * a.groups) * kGroup + lane;
+        token[j] = base + j < n_live && in_chunk < a.chunk_len ? chunk * a.chunk_len + in_chunk : a.vocab;
+        v[j] = e[min(token[j], a.vocab - 1)];
+      }
+#pragma unroll
+      for (int j = 0; j < kEach; ++j) {
+        if (token[j] < a.vocab && v[j] >= 0.f && __float_as_uint(v[j]) >= lower) {
+          const int at = atomicAdd(&l.count, 1);
+          if (at < kFinishMost) l.list.raw[at] = uint2{__float_as_uint(v[j]), static_cast<unsigned int>(token[j])};
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int n = l.count;
+  if (n_live > kFinishMost || n > kFinishMost) {
+    finish_by_passes(a, row, r, s, l);
+    return;
+  }
+  // four threads a token compare it with all
+  const int quarter = tid & 3;
+  for (int i = tid / 4; i < n; i += kFinishThreads / 4) {
+    const uint2 own_pair = l.list.raw[i];
+    const unsigned int bits = own_pair.x, token = own_pair.y;
+    unsigned int rank = 0, above = 0, reach = 0;
+#pragma unroll 4
+    for (int j = quarter; j < n; j += 4) {
+      const uint2 other = l.list.raw[j];
+      rank += other.y < token;
+      above += other.x > bits;
+      reach += other.x >= bits;
+    }
+    rank += __shfl_xor(rank, 1, kWave), above += __shfl_xor(above, 1, kWave), reach += __shfl_xor(reach, 1, kWave);
+    rank += __shfl_xor(rank, 2, kWave), above += __shfl_xor(above, 2, kWave), reach += __shfl_xor(reach, 2, kWave);
+    if (quarter == 0) {
+      l.list.bits[rank] = bits;
+      l.list.token[rank] = static_cast<int>(token);
+      l.list.mass[rank] = static_cast<unsigned long long>(__uint_as_float(bits) * kMassScale);
+      if (!open && above < k && k <= reach) l.threshold = max(mp, bits);   // the k-th largest, and its ties
+    }
+  }
+  __syncthreads();
+  unsigned int thr = l.threshold;
+  if (r.p_active) {
+    for (int i = tid / 4; i < n; i += kFinishThreads / 4) {
+      const unsigned int bits = l.list.bits[i];
+      unsigned long long above = 0ull, reach = 0ull, total = 0ull;
+#pragma unroll 4
+      for (int j = quarter; j < n; j += 4) {
+        const unsigned int other = l.list.bits[j];
+        const unsigned long long m = other >= thr ? l.list.mass[j] : 0ull;
+        total += m;
+        reach += other >= bits ? m : 0ull;
+        above += other > bits ? m : 0ull;
+      }
+#pragma unroll
+      for (int off = 1; off < 4; off <<= 1) {
+        total += shfl_any(total, lane ^ off);
+        reach += shfl_any(reach, lane ^ off);
+        above += shfl_any(above, lane ^ off);
+      }
+      const unsigned long long need = top_p_need(r.top_p, total);
+      if (quarter == 0 && bits >= thr && above < need && need <= reach) l.digit = bits, l.ok = 2u;
+    }
+    __syncthreads();
+    if (l.ok == 2u) thr = l.digit;
+  }
+  for (int i = tid; i < n; i += kFinishThreads) {
+    const int chunk = l.list.token[i] / a.chunk_len;
+    if (i == 0 || l.list.token[i - 1] / a.chunk_len != chunk) l.first[chunk] = i;
+    if (i == n - 1 || l.list.token[i + 1] / a.chunk_len != chunk) l.behind[chunk] = i + 1;
+  }
+  __syncthreads();
+  for (int c = wave; c < a.chunks; c += kFinishThreads / kWave) {
+    const int from = l.first[c], to = l.behind[c];
+    if (from == to) continue;
+    float mass[kSelWaves] = {};      // what the waves of the chunk's workgroup would have found
+    for (int i = from; i < to; ++i) {
+      const unsigned int bits = l.list.bits[i];
+      const int slot = (l.list.token[i] - c * a.chunk_len) % kSelThreads;
+#pragma unroll
+      for (int w = 0; w < kSelWaves; ++w)
+        if (bits >= thr && slot == w * kWave + lane) mass[w] += __uint_as_float(bits);
+    }
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSelWaves; ++w) total += wave_sum(mass[w]);
+    if (lane == 0) l.masses[c] = total;
+  }
+  __syncthreads();
+
+  // pick_token's steps on the list
+  find_target(a, u, l.masses, l.pick);
+  const int chunk = l.pick.chunk_of_target;
+  const float target = l.pick.target;
+  const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
+  const int per = (end - begin + kSelThreads - 1) / kSelThreads;
+  const bool owns = tid < kSelThreads;
+  const int lo = owns ? min(begin + tid * per, end) : end, hi = owns ? min(lo + per, end) : end;
+  const int from = l.first[chunk], to = l.behind[chunk];
+  auto mine_is = [&](int i) { return l.list.bits[i] >= thr && l.list.token[i] >= lo && l.list.token[i] < hi; };
+  float mine = 0.f;
+  for (int i = from; i < to; ++i)
+    if (mine_is(i)) mine += __uint_as_float(l.list.bits[i]);
+  if (owns) l.pick.part[tid] = mine;
+  add_up_parts(l.pick, l.pick.chunk_start);
+  const float start = owns ? l.pick.part[tid] : 0.f;
+  if (target >= start && target < start + mine && hi > lo) {
+    float run = start;
+    int pick = -1, last = -1;
+    for (int i = from; i < to && pick < 0; ++i) {
+      if (!mine_is(i)) continue;
+      const float v = __uint_as_float(l.list.bits[i]);
+      run += v;
+      if (v > 0.f) last = l.list.token[i];
+      if (target < run) pick = l.list.token[i];
+    }
+    if (pick < 0) pick = last;
+    if (pick >= 0) atomicMax(&l.pick.chosen, pick);
+  }
+  __syncthreads();
+  if (l.pick.chosen < 0) {
+    int in_chunk = -1, in_row = -1;
+    for (int i = tid; i < n; i += kFinishThreads)
+      if (l.list.bits[i] >= thr && l.list.bits[i] > 0u) {
+        in_row = max(in_row, l.list.token[i]);
+        if (l.list.token[i] >= begin && l.list.token[i] < end) in_chunk = max(in_chunk, l.list.token[i]);
+      }
+    __syncthreads();
+    if (in_chunk >= 0) atomicMax(&l.pick.chosen, in_chunk);
+    __syncthreads();
+    const bool none = l.pick.chosen < 0;
+    __syncthreads();
+    if (none && in_row >= 0) atomicMax(&l.pick.chosen, in_row);
+    __syncthreads();
+  }
+  if (tid == 0) a.out[row] = max(l.pick.chosen, 0);
 }
 
 // logits[row, tok] for each (tok, count) listed for the row:
@@ -741,7 +1120,7 @@ extern "C" int arle_argmax_rows(const float* logits, int rows, int vocab, int* o
   if (parts == nullptr) return static_cast<int>(hipErrorInvalidValue);
   const int chunk_len = (((vocab + chunks - 1) / chunks) + 3) & ~3;
   argmax_chunks_kernel<<<dim3(chunks, rows), kChunkThreads, 0, s>>>(logits, vocab, chunk_len,
-                                                                    static_cast<ArgMax*>(parts));
+                                                                    static_cast<ArgMax*>(parts), ClearRows{nullptr, nullptr, 0, 0, 0, 0});
   argmax_merge_kernel<<<rows, kWave, 0, s>>>(static_cast<const ArgMax*>(parts), chunks, out);
   return launch_status();
 }
@@ -761,16 +1140,20 @@ extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
                                 rows * sizeof(unsigned int));
 }
 
+// Rows from whose top_k on the passes of many workgroups are the faster way to the threshold: the tokens that a first digit
+// leaves are at least as many, and the finishing kernel compares each with each.
+extern "C" int arle_sample_finish_most() { return kFinishMost / 4; }
+
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
-// arle_sample_scratch_bytes(rows, vocab) bytes, 8-byte aligned, of which the caller zeroes the first
-// arle_sample_hist_k_bytes(rows) with use_top_k and the arle_sample_hist_p_bytes(rows) behind those with use_top_p.  use_top_k / use_top_p == 0 promise that
-// no row of the call has the filter switched on (top_k in 1..vocab-1, top_p < 1); its passes are then left out.
+// arle_sample_scratch_bytes(rows, vocab) bytes, 16-byte aligned.  use_top_k / use_top_p == 0 promise that no row of the call has
+// the filter switched on (top_k in 1..vocab-1, top_p < 1); its passes are then left out.  small_k != 0 promises that every row is
+// greedy or has a top_k of 1 to arle_sample_finish_most(), below vocab.
 extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float* probs,
                                 const float* temperature, const int* top_k, const float* top_p,
                                 const float* min_p, const float* u, int* out, void* scratch, int use_top_k,
-                                int use_top_p, void* stream) {
+                                int use_top_p, int small_k, void* stream) {
   if (rows == 0) return 0;
-  if (scratch == nullptr || reinterpret_cast<uintptr_t>(scratch) % 8 != 0 || rows > 65535)
+  if (scratch == nullptr || reinterpret_cast<uintptr_t>(scratch) % 16 != 0 || rows > 65535)
     return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
   SampleArgs a;
@@ -804,8 +1187,18 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.use_top_p = use_top_p;
   a.out = out;
   const dim3 grid(a.chunks, rows);
-  argmax_chunks_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, part_max);
+  const bool finish = small_k && use_top_k;
+  // the histograms start at zero: those of the filters that are on, of the finishing kernel's rows the first one
+  const int k_row = kRowBins * sizeof(unsigned int) / 16, p_row = kRowBins * sizeof(unsigned long long) / 16;
+  const ClearRows clear{reinterpret_cast<uint4*>(a.hist_k), reinterpret_cast<uint4*>(a.hist_p),
+                        finish ? static_cast<int>(kBins0 * sizeof(unsigned int) / 16) : (use_top_k ? k_row : 0), k_row,
+                        !finish && use_top_p ? p_row : 0, p_row};
+  argmax_chunks_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, part_max, clear);
   sample_exp_kernel<<<grid, kSelThreads, 0, s>>>(a);
+  if (finish) {
+    sample_finish_kernel<<<rows, kFinishThreads, 0, s>>>(a);
+    return launch_status();
+  }
   if (use_top_k || use_top_p) {
     sample_pass_kernel<kFirst><<<grid, kSelThreads, 0, s>>>(a);
     sample_pass_kernel<kSecond><<<grid, kSelThreads, 0, s>>>(a);

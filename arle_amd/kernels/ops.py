@@ -652,16 +652,18 @@ def _sample_scratch_bytes(rows: int, vocab: int) -> int:
 
 
 @functools.lru_cache(maxsize=None)
-def _sample_hist_bytes(name: str, rows: int) -> int:
-    return int(lib.function_raw(f"arle_sample_hist_{name}_bytes", ctypes.c_longlong, "sampling", (ctypes.c_int,))(rows))
+def sample_small_k() -> int:
+    """The largest top_k that the kernel which finishes a row by itself is for."""
+    return int(lib.function("arle_sample_finish_most")())
 
 
 def sample_rows(logits, temperature, top_k, top_p, min_p, u, *, use_top_k: bool = True,
-                use_top_p: bool = True) -> torch.Tensor:
+                use_top_p: bool = True, small_k: bool = False) -> torch.Tensor:
     """One token id per row; per-row float32 temperature/top_p/min_p/u and int32 top_k.
 
     use_top_k / use_top_p = False promise that no row has that filter switched on (top_k in 1..vocab-1,
-    top_p < 1): the passes over the row that look for its threshold are then not launched.
+    top_p < 1): the passes over the row that look for its threshold are then not launched.  small_k promises that every
+    row is greedy or has a top_k of 1 to `sample_small_k()`, below vocab: one kernel then does what follows the first histogram.
     """
     rows, vocab = _logits(logits)
     for name, t, dt in (("temperature", temperature, torch.float32), ("top_k", top_k, torch.int32),
@@ -671,16 +673,11 @@ def sample_rows(logits, temperature, top_k, top_p, min_p, u, *, use_top_k: bool 
         _need(t.dtype == dt and t.shape == (rows,) and t.is_contiguous(), f"{name} must be {dt} [rows]")
     probs = torch.empty((rows, vocab), dtype=torch.float32, device=logits.device)
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
-    # histograms start at zero, those of the filters that are switched on (64 rows: 3.1 MB with both, the rest 0.6)
     scratch = torch.empty((-(-_sample_scratch_bytes(rows, vocab) // 8),), dtype=torch.int64, device=logits.device)
-    if use_top_k or use_top_p:
-        behind_k = _sample_hist_bytes("k", rows) // 8
-        first = 0 if use_top_k else behind_k
-        scratch[first:behind_k + _sample_hist_bytes("p", rows) // 8 if use_top_p else behind_k].zero_()
     lib.call("arle_sample_rows", logits.data_ptr(), rows, vocab, probs.data_ptr(),
              temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), min_p.data_ptr(),
              u.data_ptr(), out.data_ptr(), scratch.data_ptr(), int(bool(use_top_k)), int(bool(use_top_p)),
-             _stream())
+             int(bool(small_k)), _stream())
     return out
 
 

@@ -139,10 +139,12 @@ class Sampler:
         packed[2] = [p.min_p for p in params]
         packed[3] = uniforms(seeds, indices)
         packed[4].view(np.int32)[:] = [p.top_k for p in params]
+        small = ops.sample_small_k()
         dev = upload(packed, self.device)      # queued: the host does not wait for the step that made the logits
         out = ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3],
                               use_top_k=any(0 < p.top_k < vocab for p, _, _, _ in rows),
-                              use_top_p=any(p.top_p < 1.0 for p, _, _, _ in rows))
+                              use_top_p=any(p.top_p < 1.0 for p, _, _, _ in rows),
+                              small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in params))
         return out
 
     def _penalise(self, logits, rows) -> None:

@@ -36,6 +36,7 @@ _SIGNATURES = {
     "arle_retract_victim": (_i, [_i, _ip, _ip]),
     "arle_plan_prefill": (_i, [_i, _p, _i, _p, _ip, _i, _p, _ip, _ip, _i, _i, _i, _i, _i, _i, _i, _ip, _ip]),
     "arle_aligned_portion": (_i, [_i, _i, _i, _i]),
+    "arle_uniforms": (None, [_i, _p, _p, _p]),
     "arle_admit": (_i, [_i, _ip, _ip, _i, _i, _ip, _ip, _i, _ip, _ip]),
 }
 

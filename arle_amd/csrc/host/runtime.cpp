@@ -445,4 +445,16 @@ int arle_admit(int n_groups, const int* page_size, const int* free_pages, int fr
   return count;
 }
 
+// The draws' uniform numbers in [0, 1): out[i] = the top 24 bits of mix(mix(seeds[i]) ^ indices[i]) / 2^24, exact in a float, where
+// mix is the splitmix64 step.
+void arle_uniforms(int n, const unsigned long long* seeds, const unsigned long long* indices, float* out) {
+  auto mix = [](unsigned long long x) {
+    x += 0x9E3779B97F4A7C15ull;
+    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+    x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+    return x ^ (x >> 31);
+  };
+  for (int i = 0; i < n; ++i) out[i] = static_cast<float>(mix(mix(seeds[i]) ^ indices[i]) >> 40) * (1.0f / 16777216.0f);
+}
+
 }  // extern "C"

@@ -12,9 +12,12 @@ is not kept.
 """
 from __future__ import annotations
 
+from array import array
+
 import numpy as np
 import torch
 
+from ..cache import native
 from ..engine.batch import DeviceToken
 from ..kernels import ops
 from ..kernels.upload import upload
@@ -36,20 +39,21 @@ def uniform(seed: int, index: int) -> float:
     return (_splitmix64(_splitmix64(seed & _MASK) ^ (index & _MASK)) >> 40) / float(1 << 24)
 
 
-def uniforms(seeds, indices) -> np.ndarray:
-    """uniform(seed, index) of every pair, float32.  From sixteen pairs on in arithmetic on whole arrays: sixteen
-    cost about 35 us either way, 64 one by one 131 us and as arrays 36 to 53."""
-    if len(seeds) < 16:
-        return np.array([uniform(s, i) for s, i in zip(seeds, indices)], dtype=np.float32)
+def _words(values) -> array:
+    """The values modulo 2^64."""
+    try:
+        return array("Q", values)
+    except OverflowError:
+        return array("Q", [v & _MASK for v in values])
 
-    def mix(x):
-        x = x + np.uint64(0x9E3779B97F4A7C15)      # wraps, as the mask above does
-        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
-        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
-        return x ^ (x >> np.uint64(31))
-    whole = lambda values: np.array([v & _MASK for v in values], dtype=np.uint64)
-    bits = mix(mix(whole(seeds)) ^ whole(indices)) >> np.uint64(40)
-    return bits.astype(np.float32) * np.float32(1.0 / (1 << 24))   # 24 bits: both steps are exact
+
+def uniforms(seeds, indices) -> np.ndarray:
+    """uniform(seed, index) of every pair, float32, by the host runtime (64 pairs took 46 us in arithmetic on whole arrays,
+    and 6 of these are left)."""
+    out = np.empty(len(seeds), dtype=np.float32)
+    s, i = _words(seeds), _words(indices)
+    native.lib().arle_uniforms(len(out), s.buffer_info()[0], i.buffer_info()[0], out.ctypes.data)
+    return out
 
 
 class Chosen:
@@ -119,33 +123,33 @@ class Sampler:
         """As sample_with_logprobs, but nothing is read back: the kernels are queued and the result stays on the GPU."""
         if logits.shape[0] != len(rows):
             raise ValueError("one sampling row per row of logits is needed")
-        if any(p.has_penalties() and gen for p, _, _, gen in rows):
+        # the parameters that differ: a batch's requests mostly share one object, and every rule below asks them alone
+        kinds = list({id(p): p for p, _, _, _ in rows}.values())
+        if any(p.has_penalties() for p in kinds) and any(p.has_penalties() and gen for p, _, _, gen in rows):
             logits = logits.clone()
             self._penalise(logits, rows)
-        chosen = self._choose(logits, rows)
-        if not any(p.logprobs for p, _, _, _ in rows):
+        chosen = self._choose(logits, rows, kinds)
+        if not any(p.logprobs for p in kinds):
             return Chosen(chosen)
         return Chosen(chosen, ops.token_logprobs(logits, chosen))
 
-    def _choose(self, logits: torch.Tensor, rows) -> torch.Tensor:
-        if all(p.is_greedy() for p, _, _, _ in rows):
+    def _choose(self, logits: torch.Tensor, rows, kinds) -> torch.Tensor:
+        if all(p.is_greedy() for p in kinds):
             return ops.argmax_rows(logits)
         # one host->device copy for the five per-row arrays (top_k travels as the bits of an int32)
-        n, vocab = len(rows), logits.shape[1]
+        n, vocab, small = len(rows), logits.shape[1], ops.sample_small_k()
         packed = np.empty((5, n), dtype=np.float32)
         params, seeds, indices, _ = zip(*rows)
-        packed[0] = [p.temperature for p in params]
-        packed[1] = [p.top_p for p in params]
-        packed[2] = [p.min_p for p in params]
+        column = lambda name: getattr(kinds[0], name) if len(kinds) == 1 else [getattr(p, name) for p in params]
+        packed[0] = column("temperature")
+        packed[1] = column("top_p")
+        packed[2] = column("min_p")
         packed[3] = uniforms(seeds, indices)
-        packed[4].view(np.int32)[:] = [p.top_k for p in params]
-        small = ops.sample_small_k()
+        packed[4].view(np.int32)[:] = column("top_k")
         dev = upload(packed, self.device)      # queued: the host does not wait for the step that made the logits
-        out = ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3],
-                              use_top_k=any(0 < p.top_k < vocab for p, _, _, _ in rows),
-                              use_top_p=any(p.top_p < 1.0 for p, _, _, _ in rows),
-                              small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in params))
-        return out
+        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3],
+                               use_top_k=any(0 < p.top_k < vocab for p in kinds), use_top_p=any(p.top_p < 1.0 for p in kinds),
+                               small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in kinds))
 
     def _penalise(self, logits, rows) -> None:
         indptr, toks, counts = [0], [], []

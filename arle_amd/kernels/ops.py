@@ -1058,7 +1058,7 @@ _WIDE_MOST_ROWS = {(64, 64): 256, (64, 96): 256, (64, 128): 256, (192, 128): 102
 _WIDE_FIXED_US = 4.0
 _XCDS = 8
 _WIDE_MAX_PARTS = 8
-_WIDE_FROM_ROWS = 9             # fewer rows stay with the kernels that stream W through registers
+_WIDE_FROM_ROWS = 9             # by rule; fewer rows stay with the kernels that stream W through registers
 _WIDE_CANDIDATE_SHAPES = 3      # shapes that a tuner tries for a number of parts
 _WIDE_K = 64            # K comes in whole stages
 
@@ -1449,7 +1449,7 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                         found.append(ProductChoice("rounds", (round_steps,)))
         if tiled and eight and n % 32 == 0 and rows > ROWS_KERNEL_MAX:
             found += [ProductChoice("tiles", v) for v in ((4, 44), (8, 144))]
-        if rows >= _WIDE_FROM_ROWS and gemm_wide_supported(n, k, x_stride):
+        if gemm_wide_supported(n, k, x_stride):
             found += [ProductChoice("wide", shape, 0) for shape, _ in wide_shapes(rows, n, k)[:_WIDE_CANDIDATE_SHAPES]]
         return found
     if few:
@@ -1465,7 +1465,7 @@ def product_candidates(rows: int, n: int, k: int, x_stride: int, *, tiled: bool,
                     found.append(ProductChoice("stream", (variant,), parts))
                     if parts in (2, 4, 8):      # and with two workgroups for every compute unit
                         found.append(ProductChoice("stream", (variant, 2 * _STREAM_TARGET_WORKGROUPS // parts), parts))
-    if rows >= _WIDE_FROM_ROWS and gemm_wide_supported(n, k, x_stride):
+    if rows and gemm_wide_supported(n, k, x_stride):
         for parts in range(1, _WIDE_MAX_PARTS + 1):
             if parts == 1 or (k >= 256 * parts and small(parts / 3)):
                 found += [ProductChoice("wide", shape, parts) for shape, _ in wide_shapes(rows, n, k, parts)[:_WIDE_CANDIDATE_SHAPES]]

@@ -1890,14 +1890,14 @@ def mlstm_decode_supported(key_dim: int, value_dim: int, s_state) -> bool:
 def mlstm_decode(y, gates, bias_i, bias_f, cap: float, s_state, n_state, m_state, seg_row0, seg_slot, weight, eps: float, out_dtype, *,
                  heads: int, key_dim: int, value_dim: int):
     """mlstm_scan and mlstm_output for a step of single rows, one a request (no slot comes twice), in one kernel.  y float32
-    [T, 2 H D + 2 H Dv] (q, k, v and the output gate side by side), gates float32 [T, >= 2 H]; either may be a contiguous stack
+    [T, >= 2 H D + 2 H Dv] (q, k, v and the output gate side by side), gates float32 [T, >= 2 H]; either may be a stack
     [S, T, ...] of partial sums, added in order.  Returns [T, H * Dv]."""
     _gpu(y, gates, bias_i, bias_f, s_state, n_state, m_state, seg_row0, seg_slot, weight)
     H, D, Dv = heads, key_dim, value_dim
     tokens, width = y.shape[-2], H * Dv
     for name, t, least in (("y", y, 2 * H * (D + Dv)), ("gates", gates, 2 * H)):
-        _need(t.dtype == torch.float32 and t.dim() in (2, 3) and t.shape[-2] == tokens and t.shape[-1] >= least and t.stride(-1) == 1
-              and (t.dim() == 2 or t.is_contiguous()), f"{name} must be float32 rows of the heads' values, or a contiguous stack")
+        _need(t.dtype == torch.float32 and t.dim() in (2, 3) and t.shape[-2] == tokens and t.shape[-1] >= least and t.stride(-1) == 1,
+              f"{name} must be float32 rows of the heads' values, or a stack")
     _need(mlstm_decode_supported(D, Dv, s_state), "mlstm_decode takes heads of up to 128 x 32, 64 or 128")
     _need(bias_i.shape == (H,) and bias_f.shape == (H,) and bias_i.dtype == bias_f.dtype == torch.float32
           and bias_i.is_contiguous() and bias_f.is_contiguous(), "gate biases must be float32 [heads]")

@@ -59,17 +59,29 @@ class MLSTMMixer(Part):
         fused = [tensors[n] for n in ("q", "k", "v", "g")]
         if len({t.dtype for t in fused}) != 1:
             raise ValueError("q, k, v and gate projections must be stored in one type")
-        self.qkvg = Linear(torch.cat(fused, dim=0).contiguous(), rt.weight_tiles)
         # The gates enter the recurrence: their projection hands over 32-bit sums whatever the mode.  In bfloat16 it
-        # is a product of bfloat16 operands like every projection (rows padded with zeros to whole tiles of 16 outputs),
-        # in float32 the fixed-order 32-bit product.
+        # is a product of bfloat16 operands like every projection (rows padded with zeros to whole pairs of tiles of 16
+        # outputs), in float32 the fixed-order 32-bit product.
         gates = torch.cat([tensors["i"], tensors["f"]], dim=0)
+        self.whole = None
         if gates.dtype == torch.bfloat16 and not rt.is_f32:
-            pad = -gates.shape[0] % 16
+            pad = -gates.shape[0] % 32
             gates = torch.cat([gates, gates.new_zeros((pad, gates.shape[1]))], dim=0) if pad else gates
-            self.gates = Linear(gates.contiguous(), rt.weight_tiles)
+            rows = sum(t.shape[0] for t in fused)
+            if fused[0].dtype == torch.bfloat16 and rows % 16 == 0:
+                # A step of single rows makes both in one product: at 8 rows a second one costs 4.6 us of launch and
+                # ramp for 32 outputs (a step of 8 rows and 8 layers: 774 -> 754 us).  A portion keeps them apart: the
+                # tiles of the wide product would be a column of workgroups more, most of it beyond the last output.
+                self.whole = Linear(torch.cat(fused + [gates], dim=0).contiguous(), rt.weight_tiles)
+                weight, tiles = self.whole.weight, self.whole.tiles
+                self.qkvg = Linear(weight[:rows], packed=tiles)
+                self.gates = Linear(weight[rows:], packed=tiles[rows // 16:] if tiles is not None else None)
+            else:
+                self.gates = Linear(gates.contiguous(), rt.weight_tiles)
         else:
             self.gates = Linear(gates.float().contiguous())
+        if self.whole is None:
+            self.qkvg = Linear(torch.cat(fused, dim=0).contiguous(), rt.weight_tiles)
         self.i_bias, self.f_bias = tensors["i_bias"].float().contiguous(), tensors["f_bias"].float().contiguous()
         self.norm = tensors["norm"]
         self.o = Linear(tensors["o"], rt.weight_tiles)
@@ -87,8 +99,12 @@ class MLSTMMixer(Part):
         # on a single one), and what rounding them to bfloat16 costs there is ten times a usual row's error
         S, n, m = cache["S"].state, cache["n"].state, cache["m"].state
         if not self.rt.is_f32 and batch.max_qlen == 1 and ops.mlstm_decode_supported(self.D, self.Dv, S):
-            y = ops.mlstm_decode(self.qkvg(x, out_dtype=torch.float32, partials_ok=True),
-                                 self.gates(x, out_dtype=torch.float32, partials_ok=True), self.i_bias, self.f_bias, self.cap, S, n, m,
+            if self.whole is not None:
+                p = self.whole(x, out_dtype=torch.float32, partials_ok=True)
+                gates = p[..., self.qkvg.out_features:]
+            else:
+                p, gates = (product(x, out_dtype=torch.float32, partials_ok=True) for product in (self.qkvg, self.gates))
+            y = ops.mlstm_decode(p, gates, self.i_bias, self.f_bias, self.cap, S, n, m,
                                  batch.seg_row0, batch.seg_slot, self.norm, self.eps, self.rt.act_dtype, heads=self.H,
                                  key_dim=self.D, value_dim=self.Dv)
             return self.o(y, out_dtype=torch.float32, partials_ok=True)

@@ -62,6 +62,8 @@ def test_the_memory_in_one_kernel(rows, H, D, Dv, gate_std):
     noise = torch.randn_like(c["qkvg"]) * 0.5
     wide = torch.cat([c["gates"], torch.zeros(rows, 16, device="cuda")], 1).contiguous()
     forms = [(c["qkvg"], c["gates"]), (torch.stack([c["qkvg"] - noise, noise]), torch.stack([wide * 0.25, wide * 0.5, wide * 0.25]))]
+    whole = torch.stack([torch.cat([t, g], 1) for t, g in zip(forms[1][0], (wide * 0.25, wide * 0.75))])     # one product for both
+    forms.append((whole, whole[..., c["qkvg"].shape[1]:]))
     for y, gates in forms:
         mine = [t.clone() for t in c["state"]]
         got = ops.mlstm_decode(y, gates, c["bi"], c["bf"], 15.0, *mine, c["row0"], c["slot"], c["weight"], 1e-6, torch.float32, heads=H,

@@ -87,12 +87,24 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_kernel(
 // The same for the usual types: terms that are float32 (a projection's 32-bit output or its stack of partial
 // products), biases, weights and outputs of one type TA, a width that is a multiple of 4.  Four elements a lane and
 // access, every load of a row issued without a condition on data, before anything is stored.
-template <typename TA, int NT, int PER4>
+//
+// CT > 0: the rows are single ones of different requests, and the first norm's output goes through a causal convolution of CT taps
+// with its input added before it is written (LnConv): a lane holds the same four channels of the row, of the taps and of the
+// request's state, which it moves on, and everything it needs is on its way before the reductions.  One kernel less to
+// wait for in front of every layer; decode steps of 8 rows of 2,560, MI355X: norm 4.8 + convolution 4.4 us before.
+template <typename TA>
+struct LnConv {
+  const TA* w;         // [width, CT]
+  TA* state;           // [slots, CT - 1, width]
+  const int* slot;     // of every row
+};
+
+template <typename TA, int NT, int PER4, int CT>
 __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     float* __restrict__ residual, const float* __restrict__ t0, int n0, long long s0, const TA* __restrict__ b0,
     const float* __restrict__ t1, int n1, long long s1, const TA* __restrict__ b1, const TA* __restrict__ wa,
     const TA* __restrict__ wb, TA* __restrict__ out_a, TA* __restrict__ out_b, const int* __restrict__ rows, int width,
-    float eps, const TA* __restrict__ ca, const TA* __restrict__ cb) {
+    float eps, const TA* __restrict__ ca, const TA* __restrict__ cb, const LnConv<TA> conv) {
   __shared__ float lds[(NT / kWave)];
   const int r = blockIdx.x;
   const int64_t src = rows ? rows[r] : r;
@@ -147,6 +159,20 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     if (!ca) c_a[k] = float4{0.f, 0.f, 0.f, 0.f};
     if (!cb) c_b[k] = float4{0.f, 0.f, 0.f, 0.f};
   }
+  constexpr int BACK = CT > 0 ? CT - 1 : 1, TAPS = CT > 0 ? CT : 1;
+  [[maybe_unused]] float4 before[PER4][BACK], tap[PER4][TAPS];   // the rows before this one, oldest first; 4 channels' taps
+  [[maybe_unused]] TA* mine = nullptr;
+  if constexpr (CT > 0) {
+    mine = conv.state + static_cast<int64_t>(conv.slot[r]) * (CT - 1) * width;
+#pragma unroll
+    for (int k = 0; k < PER4; ++k) {
+      const int i = min((tid + k * NT) * 4, last);
+#pragma unroll
+      for (int j = 0; j < CT - 1; ++j) before[k][j] = ld4<TA>(mine + static_cast<int64_t>(j) * width + i);
+#pragma unroll
+      for (int j = 0; j < CT; ++j) tap[k][j] = ld4<TA>(conv.w + static_cast<int64_t>(i) * CT + 4 * j);
+    }
+  }
   if (t0) add_term(t0, n0, s0, b0);
   if (t1) add_term(t1, n1, s1, b1);
   float sum = 0.f;
@@ -173,8 +199,31 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     const int i = (tid + k * NT) * 4;
     if (i < width) {
       const float4 w = w_a[k], c = c_a[k];
-      st4<TA>(out_a + o + i, float4{fmaf(x[k].x * inv, w.x, c.x), fmaf(x[k].y * inv, w.y, c.y), fmaf(x[k].z * inv, w.z, c.z),
-                                    fmaf(x[k].w * inv, w.w, c.w)});
+      float4 a = float4{fmaf(x[k].x * inv, w.x, c.x), fmaf(x[k].y * inv, w.y, c.y), fmaf(x[k].z * inv, w.z, c.z), fmaf(x[k].w * inv, w.w, c.w)};
+      if constexpr (CT > 0) {
+        // the convolution reads what the norm alone would have written, and adds in the order of conv_step
+        const float now[4] = {to_float(from_float<TA>(a.x)), to_float(from_float<TA>(a.y)), to_float(from_float<TA>(a.z)), to_float(from_float<TA>(a.w))};
+        float wt[4][TAPS], acc[4];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          const float e[4] = {tap[k][j].x, tap[k][j].y, tap[k][j].z, tap[k][j].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) wt[(4 * j + q) / TAPS][(4 * j + q) % TAPS] = e[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = fmaf(wt[q][TAPS - 1], now[q], now[q]);
+#pragma unroll
+        for (int j = CT - 2; j >= 0; --j) {
+          const float v[4] = {before[k][j].x, before[k][j].y, before[k][j].z, before[k][j].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[q] = fmaf(wt[q][j], v[q], acc[q]);
+        }
+#pragma unroll
+        for (int j = 0; j + 1 < CT - 1; ++j) st4<TA>(mine + static_cast<int64_t>(j) * width + i, before[k][j + 1]);
+        st4<TA>(mine + static_cast<int64_t>(CT - 2) * width + i, float4{now[0], now[1], now[2], now[3]});
+        a = float4{acc[0], acc[1], acc[2], acc[3]};
+      }
+      st4<TA>(out_a + o + i, a);
       if (out_b) {
         const float4 v = w_b[k], e = c_b[k];
         st4<TA>(out_b + o + i, float4{fmaf(x[k].x * inv, v.x, e.x), fmaf(x[k].y * inv, v.y, e.y), fmaf(x[k].z * inv, v.z, e.z),
@@ -187,13 +236,18 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
 template <typename TA>
 static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, const void* wa, const void* wb, void* out_a,
                          void* out_b, const int* rows, int n_rows, int width, float eps, const void* ca, const void* cb,
-                         hipStream_t s) {
-#define ARLE_LNV(NT, PER4)                                                                                          \
-  add_layernorm_vec_kernel<TA, NT, PER4><<<n_rows, NT, 0, s>>>(                                                  \
+                         const LnConv<TA>& conv, int taps, hipStream_t s) {
+#define ARLE_LNV_CT(NT, PER4, CT)                                                                                   \
+  add_layernorm_vec_kernel<TA, NT, PER4, CT><<<n_rows, NT, 0, s>>>(                                                  \
       residual, static_cast<const float*>(t0.data), t0.n_stack, t0.stack_stride, static_cast<const TA*>(t0.bias),  \
       static_cast<const float*>(t1.data), t1.n_stack, t1.stack_stride, static_cast<const TA*>(t1.bias),            \
       static_cast<const TA*>(wa), static_cast<const TA*>(wb), static_cast<TA*>(out_a), static_cast<TA*>(out_b), rows, \
-      width, eps, static_cast<const TA*>(ca), static_cast<const TA*>(cb))
+      width, eps, static_cast<const TA*>(ca), static_cast<const TA*>(cb), conv)
+#define ARLE_LNV(NT, PER4)                                                            \
+  do {                                                                                \
+    if (taps == 0) ARLE_LNV_CT(NT, PER4, 0); else if (taps == 2) ARLE_LNV_CT(NT, PER4, 2); \
+    else if (taps == 3) ARLE_LNV_CT(NT, PER4, 3); else ARLE_LNV_CT(NT, PER4, 4);      \
+  } while (0)
   // Workgroups as wide as the row where that is more than 2,048 elements: nearly every load of a row is then on its way at once
   // and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
   // 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
@@ -209,14 +263,15 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
     ARLE_LNV(1024, 1);
   } else if (width <= 5120) {
     ARLE_LNV(640, 2);
-  } else if (width <= 8192 && n_rows < 1024) {
+  } else if (width <= 8192 && (n_rows < 1024 || taps > 0)) {
     ARLE_LNV(1024, 2);
   } else if (width <= 8192) {
-    ARLE_LNV(256, 8);
+    ARLE_LNV_CT(256, 8, 0);
   } else {
-    ARLE_LNV(256, 16);
+    ARLE_LNV_CT(256, 16, 0);
   }
 #undef ARLE_LNV
+#undef ARLE_LNV_CT
   return launch_status();
 }
 
@@ -240,8 +295,8 @@ extern "C" int arle_add_layernorm(float* residual, const void* term0, int n0, lo
   // the usual case: float32 terms, everything else of the output's type, whole groups of four
   const auto fits = [&](const LnTerm& t) { return !t.data || (t.dtype == kF32 && (!t.bias || t.bias_dtype == out_dtype)); };
   if (width % 4 == 0 && fits(t0) && fits(t1) && w_dtype == out_dtype) {
-    return out_dtype == kF32 ? launch_ln_vec<float>(residual, t0, t1, wa, wb, out_a, out_b, rows, n_rows, width, eps, norm_bias_a, norm_bias_b, s)
-                             : launch_ln_vec<bf16>(residual, t0, t1, wa, wb, out_a, out_b, rows, n_rows, width, eps, norm_bias_a, norm_bias_b, s);
+    return out_dtype == kF32 ? launch_ln_vec<float>(residual, t0, t1, wa, wb, out_a, out_b, rows, n_rows, width, eps, norm_bias_a, norm_bias_b, {}, 0, s)
+                             : launch_ln_vec<bf16>(residual, t0, t1, wa, wb, out_a, out_b, rows, n_rows, width, eps, norm_bias_a, norm_bias_b, {}, 0, s);
   }
 #define ARLE_LN(PER)                                                                                          \
   add_layernorm_kernel<PER><<<n_rows, kLnThreads, 0, s>>>(residual, t0, t1, wa, wb, w_dtype, out_a, out_b, \
@@ -255,4 +310,24 @@ extern "C" int arle_add_layernorm(float* residual, const void* term0, int n0, lo
   }
 #undef ARLE_LN
   return launch_status();
+}
+
+// Every row a single one of a request (no slot twice): as arle_add_layernorm, with a convolution of `taps` taps and its own input on
+// the first norm's output and the requests' states moved on.  Terms float32, everything else of `dtype` and on the 16-byte grid;
+// width a multiple of 4 up to 8,192, taps 2 to 4.  conv_w [width, taps], conv_state [slots, taps - 1, width].
+extern "C" int arle_add_layernorm_conv(float* residual, const void* term0, int n0, long long stride0, const void* bias0, const void* term1,
+                                       int n1, long long stride1, const void* bias1, const void* wa, const void* wb, void* out_a,
+                                       void* out_b, int dtype, int n_rows, int width, float eps, const void* norm_bias_a,
+                                       const void* norm_bias_b, const void* conv_w, void* conv_state, const int* slot_of_row, int taps,
+                                       void* stream) {
+  if (n_rows == 0) return 0;
+  const auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (width <= 0 || width > 8192 || width % 4 != 0 || taps < 2 || taps > 4 || (dtype != kF32 && dtype != kBF16) || !at16(conv_w) || !at16(conv_state))
+    return static_cast<int>(hipErrorInvalidValue);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const LnTerm t0{term0, n0, stride0, kF32, bias0, dtype}, t1{term1, n1, stride1, kF32, bias1, dtype};
+  return dtype == kF32 ? launch_ln_vec<float>(residual, t0, t1, wa, wb, out_a, out_b, nullptr, n_rows, width, eps, norm_bias_a, norm_bias_b,
+                                              {static_cast<const float*>(conv_w), static_cast<float*>(conv_state), slot_of_row}, taps, s)
+                       : launch_ln_vec<bf16>(residual, t0, t1, wa, wb, out_a, out_b, nullptr, n_rows, width, eps, norm_bias_a, norm_bias_b,
+                                             {static_cast<const bf16*>(conv_w), static_cast<bf16*>(conv_state), slot_of_row}, taps, s);
 }

@@ -1654,6 +1654,43 @@ def add_layernorm(residual: torch.Tensor, terms, weight: torch.Tensor, eps: floa
     return out if weight_b is None else (out, out_b)
 
 
+def add_layernorm_conv_supported(residual, terms, weight, out_dtype, conv_weight, conv_state, *, weight_b=None, biases=()) -> bool:
+    """Whether add_layernorm_conv takes these: one type throughout beside float32 terms, rows of whole groups of four up to 8,192."""
+    typed = [weight, conv_weight, *(t for t in (weight_b, *biases, *(b for _, b in terms)) if t is not None)]
+    return (residual.shape[1] % 4 == 0 and residual.shape[1] <= 8192 and len(terms) <= 2 and all(t.dtype == torch.float32 for t, _ in terms)
+            and all(t.dtype == out_dtype for t in typed) and conv_step_supported(conv_weight, conv_state))
+
+
+def add_layernorm_conv(residual: torch.Tensor, terms, weight: torch.Tensor, eps: float, out_dtype: torch.dtype, conv_weight, conv_state,
+                       slot_of_token: torch.Tensor, weight_b: torch.Tensor | None = None, *, bias=None, bias_b=None):
+    """add_layernorm and, on its first output, conv_step with its input added (a step of single rows, no slot twice), in one
+    kernel.  Returns (the convolution's rows, the second norm's rows; without `weight_b` those of the norm itself)."""
+    terms = list(terms or [])
+    _gpu(residual, weight, weight_b, bias, bias_b, conv_weight, conv_state, slot_of_token, *[t for pair in terms for t in pair])
+    _need(residual.dtype == torch.float32 and residual.dim() == 2 and residual.is_contiguous(), "residual must be contiguous float32 [T, H]")
+    tokens, width = residual.shape
+    _need(bias_b is None or weight_b is not None, "a second bias without a second weight")
+    if weight_b is None:
+        weight_b, bias_b = weight, bias
+    _need(add_layernorm_conv_supported(residual, terms, weight, out_dtype, conv_weight, conv_state, weight_b=weight_b, biases=(bias, bias_b)),
+          "add_layernorm_conv does not take these")
+    for t in (weight, weight_b, bias, bias_b):
+        _need(t is None or (t.shape == (width,) and t.is_contiguous()), "a norm's weight and bias must be [width]")
+    taps = conv_weight.shape[1]
+    _need(conv_weight.shape[0] == width and conv_state.dim() == 3 and tuple(conv_state.shape[1:]) == (taps - 1, width),
+          "the convolution must be of the norm's width")
+    _i32(slot_of_token, "slot_of_token", tokens)
+    out, out_b = torch.empty((2, tokens, width), dtype=out_dtype, device=residual.device).unbind(0)
+    args = []
+    for i in range(2):
+        data, parts, stride, _, b, _ = _term_args(*(terms[i] if i < len(terms) else (None, None)), residual.shape)
+        args += [data, parts, stride, b]
+    lib.call("arle_add_layernorm_conv", residual.data_ptr(), *args, weight.data_ptr(), weight_b.data_ptr(), out.data_ptr(), out_b.data_ptr(),
+             _code(out), tokens, width, float(eps), _ptr(bias), _ptr(bias_b), conv_weight.data_ptr(), conv_state.data_ptr(),
+             slot_of_token.data_ptr(), taps, _stream())
+    return out, out_b
+
+
 # ------------------------------------------------------------- short causal convolution with state
 
 CONV_MAX_TAPS = 16

@@ -103,12 +103,17 @@ class ParallelBlock:
     def forward(self, residual, delta, batch, cache_view):
         from .base import Pending
 
-        if self.norm_ffn is not None:
+        conv = None
+        if hasattr(self.mixer, "step_conv") and hasattr(self.norm_mixer, "add_norm_conv"):
+            conv = self.mixer.step_conv(batch, cache_view)
+        if conv is not None:    # a step of single rows: the norm's kernel makes the convolution that the mixer begins with
+            a, b = self.norm_mixer.add_norm_conv(residual, delta, conv, also=self.norm_ffn)
+        elif self.norm_ffn is not None:
             a, b = self.norm_mixer.add_norm(residual, delta, also=self.norm_ffn)
         else:
             a = b = self.norm_mixer.add_norm(residual, delta)
         left = Pending()
-        for out in (self.mixer.forward(a, batch, cache_view),
+        for out in (self.mixer.forward(a, batch, cache_view) if conv is None else self.mixer.forward_convolved(a, batch, cache_view),
                     self.feed_forward.forward(b) if self.feed_forward is not None else None):
             if isinstance(out, list):
                 left.extend((term, None) for term in out)

@@ -107,6 +107,21 @@ class LayerNorm(Part):
                                  weight_b=also.weight if also is not None else None, rows=rows, bias=self.bias,
                                  bias_b=also.bias if also is not None else None)
 
+    def add_norm_conv(self, residual, delta, conv, also=None):
+        """`add_norm` for a step of single rows whose mixer begins with a convolution (conv: what its `step_conv` named): that
+        convolution of the norm's rows, and the rows of `also` or, without it, the norm's own."""
+        short_conv, batch, view = conv
+        terms = delta if isinstance(delta, list) else ([] if delta is None else [(delta, None)])
+        other = also if also is not None else self
+        if (also is None or (also.eps == self.eps and also.width == self.width)) and ops.add_layernorm_conv_supported(
+                residual, terms, self.weight, self.rt.act_dtype, short_conv.weight, view.state, weight_b=other.weight,
+                biases=(self.bias, other.bias)):
+            return ops.add_layernorm_conv(residual, terms, self.weight, self.eps, self.rt.act_dtype, short_conv.weight, view.state,
+                                          batch.slot_of_token, other.weight, bias=self.bias, bias_b=other.bias)
+        out = self.add_norm(residual, delta, also=also)
+        a, b = out if also is not None else (out, out)
+        return short_conv(a, batch, view, add_input=True), b
+
 
 @register("norm", "group_rmsnorm")
 class GroupRMSNorm(Part):

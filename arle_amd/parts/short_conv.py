@@ -102,6 +102,15 @@ class InputConvMixer(Part):
     def decode_class_sizes(self):
         return nested_class_sizes((self.inner,))
 
+    def step_conv(self, batch, cache):
+        """(convolution, batch, its state) where the step is one of single rows, so that the norm in front may make the
+        convolution too and `forward_convolved` goes on with its rows; otherwise None."""
+        view = (cache or {}).get("input_conv")
+        return (self.conv, batch, view) if self.conv.takes_parts(batch, view) else None
+
+    def forward_convolved(self, h, batch, cache):
+        return self.inner.forward(h, batch, (cache or {}).get("inner"))
+
     def forward(self, x, batch, cache):
         cache = cache or {}
         h = self.conv(x, batch, cache.get("input_conv"), add_input=True)

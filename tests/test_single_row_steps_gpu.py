@@ -1,6 +1,6 @@
 """Kernels of steps in which every request brings one row: the convolution with its state (`ops.conv_step`) and PolyNorm of a
 stack against the kernels that they stand for, bit for bit (the same sums in the same order, stacks rounded as the kernel that
-adds them does); the mLSTM in one kernel (`ops.mlstm_decode`) against the 64-bit recurrence (bounds as in
+adds them does), and alike for the layer norm with the convolution behind it; the mLSTM in one kernel (`ops.mlstm_decode`) against the 64-bit recurrence (bounds as in
 test_mlstm_chunks_gpu); the layer norm at the edges of its workgroups' widths (two 32-bit passes: 1e-5)."""
 import pytest
 import torch
@@ -87,3 +87,29 @@ def test_layer_norm_at_the_edges_of_its_workgroups(width, rows):
     assert _rel(residual, want) < 1e-6
     d = want - want.mean(-1, keepdim=True)
     assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width,rows,taps", [(4, 1, 2), (1024, 3, 4), (2044, 2, 3), (2560, 8, 4), (4100, 5, 4), (8192, 70, 2)])
+@pytest.mark.parametrize("biased,both", [(False, False), (True, True), (True, False)])
+def test_layer_norm_and_the_convolution_behind_it(dtype, width, rows, taps, biased, both):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width + taps)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    typed = lambda *s: rand(*s).to(dtype)
+    residual, weight, weight_b = rand(rows, width) + 3, typed(width), typed(width) if both else None
+    terms = [(rand(3, rows, width), typed(width)), (rand(rows, width), None)] if biased else []
+    bias, bias_b = typed(width) if biased else None, typed(width) if both else None
+    w, state = typed(width, taps), typed(rows + 2, taps - 1, width)
+    slots = torch.tensor([rows + 1 - r for r in range(rows)], dtype=torch.int32, device="cuda")
+    res, got_state = residual.clone(), state.clone()
+    out = ops.add_layernorm(residual, terms, weight, 1e-6, dtype, weight_b, bias=bias, bias_b=bias_b)
+    norm, other = out if both else (out, out)
+    want = ops.conv_step(norm, w, state, slots, add_input=True)
+    got, got_other = ops.add_layernorm_conv(res, terms, weight, 1e-6, dtype, w, got_state, slots, weight_b, bias=bias, bias_b=bias_b)
+    for a, b in ((got, want), (got_other, other), (got_state, state), (res, residual)):
+        assert torch.equal(a, b)
+    mixed = [(rand(rows, width).bfloat16(), None)]
+    assert not ops.add_layernorm_conv_supported(res, mixed, weight, dtype, w, got_state)
+    assert not ops.add_layernorm_conv_supported(rand(rows, 8196), [], weight, dtype, w, got_state)

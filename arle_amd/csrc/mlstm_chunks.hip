@@ -19,7 +19,7 @@
 //   mlstm_chunk_out     a workgroup a (chunk, head): scores, weights, both products, the denominator, the head norm, the
 //                       norm weight and the output gate
 //
-// Measured on MI355X, 2,048 rows, 20 heads, D = Dv = 128, us a layer: 5 + 42 + 61 (5 + 86 + 61 with the walk) where the
+// Measured on MI355X, 2,048 rows, 20 heads, D = Dv = 128, us a layer: 5 + 47 + 50 (5 + 91 + 50 with the walk) where the
 // token-by-token kernels take 125 (gates) + 708 (memory) + 18 (output); the error of a layer's output against 64 bits is the same (2e-7 to 6e-6 either way).
 // A NaN or an infinity in a row's v spoils that row and the later ones, as token by token (where an infinity meets a
 // state's column with both signs).  The second product would carry it to the chunk's earlier rows too, as a weight of zero
@@ -335,16 +335,23 @@ __global__ __launch_bounds__(kScanThreads) void mlstm_chunk_scan_kernel(const Ml
 
 constexpr int kOutWaves = 4;
 
+// What bounds it: a chunk is 195 KB of loads, then 240 float32 matrix instructions a wave, then its rows' ends, with barriers
+// between, so other workgroups of the compute unit have to fill the waits: three fit (k through LDS in halves of its columns, v and
+// the gate fetched when the registers of what came before are free; two before, with 69 KB of LDS and 244 registers), and a
+// prompt of 2,048 rows and 20 heads, 660 of them, is one turn of the chip instead of one and a third.  No load stands behind a
+// wait that it does not need, the weight comes once through LDS.  65.9 -> 50.5 us a layer at that size.
 template <int KD>
-__global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const MlstmChunkArgs a) {
+__global__ __launch_bounds__(kOutWaves* kWave, 3) void mlstm_chunk_out_kernel(const MlstmChunkArgs a) {
   constexpr int D = 32 * KD;
   constexpr int kQPitch = D + 2;              // a pitch of 2 modulo 64: the 32 rows and two columns of an operand meet 64 banks
   constexpr int kPPitch = kChunkRows + 2;
   constexpr int kOPitch = 128 + 2;
   constexpr int kQFloats = kChunkRows * (kQPitch > kOPitch ? kQPitch : kOPitch);   // q, later the outputs
-  constexpr int kKFloats = kChunkRows * (kQPitch > kPPitch ? kQPitch : kPPitch);   // k, later the weighted scores
+  constexpr int kKPitch = D / 2 + 2;
+  constexpr int kKFloats = kChunkRows * (kKPitch > kPPitch ? kKPitch : kPPitch);   // half of k's columns, then the other, later the weighted scores
   __shared__ __align__(16) float q_lds[kQFloats];
   __shared__ __align__(16) float k_lds[kKFloats];
+  __shared__ __align__(16) float w_lds[128];   // the norm's weight
   __shared__ float n_lds[D], inter[kChunkRows], inv_den[kChunkRows];
   __shared__ ChunkRow row_lds[kChunkRows];
   const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
@@ -356,35 +363,57 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
   const float m0 = a.m0[at * 2];
   const bool has_cols = 32 * wave < Dv;       // the wave's 32 columns of Dv
 
-  // the wave's operands of the state and of v leave for their registers first
-  float s0[D / 2], vr[32];
-  {
-    const float* sp = a.s0 + at * D * Dv + (has_cols ? 32 * wave : 0) + i;
+  float4 kh[2][KD];
 #pragma unroll
-    for (int j = 0; j < D / 2; ++j) s0[j] = sp[static_cast<int64_t>(2 * j + half) * Dv];
-    const float* vp = a.v + static_cast<int64_t>(h) * Dv + (has_cols ? 32 * wave : 0) + i;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) vr[j] = vp[static_cast<int64_t>(c.row0 + min(2 * j + half, c.rows - 1)) * a.row_stride];
+  for (int x = 0; x < 2 * KD; ++x) {
+    const int e = tid + (x % KD) * (kOutWaves * kWave), r = e / (D / 8), d = (e % (D / 8)) * 4 + (x / KD) * (D / 2);
+    kh[x / KD][x % KD] = ld4<float>(a.k + (c.row0 + min(r, c.rows - 1)) * a.row_stride + static_cast<int64_t>(h) * D + d);
   }
-  for (int e = tid; e < kChunkRows * (D / 4); e += kOutWaves * kWave) {
-    const int r = e / (D / 4), d = (e % (D / 4)) * 4;
-    const int64_t t = (c.row0 + min(r, c.rows - 1)) * a.row_stride + static_cast<int64_t>(h) * D + d;
-    const float4 qv = ld4<float>(a.q + t), kv = ld4<float>(a.k + t);
-    float* qd = q_lds + r * kQPitch + d;
-    float* kd = k_lds + r * kQPitch + d;
+  float4 qh[2 * KD];
+#pragma unroll
+  for (int x = 0; x < 2 * KD; ++x) {
+    const int e = tid + x * (kOutWaves * kWave), r = e / (D / 4), d = (e % (D / 4)) * 4;
+    qh[x] = ld4<float>(a.q + (c.row0 + min(r, c.rows - 1)) * a.row_stride + static_cast<int64_t>(h) * D + d);
+  }
+  // (loads without a condition around them: one under a condition is waited for on the spot)
+  const float n_mine = a.n0[at * D + min(tid, D - 1)];
+  const ChunkRow row_mine = a.rows[at * kChunkRows + tid % kChunkRows];
+  const float w_mine = load_as_float(a.weight, a.w_dtype, static_cast<int64_t>(h) * Dv + min(tid, Dv - 1));
+  auto put_keys = [&](const float4 (&from)[KD]) {
+#pragma unroll
+    for (int x = 0; x < KD; ++x) {
+      const int e = tid + x * (kOutWaves * kWave);
+      float* kd = k_lds + e / (D / 8) * kKPitch + (e % (D / 8)) * 4;
+      *reinterpret_cast<float2*>(kd) = float2{from[x].x, from[x].y};
+      *reinterpret_cast<float2*>(kd + 2) = float2{from[x].z, from[x].w};
+    }
+  };
+#pragma unroll
+  for (int x = 0; x < 2 * KD; ++x) {
+    const int e = tid + x * (kOutWaves * kWave);
+    const float4 qv = qh[x];
+    float* qd = q_lds + e / (D / 4) * kQPitch + (e % (D / 4)) * 4;
     *reinterpret_cast<float2*>(qd) = float2{qv.x * a.q_scale, qv.y * a.q_scale};
     *reinterpret_cast<float2*>(qd + 2) = float2{qv.z * a.q_scale, qv.w * a.q_scale};
-    *reinterpret_cast<float2*>(kd) = float2{kv.x, kv.y};
-    *reinterpret_cast<float2*>(kd + 2) = float2{kv.z, kv.w};
   }
-  if (tid < D) n_lds[tid] = a.n0[at * D + tid];
+  put_keys(kh[0]);
+  if (tid < Dv) w_lds[tid] = w_mine;
+  if (tid < D) n_lds[tid] = n_mine;
   if (tid < kChunkRows) {
-    const ChunkRow r = a.rows[at * kChunkRows + tid];
+    const ChunkRow r = row_mine;
     ChunkRow kept = r;
     // M_t = max(m_0, top_t), as a pair
     if (!(r.top_hi > m0 || (r.top_hi == m0 && r.top_lo > 0.f))) kept.top_hi = m0, kept.top_lo = 0.f;
     row_lds[tid] = kept;
     inter[tid] = expf((m0 - kept.top_hi) - kept.top_lo);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // the wave's operands of the state leave for their registers, to be there behind the scores
+  float s0[D / 2];
+  {
+    const float* sp = a.s0 + at * D * Dv + (has_cols ? 32 * wave : 0) + i + half * Dv;
+#pragma unroll
+    for (int j = 0; j < D / 2; ++j) s0[j] = sp[static_cast<int64_t>(2 * j) * Dv];
   }
   __syncthreads();
 
@@ -393,11 +422,19 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
   f32x16 p;
 #pragma unroll
   for (int r = 0; r < 16; ++r) p[r] = 0.f;
-  if (!(rt == 0 && ct == 1)) {
-    const float* qa = q_lds + (32 * rt + i) * kQPitch + half;
-    const float* kb = k_lds + (32 * ct + i) * kQPitch + half;
-#pragma unroll 16
-    for (int j = 0; j < D / 2; ++j) p = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[2 * j], kb[2 * j], p, 0, 0, 0);
+  const bool seen = !(rt == 0 && ct == 1);
+  const float* qa = q_lds + (32 * rt + i) * kQPitch + half;
+  const float* kb = k_lds + (32 * ct + i) * kKPitch + half;
+  if (seen) {
+#pragma unroll 8
+    for (int j = 0; j < D / 4; ++j) p = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[2 * j], kb[2 * j], p, 0, 0, 0);
+  }
+  __syncthreads();   // the first half of k has been read
+  put_keys(kh[1]);
+  __syncthreads();
+  if (seen) {
+#pragma unroll 8
+    for (int j = 0; j < D / 4; ++j) p = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[D / 2 + 2 * j], kb[2 * j], p, 0, 0, 0);
     const ChunkRow key = row_lds[32 * ct + i];
     const int s = 32 * ct + i;
 #pragma unroll
@@ -407,16 +444,22 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
       p[r] = s <= t ? p[r] * w : 0.f;
     }
   }
-  // four threads a row from here on: q . n_0 now, and the output gate's columns 16 x + 4 part .. + 3 on their way
+  // four threads a row from here on: q . n_0 now
   const int my_row = tid >> 2, part = tid & 3;
   const int64_t my_t = c.row0 + min(my_row, c.rows - 1);
   float qn = 0.f;
 #pragma unroll 8
   for (int d = part; d < D; d += 4) qn = fmaf(q_lds[my_row * kQPitch + d], n_lds[d], qn);
-  float4 gate[8];
-  const float* gp = a.gate + my_t * a.row_stride + static_cast<int64_t>(h) * Dv;
+  // the wave's operands of v, to be there behind the state's product (and neither their addresses nor the check of their values earlier:
+  // there are no registers for them)
+  float vr[32];
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const float* vp = a.v + (c.row0 + half) * a.row_stride + static_cast<int64_t>(h) * Dv + (has_cols ? 32 * wave : 0) + i;
+    const int most = c.rows - 1 - half;      // -1 in the second half of a chunk of one row: the row in front again
 #pragma unroll
-  for (int x = 0; x < 8; ++x) gate[x] = ld4<float>(gp + min(16 * x + 4 * part, Dv - 4));
+    for (int j = 0; j < 32; ++j) vr[j] = vp[min(2 * j, most) * a.row_stride];
+  }
   __syncthreads();   // k has been read
 #pragma unroll
   for (int r = 0; r < 16; ++r) k_lds[(32 * rt + 8 * (r / 4) + 4 * half + r % 4) * kPPitch + 32 * ct + i] = p[r];
@@ -451,6 +494,7 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[t][r] *= inter[32 * t + 8 * (r / 4) + 4 * half + r % 4];
+    __builtin_amdgcn_sched_barrier(0);
     const float* p0 = k_lds + i * kPPitch + half;
     float check = 0.f;        // NaN as soon as a value is no finite number
 #pragma unroll
@@ -459,7 +503,8 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
     if (__any(check != 0.f)) {
 #pragma unroll
       for (int j = 31; j >= 0; --j)
-        if (!__builtin_isfinite(vr[j])) spoilt = 2 * j + half, vr[j] = 0.f;
+        if (!__builtin_isfinite(vr[j])) spoilt = 2 * j, vr[j] = 0.f;
+      if (spoilt < kChunkRows) spoilt += half;
       spoilt = min(spoilt, __shfl_xor(spoilt, 32, kWave));
     }
 #pragma unroll
@@ -473,6 +518,11 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
       for (int r = 0; r < 16; ++r)
         if (32 * t + 8 * (r / 4) + 4 * half + r % 4 >= spoilt) acc[t][r] = __builtin_nanf("");
   }
+  // the output gate's columns 16 x + 4 part .. + 3 leave for registers that the state and v are done with
+  float4 gate[8];
+  const float* gp = a.gate + my_t * a.row_stride + static_cast<int64_t>(h) * Dv;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) gate[x] = ld4<float>(gp + min(16 * x + 4 * part, Dv - 4));
   __syncthreads();   // q has been read
   if (has_cols) {
 #pragma unroll
@@ -505,10 +555,12 @@ __global__ __launch_bounds__(kOutWaves* kWave) void mlstm_chunk_out_kernel(const
         const int col = 16 * x + 4 * part;
         if (col >= Dv) continue;
         const int64_t w_at = static_cast<int64_t>(h) * Dv + col;
+        const float4 w4 = *reinterpret_cast<const float4*>(w_lds + col);
+        const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
         const float ov[4] = {o[x].x, o[x].y, o[x].z, o[x].w}, gv[4] = {gate[x].x, gate[x].y, gate[x].z, gate[x].w};
         float y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = ov[e] * inv * load_as_float(a.weight, a.w_dtype, w_at + e) / (1.0f + expf(-gv[e]));
+        for (int e = 0; e < 4; ++e) y[e] = ov[e] * inv * wv[e] / (1.0f + expf(-gv[e]));
         const int64_t to = my_t * H * Dv + w_at;
         if (a.out_dtype == kF32)
           st4<float>(static_cast<float*>(a.out) + to, float4{y[0], y[1], y[2], y[3]});

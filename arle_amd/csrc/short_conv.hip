@@ -178,8 +178,8 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
 }
 
 // A step of single rows, one a request: a lane's four channels of the state belong to nobody else in the step, so it
-// writes them back moved on by its row, and no second kernel has to wait for this one (decode steps of the Gufasun design have
-// twelve of these pairs, 4.4 + 3.9 us each at 8 requests; together 4.6).  PARTS: the input is a stack of float32 partial sums, added in order and
+// writes them back moved on by its row, and no second kernel has to wait for this one (decode steps of the Gufasun design had
+// twelve of these pairs, 4.4 + 3.9 us each at 8 requests; together 4.6; the eight behind a norm are in the norm's kernel now).  PARTS: the input is a stack of float32 partial sums, added in order and
 // rounded to T as the kernel that adds such stacks does.
 template <typename T, int TAPS, bool PARTS>
 __global__ void conv_step_kernel(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,

@@ -709,7 +709,7 @@ _ROWS_PARTIAL_BYTES = 3 << 20    # ... and the float32 partial products stay bel
 _ROWS_WIDE_N = 32768             # from here on (an output head) N alone gives enough workgroups
 _ROWS_NARROW_N = 4096            # up to here N gives so few that one column tile a workgroup is best
 _ROWS_FUSED_MAX = 32             # gate|up with the activation in one go: as many rows as fit into LDS with all of K (27 at K = 2560): 4.20 against 4.41 ms a step at batch 20; more rows: gemm_rows_rounds
-_ROWS_PREFERRED = 16             # with more rows the library is at least as fast on MI355X
+_ROWS_PREFERRED = 16             # with more rows gemm_wide or the library is at least as fast on MI355X
 _V_GENERAL, _V_FUSED_FEW, _V_NARROW, _V_SHARED = 0, 1, 2, 3
 ROWS_VARIANTS = 5
 
@@ -991,7 +991,7 @@ _STREAM_TARGET_WORKGROUPS = 256   # staying workgroups in all: one for every com
 # gain differs from machine to machine), 1.8 % at 4,096; hidden sizes 1,024 and 2,048: level; hidden sizes 4,096 and
 # 5,120: 9 and 8 % slower, so the library keeps those.  Kernel against kernel with cold weights the library's product
 # and the activation kernel take 234-272 us at 2,048 x 19,456 x 2,560 and this kernel 237-255 us; at 8,192 rows the
-# library is ahead.  Plain products stay with the library (q|k|v at 2,048 rows: 85 against 60 us).
+# library is ahead.  Plain products are not for this kernel (q|k|v at 2,048 rows: 85 against the library's 60 us).
 _TILES_MIN_ROWS = 2048
 _TILES_MAX_ROWS = 6144
 _TILES_MIN_N = 4096

@@ -3,9 +3,10 @@
 Which kernel runs depends only on the types of the operands:
 
 * float32 x, float32 W  -> the fixed-order float32 kernel (the true 32-bit path);
-* bfloat16 x, bfloat16 W -> the hand-written MFMA kernel for few rows (decode), the
-  vendor library (hipBLASLt through torch) for many rows, as the reference uses
-  cuBLAS for its projections (infer/src/ops/linear.rs:921-959);
+* bfloat16 x, bfloat16 W -> the kernel that ops.choose_product names for the sizes: hand-written
+  MFMA kernels for few rows (decode) and, where they were measured ahead, for many, else the
+  vendor library (hipBLASLt through torch), as the reference uses cuBLAS for its projections
+  (infer/src/ops/linear.rs:921-959);
 * bfloat16 x, float32 W (a tensor that the checkpoint stores in 32 bits stays so):
   x is widened and the float32 kernel runs.
 

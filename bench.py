@@ -77,7 +77,7 @@ def _template_args(name: str) -> list:
 
 def _completes_gate_up(name: str) -> bool:
     """Whether this kernel leaves gate|up complete: a product with the activation fused (gemm_rows_kernel<MT, WN,
-    WK, PD, XD, EPI, out> / gemm_tiles_kernel<MT, TN, PD, PX, PIPE, EPI, out> / gemm_wide_kernel<WM, WN, TM, TN, EPI, out>
+    WK, PD, XD, EPI, out> / gemm_tiles_kernel<MT, TN, PD, PX, PIPE, EPI, out> / gemm_wide_kernel<WM, WN, TM, TN, stages, EPI, out>
     with EPI = 1), or the activation kernel
     behind a plain product."""
     if "silu_mul" in name:
@@ -85,10 +85,8 @@ def _completes_gate_up(name: str) -> bool:
     args = _template_args(name)
     if "gemm_rows_kernel" in name:
         return len(args) > 5 and args[5] == "1"
-    if "gemm_tiles_kernel" in name:
+    if "gemm_tiles_kernel" in name or "gemm_wide_kernel" in name:
         return len(args) > 5 and args[5] == "1"
-    if "gemm_wide_kernel" in name:
-        return len(args) > 4 and args[4] == "1"
     return False
 
 
@@ -768,10 +766,11 @@ def gufasun_work(raw: dict, q: dict, tokens: int, batch: int, context: int) -> d
         "add_layernorm": ((L + 1) * tokens * W * (4 + 4 + 4 + 4 + 2 + 2), 0),
         "causal_conv": (tokens * 2 * 2 * (L * W + n_own * (Q + 2 * KV) + (n_att - n_own) * Q), 0),
         "polynorm": (L * tokens * F * 4, 0),
-        "qkv_norm_store_kernel": (tokens * 2 * 2 * (n_own * (Q + 2 * KV) + (n_att - n_own) * Q), 0),
+        "qkv_norm_store": (tokens * 2 * 2 * (n_own * (Q + 2 * KV) + (n_att - n_own) * Q), 0),
         "attn_softcap_mfma_kernel": (n_att * batch * 2 * KV * 2 * keys if decode else 0,
                                      n_att * tokens * keys * a["heads"] * 2 * (a["dim"] + a["vdim"])),
         "mlstm_memory_kernel": (n_mem * batch * S * 4 * 2, n_mem * tokens * S * 4),
+        "mlstm_decode_kernel": (n_mem * batch * S * 4 * 2, n_mem * tokens * S * 4),      # a step of single rows
         "mlstm_gates_kernel": (n_mem * tokens * m["heads"] * m["dim"] * 2 * 2, 0),
         "mlstm_output_kernel": (n_mem * tokens * m["heads"] * m["vdim"] * (4 + 2 + 2), 0),
     }

@@ -1365,8 +1365,11 @@ def gemm_wide_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
     return least is not None and (rows >= least or _WIDE_TWO_BLOCKS[0] <= rows <= _WIDE_TWO_BLOCKS[1])
 
 
-# Plain products by gemm_wide, for widths that no table names: outputs of 5,120 columns and more, whole sums (where a stack
-# of partial sums is welcome, the kernels of few rows keep theirs).  MI355X, cold weights, us, the other rules / gemm_wide:
+# Plain products by gemm_wide, for widths that no table names: outputs of 5,120 columns and more.  Sums are whole, but where a
+# stack of partial sums is welcome the kernels of few rows keep theirs, and where the library would leave one (N 5,120, K 2,048
+# to 5,120, 65 to 1,024 rows) gemm_wide leaves one of two parts.  With the norm that adds it, us, library in its parts / two parts
+# / four: K 2,048 97 rows 23.1 / 15.2 / 16.0, 512 36.7 / 26.4 / 30.9, 1,024 45.6 / 41.7 / 54.1; K 5,120 97 rows 28.5 / 25.1 / 21.9,
+# 192 42.4 / 27.9 / 26.5, 512 46.4 / 41.5 / 41.5, 1,024 69.0 / 64.6 / 74.7.  Whole sums otherwise: MI355X, cold weights, us, the other rules / gemm_wide:
 #   up to 1,024 rows: N 9,728, K 2,560 9 rows 15.2 / 14.8, 32 16.6 / 14.5, 64 19.5 / 17.3, 128 24.7 / 20.1, 256 38.4 / 26.3, 512
 #     37.7 / 32.5, 1,024 56.1 / 47.7; N 5,120, K 5,120 192 rows 43.7 / 27.3, 512 49.3 / 42.0, 1,024 63.8 / 56.1; N 16,384, K 5,120
 #     16 rows 45.8 / 30.2, 64 36.7 / 32.4, 256 66.8 / 56.1; narrower ones go either way (N 4,096, K 2,560 9 rows 10.2 / 12.1,
@@ -1378,10 +1381,11 @@ def gemm_wide_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
 _WIDE_PLAIN_MIN_N = 5120
 _WIDE_PLAIN_MAX_K = 5120
 _WIDE_PLAIN_ANY_SHAPE_ROWS = 1024
+_WIDE_PLAIN_PARTS = 2
 
 
 def gemm_wide_plain_preferred(rows: int, n: int, k: int, x_stride: int) -> bool:
-    """Whether a plain product runs whole in gemm_wide (the rule for widths that no table names)."""
+    """Whether a plain product runs in gemm_wide (the rule for widths that no table names)."""
     if rows < _WIDE_FROM_ROWS or n < _WIDE_PLAIN_MIN_N or k > _WIDE_PLAIN_MAX_K or not gemm_wide_supported(n, k, x_stride):
         return False
     return rows <= _WIDE_PLAIN_ANY_SHAPE_ROWS or wide_plan(rows, n, k)[0] == (256, 320)
@@ -1408,7 +1412,8 @@ def product_by_rules(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, f
     staying = aligned and gemm_stream_preferred(rows, n, k, x_stride, tiled=tiled)
     few = staying or (aligned and gemm_rows_preferred(rows, n, k, x_stride))
     if not (few and partials_ok) and aligned and w_aligned and gemm_wide_plain_preferred(rows, n, k, x_stride):
-        return ProductChoice("wide", (), 1)
+        # where the consumer would be left 32-bit parts by the library, it is left them here too: whole, the sums would be rounded
+        return ProductChoice("wide", (), _WIDE_PLAIN_PARTS if partials_ok and library_k_splits(rows, n, k) > 1 else 1)
     if few and not staying:
         return ProductChoice("rows")
     if staying:

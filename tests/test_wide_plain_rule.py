@@ -30,6 +30,19 @@ def test_sums_that_may_stay_in_parts_stay_unrounded(rows):
     assert with_parts.kernel in ("rows", "stream")
 
 
+@pytest.mark.parametrize("k", [2048, 2560, 3072, 4096, 5120])
+def test_sums_that_the_library_would_leave_in_parts_stay_unrounded(k):
+    """o and down at 5,120 columns (no table names them): rounded to bfloat16 they would go into the 32-bit residual with fewer bits."""
+    for rows in (65, 66, 97, 128, 192, 255, 256, 257, 384, 512, 513, 768, 1000, 1024):
+        assert ops.library_k_splits(rows, 5120, k) > 1
+        for tiled in (False, True):
+            choice = ops.choose_product(rows, 5120, k, k, tiled=tiled, fused=False, partials_ok=True)
+            assert choice.kernel in ("wide", "library_parts") and choice.splits > 1
+            assert ops.product_by_rules(rows, 5120, k, k, tiled=tiled, fused=False, partials_ok=False) == ops.ProductChoice("wide", (), 1)
+            off = ops.product_by_rules(rows, 5120, k, k, tiled=tiled, fused=False, partials_ok=True, w_aligned=False)
+            assert off.kernel == "library_parts"
+
+
 @pytest.mark.parametrize("rows,n,k", [(9, 6144, 2560), (64, 2560, 9728), (256, 4096, 2560), (257, 4096, 2560), (1024, 6144, 4096),
                                       (1025, 6144, 4096), (8192, 19456, 2560)])
 def test_shapes_stay_within_their_rows(rows, n, k):

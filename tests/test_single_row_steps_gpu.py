@@ -89,6 +89,30 @@ def test_layer_norm_at_the_edges_of_its_workgroups(width, rows):
     assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5
 
 
+@pytest.mark.parametrize("width", [2052, 4100, 5120, 5124, 6144, 8192, 8196])
+def test_a_float32_row_of_the_layer_norm_is_the_same_bits_in_any_step(width):
+    from arle_amd.kernels import ops
+
+    rows, taps = 1100, 3
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    residual, term, weight = rand(rows, width) + 3, rand(rows, width), rand(width)
+    at = [slice(0, 1), slice(1, 9), slice(9, 1032), slice(1032, 1100)]
+    sums = residual.clone()
+    whole = ops.add_layernorm(sums, [(term, None)], weight, 1e-6, torch.float32)
+    pieces = [ops.add_layernorm(residual[s].clone(), [(term[s], None)], weight, 1e-6, torch.float32) for s in at]
+    assert torch.equal(torch.cat(pieces), whole)
+    d = residual.double() + term.double()
+    d = d - d.mean(-1, keepdim=True)
+    assert _rel(whole, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5
+    w, state = rand(width, taps), rand(1100, taps - 1, width)
+    slots = torch.arange(8, dtype=torch.int32, device="cuda")
+    if ops.add_layernorm_conv_supported(residual, [(term, None)], weight, torch.float32, w, state):
+        few = slice(0, 8)
+        _, norm = ops.add_layernorm_conv(residual[few].clone(), [(term[few], None)], weight, 1e-6, torch.float32, w, state, slots)
+        assert torch.equal(norm, whole[few])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("width,rows,taps", [(4, 1, 2), (1024, 3, 4), (2044, 2, 3), (2560, 8, 4), (4100, 5, 4), (8192, 70, 2)])
 @pytest.mark.parametrize("biased,both", [(False, False), (True, True), (True, False)])

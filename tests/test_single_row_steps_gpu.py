@@ -53,6 +53,21 @@ def test_polynorm_of_a_stack(dtype, width):
         assert _rel(got, want) < (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5)
 
 
+@pytest.mark.parametrize("width", [2052, 4100, 6144, 8192, 8196])
+def test_a_float32_row_of_polynorm_is_the_same_bits_in_any_step(width):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    u, coef = torch.randn(1100, width, generator=gen, device="cuda"), torch.randn(4, generator=gen, device="cuda")
+    whole = ops.polynorm(u, coef, 1e-6)
+    pieces = [ops.polynorm(u[s].contiguous(), coef, 1e-6) for s in (slice(0, 1), slice(1, 9), slice(9, 1032), slice(1032, 1100))]
+    assert torch.equal(torch.cat(pieces), whole)
+    assert torch.equal(ops.polynorm(u[None, :64].contiguous(), coef, 1e-6, out_dtype=torch.float32), whole[:64])
+    z, n = u.double(), lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-6)
+    c = coef.double()
+    assert _rel(whole, c[0] * n(z) + c[1] * n(z ** 2) + c[2] * n(z ** 3) + c[3]) < 1e-5
+
+
 @pytest.mark.parametrize("rows,H,D,Dv,gate_std", [(1, 2, 128, 128, 1.0), (5, 3, 100, 64, 3.0), (9, 1, 32, 32, 20.0), (3, 2, 128, 32, 1.0), (2, 2, 7, 128, 1.0)])
 def test_the_memory_in_one_kernel(rows, H, D, Dv, gate_std):
     from arle_amd.kernels import ops

@@ -119,9 +119,12 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     float4 d[PER4];
 #pragma unroll
     for (int k = 0; k < PER4; ++k) d[k] = ld4<float>(t + base + min((tid + k * NT) * 4, last));
-    // the parts of a stack are fetched several at a time (eight for rows up to 4,096 wide) without a condition (a part past the last is the last one
-    // again, fetched and dropped), so that their loads are in flight together; they are added in the stack's order
-    constexpr int G = PER4 <= 4 ? 8 : (PER4 <= 8 ? 4 : 2);
+    // the parts of a stack are fetched several at a time without a condition (a part past the last is the last one again, fetched
+    // and dropped), so that their loads are in flight together; they are added in the stack's order.  Two at a time where a lane
+    // has eight elements and their taps besides: more do not fit the registers of 1,024 lanes (8 rows of 8,192, taps 4, two terms of
+    // 4 and 2 parts, us, eight / four / two at a time: bfloat16 12.4 / 9.1 / 8.6, float32 24.7 / 13.5 / 9.8, which spill; 5,120 wide 8.2 /
+    // 7.1 / 6.7 and 9.6 / 7.6 / 7.4)
+    constexpr int G = PER4 == 2 && NT > 256 && CT > 0 ? 2 : PER4 <= 4 ? 8 : (PER4 <= 8 ? 4 : 2);
     for (int s0 = 1; s0 < n; s0 += G) {
       float4 e[G][PER4];
 #pragma unroll

@@ -152,3 +152,22 @@ def test_layer_norm_and_the_convolution_behind_it(dtype, width, rows, taps, bias
     mixed = [(rand(rows, width).bfloat16(), None)]
     assert not ops.add_layernorm_conv_supported(res, mixed, weight, dtype, w, got_state)
     assert not ops.add_layernorm_conv_supported(rand(rows, 8196), [], weight, dtype, w, got_state)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4096, 5120, 8192])
+@pytest.mark.parametrize("parts", [1, 2, 3, 8])
+def test_stacks_in_front_of_the_norm_with_a_convolution(dtype, width, parts):
+    """Stacks of as many parts as are fetched at a time, fewer and more: bit for bit as without the convolution."""
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width + parts)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    residual, terms = rand(2, width), [(rand(parts, 2, width), rand(width).to(dtype)), (rand(4 - min(parts, 3), 2, width), None)]
+    weight, w, state = rand(width).to(dtype), rand(width, 4).to(dtype), rand(3, 3, width).to(dtype)
+    slots = torch.tensor([2, 0], dtype=torch.int32, device="cuda")
+    res, got_state = residual.clone(), state.clone()
+    norm = ops.add_layernorm(residual, terms, weight, 1e-6, dtype)
+    want = ops.conv_step(norm, w, state, slots, add_input=True)
+    got, other = ops.add_layernorm_conv(res, terms, weight, 1e-6, dtype, w, got_state, slots)
+    assert all(torch.equal(a, b) for a, b in ((got, want), (other, norm), (got_state, state), (res, residual)))

@@ -125,13 +125,15 @@ static int launch_pn_vec(const void* u, long long u_stride, int parts, long long
   polynorm_vec_kernel<T, NT, PER4, PARTS><<<tokens, NT, 0, s>>>(u, u_stride, parts, part_stride, static_cast<const T*>(bias), \
                                                                 static_cast<const T*>(coef), static_cast<T*>(out), width, eps)
   // 512 lanes where a row has more than two accesses for each; MI355X, us, 256 lanes / 512: 9,728 wide 8 rows 5.2 / 4.6, 2,048
-  // 19.6 / 18.6; 12,288 wide 5.5 / 5.0, 22.4 / 20.6; 6,144 wide 4.5 / 4.2, 13.3 / 14.8; 2,048 wide 3.5 / 3.7, 7.1 / 10.0.  The
-  // step's rows count in bfloat16 only: a float32 row's sums have one order in every step.
+  // 19.6 / 18.6; 12,288 wide 5.5 / 5.0, 22.4 / 20.6; 2,048 wide 3.5 / 3.7, 7.1 / 10.0.  Between 4,097 and 8,192 it is the step's rows
+  // that decide: 4,100 wide 8 rows 4.4 / 4.1, 256 4.7 / 4.5, 384 5.3 / 5.4, 1,024 7.1 / 7.4, 4,096 18.0 / 21.2; 6,144 wide 256 rows
+  // 5.1 / 4.8, 384 5.7 / 5.7, 1,024 8.4 / 8.7; 8,192 wide 8 rows 5.0 / 4.7, 256 5.2 / 5.1, 384 6.0 / 6.3, 768 7.5 / 8.3, 4,096 23.9 /
+  // 28.2.  They count in bfloat16 only: a float32 row's sums have one order in every step.
   if (width <= 2048) {
     ARLE_PNV(256, 2);
   } else if (width <= 4096) {
     ARLE_PNV(256, 4);
-  } else if (!std::is_same<T, float>::value && width <= 8192 && tokens >= 1024) {
+  } else if (!std::is_same<T, float>::value && width <= 8192 && tokens > 256) {
     if constexpr (!std::is_same<T, float>::value) ARLE_PNV(256, 8);
   } else if (width <= 6144) {
     ARLE_PNV(512, 3);

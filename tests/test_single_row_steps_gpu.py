@@ -68,6 +68,18 @@ def test_a_float32_row_of_polynorm_is_the_same_bits_in_any_step(width):
     assert _rel(whole, c[0] * n(z) + c[1] * n(z ** 2) + c[2] * n(z ** 3) + c[3]) < 1e-5
 
 
+@pytest.mark.parametrize("rows", [256, 257, 1025])
+@pytest.mark.parametrize("width", [4096, 4100, 8192, 8196])
+def test_polynorm_of_many_bfloat16_rows(width, rows):
+    """Both sides of the line between the workgroups; rounded once, half a unit in the last place: 2^-9 of a value, 2^-8 stated."""
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width + rows)
+    u, coef = (torch.randn(*s, generator=gen, device="cuda").bfloat16() for s in ((rows, width), (4,)))
+    z, c, n = u.double(), coef.double(), lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-6)
+    assert _rel(ops.polynorm(u, coef, 1e-6), c[0] * n(z) + c[1] * n(z ** 2) + c[2] * n(z ** 3) + c[3]) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("rows,H,D,Dv,gate_std", [(1, 2, 128, 128, 1.0), (5, 3, 100, 64, 3.0), (9, 1, 32, 32, 20.0), (3, 2, 128, 32, 1.0), (2, 2, 7, 128, 1.0)])
 def test_the_memory_in_one_kernel(rows, H, D, Dv, gate_std):
     from arle_amd.kernels import ops

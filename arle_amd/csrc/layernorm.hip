@@ -257,8 +257,9 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
   // and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
   // 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
   // wide 8.2 / 6.2, 2,048 rows 68.7 / 60.8.  Narrower rows need several a compute unit (1,536 wide, 2,048 rows 20.0 / 27.1), and
-  // so do many rows of 8,192 (8 rows 8.7 / 7.9, 2,048 86.2 / 89.8), in bfloat16: a float32 row's sums have one order in every
-  // step, so the width alone chooses there.
+  // so do many rows beyond 5,120: 6,144 wide 8 rows 8.4 / 7.8, 256 9.5 / 9.5, 512 19.6 / 17.7, 1,536 48.4 / 46.8, 2,048 62.2 / 60.7,
+  // 4,096 139.5 / 158.9; 8,192 wide 8.7 / 7.9, 11.3 / 10.6, 23.6 / 20.1, 62.6 / 55.2, 87.6 / 86.6, 172.7 / 177.5 (elsewhere 2,048 rows 86.2 /
+  // 89.8).  In bfloat16: a float32 row's sums have one order in every step, so the width alone chooses there.
   if (width <= 1024) {
     ARLE_LNV(256, 1);
   } else if (width <= 2048) {
@@ -269,7 +270,7 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
     ARLE_LNV(1024, 1);
   } else if (width <= 5120) {
     ARLE_LNV(640, 2);
-  } else if (width <= 8192 && (std::is_same<TA, float>::value || n_rows < 1024 || taps > 0)) {
+  } else if (width <= 8192 && (std::is_same<TA, float>::value || n_rows < 2048 || taps > 0)) {
     ARLE_LNV(1024, 2);
   } else if (width <= 8192) {
     if constexpr (!std::is_same<TA, float>::value) ARLE_LNV_CT(256, 8, 0);

@@ -116,6 +116,22 @@ def test_layer_norm_at_the_edges_of_its_workgroups(width, rows):
     assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5
 
 
+@pytest.mark.parametrize("rows", [2047, 2048])
+@pytest.mark.parametrize("width", [5124, 8192])
+def test_layer_norm_of_many_bfloat16_rows(width, rows):
+    """Both sides of the line between the workgroups; rounded once, half a unit in the last place: 2^-9 of a value, 2^-8 stated."""
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width + rows)
+    residual, term = (torch.randn(rows, width, generator=gen, device="cuda") + 3 for _ in range(2))
+    weight = torch.randn(width, generator=gen, device="cuda").bfloat16()
+    want = residual.double() + term.double()
+    got = ops.add_layernorm(residual, [(term, None)], weight, 1e-6, torch.bfloat16)
+    d = want - want.mean(-1, keepdim=True)
+    assert _rel(residual, want) < 1e-6
+    assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("width", [2052, 4100, 5120, 5124, 6144, 8192, 8196])
 def test_a_float32_row_of_the_layer_norm_is_the_same_bits_in_any_step(width):
     from arle_amd.kernels import ops

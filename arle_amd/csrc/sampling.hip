@@ -564,12 +564,16 @@ struct PickLds {
   int chunk_of_target, chosen;
 };
 
+// What follows is the work of the first kSelThreads threads of a workgroup, whose others, if it has any, come along from barrier to
+// barrier.
+
 // A greedy row's token: the first maximum.
 __device__ __forceinline__ void pick_greedy(const SampleArgs& a, int row, PickLds& l) {
   ArgMax m;
   m.v = -INFINITY;
   m.i = 0x7fffffff;
-  for (int c = threadIdx.x; c < a.chunks; c += kSelThreads)
+  const bool owns = threadIdx.x < kSelThreads;
+  for (int c = threadIdx.x; owns && c < a.chunks; c += kSelThreads)
     m = better(m, a.part_max[static_cast<int64_t>(row) * a.chunks + c]);
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) {
@@ -578,7 +582,7 @@ __device__ __forceinline__ void pick_greedy(const SampleArgs& a, int row, PickLd
     o.i = __shfl_xor(m.i, off, kWave);
     m = better(m, o);
   }
-  if (threadIdx.x % kWave == 0) l.best[threadIdx.x / kWave] = m;
+  if (owns && threadIdx.x % kWave == 0) l.best[threadIdx.x / kWave] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
     ArgMax t = l.best[0];
@@ -663,7 +667,8 @@ __device__ __forceinline__ void pick_token(const SampleArgs& a, int row, unsigne
   const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
   // thread t owns the tokens [lo, hi) of the chunk, in token order
   const int per = (end - begin + kSelThreads - 1) / kSelThreads;
-  const int lo = min(begin + static_cast<int>(threadIdx.x) * per, end), hi = min(lo + per, end);
+  const bool owns = threadIdx.x < kSelThreads;
+  const int lo = owns ? min(begin + static_cast<int>(threadIdx.x) * per, end) : end, hi = min(lo + per, end);
   auto kept = [&](int i) {
     const float v = e[i];
     return (v >= 0.f && __float_as_uint(v) >= thr) ? v : 0.f;
@@ -676,9 +681,9 @@ __device__ __forceinline__ void pick_token(const SampleArgs& a, int row, unsigne
   if (live)
 #pragma unroll 4
     for (int i = lo; i < hi; ++i) mine += kept(i);
-  l.part[threadIdx.x] = mine;
+  if (owns) l.part[threadIdx.x] = mine;
   add_up_parts(l, before);
-  const float start = l.part[threadIdx.x];
+  const float start = owns ? l.part[threadIdx.x] : 0.f;
   if (target >= start && target < start + mine && hi > lo) {
     float run = start;
     int pick = -1;
@@ -703,13 +708,13 @@ __device__ __forceinline__ void pick_token(const SampleArgs& a, int row, unsigne
     // the target lies outside what the threads found (rounding between the two ways of adding): the last kept
     // token of the chunk, or of the row when the chunk holds none
     int last = -1;
-    for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kSelThreads)
+    for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += blockDim.x)
       if (kept(i) > 0.f) last = max(last, i);
     __syncthreads();   // everybody has looked at `chosen`
     if (last >= 0) atomicMax(&l.chosen, last);
     __syncthreads();
     if (l.chosen < 0) {
-      for (int i = threadIdx.x; i < a.vocab; i += kSelThreads)
+      for (int i = threadIdx.x; i < a.vocab; i += blockDim.x)
         if (kept(i) > 0.f) last = max(last, i);
       __syncthreads();
       if (last >= 0) atomicMax(&l.chosen, last);
@@ -857,7 +862,6 @@ __device__ __forceinline__ void finish_by_passes(const SampleArgs& a, int row, c
     if (lane == 0) l.wave_mass[c][wave] = mass;
   }
   __syncthreads();
-  if (threadIdx.x >= kSelThreads) return;      // whole waves: the others' barriers do without them
   if (static_cast<int>(threadIdx.x) < a.chunks) {
     float total = 0.f;
 #pragma unroll
@@ -882,7 +886,6 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const Sam
   const float u = a.u[row];
   const RowParams r = row_params(a, row);
   if (r.greedy) {
-    if (tid >= kSelThreads) return;      // whole waves: the others' barriers do without them
     pick_greedy(a, row, l.pick);
     return;
   }

@@ -732,134 +732,273 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
   else pick_token(a, row, a.threshold[row], a.chunk_mass + static_cast<int64_t>(row) * a.chunks, l);
 }
 
-// Rows with a small top_k: everything behind the first histogram in one kernel, a workgroup a row.  The first digit leaves few
-// tokens that may be kept (of 151,936 with top_k 50 some seventy), whose groups' largest e tell where they are: they are
-// gathered into LDS, put into token order, and the threshold of top_k, that of top_p, the chunks' masses and the token come out
-// of comparisons of each with each.  The thresholds are the same values (exact, counts and fixed-point masses); a chunk's mass
-// is added in the order of sample_mass_kernel's threads and waves, a thread's in pick_token's, where what is not kept adds
-// nothing: the same bits, the same token.  A row with more than kFinishMost such tokens (ties) is
-// read once a digit by its workgroup (rows of 151,936 equal logits: 270 to 300 us a call, with the passes of many workgroups 86
-// for one and 256 for 64).
-// 64 rows of 151,936 logits, top_k 50 and top_p 0.9: seven kernels
-// 45 us (5.7 to 8.6 each), this one 15.5; what it is is four trips through memory and steps in LDS.
-constexpr int kFinishMost = 1024, kFinishThreads = 1024;
+// Rows with a small top_k: everything behind the first histogram in one kernel, a workgroup a row.  The tokens that the digits so
+// far leave are gathered into LDS (groups' largest e tell where they are); of more than kDirectMost the threshold's other digits
+// come from histograms of the list, and what does not reach it goes.  Each of the others is compared with all, which puts the list
+// into the order of the tokens, for the chunks' masses and the token, and into that of the values, for the threshold of top_p (and
+// gives that of top_k where it is not known yet).  The thresholds are the same values (exact, counts and fixed-point masses); a chunk's mass is added in the order of sample_mass_kernel's threads
+// and waves, a thread's in pick_token's, where what is not kept adds nothing: the same bits, the same token.
+// The first histogram says how many tokens its digit leaves.  Where the list does not hold them (flat rows: the digit is a fifth of
+// a value wide), the workgroup reads the row for the next digit, and once more for the last one; tokens above the threshold are
+// then fewer than top_k, and if their ties fill more than the list these are counted and not listed.
+// MI355X, rows of 151,936 normal logits, the kernels of a call in us, with the passes of many workgroups / with this kernel.  Spread 2
+// (over the temperature), top_k 50 and top_p 0.9: one row 38 / 28, 64 rows 72 / 41; top_k 256 39 / 38, 76 / 53.  Spread 0.2: top_k 50 38 /
+// 32, 73 / 49; top_k 256 40 / 55, 83 / 71.  Spread 0.05: top_k 50 39 / 39, 87 / 66; top_k 256 40 / 49, 91 / 74.  All logits equal:
+// 53 / 61, 235 / 81.  The host needs 60 us for a call's three launches and 80 for the nine of the passes, so that one row queued
+// behind others takes 82 / 63 us at all of these but the last, 81 / 84.  What a spread row takes is trips through memory and steps
+// in LDS; a flat one is bound by what a single workgroup reads, about 10 us a time.
+constexpr int kFinishThreads = 1024, kFinishTopK = 256;
+constexpr int kFinishMost = 4096, kDirectMost = 256, kKeptMost = 1024, kLiveMost = 4096;
+constexpr int kFinishVocab = 1 << 28;      // a group's first token / 4 and its size share a word
+static_assert(kFinishTopK <= kDirectMost, "a row that does not reach its rank has fewer tokens than that, and is not looked at by digits");
+static_assert(kFinishMost % kFinishThreads == 0 && kKeptMost == kFinishThreads, "whole rounds of the threads, and one of those kept");
 
 struct FinishLds {
   PickLds pick;
   int count, n_live;
-  unsigned int threshold, ok, digit, rest;
-  unsigned long long left, wave_sum[kFinishThreads / kWave];
+  unsigned int threshold, ok, digit, left, found;
   unsigned int wave_total[kFinishThreads / kWave];
+  unsigned long long wave_mass_total[kFinishThreads / kWave];
   float masses[256];
   int first[256], behind[256];            // of a chunk: its first token in the list, and the one behind its last
+  uint2 raw[kFinishMost];                 // bits and token, as gathered
   union {
+    unsigned int live[kLiveMost];         // groups that hold tokens for the list: 64 (first token / 4) + tokens - 1
+    unsigned int bins[kBins1];
     struct {
-      uint2 raw[kFinishMost];               // bits and token, as gathered
-      unsigned int bits[kFinishMost];       // in token order
-      int token[kFinishMost];
-      unsigned long long mass[kFinishMost];
-      int live[kFinishMost];                // groups that hold them
+      unsigned int bits[kKeptMost];       // in token order
+      int token[kKeptMost];
+      unsigned int value[kKeptMost];      // bits in descending order
     } list;
-    struct {
-      unsigned long long bins[kBins1];
-      float wave_mass[256][kSelWaves];
-    };
+    float wave_mass[256][kSelWaves];
   };
 };
 
-// One digit of a threshold of a row by one workgroup: the histogram of digit LEVEL of the tokens that reach `floor` and match the
-// digits so far (counts, or with MASS fixed-point masses) in LDS, and the bin in which, from the top, need(total) is reached.
-// Equal values of a wave are added as one.  False when the whole histogram does not reach it.
-template <int LEVEL, bool MASS, typename Need>
-__device__ __forceinline__ bool row_digit(const float* __restrict__ e, int vocab, unsigned int floor, unsigned int& prefix,
-                                          unsigned long long& rest, Need need_of, FinishLds& l) {
-  constexpr int kBins = LEVEL == 0 ? kBins0 : LEVEL == 1 ? kBins1 : kBins2;
-  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 0 ? 21 : LEVEL == 1 ? 10 : 0, kBits = LEVEL == 1 ? 11 : 10;
-  constexpr int kPer = kBins / kFinishThreads, kAhead = 8;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+// Appends the lanes' entries for which in[j] holds to a list of *count so far: put(place, j), one atomic a wave.
+template <int N, typename Put>
+__device__ __forceinline__ void append(const bool (&in)[N], int* count, Put put) {
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long some[N];
+  int all = 0;
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) l.bins[j * kFinishThreads + tid] = 0ull;
-  if (tid == 0) l.ok = 0u;
-  __syncthreads();
-  for (int base = 0; base < vocab; base += kAhead * kFinishThreads) {
-    float v[kAhead];
+  for (int j = 0; j < N; ++j) some[j] = __ballot(in[j]), all += __builtin_popcountll(some[j]);
+  if (all == 0) return;
+  int at = 0;
+  if (lane == 0) at = atomicAdd(count, all);
+  at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) v[j] = e[min(base + j * kFinishThreads + tid, vocab - 1)];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const unsigned int bits = __float_as_uint(v[j]);
-      const unsigned long long n = MASS ? static_cast<unsigned long long>(v[j] * kMassScale) : 1ull;
-      const bool in = base + j * kFinishThreads + tid < vocab && v[j] >= 0.f && bits >= floor && (LEVEL == 0 || (bits >> kHigh) == prefix) && n != 0ull;
-      const unsigned long long some = __ballot(in);
-      if (some == 0ull) continue;
-      const int lead = __builtin_ctzll(some);
-      const bool like = in && bits == static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(bits), lead));
-      const unsigned long long alike = __ballot(like);
-      if (like ? lane == lead : in)
-        atomicAdd(&l.bins[(bits >> kLow) & (kBins - 1)], like ? n * static_cast<unsigned long long>(__builtin_popcountll(alike)) : n);
-    }
+  for (int j = 0; j < N; ++j) {
+    if (in[j]) put(at + __builtin_popcountll(some[j] & ((1ull << lane) - 1ull)), j);
+    at += __builtin_popcountll(some[j]);
   }
-  __syncthreads();
-  unsigned long long m[kPer], own = 0ull;
+}
+
+// n / by and n % by by way of 1 / by (quotients below 2^20, so the estimate is one off at most; the whole division is some forty
+// instructions).
+__device__ __forceinline__ int quotient(int n, int by, float inverse, int& remainder) {
+  int q = static_cast<int>(static_cast<float>(n) * inverse), r = n - q * by;
+  if (r < 0) --q, r += by;
+  else if (r >= by) ++q, r -= by;
+  remainder = r;
+  return q;
+}
+
+// From the top, the bin of a histogram in which `rest` (>= 1) tokens are reached, a run of bins a thread: the digit goes behind the
+// prefix and `rest` becomes what is left inside the bin, `found` what is in it.  False when the whole histogram does not reach it.
+template <int PER>
+__device__ __forceinline__ bool reach_bin(const unsigned int (&m)[PER], int bits, unsigned int& prefix, unsigned int& rest,
+                                          unsigned int& found, FinishLds& l) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  unsigned int own = 0u;
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) own += m[j] = l.bins[kPer * tid + j];
-  unsigned long long suffix = own;
+  for (int j = 0; j < PER; ++j) own += m[j];
+  unsigned int suffix = own;   // over the wave's bins from these up
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) {
-    const unsigned long long other = shfl_any(suffix, min(lane + off, kWave - 1));
+    const unsigned int other = __shfl(suffix, min(lane + off, kWave - 1), kWave);
     if (lane + off < kWave) suffix += other;
   }
-  if (lane == 0) l.wave_sum[wave] = suffix;
+  if (lane == 0) l.wave_total[wave] = suffix;
+  if (tid == 0) l.ok = 0u;
   __syncthreads();
-  unsigned long long above = suffix - own, total = 0ull;
+  unsigned int above = suffix - own;
 #pragma unroll
-  for (int w = 0; w < kFinishThreads / kWave; ++w) {
-    total += l.wave_sum[w];
-    if (w > wave) above += l.wave_sum[w];
-  }
-  const unsigned long long need = need_of(total);
-  if (above < need && above + own >= need) {
+  for (int w = 0; w < kFinishThreads / kWave; ++w)
+    if (w > wave) above += l.wave_total[w];
+  if (above < rest && above + own >= rest) {
 #pragma unroll
-    for (int j = kPer - 1; j >= 0; --j) {
-      if (above < need && above + m[j] >= need) l.ok = 1u, l.digit = kPer * tid + j, l.left = need - above;
+    for (int j = PER - 1; j >= 0; --j) {
+      if (above < rest && above + m[j] >= rest) l.ok = 1u, l.digit = PER * tid + j, l.left = rest - above, l.found = m[j];
       above += m[j];
     }
   }
   __syncthreads();
   const bool ok = l.ok != 0u;
-  prefix = (LEVEL == 0 ? 0u : prefix << kBits) | l.digit;
-  rest = l.left;
-  __syncthreads();
+  if (ok) prefix = (prefix << bits) | l.digit, rest = l.left, found = l.found;
+  __syncthreads();   // l may be used again
   return ok;
 }
 
-// A row that the list does not hold, by the workgroup alone; `s`: what the first histogram gave.
-__device__ __forceinline__ void finish_by_passes(const SampleArgs& a, int row, const RowParams& r, const Slot& s, FinishLds& l) {
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  unsigned int thr = s.floor, prefix = s.prefix;
-  unsigned long long rest = s.rest;
-  auto left = [&](unsigned long long) { return rest; };
-  if (!s.open && row_digit<1, false>(e, a.vocab, s.floor, prefix, rest, left, l) && row_digit<2, false>(e, a.vocab, s.floor, prefix, rest, left, l))
-    thr = max(thr, prefix);
-  if (r.p_active) {
-    auto first = [&](unsigned long long total) { return top_p_need(r.top_p, total); };
-    const unsigned int floor = thr;
-    if (row_digit<0, true>(e, a.vocab, floor, prefix, rest, first, l) && row_digit<1, true>(e, a.vocab, floor, prefix, rest, left, l) &&
-        row_digit<2, true>(e, a.vocab, floor, prefix, rest, left, l))
-      thr = max(floor, prefix);
-  }
-  // 256 threads a chunk, as sample_mass_kernel's workgroups
-  const int t = threadIdx.x % kSelThreads, lane = threadIdx.x & (kWave - 1), wave = t / kWave;
-  for (int c = threadIdx.x / kSelThreads; c < a.chunks; c += kFinishThreads / kSelThreads) {
-    const int begin = c * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
-    float mass = 0.f;
-#pragma unroll 8
-    for (int i = begin + t; i < end; i += kSelThreads) {
-      const float v = e[i];
-      if (v >= 0.f && __float_as_uint(v) >= thr) mass += v;
+// Digit LEVEL (1 or 2) of top_k's threshold from the counts in l.bins.
+template <int LEVEL>
+__device__ __forceinline__ bool digit_of_bins(unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
+  constexpr int kPer = (LEVEL == 1 ? kBins1 : kBins2) / kFinishThreads;
+  __syncthreads();
+  unsigned int m[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) m[j] = l.bins[kPer * threadIdx.x + j];
+  return reach_bin<kPer>(m, LEVEL == 1 ? 11 : 10, prefix, rest, found, l);
+}
+template <int LEVEL>
+__device__ __forceinline__ void clear_bins(FinishLds& l) {
+#pragma unroll
+  for (int j = 0; j < (LEVEL == 1 ? kBins1 : kBins2) / kFinishThreads; ++j) l.bins[j * kFinishThreads + threadIdx.x] = 0u;
+  __syncthreads();
+}
+
+// The digit from the whole row.  Every lane has kAhead 16-byte pieces on their way at once, because one workgroup's share of the
+// memory's rate is what it has in flight; a wave whose values are all alike counts them as one.
+template <int LEVEL>
+__device__ __forceinline__ bool digit_of_row(const float* __restrict__ e, int vocab, unsigned int floor, unsigned int& prefix,
+                                             unsigned int& rest, unsigned int& found, FinishLds& l) {
+  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 1 ? 10 : 0, kMask = (LEVEL == 1 ? kBins1 : kBins2) - 1, kAhead = 8;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const unsigned int from = max(floor, prefix << kHigh), behind = (prefix + 1u) << kHigh;   // neither NaN nor -1: they are beyond any prefix
+  clear_bins<LEVEL>(l);
+  auto count = [&](float v) {
+    const unsigned int bits = __float_as_uint(v);
+    if (bits >= from && bits < behind) atomicAdd(&l.bins[(bits >> kLow) & kMask], 1u);
+  };
+  const int head = min(vocab, static_cast<int>((4u - (static_cast<unsigned int>(reinterpret_cast<uintptr_t>(e)) / 4u) % 4u) % 4u));
+  const int pieces = (vocab - head) / 4, tail = head + 4 * pieces;
+  if (tid < head) count(e[tid]);
+  if (tid < vocab - tail) count(e[tail + tid]);
+  const float4* at = reinterpret_cast<const float4*>(e + head);
+  for (int base = 0; base < pieces; base += kAhead * kFinishThreads) {
+    float4 v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = at[min(base + j * kFinishThreads + tid, pieces - 1)];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const bool in = base + j * kFinishThreads + tid < pieces;
+      const unsigned int lead = __builtin_amdgcn_readfirstlane(__float_as_int(v[j].x));
+      const bool alike = in && __float_as_uint(v[j].x) == lead && __float_as_uint(v[j].y) == lead && __float_as_uint(v[j].z) == lead && __float_as_uint(v[j].w) == lead;
+      if (__ballot(alike) == ~0ull) {
+        if (lane == 0 && lead >= from && lead < behind) atomicAdd(&l.bins[(lead >> kLow) & kMask], 4u * kWave);
+      } else if (in) {
+        count(v[j].x), count(v[j].y), count(v[j].z), count(v[j].w);
+      }
     }
-    mass = wave_sum(mass);
-    if (lane == 0) l.wave_mass[c][wave] = mass;
+  }
+  return digit_of_bins<LEVEL>(prefix, rest, found, l);
+}
+
+// The digit from the list.
+template <int LEVEL>
+__device__ __forceinline__ bool digit_of_list(int n, unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
+  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 1 ? 10 : 0, kMask = (LEVEL == 1 ? kBins1 : kBins2) - 1;
+  clear_bins<LEVEL>(l);
+  for (int i = threadIdx.x; i < n; i += kFinishThreads) {
+    const unsigned int bits = l.raw[i].x;
+    if ((bits >> kHigh) == prefix) atomicAdd(&l.bins[(bits >> kLow) & kMask], 1u);
+  }
+  return digit_of_bins<LEVEL>(prefix, rest, found, l);
+}
+
+// The row's tokens from `lower` on, into l.raw; how many there are (more than kFinishMost: some are not listed).  `most`: the
+// largest e of the first groups, fetched by the caller.
+constexpr int kGroupsAhead = 4;
+__device__ __forceinline__ int gather(const SampleArgs& a, int row, unsigned int lower, const float* gm, int groups,
+                                      const float (&most)[kGroupsAhead], FinishLds& l) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const float inverse = 1.0f / static_cast<float>(a.groups);
+  if (tid == 0) l.count = l.n_live = 0;
+  __syncthreads();
+  for (int base = 0; base < groups; base += kGroupsAhead * kFinishThreads) {
+    bool live[kGroupsAhead];
+    unsigned int entry[kGroupsAhead];
+#pragma unroll
+    for (int j = 0; j < kGroupsAhead; ++j) {
+      const int g = base + j * kFinishThreads + tid;
+      const float m = base == 0 ? most[j] : gm[min(g, groups - 1)];
+      int in_chunk;
+      const int chunk = quotient(g, a.groups, inverse, in_chunk), first = chunk * a.chunk_len + in_chunk * kGroup;
+      const int tokens = min(min(a.chunk_len - in_chunk * kGroup, a.vocab - first), kGroup);
+      // (a chunk's last groups may lie past its end, and nobody has written those)
+      live[j] = g < groups && tokens > 0 && __float_as_uint(m) >= lower;
+      entry[j] = static_cast<unsigned int>(first) / 4u * kGroup + static_cast<unsigned int>(tokens - 1);
+    }
+    append(live, &l.n_live, [&](int at, int j) { if (at < kLiveMost) l.live[at] = entry[j]; });
+  }
+  __syncthreads();
+  const int n_live = l.n_live;
+  if (n_live > kLiveMost) return kFinishMost + 1;
+  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  constexpr int kEach = 8;
+  for (int base = kEach * wave; base < n_live; base += kEach * kFinishThreads / kWave) {
+    float v[kEach];
+    int token[kEach];
+    bool in[kEach];
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const unsigned int entry = l.live[min(base + j, n_live - 1)];
+      in[j] = base + j < n_live && lane <= static_cast<int>(entry % kGroup);
+      token[j] = static_cast<int>(entry / kGroup * 4u) + min(lane, static_cast<int>(entry % kGroup));
+      v[j] = e[token[j]];
+    }
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) in[j] = in[j] && v[j] >= 0.f && __float_as_uint(v[j]) >= lower;
+    append(in, &l.count, [&](int at, int j) { if (at < kFinishMost) l.raw[at] = uint2{__float_as_uint(v[j]), static_cast<unsigned int>(token[j])}; });
+  }
+  __syncthreads();
+  return l.count;
+}
+
+// What of the list reaches `lower` stays; how many that are.
+__device__ __forceinline__ int keep_from(unsigned int lower, int n, FinishLds& l) {
+  constexpr int kEach = kFinishMost / kFinishThreads;
+  uint2 mine[kEach];
+  bool in[kEach];
+#pragma unroll
+  for (int j = 0; j < kEach; ++j) {
+    const int i = j * kFinishThreads + static_cast<int>(threadIdx.x);
+    mine[j] = l.raw[min(i, n - 1)];
+    in[j] = i < n && mine[j].x >= lower;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) l.count = 0;
+  __syncthreads();
+  append(in, &l.count, [&](int at, int j) { l.raw[at] = mine[j]; });
+  __syncthreads();
+  return l.count;
+}
+
+// The kept mass of every chunk from the row, in the order of sample_mass_kernel: 256 threads a chunk, kAhead chunks of theirs at once.
+__device__ __forceinline__ void masses_of_row(const SampleArgs& a, int row, unsigned int thr, FinishLds& l) {
+  constexpr int kAhead = 4, kUnroll = 9, kGroups = kFinishThreads / kSelThreads;
+  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  const int t = threadIdx.x % kSelThreads, lane = threadIdx.x & (kWave - 1), wave = t / kWave;
+  for (int c0 = threadIdx.x / kSelThreads; c0 < a.chunks; c0 += kAhead * kGroups) {
+    float mass[kAhead] = {};
+    for (int i = t; i < a.chunk_len; i += kUnroll * kSelThreads) {
+      float v[kAhead][kUnroll];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+#pragma unroll
+        for (int k = 0; k < kUnroll; ++k) v[j][k] = e[min(min(c0 + j * kGroups, a.chunks - 1) * a.chunk_len + i + k * kSelThreads, a.vocab - 1)];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+#pragma unroll
+        for (int k = 0; k < kUnroll; ++k) {
+          const bool in = i + k * kSelThreads < min(a.chunk_len, a.vocab - (c0 + j * kGroups) * a.chunk_len);
+          if (in && v[j][k] >= 0.f && __float_as_uint(v[j][k]) >= thr) mass[j] += v[j][k];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const float sum = wave_sum(mass[j]);
+      if (lane == 0 && c0 + j * kGroups < a.chunks) l.wave_mass[c0 + j * kGroups][wave] = sum;
+    }
   }
   __syncthreads();
   if (static_cast<int>(threadIdx.x) < a.chunks) {
@@ -869,149 +1008,127 @@ __device__ __forceinline__ void finish_by_passes(const SampleArgs& a, int row, c
     l.masses[threadIdx.x] = total;
   }
   __syncthreads();
-  pick_token(a, row, thr, l.masses, l.pick);
 }
 
 __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const SampleArgs a) {
   __shared__ FinishLds l;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   // what is wanted of the row and does not hang on anything else: all on its way at once
-  constexpr int kAhead = 4;
   const float* gm = a.group_max + static_cast<int64_t>(row) * a.chunks * a.groups;
   const int groups = a.chunks * a.groups;
-  float most[kAhead];
+  float most[kGroupsAhead];
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) most[j] = gm[min(j * kFinishThreads + tid, groups - 1)];
-  const unsigned int own = a.hist_k[static_cast<int64_t>(row) * kRowBins + tid];
+  for (int j = 0; j < kGroupsAhead; ++j) most[j] = gm[min(j * kFinishThreads + tid, groups - 1)];
+  const unsigned int own[1] = {a.hist_k[static_cast<int64_t>(row) * kRowBins + tid]};
   const float u = a.u[row];
   const RowParams r = row_params(a, row);
   if (r.greedy) {
     pick_greedy(a, row, l.pick);
     return;
   }
-  const unsigned int mp = min_p_bits(r);
-  if (tid == 0) l.count = l.n_live = 0, l.ok = 0u, l.threshold = mp;
+  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  const unsigned int mp = min_p_bits(r), k = static_cast<unsigned int>(r.k);
+  if (tid == 0) l.threshold = mp;
   for (int c = tid; c < 256; c += kFinishThreads) l.first[c] = l.behind[c] = 0, l.masses[c] = 0.f;
-  // the first digit, a bin a thread
-  static_assert(kFinishThreads == kBins0, "a bin a thread");
-  unsigned int suffix = own;   // over the wave's bins from this one up
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const unsigned int other = __shfl(suffix, min(lane + off, kWave - 1), kWave);
-    if (lane + off < kWave) suffix += other;
-  }
-  if (lane == 0) l.wave_total[wave] = suffix;
-  __syncthreads();
-  unsigned int above_bin = suffix - own;
-#pragma unroll
-  for (int w = 0; w < kFinishThreads / kWave; ++w)
-    if (w > wave) above_bin += l.wave_total[w];
-  const unsigned int k = static_cast<unsigned int>(r.k);
-  if (above_bin < k && above_bin + own >= k) l.ok = 1u, l.digit = tid, l.rest = k - above_bin;
-  __syncthreads();
-  const bool open = l.ok == 0u;      // the row does not reach the rank: everything above min_p's floor stays
-  const Slot s{open ? 0ull : static_cast<unsigned long long>(l.rest), open ? 0u : l.digit, mp, open ? 1u : 0u, 0u};
-  // tokens that may be kept, in the groups whose largest e may be.  An e of zero weighs nothing and is never drawn: where the
-  // rank is only reached among those (most logits -inf, say), the others all stay, which is what the list then gives.
-  const unsigned int lower = max(open ? mp : max(mp, s.prefix << 21), 1u);
-  for (int base = 0; base < groups; base += kAhead * kFinishThreads) {
-    if (base > 0) {
-#pragma unroll
-      for (int j = 0; j < kAhead; ++j) most[j] = gm[min(base + j * kFinishThreads + tid, groups - 1)];
+  static_assert(kFinishThreads == kBins0, "a bin of the first digit a thread");
+  unsigned int prefix = 0u, rest = k, found = 0u;
+  const bool open = !reach_bin<1>(own, 10, prefix, rest, found, l);      // the row does not reach the rank: everything above min_p's floor stays
+  // Tokens that may be kept.  An e of zero weighs nothing and is never drawn: where the rank is only reached among those (most logits
+  // -inf, say), the others all stay, which is what the list then gives.  (The lowest digit counts zeros too and says nothing of the list.)
+  unsigned int lower = max(open ? mp : max(mp, prefix << 21), 1u);
+  int digits = 1, n = kFinishMost + 1;      // digits of top_k's threshold that are known, tokens from `lower` on
+  unsigned int ties = 0u;                   // tokens at the threshold that are not listed
+  auto listed = [&] { return (k - rest) + found <= static_cast<unsigned int>(kFinishMost); };
+  if (open || prefix == 0u || listed()) n = gather(a, row, lower, gm, groups, most, l);
+  if (n > kFinishMost) {      // and then the rank is reached (fewer than top_k tokens otherwise)
+    bool ok = digit_of_row<1>(e, a.vocab, mp, prefix, rest, found, l);
+    digits = 2;
+    if (ok && !listed()) ok = digit_of_row<2>(e, a.vocab, mp, prefix, rest, found, l), digits = 3;
+    lower = max(max(mp, digits == 2 ? prefix << 10 : prefix), 1u);
+    if (digits == 3 && !listed()) {
+      if (prefix > 0u) ties = found;
+      lower = prefix + 1u;
     }
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const int g = base + j * kFinishThreads + tid;
-      const int chunk = g / a.groups, in_chunk = g - chunk * a.groups;
-      // (a chunk's last groups may lie past its end, and nobody has written those)
-      if (g < groups && in_chunk * kGroup < min(a.chunk_len, a.vocab - chunk * a.chunk_len) && __float_as_uint(most[j]) >= lower) {
-        const int at = atomicAdd(&l.n_live, 1);
-        if (at < kFinishMost) l.list.live[at] = g;
-      }
-    }
+    n = gather(a, row, lower, gm, groups, most, l);
   }
-  __syncthreads();
-  const int n_live = l.n_live;
-  if (n_live <= kFinishMost) {
-    const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-    constexpr int kEach = 8;
-    for (int base = kEach * wave; base < n_live; base += kEach * kFinishThreads / kWave) {
-      float v[kEach];
-      int token[kEach];
-#pragma unroll
-      for (int j = 0; j < kEach; ++j) {
-        const int g = l.list.live[min(base + j, n_live - 1)], chunk = g / a.groups;
-        const int in_chunk = (g - chunk * a.groups) * kGroup + lane;
-        token[j] = base + j < n_live && in_chunk < a.chunk_len ? chunk * a.chunk_len + in_chunk : a.vocab;
-        v[j] = e[min(token[j], a.vocab - 1)];
-      }
-#pragma unroll
-      for (int j = 0; j < kEach; ++j) {
-        if (token[j] < a.vocab && v[j] >= 0.f && __float_as_uint(v[j]) >= lower) {
-          const int at = atomicAdd(&l.count, 1);
-          if (at < kFinishMost) l.list.raw[at] = uint2{__float_as_uint(v[j]), static_cast<unsigned int>(token[j])};
-        }
-      }
-    }
+  unsigned int thr = digits == 3 ? max(mp, prefix) : mp;
+  bool known = open || digits == 3;
+  if (n > kDirectMost && !known) {
+    bool ok = digits == 2 || digit_of_list<1>(n, prefix, rest, found, l);
+    ok = ok && digit_of_list<2>(n, prefix, rest, found, l);
+    if (ok) thr = max(mp, prefix);
+    known = true;
+    const int all = n;
+    n = keep_from(max(thr, 1u), all, l);
   }
-  __syncthreads();
-  const int n = l.count;
-  if (n_live > kFinishMost || n > kFinishMost) {
-    finish_by_passes(a, row, r, s, l);
-    return;
+  if (n > kKeptMost) {      // ties
+    ties = found;
+    n = keep_from(thr + 1u, n, l);
   }
   // four threads a token compare it with all
   const int quarter = tid & 3;
   for (int i = tid / 4; i < n; i += kFinishThreads / 4) {
-    const uint2 own_pair = l.list.raw[i];
+    const uint2 own_pair = l.raw[i];
     const unsigned int bits = own_pair.x, token = own_pair.y;
-    unsigned int rank = 0, above = 0, reach = 0;
+    unsigned int rank = 0, above = 0, reach = 0, before = 0;      // before: of the same value, further ahead in the tokens' order
 #pragma unroll 4
     for (int j = quarter; j < n; j += 4) {
-      const uint2 other = l.list.raw[j];
-      rank += other.y < token;
+      const uint2 other = l.raw[j];
+      const bool ahead = other.y < token;
+      rank += ahead;
       above += other.x > bits;
       reach += other.x >= bits;
+      before += ahead && other.x == bits;
     }
-    rank += __shfl_xor(rank, 1, kWave), above += __shfl_xor(above, 1, kWave), reach += __shfl_xor(reach, 1, kWave);
-    rank += __shfl_xor(rank, 2, kWave), above += __shfl_xor(above, 2, kWave), reach += __shfl_xor(reach, 2, kWave);
+    auto four = [](unsigned int& v) { v += __shfl_xor(v, 1, kWave), v += __shfl_xor(v, 2, kWave); };
+    four(rank), four(above), four(reach), four(before);
     if (quarter == 0) {
       l.list.bits[rank] = bits;
       l.list.token[rank] = static_cast<int>(token);
-      l.list.mass[rank] = static_cast<unsigned long long>(__uint_as_float(bits) * kMassScale);
-      if (!open && above < k && k <= reach) l.threshold = max(mp, bits);   // the k-th largest, and its ties
+      l.list.value[above + before] = bits;
+      if (!known && above < k && k <= reach) l.threshold = max(mp, bits);   // the k-th largest, and its ties
     }
   }
+  if (tid == 0) l.ok = 0u;
   __syncthreads();
-  unsigned int thr = l.threshold;
+  if (!known) thr = l.threshold;
   if (r.p_active) {
-    for (int i = tid / 4; i < n; i += kFinishThreads / 4) {
-      const unsigned int bits = l.list.bits[i];
-      unsigned long long above = 0ull, reach = 0ull, total = 0ull;
-#pragma unroll 4
-      for (int j = quarter; j < n; j += 4) {
-        const unsigned int other = l.list.bits[j];
-        const unsigned long long m = other >= thr ? l.list.mass[j] : 0ull;
-        total += m;
-        reach += other >= bits ? m : 0ull;
-        above += other > bits ? m : 0ull;
-      }
+    // from the largest value down, one a thread, until the mass is reached
+    const unsigned int bits = tid < n ? l.list.value[tid] : 0u;
+    auto mass_of = [](unsigned int b) { return static_cast<unsigned long long>(__uint_as_float(b) * kMassScale); };
+    const unsigned long long mass = tid < n && bits >= thr ? mass_of(bits) : 0ull;
+    unsigned long long upto = mass;
 #pragma unroll
-      for (int off = 1; off < 4; off <<= 1) {
-        total += shfl_any(total, lane ^ off);
-        reach += shfl_any(reach, lane ^ off);
-        above += shfl_any(above, lane ^ off);
-      }
-      const unsigned long long need = top_p_need(r.top_p, total);
-      if (quarter == 0 && bits >= thr && above < need && need <= reach) l.digit = bits, l.ok = 2u;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const unsigned long long other = shfl_any(upto, max(lane - off, 0));
+      if (lane >= off) upto += other;
     }
+    if (lane == kWave - 1) l.wave_mass_total[wave] = upto;
     __syncthreads();
-    if (l.ok == 2u) thr = l.digit;
+    unsigned long long total = static_cast<unsigned long long>(ties) * mass_of(thr);
+#pragma unroll
+    for (int w = 0; w < kFinishThreads / kWave; ++w) {
+      const unsigned long long of_wave = l.wave_mass_total[w];
+      total += of_wave;
+      if (w < wave) upto += of_wave;
+    }
+    const unsigned long long need = top_p_need(r.top_p, total);
+    if (mass > 0ull && upto - mass < need && need <= upto) l.digit = bits, l.ok = 2u;
+    __syncthreads();
+    if (l.ok == 2u) thr = l.digit, ties = 0u;      // among those, above the ties
   }
-  for (int i = tid; i < n; i += kFinishThreads) {
-    const int chunk = l.list.token[i] / a.chunk_len;
-    if (i == 0 || l.list.token[i - 1] / a.chunk_len != chunk) l.first[chunk] = i;
-    if (i == n - 1 || l.list.token[i + 1] / a.chunk_len != chunk) l.behind[chunk] = i + 1;
+  if (ties > 0u) {
+    __syncthreads();   // the list is done with
+    masses_of_row(a, row, thr, l);
+    pick_token(a, row, thr, l.masses, l.pick);
+    return;
+  }
+  const float per_chunk = 1.0f / static_cast<float>(a.chunk_len);
+  auto chunk_of = [&](int i) { int in_chunk; return quotient(l.list.token[i], a.chunk_len, per_chunk, in_chunk); };
+  if (tid < n) {
+    const int chunk = chunk_of(tid);
+    if (tid == 0 || chunk_of(tid - 1) != chunk) l.first[chunk] = tid;
+    if (tid == n - 1 || chunk_of(tid + 1) != chunk) l.behind[chunk] = tid + 1;
   }
   __syncthreads();
   for (int c = wave; c < a.chunks; c += kFinishThreads / kWave) {
@@ -1143,9 +1260,8 @@ extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
                                 rows * sizeof(unsigned int));
 }
 
-// Rows from whose top_k on the passes of many workgroups are the faster way to the threshold: the tokens that a first digit
-// leaves are at least as many, and the finishing kernel compares each with each.
-extern "C" int arle_sample_finish_most() { return kFinishMost / 4; }
+// The largest top_k that the finishing kernel is for.
+extern "C" int arle_sample_finish_most() { return kFinishTopK; }
 
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
 // arle_sample_scratch_bytes(rows, vocab) bytes, 16-byte aligned.  use_top_k / use_top_p == 0 promise that no row of the call has
@@ -1190,7 +1306,7 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.use_top_p = use_top_p;
   a.out = out;
   const dim3 grid(a.chunks, rows);
-  const bool finish = small_k && use_top_k;
+  const bool finish = small_k && use_top_k && vocab <= kFinishVocab;
   // the histograms start at zero: those of the filters that are on, of the finishing kernel's rows the first one
   const int k_row = kRowBins * sizeof(unsigned int) / 16, p_row = kRowBins * sizeof(unsigned long long) / 16;
   const ClearRows clear{reinterpret_cast<uint4*>(a.hist_k), reinterpret_cast<uint4*>(a.hist_p),

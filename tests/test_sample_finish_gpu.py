@@ -45,6 +45,37 @@ def test_the_same_tokens(rows, vocab, monkeypatch):
                         assert torch.equal(got, want), (ks, ps, ms, temps)
 
 
+@pytest.mark.parametrize("rows,vocab", [(14, 151936), (14, 33003), (14, 5001), (14, 300001)])
+@pytest.mark.parametrize("k", [1, 50, 256])
+def test_flat_rows(rows, vocab, k):
+    """Rows whose first digit leaves more than the list holds, about as many or somewhat fewer, and ties of any number at the
+    threshold, below it and above it; odd lengths, so that rows begin anywhere on the 16-byte grid."""
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(vocab + k)
+    x = torch.randn(rows, vocab, generator=gen)
+    for i, spread in enumerate((0.005, 0.02, 0.05, 0.1, 0.2, 0.3, 0.5)):
+        x[i] *= spread
+    x[7] = torch.where(x[7] > 0.5, 1.0, 0.0)                                  # two values
+    x[8] = torch.where(torch.arange(vocab) % 13 < k % 13, 0.1, 0.0)
+    x[8, 5:5 + 100] = 0.11 + 0.001 * torch.arange(100)                          # some above the ties
+    x[9] = 0.0
+    x[9, vocab // 2:vocab // 2 + 300] = 1.0                                    # fewer than the list holds, more than top_k
+    x[10] = (x[10] * 0.1 * 40).round() / 40
+    x[11] = x[11] * 2 - 95                                                     # denormal e behind one large logit
+    x[11, 17] = 0.0
+    x[12] = torch.where(torch.arange(vocab) % 5 == 0, x[12] * 0.01, -float("inf"))
+    x[13, :2500] = 3.0                                                         # ties that the list holds and the kept ones do not
+    logits = x.cuda()
+    full = lambda v, dtype=torch.float32: torch.full((rows,), v, dtype=dtype, device="cuda")
+    for p in (1.0, 0.9, 0.02):
+        for min_p in (0.0, 0.3, 1.0):
+            for u in (torch.rand(rows, generator=gen).cuda(), full(0.0), full(0.99999994)):
+                args = (logits, full(1.0), full(k, torch.int32), full(p), full(min_p), u)
+                want = ops.sample_rows(*args, use_top_p=p < 1)
+                assert torch.equal(ops.sample_rows(*args, use_top_p=p < 1, small_k=True), want), (p, min_p)
+
+
 def test_the_sampler_promises_it_only_where_it_holds(monkeypatch):
     from arle_amd.kernels import ops
     from arle_amd.sampling import Sampler, SamplingParams

@@ -266,11 +266,28 @@ __global__ __launch_bounds__(KD* kWave) void mlstm_chunk_sums_kernel(const Mlstm
 // ahead and whose places take S_0 (the last blockIdx.z: n, an element a thread).  Bound by reading U and writing S_0, 84 MB
 // a layer at 2,048 rows of 20 heads.
 constexpr int kScanThreads = 256, kScanAhead = 8;
-// Rows of the longest request from which on sums and scan take the walk's place.  MI355X, all kernels of a layer, us, walk /
-// sums and scan: 20 heads of 128 one request of 256 rows 41.8 / 43.3, 320 44.9 / 44.9, 512 54.7 / 48.6, 1,024 84.7 / 67.8, 2,048
-// 149.8 / 108.1, 8,192 546 / 392, eight of 512 182 / 184; 8 heads of 64 256 rows 30.1 / 26.7, 2,048 108 / 43; 4 heads of
-// 128 256 rows 38.0 / 37.9, 2,048 115 / 52, eight of 256 43.8 / 48.6.
-constexpr int kSumsMinRows = 384;
+// Sums and scan take the walk's place for requests of kSumsMinRows and more, unless the walk keeps the matrix cores busy: a wave of
+// it is a chain of products, so it is its waves for every SIMD of the chip (1,024) that decide, and requests of unequal length leave
+// it with a tail.  MI355X, all kernels of a layer, us, walk / sums and scan, by the walk's waves:
+//   320 (20 heads of 128, one request) 256 rows 37.8 / 39.5, 384 43.3 / 42.7, 512 49.5 / 44.6, 1,024 81 / 64, 2,048 134 / 92; 128 (8 heads
+//     of 128) 384 rows 40.0 / 36.3, 2,048 120 / 65; 512 (4 heads of 128, eight requests) 384 rows 45.3 / 44.7, 1,024 92 / 80, 2,048
+//     150 / 123; 512 (8 heads of 64, 16) 384 rows 53.1 / 55.1, 512 70.6 / 69.8, 1,024 117 / 111
+//   640 (20 heads, two) 384 rows 54.3 / 59.4, 512 60.0 / 62.4, 640 67.3 / 66.2, 2,048 168 / 154
+//   1,024 (8 heads of 128, eight) 384 rows 56.6 / 65.7, 1,024 113 / 123, 2,048 223 / 254; (8 heads of 64, 32) 384 rows 78.9 / 89.9
+//   1,280 (20 heads, four), the walk's second turn mostly empty: 384 rows 83.2 / 78.7, 512 94.3 / 89.2, 2,048 323 / 307; 1,536 (8 heads,
+//     12) 600 rows 126 / 121
+//   2,048 and more: (8 heads, 16) 384 rows 91.8 / 101.8, 1,024 221 / 250; (20 heads, 16) 1,024 rows 535 / 589
+//   unequal requests, 20 heads: 4,631 rows in 16 up to 681 248 / 206, 3,584 in 8 up to 798 185 / 154, 2,471 in 4 up to 883 139 / 118,
+//     7,505 in 16 up to 584 316 / 315, 3,765 in 3 up to 1,380 137 / 145; 8 heads: 4,100 in 8 up to 700 81 / 88, 4,631 in 16 112 / 95
+constexpr int kSumsMinRows = 384, kSumsMinRowsFuller = 640, kWalkWaves = 1024;
+
+static bool sums_preferred(long long tokens, long long segments, long long longest, int H, int D, int Dv) {
+  if (longest < kSumsMinRows) return false;
+  if (4 * tokens <= 3 * segments * longest) return true;      // far from equal
+  const long long waves = segments * H * (Dv / 32) * (D / 32), turns = (waves + kWalkWaves - 1) / kWalkWaves;
+  if (turns > 1) return 4 * waves <= 3 * turns * kWalkWaves;
+  return waves <= kWalkWaves / 2 || (waves <= kWalkWaves * 5 / 8 && longest >= kSumsMinRowsFuller);
+}
 
 __global__ __launch_bounds__(kScanThreads) void mlstm_chunk_scan_kernel(const MlstmChunkArgs a, int D) {
   const int seg = blockIdx.x, h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
@@ -574,9 +591,9 @@ __global__ __launch_bounds__(kOutWaves* kWave, 3) void mlstm_chunk_out_kernel(co
 }
 
 template <int KD>
-int launch_chunks(const MlstmChunkArgs& a, int longest, hipStream_t s) {
+int launch_chunks(const MlstmChunkArgs& a, bool sums, hipStream_t s) {
   mlstm_chunk_gates_kernel<<<dim3(a.items, a.H), kWave, 0, s>>>(a);
-  if (longest >= kSumsMinRows) {
+  if (sums) {
     constexpr int D = 32 * KD;
     mlstm_chunk_sums_kernel<KD><<<dim3(a.items, a.H), KD * kWave, 0, s>>>(a);
     mlstm_chunk_scan_kernel<<<dim3(a.segments, a.H, (D * a.Dv / 4 + kScanThreads - 1) / kScanThreads + 1), kScanThreads, 0, s>>>(a, D);
@@ -605,7 +622,7 @@ extern "C" long long arle_mlstm_chunks_bytes(int items, int H, int D, int Dv) {
 extern "C" int arle_mlstm_chunks(const float* q, const float* k, const float* v, const float* gate, long long row_stride,
                                  const float* gates, long long gates_stride, const float* bias_i, const float* bias_f, float cap,
                                  float* s_state, float* n_state, float* m_state, const int* seg_row0, const int* seg_slot,
-                                 int segments, int items, int longest, int H, int D, int Dv, void* workspace, const void* weight, int w_dtype,
+                                 int segments, int items, int tokens, int longest, int H, int D, int Dv, void* workspace, const void* weight, int w_dtype,
                                  void* out, int out_dtype, float eps, void* stream) {
   if (segments == 0 || items == 0) return 0;
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
@@ -623,11 +640,11 @@ extern "C" int arle_mlstm_chunks(const float* q, const float* k, const float* v,
   a.rows = reinterpret_cast<ChunkRow*>(at), at += pairs * kChunkRows * sizeof(ChunkRow);
   a.m0 = reinterpret_cast<float*>(at);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!aligned(s_state)) longest = 0;      // the states' kernel reads four elements at a time
+  const bool sums = aligned(s_state) && sums_preferred(tokens, segments, longest, H, D, Dv);      // the states' kernel reads four elements at a time
   switch (D / 32) {
-    case 1: return launch_chunks<1>(a, longest, s);
-    case 2: return launch_chunks<2>(a, longest, s);
-    case 3: return launch_chunks<3>(a, longest, s);
-    default: return launch_chunks<4>(a, longest, s);
+    case 1: return launch_chunks<1>(a, sums, s);
+    case 2: return launch_chunks<2>(a, sums, s);
+    case 3: return launch_chunks<3>(a, sums, s);
+    default: return launch_chunks<4>(a, sums, s);
   }
 }

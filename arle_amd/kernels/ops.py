@@ -1919,8 +1919,8 @@ def mlstm_chunks(qkvg, gates, bias_i, bias_f, cap: float, s_state, n_state, m_st
     at = lambda column: qkvg.data_ptr() + 4 * column
     lib.call("arle_mlstm_chunks", at(0), at(H * D), at(2 * H * D), at(2 * H * D + width), qkvg.stride(0), gates.data_ptr(),
              gates.stride(0), bias_i.data_ptr(), bias_f.data_ptr(), float(cap), s_state.data_ptr(), n_state.data_ptr(),
-             m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), segments, items, tokens if longest is None else int(longest), H, D, Dv,
-             scratch.data_ptr(), weight.data_ptr(), _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
+             m_state.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), segments, items, tokens, tokens if longest is None else int(longest),
+             H, D, Dv, scratch.data_ptr(), weight.data_ptr(), _code(weight), out.data_ptr(), _code(out), float(eps), _stream())
     return out
 
 

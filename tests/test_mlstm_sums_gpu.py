@@ -26,3 +26,20 @@ def test_sums_and_scan_give_what_the_walk_gives(lengths, H, D, Dv, gate_std):
     assert _rel(summed, walked.double()) < 1e-5
     for a, b, before in zip(s1, s0, c["state"]):
         assert _rel(a, b.double()) < 2e-6 and torch.equal(a[0], before[0])
+
+
+@pytest.mark.parametrize("lengths,H,D,sums", [([384], 2, 128, True), ([384] * 8, 8, 128, False), ([640] * 2, 20, 128, True), ([639] * 2, 20, 128, False),
+                                              ([700, 1, 1, 1, 1, 1, 1, 1, 1, 1], 8, 128, True), ([383], 1, 32, False)])
+def test_which_of_them_a_step_takes(lengths, H, D, sums):
+    """A walk that keeps the matrix cores busy stays (8 requests of 384 rows, 8 heads of 128: 56.6 against 65.7 us)."""
+    from arle_amd.kernels import ops
+
+    c = _case(lengths, H, D, D, 1.0, 5)
+
+    def run(longest):
+        state = [t.clone() for t in c["state"]]
+        return ops.mlstm_chunks(c["qkvg"], c["gates"], c["bi"], c["bf"], 15.0, *state, c["row0"], c["slot"], c["weight"], 1e-6, torch.float32,
+                                heads=H, key_dim=D, value_dim=D, longest=longest), state
+
+    (got, state), (like, want) = run(max(lengths)), run(1 << 20 if sums else 1)
+    assert torch.equal(got, like) and all(torch.equal(a, b) for a, b in zip(state, want))

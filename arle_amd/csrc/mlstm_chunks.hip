@@ -316,8 +316,8 @@ __global__ __launch_bounds__(kScanThreads) void mlstm_chunk_scan_kernel(const Ml
         if (c < chunks) {
           const T u = ahead[j];
           const ChunkEnd end = ends[j];
-          const int next = min(c + kScanAhead, chunks - 1);      // past the end: the last one again, whose place nobody has written yet
-          if (c + kScanAhead < chunks) {
+          // (nothing past the last chunk: the places in front of this one hold S_0 by now, not sums)
+          if (const int next = c + kScanAhead; next < chunks) {
             ahead[j] = sums[next * a_chunk];
             ends[j] = a.ends[first + static_cast<int64_t>(next) * H];
           }

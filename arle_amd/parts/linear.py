@@ -28,7 +28,7 @@ from ..kernels import ops
 
 class Linear:
     def __init__(self, weight: torch.Tensor, tiles: bool = False, packed: torch.Tensor | None = None):
-        """packed: operand tiles that exist already (of a matrix this weight is the first rows of)."""
+        """packed: operand tiles that exist already (of a matrix that this weight is rows of, from the first row of a tile on)."""
         if weight.dim() != 2 or not weight.is_contiguous():
             raise ValueError("a projection weight must be a contiguous [out, in] matrix")
         self.weight = weight

@@ -89,7 +89,9 @@ class MLSTMMixer(Part):
     def products(self):
         if self.qkvg.weight.dtype != torch.bfloat16:
             return []
-        return [("qkvg", self.qkvg.out_features, self.qkvg.in_features, False, None),
+        # steps of single rows run q|k|v|gate and the gates as one product, whose stack their kernel adds
+        whole = [] if self.whole is None else [("qkvgif", self.whole.out_features, self.whole.in_features, False, "norm")]
+        return [("qkvg", self.qkvg.out_features, self.qkvg.in_features, False, None), *whole,
                 ("o", self.o.out_features, self.o.in_features, False, "norm")]
 
     def forward(self, x, batch, cache):

@@ -50,8 +50,10 @@ def _words(values) -> array:
 def uniforms(seeds, indices) -> np.ndarray:
     """uniform(seed, index) of every pair, float32, by the host runtime (64 pairs took 46 us in arithmetic on whole arrays,
     and 6 of these are left)."""
-    out = np.empty(len(seeds), dtype=np.float32)
     s, i = _words(seeds), _words(indices)
+    if len(s) != len(i):
+        raise ValueError(f"{len(s)} seeds and {len(i)} indices do not make pairs")
+    out = np.empty(len(s), dtype=np.float32)
     native.lib().arle_uniforms(len(out), s.buffer_info()[0], i.buffer_info()[0], out.ctypes.data)
     return out
 

@@ -307,3 +307,11 @@ def test_uniform_numbers_of_many_rows_are_those_of_single_rows(rows):
     indices = [i * i if i % 3 else 2 ** 40 + i for i in range(rows)]
     got = uniforms(seeds, indices)
     assert got.dtype.name == "float32" and got.tolist() == [uniform(s, i) for s, i in zip(seeds, indices)]
+
+
+@pytest.mark.parametrize("seeds,indices", [([1, 2], [3]), ([1], [2, 3]), (list(range(20)), list(range(19))), ([-1, 2], [])])
+def test_seeds_and_indices_that_are_no_pairs_are_refused(seeds, indices):
+    from arle_amd.sampling.sampler import uniforms
+
+    with pytest.raises(ValueError, match="pairs"):
+        uniforms(seeds, indices)

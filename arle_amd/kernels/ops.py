@@ -1351,6 +1351,10 @@ PRODUCT_KERNELS = ("rows", "stream", "rounds", "tiles", "tiles_parts", "wide", "
 #     K 3,072 128 rows 35.6 / 37.1, 256 48.1 / 41.1, 640 72.3 / 79.1, 1,024 100.9 / 88.6.
 #   K 8,192, N 57,344: 128 rows 228 / 259, 512 440 / 443, 1,536 1,101 / 1,216.
 # Of 261 such products taken from 65 to 8,192 rows six were slower by 3 % and more (10 % at most), all of them 17 % faster.
+# The figures and the lines are of the kernel with two stages and W in rows.  With the deeper stages and operand tiles that it has now
+# it is ahead on the other side of these lines too (N 6,144, K 1,024 32 rows 9.2 / 6.7; N 12,288, K 2,048 64 rows 18.2 / 14.6; N 28,672,
+# K 5,120 64 rows 67.7 / 55.7, 128 74.4 / 62.9, 384 116.7 / 107.6; K 8,192, N 57,344 128 rows 220 / 182, but 512 403 / 425): they
+# have not been moved.
 _WIDE_BY_K = ((1024, 65), (2560, 129), (6144, 512))     # (K up to, rows from)
 _WIDE_TWO_BLOCKS = (193, 256)                           # and these rows, two row blocks of 128 that are all but full
 _WIDE_ANY_ROWS_K = 3072

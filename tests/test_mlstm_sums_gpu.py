@@ -1,6 +1,6 @@
 """The mLSTM's chunks with their sums side by side and the states in front of them element by element (requests of 384 rows
 and more) against the walk from chunk to chunk: more chunks than are fetched ahead, remainders, several requests of unequal
-length, gates far apart.  Both are 32-bit sums of the same terms: within 1e-5 of each other, states within 2e-6."""
+length, gates far apart; and which of the two a step takes.  Both are 32-bit sums of the same terms: within 1e-5 of each other, states within 2e-6."""
 import pytest
 import torch
 

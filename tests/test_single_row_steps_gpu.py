@@ -1,7 +1,8 @@
 """Kernels of steps in which every request brings one row: the convolution with its state (`ops.conv_step`) and PolyNorm of a
 stack against the kernels that they stand for, bit for bit (the same sums in the same order, stacks rounded as the kernel that
 adds them does), and alike for the layer norm with the convolution behind it; the mLSTM in one kernel (`ops.mlstm_decode`) against the 64-bit recurrence (bounds as in
-test_mlstm_chunks_gpu); the layer norm at the edges of its workgroups' widths (two 32-bit passes: 1e-5)."""
+test_mlstm_chunks_gpu); the layer norm at the edges of its workgroups' widths (two 32-bit passes: 1e-5), and it and PolyNorm in
+steps of many rows, where a float32 row keeps its bits."""
 import pytest
 import torch
 

@@ -1,5 +1,5 @@
 """Rows with a small top_k finished by one kernel (`sample_rows(..., small_k=True)`) against the passes of many workgroups: the
-same tokens, for every draw.  Ties that fill more than the kernel's list (which then does the passes by itself), rows whose
+same tokens, for every draw.  Ties that fill more than the kernel's list (which then reads the row again), rows whose
 kept tokens lie at the ends of groups and chunks, rows that do not reach the rank, greedy rows, NaN and infinities, new
 buffers full of ones."""
 import pytest

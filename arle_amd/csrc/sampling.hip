@@ -745,7 +745,7 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
 // (over the temperature), top_k 50 and top_p 0.9: one row 38 / 28, 64 rows 72 / 41; top_k 256 39 / 38, 76 / 53.  Spread 0.2: top_k 50 38 /
 // 32, 73 / 49; top_k 256 40 / 55, 83 / 71.  Spread 0.05: top_k 50 39 / 39, 87 / 66; top_k 256 40 / 49, 91 / 74.  All logits equal:
 // 53 / 61, 235 / 81.  The host needs 60 us for a call's three launches and 80 for the nine of the passes, so that one row queued
-// behind others takes 82 / 63 us at all of these but the last, 81 / 84.  What a spread row takes is trips through memory and steps
+// behind others takes 82 / 63 us, 82 / 78 at the slowest of the spread ones and 81 / 83 with all logits equal.  What a spread row takes is trips through memory and steps
 // in LDS; a flat one is bound by what a single workgroup reads, about 10 us a time.
 constexpr int kFinishThreads = 1024, kFinishTopK = 256;
 constexpr int kFinishMost = 4096, kDirectMost = 256, kKeptMost = 1024, kLiveMost = 4096;

@@ -127,23 +127,21 @@ int launch_prefill_lds(const AttnArgs& a, dim3 grid, int min_rows, int max_kv_le
   const int fixed_rounds = g_prefill_fixed_rounds >= 0 ? g_prefill_fixed_rounds : (max_kv_len <= kDealtMaxKeys ? 1 << 20 : 2);
   attn_prefill_lds_kernel<DMAX, EXACT><<<workgroups, kPfWaves * kWave, lds, s>>>(a, min_rows, static_cast<int>(grid.x),
                                                                                 static_cast<int>(grid.z), listed, fixed_rounds);
-  if (a.portion_splits > 1) {
-    const long long most = static_cast<long long>(grid.x) * grid.y * grid.z * (kPfRows / kPfWaves);
-    attn_merge_portions_kernel<<<static_cast<unsigned>(most < 4LL * cus ? most : 4LL * cus), kPfWaves * kWave, 0, s>>>(a);
-  }
+  if (a.portion_splits > 1) launch_merge_portions(a, grid, cus, s);
   return launch_status();
 }
 
 
 static int g_prefill_groups = -1;  // -1: the launcher decides; 1, 2: forced (measurements and tests)
 
-template <int GROUPS>
-int launch_prefill_dma_groups(const AttnArgs& a, dim3 grid, int min_rows, int cus, int max_kv_len, hipStream_t s) {
+template <int GROUPS, bool BESIDE = false>
+int launch_prefill_dma_groups(const AttnArgs& a, dim3 grid, int min_rows, int cus, int max_kv_len, hipStream_t s, int longs,
+                              int beside_parts = 1) {
   const size_t lds = GROUPS * 2 * kDmStageBytes;
   static bool asked = false;  // dynamic LDS of 64 KiB and more has to be asked for, once
   if (!asked) {
-    for (const void* kernel : {reinterpret_cast<const void*>(&attn_prefill_dma_kernel<true, GROUPS>),
-                               reinterpret_cast<const void*>(&attn_prefill_dma_kernel<false, GROUPS>)}) {
+    for (const void* kernel : {reinterpret_cast<const void*>(&attn_prefill_dma_kernel<true, GROUPS, BESIDE>),
+                               reinterpret_cast<const void*>(&attn_prefill_dma_kernel<false, GROUPS, BESIDE>)}) {
       hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
       if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -152,8 +150,10 @@ int launch_prefill_dma_groups(const AttnArgs& a, dim3 grid, int min_rows, int cu
     }
     asked = true;
   }
-  const long long items = static_cast<long long>(grid.x) * grid.y * grid.z * a.portion_splits;
+  const long long items = static_cast<long long>(grid.x) * grid.y * longs * a.portion_splits;
   const long long places = (GROUPS == 1 ? 2LL : 1LL) * cus;  // two workgroups of four waves a CU, or one of eight
+  const int beside = BESIDE ? static_cast<int>(grid.z * grid.y) * beside_parts : 0;
+  const int beside_first = beside < cus ? beside : cus / static_cast<int>(grid.y) * static_cast<int>(grid.y);
   const unsigned workgroups = static_cast<unsigned>(items < places ? items : places);
   const int listed = static_cast<long long>(grid.x) * grid.z <= kPfPlanMax && grid.x <= 65535 && grid.z <= 65535;
   if (a.portion_splits > 1 && !listed) return static_cast<int>(hipErrorInvalidValue);
@@ -169,15 +169,12 @@ int launch_prefill_dma_groups(const AttnArgs& a, dim3 grid, int min_rows, int cu
   // of 64 to 800 tokens behind 0 to 2,300 372 against 387; a fresh prompt of 8,192 tokens 615 against 598.
   const int fixed_rounds = g_prefill_fixed_rounds >= 0 ? g_prefill_fixed_rounds : (max_kv_len <= kDealtMaxKeys ? 1 << 20 : 2);
   if (a.P % kDmKeys == 0)
-    attn_prefill_dma_kernel<true, GROUPS><<<workgroups, GROUPS * kDmWaves * kWave, lds, s>>>(
-        a, min_rows, static_cast<int>(grid.x), static_cast<int>(grid.z), listed, pair_up, fixed_rounds);
+    attn_prefill_dma_kernel<true, GROUPS, BESIDE><<<workgroups + beside, GROUPS * kDmWaves * kWave, lds, s>>>(
+        a, min_rows, static_cast<int>(grid.x), static_cast<int>(grid.z), listed, pair_up, fixed_rounds, beside, beside_first, beside_parts);
   else
-    attn_prefill_dma_kernel<false, GROUPS><<<workgroups, GROUPS * kDmWaves * kWave, lds, s>>>(
-        a, min_rows, static_cast<int>(grid.x), static_cast<int>(grid.z), listed, pair_up, fixed_rounds);
-  if (a.portion_splits > 1) {
-    const long long most = static_cast<long long>(grid.x) * grid.y * grid.z * (kPfRows / kPfWaves);
-    attn_merge_portions_kernel<<<static_cast<unsigned>(most < 4LL * cus ? most : 4LL * cus), kPfWaves * kWave, 0, s>>>(a);
-  }
+    attn_prefill_dma_kernel<false, GROUPS, BESIDE><<<workgroups + beside, GROUPS * kDmWaves * kWave, lds, s>>>(
+        a, min_rows, static_cast<int>(grid.x), static_cast<int>(grid.z), listed, pair_up, fixed_rounds, beside, beside_first, beside_parts);
+  if (a.portion_splits > 1) launch_merge_portions(a, grid, cus, s);
   return launch_status();
 }
 
@@ -202,8 +199,22 @@ int launch_prefill_dma(const AttnArgs& a, dim3 grid, int min_rows, int max_qlen,
   const bool unequal = 2LL * max_qlen > max_kv_len;  // the first rows see less than half of what the last see
   const bool two = g_prefill_groups >= 0 ? g_prefill_groups == 2
                                          : (4 * items > cus && (2 * items <= 3LL * cus || (unequal && items <= 2LL * cus)));
-  return two ? launch_prefill_dma_groups<2>(a, grid, min_rows, cus, max_kv_len, s)
-             : launch_prefill_dma_groups<1>(a, grid, min_rows, cus, max_kv_len, s);
+  const int longs = static_cast<int>(grid.z);
+  return two ? launch_prefill_dma_groups<2>(a, grid, min_rows, cus, max_kv_len, s, longs)
+             : launch_prefill_dma_groups<1>(a, grid, min_rows, cus, max_kv_len, s, longs);
+}
+
+// Portions and, in the same launch, the step's short segments: `parts` workgroups of four waves for each of them and kv
+// head, in front of the portions' workgroups.  longs: how many segments are portions.
+int launch_prefill_beside(const AttnArgs& a, dim3 grid, int min_rows, int parts, int longs, int max_kv_len, hipStream_t s) {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cus = n;
+  }
+  return launch_prefill_dma_groups<1, true>(a, grid, min_rows, cus, max_kv_len, s, longs > 0 ? longs : 1, parts);
 }
 
 // -1: the launcher decides (below); 1: head_dim 128 portions always run attn_prefill_dma_kernel; 0: always
@@ -225,12 +236,11 @@ inline bool prefill_dma_pays(dim3 grid, int max_qlen, int max_kv_len) {
 
 using namespace arle;
 
-// A mixed step's decoded tokens beside its portions: the two kinds of segments go to kernels of their own that do
-// not depend on each other.  With a side branch the split-KV kernel and its merge are queued on a second stream
+// A mixed step's decoded tokens beside its portions, where the portions kernel does not take both in one launch
+// (launch_prefill_beside: head_dim 128 on pages of eight slots and more): the two kinds of segments go to kernels of their
+// own that do not depend on each other.  With a side branch the split-KV kernel and its merge are queued on a second stream
 // (default priority) between an event that forks it off the caller's stream and one that joins it again, so that
 // they run beside the portions kernel; a capture of the caller's stream takes the branch in as parallel nodes.
-// Measured on MI355X, 8 decoding requests at 2,048 tokens beside a fresh portion of 504 (Qwen3-4B shape): 8.45
-// against 8.80 ms a step, the same bits.
 static int g_side_branch = 1;
 extern "C" void arle_attn_side_branch(int on) { g_side_branch = on; }
 
@@ -339,7 +349,8 @@ static AttnArgs make_args(const void* q, long long q_stride, void* out, long lon
 // must hold [token rows][nq][portion_splits][D] and [..][2] floats, and a merge of their own runs after.
 // plan_token: 0, or a number that names the step (the same for every layer of it, another for every other step of
 // the process): the portions kernels then list their work once a step instead of once a call.
-// sink: float32 [nq] or null; out_scale: a factor on the output (see AttnArgs).
+// sink: float32 [nq] or null; out_scale: a factor on the output (see AttnArgs).  short_segments: how many segments have
+// 16 rows at most, as far as the caller knows (choices of launches only).
 // Requires D % 16 == 0, D <= 256, page_size a power of two >= 4; rows of out 8-byte aligned.
 extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out, long long o_stride,
                                     const void* k_pages, const void* v_pages, const int* block_table,
@@ -349,7 +360,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
                                     int nq, int nkv, int D, int page_size, float scale, int window,
                                     int splits, float* ws_o, float* ws_ml, int portion_splits, float* pws_o,
                                     float* pws_ml, long long plan_token, const float* sink, float out_scale,
-                                    void* stream) {
+                                    int short_segments, void* stream) {
   if (segments == 0 || token_rows == 0) return 0;
   if (D % 16 != 0 || D > 256 || D <= 0 || page_size < 4 || (page_size & (page_size - 1)) != 0 || nq % nkv != 0 ||
       splits < 1 || splits > 64 || portion_splits < 1 || portion_splits > kPortionPartsMax ||
@@ -374,6 +385,17 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
     // prompt portions through the LDS kernel; segments of at most 16 rows (decoded tokens of a mixed
     // step) through the streaming kernel
     dim3 grid((max_rows + kPfRows - 1) / kPfRows, nkv, segments);
+    const bool dma = D == 128 && page_size % 8 == 0 && static_cast<long long>(nkv) * page_size * D < (1LL << 31) &&
+                     prefill_dma_pays(grid, max_qlen, max_kv_len);
+    if (dma && min_rows <= 16) {
+      const int parts = splits / kDmWaves > 1 ? splits / kDmWaves : 1;   // of a segment's keys; each is four waves
+      a.rows_max = 16;
+      rc = launch_prefill_beside(a, grid, 17, parts, segments - short_segments, max_kv_len, s);
+      if (rc != 0 || parts == 1) return rc;
+      attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
+          ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, a.rows_max, nq, nkv, D, parts, a.sink, a.out_scale, a.ws_plan);
+      return launch_status();
+    }
     SideBranch* side = (min_rows <= 16 && g_side_branch) ? side_branch(s) : nullptr;
     if (side != nullptr) {   // fork: what follows on the side stream waits for what the caller queued so far
       if (hipEventRecord(side->fork, s) != hipSuccess) return static_cast<int>(hipGetLastError());
@@ -402,8 +424,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
     }
     if (D == 64)
       rc = launch_prefill_lds<64, true>(a, grid, 17, max_kv_len, s);
-    else if (D == 128 && page_size % 8 == 0 && static_cast<long long>(nkv) * page_size * D < (1LL << 31) &&
-             prefill_dma_pays(grid, max_qlen, max_kv_len))
+    else if (dma)
       rc = launch_prefill_dma(a, grid, 17, max_qlen, max_kv_len, s);
     else if (D == 128)
       rc = launch_prefill_lds<128, true>(a, grid, 17, max_kv_len, s);

@@ -528,34 +528,41 @@ __global__ __launch_bounds__(kPfWaves* kWave, 1) __attribute__((amdgpu_waves_per
 }
 
 // The parts of a portion's rows put together: out = sum_p o_p 2^(m_p - m) / sum_p l_p 2^(m_p - m), in the order
-// of the parts.  Work items are (listed pair, kv head, eight rows of the row block): a workgroup of eight waves
-// takes items blockIdx.x, blockIdx.x + gridDim.x, ... and each wave one row of the item, a lane four columns
-// (head_dim <= 256).  No workgroup is launched for nothing, and no wave walks rows one after the other (a row
-// is two dependent loads: walking sixteen of them took longer than the attention itself).
+// of the parts, of which there are MOST at most.  Work items are (listed pair, kv head, a few rows of the row block): a
+// workgroup of eight waves takes items blockIdx.x, blockIdx.x + gridDim.x, ... and a row goes to as many lanes as it has
+// groups of four columns (head_dim <= 256).  No workgroup is launched for nothing, and no lane walks rows one after the other
+// (a row is two dependent loads, the list's entry with its segment and then all parts at once: walking sixteen of
+// them took longer than the attention itself).
 constexpr int kPortionPartsMax = 8;
+inline __host__ __device__ int merge_lane_bits(int D) { return D <= 64 ? 4 : D <= 128 ? 5 : 6; }   // lanes a row: 16, 32, 64
+inline __host__ __device__ int merge_items_a_block(int D) { return (kPfRows >> (6 - merge_lane_bits(D))) / kPfWaves; }
+template <int MOST>
 __global__ __launch_bounds__(kPfWaves* kWave) void attn_merge_portions_kernel(const AttnArgs a) {
   const int G = a.nq / a.nkv, D = a.D, parts = a.portion_splits;
+  const int bits = merge_lane_bits(D);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int d0 = 4 * lane;
-  constexpr int kSubBlocks = kPfRows / kPfWaves;  // items of eight rows in a row block
-  const unsigned int items = g_prefill_pairs * a.nkv * kSubBlocks;
-  for (unsigned int item = blockIdx.x; item < items; item += gridDim.x) {
-    const unsigned int pair = item / (a.nkv * kSubBlocks);
-    const int kvh = static_cast<int>((item / kSubBlocks) % a.nkv), sub = static_cast<int>(item % kSubBlocks);
+  const int d0 = 4 * (lane & ((1 << bits) - 1));
+  const int sub_row = (wave << (6 - bits)) + (lane >> bits);   // of an item's rows, the lane's
+  const unsigned int blocks = merge_items_a_block(D), per_pair = a.nkv * blocks;
+  unsigned int items = 0u;
+  for (unsigned int item = blockIdx.x; items == 0u || item < items; item += gridDim.x) {
+    // the list's entry goes out beside its length
+    const unsigned int pair = min(item / per_pair, static_cast<unsigned int>(kPfPlanMax - 1));
     const unsigned int entry = g_prefill_plan[pair];
-    const int seg = static_cast<int>(entry & 0xffffu);
-    const int row = static_cast<int>(entry >> 16) * kPfRows + sub * kPfWaves + wave;
-    const int row0 = a.seg_row0[seg];
-    const int rows = (a.seg_row0[seg + 1] - row0) * G;
-    if (row >= rows) continue;  // this wave only
+    const int4 of_seg = g_prefill_seg[pair];
+    if (items == 0u) items = g_prefill_pairs * per_pair;
+    if (item >= items) return;   // the whole workgroup
+    const int kvh = static_cast<int>((item / blocks) % a.nkv), sub = static_cast<int>(item % blocks);
+    const int row = static_cast<int>(entry >> 16) * kPfRows + sub * (kPfRows / static_cast<int>(blocks)) + sub_row;
+    if (row >= of_seg.y * G) continue;  // these lanes only
     const int head = kvh * G + row % G;
-    const int64_t tok_row = row0 + row / G;
+    const int64_t tok_row = of_seg.x + row / G;
     const int64_t base = (tok_row * a.nq + head) * parts;
-    float ms[kPortionPartsMax], ls[kPortionPartsMax];
-    float4 os[kPortionPartsMax];
+    float ms[MOST], ls[MOST];
+    float4 os[MOST];
     const float* src = a.pws_o + base * D + (d0 < D ? d0 : 0);
 #pragma unroll
-    for (int p = 0; p < kPortionPartsMax; ++p) {  // every load first, none under a condition
+    for (int p = 0; p < MOST; ++p) {  // every load first, none under a condition
       const int q = min(p, parts - 1);
       const float2 ml = *reinterpret_cast<const float2*>(a.pws_ml + (base + q) * 2);
       os[p] = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(q) * D);
@@ -564,11 +571,11 @@ __global__ __launch_bounds__(kPfWaves* kWave) void attn_merge_portions_kernel(co
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int p = 0; p < kPortionPartsMax; ++p) mx = fmaxf(mx, ms[p]);
+    for (int p = 0; p < MOST; ++p) mx = fmaxf(mx, ms[p]);
     float denom = 0.f;
     float4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int p = 0; p < kPortionPartsMax; ++p) {
+    for (int p = 0; p < MOST; ++p) {
       const float w = ms[p] > -INFINITY ? exp2f(ms[p] - mx) : 0.f;  // an empty part weighs nothing
       denom += ls[p] * w;
       o.x += os[p].x * w;
@@ -584,6 +591,18 @@ __global__ __launch_bounds__(kPfWaves* kWave) void attn_merge_portions_kernel(co
       *reinterpret_cast<uint2*>(a.out + tok_row * a.o_stride + head * D + d0) = w;
     }
   }
+}
+
+// The launch behind a portions kernel whose grid was `grid` (row blocks, kv heads, segments).
+inline void launch_merge_portions(const AttnArgs& a, dim3 grid, int cus, hipStream_t s) {
+  const long long most = static_cast<long long>(grid.x) * grid.y * grid.z * merge_items_a_block(a.D);
+  const dim3 wgs(static_cast<unsigned>(most < 4LL * cus ? most : 4LL * cus));
+  if (a.portion_splits <= 2)
+    attn_merge_portions_kernel<2><<<wgs, kPfWaves * kWave, 0, s>>>(a);
+  else if (a.portion_splits <= 4)
+    attn_merge_portions_kernel<4><<<wgs, kPfWaves * kWave, 0, s>>>(a);
+  else
+    attn_merge_portions_kernel<kPortionPartsMax><<<wgs, kPfWaves * kWave, 0, s>>>(a);
 }
 
 }  // namespace arle

@@ -82,9 +82,19 @@ __device__ __forceinline__ void load_to_lds_16(const void* base_uniform, uint32_
 // of two of four waves: a row block is done in half the time, which is what a launch waits for when it has about
 // as many row blocks as the chip has places for them (a causal prompt of 2,048 tokens: 512 row blocks from 1 to 32
 // tiles of keys, and the launch lasts as long as the heaviest).
-template <bool WHOLE, int GROUPS>
+//
+// BESIDE: `beside` of the workgroups take the step's short segments (decoded tokens: attn_mfma_body, four waves that share
+// the keys of a segment and kv head, or of one of `beside_parts` cuts of them, and merge in LDS), the others the portions.
+// The former wait for memory where the latter multiply, so a compute unit should hold one of each: the launch begins
+// with up to `beside_first` of them (one a compute unit), then come the portions' workgroups, then the rest.
+// One launch takes the place of two on streams of their own that were forked and joined around them, and spares a merge
+// where a segment's keys are not cut (32 requests at 1,024 tokens beside a portion of 512 behind 0, 512, 1,024 and
+// 1,536 at 32 q heads over 8 kv heads, us a layer: 59, 60, 63, 73 -> 36, 43, 45, 55).
+template <bool WHOLE, int GROUPS, bool BESIDE>
 __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void attn_prefill_dma_kernel(
-    const AttnArgs a, int min_rows, int blocks_x, int segments, int listed, int pair_up, int fixed_rounds) {
+    const AttnArgs a, int min_rows, int blocks_x, int segments, int listed, int pair_up, int fixed_rounds, int beside,
+    int beside_first, int beside_parts) {
+  static_assert(!BESIDE || GROUPS == 1, "a workgroup of decoded tokens is four waves");
   constexpr int D = kDmD;
   extern __shared__ __align__(16) unsigned char lds_all[];
   __shared__ unsigned int item_of_workgroup;
@@ -94,26 +104,40 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
   unsigned char* const lds_raw = lds_all + grp * (2 * kDmStageBytes);
   const int G = a.nq / a.nkv;
   const unsigned int nkv = static_cast<unsigned int>(a.nkv);
+  unsigned int wg = blockIdx.x, wgs = gridDim.x;   // this workgroup's place among those of the portions
+  if constexpr (BESIDE) {
+    wgs -= beside;
+    const unsigned int first = static_cast<unsigned int>(beside_first);
+    if (wg < first || wg >= first + wgs) {
+      if (wg >= first) wg -= wgs;
+      const int at = static_cast<int>(wg / nkv);
+      attn_mfma_body<1, kDmD, true, false, true, false>(a, at / beside_parts, static_cast<int>(wg % nkv), 0, kDmWaves, beside_parts,
+                                                        at % beside_parts, reinterpret_cast<float*>(lds_all));
+      return;
+    }
+    wg -= first;
+    __builtin_amdgcn_s_setprio(2);   // the portions' waves multiply where those of the decoded tokens mostly wait for memory
+  }
   const unsigned int pairs = listed ? g_prefill_pairs : static_cast<unsigned int>(blocks_x) * segments;
   const unsigned int parts = static_cast<unsigned int>(a.portion_splits);
   const unsigned int items = pairs * nkv * parts;
   const int P = a.P, ps = a.p_shift, pm = P - 1;
   const uint32_t page_elems32 = static_cast<uint32_t>(a.nkv) * P * D;  // the launcher refuses pages of 2^31 elements
  // With few items a workgroup (up to fixed_rounds) the items are dealt out before the launch instead of taken from
- // the counter: workgroup b takes item b of the first round of gridDim.x items, item gridDim.x - 1 - b of the
+ // the counter: workgroup b takes item b of the first round of wgs items, item wgs - 1 - b of the
  // second, and so on to and fro, so that on a list that runs from heavy to light every workgroup gets about the
  // same, and an item begins without the counter's round trip to memory; its list entry was asked for while the
  // item before it ran.
- const bool dealt = fixed_rounds > 0 && listed && items <= static_cast<unsigned long long>(fixed_rounds) * gridDim.x;
+ const bool dealt = fixed_rounds > 0 && listed && items <= static_cast<unsigned long long>(fixed_rounds) * wgs;
  unsigned int round = 0u;
  unsigned int ahead_entry = 0u;
  int4 ahead_seg = {0, 0, 0, 0};
  auto dealt_item = [&](unsigned int r) {
-   return r * gridDim.x + ((r & 1u) ? gridDim.x - 1u - blockIdx.x : blockIdx.x);
+   return r * wgs + ((r & 1u) ? wgs - 1u - wg : wg);
  };
- if (dealt && blockIdx.x < items) {
-   ahead_entry = g_prefill_plan[blockIdx.x / (nkv * parts)];
-   ahead_seg = g_prefill_seg[blockIdx.x / (nkv * parts)];
+ if (dealt && wg < items) {
+   ahead_entry = g_prefill_plan[wg / (nkv * parts)];
+   ahead_seg = g_prefill_seg[wg / (nkv * parts)];
  }
  for (;;) {
   unsigned int item;
@@ -130,7 +154,7 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
     if (item >= items) {
       // The last workgroup to leave puts the counters back to zero: the layers of a step hand out the same list one
       // after the other, and only the first of them runs the planning kernel.
-      if (tid == 0 && atomicAdd(&g_prefill_left, 1u) == gridDim.x - 1) {
+      if (tid == 0 && atomicAdd(&g_prefill_left, 1u) == wgs - 1) {
         g_prefill_next_item = 0u;
         g_prefill_left = 0u;
       }

@@ -24,10 +24,17 @@ namespace arle {
 // partial results in memory and no merge kernel.  For launches with a workgroup for every compute unit without it
 // (many requests, few splits); with fewer, one-wave workgroups spread the same waves over more compute units.
 constexpr int kInWgWavesMax = 4;
-template <int NT, int DMAX, bool EXACT, bool PREP = false, bool INWG = false, bool WHOLE_IN = false>
-__global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfma_kernel(const AttnArgs a) {
+//
+// A workgroup's place in the launch is handed in: its segment, kv head and first row, and with INWG the number of its
+// waves, in how many parts the segment's keys are cut over workgroups (`parts`) and which of them this one takes;
+// without INWG, parts is the number of splits.  `handed`: LDS for what the waves of a workgroup hand to wave 0.
+constexpr int kHandedPitch = 4 * (128 / 16) + 4;   // floats a lane: its sums, m and l, and padding to 16 bytes (head_dim 128 at most)
+constexpr int kHandedFloats = (kInWgWavesMax - 1) * kWave * kHandedPitch;
+template <int NT, int DMAX, bool EXACT, bool PREP, bool INWG, bool WHOLE_IN>
+__device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const int kvh, const int row_begin, const int waves,
+                                               const int parts, const int part, float* const handed) {
   static_assert(!PREP || (NT == 1 && EXACT), "the folded preparation is written for one row tile and a head_dim known here");
-  static_assert(!INWG || NT == 1, "the merge inside the workgroup is written for one row tile");
+  static_assert(!INWG || (NT == 1 && DMAX <= 128), "the merge inside the workgroup is written for one row tile");
   constexpr int DCH = DMAX / 32;  // contraction chunks of the first product
   constexpr int DTL = DMAX / 16;  // d tiles of the output
   const int lane = threadIdx.x & (kWave - 1), li = lane & 15, g = lane >> 4;
@@ -36,10 +43,11 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
   // are done.  Whole decode steps of the Qwen3-4B shape on MI355X, 19 requests of 16 to 4,000 tokens, 855 in the mean: 3.15
   // instead of 3.93 ms (the launch as long as the longest request's waves, 42 us a layer, before); equal contexts as before.
   constexpr bool SHARED_OUT = PREP && !INWG;
-  int seg = INWG ? static_cast<int>(blockIdx.z) : static_cast<int>(blockIdx.z) / a.splits;
-  int split = INWG ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) : static_cast<int>(blockIdx.z) % a.splits;
+  const int my_wave = INWG ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) : 0;
+  int split = INWG ? part * waves + my_wave : part;
+  const int splits = INWG ? parts * waves : parts;    // over how many waves the segment's keys go
   [[maybe_unused]] DecodeShare share{};
-  const bool shared_out = SHARED_OUT && a.splits > 1;
+  const bool shared_out = SHARED_OUT && splits > 1;
   if constexpr (SHARED_OUT) {
     if (shared_out) {
       const int wave = static_cast<int>(blockIdx.z), waves = static_cast<int>(gridDim.z);
@@ -63,13 +71,11 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
       seg = share.seg, split = share.split;
     }
   }
-  const int kvh = blockIdx.y;
   const int G = a.nq / a.nkv;
   const int row0 = shared_out ? seg : a.seg_row0[seg];                      // segments of one token: their rows in order
   const int qlen = shared_out ? 1 : a.seg_row0[seg + 1] - row0;
   const int rows = qlen * G;
-  const int row_begin = blockIdx.x * (16 * NT);
-  if (row_begin >= rows) return;  // the whole wave leaves
+  if (row_begin >= rows) return;  // the whole workgroup leaves
   if (a.rows_max > 0 && rows > a.rows_max) return;  // long segments belong to the LDS kernel
   const int start = shared_out ? share.start : a.seg_start[seg];
   const int* table = a.block_table + static_cast<int64_t>(shared_out ? share.slot : a.seg_slot[seg]) * a.table_stride;
@@ -82,8 +88,8 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
   const int kv_hi = start + tok_max + 1;   // exclusive bound of the keys any row here sees
   const int kv_lo = a.window > 0 ? max(0, start + tok_min - a.window + 1) : 0;
   int b0 = kv_lo / 32, b1 = (kv_hi + 31) / 32;
-  if (a.splits > 1) {
-    const int per = shared_out ? share.per : (b1 - b0 + a.splits - 1) / a.splits;
+  if (splits > 1) {
+    const int per = shared_out ? share.per : (b1 - b0 + splits - 1) / splits;
     b0 = b0 + split * per;
     b1 = min(b0 + per, b1);
   }
@@ -544,21 +550,20 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
   }
 
   if constexpr (INWG) {
-    // the waves 1 .. splits - 1 hand their sums to wave 0, lane to lane (a lane holds the same rows and columns in
+    // the waves behind the first hand their sums to wave 0, lane to lane (a lane holds the same rows and columns in
     // every wave): out = sum_s o_s 2^(m_s - m) / sum_s l_s 2^(m_s - m), added in the order of the splits
-    constexpr int kPitch = 4 * DTL + 4;   // floats a lane: its sums, m and l, and padding to 16 bytes
-    __shared__ __align__(16) float handed[kInWgWavesMax - 1][kWave][kPitch];
-    if (split > 0) {
-      float* mine = handed[split - 1][lane];
+    static_assert(4 * DTL + 4 <= kHandedPitch, "a lane's sums fit its place");
+    if (my_wave > 0) {
+      float* mine = handed + ((my_wave - 1) * kWave + lane) * kHandedPitch;
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt)
         *reinterpret_cast<float4*>(mine + 4 * dt) = float4{acc[0][dt][0], acc[0][dt][1], acc[0][dt][2], acc[0][dt][3]};
       *reinterpret_cast<float2*>(mine + 4 * DTL) = float2{m[0], l[0]};
     }
     __syncthreads();
-    if (split > 0) return;
-    for (int w = 1; w < a.splits; ++w) {
-      const float* theirs = handed[w - 1][lane];
+    if (my_wave > 0) return;
+    for (int w = 1; w < waves; ++w) {
+      const float* theirs = handed + ((w - 1) * kWave + lane) * kHandedPitch;
       const float2 ml = *reinterpret_cast<const float2*>(theirs + 4 * DTL);
       const float m_all = fmaxf(m[0], ml.x);
       const float m_ref = m_all == -INFINITY ? 0.f : m_all;
@@ -581,7 +586,7 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
   for (int n = 0; n < NT; ++n) {
     if (!row_ok[n]) continue;
     const int64_t tok_row = row0 + my_tok[n];
-    if (INWG || a.splits == 1 || (shared_out && share.count == 1)) {
+    if (parts == 1 || (shared_out && share.count == 1)) {
       const float inv_l = row_factor(a.sink, a.out_scale, my_head[n], m[n], l[n]);
       uint16_t* op = a.out + tok_row * a.o_stride + my_head[n] * D;
 #pragma unroll
@@ -598,7 +603,7 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
     } else {
       const int64_t ws_row = static_cast<int64_t>(seg) * a.ws_rows + my_tok[n];
       const int64_t slot = shared_out ? static_cast<int64_t>(share.first) * a.nq + my_head[n] * share.count + split
-                                      : (ws_row * a.nq + my_head[n]) * a.splits + split;
+                                      : (ws_row * a.nq + my_head[n]) * parts + part;
       float* wo = a.ws_o + slot * D;
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt) {
@@ -612,6 +617,17 @@ __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfm
         a.ws_ml[slot * 2 + 1] = l[n];
       }
     }
+  }
+}
+
+template <int NT, int DMAX, bool EXACT, bool PREP = false, bool INWG = false, bool WHOLE_IN = false>
+__global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfma_kernel(const AttnArgs a) {
+  const int z = static_cast<int>(blockIdx.z), row_begin = static_cast<int>(blockIdx.x) * (16 * NT);
+  if constexpr (INWG) {
+    __shared__ __align__(16) float handed[kHandedFloats];
+    attn_mfma_body<NT, DMAX, EXACT, PREP, true, WHOLE_IN>(a, z, blockIdx.y, row_begin, a.splits, 1, 0, handed);
+  } else {
+    attn_mfma_body<NT, DMAX, EXACT, PREP, false, WHOLE_IN>(a, z / a.splits, blockIdx.y, row_begin, 1, a.splits, z % a.splits, nullptr);
   }
 }
 

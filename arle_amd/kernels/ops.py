@@ -379,15 +379,28 @@ def _compute_units(device_index: int) -> int:
     return int(torch.cuda.get_device_properties(device_index).multi_processor_count)
 
 
+def beside_splits(segments: int, num_kv_heads: int, max_kv_len: int, device) -> int:
+    """Over how many waves the keys of every short segment go (four a workgroup) in a step whose portions the same launch
+    takes: a workgroup of them for every compute unit at most, beside which a portion's workgroup fits, and 512 keys each.
+    us a layer with 1 / 2 / 3 / 4 workgroups a segment and kv head (32 q heads over 8 kv heads): 32 requests at 1,024 tokens beside a
+    portion of 512 36 / 51 / 49 / 55, 16 at 4,000 beside 512 behind 2,000 90 / 74 / 95 / 97, 8 at 2,048 beside 504 35 / 32 / 29 / 30,
+    10 at 700 beside 333 18 / 22 / 24 / 24; 4 at 16,000 beside 512 with 1 / 4 / 8 of them 208 / 82 / 64."""
+    units = _compute_units(device.index if device.index is not None else torch.cuda.current_device())
+    keys = 1 << (max(int(max_kv_len), 1).bit_length() - 1)
+    return 4 * max(1, min(units // (segments * num_kv_heads), keys // 512, 16))
+
+
 def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_heads: int, num_kv_heads: int,
                        head_dim: int, max_kv_len: int, device) -> int:
     """Into how many parts the keys of every row block of a prompt portion are cut.
 
     The portions kernel gives a row block of 128 rows (tokens x q heads of a kv head) to a workgroup.  A short
     portion has fewer row blocks than the chip has compute units, however long its context: then the keys are
-    cut too, each part about a thousand keys long at least (the parts are merged by a kernel of its own, which
-    writes and reads every part's rows: for a fresh 512-token prompt two parts cost more than they save), and
-    the parts are merged afterwards.  The number depends on the shape of the step and on the power-of-two class of
+    cut too, as far as every part has a compute unit of its own and 512 keys, and the parts are merged by a kernel of
+    its own, which writes and reads every part's rows (5 to 8 us).  us a layer, 32 q heads over 8 kv heads, whole / 2 / 4 parts: a portion of 512
+    tokens behind 512 26 / 28 / 29, behind 1,024 34 / 32 / 32, behind 3,584 72 / 55 / 54; of 100 behind 2,000 56 / 36 / 24; of 300 behind
+    3,000 60 / 43 / 49 (3 parts: 37); of 512 beside 32 requests that decode at 1,024, behind 0, 512, 1,024 and 1,536: 36 / 41,
+    43 / 43, 54 / 46 and 68 / 52.  The number depends on the shape of the step and on the power-of-two class of
     the longest context only, like the split of decoded tokens, so that a captured step and an eager one choose
     alike.
     """
@@ -397,8 +410,8 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
     units = _compute_units(device.index if device.index is not None else torch.cuda.current_device())
     if items >= units or blocks * max(1, long_segments) > _PORTION_LIST_MAX:
         return 1
-    most = max(1, (1 << (max(int(max_kv_len), 1).bit_length() - 1)) // 1024)    # 2 from 2,048 keys on, 4 from 4,096, ...
-    parts = min(-(-2 * units // items), _PORTION_SPLITS_MAX, most)    # up to two items a compute unit
+    most = (1 << (max(int(max_kv_len), 1).bit_length() - 1)) // 512    # 2 from 1,024 keys on, 4 from 2,048, ...
+    parts = max(1, min(units // items, _PORTION_SPLITS_MAX, most))
     while parts > 1 and tokens * num_q_heads * parts * (head_dim + 2) * 4 > _PORTION_WS_BYTES:
         parts -= 1
     return parts
@@ -414,7 +427,8 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
     Segments: rows seg_row0[s]..seg_row0[s+1] belong to block-table row seg_slot[s] and start at
     position seg_start[s].  Segments whose rows (tokens x q heads of a kv head) fit one row tile of 16,
     decoded tokens above all, are split over the keys (split-KV), also beside longer portions in one
-    step; `short_segments` says how many there are (default: all), which sets the number of splits.
+    step (at head_dim 128 in one launch with them); `short_segments` says how many there are (default: all), which sets
+    the number of splits.
     Longer portions that are too few to fill the chip have their keys cut into `portion_splits` parts
     (default: portion_key_splits).  `plan_token` (new_plan_token()) names the step: with the same token and the
     same segments the portions kernels list their work once, for the first layer, and not once a layer.
@@ -450,7 +464,9 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
         splits = 1                      # no segment is short enough for the kernel that splits the keys
     elif splits is None:
         short = segments if short_segments is None else max(1, min(short_segments, segments))
-        splits = decode_splits(short, num_kv_heads, max_kv_len)
+        # beside portions in the kernel that takes both (csrc/attention_portions_dma.h), or in a launch of their own
+        both = max_qlen * group > _ATTN_ROW_TILE and head_dim == 128 and page_size % 8 == 0
+        splits = beside_splits(short, num_kv_heads, max_kv_len, q.device) if both else decode_splits(short, num_kv_heads, max_kv_len)
     _need(segments * splits <= _GRID_Y_MAX and num_kv_heads <= _GRID_Y_MAX, "too many segments for one launch")
     ws_o = ws_ml = None
     if splits > 1:
@@ -474,7 +490,7 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
              int(min_qlen), int(max_portion_kv_len or max_kv_len), tokens,
              num_q_heads, num_kv_heads, head_dim, page_size, float(scale), int(window), int(splits),
              _ptr(ws_o), _ptr(ws_ml), int(portion_splits), _ptr(pws_o), _ptr(pws_ml), int(plan_token),
-             _ptr(sink), float(out_scale), _stream())
+             _ptr(sink), float(out_scale), min(short_segments or 0, segments), _stream())
     return out
 
 

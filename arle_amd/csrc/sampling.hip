@@ -15,6 +15,7 @@
 // log-probability of a chosen token (the reference has it for greedy rows only,
 // sampling.cu:252-317) is a kernel of its own that serves greedy and sampled rows.
 #include "common.h"
+#include <cstring>
 #include <type_traits>
 
 namespace arle {
@@ -134,6 +135,44 @@ __global__ __launch_bounds__(kChunkThreads) void argmax_chunks_kernel(const floa
   }
 }
 
+// What a sampling call of rows with a small top_k wants of the logits: the largest of every 64 tokens of a chunk (a NaN is no
+// candidate; -inf of a group without tokens or with NaNs alone).  One read of the logits, kAhead pieces of 16 bytes a lane on
+// their way at once: 64 rows of 151,936 8.6 us, which with the launch's ramp is what reading 39 MB takes (11.0 with the
+// index of every chunk's largest beside it, which only greedy rows want and find in one group).
+__device__ __forceinline__ float row16_max(float v);
+__global__ __launch_bounds__(kChunkThreads) void group_max_kernel(const float* __restrict__ logits, int vocab, int chunk_len, int groups,
+                                                                  float* __restrict__ group_max) {
+  constexpr int kAhead = 5, kTokens = 64;
+  const int row = blockIdx.y, chunk = blockIdx.x, lane = threadIdx.x & (kWave - 1);
+  const int begin = chunk * chunk_len, len = min(vocab - begin, chunk_len);   // len: zero or less behind the row's end
+  const float* x = logits + static_cast<int64_t>(row) * vocab + begin;
+  float* gm = group_max + (static_cast<int64_t>(row) * gridDim.x + chunk) * groups;
+  const bool wide = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  for (int base = 4 * static_cast<int>(threadIdx.x); base < groups * kTokens; base += 4 * kChunkThreads * kAhead) {
+    float4 v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int at = base + 4 * kChunkThreads * j;
+      v[j] = float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (wide && at + 4 <= len) {
+        v[j] = *reinterpret_cast<const float4*>(x + at);
+      } else {
+        if (at < len) v[j].x = x[at];
+        if (at + 1 < len) v[j].y = x[at + 1];
+        if (at + 2 < len) v[j].z = x[at + 2];
+        if (at + 3 < len) v[j].w = x[at + 3];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int at = base + 4 * kChunkThreads * j;
+      // -inf among them: fmaxf of two NaNs is one
+      const float most = row16_max(fmaxf(fmaxf(fmaxf(v[j].x, -INFINITY), fmaxf(v[j].y, -INFINITY)), fmaxf(fmaxf(v[j].z, -INFINITY), fmaxf(v[j].w, -INFINITY))));
+      if ((lane & 15) == 0 && at < groups * kTokens) gm[at / kTokens] = most;
+    }
+  }
+}
+
 __global__ __launch_bounds__(kWave) void argmax_merge_kernel(const ArgMax* __restrict__ parts, int chunks,
                                                              int* __restrict__ out) {
   const ArgMax* p = parts + static_cast<int64_t>(blockIdx.x) * chunks;
@@ -215,24 +254,52 @@ struct SampleArgs {
   int* out;
 };
 
+// The e of a logit, the same bits wherever it is computed; mx: the row's largest logit over the temperature.
+__device__ __forceinline__ float weight_of(float x, float inv_t, float mx) { return expf(fmaf(x, inv_t, -mx)); }
+
+// Where a row's e are read: in memory, as sample_exp_kernel left them with the largest e of every group, or made from the logits,
+// with the groups' largest logits (group_max_kernel).  A larger logit may have an e that is smaller by the
+// rounding of two exponentials (expf is off by one unit at most): a group is looked at where its largest is kSlack units short.
+struct StoredWeights {
+  const float* e;
+  __device__ __forceinline__ float at(int i) const { return e[i]; }
+  __device__ __forceinline__ float of(float stored) const { return stored; }
+  __device__ __forceinline__ bool group_reaches(float most, unsigned int lower) const { return __float_as_uint(most) >= lower; }
+  __device__ __forceinline__ const float* row() const { return e; }
+};
+struct MadeWeights {
+  static constexpr unsigned int kSlack = 4;
+  const float* x;
+  float inv_t, mx;
+  __device__ __forceinline__ float at(int i) const { return weight_of(x[i], inv_t, mx); }
+  __device__ __forceinline__ float of(float logit) const { return weight_of(logit, inv_t, mx); }
+  __device__ __forceinline__ bool group_reaches(float most, unsigned int lower) const {
+    const float e = of(most);
+    return e >= 0.f && __float_as_uint(e) + kSlack >= lower;
+  }
+  __device__ __forceinline__ const float* row() const { return x; }
+};
+
 struct RowParams {
   float inv_t, min_p, top_p;
   int k;
   bool greedy, k_active, p_active;
 };
 
-__device__ __forceinline__ RowParams row_params(const SampleArgs& a, int row) {
+__device__ __forceinline__ RowParams row_params(const SampleArgs& a, float temp, int top_k, float top_p, float min_p) {
   RowParams r;
-  const float temp = a.temperature[row];
-  r.k = a.top_k[row];
-  r.top_p = a.top_p[row];
-  r.min_p = a.min_p[row];
+  r.k = top_k;
+  r.top_p = top_p;
+  r.min_p = min_p;
   // Greedy rule of the reference: (T <= 0 or top_k == 1) and no stochastic filter.
   r.greedy = (temp <= 0.f || r.k == 1) && r.top_p >= 1.f && r.min_p <= 0.f;
   r.inv_t = temp > 0.f ? 1.0f / temp : 1.0f;
   r.k_active = a.use_top_k && r.k > 0 && r.k < a.vocab;
   r.p_active = a.use_top_p && r.top_p < 1.f;
   return r;
+}
+__device__ __forceinline__ RowParams row_params(const SampleArgs& a, int row) {
+  return row_params(a, a.temperature[row], a.top_k[row], a.top_p[row], a.min_p[row]);
 }
 
 __device__ __forceinline__ unsigned int min_p_bits(const RowParams& r) {
@@ -453,8 +520,8 @@ __global__ __launch_bounds__(kSelThreads) void sample_exp_kernel(const SampleArg
     const int at = base + 4 * static_cast<int>(threadIdx.x);
     const float4 in = next;
     next = load(at + 4 * kSelThreads);
-    const float v[4] = {expf(in.x * r.inv_t - mx), expf(in.y * r.inv_t - mx), expf(in.z * r.inv_t - mx),
-                        expf(in.w * r.inv_t - mx)};
+    const float v[4] = {weight_of(in.x, r.inv_t, mx), weight_of(in.y, r.inv_t, mx), weight_of(in.z, r.inv_t, mx),
+                        weight_of(in.w, r.inv_t, mx)};
     float most = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -659,24 +726,24 @@ __device__ __forceinline__ void add_up_parts(PickLds& l, float before) {
 }
 
 // The token by the inverse CDF in token order, from e, the threshold and the chunks' kept masses.
-__device__ __forceinline__ void pick_token(const SampleArgs& a, int row, unsigned int thr, const float* masses, PickLds& l) {
-  find_target(a, a.u[row], masses, l);
+template <typename Weights>
+__device__ __forceinline__ void pick_token(const SampleArgs& a, int row, float u, unsigned int thr, const float* masses, const Weights& w, PickLds& l) {
+  find_target(a, u, masses, l);
   const int chunk = l.chunk_of_target;
   const float target = l.target, before = l.chunk_start;
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
   const int begin = chunk * a.chunk_len, end = min(a.vocab, begin + a.chunk_len);
   // thread t owns the tokens [lo, hi) of the chunk, in token order
   const int per = (end - begin + kSelThreads - 1) / kSelThreads;
   const bool owns = threadIdx.x < kSelThreads;
   const int lo = owns ? min(begin + static_cast<int>(threadIdx.x) * per, end) : end, hi = min(lo + per, end);
   auto kept = [&](int i) {
-    const float v = e[i];
+    const float v = w.at(i);
     return (v >= 0.f && __float_as_uint(v) >= thr) ? v : 0.f;
   };
   const float* gm = a.group_max + (static_cast<int64_t>(row) * a.chunks + chunk) * a.groups;
   bool live = false;   // a group that the thread's tokens lie in reaches the threshold
   if (lo < hi)
-    for (int g = (lo - begin) / kGroup; g <= (hi - 1 - begin) / kGroup; ++g) live |= __float_as_uint(gm[g]) >= thr;
+    for (int g = (lo - begin) / kGroup; g <= (hi - 1 - begin) / kGroup; ++g) live |= w.group_reaches(gm[g], thr);
   float mine = 0.f;
   if (live)
 #pragma unroll 4
@@ -729,24 +796,28 @@ __global__ __launch_bounds__(kSelThreads) void sample_pick_kernel(const SampleAr
   __shared__ PickLds l;
   const int row = blockIdx.x;
   if (row_params(a, row).greedy) pick_greedy(a, row, l);
-  else pick_token(a, row, a.threshold[row], a.chunk_mass + static_cast<int64_t>(row) * a.chunks, l);
+  else pick_token(a, row, a.u[row], a.threshold[row], a.chunk_mass + static_cast<int64_t>(row) * a.chunks, StoredWeights{a.e + static_cast<int64_t>(row) * a.vocab}, l);
 }
 
-// Rows with a small top_k: everything behind the first histogram in one kernel, a workgroup a row.  The tokens that the digits so
-// far leave are gathered into LDS (groups' largest e tell where they are); of more than kDirectMost the threshold's other digits
-// come from histograms of the list, and what does not reach it goes.  Each of the others is compared with all, which puts the list
+// Rows with a small top_k: everything behind the groups' maxima (group_max_kernel) in one kernel, a workgroup a row.  The
+// top_k-th largest of the maxima is a value that top_k tokens reach, and the tokens that do lie in the groups whose maxima do:
+// some fifty groups of 2,374 for top_k 50.  Their e are made again from the logits, with the same function, and gathered into
+// LDS; nothing else of the row is read and no e is written.  Of more than kDirectMost tokens the threshold's digits come from
+// histograms of the list, and what does not reach it goes.  Each of the others is compared with all, which puts the list
 // into the order of the tokens, for the chunks' masses and the token, and into that of the values, for the threshold of top_p (and
-// gives that of top_k where it is not known yet).  The thresholds are the same values (exact, counts and fixed-point masses); a chunk's mass is added in the order of sample_mass_kernel's threads
+// gives that of top_k where it is not known yet).  The thresholds are the same values as by the passes (exact, counts and
+// fixed-point masses); a chunk's mass is added in the order of sample_mass_kernel's threads
 // and waves, a thread's in pick_token's, where what is not kept adds nothing: the same bits, the same token.
-// The first histogram says how many tokens its digit leaves.  Where the list does not hold them (flat rows: the digit is a fifth of
-// a value wide), the workgroup reads the row for the next digit, and once more for the last one; tokens above the threshold are
-// then fewer than top_k, and if their ties fill more than the list these are counted and not listed.
-// MI355X, rows of 151,936 normal logits, the kernels of a call in us, with the passes of many workgroups / with this kernel.  Spread 2
-// (over the temperature), top_k 50 and top_p 0.9: one row 38 / 28, 64 rows 72 / 41; top_k 256 39 / 38, 76 / 53.  Spread 0.2: top_k 50 38 /
-// 32, 73 / 49; top_k 256 40 / 55, 83 / 71.  Spread 0.05: top_k 50 39 / 39, 87 / 66; top_k 256 40 / 49, 91 / 74.  All logits equal:
-// 53 / 61, 235 / 81.  The host needs 60 us for a call's three launches and 80 for the nine of the passes, so that one row queued
-// behind others takes 82 / 63 us, 82 / 78 at the slowest of the spread ones and 81 / 83 with all logits equal.  What a spread row takes is trips through memory and steps
-// in LDS; a flat one is bound by what a single workgroup reads, about 10 us a time.
+// Where more than kManyGroups maxima end in the threshold's value, the workgroup reads the row for the tokens above it: fewer
+// than top_k, and their ties are counted and not listed.  A list that overflows all the same (or a row of fewer groups than top_k) is
+// told from the row by digits.
+// MI355X, rows of 151,936 normal logits, the kernels of a call in us, with the passes of many workgroups / with this kernel.  Spread 2.5
+// (over the temperature), top_k 50 and top_p 0.9: one row 37 / 21, 64 rows 73 / 26; top_k 256 39 / 36, 76 / 40.  Spread 0.2: top_k 50 38 /
+// 24, 74 / 28; top_k 256 40 / 38, 82 / 44.  Spread 0.05: top_k 50 39 / 24, 90 / 28; top_k 256 41 / 39, 94 / 44.  All logits equal:
+// 53 / 69, 236 / 78.  (With a first histogram of all e in front of it, e written to memory and read again: 26, 41 and 39, 54 at
+// spread 2.5, 61 and 82 for equal logits.)  The host needs 36 us for a call with one object of parameters, so that a call queued behind others takes 35 us for one row
+// and 40 for 64; before 67 and 72.  What a spread row takes is trips through memory and steps in LDS; a flat one is
+// bound by what a single workgroup reads, about 10 us a time.
 constexpr int kFinishThreads = 1024, kFinishTopK = 256;
 constexpr int kFinishMost = 4096, kDirectMost = 256, kKeptMost = 1024, kLiveMost = 4096;
 constexpr int kFinishVocab = 1 << 28;      // a group's first token / 4 and its size share a word
@@ -758,6 +829,7 @@ struct FinishLds {
   int count, n_live;
   unsigned int threshold, ok, digit, left, found;
   unsigned int wave_total[kFinishThreads / kWave];
+  float largest[kFinishThreads / kWave];
   unsigned long long wave_mass_total[kFinishThreads / kWave];
   float masses[256];
   int first[256], behind[256];            // of a chunk: its first token in the list, and the one behind its last
@@ -839,41 +911,47 @@ __device__ __forceinline__ bool reach_bin(const unsigned int (&m)[PER], int bits
   return ok;
 }
 
-// Digit LEVEL (1 or 2) of top_k's threshold from the counts in l.bins.
-template <int LEVEL>
-__device__ __forceinline__ bool digit_of_bins(unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
-  constexpr int kPer = (LEVEL == 1 ? kBins1 : kBins2) / kFinishThreads;
+// Digit `level` of 31 bits, ten, eleven and ten at a time from the top (a run-time number: the three digits share their code).
+struct Digit {
+  int low, bits, high;
+  __device__ __forceinline__ explicit Digit(int level) : low(level == 0 ? 21 : level == 1 ? 10 : 0), bits(level == 1 ? 11 : 10), high(low + bits) {}
+  __device__ __forceinline__ int bin(unsigned int v) const { return static_cast<int>((v >> low) & ((1u << bits) - 1u)); }
+};
+__device__ __forceinline__ void clear_bins(FinishLds& l) {
+#pragma unroll
+  for (int j = 0; j < kBins1 / kFinishThreads; ++j) l.bins[j * kFinishThreads + threadIdx.x] = 0u;
+  __syncthreads();
+}
+// The digit of a threshold from the counts in l.bins (those behind a digit's last bin are zero).
+__device__ __forceinline__ bool digit_of_bins(const Digit& d, unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
+  constexpr int kPer = kBins1 / kFinishThreads;
+  static_assert(kBins0 <= kBins1 && kBins2 <= kBins1, "the bins of any digit");
   __syncthreads();
   unsigned int m[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) m[j] = l.bins[kPer * threadIdx.x + j];
-  return reach_bin<kPer>(m, LEVEL == 1 ? 11 : 10, prefix, rest, found, l);
-}
-template <int LEVEL>
-__device__ __forceinline__ void clear_bins(FinishLds& l) {
-#pragma unroll
-  for (int j = 0; j < (LEVEL == 1 ? kBins1 : kBins2) / kFinishThreads; ++j) l.bins[j * kFinishThreads + threadIdx.x] = 0u;
-  __syncthreads();
+  return reach_bin<kPer>(m, d.bits, prefix, rest, found, l);
 }
 
 // The digit from the whole row.  Every lane has kAhead 16-byte pieces on their way at once, because one workgroup's share of the
 // memory's rate is what it has in flight; a wave whose values are all alike counts them as one.
-template <int LEVEL>
-__device__ __forceinline__ bool digit_of_row(const float* __restrict__ e, int vocab, unsigned int floor, unsigned int& prefix,
+__device__ __forceinline__ bool digit_of_row(const Digit& d, const MadeWeights& w, int vocab, unsigned int floor, unsigned int& prefix,
                                              unsigned int& rest, unsigned int& found, FinishLds& l) {
-  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 1 ? 10 : 0, kMask = (LEVEL == 1 ? kBins1 : kBins2) - 1, kAhead = 8;
+  constexpr int kAhead = 8;
+  const float* __restrict__ x = w.row();
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const unsigned int from = max(floor, prefix << kHigh), behind = (prefix + 1u) << kHigh;   // neither NaN nor -1: they are beyond any prefix
-  clear_bins<LEVEL>(l);
+  // neither NaN nor -1: they are beyond any prefix
+  const unsigned int from = max(floor, prefix << d.high), behind = min((prefix + 1u) << d.high, 0x7f800000u);
+  clear_bins(l);
   auto count = [&](float v) {
     const unsigned int bits = __float_as_uint(v);
-    if (bits >= from && bits < behind) atomicAdd(&l.bins[(bits >> kLow) & kMask], 1u);
+    if (bits >= from && bits < behind) atomicAdd(&l.bins[d.bin(bits)], 1u);
   };
-  const int head = min(vocab, static_cast<int>((4u - (static_cast<unsigned int>(reinterpret_cast<uintptr_t>(e)) / 4u) % 4u) % 4u));
+  const int head = min(vocab, static_cast<int>((4u - (static_cast<unsigned int>(reinterpret_cast<uintptr_t>(x)) / 4u) % 4u) % 4u));
   const int pieces = (vocab - head) / 4, tail = head + 4 * pieces;
-  if (tid < head) count(e[tid]);
-  if (tid < vocab - tail) count(e[tail + tid]);
-  const float4* at = reinterpret_cast<const float4*>(e + head);
+  if (tid < head) count(w.at(tid));
+  if (tid < vocab - tail) count(w.at(tail + tid));
+  const float4* at = reinterpret_cast<const float4*>(x + head);
   for (int base = 0; base < pieces; base += kAhead * kFinishThreads) {
     float4 v[kAhead];
 #pragma unroll
@@ -884,34 +962,111 @@ __device__ __forceinline__ bool digit_of_row(const float* __restrict__ e, int vo
       const unsigned int lead = __builtin_amdgcn_readfirstlane(__float_as_int(v[j].x));
       const bool alike = in && __float_as_uint(v[j].x) == lead && __float_as_uint(v[j].y) == lead && __float_as_uint(v[j].z) == lead && __float_as_uint(v[j].w) == lead;
       if (__ballot(alike) == ~0ull) {
-        if (lane == 0 && lead >= from && lead < behind) atomicAdd(&l.bins[(lead >> kLow) & kMask], 4u * kWave);
+        const unsigned int bits = __float_as_uint(w.of(__uint_as_float(lead)));
+        if (lane == 0 && bits >= from && bits < behind) atomicAdd(&l.bins[d.bin(bits)], 4u * kWave);
       } else if (in) {
-        count(v[j].x), count(v[j].y), count(v[j].z), count(v[j].w);
+        count(w.of(v[j].x)), count(w.of(v[j].y)), count(w.of(v[j].z)), count(w.of(v[j].w));
       }
     }
   }
-  return digit_of_bins<LEVEL>(prefix, rest, found, l);
+  return digit_of_bins(d, prefix, rest, found, l);
+}
+
+// The row's tokens above `tie`, into l.raw; how many there are, and in `reach` those from `tie` on.
+__device__ __forceinline__ int above_tie(const MadeWeights& w, int vocab, unsigned int tie, int& reach, FinishLds& l) {
+  constexpr int kAhead = 8;
+  const float* __restrict__ x = w.row();
+  const int tid = threadIdx.x;
+  if (tid == 0) l.count = l.n_live = 0;
+  __syncthreads();
+  int mine = 0;
+  auto take = [&](const float (&v)[4], int token, bool in) {      // every lane of the wave; token: the first of four
+    bool more[4];
+    float e[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      e[j] = w.of(v[j]);
+      const bool ok = in && e[j] >= 0.f;
+      mine += ok && __float_as_uint(e[j]) >= tie;
+      more[j] = ok && __float_as_uint(e[j]) > tie;
+    }
+    append(more, &l.count, [&](int at, int j) { if (at < kFinishMost) l.raw[at] = uint2{__float_as_uint(e[j]), static_cast<unsigned int>(token + j)}; });
+  };
+  const int head = min(vocab, static_cast<int>((4u - (static_cast<unsigned int>(reinterpret_cast<uintptr_t>(x)) / 4u) % 4u) % 4u));
+  const int pieces = (vocab - head) / 4, tail = head + 4 * pieces;
+  const float none = -INFINITY;
+  unsigned int last = 0x7fc00000u, lead_bits = 0x7fc00000u;   // a NaN, and its e
+  take({tid < head ? x[tid] : none, none, none, none}, tid, tid < head);
+  take({tid < vocab - tail ? x[tail + tid] : none, none, none, none}, tail + tid, tid < vocab - tail);
+  const float4* at = reinterpret_cast<const float4*>(x + head);
+  for (int base = 0; base < pieces; base += kAhead * kFinishThreads) {
+    float4 v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = at[min(base + j * kFinishThreads + tid, pieces - 1)];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int piece = base + j * kFinishThreads + tid;
+      const bool in = piece < pieces;
+      const unsigned int lead = __builtin_amdgcn_readfirstlane(__float_as_int(v[j].x));
+      const bool alike = in && __float_as_uint(v[j].x) == lead && __float_as_uint(v[j].y) == lead && __float_as_uint(v[j].z) == lead && __float_as_uint(v[j].w) == lead;
+      if (__builtin_expect(lead != last, 0)) last = lead, lead_bits = __float_as_uint(w.of(__uint_as_float(lead)));
+      const unsigned int bits = lead_bits;
+      if (__ballot(alike) == ~0ull && bits <= tie)
+        mine += bits == tie ? 4 : 0;
+      else
+        take({v[j].x, v[j].y, v[j].z, v[j].w}, head + 4 * piece, in);
+    }
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) mine += __shfl_xor(mine, off, kWave);
+  if ((tid & (kWave - 1)) == 0 && mine != 0) atomicAdd(&l.n_live, mine);
+  __syncthreads();
+  reach = l.n_live;
+  return l.count;
 }
 
 // The digit from the list.
-template <int LEVEL>
-__device__ __forceinline__ bool digit_of_list(int n, unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
-  constexpr int kHigh = LEVEL == 1 ? 21 : 10, kLow = LEVEL == 1 ? 10 : 0, kMask = (LEVEL == 1 ? kBins1 : kBins2) - 1;
-  clear_bins<LEVEL>(l);
+__device__ __forceinline__ bool digit_of_list(const Digit& d, int n, unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
+  clear_bins(l);
   for (int i = threadIdx.x; i < n; i += kFinishThreads) {
     const unsigned int bits = l.raw[i].x;
-    if ((bits >> kHigh) == prefix) atomicAdd(&l.bins[(bits >> kLow) & kMask], 1u);
+    if ((bits >> d.high) == prefix) atomicAdd(&l.bins[d.bin(bits)], 1u);
   }
-  return digit_of_bins<LEVEL>(prefix, rest, found, l);
+  return digit_of_bins(d, prefix, rest, found, l);
+}
+
+// The digit of the rank-th largest of the groups' largest e.  `most`: the first groups' largest logits, fetched by the caller.
+constexpr int kGroupsAhead = 4;
+__device__ __forceinline__ bool digit_of_groups(const Digit& d, const MadeWeights& w, const float* gm, int groups, const float (&most)[kGroupsAhead],
+                                                unsigned int& prefix, unsigned int& rest, unsigned int& found, FinishLds& l) {
+  clear_bins(l);
+  for (int base = 0; base < groups; base += kGroupsAhead * kFinishThreads) {
+#pragma unroll
+    for (int j = 0; j < kGroupsAhead; ++j) {
+      const int g = base + j * kFinishThreads + static_cast<int>(threadIdx.x);
+      const float e = w.of(base == 0 ? most[j] : gm[min(g, groups - 1)]);
+      const unsigned int bits = __float_as_uint(e);
+      // (a wave whose lanes all fall into one bin adds them at once: flat rows)
+      const bool in = g < groups && e >= 0.f && (bits >> d.high) == prefix;
+      const int bin = d.bin(bits), lead = __builtin_amdgcn_readfirstlane(bin);
+      const unsigned long long some = __ballot(in);
+      if (some == __ballot(in && bin == lead)) {
+        if ((threadIdx.x & (kWave - 1)) == 0 && some != 0ull) atomicAdd(&l.bins[lead], static_cast<unsigned int>(__builtin_popcountll(some)));
+      } else if (in) {
+        atomicAdd(&l.bins[bin], 1u);
+      }
+    }
+  }
+  return digit_of_bins(d, prefix, rest, found, l);
 }
 
 // The row's tokens from `lower` on, into l.raw; how many there are (more than kFinishMost: some are not listed).  `most`: the
-// largest e of the first groups, fetched by the caller.
-constexpr int kGroupsAhead = 4;
-__device__ __forceinline__ int gather(const SampleArgs& a, int row, unsigned int lower, const float* gm, int groups,
+// largest logits of the first groups, fetched by the caller.
+__device__ __forceinline__ int gather(const SampleArgs& a, unsigned int lower, const MadeWeights& w, const float* gm, int groups,
                                       const float (&most)[kGroupsAhead], FinishLds& l) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const float inverse = 1.0f / static_cast<float>(a.groups);
+  static_assert(kGroupsAhead * kFinishThreads <= kLiveMost, "a round's groups fit the list");
   if (tid == 0) l.count = l.n_live = 0;
   __syncthreads();
   for (int base = 0; base < groups; base += kGroupsAhead * kFinishThreads) {
@@ -924,31 +1079,34 @@ __device__ __forceinline__ int gather(const SampleArgs& a, int row, unsigned int
       int in_chunk;
       const int chunk = quotient(g, a.groups, inverse, in_chunk), first = chunk * a.chunk_len + in_chunk * kGroup;
       const int tokens = min(min(a.chunk_len - in_chunk * kGroup, a.vocab - first), kGroup);
-      // (a chunk's last groups may lie past its end, and nobody has written those)
-      live[j] = g < groups && tokens > 0 && __float_as_uint(m) >= lower;
+      // (a chunk's last groups may lie past its end)
+      live[j] = g < groups && tokens > 0 && w.group_reaches(m, lower);
       entry[j] = static_cast<unsigned int>(first) / 4u * kGroup + static_cast<unsigned int>(tokens - 1);
     }
-    append(live, &l.n_live, [&](int at, int j) { if (at < kLiveMost) l.live[at] = entry[j]; });
-  }
-  __syncthreads();
-  const int n_live = l.n_live;
-  if (n_live > kLiveMost) return kFinishMost + 1;
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
-  constexpr int kEach = 8;
-  for (int base = kEach * wave; base < n_live; base += kEach * kFinishThreads / kWave) {
-    float v[kEach];
-    int token[kEach];
-    bool in[kEach];
+    append(live, &l.n_live, [&](int at, int j) { l.live[at] = entry[j]; });
+    __syncthreads();
+    const int n_live = l.n_live;
+    constexpr int kEach = 8;
+    for (int from = kEach * wave; from < n_live; from += kEach * kFinishThreads / kWave) {
+      float v[kEach];
+      int token[kEach];
+      bool in[kEach];
 #pragma unroll
-    for (int j = 0; j < kEach; ++j) {
-      const unsigned int entry = l.live[min(base + j, n_live - 1)];
-      in[j] = base + j < n_live && lane <= static_cast<int>(entry % kGroup);
-      token[j] = static_cast<int>(entry / kGroup * 4u) + min(lane, static_cast<int>(entry % kGroup));
-      v[j] = e[token[j]];
+      for (int j = 0; j < kEach; ++j) {
+        const unsigned int entry = l.live[min(from + j, n_live - 1)];
+        in[j] = from + j < n_live && lane <= static_cast<int>(entry % kGroup);
+        token[j] = static_cast<int>(entry / kGroup * 4u) + min(lane, static_cast<int>(entry % kGroup));
+        v[j] = w.row()[token[j]];
+      }
+#pragma unroll
+      for (int j = 0; j < kEach; ++j) v[j] = w.of(v[j]);
+#pragma unroll
+      for (int j = 0; j < kEach; ++j) in[j] = in[j] && v[j] >= 0.f && __float_as_uint(v[j]) >= lower;
+      append(in, &l.count, [&](int at, int j) { if (at < kFinishMost) l.raw[at] = uint2{__float_as_uint(v[j]), static_cast<unsigned int>(token[j])}; });
     }
-#pragma unroll
-    for (int j = 0; j < kEach; ++j) in[j] = in[j] && v[j] >= 0.f && __float_as_uint(v[j]) >= lower;
-    append(in, &l.count, [&](int at, int j) { if (at < kFinishMost) l.raw[at] = uint2{__float_as_uint(v[j]), static_cast<unsigned int>(token[j])}; });
+    __syncthreads();
+    if (tid == 0) l.n_live = 0;
+    if (base + kGroupsAhead * kFinishThreads < groups) __syncthreads();
   }
   __syncthreads();
   return l.count;
@@ -974,9 +1132,18 @@ __device__ __forceinline__ int keep_from(unsigned int lower, int n, FinishLds& l
 }
 
 // The kept mass of every chunk from the row, in the order of sample_mass_kernel: 256 threads a chunk, kAhead chunks of theirs at once.
-__device__ __forceinline__ void masses_of_row(const SampleArgs& a, int row, unsigned int thr, FinishLds& l) {
+__device__ __forceinline__ void masses_of_row(const SampleArgs& a, const MadeWeights& w, unsigned int thr, FinishLds& l) {
   constexpr int kAhead = 4, kUnroll = 9, kGroups = kFinishThreads / kSelThreads;
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  const float* x = w.row();
+  float last = __uint_as_float(0x7fc00000u), last_kept = 0.f;   // rows of many ties: an exponential only where a lane's logit is another than before
+  auto kept = [&](float logit) {
+    if (__builtin_expect(__ballot(logit != last) != 0ull, 0)) {
+      asm volatile("");   // a branch, not two values to choose from
+      const float e = w.of(logit);
+      last = logit, last_kept = e >= 0.f && __float_as_uint(e) >= thr ? e : 0.f;
+    }
+    return last_kept;
+  };
   const int t = threadIdx.x % kSelThreads, lane = threadIdx.x & (kWave - 1), wave = t / kWave;
   for (int c0 = threadIdx.x / kSelThreads; c0 < a.chunks; c0 += kAhead * kGroups) {
     float mass[kAhead] = {};
@@ -985,13 +1152,14 @@ __device__ __forceinline__ void masses_of_row(const SampleArgs& a, int row, unsi
 #pragma unroll
       for (int j = 0; j < kAhead; ++j)
 #pragma unroll
-        for (int k = 0; k < kUnroll; ++k) v[j][k] = e[min(min(c0 + j * kGroups, a.chunks - 1) * a.chunk_len + i + k * kSelThreads, a.vocab - 1)];
+        for (int k = 0; k < kUnroll; ++k) v[j][k] = x[min(min(c0 + j * kGroups, a.chunks - 1) * a.chunk_len + i + k * kSelThreads, a.vocab - 1)];
 #pragma unroll
       for (int j = 0; j < kAhead; ++j)
 #pragma unroll
         for (int k = 0; k < kUnroll; ++k) {
           const bool in = i + k * kSelThreads < min(a.chunk_len, a.vocab - (c0 + j * kGroups) * a.chunk_len);
-          if (in && v[j][k] >= 0.f && __float_as_uint(v[j][k]) >= thr) mass[j] += v[j][k];
+          const float e = kept(v[j][k]);
+          if (in) mass[j] += e;
         }
     }
 #pragma unroll
@@ -1010,7 +1178,45 @@ __device__ __forceinline__ void masses_of_row(const SampleArgs& a, int row, unsi
   __syncthreads();
 }
 
-__global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const SampleArgs a) {
+// The first token with the row's largest logit: in the first group that has it; where the largest is -inf a group of NaNs alone
+// looks the same, and the whole row is searched.
+__device__ __forceinline__ void first_of(const SampleArgs& a, int row, float largest, const float* gm, int groups, FinishLds& l) {
+  const float* x = a.logits + static_cast<int64_t>(row) * a.vocab;
+  constexpr int kNone = 0x7fffffff;
+  if (threadIdx.x == 0) l.count = l.n_live = kNone;
+  __syncthreads();
+  int group = kNone;
+  for (int g = threadIdx.x; g < groups && group == kNone; g += kFinishThreads)
+    if (gm[g] == largest) group = g;
+  if (group != kNone) atomicMin(&l.count, group);
+  __syncthreads();
+  group = l.count;
+  int from = 0, to = a.vocab;
+  if (largest > -INFINITY) {
+    const int chunk = group / a.groups, in_chunk = group % a.groups;
+    from = chunk * a.chunk_len + in_chunk * kGroup;
+    to = min(min(from + kGroup, (chunk + 1) * a.chunk_len), a.vocab);
+  }
+  for (int i = from + static_cast<int>(threadIdx.x); i < to; i += kFinishThreads)
+    if (x[i] == largest) {
+      atomicMin(&l.n_live, i);
+      break;
+    }
+  __syncthreads();
+  if (threadIdx.x == 0) a.out[row] = l.n_live == kNone ? 0 : l.n_live;
+}
+
+constexpr unsigned int kManyGroups = 512;
+// The parameters of up to kInlineRows rows as an argument of the kernel: no copy to the GPU in front of it.
+constexpr int kInlineRows = 64;
+struct InlineRows {
+  float temperature[kInlineRows], top_p[kInlineRows], min_p[kInlineRows], u[kInlineRows];
+  int top_k[kInlineRows];
+};
+struct NoRows {};
+
+template <typename Rows>
+__global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const SampleArgs a, const Rows rows) {
   __shared__ FinishLds l;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   // what is wanted of the row and does not hang on anything else: all on its way at once
@@ -1019,51 +1225,73 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const Sam
   float most[kGroupsAhead];
 #pragma unroll
   for (int j = 0; j < kGroupsAhead; ++j) most[j] = gm[min(j * kFinishThreads + tid, groups - 1)];
-  const unsigned int own[1] = {a.hist_k[static_cast<int64_t>(row) * kRowBins + tid]};
-  const float u = a.u[row];
-  const RowParams r = row_params(a, row);
+  RowParams r;
+  float u;
+  if constexpr (std::is_same_v<Rows, InlineRows>) {
+    r = row_params(a, rows.temperature[row], rows.top_k[row], rows.top_p[row], rows.min_p[row]);
+    u = rows.u[row];
+  } else {
+    r = row_params(a, row);
+    u = a.u[row];
+  }
+  float largest = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < kGroupsAhead; ++j) largest = fmaxf(largest, most[j]);
+  for (int g = kGroupsAhead * kFinishThreads + tid; g < groups; g += kFinishThreads) largest = fmaxf(largest, gm[g]);
+  largest = block_max<kFinishThreads / kWave>(largest, l.largest);
   if (r.greedy) {
-    pick_greedy(a, row, l.pick);
+    first_of(a, row, largest, gm, groups, l);
     return;
   }
-  const float* e = a.e + static_cast<int64_t>(row) * a.vocab;
+  const MadeWeights w{a.logits + static_cast<int64_t>(row) * a.vocab, r.inv_t, largest * r.inv_t};
   const unsigned int mp = min_p_bits(r), k = static_cast<unsigned int>(r.k);
   if (tid == 0) l.threshold = mp;
   for (int c = tid; c < 256; c += kFinishThreads) l.first[c] = l.behind[c] = 0, l.masses[c] = 0.f;
-  static_assert(kFinishThreads == kBins0, "a bin of the first digit a thread");
+  // The top_k-th largest of the groups' largest e, or a digit's lower end that not many more groups reach: top_k tokens are there
+  // or above, and those that are lie in these groups.  (An e of zero weighs nothing and is never drawn: where the rank is
+  // only reached among those, most logits -inf, say, the others all stay, which is what the list then gives.)
   unsigned int prefix = 0u, rest = k, found = 0u;
-  const bool open = !reach_bin<1>(own, 10, prefix, rest, found, l);      // the row does not reach the rank: everything above min_p's floor stays
-  // Tokens that may be kept.  An e of zero weighs nothing and is never drawn: where the rank is only reached among those (most logits
-  // -inf, say), the others all stay, which is what the list then gives.  (The lowest digit counts zeros too and says nothing of the list.)
-  unsigned int lower = max(open ? mp : max(mp, prefix << 21), 1u);
-  int digits = 1, n = kFinishMost + 1;      // digits of top_k's threshold that are known, tokens from `lower` on
-  unsigned int ties = 0u;                   // tokens at the threshold that are not listed
-  auto listed = [&] { return (k - rest) + found <= static_cast<unsigned int>(kFinishMost); };
-  if (open || prefix == 0u || listed()) n = gather(a, row, lower, gm, groups, most, l);
-  if (n > kFinishMost) {      // and then the rank is reached (fewer than top_k tokens otherwise)
-    bool ok = digit_of_row<1>(e, a.vocab, mp, prefix, rest, found, l);
-    digits = 2;
-    if (ok && !listed()) ok = digit_of_row<2>(e, a.vocab, mp, prefix, rest, found, l), digits = 3;
-    lower = max(max(mp, digits == 2 ? prefix << 10 : prefix), 1u);
-    if (digits == 3 && !listed()) {
-      if (prefix > 0u) ties = found;
-      lower = prefix + 1u;
-    }
-    n = gather(a, row, lower, gm, groups, most, l);
+  auto few = [&] { return (k - rest) + found <= max(2u * k, 128u); };
+  int digits = 0;
+  while (digits < 3 && (digits == 0 || !few()) && digit_of_groups(Digit(digits), w, gm, groups, most, prefix, rest, found, l)) ++digits;
+  const unsigned int reached = digits == 0 ? 0u : prefix << Digit(digits - 1).low;   // 0 where fewer groups than that are there
+  const unsigned int reaching = digits == 3 ? (k - rest) + found : 0u;   // groups whose largest reaches the threshold of the groups
+  unsigned int lower = max(max(mp, reached), 1u), thr = mp, ties = 0u;   // ties: tokens at the threshold that are not listed
+  bool known = false;
+  int n;
+  if (reaching > kManyGroups && lower == reached) {
+    // so many groups end in one value that it is most likely the threshold: those above it are the list
+    int reach;
+    n = above_tie(w, a.vocab, lower, reach, l);
+    if (static_cast<unsigned int>(n) < k) thr = lower, ties = static_cast<unsigned int>(reach - n), known = true;
+  } else {
+    n = gather(a, lower, w, gm, groups, most, l);
   }
-  unsigned int thr = digits == 3 ? max(mp, prefix) : mp;
-  bool known = open || digits == 3;
+  rest = k, found = 0u, prefix = 0u;
+  if (n > kFinishMost) {      // the row by digits: the rank is reached from `lower` on (fewer than top_k tokens otherwise)
+    auto listed = [&] { return (k - rest) + found <= static_cast<unsigned int>(kFinishMost); };
+    int row_digits = 0;
+    while (row_digits < 3 && (row_digits == 0 || !listed()) && digit_of_row(Digit(row_digits), w, a.vocab, lower, prefix, rest, found, l)) ++row_digits;
+    if (row_digits > 0) lower = max(lower, prefix << Digit(row_digits - 1).low);
+    if (row_digits == 3) {
+      thr = max(mp, prefix), known = true;
+      if (!listed()) ties = found, lower = prefix + 1u;
+    }
+    n = gather(a, lower, w, gm, groups, most, l);
+    rest = k, found = 0u, prefix = 0u;
+  }
   if (n > kDirectMost && !known) {
-    bool ok = digits == 2 || digit_of_list<1>(n, prefix, rest, found, l);
-    ok = ok && digit_of_list<2>(n, prefix, rest, found, l);
-    if (ok) thr = max(mp, prefix);
+    int list_digits = 0;
+    while (list_digits < 3 && digit_of_list(Digit(list_digits), n, prefix, rest, found, l)) ++list_digits;
+    if (list_digits == 3) thr = max(mp, prefix);
     known = true;
     const int all = n;
     n = keep_from(max(thr, 1u), all, l);
   }
   if (n > kKeptMost) {      // ties
-    ties = found;
+    const int all = n;
     n = keep_from(thr + 1u, n, l);
+    ties += static_cast<unsigned int>(all - n);
   }
   // four threads a token compare it with all
   const int quarter = tid & 3;
@@ -1119,8 +1347,8 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(const Sam
   }
   if (ties > 0u) {
     __syncthreads();   // the list is done with
-    masses_of_row(a, row, thr, l);
-    pick_token(a, row, thr, l.masses, l.pick);
+    masses_of_row(a, w, thr, l);
+    pick_token(a, row, u, thr, l.masses, w, l.pick);
     return;
   }
   const float per_chunk = 1.0f / static_cast<float>(a.chunk_len);
@@ -1266,11 +1494,14 @@ extern "C" int arle_sample_finish_most() { return kFinishTopK; }
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
 // arle_sample_scratch_bytes(rows, vocab) bytes, 16-byte aligned.  use_top_k / use_top_p == 0 promise that no row of the call has
 // the filter switched on (top_k in 1..vocab-1, top_p < 1); its passes are then left out.  small_k != 0 promises that every row is
-// greedy or has a top_k of 1 to arle_sample_finish_most(), below vocab.
+// greedy or has a top_k of 1 to arle_sample_finish_most(), below vocab: with vocab up to 2^28 two kernels then do all, probs may be
+// null, and with on_host != 0 temperature is a host array [5][rows] of the temperatures, top_p, min_p, u and the bits of top_k of up to
+// arle_sample_host_rows() rows (the other four pointers are not looked at), which travel with the launch.
+extern "C" int arle_sample_host_rows() { return kInlineRows; }
 extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float* probs,
                                 const float* temperature, const int* top_k, const float* top_p,
                                 const float* min_p, const float* u, int* out, void* scratch, int use_top_k,
-                                int use_top_p, int small_k, void* stream) {
+                                int use_top_p, int small_k, int on_host, void* stream) {
   if (rows == 0) return 0;
   if (scratch == nullptr || reinterpret_cast<uintptr_t>(scratch) % 16 != 0 || rows > 65535)
     return static_cast<int>(hipErrorInvalidValue);
@@ -1306,18 +1537,27 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.use_top_p = use_top_p;
   a.out = out;
   const dim3 grid(a.chunks, rows);
-  const bool finish = small_k && use_top_k && vocab <= kFinishVocab;
-  // the histograms start at zero: those of the filters that are on, of the finishing kernel's rows the first one
-  const int k_row = kRowBins * sizeof(unsigned int) / 16, p_row = kRowBins * sizeof(unsigned long long) / 16;
-  const ClearRows clear{reinterpret_cast<uint4*>(a.hist_k), reinterpret_cast<uint4*>(a.hist_p),
-                        finish ? static_cast<int>(kBins0 * sizeof(unsigned int) / 16) : (use_top_k ? k_row : 0), k_row,
-                        !finish && use_top_p ? p_row : 0, p_row};
-  argmax_chunks_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, part_max, clear);
-  sample_exp_kernel<<<grid, kSelThreads, 0, s>>>(a);
-  if (finish) {
-    sample_finish_kernel<<<rows, kFinishThreads, 0, s>>>(a);
+  if (small_k && use_top_k && vocab <= kFinishVocab) {
+    if (on_host && rows > kInlineRows) return static_cast<int>(hipErrorInvalidValue);
+    group_max_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, a.groups, a.group_max);
+    if (on_host) {
+      InlineRows values;
+      float* const to[4] = {values.temperature, values.top_p, values.min_p, values.u};
+      for (int i = 0; i < 4; ++i) std::memcpy(to[i], temperature + static_cast<size_t>(i) * rows, rows * sizeof(float));
+      std::memcpy(values.top_k, temperature + static_cast<size_t>(4) * rows, rows * sizeof(int));
+      sample_finish_kernel<InlineRows><<<rows, kFinishThreads, 0, s>>>(a, values);
+    } else {
+      sample_finish_kernel<NoRows><<<rows, kFinishThreads, 0, s>>>(a, NoRows{});
+    }
     return launch_status();
   }
+  if (on_host || probs == nullptr) return static_cast<int>(hipErrorInvalidValue);
+  // the histograms of the filters that are on start at zero
+  const int k_row = kRowBins * sizeof(unsigned int) / 16, p_row = kRowBins * sizeof(unsigned long long) / 16;
+  const ClearRows clear{reinterpret_cast<uint4*>(a.hist_k), reinterpret_cast<uint4*>(a.hist_p), use_top_k ? k_row : 0, k_row,
+                        use_top_p ? p_row : 0, p_row};
+  argmax_chunks_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, part_max, clear);
+  sample_exp_kernel<<<grid, kSelThreads, 0, s>>>(a);
   if (use_top_k || use_top_p) {
     sample_pass_kernel<kFirst><<<grid, kSelThreads, 0, s>>>(a);
     sample_pass_kernel<kSecond><<<grid, kSelThreads, 0, s>>>(a);

@@ -14,6 +14,7 @@ import itertools
 import math
 import os
 
+import numpy as np
 import torch
 
 from . import lib
@@ -673,27 +674,45 @@ def sample_small_k() -> int:
     return int(lib.function("arle_sample_finish_most")())
 
 
-def sample_rows(logits, temperature, top_k, top_p, min_p, u, *, use_top_k: bool = True,
+@functools.lru_cache(maxsize=None)
+def sample_host_rows() -> int:
+    """Up to how many rows sample_rows with small_k takes its parameters from host memory."""
+    return int(lib.function("arle_sample_host_rows")())
+
+
+SAMPLE_FINISH_VOCAB = 1 << 28    # up to here small_k holds
+
+
+def sample_rows(logits, temperature, top_k=None, top_p=None, min_p=None, u=None, *, use_top_k: bool = True,
                 use_top_p: bool = True, small_k: bool = False) -> torch.Tensor:
     """One token id per row; per-row float32 temperature/top_p/min_p/u and int32 top_k.
 
     use_top_k / use_top_p = False promise that no row has that filter switched on (top_k in 1..vocab-1,
     top_p < 1): the passes over the row that look for its threshold are then not launched.  small_k promises that every
-    row is greedy or has a top_k of 1 to `sample_small_k()`, below vocab: one kernel then does what follows the first histogram.
+    row is greedy or has a top_k of 1 to `sample_small_k()`, below vocab: one kernel behind the rows' maxima then does all, and
+    the parameters of up to `sample_host_rows()` rows may come as one numpy array in the place of `temperature`, float32 [5, rows] of
+    temperature, top_p, min_p, u and the bits of top_k, which travels with its launch.
     """
     rows, vocab = _logits(logits)
-    for name, t, dt in (("temperature", temperature, torch.float32), ("top_k", top_k, torch.int32),
-                        ("top_p", top_p, torch.float32), ("min_p", min_p, torch.float32),
-                        ("u", u, torch.float32)):
-        _gpu(t)
-        _need(t.dtype == dt and t.shape == (rows,) and t.is_contiguous(), f"{name} must be {dt} [rows]")
-    probs = torch.empty((rows, vocab), dtype=torch.float32, device=logits.device)
+    finish = small_k and use_top_k and vocab <= SAMPLE_FINISH_VOCAB
+    on_host = isinstance(temperature, np.ndarray)
+    if on_host:
+        _need(finish and rows <= sample_host_rows(), f"parameters in host memory need small_k and at most {sample_host_rows()} rows")
+        _need(temperature.dtype == np.float32 and temperature.shape == (5, rows) and temperature.flags.c_contiguous,
+              "parameters in host memory must be float32 [5, rows]")
+        params = (temperature.ctypes.data, None, None, None, None)
+    else:
+        for name, t, dt in (("temperature", temperature, torch.float32), ("top_k", top_k, torch.int32),
+                            ("top_p", top_p, torch.float32), ("min_p", min_p, torch.float32),
+                            ("u", u, torch.float32)):
+            _gpu(t)
+            _need(t.dtype == dt and t.shape == (rows,) and t.is_contiguous(), f"{name} must be {dt} [rows]")
+        params = [t.data_ptr() for t in (temperature, top_k, top_p, min_p, u)]
+    probs = None if finish else torch.empty((rows, vocab), dtype=torch.float32, device=logits.device)
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
     scratch = torch.empty((-(-_sample_scratch_bytes(rows, vocab) // 8),), dtype=torch.int64, device=logits.device)
-    lib.call("arle_sample_rows", logits.data_ptr(), rows, vocab, probs.data_ptr(),
-             temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), min_p.data_ptr(),
-             u.data_ptr(), out.data_ptr(), scratch.data_ptr(), int(bool(use_top_k)), int(bool(use_top_p)),
-             int(bool(small_k)), _stream())
+    lib.call("arle_sample_rows", logits.data_ptr(), rows, vocab, _ptr(probs), *params, out.data_ptr(), scratch.data_ptr(),
+             int(bool(use_top_k)), int(bool(use_top_p)), int(bool(small_k)), int(on_host), _stream())
     return out
 
 

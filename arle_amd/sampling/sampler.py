@@ -125,8 +125,8 @@ class Sampler:
         """As sample_with_logprobs, but nothing is read back: the kernels are queued and the result stays on the GPU."""
         if logits.shape[0] != len(rows):
             raise ValueError("one sampling row per row of logits is needed")
-        # the parameters that differ, which every rule below asks alone: one where the requests share an object (64 rows 68 us a
-        # call), else as many as there are objects, equal ones too (90 us)
+        # the parameters that differ, which every rule below asks alone: one where the requests share an object (64 rows with a
+        # small top_k 40 us a call), else as many as there are objects, equal ones too (58 us)
         kinds = list({id(p): p for p, _, _, _ in rows}.values())
         if any(p.has_penalties() for p in kinds) and any(p.has_penalties() and gen for p, _, _, gen in rows):
             logits = logits.clone()
@@ -139,20 +139,23 @@ class Sampler:
     def _choose(self, logits: torch.Tensor, rows, kinds) -> torch.Tensor:
         if all(p.is_greedy() for p in kinds):
             return ops.argmax_rows(logits)
-        # one host->device copy for the five per-row arrays (top_k travels as the bits of an int32)
         n, vocab, small = len(rows), logits.shape[1], ops.sample_small_k()
-        packed = np.empty((5, n), dtype=np.float32)
         params, seeds, indices, _ = zip(*rows)
-        column = lambda name: getattr(kinds[0], name) if len(kinds) == 1 else [getattr(p, name) for p in params]
-        packed[0] = column("temperature")
-        packed[1] = column("top_p")
-        packed[2] = column("min_p")
+        packed = np.empty((5, n), dtype=np.float32)       # top_k as the bits of an int32
+        if len(kinds) == 1:
+            p = kinds[0]
+            packed[:3] = [[p.temperature], [p.top_p], [p.min_p]]
+            packed.view(np.int32)[4] = p.top_k
+        else:
+            packed[:3] = [[p.temperature for p in params], [p.top_p for p in params], [p.min_p for p in params]]
+            packed.view(np.int32)[4] = [p.top_k for p in params]
         packed[3] = uniforms(seeds, indices)
-        packed[4].view(np.int32)[:] = column("top_k")
-        dev = upload(packed, self.device)      # queued: the host does not wait for the step that made the logits
-        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3],
-                               use_top_k=any(0 < p.top_k < vocab for p in kinds), use_top_p=any(p.top_p < 1.0 for p in kinds),
-                               small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in kinds))
+        promises = dict(use_top_k=any(0 < p.top_k < vocab for p in kinds), use_top_p=any(p.top_p < 1.0 for p in kinds),
+                        small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in kinds))
+        if promises["small_k"] and n <= ops.sample_host_rows() and vocab <= ops.SAMPLE_FINISH_VOCAB:
+            return ops.sample_rows(logits, packed, **promises)     # they travel with the launch
+        dev = upload(packed, self.device)      # one copy, queued: the host does not wait for the step that made the logits
+        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3], **promises)
 
     def _penalise(self, logits, rows) -> None:
         indptr, toks, counts = [0], [], []

@@ -532,6 +532,10 @@ struct CapArgs {
   float out_scale;    // a factor on the output, in 32 bits
 };
 
+}  // namespace arle
+#include "attention_softcap_portions.h"
+namespace arle {
+
 // KC: chunks of 32 of the key size held (Dk <= 32 KC); VC: chunks of 16 of the value size (Dv <= 16 VC).
 // HEADS: a work item is one row (a segment of one row) and the q heads of a kv head, and the WAVES waves of the
 // workgroup take its tiles of keys in turn and add their sums through LDS; else an item is 16 QB rows of one q head,
@@ -543,7 +547,8 @@ struct CapArgs {
 // fetched while this one's probabilities are made and values while its scores are, masks are worked out in the tiles at
 // the ends only, sums are rescaled only where a maximum moved, and the lanes' sums meet once at the end.  A layer of 2,048
 // rows, 32 q heads and 8 kv heads of 128, window 1,024: 173 us before, 89 now (184 and 110 between the other kernels of a
-// prompt; the masks that each block of sixteen rows has of its own are 4 and 8 of these); 256 rows 25 -> 16; eight decoded
+// prompt; the masks that each block of sixteen rows has of its own are 4 and 8 of these; at heads of 128 most of these now go to
+// the kernel of attention_softcap_portions.h); 256 rows 25 -> 16; eight decoded
 // rows behind 2,048 keys 21 -> 17.  (Portions of heads up to 128 are held to the registers of two waves a SIMD.)
 template <int KC, int VC, bool HEADS, int WAVES, int QB>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(!HEADS && KC <= 4 && VC <= 8 ? 2 : 1)))
@@ -904,6 +909,11 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
 // and 45 us; 1,024 rows, 1,056 waves, 62 and 64; 1,150 rows 72 and 73; 1,250 rows 81 and 74; four portions of 300 rows 33
 // and 32; 2,048 rows 136 and 89).
 constexpr long long kCapTwoBlocks = 1024;
+// Workgroups of 128 rows (tokens times the q heads of a kv head) from which on heads of 128 go to the kernel whose waves share
+// their tiles (attention_softcap_portions.h): with fewer, one-wave items spread over more of the chip.  32 q heads over 8 kv heads,
+// window 1,024, cap and penalty, this kernel / that one, us: 100 rows 11.5 / 13.1, 400 rows (112 of them) 22.7 / 23.2, 512 behind 3,000
+// (136) 52.1 / 53.9, 300 beside eight decoded rows (144) 50 / 43, 640 (168) 36.9 / 31.0, 1,024 72 / 44, 2,048 110 / 66, 4,096 195 / 120.
+constexpr long long kCapPortions = 144;
 constexpr int kCapSplitWaves = 8;   // waves that share the keys of a decoded row
 constexpr int kCapLdsMost = 160 * 1024;   // LDS of a gfx950 compute unit: no workgroup can ask for more
 
@@ -962,6 +972,12 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
   const int wide_blocks = (row_blocks - segments) / 2 + segments;   // as row_blocks, of 32 rows
   const bool two = Dk <= 128 && Dv <= 128 && static_cast<long long>(wide_blocks) * nq >= kCapTwoBlocks &&
                    page_bytes + 2 * sizeof(int) <= 48 * 1024;
+  const int tokens_most = 16 * (row_blocks - segments) + 15;      // what row_blocks was counted from
+  const int blocks = tokens_most * group / kCpRows + segments;   // no fewer than the blocks of kCpRows rows of all segments
+  if (!heads_mode && cap_portions_take(a) && static_cast<long long>(blocks) * nkv >= kCapPortions) {
+    if (r1 == nullptr) return launch_cap_portions<0>(a, blocks, s);
+    return group == kCpTableGroup && window > 0 && window <= kCpTableMax ? launch_cap_portions<1>(a, blocks, s) : launch_cap_portions<2>(a, blocks, s);
+  }
 #define ARLE_CAP_ROWS(KC, VC, QB, BLOCKS, BYTES)                                                                   \
   do {                                                                                                             \
     constexpr int kQb = KC <= 4 && VC <= 8 ? QB : 1;                                                               \

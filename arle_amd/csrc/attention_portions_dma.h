@@ -218,17 +218,11 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
   // what a lane fetches for a tile never changes but for the page: four pieces of keys and four of values
   //   keys:   LDS piece q = 64 (4 wave + jj) + lane -> key q / 16 of the tile, position q % 16 in its row
   //   values: LDS piece q                           -> d row q / 8,            position q % 8
-  int k_key[4], k_src[4], v_key[4], v_src[4];
-#pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const int q = 64 * (4 * wave + jj) + lane;
-    const int key = q / 16, pos = q % 16;
-    k_key[jj] = key;
-    k_src[jj] = 8 * (pos ^ (key & 15));              // element offset of the piece inside its key row
-    const int d = q / 8, vpos = q % 8;
-    v_key[jj] = 8 * (vpos ^ ((d >> 1) & 7));               // first of the piece's eight keys, inside the tile
-    v_src[jj] = d * P;                                // element offset of the d row inside a page
-  }
+  const int k_lane = (lane >> 4) * D + 8 * ((lane & 15) ^ (lane >> 4));   // element of the piece among four keys (jj 0)
+  const int v_lane = 8 * ((lane & 7) ^ (lane >> 4));                      // first of the piece's eight keys, inside the tile (even jj)
+  auto k_src = [&](int jj) { return k_lane ^ (32 * jj); };
+  auto v_key = [&](int jj) { return v_lane ^ (32 * (jj & 1)); };
+  auto v_src = [&](int jj) { return (32 * wave + 8 * jj + (lane >> 3)) * P; };   // element offset of the d row inside a page
   auto fetch = [&](int tile, int stage) {
     const int base = tile * kDmKeys;
     unsigned char* at = lds_raw + stage * kDmStageBytes + (4 * wave) * 1024;
@@ -236,42 +230,45 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
       // keys of the tile that lie outside the request are read as they are (the page is there) and masked
       const int page = __builtin_amdgcn_readlane(pg_reg, __builtin_amdgcn_readfirstlane((base >> ps) - pg_base));
       const uint64_t first = static_cast<uint64_t>(static_cast<uint32_t>(page)) * page_elems32 + head_off32;
-      const uint16_t* kb = a.k_pages + first + static_cast<uint32_t>(base & pm) * D;
+      const uint16_t* kb = a.k_pages + first + static_cast<uint32_t>((base & pm) + 16 * wave) * D;
       const uint16_t* vb = a.v_pages + first + static_cast<uint32_t>(base & pm);
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-        load_to_lds_16(kb, 2u * static_cast<uint32_t>(k_key[jj] * D + k_src[jj]), at + jj * 1024);
+      for (int jj = 0; jj < 4; ++jj) load_to_lds_16(kb, 2u * static_cast<uint32_t>(k_src(jj) + 4 * jj * D), at + jj * 1024);
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj)
-        load_to_lds_16(vb, 2u * static_cast<uint32_t>(v_src[jj] + v_key[jj]), at + kDmKeys * D * 2 + jj * 1024);
+        load_to_lds_16(vb, 2u * static_cast<uint32_t>(v_src(jj) + v_key(jj)), at + kDmKeys * D * 2 + jj * 1024);
       return;
     }
-    // Keys: one load takes four keys in a row, which lie in one page (a page holds eight at least), so the page
-    // is the wave's and the address scalar arithmetic as above; keys outside the request are read from the
+    // Keys: a wave takes sixteen in a row, and eight of them lie in one page (a page holds eight at least), so two pages
+    // are the wave's and the addresses scalar arithmetic as above; keys outside the request are read from the
     // nearest page that is there and masked.  Values: a lane's piece holds eight keys of its own, so a lane
-    // looks up its own page: the four page ids first (lane exchanges that answer together), then the loads.
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    int v_at[4], v_page[4];
+    // looks up its own pages: the two page ids first (lane exchanges that answer together), then the loads.  (A lookup and an
+    // address for each of the eight loads were a tenth of a wave's instructions: a fresh prompt of 8,192 tokens 610 us, of
+    // 4,096 179, 512 tokens behind 3,584 cached 61; now 581, 168 and 56.)
+    int v_at[2], v_page[2];
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      v_at[jj] = min(max(base + v_key[jj], kv_lo & ~7), (kv_hi - 1) & ~7);
-      v_page[jj] = __shfl(pg_reg, (v_at[jj] >> ps) - pg_base, kWave);
+    for (int i = 0; i < 2; ++i) {
+      v_at[i] = min(max(base + v_key(i), kv_lo & ~7), (kv_hi - 1) & ~7);
+      v_page[i] = __shfl(pg_reg, (v_at[i] >> ps) - pg_base, kWave);
     }
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int first_key = base + 4 * (4 * wave_u + jj);
+    for (int i = 0; i < 2; ++i) {
+      const int first_key = base + 16 * wave + 8 * i;
       const int page_at = min(max(first_key >> ps, kv_lo >> ps), pg_last) - pg_base;
       const int page = __builtin_amdgcn_readlane(pg_reg, __builtin_amdgcn_readfirstlane(page_at));
       const uint16_t* kb = a.k_pages + static_cast<uint64_t>(static_cast<uint32_t>(page)) * page_elems32 + head_off32 +
                            static_cast<uint32_t>(first_key & pm) * D;
-      load_to_lds_16(kb, 2u * static_cast<uint32_t>((lane >> 4) * D + k_src[jj]), at + jj * 1024);
-    }
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const uint16_t* src = a.v_pages + static_cast<uint64_t>(static_cast<uint32_t>(v_page[jj])) * page_elems32 +
-                            (head_off32 + v_src[jj] + static_cast<uint32_t>(v_at[jj] & pm));
-      load_to_lds_16(src, at + kDmKeys * D * 2 + jj * 1024);
+      for (int jj = 2 * i; jj < 2 * i + 2; ++jj)
+        load_to_lds_16(kb, 2u * static_cast<uint32_t>(k_src(jj) + 4 * (jj & 1) * D), at + jj * 1024);
     }
+    const uint16_t* vb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      vb[i] = a.v_pages + static_cast<uint64_t>(static_cast<uint32_t>(v_page[i])) * page_elems32 +
+              (head_off32 + v_src(i) + static_cast<uint32_t>(v_at[i] & pm));
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) load_to_lds_16(vb[jj & 1] + (jj & 2) * 8 * P, at + kDmKeys * D * 2 + jj * 1024);
   };
   // Slots past the request's last token may hold anything, also NaN, and 0 * NaN is NaN: in the request's last
   // tile every lane puts the values of such keys to zero in the pieces that it fetched itself.
@@ -281,7 +278,7 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
     unsigned char* at = lds_raw + stage * kDmStageBytes + kDmKeys * D * 2 + (4 * wave) * 1024 + lane * 16;
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj) {
-      const int key8 = WHOLE ? base + v_key[jj] : min(max(base + v_key[jj], kv_lo & ~7), (kv_hi - 1) & ~7);  // as fetched
+      const int key8 = WHOLE ? base + v_key(jj) : min(max(base + v_key(jj), kv_lo & ~7), (kv_hi - 1) & ~7);  // as fetched
       if (key8 + 8 > kv_total) {
         u32x4 v = *reinterpret_cast<u32x4*>(at + jj * 1024);
 #pragma unroll

@@ -183,17 +183,20 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(TIn* __restri
 
 // A stack of float32 deltas (the partial products of a matrix product whose K was split over
 // workgroups) added into the residual row, then the norm.  Few rows make few workgroups here, so the
-// time is the latency of the loads: a workgroup of 1024 threads owns a row, every thread one group of
-// four columns, and the loads of the whole stack (up to kStackUnroll at a time) are in flight together.
-// Order of addition: residual + (delta 0 + delta 1 + ...), as in the kernels above.
+// time is the latency of the loads: a workgroup owns a row, every thread one group of four columns (THREADS: the waves that the
+// width takes, up to 1,024 threads), and the loads of the whole stack, UNROLL parts at a time, are in flight together: four for
+// stacks of up to four, else eight (six parts as a round of four and one behind it were two trips to memory, and 1,024
+// threads for 2,560 columns six idle waves to start: whole decode steps of the Qwen3-4B shape 2,461 -> 2,436 us with one request,
+// 2,985 -> 2,956 with 19).
+// Order of addition: residual + (delta 0 + delta 1 + ...), as in the kernels above; idle waves would add zeros to the
+// sum of squares, so the threads do not change a bit.
 constexpr int kStackThreads = 1024;
-constexpr int kStackUnroll = 4;   // parts of the stack that a thread has in flight at a time
 
-template <typename TOut, typename TW>
-__global__ __launch_bounds__(kStackThreads) void add_stack_rmsnorm_kernel(
+template <typename TOut, typename TW, int THREADS, int UNROLL>
+__global__ __launch_bounds__(THREADS) void add_stack_rmsnorm_kernel(
     float* __restrict__ residual, const float* __restrict__ delta, int n_delta, int64_t delta_stride,
     const TW* __restrict__ w, TOut* __restrict__ out, const int* __restrict__ rows, int width, float eps) {
-  __shared__ float lds[kStackThreads / kWave];
+  __shared__ float lds[THREADS / kWave];
   const int r = blockIdx.x;
   const int64_t src = rows ? rows[r] : r;
   const int i = 4 * threadIdx.x;
@@ -204,29 +207,15 @@ __global__ __launch_bounds__(kStackThreads) void add_stack_rmsnorm_kernel(
   float4 v = load4<float>(res + ic), d = {0.f, 0.f, 0.f, 0.f};
   const float4 wv = load4<TW>(w + ic);
   // The loads of a round carry no condition (a load under a condition is waited for before the next one is
-  // issued, and the parts would arrive one after the other): whole rounds of four parts first, then one round
-  // whose loads past the last part fetch the last part again and are not added.  Threads past the width read
-  // column 0.
+  // issued, and the parts would arrive one after the other): those past the last part fetch the last part again and are
+  // not added.  Threads past the width read column 0.
   const float* dc = dr + ic;
-  int base = 0;
-  for (; base + kStackUnroll <= n_delta; base += kStackUnroll) {
-    float4 e[kStackUnroll];
+  for (int base = 0; base < n_delta; base += UNROLL) {
+    float4 e[UNROLL];
 #pragma unroll
-    for (int u = 0; u < kStackUnroll; ++u) e[u] = load4<float>(dc + (base + u) * delta_stride);
+    for (int u = 0; u < UNROLL; ++u) e[u] = load4<float>(dc + min(base + u, n_delta - 1) * delta_stride);
 #pragma unroll
-    for (int u = 0; u < kStackUnroll; ++u) {
-      d.x += e[u].x;
-      d.y += e[u].y;
-      d.z += e[u].z;
-      d.w += e[u].w;
-    }
-  }
-  if (base < n_delta) {
-    float4 e[kStackUnroll - 1];
-#pragma unroll
-    for (int u = 0; u < kStackUnroll - 1; ++u) e[u] = load4<float>(dc + min(base + u, n_delta - 1) * delta_stride);
-#pragma unroll
-    for (int u = 0; u < kStackUnroll - 1; ++u) {
+    for (int u = 0; u < UNROLL; ++u) {
       const bool in = base + u < n_delta;
       d.x += in ? e[u].x : 0.f;
       d.y += in ? e[u].y : 0.f;
@@ -240,7 +229,7 @@ __global__ __launch_bounds__(kStackThreads) void add_stack_rmsnorm_kernel(
   v.w += d.w;
   if (mine && !rows) store4<float>(res + i, v);
   const float total =
-      block_sum<kStackThreads / kWave>(mine ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f, lds);
+      block_sum<THREADS / kWave>(mine ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f, lds);
   const float inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
   if (mine)
     store4<TOut>(out + static_cast<int64_t>(r) * width + i,
@@ -283,14 +272,23 @@ int launch_add_rmsnorm(float* residual, const void* delta, int n_delta, long lon
   if constexpr (sizeof(TD) == 4) {
     if (n_delta > 1 && vec_ok(width, width, residual, delta, w, out) && delta_stride % 4 == 0 &&
         width <= 4 * kStackThreads) {
-      if (w_dtype == kF32)
-        add_stack_rmsnorm_kernel<TOut, float><<<n_rows, kStackThreads, 0, s>>>(
-            residual, static_cast<const float*>(delta), n_delta, delta_stride, static_cast<const float*>(w),
-            static_cast<TOut*>(out), rows, width, eps);
-      else
-        add_stack_rmsnorm_kernel<TOut, bf16><<<n_rows, kStackThreads, 0, s>>>(
-            residual, static_cast<const float*>(delta), n_delta, delta_stride, static_cast<const bf16*>(w),
-            static_cast<TOut*>(out), rows, width, eps);
+#define ARLE_STACK(TW, THREADS, UNROLL)                                                                             \
+  add_stack_rmsnorm_kernel<TOut, TW, THREADS, UNROLL><<<n_rows, THREADS, 0, s>>>(                                   \
+      residual, static_cast<const float*>(delta), n_delta, delta_stride, static_cast<const TW*>(w),                  \
+      static_cast<TOut*>(out), rows, width, eps)
+#define ARLE_STACK_WIDTH(TW, UNROLL)                                                                                \
+  do {                                                                                                              \
+    if (width <= 4 * 320) ARLE_STACK(TW, 320, UNROLL);                                                              \
+    else if (width <= 4 * 640) ARLE_STACK(TW, 640, UNROLL);                                                         \
+    else ARLE_STACK(TW, kStackThreads, UNROLL);                                                                     \
+  } while (0)
+      if (w_dtype == kF32) {
+        if (n_delta <= 4) ARLE_STACK_WIDTH(float, 4); else ARLE_STACK_WIDTH(float, 8);
+      } else {
+        if (n_delta <= 4) ARLE_STACK_WIDTH(bf16, 4); else ARLE_STACK_WIDTH(bf16, 8);
+      }
+#undef ARLE_STACK_WIDTH
+#undef ARLE_STACK
       return launch_status();
     }
   }

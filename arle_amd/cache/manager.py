@@ -262,6 +262,12 @@ class CacheManager:
                 if isinstance(need, StateNeed):
                     self.state_buffers[entry] = torch.zeros((max_slots, *need.shape),
                                                             dtype=need.dtype or dtype, device=device)
+        # A slot is zeroed by a launch for each element type: a launch for each buffer was 24 of 5 us
+        # for an admitted request of a model of eight layers with three states each.
+        by_type = {}
+        for buf in self.state_buffers.values():
+            by_type.setdefault(buf.dtype, []).append(buf)
+        self._state_by_type = list(by_type.values())
 
     @staticmethod
     def _leaf_key(entry: int, path: tuple):
@@ -279,8 +285,8 @@ class CacheManager:
         self._lengths[key] = 0
         for group in self.groups:
             group.open(key)
-        for buf in self.state_buffers.values():
-            buf[slot].zero_()
+        for bufs in self._state_by_type:
+            torch._foreach_zero_([buf[slot] for buf in bufs])
         return slot
 
     def release(self, key) -> None:

@@ -88,12 +88,22 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_kernel(
 
 // The same for the usual types: terms that are float32 (a projection's 32-bit output or its stack of partial
 // products), biases, weights and outputs of one type TA, a width that is a multiple of 4.  Four elements a lane and
-// access, every load of a row issued without a condition on data, before anything is stored.
+// access, every load of a row issued without a condition on data, before anything is stored.  Bound by the latency of that one trip to
+// memory and of two reductions for few rows, by the memory for many (2,048 rows of 2,560, terms of one and two parts: 5.9 TB/s).
 //
 // CT > 0: the rows are single ones of different requests, and the first norm's output goes through a causal convolution of CT taps
 // with its input added before it is written (LnConv): a lane holds the same four channels of the row, of the taps and of the
 // request's state, which it moves on, and everything it needs is on its way before the reductions.  One kernel less to
 // wait for in front of every layer; decode steps of 8 rows of 2,560, MI355X: norm 4.8 + convolution 4.4 us before.
+// Four consecutive elements as they are stored: widened where they are used, as a conversion waits for its load.
+template <typename T>
+using Raw4 = std::conditional_t<std::is_same<T, float>::value, float4, uint2>;
+
+template <typename T>
+__device__ __forceinline__ Raw4<T> ld_raw(const T* p) { return *reinterpret_cast<const Raw4<T>*>(p); }
+template <typename T>
+__device__ __forceinline__ float4 widen(const Raw4<T>& v) { return ld4<T>(reinterpret_cast<const T*>(&v)); }
+
 template <typename TA>
 struct LnConv {
   const TA* w;         // [width, CT]
@@ -101,13 +111,13 @@ struct LnConv {
   const int* slot;     // of every row
 };
 
-template <typename TA, int NT, int PER4, int CT>
+template <typename TA, int NT, int PER4, int CT, int U>
 __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     float* __restrict__ residual, const float* __restrict__ t0, int n0, long long s0, const TA* __restrict__ b0,
     const float* __restrict__ t1, int n1, long long s1, const TA* __restrict__ b1, const TA* __restrict__ wa,
     const TA* __restrict__ wb, TA* __restrict__ out_a, TA* __restrict__ out_b, const int* __restrict__ rows, int width,
     float eps, const TA* __restrict__ ca, const TA* __restrict__ cb, const LnConv<TA> conv) {
-  __shared__ float lds[(NT / kWave)];
+  __shared__ float lds[2][(NT / kWave)];
   const int r = blockIdx.x;
   const int64_t src = rows ? rows[r] : r;
   const int64_t base = src * width;
@@ -115,7 +125,46 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
   float4 x[PER4];
 #pragma unroll
   for (int k = 0; k < PER4; ++k) x[k] = ld4<float>(residual + base + min((tid + k * NT) * 4, last));
-  auto add_term = [&](const float* t, int n, long long stride, const TA* bias) {
+  // U > 0: both terms have at most U parts, and all that there are are on their way with the row (a condition that is the same for
+  // the whole workgroup is a jump and waits for no load, as long as nothing is made of the value in front of its use)
+  [[maybe_unused]] float4 e0[U > 0 ? U : 1][PER4], e1[U > 0 ? U : 1][PER4];
+  if constexpr (U > 0) {
+    const float *p0 = t0 + base, *p1 = t1 + base;
+    const int last0 = t0 ? n0 - 1 : -1, last1 = t1 ? n1 - 1 : -1;
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+      if (j <= last0)
+#pragma unroll
+        for (int k = 0; k < PER4; ++k) e0[j][k] = ld4<float>(p0 + j * s0 + min((tid + k * NT) * 4, last));
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+      if (j <= last1)
+#pragma unroll
+        for (int k = 0; k < PER4; ++k) e1[j][k] = ld4<float>(p1 + j * s1 + min((tid + k * NT) * 4, last));
+  }
+  [[maybe_unused]] Raw4<TA> bias0[PER4], bias1[PER4];
+  if constexpr (U > 0) {
+#pragma unroll
+    for (int k = 0; k < PER4; ++k) {
+      if (t0 && b0) bias0[k] = ld_raw<TA>(b0 + min((tid + k * NT) * 4, last));
+      if (t1 && b1) bias1[k] = ld_raw<TA>(b1 + min((tid + k * NT) * 4, last));
+    }
+  }
+  [[maybe_unused]] auto add_fetched = [&](const auto& e, int n, const Raw4<TA> (&bias)[PER4], bool biased) {
+#pragma unroll
+    for (int k = 0; k < PER4; ++k) {
+      float4 d = e[0][k];
+#pragma unroll
+      for (int j = 1; j < U; ++j)
+        if (j < n) d.x += e[j][k].x, d.y += e[j][k].y, d.z += e[j][k].z, d.w += e[j][k].w;
+      if (biased) {
+        const float4 b = widen<TA>(bias[k]);
+        d.x += b.x; d.y += b.y; d.z += b.z; d.w += b.w;
+      }
+      x[k].x += d.x; x[k].y += d.y; x[k].z += d.z; x[k].w += d.w;
+    }
+  };
+  [[maybe_unused]] auto add_term = [&](const float* t, int n, long long stride, const TA* bias) {
     float4 d[PER4];
 #pragma unroll
     for (int k = 0; k < PER4; ++k) d[k] = ld4<float>(t + base + min((tid + k * NT) * 4, last));
@@ -153,19 +202,15 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     }
   };
   // the norm weights are fetched now, not behind the two reductions that their use waits for
-  float4 w_a[PER4], w_b[PER4], c_a[PER4], c_b[PER4];
+  const TA* weights[4] = {wa, wb, ca, cb};
+  Raw4<TA> w_raw[4][PER4];
 #pragma unroll
-  for (int k = 0; k < PER4; ++k) {
-    w_a[k] = ld4<TA>(wa + min((tid + k * NT) * 4, last));
-    w_b[k] = ld4<TA>((wb ? wb : wa) + min((tid + k * NT) * 4, last));
-    // (a bias that is absent is the weight again, fetched and dropped)
-    c_a[k] = ld4<TA>((ca ? ca : wa) + min((tid + k * NT) * 4, last));
-    c_b[k] = ld4<TA>((cb ? cb : wa) + min((tid + k * NT) * 4, last));
-    if (!ca) c_a[k] = float4{0.f, 0.f, 0.f, 0.f};
-    if (!cb) c_b[k] = float4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int m = 0; m < 4; ++m)
+    if (weights[m])
+#pragma unroll
+      for (int k = 0; k < PER4; ++k) w_raw[m][k] = ld_raw<TA>(weights[m] + min((tid + k * NT) * 4, last));
   constexpr int BACK = CT > 0 ? CT - 1 : 1, TAPS = CT > 0 ? CT : 1;
-  [[maybe_unused]] float4 before[PER4][BACK], tap[PER4][TAPS];   // the rows before this one, oldest first; 4 channels' taps
+  [[maybe_unused]] Raw4<TA> before[PER4][BACK], tap[PER4][TAPS];   // the rows before this one, oldest first; 4 channels' taps
   [[maybe_unused]] TA* mine = nullptr;
   if constexpr (CT > 0) {
     mine = conv.state + static_cast<int64_t>(conv.slot[r]) * (CT - 1) * width;
@@ -173,13 +218,18 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     for (int k = 0; k < PER4; ++k) {
       const int i = min((tid + k * NT) * 4, last);
 #pragma unroll
-      for (int j = 0; j < CT - 1; ++j) before[k][j] = ld4<TA>(mine + static_cast<int64_t>(j) * width + i);
+      for (int j = 0; j < CT - 1; ++j) before[k][j] = ld_raw<TA>(mine + static_cast<int64_t>(j) * width + i);
 #pragma unroll
-      for (int j = 0; j < CT; ++j) tap[k][j] = ld4<TA>(conv.w + static_cast<int64_t>(i) * CT + 4 * j);
+      for (int j = 0; j < CT; ++j) tap[k][j] = ld_raw<TA>(conv.w + static_cast<int64_t>(i) * CT + 4 * j);
     }
   }
-  if (t0) add_term(t0, n0, s0, b0);
-  if (t1) add_term(t1, n1, s1, b1);
+  if constexpr (U > 0) {
+    if (t0) add_fetched(e0, n0, bias0, b0);
+    if (t1) add_fetched(e1, n1, bias1, b1);
+  } else {
+    if (t0) add_term(t0, n0, s0, b0);
+    if (t1) add_term(t1, n1, s1, b1);
+  }
   float sum = 0.f;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
@@ -189,7 +239,16 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
       sum += (x[k].x + x[k].y) + (x[k].z + x[k].w);
     }
   }
-  const float mu = block_sum<(NT / kWave)>(sum, lds) / static_cast<float>(width);
+  auto row_sum = [&](float v, float* own) {      // block_sum with words of its own: nothing waits behind it for them to be free
+    v = wave_sum(v);
+    if (tid % kWave == 0) own[tid / kWave] = v;
+    __syncthreads();
+    float total = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT / kWave; ++j) total += own[j];
+    return total;
+  };
+  const float mu = row_sum(sum, lds[0]) / static_cast<float>(width);
   float sq = 0.f;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
@@ -197,13 +256,13 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     x[k].x -= mu; x[k].y -= mu; x[k].z -= mu; x[k].w -= mu;
     if (i < width) sq += (x[k].x * x[k].x + x[k].y * x[k].y) + (x[k].z * x[k].z + x[k].w * x[k].w);
   }
-  const float inv = 1.0f / sqrtf(block_sum<(NT / kWave)>(sq, lds) / static_cast<float>(width) + eps);
+  const float inv = 1.0f / sqrtf(row_sum(sq, lds[1]) / static_cast<float>(width) + eps);
   const int64_t o = static_cast<int64_t>(r) * width;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
     const int i = (tid + k * NT) * 4;
     if (i < width) {
-      const float4 w = w_a[k], c = c_a[k];
+      const float4 w = widen<TA>(w_raw[0][k]), c = ca ? widen<TA>(w_raw[2][k]) : float4{0.f, 0.f, 0.f, 0.f};
       float4 a = float4{fmaf(x[k].x * inv, w.x, c.x), fmaf(x[k].y * inv, w.y, c.y), fmaf(x[k].z * inv, w.z, c.z), fmaf(x[k].w * inv, w.w, c.w)};
       if constexpr (CT > 0) {
         // the convolution reads what the norm alone would have written, and adds in the order of conv_step
@@ -211,7 +270,8 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
         float wt[4][TAPS], acc[4];
 #pragma unroll
         for (int j = 0; j < CT; ++j) {
-          const float e[4] = {tap[k][j].x, tap[k][j].y, tap[k][j].z, tap[k][j].w};
+          const float4 taps = widen<TA>(tap[k][j]);
+          const float e[4] = {taps.x, taps.y, taps.z, taps.w};
 #pragma unroll
           for (int q = 0; q < 4; ++q) wt[(4 * j + q) / TAPS][(4 * j + q) % TAPS] = e[q];
         }
@@ -219,18 +279,19 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
         for (int q = 0; q < 4; ++q) acc[q] = fmaf(wt[q][TAPS - 1], now[q], now[q]);
 #pragma unroll
         for (int j = CT - 2; j >= 0; --j) {
-          const float v[4] = {before[k][j].x, before[k][j].y, before[k][j].z, before[k][j].w};
+          const float4 in = widen<TA>(before[k][j]);
+          const float v[4] = {in.x, in.y, in.z, in.w};
 #pragma unroll
           for (int q = 0; q < 4; ++q) acc[q] = fmaf(wt[q][j], v[q], acc[q]);
         }
 #pragma unroll
-        for (int j = 0; j + 1 < CT - 1; ++j) st4<TA>(mine + static_cast<int64_t>(j) * width + i, before[k][j + 1]);
+        for (int j = 0; j + 1 < CT - 1; ++j) *reinterpret_cast<Raw4<TA>*>(mine + static_cast<int64_t>(j) * width + i) = before[k][j + 1];
         st4<TA>(mine + static_cast<int64_t>(CT - 2) * width + i, float4{now[0], now[1], now[2], now[3]});
         a = float4{acc[0], acc[1], acc[2], acc[3]};
       }
       st4<TA>(out_a + o + i, a);
       if (out_b) {
-        const float4 v = w_b[k], e = c_b[k];
+        const float4 v = widen<TA>(w_raw[1][k]), e = cb ? widen<TA>(w_raw[3][k]) : float4{0.f, 0.f, 0.f, 0.f};
         st4<TA>(out_b + o + i, float4{fmaf(x[k].x * inv, v.x, e.x), fmaf(x[k].y * inv, v.y, e.y), fmaf(x[k].z * inv, v.z, e.z),
                                       fmaf(x[k].w * inv, v.w, e.w)});
       }
@@ -242,17 +303,32 @@ template <typename TA>
 static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, const void* wa, const void* wb, void* out_a,
                          void* out_b, const int* rows, int n_rows, int width, float eps, const void* ca, const void* cb,
                          const LnConv<TA>& conv, int taps, hipStream_t s) {
-#define ARLE_LNV_CT(NT, PER4, CT)                                                                                   \
-  add_layernorm_vec_kernel<TA, NT, PER4, CT><<<n_rows, NT, 0, s>>>(                                                  \
+#define ARLE_LNV_U(NT, PER4, CT, U)                                                                                 \
+  add_layernorm_vec_kernel<TA, NT, PER4, CT, U><<<n_rows, NT, 0, s>>>(                                                  \
       residual, static_cast<const float*>(t0.data), t0.n_stack, t0.stack_stride, static_cast<const TA*>(t0.bias),  \
       static_cast<const float*>(t1.data), t1.n_stack, t1.stack_stride, static_cast<const TA*>(t1.bias),            \
       static_cast<const TA*>(wa), static_cast<const TA*>(wb), static_cast<TA*>(out_a), static_cast<TA*>(out_b), rows, \
       width, eps, static_cast<const TA*>(ca), static_cast<const TA*>(cb), conv)
+#define ARLE_LNV_CT(NT, PER4, CT)                                                     \
+  do {                                                                                \
+    constexpr int two = PER4 <= 2 && !(PER4 == 2 && NT > 640 && CT > 0) ? 2 : 0;      \
+    constexpr bool fits = PER4 == 2 && CT == 0 && (NT <= 256 || (NT <= 640 && std::is_same<TA, bf16>::value)); \
+    constexpr int more = PER4 == 1 || fits ? 8 : 0;                                   \
+    if (two && parts <= two) ARLE_LNV_U(NT, PER4, CT, two);                           \
+    else if (more && parts <= more) ARLE_LNV_U(NT, PER4, CT, more);                   \
+    else ARLE_LNV_U(NT, PER4, CT, 0);                                                 \
+  } while (0)
 #define ARLE_LNV(NT, PER4)                                                            \
   do {                                                                                \
     if (taps == 0) ARLE_LNV_CT(NT, PER4, 0); else if (taps == 2) ARLE_LNV_CT(NT, PER4, 2); \
     else if (taps == 3) ARLE_LNV_CT(NT, PER4, 3); else ARLE_LNV_CT(NT, PER4, 4);      \
   } while (0)
+  // How many parts of both terms a lane fetches together: two or eight where the registers hold them, else one term after the other.
+  // MI355X, terms of 4 and 6 parts / 1 and 2 / 1 and 1, us, term after term with the parts past the last fetched again / as here: 8 rows
+  // of 2,560 4.9, 4.1, 3.6 / 4.1, 3.4, 3.3, with the convolution 5.6, 4.7, 4.2 / 4.6, 3.9, 3.9; 2,048 rows - 23.9, 19.7 / - 21.5, 18.8
+  // (126 and 105 MB); 8 rows of 5,120 6.9, 5.3, 4.3 / 5.7, 4.2, 4.1; 2,048 rows - 50.1, 37.0 / - 38.7, 33.2; 512 rows of 8,192 - 20.5, 17.0
+  // / - 18.9, 16.9.  (Eight parts of eight float32 elements a lane spill: 8 rows of 5,120 7.0 / 9.1.)
+  const int parts = max(t0.data ? t0.n_stack : 0, t1.data ? t1.n_stack : 0);
   // Workgroups as wide as the row where that is more than 2,048 elements: nearly every load of a row is then on its way at once
   // and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
   // 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
@@ -279,6 +355,7 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
   }
 #undef ARLE_LNV
 #undef ARLE_LNV_CT
+#undef ARLE_LNV_U
   return launch_status();
 }
 

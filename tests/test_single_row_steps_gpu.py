@@ -117,6 +117,28 @@ def test_layer_norm_at_the_edges_of_its_workgroups(width, rows):
     assert _rel(got, d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * weight.double()) < 1e-5
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [1024, 2048, 2560, 4096, 5120, 8192, 8196])
+def test_parts_of_both_terms_fetched_together(width, dtype):
+    """As many parts as are fetched together, one less and one more, absent terms and biases.  A sum of n + 2 numbers in float32 is off
+    by at most (n + 1) 2^-24 of the sum of their sizes: 1e-6 of the largest here; the outputs as in the tests beside this one."""
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    weight, other, bias, c = (rand(width).to(dtype) for _ in range(4))
+    for parts in ((), (1,), (2,), (3,), (8,), (9,), (1, 1), (1, 2), (2, 1), (2, 2), (2, 3), (8, 1), (4, 6), (8, 8), (9, 1), (1, 9)):
+        residual = rand(3, width) + 3
+        terms = [(rand(n, 3, width), bias if n % 2 else None) for n in parts]
+        want = residual.double() + sum((t.double().sum(0) + (0 if b is None else b.double()) for t, b in terms), torch.zeros_like(residual).double())
+        a, b = ops.add_layernorm(residual, terms, weight, 1e-6, dtype, other, bias_b=c)
+        d = want - want.mean(-1, keepdim=True)
+        d = d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6)
+        assert _rel(residual, want) < 1e-6
+        assert _rel(a, d * weight.double()) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
+        assert _rel(b, d * other.double() + c.double()) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("rows", [2047, 2048])
 @pytest.mark.parametrize("width", [5124, 8192])
 def test_layer_norm_of_many_bfloat16_rows(width, rows):

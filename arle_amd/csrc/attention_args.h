@@ -156,12 +156,12 @@ __device__ __forceinline__ DecodeShare decode_share(const int* seg_start, const 
 }
 
 __device__ __forceinline__ float group_max4(float v) {  // over the 4 lanes i, i+16, i+32, i+48
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  return fmaxf(v, __shfl_xor(v, 32, kWave));
+  const LanePair near = across16(v), far = across32(fmaxf(near.lo, near.hi));
+  return fmaxf(far.lo, far.hi);
 }
 __device__ __forceinline__ float group_sum4(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
+  const LanePair near = across16(v), far = across32(near.lo + near.hi);
+  return far.lo + far.hi;
 }
 
 }  // namespace arle

@@ -364,7 +364,7 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
 #pragma unroll
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, st[t][r]);
     {
-      const HalfPair both = both_halves(bmax);
+      const LanePair both = across32(bmax);
       bmax = fmaxf(both.lo, both.hi) * a.scale_log2;  // scale > 0: the maximum commutes with it
     }
     // m is the point that the row's exponentials are taken from, not its exact maximum: it moves only when
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
         pb[t][u] = __builtin_bit_cast(bf16x8, packed);
       }
     {
-      const HalfPair both = both_halves(psum);
+      const LanePair both = across32(psum);
       psum = both.lo + both.hi;
     }
     l = l * alpha + psum;

@@ -163,8 +163,7 @@ __global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
-#pragma unroll
-    for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+    ss = lanes_sum<LPH>(ss);
     const float f = 1.0f / sqrtf(ss / static_cast<float>(D) + eps) * temp;
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = x[e] * f * w[e];
@@ -754,8 +753,8 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
       float m_new = m_run[b];
 #pragma unroll
       for (int i = 0; i < 8; ++i) m_new = fmaxf(m_new, s[b][i]);
-      m_new = fmaxf(m_new, __shfl_xor(m_new, 16, kWave));
-      m_new = fmaxf(m_new, __shfl_xor(m_new, 32, kWave));
+      const LanePair near = across16(m_new), far = across32(fmaxf(near.lo, near.hi));
+      m_new = fmaxf(far.lo, far.hi);
       // a query whose window begins behind this tile has seen nothing yet: keep its sums at zero without 0 * inf
       const float m_safe = m_new == -INFINITY ? 0.f : m_new;
       if (__any(m_new != m_run[b])) {   // later tiles seldom hold a larger score for any of the rows
@@ -840,8 +839,8 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
   }
 #pragma unroll
   for (int b = 0; b < QB; ++b) {   // a row's sum: its four lanes' parts
-    l_run[b] += __shfl_xor(l_run[b], 16, kWave);
-    l_run[b] += __shfl_xor(l_run[b], 32, kWave);
+    const LanePair near = across16(l_run[b]), far = across32(near.lo + near.hi);
+    l_run[b] = far.lo + far.hi;
   }
 
   if (HEADS && WAVES > 1) {

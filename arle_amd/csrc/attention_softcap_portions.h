@@ -268,7 +268,7 @@ __global__ __launch_bounds__(kCpWaves* kWave, 2) void cap_portions_kernel(const 
 #pragma unroll
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, st[t][r]);
     {
-      const HalfPair both = both_halves(bmax);
+      const LanePair both = across32(bmax);
       bmax = fmaxf(both.lo, both.hi);
     }
     // m is what the row's exponentials are taken from, not its exact maximum: it moves when that has grown by more than kCpLazyBits
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kCpWaves* kWave, 2) void cap_portions_kernel(const 
       __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 1);
     }
   }
-  const HalfPair both = both_halves(l);
+  const LanePair both = across32(l);
   l = both.lo + both.hi;
 
   // o[dt][r] is O^T[d = 32 dt + 8 (r / 4) + 4 h + r % 4][this lane's row]

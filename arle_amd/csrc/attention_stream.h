@@ -387,18 +387,18 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
         for (int dt = 0; dt < DTL; ++dt) vsum[dt] += u < n_parts ? one_of(vgot[dt], v_col + 16 * dt) : 0.f;
       }
       if (vp > 1) {
-        float far[DTL];
 #pragma unroll
-        for (int dt = 0; dt < DTL; ++dt) far[dt] = __shfl_xor(vsum[dt], 16, kWave);
-#pragma unroll
-        for (int dt = 0; dt < DTL; ++dt) vsum[dt] += far[dt];
+        for (int dt = 0; dt < DTL; ++dt) {
+          const LanePair near = across16(vsum[dt]);
+          vsum[dt] = near.lo + near.hi;
+        }
       }
       if (vp > 2) {
-        float far[DTL];
 #pragma unroll
-        for (int dt = 0; dt < DTL; ++dt) far[dt] = __shfl_xor(vsum[dt], 32, kWave);
-#pragma unroll
-        for (int dt = 0; dt < DTL; ++dt) vsum[dt] += far[dt];
+        for (int dt = 0; dt < DTL; ++dt) {
+          const LanePair far = across32(vsum[dt]);
+          vsum[dt] = far.lo + far.hi;
+        }
       }
       finish_head(xk, a.prep_kw != nullptr, wk, knew);
 #pragma unroll

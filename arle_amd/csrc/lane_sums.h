@@ -5,10 +5,6 @@
 
 namespace arle {
 
-template <int CTRL>
-__device__ __forceinline__ float row_move(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
 __device__ __forceinline__ float row_sum16(float v) {
   v += row_move<0xB1>(v);    // quad_perm [1, 0, 3, 2]
   v += row_move<0x4E>(v);    // quad_perm [2, 3, 0, 1]

@@ -1,19 +1,8 @@
-// Loads from memory straight into LDS that the compiler does not count, and an exchange between the halves of a wave.
+// Loads from memory straight into LDS that the compiler does not count.
 #pragma once
 #include "common.h"
 
 namespace arle {
-
-// A value of lane i and the value of lane i ^ 32, in the same order in both lanes (v_permlane32_swap: one vector
-// instruction, where a shuffle is a trip through the LDS unit).
-struct HalfPair {
-  float lo, hi;
-};
-__device__ __forceinline__ HalfPair both_halves(float x) {
-  const unsigned bits = __float_as_uint(x);
-  const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
-}
 
 // Sixteen bytes a lane from memory straight into LDS: the wave's 64 pieces land one after the other from
 // lds_base on, which has to be the same in all lanes.  Written as assembly, and not with the compiler's builtin,

@@ -251,8 +251,7 @@ __global__ __launch_bounds__(256) void qk_prep_bf16x8_kernel(
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-#pragma unroll
-      for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+      ss = lanes_sum<LPH>(ss);
       const float inv = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = x[e] * inv * wt[e];

@@ -217,9 +217,7 @@ __global__ __launch_bounds__(256) void rotary_qkv_store_x8_kernel(
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
-#pragma unroll
-    for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
-    return ss;
+    return lanes_sum<LPH>(ss);
   };
   if (weight) {
     float wv[8];

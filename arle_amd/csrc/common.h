@@ -108,7 +108,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // of additions is fixed (butterfly inside a wave, then waves 0..n-1), so a row's
 // reduction never depends on what else is in the launch.
 template <int kWaves>
-__device__ __forceinline__ float block_sum(float v, float* lds /* [kWaves] */) {
+__device__ __forceinline__ float block_sum_once(float v, float* lds /* [kWaves], used for nothing else */) {
   v = wave_sum(v);
   const int wave = threadIdx.x / kWave;
   if ((threadIdx.x % kWave) == 0) lds[wave] = v;
@@ -116,6 +116,12 @@ __device__ __forceinline__ float block_sum(float v, float* lds /* [kWaves] */) {
   float total = 0.f;
 #pragma unroll
   for (int i = 0; i < kWaves; ++i) total += lds[i];
+  return total;
+}
+// The same with words that are free again behind it.
+template <int kWaves>
+__device__ __forceinline__ float block_sum(float v, float* lds /* [kWaves] */) {
+  const float total = block_sum_once<kWaves>(v, lds);
   __syncthreads();
   return total;
 }

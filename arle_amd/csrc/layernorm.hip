@@ -239,16 +239,7 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
       sum += (x[k].x + x[k].y) + (x[k].z + x[k].w);
     }
   }
-  auto row_sum = [&](float v, float* own) {      // block_sum with words of its own: nothing waits behind it for them to be free
-    v = wave_sum(v);
-    if (tid % kWave == 0) own[tid / kWave] = v;
-    __syncthreads();
-    float total = 0.f;
-#pragma unroll
-    for (int j = 0; j < NT / kWave; ++j) total += own[j];
-    return total;
-  };
-  const float mu = row_sum(sum, lds[0]) / static_cast<float>(width);
+  const float mu = block_sum_once<NT / kWave>(sum, lds[0]) / static_cast<float>(width);
   float sq = 0.f;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {
@@ -256,7 +247,7 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
     x[k].x -= mu; x[k].y -= mu; x[k].z -= mu; x[k].w -= mu;
     if (i < width) sq += (x[k].x * x[k].x + x[k].y * x[k].y) + (x[k].z * x[k].z + x[k].w * x[k].w);
   }
-  const float inv = 1.0f / sqrtf(row_sum(sq, lds[1]) / static_cast<float>(width) + eps);
+  const float inv = 1.0f / sqrtf(block_sum_once<NT / kWave>(sq, lds[1]) / static_cast<float>(width) + eps);
   const int64_t o = static_cast<int64_t>(r) * width;
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {

@@ -9,6 +9,8 @@
 // updates a float row and adds a delta of the activation type.
 #include "common.h"
 
+#include <type_traits>
+
 namespace arle {
 
 constexpr int kNormThreads = 256;
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(TIn* __restri
     }
     if (in[j]) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
   }
-  const float total = block_sum<kNormWaves>(ss, lds);
+  const float total = block_sum_once<kNormWaves>(ss, lds);
   const float inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
   TOut* o = out + static_cast<int64_t>(r) * width;
 #pragma unroll
@@ -188,6 +190,8 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(TIn* __restri
 // stacks of up to four, else eight (six parts as a round of four and one behind it were two trips to memory, and 1,024
 // threads for 2,560 columns six idle waves to start: whole decode steps of the Qwen3-4B shape 2,461 -> 2,436 us with one request,
 // 2,985 -> 2,956 with 19).
+// Only the parts that there are are fetched: fetching the last one again for those past the end cost 8 rows of 2,560 with six parts
+// 3.2 us, so 3.0, with two 2.8 / 2.7; 97 rows 3.4 / 3.2.
 // Order of addition: residual + (delta 0 + delta 1 + ...), as in the kernels above; idle waves would add zeros to the
 // sum of squares, so the threads do not change a bit.
 constexpr int kStackThreads = 1024;
@@ -205,23 +209,25 @@ __global__ __launch_bounds__(THREADS) void add_stack_rmsnorm_kernel(
   const float* dr = delta + src * width;
   const int ic = mine ? i : 0;
   float4 v = load4<float>(res + ic), d = {0.f, 0.f, 0.f, 0.f};
-  const float4 wv = load4<TW>(w + ic);
-  // The loads of a round carry no condition (a load under a condition is waited for before the next one is
-  // issued, and the parts would arrive one after the other): those past the last part fetch the last part again and are
-  // not added.  Threads past the width read column 0.
+  // A round's loads carry no condition but on its number of parts, the same for the workgroup: a jump, which waits for
+  // no load (one under a condition of the lane's is waited for before the next is issued, and the parts would arrive one after
+  // the other).  Threads past the width read column 0.
   const float* dc = dr + ic;
+  // (widened behind the sum: a conversion waits for its load)
+  const auto w_raw = *reinterpret_cast<const std::conditional_t<sizeof(TW) == 4, float4, uint2>*>(w + ic);
   for (int base = 0; base < n_delta; base += UNROLL) {
     float4 e[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) e[u] = load4<float>(dc + min(base + u, n_delta - 1) * delta_stride);
+    for (int u = 0; u < UNROLL; ++u)
+      if (base + u < n_delta) e[u] = load4<float>(dc + (base + u) * delta_stride);
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const bool in = base + u < n_delta;
-      d.x += in ? e[u].x : 0.f;
-      d.y += in ? e[u].y : 0.f;
-      d.z += in ? e[u].z : 0.f;
-      d.w += in ? e[u].w : 0.f;
-    }
+    for (int u = 0; u < UNROLL; ++u)
+      if (base + u < n_delta) {
+        d.x += e[u].x;
+        d.y += e[u].y;
+        d.z += e[u].z;
+        d.w += e[u].w;
+      }
   }
   v.x += d.x;
   v.y += d.y;
@@ -229,8 +235,9 @@ __global__ __launch_bounds__(THREADS) void add_stack_rmsnorm_kernel(
   v.w += d.w;
   if (mine && !rows) store4<float>(res + i, v);
   const float total =
-      block_sum<THREADS / kWave>(mine ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f, lds);
+      block_sum_once<THREADS / kWave>(mine ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f, lds);
   const float inv = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
+  const float4 wv = load4<TW>(reinterpret_cast<const TW*>(&w_raw));
   if (mine)
     store4<TOut>(out + static_cast<int64_t>(r) * width + i,
                  float4{v.x * inv * wv.x, v.y * inv * wv.y, v.z * inv * wv.z, v.w * inv * wv.w});

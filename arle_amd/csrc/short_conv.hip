@@ -181,24 +181,28 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
 // writes them back moved on by its row, and no second kernel has to wait for this one (decode steps of the Gufasun design had
 // twelve of these pairs, 4.4 + 3.9 us each at 8 requests; together 4.6; the eight behind a norm are in the norm's kernel now).  PARTS: the input is a stack of float32 partial sums, added in order and
 // rounded to T as the kernel that adds such stacks does.
+// Four channels of a row from c on: the convolution's outputs (before a silu), and their state moved on (`live`: else nothing is
+// written, and c is a group that exists).
 template <typename T, int TAPS, bool PARTS>
-__global__ void conv_step_kernel(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,
-                                 const T* __restrict__ bias, const T* __restrict__ out_bias, const T* __restrict__ w,
-                                 T* __restrict__ state, const int* __restrict__ slot_of_token, T* __restrict__ out,
-                                 long long out_stride, int channels, int flags) {
-  const int64_t t = blockIdx.x;
-  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
-  if (c >= channels) return;
-  T* mine = state + static_cast<int64_t>(slot_of_token[t]) * (TAPS - 1) * channels + c;
+__device__ __forceinline__ float4 conv_step_channels(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,
+                                                     const T* __restrict__ bias, const T* __restrict__ out_bias,
+                                                     const T* __restrict__ w, T* __restrict__ state, int64_t slot, int64_t t, int c,
+                                                     int channels, int flags, bool live) {
+  T* mine = state + slot * (TAPS - 1) * channels + c;
   float4 in[TAPS];     // in[back]: the input `back` rows before this one
 #pragma unroll
   for (int back = 1; back < TAPS; ++back) in[back] = ld4<T>(mine + static_cast<int64_t>(TAPS - 1 - back) * channels);
   if constexpr (PARTS) {
     const float* at = static_cast<const float*>(u) + t * u_stride + c;
     float4 v = ld4<float>(at);
-    for (int s = 1; s < parts; ++s) {
-      const float4 e = ld4<float>(at + s * part_stride);
-      v = float4{v.x + e.x, v.y + e.y, v.z + e.z, v.w + e.w};
+    for (int s0 = 1; s0 < parts; s0 += 7) {      // seven more at a time; a jump that all lanes take together waits for no load
+      float4 e[7];
+#pragma unroll
+      for (int j = 0; j < 7; ++j)
+        if (s0 + j < parts) e[j] = ld4<float>(at + (s0 + j) * part_stride);
+#pragma unroll
+      for (int j = 0; j < 7; ++j)
+        if (s0 + j < parts) v = float4{v.x + e[j].x, v.y + e[j].y, v.z + e[j].z, v.w + e[j].w};
     }
     in[0] = float4{to_float(from_float<T>(v.x)), to_float(from_float<T>(v.y)), to_float(from_float<T>(v.z)), to_float(from_float<T>(v.w))};
   } else {
@@ -225,9 +229,84 @@ __global__ void conv_step_kernel(const void* __restrict__ u, long long u_stride,
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt[i][TAPS - 1 - back], v[i], acc[i]);
   }
+  if (live) {
 #pragma unroll
-  for (int back = 0; back < TAPS - 1; ++back) st4<T>(mine + static_cast<int64_t>(TAPS - 2 - back) * channels, in[back]);
-  st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], flags), conv_out(acc[1], flags), conv_out(acc[2], flags), conv_out(acc[3], flags)});
+    for (int back = 0; back < TAPS - 1; ++back) st4<T>(mine + static_cast<int64_t>(TAPS - 2 - back) * channels, in[back]);
+  }
+  return float4{acc[0], acc[1], acc[2], acc[3]};
+}
+
+template <typename T, int TAPS, bool PARTS>
+__global__ void conv_step_kernel(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,
+                                 const T* __restrict__ bias, const T* __restrict__ out_bias, const T* __restrict__ w,
+                                 T* __restrict__ state, const int* __restrict__ slot_of_token, T* __restrict__ out,
+                                 long long out_stride, int channels, int flags) {
+  const int64_t t = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (c >= channels) return;
+  const float4 y = conv_step_channels<T, TAPS, PARTS>(u, u_stride, parts, part_stride, bias, out_bias, w, state, slot_of_token[t], t, c,
+                                                      channels, flags, true);
+  st4<T>(out + t * out_stride + c, float4{conv_out(y.x, flags), conv_out(y.y, flags), conv_out(y.z, flags), conv_out(y.w, flags)});
+}
+
+// The same with what an attention makes of its channels, q's, k's and v's one after the other: every head of q and k over the root
+// mean square of its outputs, times the norm's weight and q's factor for its position, k and v into the request's pages (k a row, v
+// turned).  A head of q or k is 4 * LPH channels, LPH lanes.  One kernel less to wait for in a step of single rows, which is a chain
+// of such kernels: 8 rows of 6,144 channels, a convolution of 4.5 us and norms and stores of 4.5 became one of 5.3 on MI355X (a step of 8 requests
+// of the Gufasun design 719 -> 709 us).
+struct ConvHeads {
+  const bf16* q_weight;      // [4 * LPH] or null
+  const bf16* k_weight;
+  float eps, temp_coef;
+  int temp_every;
+  const int* positions;
+  const int* block_table;
+  int table_stride;
+  bf16* k_pages;             // [page, nkv, page_size, key_dim]
+  bf16* v_pages;             // [page, nkv, value_dim, page_size]
+  int nq, nkv, value_dim, page_size;
+};
+
+template <int TAPS, bool PARTS, int LPH>
+__global__ __launch_bounds__(256) void conv_step_store_kernel(const void* __restrict__ u, long long u_stride, int parts,
+                                                              long long part_stride, const bf16* __restrict__ bias,
+                                                              const bf16* __restrict__ w, bf16* __restrict__ state,
+                                                              const int* __restrict__ slot_of_token, bf16* __restrict__ q,
+                                                              int channels, const ConvHeads a) {
+  constexpr int Dk = 4 * LPH;
+  const int64_t t = blockIdx.x;
+  const int at = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  const bool live = at < channels;      // lanes behind the last channel take part in the sums below
+  const int c = live ? at : channels - 4;
+  const int q_end = a.nq * Dk, k_end = q_end + a.nkv * Dk;
+  const int pos = a.positions[t], slot = slot_of_token[t];
+  const int64_t page = a.nkv ? a.block_table[static_cast<int64_t>(slot) * a.table_stride + pos / a.page_size] : 0;
+  const bool is_q = c < q_end, is_k = !is_q && c < k_end;
+  const bf16* weight = is_q ? a.q_weight : a.k_weight;
+  const int d = c % Dk;                 // of a head of q or k: they end on whole heads
+  const float4 wv = weight ? ld4<bf16>(weight + d) : float4{1.f, 1.f, 1.f, 1.f};
+  const float4 y = conv_step_channels<bf16, TAPS, PARTS>(u, u_stride, parts, part_stride, bias, nullptr, w, state, slot, t, c, channels, 0, live);
+  // what the convolution alone would have written
+  const float x[4] = {to_float(from_float<bf16>(y.x)), to_float(from_float<bf16>(y.y)), to_float(from_float<bf16>(y.z)),
+                      to_float(from_float<bf16>(y.w))};
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss = fmaf(x[e], x[e], ss);
+  ss = lanes_sum<LPH>(ss);
+  if (!live) return;
+  float f = 1.0f / sqrtf(ss / static_cast<float>(Dk) + a.eps);
+  if (is_q) {
+    if (a.temp_coef != 0.f) f *= 1.0f + a.temp_coef * logf(static_cast<float>((pos + 1) / a.temp_every + 1));
+    st4<bf16>(q + t * q_end + c, float4{x[0] * f * wv.x, x[1] * f * wv.y, x[2] * f * wv.z, x[3] * f * wv.w});
+  } else if (is_k) {
+    const int64_t row = (page * a.nkv + (c - q_end) / Dk) * a.page_size + pos % a.page_size;
+    st4<bf16>(a.k_pages + row * Dk + d, float4{x[0] * f * wv.x, x[1] * f * wv.y, x[2] * f * wv.z, x[3] * f * wv.w});
+  } else {
+    // channel j of v: element j % value_dim of kv head j / value_dim
+    bf16* v = a.v_pages + (page * a.nkv * a.value_dim + (c - k_end)) * a.page_size + pos % a.page_size;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[static_cast<int64_t>(e) * a.page_size] = from_float<bf16>(x[e]);
+  }
 }
 
 // One thread a (segment, channel): the new state is the last taps-1 of (old state, this step's inputs).
@@ -351,5 +430,43 @@ extern "C" int arle_conv_step(const void* u, long long u_stride, int parts, long
   }
 #undef ARLE_CONV_STEP_TAPS
 #undef ARLE_CONV_STEP
+  return launch_status();
+}
+
+// arle_conv_step in bfloat16 with q's and k's head norm and the store behind it (conv_step_store_kernel): channels = (nq + nkv) *
+// key_dim + nkv * value_dim, key_dim 64, 128 or 256, value_dim a multiple of 4; nkv 0: q alone, no pages.  q [T, nq * key_dim].
+extern "C" int arle_conv_step_store(const void* u, long long u_stride, int parts, long long part_stride, const void* bias, const void* w,
+                                    void* state, const int* slot_of_token, void* q, int tokens, int taps, const void* q_weight,
+                                    const void* k_weight, float eps, float temp_coef, int temp_every, const int* positions,
+                                    const int* block_table, int table_stride, void* k_pages, void* v_pages, int nq, int nkv, int key_dim,
+                                    int value_dim, int page_size, void* stream) {
+  if (tokens == 0) return 0;
+  const auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (taps < 2 || taps > 4 || u_stride % 4 != 0 || part_stride % 4 != 0 || parts < 0 || !at16(u) || !at16(q) || !at16(state) || !at16(w) ||
+      !at16(bias) || !at16(q_weight) || !at16(k_weight) || !at16(k_pages) || nq < 1 || nkv < 0 || value_dim % 4 != 0 ||
+      (key_dim != 64 && key_dim != 128 && key_dim != 256) || (nkv > 0 && (page_size < 1 || !k_pages || !v_pages || !block_table)) ||
+      (temp_coef != 0.f && temp_every < 1))
+    return static_cast<int>(hipErrorInvalidValue);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int channels = (nq + nkv) * key_dim + nkv * value_dim;
+  const ConvHeads heads{static_cast<const bf16*>(q_weight), static_cast<const bf16*>(k_weight), eps, temp_coef, temp_every, positions,
+                        block_table, table_stride, static_cast<bf16*>(k_pages), static_cast<bf16*>(v_pages), nq, nkv, value_dim, page_size};
+  const dim3 grid(tokens, (channels / 4 + 255) / 256);
+#define ARLE_STORE(TAPS, PARTS, LPH)                                                                                          \
+  conv_step_store_kernel<TAPS, PARTS, LPH><<<grid, 256, 0, s>>>(u, u_stride, parts, part_stride, static_cast<const bf16*>(bias), \
+                                                                static_cast<const bf16*>(w), static_cast<bf16*>(state), slot_of_token, \
+                                                                static_cast<bf16*>(q), channels, heads)
+#define ARLE_STORE_DIM(TAPS, PARTS)                                                                                           \
+  do {                                                                                                                        \
+    if (key_dim == 64) ARLE_STORE(TAPS, PARTS, 16); else if (key_dim == 128) ARLE_STORE(TAPS, PARTS, 32); else ARLE_STORE(TAPS, PARTS, 64); \
+  } while (0)
+#define ARLE_STORE_TAPS(PARTS)                                                                                                \
+  do {                                                                                                                        \
+    if (taps == 2) ARLE_STORE_DIM(2, PARTS); else if (taps == 3) ARLE_STORE_DIM(3, PARTS); else ARLE_STORE_DIM(4, PARTS);     \
+  } while (0)
+  if (parts > 0) ARLE_STORE_TAPS(true); else ARLE_STORE_TAPS(false);
+#undef ARLE_STORE_TAPS
+#undef ARLE_STORE_DIM
+#undef ARLE_STORE
   return launch_status();
 }

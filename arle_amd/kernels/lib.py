@@ -66,6 +66,8 @@ SIGNATURES = {
     "arle_causal_conv": ("short_conv", [_p, _ll, _i, _p, _i, _p, _i, _p, _i, _p, _i, _p, _p, _ll, _i, _i, _i, _i, _i, _p]),
     "arle_conv_state_update": ("short_conv", [_p, _ll, _i, _p, _i, _p, _i, _p, _p, _i, _i, _i, _p]),
     "arle_conv_step": ("short_conv", [_p, _ll, _i, _ll, _i, _p, _p, _p, _p, _p, _p, _ll, _i, _i, _i, _i, _p]),
+    "arle_conv_step_store": ("short_conv", [_p, _ll, _i, _ll, _p, _p, _p, _p, _p, _i, _i, _p, _p, _f, _f, _i, _p, _p, _i, _p, _p, _i, _i, _i,
+                                            _i, _i, _p]),
     "arle_polynorm_parts": ("polynorm", [_p, _i, _p, _p, _p, _i, _i, _i, _f, _p]),
     "arle_mlstm_decode": ("mlstm", [_p, _ll, _ll, _i, _p, _ll, _ll, _i, _p, _p, _f, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _i, _p, _i,
                                     _f, _p]),

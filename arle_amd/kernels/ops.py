@@ -1808,6 +1808,51 @@ def conv_step(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, bi
     return out
 
 
+CONV_STORE_KEY_DIMS = (64, 128, 256)
+
+
+def conv_step_store_supported(weight, state, key_dim: int, value_dim: int, *, bias=None, norms=()) -> bool:
+    """Whether conv_step_store takes a convolution that conv_step takes (of bfloat16) in front of heads of these sizes."""
+    return (conv_step_supported(weight, state, bias=bias) and weight.dtype == torch.bfloat16 and key_dim in CONV_STORE_KEY_DIMS
+            and value_dim % 4 == 0 and all(n is None or (n.dtype == torch.bfloat16 and n.data_ptr() % 16 == 0) for n in norms))
+
+
+def conv_step_store(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, num_q_heads: int, num_kv_heads: int, key_dim: int,
+                    value_dim: int, eps: float, positions, bias=None, q_weight=None, k_weight=None, temp_coef: float = 0.0,
+                    temp_every: int = 1, block_table=None, k_pages=None, v_pages=None, page_size: int = 0):
+    """conv_step and qkv_norm_store of its channels (q's, k's, v's) in one kernel; returns q [T, heads * Dk].  num_kv_heads 0: q alone."""
+    _gpu(u, weight, state, slot_of_token, bias, q_weight, k_weight, positions, block_table, k_pages, v_pages)
+    parts = u.shape[0] if u.dim() == 3 else 0
+    tokens, channels = u.shape[-2:]
+    _i32(slot_of_token, "slot_of_token", tokens)
+    _i32(positions, "positions", tokens)
+    _need(num_q_heads > 0 and num_kv_heads >= 0 and channels == (num_q_heads + num_kv_heads) * key_dim + num_kv_heads * value_dim,
+          "the convolution's channels must be those of q, k and v")
+    _need(weight.shape[0] == channels and tuple(state.shape[1:]) == (weight.shape[1] - 1, channels)
+          and conv_step_store_supported(weight, state, key_dim, value_dim, bias=bias, norms=(q_weight, k_weight)),
+          "conv_step_store does not take this convolution")
+    _need((u.dtype == torch.float32 and u.is_contiguous()) if parts else (u.dtype == weight.dtype and u.stride(1) == 1),
+          "conv_step_store takes rows of the weight's type, or a contiguous float32 stack")
+    _need(u.stride(-2) % 4 == 0 and u.data_ptr() % 16 == 0, "conv_step_store takes rows on the 16-byte grid")
+    _need(bias is None or bias.shape == (channels,), "a convolution's bias must be [channels]")
+    for w in (q_weight, k_weight):
+        _need(w is None or (w.shape == (key_dim,) and w.is_contiguous()), "a q/k norm weight must be [Dk]")
+    _need(temp_coef == 0.0 or temp_every >= 1, "the query temperature's period must be positive")
+    table_stride = 0
+    if num_kv_heads:
+        _check_kv_pages(k_pages, v_pages, num_kv_heads, page_size, key_dim, value_dim, weight.dtype)
+        _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.is_contiguous(),
+              "block_table must be contiguous int32 [slots, pages]")
+        table_stride = block_table.shape[1]
+    q = torch.empty((tokens, num_q_heads * key_dim), dtype=weight.dtype, device=u.device)
+    lib.call("arle_conv_step_store", u.data_ptr(), u.stride(-2), parts, u.stride(0) if parts else 0, _ptr(bias), weight.data_ptr(),
+             state.data_ptr(), slot_of_token.data_ptr(), q.data_ptr(), tokens, weight.shape[1], _ptr(q_weight), _ptr(k_weight), float(eps),
+             float(temp_coef), int(temp_every), positions.data_ptr(), _ptr(block_table) if num_kv_heads else 0, table_stride,
+             _ptr(k_pages) if num_kv_heads else 0, _ptr(v_pages) if num_kv_heads else 0, num_q_heads, num_kv_heads, key_dim, value_dim,
+             int(page_size), _stream())
+    return q
+
+
 def conv_state_update(u: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor, *, bias=None):
     """state[slot] <- the last taps-1 rows of (state[slot], the request's rows of u (+ bias)), for every segment."""
     _gpu(u, state, seg_row0, seg_slot, bias)

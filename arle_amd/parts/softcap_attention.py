@@ -117,6 +117,14 @@ class SoftcapAttention(Part):
     def reader_cache_need(self):
         return self.declare_reader_cache(self.params)
 
+    def _stores_behind_conv(self, u, x, batch, conv) -> bool:
+        """Whether the convolution of the step's rows is one kernel with the norm and the store: steps of single rows in bfloat16, a
+        convolution on the products alone, heads of a size that kernel takes."""
+        return (x.dtype == torch.bfloat16 and (u.dim() == 3 or (u.dtype == torch.bfloat16 and u.stride(0) % 4 == 0 and u.data_ptr() % 16 == 0))
+                and self.conv.out_bias is None and self.conv.takes_parts(batch, conv)
+                and ops.conv_step_store_supported(self.conv.weight, conv.state, self.Dk, self.Dv, bias=self.conv.bias,
+                                                  norms=(self.q_norm, self.k_norm)))
+
     def products(self):
         if self.proj.weight.dtype != torch.bfloat16:
             return []
@@ -130,21 +138,22 @@ class SoftcapAttention(Part):
             raise ValueError("a layer that shares keys and values must read another entry's pages, and only such a layer")
         conv = cache.get("conv")
         few = x.shape[0] <= ops.ROWS_KERNEL_MAX and self.conv.takes_parts(batch, conv) and self.conv.weight.dtype == x.dtype
-        y = self.conv(self.proj(x, partials_ok=few), batch, conv)
+        u = self.proj(x, partials_ok=few)
+        own = {} if self.shares_kv else dict(block_table=kv.block_table, k_pages=kv.pages["k"], v_pages=kv.pages["v"], page_size=kv.page_size)
+        heads = dict(num_q_heads=self.nq, num_kv_heads=0 if self.shares_kv else self.nkv, key_dim=self.Dk, value_dim=self.Dv, eps=self.eps,
+                     q_weight=self.q_norm, k_weight=None if self.shares_kv else self.k_norm, temp_coef=self.temp_coef,
+                     temp_every=self.temp_every, positions=batch.positions, **own)
         Q = self.widths[0]
-        q = y[:, :Q]
-        if self.shares_kv:
-            ops.qkv_norm_store(q, None, None, num_q_heads=self.nq, num_kv_heads=0, key_dim=self.Dk, value_dim=self.Dv,
-                               eps=self.eps, q_weight=self.q_norm, temp_coef=self.temp_coef, temp_every=self.temp_every,
-                               positions=batch.positions)
+        if self._stores_behind_conv(u, x, batch, conv):
+            q = ops.conv_step_store(u, self.conv.weight, conv.state, batch.slot_of_token, bias=self.conv.bias, **heads)
         else:
-            K = self.widths[1]
-            ops.qkv_norm_store(q, y[:, Q:Q + K], y[:, Q + K:], num_q_heads=self.nq, num_kv_heads=self.nkv,
-                               key_dim=self.Dk, value_dim=self.Dv, eps=self.eps, q_weight=self.q_norm,
-                               k_weight=self.k_norm, temp_coef=self.temp_coef, temp_every=self.temp_every,
-                               positions=batch.positions, slot_of_token=batch.slot_of_token,
-                               block_table=kv.block_table, k_pages=kv.pages["k"], v_pages=kv.pages["v"],
-                               page_size=kv.page_size)
+            y = self.conv(u, batch, conv)
+            q, k, v = y[:, :Q], None, None
+            if not self.shares_kv:
+                K = self.widths[1]
+                k, v = y[:, Q:Q + K], y[:, Q + K:]
+                heads["slot_of_token"] = batch.slot_of_token
+            ops.qkv_norm_store(q, k, v, **heads)
         out = torch.empty((x.shape[0], self.nq * self.Dv), dtype=x.dtype, device=x.device)
         softcap_attention(q, out, kv, batch, num_q_heads=self.nq, num_kv_heads=self.nkv, key_dim=self.Dk,
                           value_dim=self.Dv, scale=self.scale, softcap=self.softcap, r1=self.r1, r2=self.r2,

@@ -56,26 +56,41 @@ __global__ __launch_bounds__(kPnThreads) void polynorm_kernel(const void* __rest
 }
 
 // One element type T for input, bias, coefficients and output, a width that is a multiple of 4: four elements a lane
-// and access, all loads of the row issued together.  PARTS: u is a stack of float32 partial sums instead, added in order and
+// and access, all loads of the row and what its end takes issued together, one barrier for the three sums: a chain of latencies for
+// few rows (8 rows of 9,728 in three parts 4.4 us; a part at a time, the coefficients behind the sums and two barriers a sum 4.7),
+// the bytes for many (2,048 rows, no parts, 15.0 -> 14.4 us for 80 MB).  PARTS: u is a stack of float32 partial sums instead, added in order and
 // rounded to T, as the kernel that adds such stacks does.
 template <typename T, int NT, int PER4, bool PARTS>
 __global__ __launch_bounds__(NT) void polynorm_vec_kernel(const void* __restrict__ u, long long u_stride, int parts, long long part_stride,
                                                                   const T* __restrict__ bias, const T* __restrict__ coef,
                                                                   T* __restrict__ out, int width, float eps) {
-  __shared__ float lds[(NT / kWave)];
+  __shared__ float lds[3][(NT / kWave)];
   const int64_t r = blockIdx.x;
   const int last = width - 4, tid = threadIdx.x;
+  // everything that the row's end takes is on its way with the row
+  T a1[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) a1[j] = coef[j];
   float4 z[PER4];
   if constexpr (PARTS) {
     const float* at = static_cast<const float*>(u) + r * u_stride;
 #pragma unroll
     for (int k = 0; k < PER4; ++k) z[k] = ld4<float>(at + min((tid + k * NT) * 4, last));
-    for (int s = 1; s < parts; ++s) {
-      float4 e[PER4];
+    // Parts at a time (a jump that all lanes take together waits for no load); two of seven accesses each, or three in float32, cost
+    // many rows more in waves a SIMD than they gain (2,048 rows of 12,288, one part, 24.9 us / 29.9).
+    constexpr int G = !std::is_same<T, float>::value && PER4 <= 5 ? 3 : 1;
+    for (int s0 = 1; s0 < parts; s0 += G) {
+      float4 e[G][PER4];
 #pragma unroll
-      for (int k = 0; k < PER4; ++k) e[k] = ld4<float>(at + s * part_stride + min((tid + k * NT) * 4, last));
+      for (int j = 0; j < G; ++j)
+        if (s0 + j < parts)
 #pragma unroll
-      for (int k = 0; k < PER4; ++k) z[k] = float4{z[k].x + e[k].x, z[k].y + e[k].y, z[k].z + e[k].z, z[k].w + e[k].w};
+          for (int k = 0; k < PER4; ++k) e[j][k] = ld4<float>(at + (s0 + j) * part_stride + min((tid + k * NT) * 4, last));
+#pragma unroll
+      for (int j = 0; j < G; ++j)
+        if (s0 + j < parts)
+#pragma unroll
+          for (int k = 0; k < PER4; ++k) z[k] = float4{z[k].x + e[j][k].x, z[k].y + e[j][k].y, z[k].z + e[j][k].z, z[k].w + e[j][k].w};
     }
 #pragma unroll
     for (int k = 0; k < PER4; ++k)
@@ -106,10 +121,22 @@ __global__ __launch_bounds__(NT) void polynorm_vec_kernel(const void* __restrict
     }
   }
   const float n = static_cast<float>(width);
-  const float i1 = 1.0f / sqrtf(block_sum<(NT / kWave)>(s2, lds) / n + eps);
-  const float i2 = 1.0f / sqrtf(block_sum<(NT / kWave)>(s4, lds) / n + eps);
-  const float i3 = 1.0f / sqrtf(block_sum<(NT / kWave)>(s6, lds) / n + eps);
-  const float a = to_float(coef[0]) * i1, b = to_float(coef[1]) * i2, c = to_float(coef[2]) * i3, e = to_float(coef[3]);
+  // the three sums meet behind one barrier, each in the order of block_sum
+  const float waves[3] = {wave_sum(s2), wave_sum(s4), wave_sum(s6)};
+  if (tid % kWave == 0) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) lds[j][tid / kWave] = waves[j];
+  }
+  __syncthreads();
+  float inv[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    float total = 0.f;
+#pragma unroll
+    for (int k = 0; k < NT / kWave; ++k) total += lds[j][k];
+    inv[j] = 1.0f / sqrtf(total / n + eps);
+  }
+  const float a = to_float(a1[0]) * inv[0], b = to_float(a1[1]) * inv[1], c = to_float(a1[2]) * inv[2], e = to_float(a1[3]);
   auto poly = [&](float v) { return fmaf(v, fmaf(v, fmaf(v, c, b), a), e); };
 #pragma unroll
   for (int k = 0; k < PER4; ++k) {

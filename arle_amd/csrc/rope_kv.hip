@@ -132,7 +132,10 @@ __global__ __launch_bounds__(kPrepWaves* kWave) void qk_prep_kernel(
 // A workgroup takes one head of TPB = 256 / LPH consecutive tokens; a lane holds eight consecutive
 // columns: one 16-byte load and one 16-byte store (q in place, k into its cache row), LPH = head_dim / 8
 // lanes a token.  The per-head sum of squares and the rotation partner (the lane rot/16 away) go through
-// lane shuffles.  A value head is only moved: its pages keep the head's columns as rows ([D][page_size]),
+// lane moves, or shuffles where there is no move of that distance.  Bound by memory for many tokens, by one trip to it for few, as
+// long as no load stands under a lane's condition and both halves of a rotation are the same instructions (a branch a column
+// before): 32 + 2 * 8 heads of 128, 97 tokens 5.8 -> 4.3 us, 2,048 13.7 -> 10.3, 8,192 37.8 -> 34.5 (5.8 TB/s); heads of 64 at 2,048
+// 7.9 -> 5.8; of 256 13.7 -> 8.4.  Only half of a head of 128 rotated: 2,048 11.8 -> 10.3, 8,192 32.5 / 34.6.  A value head is only moved: its pages keep the head's columns as rows ([D][page_size]),
 // so when the workgroup's tokens are one run of consecutive positions of one request that starts at a
 // multiple of 16 (the usual case in a prompt portion), the tile is turned in LDS and written as 16-byte
 // pieces of eight slots; otherwise every element goes to its slot by itself.
@@ -201,32 +204,29 @@ __global__ __launch_bounds__(256) void qk_prep_bf16x8_kernel(
     }
     return;
   }
-  // q or k: up to kPrepHeads heads of this token, all loads first; the angles and the norm's weight are
-  // read once for all of them
+  // q or k: up to kPrepHeads heads of this token, all loads first and none under a condition of the lane's (a token or head past the
+  // last is the last one again, and not stored); the angles and the norm's weight are read once for all of them
   const int count = is_q ? nq : nkv;
   const int n_heads = min(kPrepHeads, count - local);
-  uint16_t* base = is_q ? q + static_cast<int64_t>(t) * q_stride + d0 : k + static_cast<int64_t>(t) * k_stride + d0;
+  const int64_t tc = min(t, tokens - 1);
+  uint16_t* base = is_q ? q + tc * q_stride + d0 : k + tc * k_stride + d0;
   u32x4 raw[kPrepHeads];
 #pragma unroll
-  for (int h = 0; h < kPrepHeads; ++h) {
-    const bool live = valid && h < n_heads;
-    const u32x4 got = *reinterpret_cast<const u32x4*>(live ? base + (local + h) * D : (is_q ? q : k));
-    raw[h] = live ? got : u32x4{0u, 0u, 0u, 0u};
-  }
+  for (int h = 0; h < kPrepHeads; ++h) raw[h] = *reinterpret_cast<const u32x4*>(base + (local + min(h, n_heads - 1)) * D);
   const int half = rot / 2;
   const bool low = d0 < half, rotated = d0 < rot;
   const int lane = threadIdx.x % kWave;
   const int from = rotated ? (low ? lane + half / 8 : lane - half / 8) : lane;
+  const bool turned = LPH == 16 && rot == D;      // the partner's columns are eight lanes on in the row of sixteen
   float cs[8], sn[8], wt[8];
-  {
-    const int cd = low ? d0 : d0 - half;  // column of the cos/sin row
-    const float* cp = cos_t + static_cast<int64_t>(pos) * half + cd;
-    const float* sp = sin_t + static_cast<int64_t>(pos) * half + cd;
+  if (rot > 0) {
+    const int64_t at = static_cast<int64_t>(positions[tc]) * half + (rotated ? (low ? d0 : d0 - half) : 0);   // column of the cos/sin row
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      cs[e] = (rotated && valid) ? cp[e] : 1.0f;
-      sn[e] = (rotated && valid) ? sp[e] : 0.0f;
-    }
+    for (int e = 0; e < 8; ++e) cs[e] = cos_t[at + e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sn[e] = sin_t[at + e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sn[e] = low ? -sn[e] : sn[e];
   }
   const TW* w = is_q ? q_w : k_w;
   if (w != nullptr) {
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256) void qk_prep_bf16x8_kernel(
     const int page = block_table[static_cast<int64_t>(slot) * table_stride + pos / page_size];
     page_row = static_cast<int64_t>(page) * nkv * page_size + pos % page_size;
   }
-  // every lane takes part in the shuffles below (lanes past the last token or head with zeros)
+  // every lane takes part in the exchanges below
 #pragma unroll
   for (int h = 0; h < kPrepHeads; ++h) {
     float x[8];
@@ -256,11 +256,19 @@ __global__ __launch_bounds__(256) void qk_prep_bf16x8_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = x[e] * inv * wt[e];
     }
-    float y[8];
+    float other[8], y[8];
+    if (turned) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) other[e] = row_move<0x128>(x[e]);   // row_ror:8
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) other[e] = __shfl(x[e], from, kWave);
+    }
+    // x cos - other sin in the lower half, x cos + other sin in the upper one: the sign lies in the sine
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float other = __shfl(x[e], from, kWave);
-      y[e] = rotated ? (low ? x[e] * cs[e] - other * sn[e] : other * sn[e] + x[e] * cs[e]) : x[e];
+      const float turn = fmaf(x[e], cs[e], other[e] * sn[e]);
+      y[e] = rotated ? turn : x[e];
     }
     if (valid && h < n_heads) {
       uint16_t* dst = base + (local + h) * D;

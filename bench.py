@@ -769,6 +769,8 @@ def gufasun_work(raw: dict, q: dict, tokens: int, batch: int, context: int) -> d
         "qkv_norm_store": (tokens * 2 * 2 * (n_own * (Q + 2 * KV) + (n_att - n_own) * Q), 0),
         "attn_softcap_mfma_kernel": (n_att * batch * 2 * KV * 2 * keys if decode else 0,
                                      n_att * tokens * keys * a["heads"] * 2 * (a["dim"] + a["vdim"])),
+        "cap_portions_kernel": (0, n_att * tokens * keys * a["heads"] * 2 * (a["dim"] + a["vdim"])),      # portions of heads of 128
+        "conv_step_store_kernel": (tokens * 2 * 2 * (n_own * (Q + 2 * KV) + (n_att - n_own) * Q), 0),     # a step of single rows
         "mlstm_memory_kernel": (n_mem * batch * S * 4 * 2, n_mem * tokens * S * 4),
         "mlstm_decode_kernel": (n_mem * batch * S * 4 * 2, n_mem * tokens * S * 4),      # a step of single rows
         "mlstm_gates_kernel": (n_mem * tokens * m["heads"] * m["dim"] * 2 * 2, 0),

@@ -395,15 +395,26 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
                        head_dim: int, max_kv_len: int, device) -> int:
     """Into how many parts the keys of every row block of a prompt portion are cut.
 
-    The portions kernel gives a row block of 128 rows (tokens x q heads of a kv head) to a workgroup.  A short
-    portion has fewer row blocks than the chip has compute units, however long its context: then the keys are
-    cut too, as far as every part has a compute unit of its own and 512 keys, and the parts are merged by a kernel of
-    its own, which writes and reads every part's rows (5 to 8 us).  us a layer, 32 q heads over 8 kv heads, whole / 2 / 4 parts: a portion of 512
-    tokens behind 512 26 / 28 / 29, behind 1,024 34 / 32 / 32, behind 3,584 72 / 55 / 54; of 100 behind 2,000 56 / 36 / 24; of 300 behind
-    3,000 60 / 43 / 49 (3 parts: 37); of 512 beside 32 requests that decode at 1,024, behind 0, 512, 1,024 and 1,536: 36 / 41,
-    43 / 43, 54 / 46 and 68 / 52.  The number depends on the shape of the step and on the power-of-two class of
-    the longest context only, like the split of decoded tokens, so that a captured step and an eager one choose
-    alike.
+    The portions kernels give a row block of 128 rows (tokens x q heads of a kv head) to a workgroup, and a compute unit
+    has room for one (two at head_dim 128, which share its rate).  A short portion has fewer row blocks than the chip has compute
+    units, however long its context: then the keys are cut too, into parts of 512 keys and more, and the parts are merged by a kernel of
+    its own, which writes and reads every part's rows (5 to 8 us).  Parts are worth it by the turns that the compute units take
+    them in: items * parts / units, rounded up, turns of a part's length each.
+      * up to half as many row blocks as units: as many parts as fit one turn.  us a layer, 32 q heads over 8 kv heads of 128, whole / 2 / 4
+        parts: a portion of 512 tokens behind 512 26 / 28 / 29, behind 1,024 34 / 32 / 32, behind 3,584 72 / 55 / 54; of 100 behind 2,000
+        56 / 36 / 24; of 300 behind 3,000 60 / 43 / 49 (3 parts: 37); of 512 beside 32 requests that decode at 1,024, behind 0, 512,
+        1,024 and 1,536: 36 / 41, 43 / 43, 54 / 46 and 68 / 52.
+      * up to two thirds of the units: three parts in two turns, up to three quarters: four in three.  Behind 3,100 / 7,000 / 15,000, whole and
+        cut: 520 tokens (136 row blocks) at heads of 64 75, 61 / 146, 108 / 290, 204, of 96 149, 111 / 295, 209 / 590, 408, of 128 67, 57 / 125,
+        96 / 248, 179; 768 tokens (192) at heads of 64 81, 76 / 151, 144 / 295, 250 (behind 1,500 52, 54), of 96 159, 137 / 305, 253 /
+        601, 475, of 128, whose two workgroups a unit smooth the turns, 72, 79 / 129, 131 / 254, 242.  Beyond that the
+        merge costs what little the turns give: 900 tokens (232), whole and in two parts, 83, 86 / 153, 157 / 298, 299 at heads of 64.
+      * heads beyond 128, whose row blocks last long beside the merge: the fewest turns of a part's length, and of those the fewest parts from
+        two on, which also evens out causal row blocks.  Heads of 256, whole / 2 / 3 / 4 / 5 / 6 parts, behind 15,000, ms: 360 tokens (96) 7.0 / 4.0
+        / 4.9 / 4.1 / 3.4 / 4.0, 512 (128) 8.1 / 4.8 / 5.8 / 4.6 / 5.1 / 4.4, 800 (200) 8.9 / 8.7 / 8.5 / 8.2 / 7.0 / 7.3, 832 (208) 9.0 / 8.8 / 8.6
+        / 8.3 / 8.2 / 7.4, 900 (232) 8.3 / 8.4 / 8.3 / 8.4 / 8.4 / 8.5, and behind 1,500 1.24 / 1.11 / 1.16 / 1.18 / 1.22 / 1.26.
+    The number depends on the shape of the step and on the power-of-two class of the longest context only, up to 4,096, like the split
+    of decoded tokens, so that a captured step and an eager one choose alike.
     """
     group = num_q_heads // num_kv_heads
     blocks = -(-max_qlen * group // _PORTION_ROWS)
@@ -411,8 +422,17 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
     units = _compute_units(device.index if device.index is not None else torch.cuda.current_device())
     if items >= units or blocks * max(1, long_segments) > _PORTION_LIST_MAX:
         return 1
-    most = (1 << (max(int(max_kv_len), 1).bit_length() - 1)) // 512    # 2 from 1,024 keys on, 4 from 2,048, ...
-    parts = max(1, min(units // items, _PORTION_SPLITS_MAX, most))
+    keys = 1 << (max(int(max_kv_len), 1).bit_length() - 1)
+    most = min(_PORTION_SPLITS_MAX, keys // 512)
+    turns = lambda parts: -(-items * parts // units)
+    if head_dim > 128:
+        parts = min(range(2, most + 1), key=lambda p: (turns(p) / p, p), default=1)
+    else:
+        parts = max(1, min(units // items, most))
+        if parts == 1 and turns(3) == 2 and keys >= 3 * 512:
+            parts = 3
+        elif parts == 1 and turns(4) == 3 and head_dim != 128 and keys >= 4 * (1024 if head_dim == 64 else 512):
+            parts = 4
     while parts > 1 and tokens * num_q_heads * parts * (head_dim + 2) * 4 > _PORTION_WS_BYTES:
         parts -= 1
     return parts

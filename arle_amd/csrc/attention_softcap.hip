@@ -911,11 +911,29 @@ void attn_softcap_mfma_kernel(const CapArgs a) {
 // and 45 us; 1,024 rows, 1,056 waves, 62 and 64; 1,150 rows 72 and 73; 1,250 rows 81 and 74; four portions of 300 rows 33
 // and 32; 2,048 rows 136 and 89).
 constexpr long long kCapTwoBlocks = 1024;
-// Workgroups of 128 rows (tokens times the q heads of a kv head) from which on heads of 128 go to the kernel whose waves share
-// their tiles (attention_softcap_portions.h): with fewer, one-wave items spread over more of the chip.  32 q heads over 8 kv heads,
-// window 1,024, cap and penalty, this kernel / that one, us: 100 rows 11.5 / 13.1, 400 rows (112 of them) 22.7 / 23.2, 512 behind 3,000
+// From how many workgroups of 128 rows on (tokens times the q heads of a kv head; every segment ends one) heads of 128 go to the
+// kernel whose waves share their tiles (attention_softcap_portions.h): with fewer, one-wave items spread over more of the chip.  32 q heads over 8
+// kv heads, window 1,024, cap and penalty, this kernel / that one, us: 100 rows 11.5 / 13.1, 400 rows (112 of them) 22.7 / 23.2, 512 behind 3,000
 // (136) 52.1 / 53.9, 300 beside eight decoded rows (144) 50 / 43, 640 (168) 36.9 / 31.0, 1,024 72 / 44, 2,048 110 / 66, 4,096 195 / 120.
+// The same line for 32 q heads over 16 and 4 kv heads, 64 and 16 over 8, no window, no penalty and no cap: 0.97 to 1.00 of
+// the time one step below it, 0.48 to 0.87 from there on.
 constexpr long long kCapPortions = 144;
+// Steps of short segments leave most rows of their workgroups empty, which costs more than shared tiles give while there are
+// few keys to share: with two q heads a kv head (of which one-wave items hold as many as that kernel's waves) up to 224 keys
+// where a workgroup has 64 rows and less, with more up to 96 keys where it has 80 and less (96 and 224 end classes of contexts that
+// captured steps are told apart by).  This kernel / that one, us: 20 prompts of
+// 16 tokens 10.2 / 11.5 (18.0 / 18.6 behind 200), 100 of 20 35.4 / 39.1, and over 16 kv heads 40 of 30 15.9 / 22.1, behind 100 28 / 35, behind 400 55 /
+// 54, 100 of 8 30 / 44, 67 / 75 behind 200, 110 / 105 behind 400.  Decoded rows beside a portion, as good as empty workgroups all,
+// gain by their keys: 32 of them behind 1,000 beside 20 tokens 81 / 47.
+inline bool cap_portions_pay(long long tokens, int segments, int max_qlen, int max_keys, int group, int nkv) {
+  const long long longest = (static_cast<long long>(max_qlen) * group + kCpRows - 1) / kCpRows;
+  const long long most = tokens * group / kCpRows + segments, each = longest * segments;
+  const long long blocks = most < each ? most : each;   // no fewer than there are
+  if (blocks * nkv < kCapPortions) return false;
+  const int few_keys = group == 2 ? 224 : 96;
+  const bool empty = tokens * group <= (group == 2 ? 64 : 80) * blocks;
+  return max_keys == 0 || max_keys > few_keys || !empty;
+}
 constexpr int kCapSplitWaves = 8;   // waves that share the keys of a decoded row
 constexpr int kCapLdsMost = 160 * 1024;   // LDS of a gfx950 compute unit: no workgroup can ask for more
 
@@ -938,13 +956,19 @@ inline int cap_lds_limit() {
 // Bytes of LDS that a workgroup of the matrix-core kernel may use on this device (the return value, not an error code).
 extern "C" int arle_attn_softcap_lds_limit() { return cap_lds_limit(); }
 
+// Whether portions of heads of 128 of a step of these sizes go to the kernel whose waves share their tiles, as far as sizes decide it.
+extern "C" int arle_attn_softcap_shares_tiles(int tokens, int segments, int max_qlen, int max_keys, int nq, int nkv) {
+  return nkv > 0 && cap_portions_pay(tokens, segments, max_qlen, max_keys, nq / nkv, nkv);
+}
+
 // bfloat16 only.  Dk a multiple of 8 up to 256, Dv a multiple of 16 up to 256, page_size a multiple of 16, rows of
 // q and out 16-byte aligned (strides multiples of 8).  heads_mode: every segment is one row.
-// row_blocks: an upper bound of the sixteen-row blocks of all segments (blocks past the last one return).
+// tokens: rows of all segments; max_qlen: rows of the longest one.  max_keys: the longest context with its rows, 0 where the caller
+// does not know it (a choice between kernels only).
 extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* out, long long o_stride,
                                       const void* k_pages, const void* v_pages, const int* block_table,
                                       int table_stride, const int* seg_row0, const int* seg_slot, const int* seg_start,
-                                      int segments, int row_blocks, int heads_mode, int nq, int nkv, int Dk, int Dv,
+                                      int segments, int tokens, int max_qlen, int max_keys, int heads_mode, int nq, int nkv, int Dk, int Dv,
                                       int page_size, float scale, float cap, const void* r1, const void* r2,
                                       int r_dtype, int window, int chunk, const void* sink, int sink_dtype,
                                       int keep_first, float out_scale, void* stream) {
@@ -971,12 +995,12 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
   const int head_waves = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);   // q heads of one kv head that share a workgroup
   const size_t merge_bytes = static_cast<size_t>(kCapSplitWaves) * ((Dv / 16) * kWave * 4 + 32) * sizeof(float) + page_bytes;
   if (heads_mode && merge_bytes > static_cast<size_t>(cap_lds_limit())) return static_cast<int>(hipErrorInvalidValue);
+  const int row_blocks = tokens / 16 + segments;                    // no fewer than the sixteen-row blocks of all segments
   const int wide_blocks = (row_blocks - segments) / 2 + segments;   // as row_blocks, of 32 rows
   const bool two = Dk <= 128 && Dv <= 128 && static_cast<long long>(wide_blocks) * nq >= kCapTwoBlocks &&
                    page_bytes + 2 * sizeof(int) <= 48 * 1024;
-  const int tokens_most = 16 * (row_blocks - segments) + 15;      // what row_blocks was counted from
-  const int blocks = tokens_most * group / kCpRows + segments;   // no fewer than the blocks of kCpRows rows of all segments
-  if (!heads_mode && cap_portions_take(a) && static_cast<long long>(blocks) * nkv >= kCapPortions) {
+  if (!heads_mode && cap_portions_take(a) && cap_portions_pay(tokens, segments, max_qlen, max_keys, group, nkv)) {
+    const int blocks = static_cast<int>(static_cast<long long>(tokens) * group / kCpRows) + segments;   // no fewer than there are
     if (r1 == nullptr) return launch_cap_portions<0>(a, blocks, s);
     return group == kCpTableGroup && window > 0 && window <= kCpTableMax ? launch_cap_portions<1>(a, blocks, s) : launch_cap_portions<2>(a, blocks, s);
   }

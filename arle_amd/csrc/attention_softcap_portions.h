@@ -138,7 +138,8 @@ __global__ __launch_bounds__(kCpWaves* kWave, 2) void cap_portions_kernel(const 
   if constexpr (PEN == 1) {
     const int hg = tid % kCpTableGroup;
     const float p1 = load_as_float(a.r1, a.r_dtype, kvh * G + hg), p2 = load_as_float(a.r2, a.r_dtype, kvh * G + hg);
-    for (int e = tid / kCpTableGroup; e < span; e += kCpWaves * kWave / kCpTableGroup)
+    // (of the distances that occur between this workgroup's rows and keys; what a masked lane reads elsewhere is dropped)
+    for (int e = max(0, span - (kv_hi - kv_lo)) + tid / kCpTableGroup; e < span; e += kCpWaves * kWave / kCpTableGroup)
       table_lds[e * kCpTableGroup + hg] = p1 * __builtin_amdgcn_logf(1.0f + p2 * static_cast<float>(span - 1 - e));
   }
 

@@ -81,8 +81,9 @@ SIGNATURES = {
                                                   _p, _p, _i, _i, _i, _i, _i, _i, _p]),
     "arle_attn_softcap_simt": ("attention_softcap", [_p, _ll, _p, _ll, _p, _p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _i, _i,
                                                      _f, _f, _p, _p, _i, _i, _i, _p, _i, _i, _f, _p]),
-    "arle_attn_softcap_mfma": ("attention_softcap", [_p, _ll, _p, _ll, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i,
+    "arle_attn_softcap_mfma": ("attention_softcap", [_p, _ll, _p, _ll, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i,
                                                      _i, _f, _f, _p, _p, _i, _i, _i, _p, _i, _i, _f, _p]),
+    "arle_attn_softcap_shares_tiles": ("attention_softcap", [_i, _i, _i, _i, _i, _i]),
     "arle_attn_softcap_lds_limit": ("attention_softcap", []),
     "arle_wide_norm_store": ("attention_softcap", [_p, _ll, _p, _ll, _p, _ll, _p, _ll, _i, _p, _p, _i, _p, _i, _f, _p, _p,
                                                    _p, _i, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i, _i, _p]),

@@ -2209,10 +2209,11 @@ def _softcap_lds_limit() -> int:
 def attn_softcap_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, seg_start, *, max_qlen: int,
                       num_q_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, page_size: int, scale: float,
                       softcap: float = 0.0, r1=None, r2=None, window: int = 0, chunk: int = 0, sink=None,
-                      keep_first: int = 0, out_scale: float = 1.0):
+                      keep_first: int = 0, out_scale: float = 1.0, max_kv_len: int = 0):
     """`attn_softcap_simt` on the matrix cores, bfloat16: sixteen or 32 rows of a segment a wave, or (when every segment is
     one decoded row) one row's q heads of a kv head, sixteen at a time, a wave.  keep_first (with a window and no
-    chunks): the request's first so many keys stay visible to rows whose window has passed them."""
+    chunks): the request's first so many keys stay visible to rows whose window has passed them.  max_kv_len: the longest context with
+    the step's rows, where the caller knows it (it helps to choose between kernels)."""
     _need(keep_first >= 0 and (keep_first == 0 or (window > 0 and chunk == 0)),
           "kept first keys go with a window and without chunks in the matrix-core kernel")
     _gpu(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, seg_start, r1, r2, sink)
@@ -2244,11 +2245,10 @@ def attn_softcap_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot,
     page_ids = _softcap_page_ids(mask_span(window, chunk), block_table.shape[1], page_size, keep_first)
     heads_mode = (max_qlen == 1 and segments == tokens
                   and 8 * ((value_dim // 16) * 256 + 32) * 4 + page_ids * 4 <= _softcap_lds_limit())
-    row_blocks = tokens // 16 + segments      # no fewer than the sixteen-row blocks of all segments together
     lib.call("arle_attn_softcap_mfma", q.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0), k_pages.data_ptr(),
              v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], seg_row0.data_ptr(), seg_slot.data_ptr(),
-             seg_start.data_ptr(), segments, row_blocks, 1 if heads_mode else 0, num_q_heads, num_kv_heads, key_dim,
-             value_dim, page_size, float(scale), float(softcap), _ptr(r1), _ptr(r2),
+             seg_start.data_ptr(), segments, tokens, int(max_qlen), max(0, int(max_kv_len)), 1 if heads_mode else 0, num_q_heads,
+             num_kv_heads, key_dim, value_dim, page_size, float(scale), float(softcap), _ptr(r1), _ptr(r2),
              _code(r1) if r1 is not None else 0, int(window), int(chunk), _ptr(sink),
              _code(sink) if sink is not None else 0, int(keep_first), float(out_scale), _stream())
     return out

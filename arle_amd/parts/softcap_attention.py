@@ -176,7 +176,7 @@ def softcap_attention(q, out, kv, batch, *, num_q_heads, num_kv_heads, key_dim, 
             and not (keep_first and chunk)
             and ops.attn_softcap_mfma_fits(ops.mask_span(window, chunk), kv.block_table.shape[1], kv.page_size, keep_first)):
         ops.attn_softcap_mfma(q, out, kv.pages["k"], kv.pages["v"], kv.block_table, batch.seg_row0, batch.seg_slot,
-                              batch.seg_start, max_qlen=batch.max_qlen, **common)
+                              batch.seg_start, max_qlen=batch.max_qlen, max_kv_len=batch.max_position + 1, **common)
     else:
         ops.attn_softcap_simt(q, out, kv.pages["k"], kv.pages["v"], kv.block_table, batch.positions,
                               batch.slot_of_token, **common)

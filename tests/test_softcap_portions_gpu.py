@@ -25,7 +25,8 @@ def _run(q, k_pages, v_pages, table, lens, contexts, nq, nkv, page, window, cap,
                                  r1=r1, r2=r2, window=window, out_scale=out_scale)
 
 
-def _inputs(lens, contexts, nkv, page, seed):
+def _inputs(lens, contexts, nkv, page, seed, window=0):
+    """Pages of keys and values; with a window, pages that no row sees any more have been given back (-1 in the table)."""
     g = torch.Generator().manual_seed(seed)
     need = [(c + n + page - 1) // page for c, n in zip(contexts, lens)]
     order = torch.randperm(sum(need), generator=g).to(torch.int32)
@@ -41,6 +42,7 @@ def _inputs(lens, contexts, nkv, page, seed):
         pages = table[i, where // page].long()
         k_pages[pages, :, where % page] = k
         v_pages[pages, :, :, where % page] = v
+        table[i, :max(0, c - window + 1) // page if window else 0] = -1
         keys.append(k)
         values.append(v)
     return g, table, k_pages, v_pages, keys, values
@@ -49,6 +51,8 @@ def _inputs(lens, contexts, nkv, page, seed):
 @pytest.mark.parametrize("lens,contexts,nq,nkv,page,window,cap,penalty,loud", [
     ([300, 70], [0, 100], 64, 16, 16, 100, 30.0, True, 1.0),        # the table
     ([200], [1500], 64, 16, 32, 1024, 30.0, True, 1.0),             # its longest window
+    ([40, 33, 1] * 6, [0, 5, 70] * 6, 64, 16, 16, 1000, 30.0, True, 1.0),   # the little of it that short contexts take
+    ([190], [2100], 64, 16, 64, 300, 30.0, True, 1.0),              # pages given back in front of the window
     ([200], [1500], 64, 16, 16, 1025, 30.0, True, 1.0),             # one more: computed
     ([400], [33], 64, 16, 16, 0, 30.0, True, 1.0),                  # no window: computed
     ([300, 31], [5, 64], 64, 32, 16, 40, 30.0, True, 1.0),          # a group of two
@@ -60,7 +64,7 @@ def _inputs(lens, contexts, nkv, page, seed):
     ([150, 1, 1, 40, 128], [3, 500, 63, 64, 0], 64, 16, 16, 70, 30.0, True, 1.0),
 ])
 def test_portions_whose_waves_share_tiles_match_64_bits(lens, contexts, nq, nkv, page, window, cap, penalty, loud):
-    g, table, k_pages, v_pages, keys, values = _inputs(lens, contexts, nkv, page, 11 + len(lens))
+    g, table, k_pages, v_pages, keys, values = _inputs(lens, contexts, nkv, page, 11 + len(lens), window)
     q = (torch.randn(sum(lens), nq * D, generator=g) * torch.linspace(0.1, loud, sum(lens))[:, None] if loud > 1.0
          else torch.randn(sum(lens), nq * D, generator=g)).bfloat16()
     r1, r2 = (torch.rand(nq, generator=g).bfloat16(), torch.rand(nq, generator=g).bfloat16()) if penalty else (None, None)

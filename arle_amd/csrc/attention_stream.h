@@ -28,8 +28,8 @@ constexpr int kInWgWavesMax = 4;
 // A workgroup's place in the launch is handed in: its segment, kv head and first row, and with INWG the number of its
 // waves, in how many parts the segment's keys are cut over workgroups (`parts`) and which of them this one takes;
 // without INWG, parts is the number of splits.  `handed`: LDS for what the waves of a workgroup hand to wave 0.
-constexpr int kHandedPitch = 4 * (128 / 16) + 4;   // floats a lane: its sums, m and l, and padding to 16 bytes (head_dim 128 at most)
-constexpr int kHandedFloats = (kInWgWavesMax - 1) * kWave * kHandedPitch;
+constexpr int handed_pitch(int head_dim) { return 4 * (head_dim / 16) + 4; }   // floats a lane: its sums, m and l, and padding to 16 bytes
+constexpr int handed_floats(int head_dim) { return (kInWgWavesMax - 1) * kWave * handed_pitch(head_dim); }
 template <int NT, int DMAX, bool EXACT, bool PREP, bool INWG, bool WHOLE_IN>
 __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const int kvh, const int row_begin, const int waves,
                                                const int parts, const int part, float* const handed) {
@@ -552,9 +552,10 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
   if constexpr (INWG) {
     // the waves behind the first hand their sums to wave 0, lane to lane (a lane holds the same rows and columns in
     // every wave): out = sum_s o_s 2^(m_s - m) / sum_s l_s 2^(m_s - m), added in the order of the splits
-    static_assert(4 * DTL + 4 <= kHandedPitch, "a lane's sums fit its place");
+    constexpr int kPitch = handed_pitch(DMAX);
+    static_assert(4 * DTL + 4 <= kPitch, "a lane's sums fit its place");
     if (my_wave > 0) {
-      float* mine = handed + ((my_wave - 1) * kWave + lane) * kHandedPitch;
+      float* mine = handed + ((my_wave - 1) * kWave + lane) * kPitch;
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt)
         *reinterpret_cast<float4*>(mine + 4 * dt) = float4{acc[0][dt][0], acc[0][dt][1], acc[0][dt][2], acc[0][dt][3]};
@@ -563,20 +564,21 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
     __syncthreads();
     if (my_wave > 0) return;
     for (int w = 1; w < waves; ++w) {
-      const float* theirs = handed + ((w - 1) * kWave + lane) * kHandedPitch;
+      const float* theirs = handed + ((w - 1) * kWave + lane) * kPitch;
       const float2 ml = *reinterpret_cast<const float2*>(theirs + 4 * DTL);
       const float m_all = fmaxf(m[0], ml.x);
       const float m_ref = m_all == -INFINITY ? 0.f : m_all;
       const float f0 = exp2f(m[0] - m_ref), f1 = exp2f(ml.x - m_ref);
-      l[0] = l[0] * f0 + ml.y * f1;
+      // (which product is rounded by itself is said here: left to the compiler it was another one from column to column)
+      l[0] = fmaf(l[0], f0, ml.y * f1);
       m[0] = m_all;
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt) {
         const float4 v = *reinterpret_cast<const float4*>(theirs + 4 * dt);
-        acc[0][dt][0] = acc[0][dt][0] * f0 + v.x * f1;
-        acc[0][dt][1] = acc[0][dt][1] * f0 + v.y * f1;
-        acc[0][dt][2] = acc[0][dt][2] * f0 + v.z * f1;
-        acc[0][dt][3] = acc[0][dt][3] * f0 + v.w * f1;
+        acc[0][dt][0] = fmaf(v.x, f1, acc[0][dt][0] * f0);
+        acc[0][dt][1] = fmaf(v.y, f1, acc[0][dt][1] * f0);
+        acc[0][dt][2] = fmaf(v.z, f1, acc[0][dt][2] * f0);
+        acc[0][dt][3] = fmaf(v.w, f1, acc[0][dt][3] * f0);
       }
     }
   }
@@ -624,7 +626,7 @@ template <int NT, int DMAX, bool EXACT, bool PREP = false, bool INWG = false, bo
 __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfma_kernel(const AttnArgs a) {
   const int z = static_cast<int>(blockIdx.z), row_begin = static_cast<int>(blockIdx.x) * (16 * NT);
   if constexpr (INWG) {
-    __shared__ __align__(16) float handed[kHandedFloats];
+    __shared__ __align__(16) float handed[handed_floats(DMAX)];
     attn_mfma_body<NT, DMAX, EXACT, PREP, true, WHOLE_IN>(a, z, blockIdx.y, row_begin, a.splits, 1, 0, handed);
   } else {
     attn_mfma_body<NT, DMAX, EXACT, PREP, false, WHOLE_IN>(a, z / a.splits, blockIdx.y, row_begin, 1, a.splits, z % a.splits, nullptr);

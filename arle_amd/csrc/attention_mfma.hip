@@ -344,7 +344,8 @@ static AttnArgs make_args(const void* q, long long q_stride, void* out, long lon
 // keys that a segment of more than one token holds after the step (it only steers choices of the portions kernels).  With splits > 1,
 // ws_o/ws_ml must hold [segments * ws_rows][nq][splits][D] and [..][2] floats, ws_rows = arle_attn_ws_rows(...),
 // and the merge runs after; the split is over the keys of segments of at most 16 rows (decoded tokens and
-// portions of a few tokens).  Longer portions go to the LDS kernel; when they have too few row blocks to fill
+// portions of a few tokens).  (Where the portions kernel takes them beside the portions a split is a workgroup of four waves, which merge
+// among themselves.)  Longer portions go to the LDS kernel; when they have too few row blocks to fill
 // the chip, portion_splits > 1 cuts the keys of every row block into that many parts (at most 8), pws_o/pws_ml
 // must hold [token rows][nq][portion_splits][D] and [..][2] floats, and a merge of their own runs after.
 // plan_token: 0, or a number that names the step (the same for every layer of it, another for every other step of
@@ -364,6 +365,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
   if (segments == 0 || token_rows == 0) return 0;
   if (D % 16 != 0 || D > 256 || D <= 0 || page_size < 4 || (page_size & (page_size - 1)) != 0 || nq % nkv != 0 ||
       splits < 1 || splits > 64 || portion_splits < 1 || portion_splits > kPortionPartsMax ||
+      (splits > 1 && (ws_o == nullptr || ws_ml == nullptr)) ||
       (portion_splits > 1 && (pws_o == nullptr || pws_ml == nullptr)))
     return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -388,12 +390,11 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
     const bool dma = D == 128 && page_size % 8 == 0 && static_cast<long long>(nkv) * page_size * D < (1LL << 31) &&
                      prefill_dma_pays(grid, max_qlen, max_kv_len);
     if (dma && min_rows <= 16) {
-      const int parts = splits / kDmWaves > 1 ? splits / kDmWaves : 1;   // of a segment's keys; each is four waves
       a.rows_max = 16;
-      rc = launch_prefill_beside(a, grid, 17, parts, segments - short_segments, max_kv_len, s);
-      if (rc != 0 || parts == 1) return rc;
+      rc = launch_prefill_beside(a, grid, 17, splits, segments - short_segments, max_kv_len, s);
+      if (rc != 0 || splits == 1) return rc;
       attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(
-          ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, a.rows_max, nq, nkv, D, parts, a.sink, a.out_scale, a.ws_plan);
+          ws_o, ws_ml, a.out, o_stride, seg_row0, a.ws_rows, a.rows_max, nq, nkv, D, splits, a.sink, a.out_scale, a.ws_plan);
       return launch_status();
     }
     SideBranch* side = (min_rows <= 16 && g_side_branch) ? side_branch(s) : nullptr;

@@ -380,15 +380,21 @@ def _compute_units(device_index: int) -> int:
     return int(torch.cuda.get_device_properties(device_index).multi_processor_count)
 
 
-def beside_splits(segments: int, num_kv_heads: int, max_kv_len: int, device) -> int:
-    """Over how many waves the keys of every short segment go (four a workgroup) in a step whose portions the same launch
+def takes_beside(max_qlen: int, min_qlen: int, group: int, num_kv_heads: int, head_dim: int, page_size: int) -> bool:
+    """Whether a step's short segments and its portions go to the portions kernel in one launch (csrc/attention_portions_dma.h)."""
+    return (head_dim == 128 and page_size % 8 == 0 and num_kv_heads * page_size * head_dim < 1 << 31
+            and min_qlen * group <= _ATTN_ROW_TILE < max_qlen * group)
+
+
+def beside_parts(segments: int, num_kv_heads: int, max_kv_len: int, device) -> int:
+    """Over how many workgroups (of four waves) the keys of every short segment go in a step whose portions the same launch
     takes: a workgroup of them for every compute unit at most, beside which a portion's workgroup fits, and 512 keys each.
     us a layer with 1 / 2 / 3 / 4 workgroups a segment and kv head (32 q heads over 8 kv heads): 32 requests at 1,024 tokens beside a
     portion of 512 36 / 51 / 49 / 55, 16 at 4,000 beside 512 behind 2,000 90 / 74 / 95 / 97, 8 at 2,048 beside 504 35 / 32 / 29 / 30,
     10 at 700 beside 333 18 / 22 / 24 / 24; 4 at 16,000 beside 512 with 1 / 4 / 8 of them 208 / 82 / 64."""
     units = _compute_units(device.index if device.index is not None else torch.cuda.current_device())
     keys = 1 << (max(int(max_kv_len), 1).bit_length() - 1)
-    return 4 * max(1, min(units // (segments * num_kv_heads), keys // 512, 16))
+    return max(1, min(units // (segments * num_kv_heads), keys // 512, 16))
 
 
 def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_heads: int, num_kv_heads: int,
@@ -449,7 +455,7 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
     position seg_start[s].  Segments whose rows (tokens x q heads of a kv head) fit one row tile of 16,
     decoded tokens above all, are split over the keys (split-KV), also beside longer portions in one
     step (at head_dim 128 in one launch with them); `short_segments` says how many there are (default: all), which sets
-    the number of splits.
+    the number of splits (beside portions at head_dim 128 a workgroup takes four of them).
     Longer portions that are too few to fill the chip have their keys cut into `portion_splits` parts
     (default: portion_key_splits).  `plan_token` (new_plan_token()) names the step: with the same token and the
     same segments the portions kernels list their work once, for the first layer, and not once a layer.
@@ -481,13 +487,14 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
     _i32(seg_start, "seg_start", segments)
     _need(1 <= min_qlen <= max_qlen <= tokens, "need 1 <= min_qlen <= max_qlen <= tokens")
     group = num_q_heads // num_kv_heads
+    short = segments if short_segments is None else max(1, min(short_segments, segments))
     if min_qlen * group > _ATTN_ROW_TILE:
         splits = 1                      # no segment is short enough for the kernel that splits the keys
+    elif takes_beside(max_qlen, min_qlen, group, num_kv_heads, head_dim, page_size):
+        # parts that are merged are workgroups there, whose four waves merge among themselves
+        splits = beside_parts(short, num_kv_heads, max_kv_len, q.device) if splits is None else max(1, splits // 4)
     elif splits is None:
-        short = segments if short_segments is None else max(1, min(short_segments, segments))
-        # beside portions in the kernel that takes both (csrc/attention_portions_dma.h), or in a launch of their own
-        both = max_qlen * group > _ATTN_ROW_TILE and head_dim == 128 and page_size % 8 == 0
-        splits = beside_splits(short, num_kv_heads, max_kv_len, q.device) if both else decode_splits(short, num_kv_heads, max_kv_len)
+        splits = decode_splits(short, num_kv_heads, max_kv_len)
     _need(segments * splits <= _GRID_Y_MAX and num_kv_heads <= _GRID_Y_MAX, "too many segments for one launch")
     ws_o = ws_ml = None
     if splits > 1:

@@ -505,6 +505,8 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
         long_segments = segments if short_segments is None else max(1, segments - short_segments)
         portion_splits = portion_key_splits(tokens, max_qlen, long_segments, num_q_heads, num_kv_heads, head_dim,
                                             max_portion_kv_len or max_kv_len, q.device)
+        if -(-max_qlen * group // _PORTION_ROWS) * segments > _PORTION_LIST_MAX:
+            portion_splits = 1          # parts need the list of pairs, which has no room for the short segments' as well
     if max_qlen * group <= _ATTN_ROW_TILE:
         portion_splits = 1              # no portion for the kernel that they are for
     _need(1 <= portion_splits <= _PORTION_SPLITS_MAX, f"portion_splits must be 1..{_PORTION_SPLITS_MAX}")

@@ -501,9 +501,9 @@ def test_kernels_refuse_what_they_were_not_written_for():
         ops.embed_gather(torch.zeros(4, 4, device=DEV), torch.zeros(2, dtype=torch.int64, device=DEV))
 
 
-def _mfma_case(nq, nkv, D, P, segs, window, splits, seed, portion_splits=None, stale_nan=False):
+def _mfma_case(nq, nkv, D, P, segs, window, splits, seed, portion_splits=None, stale_nan=False, short=None):
     """segs: [(cached length before the step, rows in the step)].  Returns (got, want) [T, nq*D].
-    stale_nan: every slot that no request has written holds NaN."""
+    stale_nan: every slot that no request has written holds NaN; short: how many segments the call is told are short."""
     dt = torch.bfloat16
     lengths = [a + b for a, b in segs]
     table, k_pages, v_pages = _paged_setup(lengths, nkv, D, P, dt, seed)
@@ -529,7 +529,7 @@ def _mfma_case(nq, nkv, D, P, segs, window, splits, seed, portion_splits=None, s
     ops.attn_paged_mfma(q_all, out, k_pages.to(DEV), v_pages.to(DEV), table.to(DEV), i32(row0),
                         i32(list(range(len(segs)))), i32(seg_start), max_qlen=max(n for _, n in segs), min_qlen=min(n for _, n in segs),
                         max_kv_len=max(lengths), num_q_heads=nq, num_kv_heads=nkv, head_dim=D, page_size=P,
-                        scale=1.0 / math.sqrt(D), window=window, splits=splits, portion_splits=portion_splits)
+                        scale=1.0 / math.sqrt(D), window=window, splits=splits, portion_splits=portion_splits, short_segments=short)
     return out.cpu(), torch.cat(wants)
 
 

@@ -114,3 +114,12 @@ def test_a_sink_and_a_factor_beside_portions(segs, splits):
                         num_kv_heads=nkv, head_dim=D, page_size=P, scale=D ** -0.5, splits=splits, sink=sink.to(DEV), out_scale=out_scale)
     for want, first, last in zip(wants, row0, row0[1:]):
         assert _rel(out[first:last].cpu(), want) < (8e-3 if last - first > 1 else 2.5e-2)
+
+
+def test_more_pairs_than_the_portions_list_holds():
+    """1,100 decoded tokens beside a portion whose keys would be cut into parts: its row blocks times all segments are more
+    than the list of pairs holds, without which there are no parts."""
+    segs = [(i % 5, 1) for i in range(1100)] + [(700, 500)]
+    got, want = _mfma_case(16, 4, 128, 16, segs, 0, None, 77, short=1100)
+    assert torch.isfinite(got).all()
+    assert _rel(got, want) < 8e-3 and _rel(got[-500:], want[-500:]) < 8e-3

@@ -419,8 +419,8 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
         two on, which also evens out causal row blocks.  Heads of 256, whole / 2 / 3 / 4 / 5 / 6 parts, behind 15,000, ms: 360 tokens (96) 7.0 / 4.0
         / 4.9 / 4.1 / 3.4 / 4.0, 512 (128) 8.1 / 4.8 / 5.8 / 4.6 / 5.1 / 4.4, 800 (200) 8.9 / 8.7 / 8.5 / 8.2 / 7.0 / 7.3, 832 (208) 9.0 / 8.8 / 8.6
         / 8.3 / 8.2 / 7.4, 900 (232) 8.3 / 8.4 / 8.3 / 8.4 / 8.4 / 8.5, and behind 1,500 1.24 / 1.11 / 1.16 / 1.18 / 1.22 / 1.26.
-    The number depends on the shape of the step and on the power-of-two class of the longest context only, up to 4,096, like the split
-    of decoded tokens, so that a captured step and an eager one choose alike.
+    The number depends on the shape of the step and on the power-of-two class of the longest context only, up to 4,096, so that a
+    growing context passes through few of them; a step replayed from its capture keeps the number that it was captured with.
     """
     group = num_q_heads // num_kv_heads
     blocks = -(-max_qlen * group // _PORTION_ROWS)

@@ -658,18 +658,21 @@ def test_attention_mfma_both_portion_kernels_at_head_dim_128(variant, nq, nkv, P
     rows a wave with tiles loaded straight into LDS, by one group of four waves or by two that take every other
     tile of keys each), chosen by the shape of the step; here each is forced in turn: portions that start inside a
     page after a cached prefix, whole prompts of several row blocks, a single first token and decoded tokens
-    beside them, windows, and keys cut into parts."""
+    beside them (which the second kernel takes in a launch of its own form, always with one group), windows, and keys cut
+    into parts."""
     from arle_amd.kernels import lib
     lib.function("arle_attn_prefill_variant")(min(variant, 1))
     lib.function("arle_attn_prefill_groups")(variant if variant else -1)
     try:
-        got, want = _mfma_case(nq, nkv, 128, P, [(300, 70), (45, 39), (0, 1), (130, 2), (0, 330), (77, 1)], window, 1,
-                               175, portion_splits=parts)
+        pairs = [_mfma_case(nq, nkv, 128, P, segs, window, 1, 175, portion_splits=parts)
+                 for segs in ([(300, 70), (45, 39), (0, 1), (130, 2), (0, 330), (77, 1)],
+                              [(300, 70), (45, 39), (0, 17), (130, 18), (0, 330), (77, 33)])]     # portions alone: both groups
     finally:
         lib.function("arle_attn_prefill_variant")(-1)
         lib.function("arle_attn_prefill_groups")(-1)
-    assert torch.isfinite(got).all()
-    assert _rel(got, want) < 8e-3
+    for got, want in pairs:
+        assert torch.isfinite(got).all()
+        assert _rel(got, want) < 8e-3
 
 
 @pytest.mark.parametrize("variant", [0, 1])
@@ -839,7 +842,8 @@ def test_decode_attention_with_the_preparation_folded_in(nq, nkv, D, rot, P, n_p
 
 @pytest.mark.parametrize("variant,groups,heads", [(1, 1, 24), (1, 2, 12), (0, -1, 12)])
 @pytest.mark.parametrize("parts", [None, 2])
-def test_attention_portions_dealt_out_before_the_launch_or_taken_from_the_counter(variant, groups, heads, parts):
+@pytest.mark.parametrize("few", [1, 20])     # a decoded token among the portions, or portions alone (with which both groups run)
+def test_attention_portions_dealt_out_before_the_launch_or_taken_from_the_counter(variant, groups, heads, parts, few):
     """Both portions kernels get their (row block, kv head, part) items either from a counter at run time or dealt
     out to and fro over the workgroups before the launch; the list of both is ordered by the keys an entry sees.
     Segments of very different lengths and contexts, more items than workgroups (so that a workgroup gets a second
@@ -848,7 +852,7 @@ def test_attention_portions_dealt_out_before_the_launch_or_taken_from_the_counte
     from arle_amd.kernels import lib
     nq = nkv = heads
     D, P, dt = 128, 16, torch.bfloat16
-    segs = [(100, 512), (0, 2048), (40, 1), (1500, 256), (700, 128)]
+    segs = [(100, 512), (0, 2048), (40, few), (1500, 256), (700, 128)]
     lengths = [a + b for a, b in segs]
     table, k_pages, v_pages = _paged_setup(lengths, nkv, D, P, dt, 410)
     qs, row0, starts, checks = [], [0], [], []
@@ -865,7 +869,7 @@ def test_attention_portions_dealt_out_before_the_launch_or_taken_from_the_counte
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
     q_all = torch.cat(qs).to(DEV)
     args = (k_pages.to(DEV), v_pages.to(DEV), table.to(DEV), i32(row0), i32(list(range(len(segs)))), i32(starts))
-    kw = dict(max_qlen=2048, min_qlen=1, max_kv_len=max(lengths), num_q_heads=nq, num_kv_heads=nkv, head_dim=D,
+    kw = dict(max_qlen=2048, min_qlen=few, max_kv_len=max(lengths), num_q_heads=nq, num_kv_heads=nkv, head_dim=D,
               page_size=P, scale=1.0 / math.sqrt(D), portion_splits=parts)
     lib.function("arle_attn_prefill_variant")(variant)
     lib.function("arle_attn_prefill_groups")(groups)
@@ -1352,12 +1356,13 @@ def test_measuring_kernels_give_plausible_ceilings():
             assert 2.5e14 < rate < 2.6e15
 
 
-@pytest.mark.parametrize("nq,nkv,D,P,splits", [(32, 8, 128, 16, 3), (4, 2, 16, 4, 1), (6, 2, 64, 8, 2)])
+@pytest.mark.parametrize("nq,nkv,D,P,splits", [(32, 8, 128, 4, 3), (32, 8, 96, 16, 3), (4, 2, 16, 4, 1), (6, 2, 64, 8, 2), (32, 8, 128, 16, 8)])
 def test_attention_decoded_tokens_on_a_side_branch_give_the_bits_of_one_stream(nq, nkv, D, P, splits):
     """In a mixed step the split-KV kernel of the decoded tokens and its merge run on a second stream beside the
     portions kernel (forked and joined by events).  With the branch and without it the result is the same bit for
     bit and right; a graph captured with the branch in it gives the same again on every replay, with eager calls
-    and synchronisations between the replays."""
+    and synchronisations between the replays.  (The last sizes have no branch: one launch takes both kinds of segments, and is
+    captured and replayed like the others.)"""
     from arle_amd.kernels import lib
     segs = [(300, 70), (45, 1), (0, 1), (130, 2), (0, 200), (77, 1), (511, 1)]
     results = {}

@@ -101,13 +101,9 @@ constexpr int kDealtMaxKeys = 4096;      // contexts up to which every launch de
 template <int DMAX, bool EXACT>
 int launch_prefill_lds(const AttnArgs& a, dim3 grid, int min_rows, int max_kv_len, hipStream_t s) {
   const size_t lds = prefill_lds_bytes(a.D);
-  static size_t allowed = 64 * 1024;  // dynamic LDS above 64 KiB has to be asked for, once per kernel
-  if (lds > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_lds_kernel<DMAX, EXACT>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (e != hipSuccess) return static_cast<int>(e);
-    allowed = lds;
-  }
+  static OnceADevice asked;
+  if (lds > 64 * 1024)
+    if (const int e = ask_lds(asked, prefill_lds_bytes(DMAX), {reinterpret_cast<const void*>(&attn_prefill_lds_kernel<DMAX, EXACT>)})) return e;
   static int cus = 0;
   if (cus == 0) {
     int dev = 0, n = 0;
@@ -138,18 +134,10 @@ template <int GROUPS, bool BESIDE = false>
 int launch_prefill_dma_groups(const AttnArgs& a, dim3 grid, int min_rows, int cus, int max_kv_len, hipStream_t s, int longs,
                               int beside_parts = 1) {
   const size_t lds = GROUPS * 2 * kDmStageBytes;
-  static bool asked = false;  // dynamic LDS of 64 KiB and more has to be asked for, once
-  if (!asked) {
-    for (const void* kernel : {reinterpret_cast<const void*>(&attn_prefill_dma_kernel<true, GROUPS, BESIDE>),
-                               reinterpret_cast<const void*>(&attn_prefill_dma_kernel<false, GROUPS, BESIDE>)}) {
-      hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-      if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return static_cast<int>(e);
-      }
-    }
-    asked = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, lds, {reinterpret_cast<const void*>(&attn_prefill_dma_kernel<true, GROUPS, BESIDE>),
+                                         reinterpret_cast<const void*>(&attn_prefill_dma_kernel<false, GROUPS, BESIDE>)}))
+    return e;
   const long long items = static_cast<long long>(grid.x) * grid.y * longs * a.portion_splits;
   const long long places = (GROUPS == 1 ? 2LL : 1LL) * cus;  // two workgroups of four waves a CU, or one of eight
   const int beside = BESIDE ? static_cast<int>(grid.z * grid.y) * beside_parts : 0;

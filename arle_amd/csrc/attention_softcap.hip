@@ -470,18 +470,11 @@ extern "C" int arle_wide_norm_store(void* q, long long q_stride, const void* k, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const size_t staged_bytes = rot ? static_cast<size_t>(nq > nkv ? nq : nkv) * Dk * sizeof(float) : 0;
   if (staged_bytes > 64 * 1024) return static_cast<int>(hipErrorInvalidValue);
-  if (staged_bytes > 48 * 1024) {
-    static bool raised = false;
-    if (!raised) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide_norm_store_kernel<float>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-      if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide_norm_store_kernel<bf16>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-      if (e != hipSuccess) return static_cast<int>(e);
-      raised = true;
-    }
-  }
+  static OnceADevice asked;
+  if (staged_bytes > 48 * 1024)
+    if (const int e = ask_lds(asked, 64 * 1024, {reinterpret_cast<const void*>(&wide_norm_store_kernel<float>),
+                                                 reinterpret_cast<const void*>(&wide_norm_store_kernel<bf16>)}))
+      return e;
   if (dtype == kF32) {
     wide_norm_store_kernel<float><<<grid, kWideThreads, staged_bytes, s>>>(
         static_cast<float*>(q), q_stride, static_cast<const float*>(k), k_stride, static_cast<const float*>(v), v_stride,
@@ -1017,14 +1010,12 @@ extern "C" int arle_attn_softcap_mfma(const void* q, long long q_stride, void* o
 #define ARLE_CAP(KC, VC)                                                                                           \
   do {                                                                                                             \
     if (heads_mode) {                                                                                              \
-      static bool raised = false;   /* more LDS than a launch gets unasked: said once for the kernel */            \
-      if (!raised && merge_bytes > 48 * 1024) {                                                                    \
+      static OnceADevice asked;                                                                                    \
+      if (merge_bytes > 48 * 1024) {                                                                               \
         const int most = kCapSplitWaves * (VC * kWave * 4 + 32) * 4 + 48 * 1024;                                   \
-        const hipError_t e = hipFuncSetAttribute(                                                                  \
-            reinterpret_cast<const void*>(&attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves, 1>),                \
-            hipFuncAttributeMaxDynamicSharedMemorySize, most < cap_lds_limit() ? most : cap_lds_limit());              \
-        if (e != hipSuccess) return static_cast<int>(e);                                                           \
-        raised = true;                                                                                             \
+        if (const int e = ask_lds(asked, most < cap_lds_limit() ? most : cap_lds_limit(),                          \
+                                  {reinterpret_cast<const void*>(&attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves, 1>)})) \
+          return e;                                                                                                \
       }                                                                                                            \
       attn_softcap_mfma_kernel<KC, VC, true, kCapSplitWaves, 1>                                                    \
           <<<dim3(segments, nkv * ((group + 15) / 16)), kCapSplitWaves * kWave, merge_bytes, s>>>(a);                                    \

@@ -370,15 +370,8 @@ inline bool cap_portions_take(const CapArgs& a) {
 template <int PEN>
 inline int launch_cap_portions(const CapArgs& a, int blocks, hipStream_t s) {
   constexpr int kBytes = 2 * kCpStage + (PEN == 1 ? kCpTable : 0);
-  static bool asked = false;   // dynamic LDS of 64 KiB and more has to be asked for, once
-  if (!asked) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cap_portions_kernel<PEN>), hipFuncAttributeMaxDynamicSharedMemorySize, kBytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return static_cast<int>(e);
-    }
-    asked = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, kBytes, {reinterpret_cast<const void*>(&cap_portions_kernel<PEN>)})) return e;
   cap_portions_kernel<PEN><<<static_cast<unsigned>(blocks) * a.nkv, kCpWaves * kWave, kBytes, s>>>(a);
   return launch_status();
 }

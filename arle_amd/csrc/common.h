@@ -8,6 +8,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
+#include "once_a_device.h"
+
 namespace arle {
 
 constexpr int kWave = 64;
@@ -188,6 +192,22 @@ __device__ __forceinline__ float gate_act(float z, int act) {
   if (act == kActSigmoid) return 1.0f / (1.0f + expf(-z));
   if (act == kActGeluTanh) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
   return z / (1.0f + expf(-z));
+}
+
+// Dynamic LDS beyond what a launch gets unasked has to be asked for, for every kernel and on every GPU: the attribute is the current
+// device's.  Returns a hipError_t, and leaves none behind for the next call to find.
+inline int ask_lds(OnceADevice& asked, size_t bytes, std::initializer_list<const void*> kernels) {
+  int device = -1;
+  hipError_t e = hipGetDevice(&device);
+  if (e == hipSuccess && asked.done(device)) return 0;
+  for (const void* kernel : kernels)
+    if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return static_cast<int>(e);
+  }
+  asked.mark(device);
+  return 0;
 }
 
 inline int launch_status() { return static_cast<int>(hipGetLastError()); }

@@ -342,16 +342,11 @@ extern "C" int arle_gated_group_norm(const float* y, const void* z, long long z_
     return launch_status();
   }
   const size_t lds = static_cast<size_t>(size) * sizeof(float);     // at most 64 KB
-  static bool raised = false;
-  if (!raised && lds > 48 * 1024) {
-    const void* kernels[] = {reinterpret_cast<const void*>(&gated_norm_kernel<float>),
-                             reinterpret_cast<const void*>(&gated_norm_kernel<bf16>)};
-    for (const void* f : kernels) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-      if (e != hipSuccess) return static_cast<int>(e);
-    }
-    raised = true;
-  }
+  static OnceADevice asked;
+  if (lds > 48 * 1024)
+    if (const int e = ask_lds(asked, 64 * 1024, {reinterpret_cast<const void*>(&gated_norm_kernel<float>),
+                                                 reinterpret_cast<const void*>(&gated_norm_kernel<bf16>)}))
+      return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == kF32)
     gated_norm_kernel<float><<<grid, kDsThreads, lds, s>>>(y, static_cast<const float*>(z), z_stride, w, eps, factor,

@@ -468,19 +468,13 @@ extern "C" int arle_gated_linear_chunks(const float* y, long long row_stride, co
   const size_t sum_lds = static_cast<size_t>(kChunkRows) * (DP + 4 + columns + 4) * sizeof(float);
   const size_t slices = static_cast<size_t>(kChunkRows + columns) * kGlSliceRow, last = static_cast<size_t>(kChunkRows) * (columns + 4 + kGlSliceRow);
   const size_t out_lds = (slices > last ? slices : last) * sizeof(float);
-  static bool raised = false;
-  if (!raised) {
-    const void* kernels[] = {reinterpret_cast<const void*>(&gated_linear_chunk_sum_kernel<4>),
-                             reinterpret_cast<const void*>(&gated_linear_chunk_sum_kernel<8>),
-                             reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<4>),
-                             reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<8>),
-                             reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<16>)};
-    for (const void* f : kernels) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
-      if (e != hipSuccess) return static_cast<int>(e);
-    }
-    raised = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, 144 * 1024, {reinterpret_cast<const void*>(&gated_linear_chunk_sum_kernel<4>),
+                                                reinterpret_cast<const void*>(&gated_linear_chunk_sum_kernel<8>),
+                                                reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<4>),
+                                                reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<8>),
+                                                reinterpret_cast<const void*>(&gated_linear_chunk_out_kernel<16>)}))
+    return e;
   const dim3 grid(items, H);
   if (columns == 64)
     gated_linear_chunk_sum_kernel<4><<<grid, kGlThreads, sum_lds, s>>>(a);

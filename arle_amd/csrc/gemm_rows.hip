@@ -409,16 +409,9 @@ int launch_rows(const RowsArgs& a, int splits, hipStream_t s) {
   const size_t lds = rows_lds_bytes(a.M, a.steps_per_split, MT, WN, WK);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
   auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, EPI, TOut>;
-  static size_t allowed = 64 * 1024;  // per instantiation: what the function may use so far
-  if (lds > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(kRowsLdsMax));
-    if (e != hipSuccess) {
-      (void)hipGetLastError();  // do not leave the error behind for the next call to find
-      return static_cast<int>(e);
-    }
-    allowed = kRowsLdsMax;
-  }
+  static OnceADevice asked;
+  if (lds > 64 * 1024)
+    if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
   const int col_groups = (a.N + WN * 16 - 1) / (WN * 16);
   kernel<<<dim3(col_groups, splits), WN * WK * 64, lds, s>>>(a);
   return launch_status();
@@ -430,16 +423,9 @@ int launch_rows_rounds(const RowsArgs& a, hipStream_t s) {
   const size_t lds = rows_lds_bytes(a.M, a.steps_per_round, MT, WN, WK);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
   auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, kEpiSiluMul, TOut, true>;
-  static size_t allowed = 64 * 1024;
-  if (lds > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(kRowsLdsMax));
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return static_cast<int>(e);
-    }
-    allowed = kRowsLdsMax;
-  }
+  static OnceADevice asked;
+  if (lds > 64 * 1024)
+    if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
   const int col_groups = (a.N + WN * 16 - 1) / (WN * 16);
   kernel<<<dim3(col_groups, 1), WN * WK * 64, lds, s>>>(a);
   return launch_status();
@@ -584,16 +570,9 @@ int launch_stream(const RowsArgs& a, int splits, int workgroups, hipStream_t s) 
   const size_t lds = stream_lds_bytes(a.M, a.steps_per_split, PD);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
   auto kernel = gemm_stream_kernel<MT, WN, PD, TOut>;
-  static size_t allowed = 64 * 1024;
-  if (lds > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(kRowsLdsMax));
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return static_cast<int>(e);
-    }
-    allowed = kRowsLdsMax;
-  }
+  static OnceADevice asked;
+  if (lds > 64 * 1024)
+    if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
   const int groups = (a.N + WN * 16 - 1) / (WN * 16);
   kernel<<<dim3(min(workgroups, groups), splits), WN * 64, lds, s>>>(a);
   return launch_status();

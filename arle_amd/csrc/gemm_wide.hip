@@ -354,16 +354,8 @@ int launch_wide(WideArgs a, int splits, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr size_t lds = NS * (BM + BN) * 128 + (NS == 2 ? 256 * WM * WN : 0);
   static_assert(lds <= 160 * 1024, "the stages fit the LDS");
-  static bool asked = false;   // more than 64 KiB of LDS has to be asked for, once
-  if (!asked) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return static_cast<int>(e);
-    }
-    asked = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, lds, {reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut>)})) return e;
   a.m_blocks = (a.M + BM - 1) / BM;
   a.n_blocks = (a.N + BN - 1) / BN;
   const long long grid = static_cast<long long>(a.m_blocks) * ((a.n_blocks + kWdXcds - 1) / kWdXcds) * kWdXcds;

@@ -191,13 +191,9 @@ static int launch_group_norm(const void* x, long long x_stride, float* back, con
     return launch_status();
   }
   const size_t lds = static_cast<size_t>(width + groups) * sizeof(float);
-  static bool raised = false;
-  if (!raised && lds > 48 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&group_norm_kernel<TIn, TOut, TW>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, kGroupLdsMax);
-    if (e != hipSuccess) return static_cast<int>(e);
-    raised = true;
-  }
+  static OnceADevice asked;
+  if (lds > 48 * 1024)
+    if (const int e = ask_lds(asked, kGroupLdsMax, {reinterpret_cast<const void*>(&group_norm_kernel<TIn, TOut, TW>)})) return e;
   group_norm_kernel<TIn, TOut, TW><<<n_rows, kGroupThreads, lds, s>>>(xp, x_stride, back, terms, wp, op, out_stride, rows,
                                                                       width, groups, eps, plain);
   return launch_status();

@@ -336,13 +336,9 @@ extern "C" int arle_head_proj(const void* in, long long in_stride, int in_head, 
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define ARLE_PROJ(TT)                                                                                              \
   do {                                                                                                             \
-    static bool raised = false;                                                                                    \
-    if (!raised && lds > 48 * 1024) {                                                                              \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&head_proj_kernel<TT>),               \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, kProjRows * 1024 * 4);  \
-      if (e != hipSuccess) return static_cast<int>(e);                                                             \
-      raised = true;                                                                                               \
-    }                                                                                                              \
+    static OnceADevice asked;                                                                                      \
+    if (lds > 48 * 1024)                                                                                           \
+      if (const int e = ask_lds(asked, kProjRows * 1024 * 4, {reinterpret_cast<const void*>(&head_proj_kernel<TT>)})) return e; \
     head_proj_kernel<TT><<<grid, kProjThreads, lds, s>>>(static_cast<const TT*>(in), in_stride, in_head,           \
                                                          static_cast<const TT*>(wt), static_cast<TT*>(out),        \
                                                          out_stride, out_head, rows, K, N);                        \

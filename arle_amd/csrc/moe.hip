@@ -669,13 +669,9 @@ extern "C" int arle_moe_route(const void* x, long long x_stride, int x_dtype, co
   if (lds > 80 * 1024) return static_cast<int>(hipErrorInvalidValue);
 #define ARLE_ROUTE_K(TX, TWT, V, TH, TK, EPL)                                                                          \
   do {                                                                                                                 \
-    static bool raised = false;                                                                                        \
-    if (!raised && lds > 48 * 1024) {                                                                                  \
-      const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_route_kernel<TX, TWT, V, TH, TK, EPL>), \
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);               \
-      if (err != hipSuccess) return static_cast<int>(err);                                                             \
-      raised = true;                                                                                                   \
-    }                                                                                                                  \
+    static OnceADevice asked;                                                                                          \
+    if (lds > 48 * 1024)                                                                                               \
+      if (const int err = ask_lds(asked, 80 * 1024, {reinterpret_cast<const void*>(&moe_route_kernel<TX, TWT, V, TH, TK, EPL>)})) return err; \
     moe_route_kernel<TX, TWT, V, TH, TK, EPL><<<(tokens + TK - 1) / TK, TH, lds, s>>>(                                 \
         static_cast<const TX*>(x), x_stride, static_cast<const TWT*>(w), bias, b_dtype, correction, c_dtype,           \
         static_cast<const TWT*>(shared_w), shared_gate, ids, weights, tokens, width, experts, top, rule);              \

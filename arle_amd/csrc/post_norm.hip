@@ -138,13 +138,9 @@ extern "C" int arle_norm_add(float* residual, const float* a, int a_parts, long 
                    (!b || (al(b) && b_part_stride % 4 == 0 && b_row_stride % 4 == 0)) && al(w) && al(act) && al(bias);
 #define ARLE_POST_V(TA, TWT, V)                                                                                \
   do {                                                                                                         \
-    static bool raised = false;                                                                                \
-    if (!raised && lds > 48 * 1024) {                                                                          \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_add_kernel<TA, TWT, V>),    \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);         \
-      if (e != hipSuccess) return static_cast<int>(e);                                                         \
-      raised = true;                                                                                           \
-    }                                                                                                          \
+    static OnceADevice asked;                                                                                  \
+    if (lds > 48 * 1024)                                                                                       \
+      if (const int e = ask_lds(asked, 64 * 1024, {reinterpret_cast<const void*>(&norm_add_kernel<TA, TWT, V>)})) return e; \
     norm_add_kernel<TA, TWT, V><<<rows, kPostThreads, lds, s>>>(residual, A, B, static_cast<const TWT*>(w),    \
                                                                 one_plus, center, static_cast<const TWT*>(bias), \
                                                                 mult, static_cast<TA*>(act), width, eps);      \

@@ -604,19 +604,13 @@ extern "C" int arle_retention_chunks(const float* y, long long row_stride, const
   const int columns = Dv <= 64 ? 64 : (Dv <= 128 ? 128 : 256);
   const size_t sum_lds = static_cast<size_t>(kChunk) * (DP + 4 + columns + 4) * sizeof(float);
   const size_t out_lds = (static_cast<size_t>(kChunk) * max(2 * kSliceRow, columns + 4) + static_cast<size_t>(columns) * kSliceRow) * sizeof(float);
-  static bool raised = false;
-  if (!raised) {
-    const void* kernels[] = {reinterpret_cast<const void*>(&retention_chunk_sum_kernel<4>),
-                             reinterpret_cast<const void*>(&retention_chunk_sum_kernel<8>),
-                             reinterpret_cast<const void*>(&retention_chunk_out_kernel<4>),
-                             reinterpret_cast<const void*>(&retention_chunk_out_kernel<8>),
-                             reinterpret_cast<const void*>(&retention_chunk_out_kernel<16>)};
-    for (const void* f : kernels) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
-      if (e != hipSuccess) return static_cast<int>(e);
-    }
-    raised = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, 144 * 1024, {reinterpret_cast<const void*>(&retention_chunk_sum_kernel<4>),
+                                                reinterpret_cast<const void*>(&retention_chunk_sum_kernel<8>),
+                                                reinterpret_cast<const void*>(&retention_chunk_out_kernel<4>),
+                                                reinterpret_cast<const void*>(&retention_chunk_out_kernel<8>),
+                                                reinterpret_cast<const void*>(&retention_chunk_out_kernel<16>)}))
+    return e;
   const dim3 grid(items, H);
   if (columns == 64)
     retention_chunk_sum_kernel<4><<<grid, kRetThreads, sum_lds, s>>>(a);

@@ -326,13 +326,9 @@ extern "C" int arle_rotary_qkv_store(void* q, long long q_stride, const void* k,
     if ((lanes + 255) / 256 <= 65535) {
       if (turned) {
         const size_t lds = static_cast<size_t>(kTurnRows) * (Dv + 2) * sizeof(uint16_t);     // at most 64 KB
-        static bool raised = false;
-        if (!raised && lds > 48 * 1024) {
-          const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&value_store_kernel),
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-          if (e != hipSuccess) return static_cast<int>(e);
-          raised = true;
-        }
+        static OnceADevice asked;
+        if (lds > 48 * 1024)
+          if (const int e = ask_lds(asked, 80 * 1024, {reinterpret_cast<const void*>(&value_store_kernel)})) return e;
         value_store_kernel<<<dim3((tokens + kTurnRows - 1) / kTurnRows, nkv), 256, lds, s>>>(
             static_cast<const bf16*>(v), v_stride, positions, slot_of_token, block_table, table_stride, static_cast<bf16*>(v_pages),
             tokens, nkv, Dv, page_size);

@@ -504,18 +504,12 @@ extern "C" int arle_state_space_chunks(const void* u, long long u_stride, const 
   const int nt = P <= 64 ? 1 : (P <= 128 ? 2 : 4), np = (N + 63) / 64 * 64;
   const size_t sum_lds = static_cast<size_t>(kChunkRows) * ((N + 15) / 16 * 16 + 3 * kSsTurned) * sizeof(bf16);
   const size_t out_lds = static_cast<size_t>(kChunkRows) * (np + 64 * nt + max(np, 3 * kChunkRows)) * sizeof(bf16);
-  static bool raised = false;
-  if (!raised) {
-    const void* kernels[] = {reinterpret_cast<const void*>(&state_space_chunk_sum_kernel),
-                             reinterpret_cast<const void*>(&state_space_chunk_out_kernel<1>),
-                             reinterpret_cast<const void*>(&state_space_chunk_out_kernel<2>),
-                             reinterpret_cast<const void*>(&state_space_chunk_out_kernel<4>)};
-    for (const void* f : kernels) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-      if (e != hipSuccess) return static_cast<int>(e);
-    }
-    raised = true;
-  }
+  static OnceADevice asked;
+  if (const int e = ask_lds(asked, 128 * 1024, {reinterpret_cast<const void*>(&state_space_chunk_sum_kernel),
+                                                reinterpret_cast<const void*>(&state_space_chunk_out_kernel<1>),
+                                                reinterpret_cast<const void*>(&state_space_chunk_out_kernel<2>),
+                                                reinterpret_cast<const void*>(&state_space_chunk_out_kernel<4>)}))
+    return e;
   const dim3 grid(items, H);
   state_space_chunk_sum_kernel<<<grid, kSsThreads, sum_lds, s>>>(a);
   state_space_chunk_carry_kernel<<<dim3(segments, H, (N / 4 * P + kSsThreads - 1) / kSsThreads), kSsThreads, 0, s>>>(a);

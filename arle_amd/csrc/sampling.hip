@@ -1479,8 +1479,10 @@ static inline int sample_chunk_len(int vocab, int chunks) { return (((vocab + ch
 static inline int sample_groups(int vocab, int chunks) { return (sample_chunk_len(vocab, chunks) + kGroup - 1) / kGroup; }
 extern "C" long long arle_sample_hist_k_bytes(int rows) { return static_cast<long long>(rows) * kRowBins * sizeof(unsigned int); }
 extern "C" long long arle_sample_hist_p_bytes(int rows) { return static_cast<long long>(rows) * kRowBins * sizeof(unsigned long long); }
-extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
+// finish != 0: for calls that the finishing kernel takes (arle_sample_rows), which keep the groups' maxima alone.
+extern "C" long long arle_sample_scratch_bytes(int rows, int vocab, int finish) {
   const int chunks = arle_argmax_chunks(rows, vocab);
+  if (finish) return static_cast<long long>(static_cast<size_t>(rows) * chunks * sample_groups(vocab, chunks) * sizeof(float));
   return arle_sample_hist_k_bytes(rows) + arle_sample_hist_p_bytes(rows) +
          static_cast<long long>(static_cast<size_t>(rows) * kPasses * sizeof(Slot) +
                                 static_cast<size_t>(rows) * chunks *
@@ -1492,7 +1494,7 @@ extern "C" long long arle_sample_scratch_bytes(int rows, int vocab) {
 extern "C" int arle_sample_finish_most() { return kFinishTopK; }
 
 // One token id per row of logits [rows, vocab] (float32).  probs is scratch [rows, vocab] float32; scratch holds
-// arle_sample_scratch_bytes(rows, vocab) bytes, 16-byte aligned.  use_top_k / use_top_p == 0 promise that no row of the call has
+// arle_sample_scratch_bytes(rows, vocab, whether two kernels do all) bytes, 16-byte aligned.  use_top_k / use_top_p == 0 promise that no row of the call has
 // the filter switched on (top_k in 1..vocab-1, top_p < 1); its passes are then left out.  small_k != 0 promises that every row is
 // greedy or has a top_k of 1 to arle_sample_finish_most(), below vocab: with vocab up to 2^28 two kernels then do all, probs may be
 // null, and with on_host != 0 temperature is a host array [5][rows] of the temperatures, top_p, min_p, u and the bits of top_k of up to
@@ -1518,6 +1520,26 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.top_p = top_p;
   a.min_p = min_p;
   a.u = u;
+  a.use_top_k = use_top_k;
+  a.use_top_p = use_top_p;
+  a.out = out;
+  const dim3 grid(a.chunks, rows);
+  if (small_k && use_top_k && vocab <= kFinishVocab) {
+    if (on_host && rows > kInlineRows) return static_cast<int>(hipErrorInvalidValue);
+    a.group_max = static_cast<float*>(scratch);
+    group_max_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, a.groups, a.group_max);
+    if (on_host) {
+      InlineRows values;
+      float* const to[4] = {values.temperature, values.top_p, values.min_p, values.u};
+      for (int i = 0; i < 4; ++i) std::memcpy(to[i], temperature + static_cast<size_t>(i) * rows, rows * sizeof(float));
+      std::memcpy(values.top_k, temperature + static_cast<size_t>(4) * rows, rows * sizeof(int));
+      sample_finish_kernel<InlineRows><<<rows, kFinishThreads, 0, s>>>(a, values);
+    } else {
+      sample_finish_kernel<NoRows><<<rows, kFinishThreads, 0, s>>>(a, NoRows{});
+    }
+    return launch_status();
+  }
+  if (on_host || probs == nullptr) return static_cast<int>(hipErrorInvalidValue);
   unsigned char* at = static_cast<unsigned char*>(scratch);
   a.hist_k = reinterpret_cast<unsigned int*>(at);
   at += arle_sample_hist_k_bytes(rows);
@@ -1533,25 +1555,6 @@ extern "C" int arle_sample_rows(const float* logits, int rows, int vocab, float*
   a.group_max = reinterpret_cast<float*>(at);
   at += static_cast<size_t>(rows) * a.chunks * a.groups * sizeof(float);
   a.threshold = reinterpret_cast<unsigned int*>(at);
-  a.use_top_k = use_top_k;
-  a.use_top_p = use_top_p;
-  a.out = out;
-  const dim3 grid(a.chunks, rows);
-  if (small_k && use_top_k && vocab <= kFinishVocab) {
-    if (on_host && rows > kInlineRows) return static_cast<int>(hipErrorInvalidValue);
-    group_max_kernel<<<grid, kChunkThreads, 0, s>>>(logits, vocab, a.chunk_len, a.groups, a.group_max);
-    if (on_host) {
-      InlineRows values;
-      float* const to[4] = {values.temperature, values.top_p, values.min_p, values.u};
-      for (int i = 0; i < 4; ++i) std::memcpy(to[i], temperature + static_cast<size_t>(i) * rows, rows * sizeof(float));
-      std::memcpy(values.top_k, temperature + static_cast<size_t>(4) * rows, rows * sizeof(int));
-      sample_finish_kernel<InlineRows><<<rows, kFinishThreads, 0, s>>>(a, values);
-    } else {
-      sample_finish_kernel<NoRows><<<rows, kFinishThreads, 0, s>>>(a, NoRows{});
-    }
-    return launch_status();
-  }
-  if (on_host || probs == nullptr) return static_cast<int>(hipErrorInvalidValue);
   // the histograms of the filters that are on start at zero
   const int k_row = kRowBins * sizeof(unsigned int) / 16, p_row = kRowBins * sizeof(unsigned long long) / 16;
   const ClearRows clear{reinterpret_cast<uint4*>(a.hist_k), reinterpret_cast<uint4*>(a.hist_p), use_top_k ? k_row : 0, k_row,

@@ -52,7 +52,7 @@ SIGNATURES = {
                                                 _i, _i, _i, _f, _i, _i, _p, _p, _i, _p, _p, _ll, _p, _f, _i, _p]),
     "arle_argmax_chunks": ("sampling", [_i, _i]),
     "arle_argmax_rows": ("sampling", [_p, _i, _i, _p, _p, _p]),
-    "arle_sample_scratch_bytes": ("sampling", [_i, _i]),
+    "arle_sample_scratch_bytes": ("sampling", [_i, _i, _i]),
     "arle_sample_finish_most": ("sampling", []),
     "arle_sample_host_rows": ("sampling", []),
     "arle_sample_rows": ("sampling", [_p, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p]),

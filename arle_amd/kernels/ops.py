@@ -691,10 +691,10 @@ def token_logprobs(logits: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
 
 
 @functools.lru_cache(maxsize=None)
-def _sample_scratch_bytes(rows: int, vocab: int) -> int:
+def _sample_scratch_bytes(rows: int, vocab: int, finish: bool) -> int:
     fn = lib.function("arle_sample_scratch_bytes")
     fn.restype = ctypes.c_longlong
-    return int(fn(rows, vocab))
+    return int(fn(rows, vocab, int(finish)))
 
 
 @functools.lru_cache(maxsize=None)
@@ -739,7 +739,7 @@ def sample_rows(logits, temperature, top_k=None, top_p=None, min_p=None, u=None,
         params = [t.data_ptr() for t in (temperature, top_k, top_p, min_p, u)]
     probs = None if finish else torch.empty((rows, vocab), dtype=torch.float32, device=logits.device)
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
-    scratch = torch.empty((-(-_sample_scratch_bytes(rows, vocab) // 8),), dtype=torch.int64, device=logits.device)
+    scratch = torch.empty((-(-_sample_scratch_bytes(rows, vocab, finish) // 8),), dtype=torch.int64, device=logits.device)
     lib.call("arle_sample_rows", logits.data_ptr(), rows, vocab, _ptr(probs), *params, out.data_ptr(), scratch.data_ptr(),
              int(bool(use_top_k)), int(bool(use_top_p)), int(bool(small_k)), int(on_host), _stream())
     return out

@@ -58,3 +58,21 @@ def test_parameters_in_host_memory_are_refused_where_they_cannot_travel():
         ops.sample_rows(logits[:4], np.ones((5, 4), dtype=np.float32))                # the passes read them on the GPU
     with pytest.raises(ops.ShapeError):
         ops.sample_rows(logits[:4], np.ones((4, 4), dtype=np.float32), small_k=True)
+
+
+def test_a_call_allocates_the_groups_maxima_alone():
+    from arle_amd.kernels import ops
+
+    rows, vocab = 64, 151936
+    logits = torch.randn(rows, vocab, device="cuda")
+    packed = np.full((5, rows), 0.5, dtype=np.float32)
+    packed.view(np.int32)[4] = 50
+    call = lambda: ops.sample_rows(logits, packed, small_k=True)
+    first = call()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    assert torch.equal(call(), first)
+    chunks = ops.lib.function("arle_argmax_chunks")(rows, vocab)
+    groups = -(-(-(-vocab // chunks) + 3) // 64) + 1
+    assert torch.cuda.max_memory_allocated() - before <= 4 * rows * chunks * groups + 4096

@@ -14,11 +14,12 @@ namespace arle {
 // What bounds it is arithmetic: a score takes the cap, the penalty, an exponential, a maximum and a sum, and quarter-rate
 // instructions cost as much as four others.  So
 //   * the cap is a polynomial where all scores of a wave's tile lie within half of it: cap tanh(x / cap) = x P((x / cap)^2) with the
-//     minimax P of degree 4 for tanh(t) / t over |t| <= 0.5 (off by 1.3e-8; six multiply-adds where the exponential and the
-//     reciprocal take 44 cycles), and the exponential form elsewhere;
+//     minimax P of degree 4 for tanh(t) / t over |t| <= 0.5 (off by 2.6e-8, and t P from tanh by 1.3e-8; six multiply-adds where
+//     the exponential and the reciprocal take 44 cycles), and the exponential form elsewhere;
 //   * the distance penalties of a group of four heads come from a table in LDS, filled once a workgroup for windows of up
 //     to 1,024 (PEN 1; the heads side by side, so that the lanes of a wave spread over the banks, and distances descending,
-//     so that a lane's sixteen keys are one base and sixteen constants); other groups and windows compute them (PEN 2);
+//     so that a lane's sixteen keys are one base and sixteen constants); other groups and windows compute them (PEN 2: the same layer
+//     in groups of two 73 us, of eight 72, by waves of their own 107 and 106; without a window 89 and 162);
 //   * masks are worked out in the tiles at the ends only, and sums are rescaled only where a maximum has grown by 2^8.
 // A layer of 2,048 rows of 32 q heads and 8 kv heads, window 1,024, cap and penalty: 66 us, 110 with every wave fetching its tiles
 // by itself into registers (attn_softcap_mfma_kernel, 32 rows a wave); without the penalty 60, with neither 50.  What a wave spends is

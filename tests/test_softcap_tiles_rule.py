@@ -1,7 +1,12 @@
-"""Which steps of the soft-capped attention at heads of 128 go to the kernel whose waves share their tiles, as far as sizes decide it."""
+"""Which steps of the soft-capped attention at heads of 128 go to the kernel whose waves share their tiles, as far as sizes decide it;
+the polynomial that this kernel caps scores with."""
+import math
+import os
+import re
+
 import pytest
 
-from arle_amd.kernels import lib, ops
+from arle_amd.kernels import build, lib, ops
 
 
 def _shares(lens, context, heads, kv_heads, known=True):
@@ -38,3 +43,16 @@ def test_decoded_rows_beside_a_portion_share_tiles_by_their_contexts():
 def test_the_lines_lie_where_captured_steps_tell_contexts_apart():
     for line in (96, 224):
         assert ops.decode_split_cap(line) < ops.decode_split_cap(line + 1)
+
+
+def test_the_caps_polynomial_is_as_far_off_as_it_says():
+    with open(os.path.join(build.CSRC_DIR, "attention_softcap_portions.h")) as fh:
+        text = fh.read()
+    said, said_of_tanh = map(float, re.search(r"off by ([\d.e-]+), and t P from tanh by ([\d.e-]+);", text).groups())
+    powers = [float(re.search(rf"c{n} = (-?[\d.]+)f \* sq", text).group(1)) for n in (1, 2, 3, 4)]
+    off = off_of_tanh = 0.0
+    for i in range(1, 20001):
+        t = 0.5 * i / 20000
+        p = 1.0 + sum(c * t ** (2 * n) for n, c in enumerate(powers, 1))
+        off, off_of_tanh = max(off, abs(p - math.tanh(t) / t)), max(off_of_tanh, abs(t * p - math.tanh(t)))
+    assert 0.9 * said < off < 1.1 * said and 0.9 * said_of_tanh < off_of_tanh < 1.1 * said_of_tanh

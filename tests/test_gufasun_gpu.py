@@ -378,6 +378,36 @@ def test_captured_steps_give_the_bits_of_eager_ones(folders):
     assert all(torch.equal(out[True][k], out[False][k]) for k in out[False])
 
 
+def test_portions_and_single_rows_of_heads_of_128_eager_and_captured(folders, monkeypatch):
+    """Portions long enough for the kernel whose waves share their tiles, twice over (the windows have passed the first pages by the
+    second one, and they are given back), then single rows through the convolution that stores, in the layer that owns the pages and
+    in the one that reads them: eager and captured steps give the plain logits, and the same bits."""
+    from arle_amd.kernels import lib, ops
+
+    cfg, weights = read_folder(folders["U"])
+    reqs = requests_for(cfg, (580, 571), 500)
+    assert all(lib.function("arle_attn_softcap_shares_tiles")(n, 1, n, 300, 64, 16) for n in (290, 281))
+    steps = []
+    for rid, toks in reqs.items():
+        n = (len(toks) - 10) // 2 + 1
+        steps += [{"entries": [(rid, toks[i:min(i + n, len(toks) - 10)], list(range(min(n, len(toks) - 10 - i))))], "end": []}
+                  for i in (0, n)]
+    for i in range(10, 0, -1):
+        steps.append({"entries": [(rid, [toks[-i]], [0]) for rid, toks in reqs.items()], "end": list(reqs) if i == 1 else []})
+    stored, store = [], ops.conv_step_store
+    monkeypatch.setattr(ops, "conv_step_store", lambda u, *a, **k: stored.append(k["num_kv_heads"]) or store(u, *a, **k))
+    out = {}
+    for graphs in (False, True):
+        stored.clear()
+        eng = engine_for(folders["U"], "U", "bfloat16", 1200, slots=2, cuda_graph=graphs)
+        out[graphs] = replay.run_steps(eng, steps)
+        assert (eng.graph_replays > 0) == graphs
+        assert {16, 0} == set(stored) and (graphs or len(stored) == 20)
+    ref = references(cfg, weights, reqs)
+    replay.check_rows(out[False], ref, MODEL_TOL["bfloat16"], "gufasun U", outlier_tol=SPREAD["bfloat16"])
+    assert all(torch.equal(out[True][k], out[False][k]) for k in out[False])
+
+
 def _plain_greedy(cfg, weights, prompt, n):
     toks = list(prompt)
     for _ in range(n):

@@ -8,6 +8,7 @@ mLSTM head, no convolution on q, k and v in one layer, a value size that is no m
 R: wider heads (a key size over 64, a value size over 64 that is no multiple of 64) and windows of several pages.
 S: nothing but matrix memories (no paged cache at all).  T: nothing but attention, five q heads a kv head, a key size
 that is a multiple of 8 only, a reader right behind its owner, and no feed-forward anywhere.
+U: heads of 128 in groups of four, many of them, four taps, a reader: the kernels that are made for such heads.
 """
 from __future__ import annotations
 
@@ -65,9 +66,15 @@ TINY_T = {"architecture": ARCH, "vocab": 150, "width": 60, "norm": {"eps": 1e-5}
           "layers": [layer("attention", attention(5, 1, 24, 48, window=19, conv=3), None),
                      layer("attention", attention(5, 1, 24, 48, window=50, conv=4, softcap=0.0, coef=0.0, kv_from=0), None)]}
 
+TINY_U = {"architecture": ARCH, "vocab": 130, "width": 64, "norm": {"eps": 1e-5}, "embedding": {"scale": 4.0},
+          "canon": {"taps": 4},
+          "layers": [layer("attention", attention(64, 16, 128, 128, window=40, conv=4, scale=0.09, every=16), 96),
+                     layer("mlstm", mlstm(2, 16, 16), 96),
+                     layer("attention", attention(64, 16, 128, 128, window=70, conv=4, scale=0.07, softcap=3.0, kv_from=0), 96)]}
+
 # name -> (config, page size, weight std, norm std, seed)
 TINY = {"P": (TINY_P, 4, 0.15, 0.1, 5), "Q": (TINY_Q, 8, 0.2, 0.2, 6), "R": (TINY_R, 16, 0.1, 0.1, 7),
-        "S": (TINY_S, 16, 0.2, 0.1, 8), "T": (TINY_T, 16, 0.2, 0.1, 9)}
+        "S": (TINY_S, 16, 0.2, 0.1, 8), "T": (TINY_T, 16, 0.2, 0.1, 9), "U": (TINY_U, 16, 0.1, 0.1, 10)}
 
 
 def make_model_dir(tmp_path, name: str) -> str:

@@ -290,6 +290,47 @@ __global__ __launch_bounds__(NT) void add_layernorm_vec_kernel(
   }
 }
 
+// Workgroups as wide as the row where that is more than 2,048 elements: nearly every load of a row is then on its way at once
+// and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
+// 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
+// wide 8.2 / 6.2, 2,048 rows 68.7 / 60.8.  Narrower rows need several a compute unit (1,536 wide, 2,048 rows 20.0 / 27.1), and
+// so do many rows beyond 5,120: 6,144 wide 8 rows 8.4 / 7.8, 256 9.5 / 9.5, 512 19.6 / 17.7, 1,536 48.4 / 46.8, 2,048 62.2 / 60.7,
+// 4,096 139.5 / 158.9; 8,192 wide 8.7 / 7.9, 11.3 / 10.6, 23.6 / 20.1, 62.6 / 55.2, 87.6 / 86.6, 172.7 / 177.5 (elsewhere 2,048 rows 86.2 /
+// 89.8).  In bfloat16: a float32 row's sums have one order in every step, so the width alone chooses there.
+struct LnShape {
+  int threads, per_lane;   // lanes a row, groups of four elements a lane
+};
+constexpr LnShape ln_shape(int width, int n_rows, bool f32, int taps) {
+  if (width <= 2048) return {256, width <= 1024 ? 1 : 2};
+  if (width <= 2560) return {640, 1};
+  if (width <= 4096) return {1024, 1};
+  if (width <= 5120) return {640, 2};
+  if (width <= 8192) return f32 || n_rows < 2048 || taps > 0 ? LnShape{1024, 2} : LnShape{256, 8};
+  return {256, 16};
+}
+
+// How many parts of both terms a lane fetches together: two or eight where the registers hold them (ln_holds), else one term after
+// the other; the order of the sums is the same.
+// MI355X, terms of 4 and 6 parts / 1 and 2 / 1 and 1, us, term after term with the parts past the last fetched again / as here: 8 rows
+// of 2,560 4.9, 4.1, 3.6 / 4.1, 3.4, 3.3, with the convolution 5.6, 4.7, 4.2 / 4.6, 3.9, 3.9; 2,048 rows - 23.9, 19.7 / - 21.5, 18.8
+// (126 and 105 MB); 8 rows of 5,120 6.9, 5.3, 4.3 / 5.7, 4.2, 4.1; 2,048 rows - 50.1, 37.0 / - 38.7, 33.2; 512 rows of 8,192 - 20.5, 17.0
+// / - 18.9, 16.9.  (Eight parts of eight float32 elements a lane spill: 8 rows of 5,120 7.0 / 9.1.)
+constexpr bool ln_holds(int threads, int per_lane, int taps, bool f32, int parts) {
+  return parts == 2 ? per_lane <= 2 && !(per_lane == 2 && threads > 640 && taps > 0)
+                    : per_lane == 1 || (per_lane == 2 && taps == 0 && (threads <= 256 || (threads <= 640 && !f32)));
+}
+// Eight at a time pay while the rows wait for one trip to memory; with more rows than the chip has at work at once it is the rows beside
+// each other that hide the trips, and the registers of eight parts leave room for fewer.  MI355X, bfloat16, us, one term after the other /
+// eight together: 2,560 wide, terms of 6 and 6 parts, 64 rows 4.6 / 4.1, 256 6.7 / 6.0, 384 10.8 / 11.5, 1,024 24.2 / 25.6, one of 3 parts 256
+// rows 4.3 / 3.8, 1,024 11.8 / 13.4; 4,096 wide, 6 parts, 256 5.5 / 5.1, 384 10.4 / 11.2, 2,048 41.7 / 48.1; 1,024 wide, 6 and 6, 768 8.2 / 7.7,
+// 1,024 11.0 / 11.2, 2,048 19.3 / 21.9; 2,048 wide, 256 5.2 / 4.6, 384 9.1 / 9.3 (8 parts 5.2 / 4.8), 512 11.3 / 12.1.  Workgroups of 640 lanes with
+// two groups each (5,120 wide) are level or ahead at all rows: 6 parts, 512 rows 16.9 / 16.4, 2,048 62.8 / 60.7.
+constexpr int ln_ahead(int threads, int per_lane, int taps, bool f32, int parts, int n_rows) {
+  if (parts <= 2) return ln_holds(threads, per_lane, taps, f32, 2) ? 2 : 0;
+  const int rows_most = threads <= 256 ? 768 / per_lane : (per_lane == 1 ? 256 : 1 << 30);
+  return parts <= 8 && n_rows <= rows_most && ln_holds(threads, per_lane, taps, f32, 8) ? 8 : 0;
+}
+
 template <typename TA>
 static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, const void* wa, const void* wb, void* out_a,
                          void* out_b, const int* rows, int n_rows, int width, float eps, const void* ca, const void* cb,
@@ -302,11 +343,11 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
       width, eps, static_cast<const TA*>(ca), static_cast<const TA*>(cb), conv)
 #define ARLE_LNV_CT(NT, PER4, CT)                                                     \
   do {                                                                                \
-    constexpr int two = PER4 <= 2 && !(PER4 == 2 && NT > 640 && CT > 0) ? 2 : 0;      \
-    constexpr bool fits = PER4 == 2 && CT == 0 && (NT <= 256 || (NT <= 640 && std::is_same<TA, bf16>::value)); \
-    constexpr int more = PER4 == 1 || fits ? 8 : 0;                                   \
-    if (two && parts <= two) ARLE_LNV_U(NT, PER4, CT, two);                           \
-    else if (more && parts <= more) ARLE_LNV_U(NT, PER4, CT, more);                   \
+    constexpr bool f32 = std::is_same<TA, float>::value;                              \
+    constexpr int two = ln_holds(NT, PER4, CT, f32, 2) ? 2 : 0, eight = ln_holds(NT, PER4, CT, f32, 8) ? 8 : 0; \
+    const int ahead = ln_ahead(NT, PER4, CT, f32, parts, n_rows);                     \
+    if (two && ahead == 2) ARLE_LNV_U(NT, PER4, CT, two);                             \
+    else if (eight && ahead == 8) ARLE_LNV_U(NT, PER4, CT, eight);                    \
     else ARLE_LNV_U(NT, PER4, CT, 0);                                                 \
   } while (0)
 #define ARLE_LNV(NT, PER4)                                                            \
@@ -314,32 +355,22 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
     if (taps == 0) ARLE_LNV_CT(NT, PER4, 0); else if (taps == 2) ARLE_LNV_CT(NT, PER4, 2); \
     else if (taps == 3) ARLE_LNV_CT(NT, PER4, 3); else ARLE_LNV_CT(NT, PER4, 4);      \
   } while (0)
-  // How many parts of both terms a lane fetches together: two or eight where the registers hold them, else one term after the other.
-  // MI355X, terms of 4 and 6 parts / 1 and 2 / 1 and 1, us, term after term with the parts past the last fetched again / as here: 8 rows
-  // of 2,560 4.9, 4.1, 3.6 / 4.1, 3.4, 3.3, with the convolution 5.6, 4.7, 4.2 / 4.6, 3.9, 3.9; 2,048 rows - 23.9, 19.7 / - 21.5, 18.8
-  // (126 and 105 MB); 8 rows of 5,120 6.9, 5.3, 4.3 / 5.7, 4.2, 4.1; 2,048 rows - 50.1, 37.0 / - 38.7, 33.2; 512 rows of 8,192 - 20.5, 17.0
-  // / - 18.9, 16.9.  (Eight parts of eight float32 elements a lane spill: 8 rows of 5,120 7.0 / 9.1.)
   const int parts = max(t0.data ? t0.n_stack : 0, t1.data ? t1.n_stack : 0);
-  // Workgroups as wide as the row where that is more than 2,048 elements: nearly every load of a row is then on its way at once
-  // and few are of the row's end again.  MI355X, terms of one and two parts (six up to 64 rows), 256 lanes / as here, us:
-  // 2,560 wide, 8 rows 6.0 / 4.7, 2,048 39.3 / 32.7, 8,192 146.8 / 109.4; 4,096 wide 6.1 / 5.7, 45.9 / 40.7, 172.8 / 152.0; 5,120
-  // wide 8.2 / 6.2, 2,048 rows 68.7 / 60.8.  Narrower rows need several a compute unit (1,536 wide, 2,048 rows 20.0 / 27.1), and
-  // so do many rows beyond 5,120: 6,144 wide 8 rows 8.4 / 7.8, 256 9.5 / 9.5, 512 19.6 / 17.7, 1,536 48.4 / 46.8, 2,048 62.2 / 60.7,
-  // 4,096 139.5 / 158.9; 8,192 wide 8.7 / 7.9, 11.3 / 10.6, 23.6 / 20.1, 62.6 / 55.2, 87.6 / 86.6, 172.7 / 177.5 (elsewhere 2,048 rows 86.2 /
-  // 89.8).  In bfloat16: a float32 row's sums have one order in every step, so the width alone chooses there.
-  if (width <= 1024) {
+  const LnShape shape = ln_shape(width, n_rows, std::is_same<TA, float>::value, taps);
+  const int lanes = shape.threads, each = shape.per_lane;
+  if (lanes == 256 && each == 1) {
     ARLE_LNV(256, 1);
-  } else if (width <= 2048) {
+  } else if (lanes == 256 && each == 2) {
     ARLE_LNV(256, 2);
-  } else if (width <= 2560) {
+  } else if (lanes == 640 && each == 1) {
     ARLE_LNV(640, 1);
-  } else if (width <= 4096) {
+  } else if (lanes == 1024 && each == 1) {
     ARLE_LNV(1024, 1);
-  } else if (width <= 5120) {
+  } else if (lanes == 640) {
     ARLE_LNV(640, 2);
-  } else if (width <= 8192 && (std::is_same<TA, float>::value || n_rows < 2048 || taps > 0)) {
+  } else if (lanes == 1024) {
     ARLE_LNV(1024, 2);
-  } else if (width <= 8192) {
+  } else if (each == 8) {
     if constexpr (!std::is_same<TA, float>::value) ARLE_LNV_CT(256, 8, 0);
   } else {
     ARLE_LNV_CT(256, 16, 0);
@@ -353,6 +384,12 @@ static int launch_ln_vec(float* residual, const LnTerm& t0, const LnTerm& t1, co
 }  // namespace arle
 
 using namespace arle;
+
+// How many parts of both terms a lane of the vector form fetches together (0: one term after the other); parts: the larger of the two stacks.
+extern "C" int arle_layernorm_parts_ahead(int width, int n_rows, int parts, int taps, int dtype) {
+  const LnShape shape = ln_shape(width, n_rows, dtype == kF32, taps);
+  return ln_ahead(shape.threads, shape.per_lane, taps, dtype == kF32, parts, n_rows);
+}
 
 // residual float32 [T, width] contiguous.  term*: null, [T, width] (n_stack 1) or a stack; bias*: null or [width].
 // out_a, out_b (out_b and wb may be null): [n_rows, width] contiguous of out_dtype.  width <= 16384.

@@ -60,6 +60,7 @@ SIGNATURES = {
     "arle_token_logprobs": ("sampling", [_p, _i, _i, _p, _p, _p]),
     "arle_attn_decode_static": ("attention_mfma", [_p, _ll, _p, _ll, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i,
                                                    _i, _f, _i, _i, _p]),
+    "arle_layernorm_parts_ahead": ("layernorm", [_i, _i, _i, _i, _i]),
     "arle_add_layernorm": ("layernorm", [_p, _p, _i, _ll, _i, _p, _i, _p, _i, _ll, _i, _p, _i, _p, _p, _i, _p, _p, _i, _p, _i,
                                          _i, _f, _p, _p, _p]),
     "arle_add_layernorm_conv": ("layernorm", [_p, _p, _i, _ll, _p, _p, _i, _ll, _p, _p, _p, _p, _p, _i, _i, _i, _f, _p, _p, _p, _p, _p, _i, _p]),

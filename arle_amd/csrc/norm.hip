@@ -187,11 +187,14 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(TIn* __restri
 // workgroups) added into the residual row, then the norm.  Few rows make few workgroups here, so the
 // time is the latency of the loads: a workgroup owns a row, every thread one group of four columns (THREADS: the waves that the
 // width takes, up to 1,024 threads), and the loads of the whole stack, UNROLL parts at a time, are in flight together: four for
-// stacks of up to four, else eight (six parts as a round of four and one behind it were two trips to memory, and 1,024
+// stacks of up to four, else mostly eight (six parts as a round of four and one behind it were two trips to memory, and 1,024
 // threads for 2,560 columns six idle waves to start: whole decode steps of the Qwen3-4B shape 2,461 -> 2,436 us with one request,
 // 2,985 -> 2,956 with 19).
 // Only the parts that there are are fetched: fetching the last one again for those past the end cost 8 rows of 2,560 with six parts
 // 3.2 us, so 3.0, with two 2.8 / 2.7; 97 rows 3.4 / 3.2.
+// Rounds of four again for stacks of eight and more under many rows, which hide each other's trips and want the registers (us, eight / four at
+// a time: 1,024 rows of 2,048, nine parts 18.3 / 16.8, sixteen 28.5 / 25.8; 2,048 rows of 4,096, nine 70.3 / 68.1; level up to 512 rows; of
+// five or six parts 2,048 wide 1,024 rows 11.0 and 13.6 / 11.7 and 12.7, 4,096 wide 19.8 and 22.6 / 19.9 and 22.2).
 // Order of addition: residual + (delta 0 + delta 1 + ...), as in the kernels above; idle waves would add zeros to the
 // sum of squares, so the threads do not change a bit.
 constexpr int kStackThreads = 1024;
@@ -279,6 +282,7 @@ int launch_add_rmsnorm(float* residual, const void* delta, int n_delta, long lon
   if constexpr (sizeof(TD) == 4) {
     if (n_delta > 1 && vec_ok(width, width, residual, delta, w, out) && delta_stride % 4 == 0 &&
         width <= 4 * kStackThreads) {
+      const bool four = n_delta <= 4 || (n_delta >= 8 && n_rows > 512);
 #define ARLE_STACK(TW, THREADS, UNROLL)                                                                             \
   add_stack_rmsnorm_kernel<TOut, TW, THREADS, UNROLL><<<n_rows, THREADS, 0, s>>>(                                   \
       residual, static_cast<const float*>(delta), n_delta, delta_stride, static_cast<const TW*>(w),                  \
@@ -290,9 +294,9 @@ int launch_add_rmsnorm(float* residual, const void* delta, int n_delta, long lon
     else ARLE_STACK(TW, kStackThreads, UNROLL);                                                                     \
   } while (0)
       if (w_dtype == kF32) {
-        if (n_delta <= 4) ARLE_STACK_WIDTH(float, 4); else ARLE_STACK_WIDTH(float, 8);
+        if (four) ARLE_STACK_WIDTH(float, 4); else ARLE_STACK_WIDTH(float, 8);
       } else {
-        if (n_delta <= 4) ARLE_STACK_WIDTH(bf16, 4); else ARLE_STACK_WIDTH(bf16, 8);
+        if (four) ARLE_STACK_WIDTH(bf16, 4); else ARLE_STACK_WIDTH(bf16, 8);
       }
 #undef ARLE_STACK_WIDTH
 #undef ARLE_STACK

@@ -54,3 +54,22 @@ def test_wide_rows():
     assert _ahead(5120, 1 << 20, 8) == 8 and _ahead(5120, 1, 8, dtype=F32) == 0      # eight float32 parts would spill there
     assert _ahead(5120, 1, 8, taps=4) == 0 and _ahead(8192, 1, 8) == 0 and _ahead(8192, 1, 2, taps=4) == 0
     assert _ahead(16384, 1, 1) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [1024, 2560, 4096])
+@pytest.mark.parametrize("parts", [7, 8, 9, 17])
+def test_rms_rows_are_the_same_bits_on_both_sides_of_the_line(width, parts):
+    from arle_amd.kernels import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(width + parts)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    residual, stack, weight = rand(513, width), rand(parts, 513, width), rand(width)
+    sums, few = residual.clone(), residual[1:].clone()
+    whole = ops.add_rmsnorm(sums, stack, weight, 1e-6, torch.float32)
+    less = ops.add_rmsnorm(few, stack[:, 1:].contiguous(), weight, 1e-6, torch.float32)
+    assert torch.equal(whole[1:], less) and torch.equal(sums[1:], few)
+    plain = residual.double() + stack.double().sum(0)
+    plain = plain / (plain.square().mean(-1, keepdim=True) + 1e-6).sqrt() * weight.double()
+    # a sum of up to eighteen terms in 32 bits, and a sum of squares over the row
+    assert ((whole.double() - plain).abs() <= 2e-6 * (plain.abs() + 1)).all()

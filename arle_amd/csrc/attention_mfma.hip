@@ -205,20 +205,11 @@ int launch_prefill_beside(const AttnArgs& a, dim3 grid, int min_rows, int parts,
   return launch_prefill_dma_groups<1, true>(a, grid, min_rows, cus, max_kv_len, s, longs > 0 ? longs : 1, parts);
 }
 
-// -1: the launcher decides (below); 1: head_dim 128 portions always run attn_prefill_dma_kernel; 0: always
-// attn_prefill_lds_kernel, as every other head_dim does.  For measurements and tests that compare the two.
+// 0: head_dim 128 portions run attn_prefill_lds_kernel, as those of every other head_dim do; else attn_prefill_dma_kernel, whatever their
+// sizes: its 32 rows a wave do a tile in two thirds of the time, and inside whole prefill steps of the Qwen3-4B shape it is level with
+// the other one for a fresh prompt of 512 tokens and 3 to 5 % of the step ahead for portions of 512 behind 512 to 3,584 cached
+// tokens.  For measurements and tests that compare the two.
 static int g_prefill_dma = -1;
-
-// The kernel with 32 rows a wave does a tile in two thirds of the time.  Measured inside whole prefill steps of the
-// Qwen3-4B shape it is level with the other one for a fresh prompt of 512 tokens and 3 to 5 % of the step ahead
-// for portions of 512 behind 512 to 3,584 cached tokens, so it takes every portion that it can.
-inline bool prefill_dma_pays(dim3 grid, int max_qlen, int max_kv_len) {
-  (void)grid;
-  (void)max_qlen;
-  (void)max_kv_len;
-  if (g_prefill_dma >= 0) return g_prefill_dma != 0;
-  return true;
-}
 
 }  // namespace arle
 
@@ -375,8 +366,7 @@ extern "C" int arle_attn_paged_mfma(const void* q, long long q_stride, void* out
     // prompt portions through the LDS kernel; segments of at most 16 rows (decoded tokens of a mixed
     // step) through the streaming kernel
     dim3 grid((max_rows + kPfRows - 1) / kPfRows, nkv, segments);
-    const bool dma = D == 128 && page_size % 8 == 0 && static_cast<long long>(nkv) * page_size * D < (1LL << 31) &&
-                     prefill_dma_pays(grid, max_qlen, max_kv_len);
+    const bool dma = D == 128 && page_size % 8 == 0 && static_cast<long long>(nkv) * page_size * D < (1LL << 31) && g_prefill_dma != 0;
     if (dma && min_rows <= 16) {
       a.rows_max = 16;
       rc = launch_prefill_beside(a, grid, 17, splits, segments - short_segments, max_kv_len, s);

@@ -77,7 +77,9 @@ __global__ __launch_bounds__(NT) void polynorm_vec_kernel(const void* __restrict
 #pragma unroll
     for (int k = 0; k < PER4; ++k) z[k] = ld4<float>(at + min((tid + k * NT) * 4, last));
     // Parts at a time (a jump that all lanes take together waits for no load); two of seven accesses each, or three in float32, cost
-    // many rows more in waves a SIMD than they gain (2,048 rows of 12,288, one part, 24.9 us / 29.9).
+    // many rows more in waves a SIMD than they gain (2,048 rows of 12,288, one part, 24.9 us / 29.9).  Where three are taken, 4,096 wide
+    // keeps four waves a SIMD for eight, 9,728 wide four for seven, and many rows are level: 2,048 rows of one, three and six parts, one at a
+    // time / three, 10.6 / 10.1, 19.0 / 18.9, 32.8 / 33.2 and 21.0 / 19.8, 42.8 / 41.5, 98.0 / 97.5; 64 rows of three parts 3.8 / 3.4 and 5.0 / 4.3.
     constexpr int G = !std::is_same<T, float>::value && PER4 <= 5 ? 3 : 1;
     for (int s0 = 1; s0 < parts; s0 += G) {
       float4 e[G][PER4];

@@ -135,7 +135,9 @@ __global__ __launch_bounds__(kPrepWaves* kWave) void qk_prep_kernel(
 // lane moves, or shuffles where there is no move of that distance.  Bound by memory for many tokens, by one trip to it for few, as
 // long as no load stands under a lane's condition and both halves of a rotation are the same instructions (a branch a column
 // before): 32 + 2 * 8 heads of 128, 97 tokens 5.8 -> 4.3 us, 2,048 13.7 -> 10.3, 8,192 37.8 -> 34.5 (5.8 TB/s); heads of 64 at 2,048
-// 7.9 -> 5.8; of 256 13.7 -> 8.4.  Only half of a head of 128 rotated: 2,048 11.8 -> 10.3, 8,192 32.5 / 34.6.  A value head is only moved: its pages keep the head's columns as rows ([D][page_size]),
+// 7.9 -> 5.8; of 256 13.7 -> 8.4.  Only half of a head of 128
+// rotated, 512, 2,048, 8,192 and 16,384 tokens 7.3 / 5.6, 12.0 / 10.7, 34.5 / 34.7 (without a norm 33.5 / 34.3, where what is read
+// just fits the last cache) and 75.5 / 72.2.  A value head is only moved: its pages keep the head's columns as rows ([D][page_size]),
 // so when the workgroup's tokens are one run of consecutive positions of one request that starts at a
 // multiple of 16 (the usual case in a prompt portion), the tile is turned in LDS and written as 16-byte
 // pieces of eight slots; otherwise every element goes to its slot by itself.

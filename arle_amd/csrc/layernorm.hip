@@ -314,7 +314,8 @@ constexpr LnShape ln_shape(int width, int n_rows, bool f32, int taps) {
 // MI355X, terms of 4 and 6 parts / 1 and 2 / 1 and 1, us, term after term with the parts past the last fetched again / as here: 8 rows
 // of 2,560 4.9, 4.1, 3.6 / 4.1, 3.4, 3.3, with the convolution 5.6, 4.7, 4.2 / 4.6, 3.9, 3.9; 2,048 rows - 23.9, 19.7 / - 21.5, 18.8
 // (126 and 105 MB); 8 rows of 5,120 6.9, 5.3, 4.3 / 5.7, 4.2, 4.1; 2,048 rows - 50.1, 37.0 / - 38.7, 33.2; 512 rows of 8,192 - 20.5, 17.0
-// / - 18.9, 16.9.  (Eight parts of eight float32 elements a lane spill: 8 rows of 5,120 7.0 / 9.1.)
+// / - 18.9, 16.9, of one term of one part 14.1 / 13.1.  Only rows of 4,096 with two terms of one part, of which there are many, lose: 512
+// 8.8 / 8.4, 2,048 28.6 / 29.6, 4,096 51.9 / 52.5, and so they do one term after the other (2,048 29.8).  (Eight parts of eight float32 elements a lane spill: 8 rows of 5,120 7.0 / 9.1.)
 constexpr bool ln_holds(int threads, int per_lane, int taps, bool f32, int parts) {
   return parts == 2 ? per_lane <= 2 && !(per_lane == 2 && threads > 640 && taps > 0)
                     : per_lane == 1 || (per_lane == 2 && taps == 0 && (threads <= 256 || (threads <= 640 && !f32)));

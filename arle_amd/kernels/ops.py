@@ -398,7 +398,7 @@ def beside_parts(segments: int, num_kv_heads: int, max_kv_len: int, device) -> i
 
 
 def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_heads: int, num_kv_heads: int,
-                       head_dim: int, max_kv_len: int, device) -> int:
+                       head_dim: int, max_kv_len: int, device, beside: bool = False, window: int = 0) -> int:
     """Into how many parts the keys of every row block of a prompt portion are cut.
 
     The portions kernels give a row block of 128 rows (tokens x q heads of a kv head) to a workgroup, and a compute unit
@@ -410,6 +410,9 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
         parts: a portion of 512 tokens behind 512 26 / 28 / 29, behind 1,024 34 / 32 / 32, behind 3,584 72 / 55 / 54; of 100 behind 2,000
         56 / 36 / 24; of 300 behind 3,000 60 / 43 / 49 (3 parts: 37); of 512 beside 32 requests that decode at 1,024, behind 0, 512,
         1,024 and 1,536: 36 / 41, 43 / 43, 54 / 46 and 68 / 52.
+        At head_dim 128 two parts become four or five from 4,096 keys on, which fit one turn of two workgroups a unit; that evens out a launch
+        with decoded tokens in it: two / four or five, behind 7,000 and 15,000, 352 tokens 71, 67 / 132, 121, beside 4 decoded ones 94, 76 / 174,
+        125; 512 tokens 83, 85 / 153, 152, beside them 99, 90 / 185, 160.
       * up to two thirds of the units: three parts in two turns, up to three quarters: four in three.  Behind 3,100 / 7,000 / 15,000, whole and
         cut: 520 tokens (136 row blocks) at heads of 64 75, 61 / 146, 108 / 290, 204, of 96 149, 111 / 295, 209 / 590, 408, of 128 67, 57 / 125,
         96 / 248, 179; 768 tokens (192) at heads of 64 81, 76 / 151, 144 / 295, 250 (behind 1,500 52, 54), of 96 159, 137 / 305, 253 /
@@ -419,25 +422,46 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
         two on, which also evens out causal row blocks.  Heads of 256, whole / 2 / 3 / 4 / 5 / 6 parts, behind 15,000, ms: 360 tokens (96) 7.0 / 4.0
         / 4.9 / 4.1 / 3.4 / 4.0, 512 (128) 8.1 / 4.8 / 5.8 / 4.6 / 5.1 / 4.4, 800 (200) 8.9 / 8.7 / 8.5 / 8.2 / 7.0 / 7.3, 832 (208) 9.0 / 8.8 / 8.6
         / 8.3 / 8.2 / 7.4, 900 (232) 8.3 / 8.4 / 8.3 / 8.4 / 8.4 / 8.5, and behind 1,500 1.24 / 1.11 / 1.16 / 1.18 / 1.22 / 1.26.
-    The number depends on the shape of the step and on the power-of-two class of the longest context only, up to 4,096, so that a
-    growing context passes through few of them; a step replayed from its capture keeps the number that it was captured with.
+    Several portions differ in rows and contexts, of which only the longest are known here, and the launch lasts as long as the few row blocks
+    that see the most keys: the turns of equal ones say little (100 tokens behind 7,000 beside 20 behind 15,000 at heads of 64: 139 us in two
+    parts, 76 in four, 47 in eight).  They take what fits one turn by the rows that there are, and no fewer than two a unit of
+    1,024 keys each.  us a layer, by turns / so: 8 q heads a kv head of 64, 2 kv heads, 512 fresh, 600 behind 1,500 and 20 behind 15,000 277 /
+    106; 32 over 8 of 128, 20 behind 7,000 and 450 behind 3,000 155 / 71, 450 behind 3,000 and 450 fresh 82 / 61; over 276 steps of two to six
+    portions 1.10 and 0.92 of the time of two a unit alone, which none of them exceeds.  Portions that are all alike lose by it where their
+    turns had been even: two of 333 behind 7,000, heads of 128, 117 / 128, two of 450 behind 3,000, heads of 64, 71 / 77.
+    beside: the launch has decoded tokens in it as well, and its row blocks go to four waves each, where portions alone have eight for a row
+    block a unit: of several portions row blocks for up to one and a half a unit are cut too, from 4,096 keys on.  512 tokens behind 15,000 and 512 behind
+    2,000 beside one decoded token (256 row blocks), launches of their own / here whole / in two parts, 259 / 327 / 195, beside four 368 / 328 / 193;
+    two of 512 behind 7,000 163 / 176 / 148; over 40 q heads (320) 242 / 217 / 222.
+    window: a row sees no more keys than that, which is what more parts than one turn are for (512 and 1,024: 768 tokens behind 7,000 at heads of
+    64 whole 19 and 29, in four parts 50 and 52, 512 tokens at heads of 128 in two 26 and 30, in four 27 and 32, beside decoded ones 30 and 37, 39 and
+    45; 300 tokens and 60 at heads of 96, window 1,024, whole, in two and in four 53, 39, 45).
+    The number depends on the shape of the step and on the power-of-two class of the longest context only, of one portion up to 4,096, so that
+    a growing context passes through few of them; a step replayed from its capture keeps the number that it was captured with.
     """
     group = num_q_heads // num_kv_heads
     blocks = -(-max_qlen * group // _PORTION_ROWS)
     items = blocks * num_kv_heads * max(1, long_segments)
     units = _compute_units(device.index if device.index is not None else torch.cuda.current_device())
-    if items >= units or blocks * max(1, long_segments) > _PORTION_LIST_MAX:
-        return 1
     keys = 1 << (max(int(max_kv_len), 1).bit_length() - 1)
+    seen = min(keys, window) if window > 0 else keys
+    cut = 2 * items <= 3 * units if beside and long_segments > 1 and seen >= 4096 else items < units
+    if not cut or blocks * max(1, long_segments) > _PORTION_LIST_MAX:
+        return 1
     most = min(_PORTION_SPLITS_MAX, keys // 512)
     turns = lambda parts: -(-items * parts // units)
-    if head_dim > 128:
+    if long_segments > 1:
+        there = min(items, (tokens * group // _PORTION_ROWS + long_segments) * num_kv_heads)    # no fewer than there are
+        parts = max(1, min(units // there, most), min(-(-2 * units // items), _PORTION_SPLITS_MAX, seen // (512 if window > 0 else 1024)))
+    elif head_dim > 128:
         parts = min(range(2, most + 1), key=lambda p: (turns(p) / p, p), default=1)
     else:
         parts = max(1, min(units // items, most))
-        if parts == 1 and turns(3) == 2 and keys >= 3 * 512:
+        if parts == 1 and turns(3) == 2 and seen >= 3 * 512:
             parts = 3
-        elif parts == 1 and turns(4) == 3 and head_dim != 128 and keys >= 4 * (1024 if head_dim == 64 else 512):
+        elif parts == 2 and head_dim == 128 and seen >= 4096:
+            parts = 2 * units // items
+        elif parts == 1 and turns(4) == 3 and head_dim != 128 and seen >= 4 * (1024 if head_dim == 64 else 512):
             parts = 4
     while parts > 1 and tokens * num_q_heads * parts * (head_dim + 2) * 4 > _PORTION_WS_BYTES:
         parts -= 1
@@ -504,7 +528,8 @@ def attn_paged_mfma(q, out, k_pages, v_pages, block_table, seg_row0, seg_slot, s
     if portion_splits is None:
         long_segments = segments if short_segments is None else max(1, segments - short_segments)
         portion_splits = portion_key_splits(tokens, max_qlen, long_segments, num_q_heads, num_kv_heads, head_dim,
-                                            max_portion_kv_len or max_kv_len, q.device)
+                                            max_portion_kv_len or max_kv_len, q.device,
+                                            takes_beside(max_qlen, min_qlen, group, num_kv_heads, head_dim, page_size), int(window))
         if -(-max_qlen * group // _PORTION_ROWS) * segments > _PORTION_LIST_MAX:
             portion_splits = 1          # parts need the list of pairs, which has no room for the short segments' as well
     if max_qlen * group <= _ATTN_ROW_TILE:

@@ -413,6 +413,8 @@ def portion_key_splits(tokens: int, max_qlen: int, long_segments: int, num_q_hea
         At head_dim 128 two parts become four or five from 4,096 keys on, which fit one turn of two workgroups a unit; that evens out a launch
         with decoded tokens in it: two / four or five, behind 7,000 and 15,000, 352 tokens 71, 67 / 132, 121, beside 4 decoded ones 94, 76 / 174,
         125; 512 tokens 83, 85 / 153, 152, beside them 99, 90 / 185, 160.
+        Where the decoded tokens alone fill the chip the parts are one row block more to wait for: 64 requests at 2,048 beside 600 tokens behind 1,500 127
+        whole, 144 in three; 16 over 16 kv heads beside 1,000 tokens behind 7,000 129 in two, 141 in four.
       * up to two thirds of the units: three parts in two turns, up to three quarters: four in three.  Behind 3,100 / 7,000 / 15,000, whole and
         cut: 520 tokens (136 row blocks) at heads of 64 75, 61 / 146, 108 / 290, 204, of 96 149, 111 / 295, 209 / 590, 408, of 128 67, 57 / 125,
         96 / 248, 179; 768 tokens (192) at heads of 64 81, 76 / 151, 144 / 295, 250 (behind 1,500 52, 54), of 96 159, 137 / 305, 253 /

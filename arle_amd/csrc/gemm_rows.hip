@@ -57,6 +57,11 @@ struct RowsArgs {
   int steps_per_round;   // ROUNDS: k steps of 32 whose X rows are in LDS at one time (the slice is walked in rounds)
 };
 
+__device__ __forceinline__ bf16x8 load_w16(const uint16_t* p) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
+}
+
 // W as operand tiles: [ceil(N/16)][ceil(K/32)][64 lanes][8], tile (t, s) lane 16 g + i = W[16 t + i][32 s + 8 g .. +7],
 // zeros past N and K.  A wave's load of one k step is then one contiguous kilobyte and its stream through a
 // column tile one contiguous run, instead of sixteen 64-byte pieces a row apart: measured 4.5 against 3.6 TB/s
@@ -105,7 +110,7 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
     const int w_step = a.tiled ? 512 : 32, w_first = a.tiled ? 0 : 8 * g, w_last = a.tiled ? (steps_total - 1) * 512 : K - 8;
     auto load_w = [&](int s) {
       const int e = min(w_step * s + w_first, w_last);  // clamped: always inside the row (the column tile)
-      return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(wrow + e));
+      return load_w16(wrow + e);
     };
 
     // the first PD steps of W are on their way before anything else happens; without a condition (a step past
@@ -300,7 +305,7 @@ __global__ __launch_bounds__(WN * 64) void gemm_stream_kernel(const RowsArgs a) 
   const int w_step = a.tiled ? 512 : 32, w_first = a.tiled ? 0 : 8 * g, w_last = a.tiled ? (steps_total - 1) * 512 : K - 8;
   auto load_w = [&](const uint16_t* row, int s) {  // s: step inside the slice (may reach past it, not past K)
     const int e = min(w_step * (s_begin + s) + w_first, w_last);
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + e));
+    return load_w16(row + e);
   };
   const uint16_t* wcur = w_row(blockIdx.x);
   bf16x8 ring[PD];

@@ -57,6 +57,11 @@ struct RowsArgs {
   int steps_per_round;   // ROUNDS: k steps of 32 whose X rows are in LDS at one time (the slice is walked in rounds)
 };
 
+// Every byte of W is read by one wave of the launch: it is loaded past the caches, where it would only displace what is read
+// again.  MI355X, cold weights, us, kept / past the caches: 19,456 x 2,560 with the activation at 9 rows 21.3 / 20.7, 2,560 x
+// 9,728 at 9 rows 11.2 / 10.6, 151,936 x 2,560 at 9 rows 142 / 125; decode steps of the Qwen3-4B shape at 1 and 8 requests
+// 2,440 / 2,381 and 2,837 / 2,756.  Not in gemm_stream_kernel, which
+// measured slower with it (2,560 x 4,096 at 9 and 16 rows 7.1 / 7.3 and 7.2 / 7.5).
 __device__ __forceinline__ bf16x8 load_w16(const uint16_t* p) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(WN * 64) void gemm_stream_kernel(const RowsArgs a) 
   const int w_step = a.tiled ? 512 : 32, w_first = a.tiled ? 0 : 8 * g, w_last = a.tiled ? (steps_total - 1) * 512 : K - 8;
   auto load_w = [&](const uint16_t* row, int s) {  // s: step inside the slice (may reach past it, not past K)
     const int e = min(w_step * (s_begin + s) + w_first, w_last);
-    return load_w16(row + e);
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + e));
   };
   const uint16_t* wcur = w_row(blockIdx.x);
   bf16x8 ring[PD];

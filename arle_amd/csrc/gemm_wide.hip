@@ -16,6 +16,8 @@
 //     with two stages and lines touched ahead 32.7 (128 x 96, 97 rows: 30.6 / 34.9; 128 x 160, 160 rows 33.4 / 37.7); a sixth stage and
 //     more change nothing.  From operand tiles, whose kilobytes lie whole in memory where rows are 128 bytes each 5 KB apart,
 //     64 rows take 23.7 us for 26.8, 128 rows 29.5 for 32.7, 256 rows 35.0 for 38.7; from 544 rows on the two are level.
+//   * Weights that one row block reads (ONCE) are loaded past the caches: whole steps of the Qwen3-4B shape, 19 requests 2,908 ->
+//     2,856 us, 64 requests 5,743 -> 5,661, a prompt of 97 tokens 3,387 -> 3,194.
 //   * Latency of what comes from memory in the large shapes: with two stages a fetch has one stage's time (1.2 to 1.8 us), which
 //     a miss of the L2 under load does not keep to.  There every wave touches, four stages ahead, a few of the 128-byte lines that its
 //     XCD's workgroups will fetch (a dword a line, into a corner of LDS that nobody reads): 2,048 rows 223 -> 186 us, 8,192
@@ -67,6 +69,11 @@ __device__ __forceinline__ void wide_load(const uint16_t* base, uint32_t lane_by
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_at), "v"(lane_bytes), "s"(base)
                : "memory", "m0");
 }
+// The same for what no other workgroup reads: past the caches, where it would only displace what is read again.
+__device__ __forceinline__ void wide_load_once(const uint16_t* base, uint32_t lane_bytes, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_at), "v"(lane_bytes), "s"(base)
+               : "memory", "m0");
+}
 // A dword of each lane's line, to a place in LDS that nobody reads: it brings the line into the L2.
 __device__ __forceinline__ void wide_touch(const uint16_t* from, uint32_t lds_at) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_at), "v"(from) : "memory", "m0");
@@ -89,7 +96,7 @@ __device__ __forceinline__ float silu_near(float x) {
 }
 __device__ __forceinline__ float silu_whole(float x) { return x / (1.0f + expf(-x)); }
 
-template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut>
+template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut, bool ONCE>
 __global__ __launch_bounds__(WM* WN* kWave, (WM * WN + 3) / 4) void gemm_wide_kernel(const WideArgs a) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, kWaves = WM * WN;
   constexpr int kRowsALoad = 8 * kWaves;                        // rows that one load of every wave brings
@@ -99,6 +106,7 @@ __global__ __launch_bounds__(WM* WN* kWave, (WM * WN + 3) / 4) void gemm_wide_ke
   constexpr int kProducts = TM * TN, kReads = TM + TN;
   constexpr int kSlots = kProducts > 1 ? kProducts - 1 : 1, kReadsASlot = (kReads + kSlots - 1) / kSlots;   // reads go behind the products 1, 2, ... (behind the only one)
   constexpr bool kTouch = NS == 2;
+  static_assert(!ONCE || !kTouch, "lines that are touched ahead have to stay in the L2");
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -149,7 +157,8 @@ __global__ __launch_bounds__(WM* WN* kWave, (WM * WN + 3) / 4) void gemm_wide_ke
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds)) + 1024u * wave);
   auto load = [&](int i, uint32_t buf, const uint16_t* xs, const uint16_t* ws) {   // i is a constant where this is called
-    wide_load(i < LX ? xs : ws, off[i], lds0 + buf + 1024u * kWaves * i);
+    if (i < LX || !ONCE) wide_load(i < LX ? xs : ws, off[i], lds0 + buf + 1024u * kWaves * i);
+    else wide_load_once(ws, off[i], lds0 + buf + 1024u * kWaves * i);
   };
   // What comes from memory and not from the L2 comes late: every stage a wave touches a few of the 128-byte lines that the
   // stage kAhead later will fetch (the workgroups that share a column block's weights or a row block's x in a patch
@@ -349,19 +358,28 @@ __global__ __launch_bounds__(WM* WN* kWave, (WM * WN + 3) / 4) void gemm_wide_ke
   else if constexpr (EPI == kEpiSiluMul) leave(std::true_type{});
 }
 
-template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut>
-int launch_wide(WideArgs a, int splits, hipStream_t s) {
+template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut, bool ONCE>
+int launch_wide_as(WideArgs a, int splits, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr size_t lds = NS * (BM + BN) * 128 + (NS == 2 ? 256 * WM * WN : 0);
   static_assert(lds <= 160 * 1024, "the stages fit the LDS");
   static OnceADevice asked;
-  if (const int e = ask_lds(asked, lds, {reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut>)})) return e;
+  if (const int e = ask_lds(asked, lds, {reinterpret_cast<const void*>(&gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut, ONCE>)})) return e;
   a.m_blocks = (a.M + BM - 1) / BM;
   a.n_blocks = (a.N + BN - 1) / BN;
   const long long grid = static_cast<long long>(a.m_blocks) * ((a.n_blocks + kWdXcds - 1) / kWdXcds) * kWdXcds;
   if (grid > 0x7fffffffLL) return static_cast<int>(hipErrorInvalidValue);
-  gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut><<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(splits)), WM * WN * kWave, lds, s>>>(a);
+  gemm_wide_kernel<WM, WN, TM, TN, NS, EPI, TOut, ONCE><<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(splits)), WM * WN * kWave, lds, s>>>(a);
   return launch_status();
+}
+
+// ONCE where there is one row block: with several, the workgroups of a column block meet in their XCD's L2.
+template <int WM, int WN, int TM, int TN, int NS, int EPI, typename TOut>
+int launch_wide(const WideArgs& a, int splits, hipStream_t s) {
+  if constexpr (NS > 2) {
+    if (a.M <= 32 * WM * TM) return launch_wide_as<WM, WN, TM, TN, NS, EPI, TOut, true>(a, splits, s);
+  }
+  return launch_wide_as<WM, WN, TM, TN, NS, EPI, TOut, false>(a, splits, s);
 }
 
 template <int WM, int WN, int TM, int TN, int NS>

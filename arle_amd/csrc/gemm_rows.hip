@@ -55,7 +55,13 @@ struct RowsArgs {
   int64_t split_stride;  // elements between the partial products of two k splits
   int tiled;             // w holds operand tiles (see below) instead of rows
   int steps_per_round;   // ROUNDS: k steps of 32 whose X rows are in LDS at one time (the slice is walked in rounds)
+  // SCALED: the rows of X still have to be divided by their root mean square, which the sums of this product are instead:
+  // sums [M][kSumsPitch], the first sums_count of a row add up to the squares of its `1 / sums_inv` columns
+  const float* sums = nullptr;
+  int sums_count = 0;
+  float sums_inv = 0.f, eps = 0.f;
 };
+constexpr int kSumsPitch = 256, kScaledRows = 8;
 
 // Every byte of W is read by one wave of the launch: it is loaded past the caches, where it would only displace what is read
 // again.  MI355X, cold weights, us, kept / past the caches: 19,456 x 2,560 with the activation at 9 rows 21.3 / 20.7, 2,560 x
@@ -79,7 +85,10 @@ __device__ __forceinline__ const uint16_t* tile_base(const RowsArgs& a, int n0, 
 // ROUNDS: the k slice of a workgroup is too long for its X rows to fit into LDS at once (more than 27 rows of
 // 2,560 columns); it is walked in rounds of steps_per_round steps, each staged, multiplied and left behind a
 // barrier, with the sums staying in registers, so that whole sums meet the fused activation for up to 64 rows.
-template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool ROUNDS = false>
+//
+// SCALED (up to eight rows): every wave adds up the sums of one or two rows; they are asked for before W, so that they are there
+// when the staging of X, which waits for its own loads, is done.
+template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool ROUNDS = false, bool SCALED = false>
 __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a) {
   constexpr int kThreads = WN * WK * 64;
   static_assert(PD % XD == 0, "the X ring must divide the W ring");
@@ -102,6 +111,15 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
   f32x4 acc[MT];
 #pragma unroll
   for (int b = 0; b < MT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  static_assert(!SCALED || (MT == 1 && !ROUNDS && 2 * WN * WK >= kScaledRows), "two rows a wave");
+  __shared__ float row_scale[SCALED ? kScaledRows : 1];
+  [[maybe_unused]] float4 squares[2];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      squares[u] = *reinterpret_cast<const float4*>(a.sums + min(wave + u * WN * WK, M - 1) * kSumsPitch + 4 * lane);
+  }
 
   // one round: the steps [s_begin, s_end) of the slice, staged and multiplied (without ROUNDS: the whole slice)
   auto round = [&](const int s_begin, const int s_end) {
@@ -148,6 +166,16 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
         const int z0 = (k1 - k0) / 8, nz = (s_end * 32 - k1) / 8;
         for (int i = tid; i < M * nz; i += kThreads)
           *reinterpret_cast<uint4*>(lds + (i / nz) * pitch + (z0 + i % nz) * 8) = uint4{0u, 0u, 0u, 0u};
+      }
+    }
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float4 q = squares[u];
+        const int first = 4 * lane, count = a.sums_count;      // what lies behind the last strip's was never written
+        const float total = wave_sum(((first < count ? q.x : 0.f) + (first + 1 < count ? q.y : 0.f)) +
+                                     ((first + 2 < count ? q.z : 0.f) + (first + 3 < count ? q.w : 0.f)));
+        if (lane == 0 && wave + u * WN * WK < kScaledRows) row_scale[wave + u * WN * WK] = 1.0f / sqrtf(total * a.sums_inv + a.eps);
       }
     }
     __syncthreads();
@@ -235,6 +263,12 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
         acc[b][2] += p[2];
         acc[b][3] += p[3];
       }
+  }
+
+  if constexpr (SCALED) {
+    const float scale = row_scale[li & (kScaledRows - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[0][r] *= scale;
   }
 
   // acc[b][r] = C[m = 16 b + li][n = n0 + 4 g + r]
@@ -414,11 +448,11 @@ inline size_t rows_lds_bytes(int M, int steps_per_split, int mt, int wn, int wk)
 }
 constexpr size_t kRowsLdsMax = 144 * 1024;  // of the 160 KB of a CU
 
-template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut>
+template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool SCALED = false>
 int launch_rows(const RowsArgs& a, int splits, hipStream_t s) {
   const size_t lds = rows_lds_bytes(a.M, a.steps_per_split, MT, WN, WK);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
-  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, EPI, TOut>;
+  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, EPI, TOut, false, SCALED>;
   static OnceADevice asked;
   if (lds > 64 * 1024)
     if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
@@ -443,6 +477,11 @@ int launch_rows_rounds(const RowsArgs& a, hipStream_t s) {
 
 template <int MT, int WN, int WK, int PD, int XD, int EPI>
 int launch_rows_out(const RowsArgs& a, int splits, int out_dtype, hipStream_t s) {
+  if constexpr (MT == 1) {
+    if (a.sums != nullptr)
+      return out_dtype == kF32 ? launch_rows<MT, WN, WK, PD, XD, EPI, float, true>(a, splits, s)
+                               : launch_rows<MT, WN, WK, PD, XD, EPI, bf16, true>(a, splits, s);
+  }
   if (out_dtype == kF32) return launch_rows<MT, WN, WK, PD, XD, EPI, float>(a, splits, s);
   return launch_rows<MT, WN, WK, PD, XD, EPI, bf16>(a, splits, s);
 }
@@ -503,9 +542,11 @@ extern "C" long long arle_gemm_rows_lds_max() { return static_cast<long long>(kR
 // splits  > 1: out [splits, M, N] float32 partial products, split_stride elements apart, no activation;
 //              split s covers steps [s * steps_per_split, (s + 1) * steps_per_split) and none may be empty.
 // w_tiled: w holds operand tiles (RowsArgs), ldw is not used.
-extern "C" int arle_gemm_rows(const void* x, long long ldx, const void* w, long long ldw, int w_tiled, void* out, long long ldo,
-                              long long split_stride, int out_dtype, int M, int N, int K, int epilogue, int variant,
-                              int splits, int steps_per_split, void* stream) {
+// sums (or null), for M <= 8: row m of x is divided by the square root of sums_inv times the sum of sums[256 m ..][sums_count], plus eps.
+extern "C" int arle_gemm_rows_scaled(const void* x, long long ldx, const void* w, long long ldw, int w_tiled, void* out, long long ldo,
+                                     long long split_stride, int out_dtype, int M, int N, int K, int epilogue, int variant,
+                                     int splits, int steps_per_split, const void* sums, int sums_count, float sums_inv, float eps,
+                                     void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || K % 8 != 0 || K <= 0 || ldx % 8 != 0 || ldw % 8 != 0 || splits < 1 || splits > 65535 ||
       steps_per_split < 1 || variant < 0 || variant >= kVariants)
@@ -518,9 +559,11 @@ extern "C" int arle_gemm_rows(const void* x, long long ldx, const void* w, long 
   if (epilogue == kEpiSiluMul && (N % 32 != 0 || (arle_gemm_rows_geometry(variant) & 15) != 1))
     return static_cast<int>(hipErrorInvalidValue);
   if (epilogue != kEpiNone && epilogue != kEpiSiluMul) return static_cast<int>(hipErrorInvalidValue);
+  if (sums != nullptr && (M > kScaledRows || sums_count < 1 || sums_count > kSumsPitch || reinterpret_cast<uintptr_t>(sums) % 16 != 0))
+    return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RowsArgs a{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(w), ldw, out, ldo, M, N, K,
-                   steps_per_split, split_stride, w_tiled ? 1 : 0, 0};
+                   steps_per_split, split_stride, w_tiled ? 1 : 0, 0, static_cast<const float*>(sums), sums_count, sums_inv, eps};
   switch (variant) {
 #define X(ID, WN, WK, PD)                                                                       \
   case ID:                                                                                      \
@@ -531,6 +574,13 @@ extern "C" int arle_gemm_rows(const void* x, long long ldx, const void* w, long 
 #undef X
   }
   return static_cast<int>(hipErrorInvalidValue);
+}
+
+extern "C" int arle_gemm_rows(const void* x, long long ldx, const void* w, long long ldw, int w_tiled, void* out, long long ldo,
+                              long long split_stride, int out_dtype, int M, int N, int K, int epilogue, int variant,
+                              int splits, int steps_per_split, void* stream) {
+  return arle_gemm_rows_scaled(x, ldx, w, ldw, w_tiled, out, ldo, split_stride, out_dtype, M, N, K, epilogue, variant, splits, steps_per_split,
+                               nullptr, 0, 0.f, 0.f, stream);
 }
 
 // gate|up with the fused activation for up to 64 rows: as arle_gemm_rows with epilogue 1, variant 3 (eight waves,

@@ -30,6 +30,7 @@ SOURCES = {
     "gemm_rows": "gemm_rows.hip",
     "gemm_tiles": "gemm_tiles.hip",
     "gemm_wide": "gemm_wide.hip",
+    "gemm_strips": "gemm_strips.hip",
     "rope_kv": "rope_kv.hip",
     "attention_simt": "attention_simt.hip",
     "attention_mfma": "attention_mfma.hip",

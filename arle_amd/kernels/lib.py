@@ -26,6 +26,9 @@ SIGNATURES = {
     "arle_sum_partials": ("elementwise", [_p, _i, _ll, _p, _i, _ll, _i, _p]),
     "arle_gemm_rows_rounds": ("gemm_rows", [_p, _ll, _p, _ll, _i, _p, _ll, _i, _i, _i, _i, _i, _p]),
     "arle_gemm_rows": ("gemm_rows", [_p, _ll, _p, _ll, _i, _p, _ll, _ll, _i, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "arle_gemm_rows_scaled": ("gemm_rows", [_p, _ll, _p, _ll, _i, _p, _ll, _ll, _i, _i, _i, _i, _i, _i, _i, _i, _p, _i, _f, _f, _p]),
+    "arle_gemm_strips": ("gemm_strips", [_p, _ll, _p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p]),
+    "arle_gemm_strips_most": ("gemm_strips", []),
     "arle_gemm_rows_geometry": ("gemm_rows", [_i]),
     "arle_gemm_stream_geometry": ("gemm_rows", [_i]),
     "arle_gemm_stream_lds": ("gemm_rows", [_i, _i, _i]),

@@ -881,8 +881,86 @@ def _check_tiles(tiles, N: int, K: int) -> None:
         raise ShapeError(f"operand tiles of a [{N}, {K}] matrix have the shape [{-(-N // 16)}, {-(-K // 32)}, 512], got {tuple(tiles.shape)}")
 
 
+STRIP_ROWS = 8                   # rows that gemm_strips takes, and that gemm_rows takes with a divisor a row
+_STRIP_COLUMNS = (4, 16)         # columns of a strip: fewer are not worth a workgroup, more are not one operand tile
+
+
+@dataclasses.dataclass(frozen=True)
+class ScaledRows:
+    """Rows that a root-mean-square norm has multiplied by its weight but not yet divided by their root mean squares: the product
+    that reads them divides its sums instead (`scaled` of gemm_rows).  sums [rows, 256] float32: the first `count` of a row add up to
+    its sum of squares over `width` columns."""
+    rows: torch.Tensor
+    sums: torch.Tensor
+    count: int
+    width: int
+    eps: float
+
+    @property
+    def shape(self):
+        return self.rows.shape
+
+    @property
+    def dtype(self):
+        return self.rows.dtype
+
+    @property
+    def device(self):
+        return self.rows.device
+
+
+def strip_columns(n: int, k: int) -> int:
+    """Columns of a strip of a [n, k] matrix, one strip a compute unit (gemm_strips); 0: it is not cut into strips."""
+    most = _strips_most()
+    columns = -(-n // most)
+    return columns if _STRIP_COLUMNS[0] <= columns <= _STRIP_COLUMNS[1] and k >= 64 and k % 64 == 0 and columns * k <= 1 << 26 else 0
+
+
+@functools.lru_cache(maxsize=None)
+def _strips_most() -> int:
+    return lib.function("arle_gemm_strips_most")()
+
+
+def pack_weight_strips(w: torch.Tensor) -> torch.Tensor:
+    """w [N, K] bfloat16 -> [ceil(N/c), K/32, 4, c, 8] with c = strip_columns(N, K): element (t, s, g, i, e) = w[c t + i, 32 s + 8 g
+    + e], zeros past N.  A rearrangement at load time; with 16 columns these are the operand tiles of pack_weight_tiles."""
+    _need(w.dim() == 2 and w.dtype == torch.bfloat16, "pack_weight_strips takes a bfloat16 [N, K] matrix")
+    N, K = w.shape
+    c = strip_columns(N, K)
+    _need(c > 0, f"a [{N}, {K}] matrix is not cut into strips")
+    if N % c:
+        w = torch.nn.functional.pad(w, (0, 0, 0, -N % c))
+    return w.reshape(-1, c, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+
+
+def gemm_strips(x, strips, residual, weight, eps: float) -> ScaledRows:
+    """residual [M, N] (float32, in place) += x . W^T for 1..8 rows of x, W given as pack_weight_strips(W); returns the
+    residual's rows times `weight` (the norm's, [N]) with the sums of squares that the norm divides them by."""
+    _gpu(x, strips, residual, weight)
+    _rows(x, "x")
+    M, K = x.shape
+    N = residual.shape[1]
+    c = strip_columns(N, K)
+    _need(1 <= M <= STRIP_ROWS and c > 0, f"gemm_strips takes 1..{STRIP_ROWS} rows and matrices that are cut into strips (got {M} rows, [{N}, {K}])")
+    _need(x.dtype == torch.bfloat16 and strips.dtype == torch.bfloat16, "gemm_strips takes bfloat16 operands")
+    _need(strips.is_contiguous() and strips.numel() == -(-N // c) * c * K, f"strips of a [{N}, {K}] matrix expected, got {tuple(strips.shape)}")
+    _need(residual.dtype == torch.float32 and residual.is_contiguous() and residual.shape[0] == M, "the residual must be contiguous float32 [M, N]")
+    _need(weight.dtype in _CODES and weight.is_contiguous() and weight.numel() == N, "the norm weight must be contiguous [N]")
+    _need(x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and strips.data_ptr() % 16 == 0, "operands must be 16-byte aligned")
+    rows = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    sums = torch.empty((M, _strips_most()), dtype=torch.float32, device=x.device)
+    lib.call("arle_gemm_strips", x.data_ptr(), x.stride(0), strips.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+             int(weight.dtype == torch.float32), rows.data_ptr(), sums.data_ptr(), M, N, K, c, _stream())
+    return ScaledRows(rows, sums, -(-N // c), N, float(eps))
+
+
+def takes_scaled(rows: int, n: int, k: int, *, tiled: bool, fused: bool) -> bool:
+    """Whether the product of these sizes runs in a kernel that can divide its sums (gemm_rows up to eight rows)."""
+    return 1 <= rows <= STRIP_ROWS and choose_product(rows, n, k, k, tiled=tiled, fused=fused, partials_ok=not fused).kernel == "rows"
+
+
 def gemm_rows(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, variant: int | None = None,
-              splits: int | None = None, tiles: torch.Tensor | None = None):
+              splits: int | None = None, tiles: torch.Tensor | None = None, scaled: ScaledRows | None = None):
     """x . w^T for 1..64 rows of x, with x shared through LDS inside a workgroup.
 
     splits == 1: returns [M, N] (or [M, N/2] with EPI_SILU_MUL) in `out_dtype`.
@@ -891,9 +969,11 @@ def gemm_rows(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, varia
     the shape decides (gemm_rows_plan), so callers must be ready for either form.
     EPI_SILU_MUL: w holds gate and up rows interleaved in blocks of 16; out[m, j] = silu(gate_j) * up_j.
     tiles: pack_weight_tiles(w); the kernel then streams these instead of the rows of w (same sums, bit for bit).
+    scaled: x are its rows; the sums are divided by their root mean squares (before the activation).
     """
     _gpu(x, w)
     _rows(x, "x")
+    _need(scaled is None or (scaled.rows is x and x.shape[0] <= STRIP_ROWS), f"a divisor a row is for 1..{STRIP_ROWS} rows")
     _need(w.dim() == 2 and w.is_contiguous(), "w must be contiguous [N, K]")
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_rows takes bfloat16 operands")
     M, K = x.shape
@@ -926,9 +1006,12 @@ def gemm_rows(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, varia
         ldo, stride, code = out.stride(0), 0, _CODES[out_dtype]
     if tiles is not None:
         _check_tiles(tiles, N, K)
-    lib.call("arle_gemm_rows", x.data_ptr(), x.stride(0), (w if tiles is None else tiles).data_ptr(), w.stride(0),
-             int(tiles is not None), out.data_ptr(), ldo, stride,
-             code, M, N, K, int(epilogue), variant, splits, per_split, _stream())
+    args = (x.data_ptr(), x.stride(0), (w if tiles is None else tiles).data_ptr(), w.stride(0), int(tiles is not None), out.data_ptr(),
+            ldo, stride, code, M, N, K, int(epilogue), variant, splits, per_split)
+    if scaled is None:
+        lib.call("arle_gemm_rows", *args, _stream())
+    else:
+        lib.call("arle_gemm_rows_scaled", *args, scaled.sums.data_ptr(), scaled.count, 1.0 / scaled.width, scaled.eps, _stream())
     return out
 
 
@@ -1236,7 +1319,7 @@ def sum_partials(parts: torch.Tensor, out_dtype: torch.dtype, act: str | None = 
 
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, partials_ok: bool = False,
-              tiles: torch.Tensor | None = None):
+              tiles: torch.Tensor | None = None, scaled: ScaledRows | None = None):
     """out[M, N] = x[M, K] . w[N, K]^T, bfloat16 operands, float32 accumulation.
 
     Few rows (decode steps, short portions) run the hand-written weight-streaming kernels.  More rows go
@@ -1246,6 +1329,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.b
     partials_ok: the caller adds a float32 stack [S, M, N] itself (in the order of S) if that is what the
     kernel leaves behind; otherwise the stack is added here by one more small kernel.
     tiles: pack_weight_tiles(w), for the hand-written kernels to stream instead of w.
+    scaled: x are its rows, still to be divided (`takes_scaled` says for which sizes).
     """
     _gpu(x, w)
     _rows(x, "x")
@@ -1256,7 +1340,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.b
     rows, n, k = x.shape[0], w.shape[0], x.shape[1]
     choice = choose_product(rows, n, k, x.stride(0), tiled=tiles is not None, fused=False, partials_ok=partials_ok,
                             aligned=x.data_ptr() % 16 == 0, w_aligned=w.data_ptr() % 16 == 0)
-    return run_product(choice, x, w, tiles, out_dtype, partials_ok)
+    return run_product(choice, x, w, tiles, out_dtype, partials_ok, scaled=scaled)
 
 
 # The library runs a product with a narrow output and a long K (o and down: 2,560 columns) as a few dozen
@@ -1615,14 +1699,15 @@ def choose_product(rows: int, n: int, k: int, x_stride: int, *, tiled: bool, fus
                             w_aligned=w_aligned)
 
 
-def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool, fused: bool = False):
+def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool, fused: bool = False, scaled: ScaledRows | None = None):
     """Launch what `choice` names.  Plain products come back as [M, N] in out_dtype, or, where the caller said
     partials_ok, possibly as a float32 stack [S, M, N]; fused ones as the activation [M, N/2]."""
     kernel = choice.kernel
+    _need(scaled is None or kernel == "rows", "only gemm_rows divides its sums (see takes_scaled)")
     if fused:
         if kernel == "rows":
             return gemm_rows(x, w, x.dtype, EPI_SILU_MUL, variant=choice.variant[0] if choice.variant else None,
-                             splits=1 if choice.variant else None, tiles=tiles)
+                             splits=1 if choice.variant else None, tiles=tiles, scaled=scaled)
         if kernel == "rounds":
             return gemm_rows_rounds(x, w, x.dtype, tiles=tiles, round_steps=choice.variant[0] if choice.variant else None)
         if kernel == "tiles":
@@ -1632,7 +1717,7 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
         return silu_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), 16)
     if kernel == "rows":
         out = gemm_rows(x, w, out_dtype, variant=choice.variant[0] if choice.variant else None,
-                        splits=choice.splits or None, tiles=tiles)
+                        splits=choice.splits or None, tiles=tiles, scaled=scaled)
     elif kernel == "stream":
         out = gemm_stream(x, w, out_dtype, variant=choice.variant[0] if choice.variant else _STREAM_VARIANT,
                           splits=choice.splits or None, workgroups=choice.variant[1] if len(choice.variant) > 1 else None,
@@ -1659,19 +1744,21 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
     return out
 
 
-def gate_up_act(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor | None = None, act: int = 0) -> torch.Tensor:
+def gate_up_act(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor | None = None, act: int = 0,
+                scaled: ScaledRows | None = None) -> torch.Tensor:
     """act(x . gate^T) * (x . up^T) for w [2I, K] holding gate and up rows interleaved in blocks of 16: [M, I];
-    act 0: silu, 1: the tanh form of gelu."""
+    act 0: silu, 1: the tanh form of gelu.  scaled (act 0): x are its rows, still to be divided."""
     _gpu(x, w)
     _rows(x, "x")
     rows, n, k = x.shape[0], w.shape[0], x.shape[1]
     if rows == 0:
         return torch.empty((0, n // 2), dtype=x.dtype, device=x.device)
+    _need(scaled is None or act == 0, "rows that are still to be divided need an activation that the product applies")
     if act != 0:     # the products that apply the activation themselves know silu only
         return act_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), act, 16)
     choice = choose_product(rows, n, k, x.stride(0), tiled=tiles is not None, fused=True, partials_ok=False,
                             aligned=x.data_ptr() % 16 == 0, w_aligned=w.is_contiguous() and w.data_ptr() % 16 == 0)
-    return run_product(choice, x, w, tiles, x.dtype, False, fused=True)
+    return run_product(choice, x, w, tiles, x.dtype, False, fused=True, scaled=scaled)
 
 
 PRODUCT_TABLE_ENV = "ARLE_AMD_PRODUCT_TABLE"   # the path of a table that is taken in when this module is loaded ("none": no table at all)

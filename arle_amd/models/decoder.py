@@ -16,6 +16,7 @@ from ..parts import (attention, block, embedding, feed_forward, gated_delta, gat
                      loop, mixer_pair, mlstm, moe, norm, position, retention, rotary_attention, short_conv, softcap_attention,
                      state_space, token_side, wide_norm_attention)
 from ..parts.base import Runtime, build_part, expected_tensors, lookup
+from ..parts.linear import LateProduct
 from ..parts.spec import ModelSpec
 
 
@@ -75,6 +76,8 @@ def debug_dump(residual, delta, label: str) -> None:
     schedule entry (first and last values, minimum, maximum, root mean square, NaN or infinity anywhere), as the
     reference prints with INFER_DEBUG_DUMP (infer/src/model/common.rs:85-124).  Synchronises; steps are then not
     captured."""
+    if isinstance(delta, LateProduct):
+        delta = delta.now()
     if residual.dim() == 3 or hasattr(delta, "settled"):      # residual streams: their sum, a pending write done
         residual = delta.settled(residual) if hasattr(delta, "settled") else residual.sum(1)
         delta = None
@@ -188,9 +191,14 @@ class DecoderModel:
         if dump:
             debug_dump(residual, None, "embedding")
         for i, entry in enumerate(self.schedule):
-            residual, delta = self.blocks[entry.layer].forward(residual, delta, batch, cache.view(i))
+            block = self.blocks[entry.layer]
+            if isinstance(delta, LateProduct) and not getattr(block, "takes_late", False):
+                delta = delta.now()
+            residual, delta = block.forward(residual, delta, batch, cache.view(i))
             if dump:
                 debug_dump(residual, delta, f"schedule entry {i} (layer {entry.layer})")
+        if isinstance(delta, LateProduct):
+            delta = delta.now()
         wanted = self.final_norm.add_norm(residual, delta, rows=batch.want_rows)
         return self.head.forward(wanted)
 

@@ -76,7 +76,8 @@ class PagedAttention(Part):
         # for a layer that reads another layer's cache: the q rows of the fused matrix, no copy (head_dim is a
         # multiple of 16, so the q rows are whole operand tiles too)
         self.q_only = Linear(self.qkv.weight[: self.q_width], packed=self.qkv.tiles)
-        self.o = Linear(tensors["o"], rt.weight_tiles)
+        self.leaves_late = bool(rt.weight_tiles)
+        self.o = Linear(tensors["o"], rt.weight_tiles, strips=self.leaves_late)
         # steps of single decoded tokens run norm, rotation and cache write inside the attention's kernel where it
         # has that form (ops.attn_decode_prep_supported); params["fold_preparation"] = False keeps the two kernels
         self.folds_preparation = bool(params.get("fold_preparation", True))
@@ -109,8 +110,17 @@ class PagedAttention(Part):
     def decode_class_sizes(self):
         return self.rt.is_f32, self.D, self.nkv, self.window, self.folds_preparation
 
-    def forward(self, x, batch, cache):
-        """x [T, H] -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear)."""
+    def takes_scaled(self, rows: int) -> bool:
+        return self.qkv.takes_scaled(rows) and self.q_only.takes_scaled(rows)
+
+    def forward(self, x, batch, cache, late: bool = False):
+        """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);
+        late: possibly the output projection for the norm behind it to run."""
+        out = self._mixed(x, batch, cache)
+        return self.o.late(out) if late and self.leaves_late else self.o(out, partials_ok=True)
+
+    def _mixed(self, x, batch, cache):
+        """x -> the heads' sums of values [T, Q], before the output projection."""
         Q, KV = self.q_width, self.kv_width
         self.position.ensure_positions(batch.max_position + 1)
         cos, sin, rot = self.position.fused_rotary()
@@ -135,7 +145,7 @@ class PagedAttention(Part):
                                  scale=self.scale, eps=self.eps, q_weight=self.q_norm, k_weight=self.k_norm, cos=cos,
                                  sin=sin, rotary_dim=rot, window=self.window or 0, splits=getattr(batch, "kv_splits", None),
                                  total_kv_len=getattr(batch, "total_context", 0) or None, carry=getattr(batch, "carry", None))
-            return self.o(out, partials_ok=True)
+            return out
         if projected.dim() == 3:
             q = torch.empty((x.shape[0], Q), dtype=x.dtype, device=x.device)
             ops.qk_prep(q, None, None, q_weight=self.q_norm, k_weight=self.k_norm, cos=cos, sin=sin,
@@ -159,7 +169,7 @@ class PagedAttention(Part):
         out = torch.empty((x.shape[0], Q), dtype=q.dtype, device=q.device)
         paged_attention(q, out, cache, batch, num_q_heads=self.nq, num_kv_heads=self.nkv,
                         head_dim=self.D, scale=self.scale, window=self.window or 0)
-        return self.o(out, partials_ok=True)
+        return out
 
 
 def paged_attention(q, out, cache, batch, *, num_q_heads, num_kv_heads, head_dim, scale, window):

@@ -8,6 +8,7 @@ predecessor has not added yet, so that every add is fused into the norm that fol
 from __future__ import annotations
 
 from .base import register
+from .linear import LateProduct
 
 
 @register("block", "pre_norm")
@@ -17,20 +18,32 @@ class PreNormBlock:
 
     norm_roles = ("mixer_in", "ffn_in")
 
+    takes_late = True      # the delta may be a projection that has not run (LateProduct): the norm's to run with the add
+
     def __init__(self, mixer, feed_forward, norms: dict):
         self.mixer = mixer
         self.feed_forward = feed_forward
         self.norms = norms
         self.norm_mixer = norms["mixer_in"]
         self.norm_ffn = norms["ffn_in"] if feed_forward is not None else None
+        self._late = [{"late": True} if getattr(part, "leaves_late", False) else {} for part in (mixer, feed_forward)]
+
+    @staticmethod
+    def _add_norm(norm, residual, delta, reader):
+        if isinstance(delta, LateProduct):
+            takes = getattr(reader, "takes_scaled", None)
+            if takes is not None and hasattr(norm, "add_late") and takes(residual.shape[0]):
+                return norm.add_late(residual, delta)
+            delta = delta.now()
+        return norm.add_norm(residual, delta)
 
     def forward(self, residual, delta, batch, cache_view):
-        a = self.norm_mixer.add_norm(residual, delta)
-        m = self.mixer.forward(a, batch, cache_view)
+        a = self._add_norm(self.norm_mixer, residual, delta, self.mixer)
+        m = self.mixer.forward(a, batch, cache_view, **self._late[0])
         if self.norm_ffn is None:
             return residual, m
-        b = self.norm_ffn.add_norm(residual, m)
-        return residual, self.feed_forward.forward(b)
+        b = self._add_norm(self.norm_ffn, residual, m, self.feed_forward)
+        return residual, self.feed_forward.forward(b, **self._late[1])
 
 
 @register("block", "post_norm")

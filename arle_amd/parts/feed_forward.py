@@ -49,7 +49,12 @@ class SwiGLU(Part):
         else:
             fused = torch.cat([gate, up], dim=0)
         self.gate_up = Linear(fused.contiguous(), rt.weight_tiles)
-        self.down = Linear(tensors["down"], rt.weight_tiles)
+        self.leaves_late = bool(rt.weight_tiles) and not self.float32_out
+        self.down = Linear(tensors["down"], rt.weight_tiles, strips=self.leaves_late)
+
+    def takes_scaled(self, rows: int) -> bool:
+        return bool(self.block) and self.act == 0 and ops.takes_scaled(rows, self.gate_up.out_features, self.gate_up.in_features,
+                                                                       tiled=self.gate_up.tiles is not None, fused=True)
 
     def products(self):
         if self.gate_up.weight.dtype != torch.bfloat16:
@@ -57,13 +62,18 @@ class SwiGLU(Part):
         return [("gate_up", self.gate_up.out_features, self.gate_up.in_features, bool(self.block), None),
                 ("down", self.down.out_features, self.down.in_features, False, "norm")]
 
-    def forward(self, x):
-        """x [T, H] -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear)."""
-        if self.block:
+    def forward(self, x, late: bool = False):
+        """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);
+        late: possibly the down projection for the norm behind it to run."""
+        if isinstance(x, ops.ScaledRows):
+            act = ops.gate_up_act(x.rows, self.gate_up.weight, self.gate_up.tiles, scaled=x)
+        elif self.block:
             act = ops.gate_up_act(x, self.gate_up.weight, self.gate_up.tiles, self.act)   # one product with the activation, or two kernels
         else:
             gu = self.gate_up(x)
             act = ops.act_mul(gu[:, : self.inter], gu[:, self.inter:], self.act)
+        if late and self.leaves_late:
+            return self.down.late(act)
         return self.down(act, out_dtype=torch.float32 if self.float32_out else None, partials_ok=True)
 
 

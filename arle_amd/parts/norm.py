@@ -53,6 +53,10 @@ class RMSNorm(Part):
             return ops.rmsnorm(residual, self.weight, self.eps, self.rt.act_dtype, rows=rows)
         return ops.add_rmsnorm(residual, delta, self.weight, self.eps, self.rt.act_dtype, rows=rows)
 
+    def add_late(self, residual, late):
+        """residual (float32) += a projection that has not run (LateProduct), in its kernel: ops.ScaledRows, for a reader that takes them."""
+        return late.norm(residual, self.weight, self.eps)
+
 
 @register("norm", "layernorm")
 class LayerNorm(Part):

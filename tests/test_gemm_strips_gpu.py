@@ -1,0 +1,82 @@
+"""A projection whose kernel adds into the residual and leaves the norm's division to the product that reads its rows, against the
+float64 sums: strips of every kind of width (whole, 16 columns, a last one with columns missing), one to eight rows, K of one pair of
+steps and of fewer pairs than waves, both types of norm weight; and the division in every variant of the reading product."""
+import pytest
+import torch
+
+import plain_qwen3 as plain
+from arle_amd.kernels import ops
+from arle_amd.parts.linear import LateProduct, Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+EPS = 1e-6
+
+
+def _made(*shape, seed, scale=1.0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+@pytest.mark.parametrize("N,K", [(1024, 64), (1500, 448), (2560, 4096), (2600, 640), (4096, 1088)])
+@pytest.mark.parametrize("M,weight_type", [(1, torch.bfloat16), (2, torch.float32), (7, torch.bfloat16), (8, torch.float32)])
+def test_strips_add_into_the_residual_and_leave_the_rows_and_their_squares(N, K, M, weight_type):
+    x = _made(M, K + 8, seed=1).bfloat16().to(DEV)[:, :K]      # rows that do not lie side by side
+    w = _made(N, K, seed=2, scale=0.05).bfloat16().to(DEV)
+    residual = _made(M, N, seed=3, scale=3.0).to(DEV)
+    weight = (1.0 + _made(N, seed=4, scale=0.3)).to(weight_type).to(DEV)
+    want = residual.double() + x.double() @ w.double().T
+    linear = Linear(w, tiles=True, strips=True)
+    late = linear.late(x)
+    assert isinstance(late, LateProduct)
+    got = late.norm(residual, weight, EPS)
+    # 32-bit sums of at most 4,096 exact products, and of N squares
+    assert _rel(residual, want) < 1e-5
+    squares = got.sums[:, :got.count].double().sum(1)
+    assert _rel(squares, (want * want).sum(1)) < 1e-5
+    # one rounding to bfloat16: 2^-9 of a value at most
+    rows = want * weight.double()
+    assert float(((got.rows.double() - rows).abs() - rows.abs() * 2.0 ** -8).max()) <= 1e-4
+    assert (got.shape, got.dtype, got.count, got.width) == ((M, N), torch.bfloat16, -(-N // -(-N // 256)), N)
+
+
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("variant,splits,fused", [(0, 1, False), (0, 3, False), (1, 2, False), (2, 1, False), (3, 1, False), (4, 2, False),
+                                                  (0, 1, True), (1, 1, True), (3, 1, True), (4, 1, True)])
+def test_the_reading_product_divides_its_sums(M, variant, splits, fused):
+    N, K, count = 352, 1096, 250
+    rows = _made(M, K, seed=5, scale=40.0).bfloat16().to(DEV)
+    w = _made(N, K, seed=6, scale=0.05).bfloat16().to(DEV)
+    sums = (_made(M, 256, seed=7).abs() * 800.0).to(DEV)
+    sums[:, count:] = float("nan")      # behind the last strip's nothing was written
+    scaled = ops.ScaledRows(rows, sums, count, K, EPS)
+    divisor = torch.sqrt(sums[:, :count].double().sum(1, keepdim=True) / K + EPS)
+    want = rows.double() @ w.double().T / divisor
+    for tiles in (None, ops.pack_weight_tiles(w)):
+        if fused:
+            got = ops.gemm_rows(rows, w, torch.float32, ops.EPI_SILU_MUL, variant=variant, splits=1, tiles=tiles, scaled=scaled)
+            pairs = want.view(M, -1, 2, 16)
+            expected = (plain.silu(pairs[:, :, 0]) * pairs[:, :, 1]).reshape(M, -1)
+        else:
+            got = ops.gemm_rows(rows, w, torch.float32, variant=variant, splits=splits, tiles=tiles, scaled=scaled)
+            got, expected = got.sum(0) if got.dim() == 3 else got, want
+        assert _rel(got, expected) < 1e-5      # 32-bit sums of exact products, one division
+
+
+def test_what_takes_no_strips_runs_as_before():
+    w = _made(2560, 640, seed=8, scale=0.05).bfloat16().to(DEV)
+    linear = Linear(w, tiles=True, strips=True)
+    assert linear.strips is not None and not isinstance(linear.late(_made(9, 640, seed=9).bfloat16().to(DEV)), LateProduct)
+    assert Linear(w, tiles=True).strips is None
+    for n, k in ((512, 640), (5120, 640), (2560, 96)):      # too narrow, too wide, half a pair of steps left
+        assert ops.strip_columns(n, k) == 0 and Linear(torch.zeros(n, k, dtype=torch.bfloat16, device=DEV), tiles=True, strips=True).strips is None
+    wide = Linear(_made(4096, 640, seed=10).bfloat16().to(DEV), tiles=True, strips=True)
+    assert wide.strips is wide.tiles      # sixteen columns: one layout
+    rows = torch.zeros(9, 640, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ops.ShapeError):
+        ops.gemm_strips(rows, linear.strips, torch.zeros(9, 2560, device=DEV), torch.ones(2560, device=DEV), EPS)
+    with pytest.raises(ops.ShapeError):
+        ops.gemm_rows(rows, w, scaled=ops.ScaledRows(rows, torch.zeros(9, 256, device=DEV), 4, 640, EPS))

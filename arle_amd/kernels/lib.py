@@ -58,7 +58,7 @@ SIGNATURES = {
     "arle_sample_scratch_bytes": ("sampling", [_i, _i, _i]),
     "arle_sample_finish_most": ("sampling", []),
     "arle_sample_host_rows": ("sampling", []),
-    "arle_sample_rows": ("sampling", [_p, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p]),
+    "arle_sample_rows": ("sampling", [_p, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p]),
     "arle_apply_penalties": ("sampling", [_p, _i, _i, _p, _p, _p, _p, _p, _p, _p]),
     "arle_token_logprobs": ("sampling", [_p, _i, _i, _p, _p, _p]),
     "arle_attn_decode_static": ("attention_mfma", [_p, _ll, _p, _ll, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i,

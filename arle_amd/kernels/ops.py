@@ -740,16 +740,19 @@ SAMPLE_FINISH_VOCAB = 1 << 28    # up to here small_k holds
 
 
 def sample_rows(logits, temperature, top_k=None, top_p=None, min_p=None, u=None, *, use_top_k: bool = True,
-                use_top_p: bool = True, small_k: bool = False) -> torch.Tensor:
+                use_top_p: bool = True, small_k: bool = False, host_out: torch.Tensor | None = None) -> torch.Tensor:
     """One token id per row; per-row float32 temperature/top_p/min_p/u and int32 top_k.
 
     use_top_k / use_top_p = False promise that no row has that filter switched on (top_k in 1..vocab-1,
     top_p < 1): the passes over the row that look for its threshold are then not launched.  small_k promises that every
     row is greedy or has a top_k of 1 to `sample_small_k()`, below vocab: one kernel behind the rows' maxima then does all, and
     the parameters of up to `sample_host_rows()` rows may come as one numpy array in the place of `temperature`, float32 [5, rows] of
-    temperature, top_p, min_p, u and the bits of top_k, which travels with its launch.
+    temperature, top_p, min_p, u and the bits of top_k, which travels with its launch.  host_out: pinned int32 [rows] that the kernel
+    writes the tokens to as well; they are there when the stream has come to an event recorded behind this call.
     """
     rows, vocab = _logits(logits)
+    _need(host_out is None or (host_out.dtype == torch.int32 and host_out.shape == (rows,) and host_out.is_contiguous() and host_out.is_pinned()),
+          "host_out must be pinned int32 [rows]")
     finish = small_k and use_top_k and vocab <= SAMPLE_FINISH_VOCAB
     on_host = isinstance(temperature, np.ndarray)
     if on_host:
@@ -768,7 +771,7 @@ def sample_rows(logits, temperature, top_k=None, top_p=None, min_p=None, u=None,
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
     scratch = torch.empty((-(-_sample_scratch_bytes(rows, vocab, finish) // 8),), dtype=torch.int64, device=logits.device)
     lib.call("arle_sample_rows", logits.data_ptr(), rows, vocab, _ptr(probs), *params, out.data_ptr(), scratch.data_ptr(),
-             int(bool(use_top_k)), int(bool(use_top_p)), int(bool(small_k)), int(on_host), _stream())
+             int(bool(use_top_k)), int(bool(use_top_p)), int(bool(small_k)), int(on_host), _ptr(host_out), _stream())
     return out
 
 

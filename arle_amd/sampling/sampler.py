@@ -13,6 +13,7 @@ is not kept.
 from __future__ import annotations
 
 from array import array
+from collections import deque
 
 import numpy as np
 import torch
@@ -58,6 +59,37 @@ def uniforms(seeds, indices) -> np.ndarray:
     return out
 
 
+class _HostSlots:
+    """Places in pinned host memory that sampling kernels write their tokens to, `SLOTS` of one row block each, and an event a place.  A
+    place is given out again once its holder has let go of it and its event has come; where none is, there is none (`take`
+    returns None) and the tokens are copied as any others.  Nothing here waits."""
+
+    SLOTS = 256
+
+    def __init__(self, rows: int):
+        self.rows = rows
+        self.memory = torch.empty((self.SLOTS, rows), dtype=torch.int32, pin_memory=True)
+        self.places, self.events = [None] * self.SLOTS, [None] * self.SLOTS      # made as they are first taken
+        self.free = deque(range(self.SLOTS))      # the longest unused first (append and popleft are atomic)
+
+    def take(self):
+        try:
+            i = self.free.popleft()
+        except IndexError:
+            return None
+        if self.events[i] is None:
+            self.places[i], self.events[i] = self.memory[i], torch.cuda.Event()
+        elif not self.events[i].query():
+            self.free.appendleft(i)
+            return None
+        return i
+
+    def __del__(self):
+        for event in self.events:      # the memory outlives the kernels that write to it
+            if event is not None:
+                event.synchronize()
+
+
 class Chosen:
     """The tokens that a step's sampling kernels chose, still on the GPU: handed to the next step as they are
     (`feed`), and on their way into pinned host memory by a copy queued right behind the kernels, before anything
@@ -67,17 +99,33 @@ class Chosen:
     out: while its wait for the step sits in a second hardware queue, every kernel of the step takes 0.7 us longer
     to start, 0.23 ms a step of the Qwen3-4B shape.)"""
 
-    def __init__(self, token_tensor, logprob_tensor=None, read_back: bool = True):
+    _slots = None
+
+    def __init__(self, token_tensor, logprob_tensor=None, read_back: bool = True, slots=None, slot=None):
+        """slots, slot: a place of a `_HostSlots` that the kernel which made the tokens writes them to; this object's from here on."""
         self.token_tensor = token_tensor       # int32 [rows]
         self.logprob_tensor = logprob_tensor   # float32 [rows] or None
         self._tokens = self._logprobs = self._arrived = None
         self._host = []
+        if slot is not None:
+            self._slots, self._slot = slots, slot
+            self._host.append(slots.places[slot][:token_tensor.shape[0]])
+            self._arrived = slots.events[slot]
         if read_back and token_tensor.is_cuda:
             for t in (token_tensor, logprob_tensor):
-                if t is not None:
+                if t is not None and not (t is token_tensor and slot is not None):
                     self._host.append(torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t, non_blocking=True))
-            self._arrived = torch.cuda.Event()
+            if slot is None:
+                self._arrived = torch.cuda.Event()
             self._arrived.record()
+
+    def _let_go(self) -> None:
+        slots, self._slots = self._slots, None
+        if slots is not None:
+            slots.free.append(self._slot)
+
+    def __del__(self):
+        self._let_go()
 
     def feed(self, row: int) -> DeviceToken:
         return DeviceToken(self.token_tensor, row)
@@ -92,6 +140,7 @@ class Chosen:
         self._arrived.synchronize()
         self._tokens = self._host[0].tolist()
         self._logprobs = self._host[1].tolist() if len(self._host) > 1 else None
+        self._let_go()
 
     def tokens(self) -> list:
         self._read()
@@ -105,6 +154,7 @@ class Chosen:
 class Sampler:
     def __init__(self, device):
         self.device = device
+        self._slots = None
 
     def sample(self, logits: torch.Tensor, rows) -> list:
         """rows: one (SamplingParams, seed, draw_index, generated_tokens) per row of `logits`."""
@@ -131,14 +181,13 @@ class Sampler:
         if any(p.has_penalties() for p in kinds) and any(p.has_penalties() and gen for p, _, _, gen in rows):
             logits = logits.clone()
             self._penalise(logits, rows)
-        chosen = self._choose(logits, rows, kinds)
-        if not any(p.logprobs for p in kinds):
-            return Chosen(chosen)
-        return Chosen(chosen, ops.token_logprobs(logits, chosen))
+        chosen, *place = self._choose(logits, rows, kinds)
+        return Chosen(chosen, ops.token_logprobs(logits, chosen) if any(p.logprobs for p in kinds) else None, True, *place)
 
-    def _choose(self, logits: torch.Tensor, rows, kinds) -> torch.Tensor:
+    def _choose(self, logits: torch.Tensor, rows, kinds) -> tuple:
+        """(the tokens,) or (the tokens, a _HostSlots, the place in it that they are written to as well)"""
         if all(p.is_greedy() for p in kinds):
-            return ops.argmax_rows(logits)
+            return ops.argmax_rows(logits),
         n, vocab, small = len(rows), logits.shape[1], ops.sample_small_k()
         params, seeds, indices, _ = zip(*rows)
         packed = np.empty((5, n), dtype=np.float32)       # top_k as the bits of an int32
@@ -153,9 +202,19 @@ class Sampler:
         promises = dict(use_top_k=any(0 < p.top_k < vocab for p in kinds), use_top_p=any(p.top_p < 1.0 for p in kinds),
                         small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in kinds))
         if promises["small_k"] and n <= ops.sample_host_rows() and vocab <= ops.SAMPLE_FINISH_VOCAB:
-            return ops.sample_rows(logits, packed, **promises)     # they travel with the launch
+            slots = self._slots
+            if slots is None:
+                slots = self._slots = _HostSlots(ops.sample_host_rows())
+            slot = slots.take()
+            if slot is None:
+                return ops.sample_rows(logits, packed, **promises),
+            try:     # the parameters travel with the launch
+                return ops.sample_rows(logits, packed, host_out=slots.places[slot][:n], **promises), slots, slot
+            except BaseException:
+                slots.free.append(slot)
+                raise
         dev = upload(packed, self.device)      # one copy, queued: the host does not wait for the step that made the logits
-        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3], **promises)
+        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3], **promises),
 
     def _penalise(self, logits, rows) -> None:
         indptr, toks, counts = [0], [], []

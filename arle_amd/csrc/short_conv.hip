@@ -9,7 +9,8 @@
 // this step comes from its state [slots][taps-1][channels] (the most recent input last), which is all zeros
 // when the request starts, so inputs before position 0 count as zero without a test.  The sums are 32-bit.
 // `conv_state_update` then shifts each request's state by the rows it brought.  The update is a kernel of its
-// own because the convolution of a step reads the old state of every request.
+// own because the convolution of a step reads the old state of every request; where one workgroup a request does all of that
+// reading (causal_conv_rows_kernel) it moves the state on itself.
 #include "common.h"
 
 namespace arle {
@@ -105,13 +106,18 @@ __global__ void causal_conv_vec_kernel(const T* __restrict__ u, long long u_stri
 
 // The same for steps of many rows: a lane takes kConvRows rows of its four channels, whose inputs it slides over (each is
 // fetched once, not once a tap), where they and the rows they look back on belong to one request; else row by row.
+//
+// UPDATE: the first TAPS - 1 rows of a segment, the only ones that look back on its state, are left to a workgroup of the segment's own
+// behind those of the rows, which reads that state, makes those rows and writes the state moved on: the update is no kernel of its own
+// (4.9 us for a few kilobytes, twelve times in a prompt of eight Gufasun layers).
 constexpr int kConvRows = 8;
 
-template <typename T, int TAPS>
+template <typename T, int TAPS, bool UPDATE>
 __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_stride, const T* __restrict__ bias,
-                                        const T* __restrict__ out_bias, const T* __restrict__ w, const T* __restrict__ state,
+                                        const T* __restrict__ out_bias, const T* __restrict__ w, T* state,
                                         const int* __restrict__ slot_of_token, T* __restrict__ out, long long out_stride,
-                                        int tokens, int channels, int add_input) {
+                                        int tokens, int channels, int add_input, const int* __restrict__ seg_row0,
+                                        const int* __restrict__ seg_slot, int row_blocks) {
   const int t0 = blockIdx.x * kConvRows, rows = min(kConvRows, tokens - t0);
   const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
   if (c >= channels) return;
@@ -139,6 +145,37 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
     st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], add_input), conv_out(acc[1], add_input), conv_out(acc[2], add_input),
                                            conv_out(acc[3], add_input)});
   };
+  if constexpr (UPDATE) {
+    if (static_cast<int>(blockIdx.x) >= row_blocks) {
+      const int seg = static_cast<int>(blockIdx.x) - row_blocks;
+      const int row0 = seg_row0[seg], len = seg_row0[seg + 1] - row0;
+      T* mine = state + static_cast<int64_t>(seg_slot[seg]) * (TAPS - 1) * channels + c;
+      float4 old[TAPS - 1], first[TAPS - 1], fresh[TAPS - 1];
+      auto input = [&](int at) {     // row `at` of the segment, at a place that exists
+        const float4 v = ld4<T>(u + static_cast<int64_t>(min(max(row0 + at, 0), tokens - 1)) * u_stride + c);
+        return float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
+      };
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) old[j] = ld4<T>(mine + static_cast<int64_t>(j) * channels), first[j] = input(j), fresh[j] = input(len - (TAPS - 1) + j);
+#pragma unroll
+      for (int r = 0; r < TAPS - 1; ++r) {
+        float4 in[TAPS];
+#pragma unroll
+        for (int back = 0; back < TAPS; ++back) in[back] = back <= r ? first[r - back] : old[TAPS - 1 - (back - r)];
+        if (r < len) row_out(row0 + r, in);
+      }
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) {
+        const int at = len - (TAPS - 1) + j;      // place among the segment's rows; negative: still in the old state
+        float4 v = fresh[j];
+#pragma unroll
+        for (int back = 1; back < TAPS; ++back)
+          if (at == -back) v = old[TAPS - 1 - back];
+        st4<T>(mine + static_cast<int64_t>(j) * channels, v);
+      }
+      return;
+    }
+  }
   const int slot = slot_of_token[t0];
   bool one = t0 >= TAPS - 1;
   for (int r = one ? 1 - TAPS : 0; r < rows; ++r) one = one && slot_of_token[t0 + r] == slot;
@@ -162,6 +199,7 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
     const int t = t0 + r, mine_slot = slot_of_token[t];
     int mine = 0;
     while (mine < TAPS - 1 && t - mine - 1 >= 0 && slot_of_token[t - mine - 1] == mine_slot) ++mine;
+    if (UPDATE && mine < TAPS - 1) continue;      // the segment's workgroup makes it
     float4 in[TAPS];
 #pragma unroll
     for (int back = 0; back < TAPS; ++back) {
@@ -339,33 +377,54 @@ __global__ void conv_state_update_kernel(const void* __restrict__ u, long long u
 
 using namespace arle;
 
+extern "C" int arle_conv_state_update(const void* u, long long u_stride, int u_dtype, const void* bias,
+                                      int bias_dtype, void* state, int state_dtype, const int* seg_row0,
+                                      const int* seg_slot, int segments, int channels, int taps, void* stream);
+
 // u [T, channels] rows u_stride apart; out likewise; w [channels, taps] or null (then out = u + bias);
 // state [slots, taps-1, channels]; slot_of_token int32 [T].
+// seg_row0 int32 [segments + 1], seg_slot (or null): the segments' states are moved on by their rows (what arle_conv_state_update does).
 extern "C" int arle_causal_conv(const void* u, long long u_stride, int u_dtype, const void* bias, int bias_dtype,
                                 const void* out_bias, int ob_dtype, const void* w, int w_dtype,
-                                const void* state, int state_dtype,
+                                void* state, int state_dtype,
                                 const int* slot_of_token, void* out, long long out_stride, int out_dtype, int tokens,
-                                int channels, int taps, int add_input, void* stream) {
+                                int channels, int taps, int add_input, const int* seg_row0, const int* seg_slot, int segments,
+                                void* stream) {
+  const bool moves = seg_row0 != nullptr;
+  if (moves && (!seg_slot || segments < 0 || !w || !state)) return static_cast<int>(hipErrorInvalidValue);
   if (tokens == 0 || channels == 0) return 0;
   if (w && (taps < 1 || taps > kConvMaxTaps)) return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const auto moved_on = [&]() {      // behind the convolution, in a kernel of its own
+    const int e = launch_status();
+    return e != 0 || !moves ? e
+                            : arle_conv_state_update(u, u_stride, u_dtype, bias, bias_dtype, state, state_dtype, seg_row0, seg_slot, segments,
+                                                     channels, taps, stream);
+  };
   const auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (w && taps >= 2 && taps <= 4 && channels % 4 == 0 && u_stride % 4 == 0 && out_stride % 4 == 0 && at16(u) && at16(out) &&
       at16(state) && at16(w) && at16(bias) && at16(out_bias) && u_dtype == out_dtype && w_dtype == out_dtype && state_dtype == out_dtype &&
       (!bias || bias_dtype == out_dtype) && (!out_bias || ob_dtype == out_dtype)) {
     if (tokens >= kConvManyRows) {
-      dim3 rgrid((tokens + kConvRows - 1) / kConvRows, (channels / 4 + 255) / 256);
+      const int row_blocks = (tokens + kConvRows - 1) / kConvRows;
+      const dim3 rgrid(static_cast<unsigned>(row_blocks + (moves ? segments : 0)), (channels / 4 + 255) / 256);
+#define ARLE_CONV_ROWS_AS(T, TAPS, UPDATE)                                                                          \
+  causal_conv_rows_kernel<T, TAPS, UPDATE><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
+                                                                 static_cast<const T*>(out_bias), static_cast<const T*>(w), \
+                                                                 static_cast<T*>(state), slot_of_token,             \
+                                                                 static_cast<T*>(out), out_stride, tokens, channels, add_input, seg_row0, \
+                                                                 seg_slot, row_blocks)
 #define ARLE_CONV_ROWS(T, TAPS)                                                                                     \
-  causal_conv_rows_kernel<T, TAPS><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
-                                                         static_cast<const T*>(out_bias), static_cast<const T*>(w),  \
-                                                         static_cast<const T*>(state), slot_of_token,               \
-                                                         static_cast<T*>(out), out_stride, tokens, channels, add_input)
+  do {                                                                                                              \
+    if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true); else ARLE_CONV_ROWS_AS(T, TAPS, false);                            \
+  } while (0)
       if (out_dtype == kF32) {
         if (taps == 2) ARLE_CONV_ROWS(float, 2); else if (taps == 3) ARLE_CONV_ROWS(float, 3); else ARLE_CONV_ROWS(float, 4);
       } else {
         if (taps == 2) ARLE_CONV_ROWS(bf16, 2); else if (taps == 3) ARLE_CONV_ROWS(bf16, 3); else ARLE_CONV_ROWS(bf16, 4);
       }
 #undef ARLE_CONV_ROWS
+#undef ARLE_CONV_ROWS_AS
       return launch_status();
     }
     dim3 vgrid(tokens, (channels / 4 + 255) / 256);
@@ -380,13 +439,13 @@ extern "C" int arle_causal_conv(const void* u, long long u_stride, int u_dtype, 
       if (taps == 2) ARLE_CONV(bf16, 2); else if (taps == 3) ARLE_CONV(bf16, 3); else ARLE_CONV(bf16, 4);
     }
 #undef ARLE_CONV
-    return launch_status();
+    return moved_on();
   }
   dim3 grid(tokens, (channels + 255) / 256);
   causal_conv_kernel<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(
       u, u_stride, u_dtype, bias, bias_dtype, out_bias, ob_dtype, w, w_dtype, state, state_dtype, slot_of_token, out, out_stride,
       out_dtype, channels, taps, add_input);
-  return launch_status();
+  return moved_on();
 }
 
 extern "C" int arle_conv_state_update(const void* u, long long u_stride, int u_dtype, const void* bias,

@@ -67,7 +67,7 @@ SIGNATURES = {
     "arle_add_layernorm": ("layernorm", [_p, _p, _i, _ll, _i, _p, _i, _p, _i, _ll, _i, _p, _i, _p, _p, _i, _p, _p, _i, _p, _i,
                                          _i, _f, _p, _p, _p]),
     "arle_add_layernorm_conv": ("layernorm", [_p, _p, _i, _ll, _p, _p, _i, _ll, _p, _p, _p, _p, _p, _i, _i, _i, _f, _p, _p, _p, _p, _p, _i, _p]),
-    "arle_causal_conv": ("short_conv", [_p, _ll, _i, _p, _i, _p, _i, _p, _i, _p, _i, _p, _p, _ll, _i, _i, _i, _i, _i, _p]),
+    "arle_causal_conv": ("short_conv", [_p, _ll, _i, _p, _i, _p, _i, _p, _i, _p, _i, _p, _p, _ll, _i, _i, _i, _i, _i, _p, _p, _i, _p]),
     "arle_conv_state_update": ("short_conv", [_p, _ll, _i, _p, _i, _p, _i, _p, _p, _i, _i, _i, _p]),
     "arle_conv_step": ("short_conv", [_p, _ll, _i, _ll, _i, _p, _p, _p, _p, _p, _p, _ll, _i, _i, _i, _i, _p]),
     "arle_conv_step_store": ("short_conv", [_p, _ll, _i, _ll, _p, _p, _p, _p, _p, _i, _i, _p, _p, _f, _f, _i, _p, _p, _i, _p, _p, _i, _i, _i,

@@ -1887,13 +1887,14 @@ CONV_MAX_TAPS = 16
 
 
 def causal_conv(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, bias=None, add_input: bool = False,
-                out_dtype: torch.dtype | None = None, silu: bool = False, out_bias=None):
+                out_dtype: torch.dtype | None = None, silu: bool = False, out_bias=None, seg_row0=None, seg_slot=None):
     """y_t = (u_t if add_input) + sum_j weight[:, j] * u_(t - taps + 1 + j) per channel, over the rows of each request
     (consecutive in u) and, further back, over its state [slots, taps-1, C]; u counts with `bias` added.  weight
     None: y = u + bias.  out_bias [C]: added to y.  silu: y / (1 + exp(-y)) is
-    what comes out.  The state is not changed: `conv_state_update`
-    does that once the step's rows are done."""
-    _gpu(u, weight, state, slot_of_token, bias, out_bias)
+    what comes out.  Without the step's segments the state is not changed: `conv_state_update`
+    does that once the step's rows are done.  seg_row0, seg_slot: the segments, one a request, whose rows slot_of_token names;
+    their states are moved on by the rows they brought."""
+    _gpu(u, weight, state, slot_of_token, bias, out_bias, seg_row0, seg_slot)
     _rows(u, "u")
     tokens, channels = u.shape
     _i32(slot_of_token, "slot_of_token", tokens)
@@ -1913,11 +1914,17 @@ def causal_conv(u: torch.Tensor, weight, state, slot_of_token: torch.Tensor, *, 
               "a bias behind the convolution must be [channels]")
     out = torch.empty((tokens, channels), dtype=out_dtype or u.dtype, device=u.device)
     has_state = weight is not None and taps > 1
+    segments = 0
+    if seg_row0 is not None:
+        _need(has_state and seg_slot is not None, "a state that is moved on has its segments' rows and slots")
+        segments = seg_slot.numel()
+        _i32(seg_slot, "seg_slot")
+        _i32(seg_row0, "seg_row0", segments + 1)
     lib.call("arle_causal_conv", u.data_ptr(), u.stride(0), _code(u), _ptr(bias), _code(bias) if bias is not None else 0,
              _ptr(out_bias), _code(out_bias) if out_bias is not None else 0, _ptr(weight),
              _code(weight) if weight is not None else 0, state.data_ptr() if has_state else 0,
              _code(state) if has_state else 0, slot_of_token.data_ptr(), out.data_ptr(), out.stride(0), _code(out),
-             tokens, channels, taps, (1 if add_input else 0) | (2 if silu else 0), _stream())
+             tokens, channels, taps, (1 if add_input else 0) | (2 if silu else 0), _ptr(seg_row0), _ptr(seg_slot), segments, _stream())
     return out
 
 

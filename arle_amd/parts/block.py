@@ -7,6 +7,7 @@ predecessor has not added yet, so that every add is fused into the norm that fol
 """
 from __future__ import annotations
 
+from ..kernels.ops import STRIP_ROWS
 from .base import register
 from .linear import LateProduct
 
@@ -26,6 +27,7 @@ class PreNormBlock:
         self.norms = norms
         self.norm_mixer = norms["mixer_in"]
         self.norm_ffn = norms["ffn_in"] if feed_forward is not None else None
+        self._never = [{}, {}]
         self._late = [{"late": True} if getattr(part, "leaves_late", False) else {} for part in (mixer, feed_forward)]
 
     @staticmethod
@@ -38,12 +40,13 @@ class PreNormBlock:
         return norm.add_norm(residual, delta)
 
     def forward(self, residual, delta, batch, cache_view):
+        late = self._late if residual.shape[0] <= STRIP_ROWS else self._never
         a = self._add_norm(self.norm_mixer, residual, delta, self.mixer)
-        m = self.mixer.forward(a, batch, cache_view, **self._late[0])
+        m = self.mixer.forward(a, batch, cache_view, **late[0])
         if self.norm_ffn is None:
             return residual, m
         b = self._add_norm(self.norm_ffn, residual, m, self.feed_forward)
-        return residual, self.feed_forward.forward(b, **self._late[1])
+        return residual, self.feed_forward.forward(b, **late[1])
 
 
 @register("block", "post_norm")

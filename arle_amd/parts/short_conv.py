@@ -42,11 +42,9 @@ class ShortConv:
                             and self.takes_parts(batch, state_view)):
             return ops.conv_step(u, self.weight, state, batch.slot_of_token, bias=self.bias, add_input=add_input, silu=silu,
                                  out_bias=self.out_bias)
-        y = ops.causal_conv(u, self.weight, state, batch.slot_of_token, bias=self.bias, add_input=add_input, silu=silu,
-                            out_bias=self.out_bias)
-        if state is not None:
-            ops.conv_state_update(u, state, batch.seg_row0, batch.seg_slot, bias=self.bias)
-        return y
+        segments = {} if state is None else {"seg_row0": batch.seg_row0, "seg_slot": batch.seg_slot}
+        return ops.causal_conv(u, self.weight, state, batch.slot_of_token, bias=self.bias, add_input=add_input, silu=silu,
+                               out_bias=self.out_bias, **segments)
 
 
 @register("mixer", "input_conv")

@@ -110,9 +110,14 @@ __global__ void causal_conv_vec_kernel(const T* __restrict__ u, long long u_stri
 // UPDATE: the first TAPS - 1 rows of a segment, the only ones that look back on its state, are left to a workgroup of the segment's own
 // behind those of the rows, which reads that state, makes those rows and writes the state moved on: the update is no kernel of its own
 // (4.9 us for a few kilobytes, twelve times in a prompt of eight Gufasun layers).
+//
+// What bounds it is a chain of trips to memory, not its bytes (21 MB at 2,048 x 2,560, 3.7 us): all inputs and slots of a lane's rows are asked
+// for at once, before the weights and before anything is looked at, and SILU is known here, or every lane takes the exponential and the
+// divide.  MI355X, 2,048 x 2,560 / 6,144 with the states: slots one by one, weights first, silu by the flags 9.4 / 15.6 us; silu known
+// 9.1 / 15.3; inputs and slots first 8.7 / 14.6 (four rows a lane 8.3 / 14.8, sixteen 11.5 / 18.3).
 constexpr int kConvRows = 8;
 
-template <typename T, int TAPS, bool UPDATE>
+template <typename T, int TAPS, bool UPDATE, bool SILU>
 __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_stride, const T* __restrict__ bias,
                                         const T* __restrict__ out_bias, const T* __restrict__ w, T* state,
                                         const int* __restrict__ slot_of_token, T* __restrict__ out, long long out_stride,
@@ -121,6 +126,13 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
   const int t0 = blockIdx.x * kConvRows, rows = min(kConvRows, tokens - t0);
   const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
   if (c >= channels) return;
+  // All that the rows of one request need is asked for before anything is looked at; nothing of it stands under a condition.
+  const int first_back = t0 - (TAPS - 1);
+  auto row_at = [&](int r) { return min(max(first_back + r, 0), tokens - 1); };
+  float4 raw[kConvRows + TAPS - 1];
+  int slots[kConvRows + TAPS - 1];
+#pragma unroll
+  for (int r = 0; r < kConvRows + TAPS - 1; ++r) raw[r] = ld4<T>(u + static_cast<int64_t>(row_at(r)) * u_stride + c), slots[r] = slot_of_token[row_at(r)];
   const float4 b = bias ? ld4<T>(bias + c) : float4{0.f, 0.f, 0.f, 0.f};
   const float4 ob = out_bias ? ld4<T>(out_bias + c) : float4{0.f, 0.f, 0.f, 0.f};
   float wt[4][TAPS];   // four channels' taps are 4 * TAPS consecutive elements
@@ -142,8 +154,8 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt[i][TAPS - 1 - back], v[i], acc[i]);
     }
-    st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], add_input), conv_out(acc[1], add_input), conv_out(acc[2], add_input),
-                                           conv_out(acc[3], add_input)});
+    constexpr int kFlags = SILU ? kConvSilu : 0;
+    st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], kFlags), conv_out(acc[1], kFlags), conv_out(acc[2], kFlags), conv_out(acc[3], kFlags)});
   };
   if constexpr (UPDATE) {
     if (static_cast<int>(blockIdx.x) >= row_blocks) {
@@ -176,16 +188,15 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
       return;
     }
   }
-  const int slot = slot_of_token[t0];
-  bool one = t0 >= TAPS - 1;
-  for (int r = one ? 1 - TAPS : 0; r < rows; ++r) one = one && slot_of_token[t0 + r] == slot;
-  if (one) {
-    float4 raw[kConvRows + TAPS - 1];
+  bool one = first_back >= 0;
 #pragma unroll
-    for (int r = 0; r < kConvRows + TAPS - 1; ++r) {
-      const float4 v = ld4<T>(u + static_cast<int64_t>(min(t0 + r - (TAPS - 1), tokens - 1)) * u_stride + c);
-      raw[r] = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
-    }
+  for (int r = 0; r < kConvRows + TAPS - 1; ++r) {
+    one = one & ((slots[r] == slots[TAPS - 1]) | (r - (TAPS - 1) >= rows));
+    asm volatile("" : "+v"(raw[r].x));      // or the load moves down to the one row that needs it, and is waited for there
+  }
+  if (one) {
+#pragma unroll
+    for (int r = 0; r < kConvRows + TAPS - 1; ++r) raw[r] = float4{raw[r].x + b.x, raw[r].y + b.y, raw[r].z + b.z, raw[r].w + b.w};
 #pragma unroll
     for (int r = 0; r < kConvRows; ++r) {
       float4 in[TAPS];
@@ -408,15 +419,19 @@ extern "C" int arle_causal_conv(const void* u, long long u_stride, int u_dtype, 
     if (tokens >= kConvManyRows) {
       const int row_blocks = (tokens + kConvRows - 1) / kConvRows;
       const dim3 rgrid(static_cast<unsigned>(row_blocks + (moves ? segments : 0)), (channels / 4 + 255) / 256);
-#define ARLE_CONV_ROWS_AS(T, TAPS, UPDATE)                                                                          \
-  causal_conv_rows_kernel<T, TAPS, UPDATE><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
-                                                                 static_cast<const T*>(out_bias), static_cast<const T*>(w), \
-                                                                 static_cast<T*>(state), slot_of_token,             \
-                                                                 static_cast<T*>(out), out_stride, tokens, channels, add_input, seg_row0, \
-                                                                 seg_slot, row_blocks)
+#define ARLE_CONV_ROWS_AS(T, TAPS, UPDATE, SILU)                                                                    \
+  causal_conv_rows_kernel<T, TAPS, UPDATE, SILU><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
+                                                                       static_cast<const T*>(out_bias), static_cast<const T*>(w), \
+                                                                       static_cast<T*>(state), slot_of_token,       \
+                                                                       static_cast<T*>(out), out_stride, tokens, channels, add_input, \
+                                                                       seg_row0, seg_slot, row_blocks)
 #define ARLE_CONV_ROWS(T, TAPS)                                                                                     \
   do {                                                                                                              \
-    if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true); else ARLE_CONV_ROWS_AS(T, TAPS, false);                            \
+    if (add_input & kConvSilu) {                                                                                    \
+      if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true, true); else ARLE_CONV_ROWS_AS(T, TAPS, false, true);              \
+    } else {                                                                                                        \
+      if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true, false); else ARLE_CONV_ROWS_AS(T, TAPS, false, false);            \
+    }                                                                                                               \
   } while (0)
       if (out_dtype == kF32) {
         if (taps == 2) ARLE_CONV_ROWS(float, 2); else if (taps == 3) ARLE_CONV_ROWS(float, 3); else ARLE_CONV_ROWS(float, 4);

@@ -85,8 +85,10 @@ class Engine:
             row count, measured for this model's widths (`bench.py --tune-products`); without one, the rules that
             were measured at the Qwen3-4B, 8B and 32B widths decide.  The table is the process's, not this engine's.
         weight_tiles: hold every bfloat16 projection weight a second time in the layout that the few-rows
-            kernels stream fastest (decode steps about a tenth faster, twice the weight memory).  Default:
-            yes if both copies together stay under a third of the GPU's memory.
+            kernels stream fastest (decode steps about a tenth faster, twice the weight memory), and the projections
+            whose results a norm takes up a third time where they have 1,024 to 4,096 columns, other than 16 a compute
+            unit (up to a sixth less a step of eight rows or fewer).  Default: yes if the weights and the first of these
+            copies together stay under a third of the GPU's memory.
         """
         self.device = _device(device)
         self.dtype = parse_dtype(dtype)

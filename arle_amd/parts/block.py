@@ -27,7 +27,6 @@ class PreNormBlock:
         self.norms = norms
         self.norm_mixer = norms["mixer_in"]
         self.norm_ffn = norms["ffn_in"] if feed_forward is not None else None
-        self._never = [{}, {}]
         self._late = [{"late": True} if getattr(part, "leaves_late", False) else {} for part in (mixer, feed_forward)]
 
     @staticmethod
@@ -40,13 +39,17 @@ class PreNormBlock:
         return norm.add_norm(residual, delta)
 
     def forward(self, residual, delta, batch, cache_view):
-        late = self._late if residual.shape[0] <= STRIP_ROWS else self._never
+        if residual.shape[0] > STRIP_ROWS:      # nothing is left to a norm here, and a step's first pass is bound by the host
+            m = self.mixer.forward(self.norm_mixer.add_norm(residual, delta), batch, cache_view)
+            if self.norm_ffn is None:
+                return residual, m
+            return residual, self.feed_forward.forward(self.norm_ffn.add_norm(residual, m))
         a = self._add_norm(self.norm_mixer, residual, delta, self.mixer)
-        m = self.mixer.forward(a, batch, cache_view, **late[0])
+        m = self.mixer.forward(a, batch, cache_view, **self._late[0])
         if self.norm_ffn is None:
             return residual, m
         b = self._add_norm(self.norm_ffn, residual, m, self.feed_forward)
-        return residual, self.feed_forward.forward(b, **late[1])
+        return residual, self.feed_forward.forward(b, **self._late[1])
 
 
 @register("block", "post_norm")

@@ -93,8 +93,8 @@ def _completes_gate_up(name: str) -> bool:
 def classify_step(names, layers: int) -> list:
     """The part of the model that each kernel of one step belongs to, from the order in which a layer launches
     them: norm, q|k|v product, q/k preparation (a kernel of its own, or inside the attention's for single decoded
-    tokens), attention (+ merges), o product, norm, gate|up (+ activation), down product; after the last layer the
-    final norm and the head."""
+    tokens), attention (+ merges), o product, norm, gate|up (+ activation), down product (o and down of up to eight rows with the norm
+    behind them in one kernel); after the last layer the final norm and the head."""
     out, phase, layers_done = [], "qkv", 0
     for name in names:
         if "qk_prep" in name:
@@ -105,6 +105,13 @@ def classify_step(names, layers: int) -> list:
                 phase = "o"
         elif "rmsnorm" in name:
             part = "norm"
+            if phase == "o":
+                phase = "gate_up"
+            elif phase == "down":
+                layers_done += 1
+                phase = "head" if layers_done >= layers else "qkv"
+        elif "gemm_strips" in name:
+            part = phase           # o or down with the norm behind it
             if phase == "o":
                 phase = "gate_up"
             elif phase == "down":
@@ -157,7 +164,8 @@ def part_times(steps, layers: int) -> dict:
     most = max(len(k) for k in steps)
     steps = [k for k in steps if len(k) == most]
     for kernels in steps:
-        seen = (sum(1 for n, _ in kernels if "rmsnorm" in n) - 1) // 2   # two norms a layer and the last one
+        # two norms a layer and the last one, some of them in the projection in front of them
+        seen = (sum(1 for n, _ in kernels if "rmsnorm" in n or "gemm_strips" in n) - 1) // 2
         if seen != layers:
             raise RuntimeError(f"a profiled step shows {seen} of {layers} layers")
     total = {p: 0.0 for p in PARTS}

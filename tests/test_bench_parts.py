@@ -57,3 +57,14 @@ def test_bytes_and_flops_of_the_parts_add_up_to_the_step():
     assert by_part["attention"] == 8 * 2064 * 147456
     flops = bench.part_flops_prefill(c, 2048)
     assert abs(sum(flops.values()) / bench.prefill_flops(c, 2048) - 1.0) < 1e-9
+
+
+def test_projections_with_the_norm_behind_them_move_a_step_on():
+    """Steps of up to eight rows: o and down add, norm and leave; the last layer's down is a product and the final norm's kernel."""
+    layer = ["gemm_rows_kernel<1, 2, 2, 4, 4, 0, float, false, true>", "attn_mfma_kernel<1, 128, true, true>", "attn_merge_kernel",
+             "gemm_strips_kernel(arle::StripArgs)", "gemm_rows_kernel<1, 8, 1, 4, 4, 1, arle::bf16, false, true>"]
+    names = (["embed_gather_kernel", "rmsnorm"] + layer + ["gemm_strips_kernel(arle::StripArgs)"] + layer
+             + ["gemm_rows_kernel<1, 2, 4, 4, 4, 0, float, false, false>", "add_stack_rmsnorm_kernel<bf16>", "gemm_rows_kernel<1, 8, 1, 4, 4, 0, float>"])
+    in_layer = ["qkv", "attention", "attention", "o", "gate_up", "down"]
+    assert bench.classify_step(names, layers=2) == ["other", "norm"] + in_layer * 2 + ["norm", "head"]
+    assert bench.part_times([[(n, 1.0) for n in names]], layers=2)["down"] == 2.0

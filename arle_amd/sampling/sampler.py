@@ -12,6 +12,7 @@ is not kept.
 """
 from __future__ import annotations
 
+import threading
 from array import array
 from collections import deque
 
@@ -59,88 +60,117 @@ def uniforms(seeds, indices) -> np.ndarray:
     return out
 
 
+class _HostPlace:
+    """Pinned host memory that one sampling kernel at a time writes its tokens to, and the event behind that kernel; written: it is
+    known to have come."""
+
+    written = True
+
+    def __init__(self, rows: int):
+        self.memory = torch.empty((rows,), dtype=torch.int32, pin_memory=True)
+        self.event = torch.cuda.Event()
+
+    def __del__(self):
+        event = getattr(self, "event", None)
+        if event is not None:
+            event.synchronize()      # the memory outlives the kernel that writes to it
+
+
+class _HeldPlace:
+    """A place of a `_HostSlots` and its owner: it goes back once, when the tokens have been read or nobody can read them any more."""
+
+    def __init__(self, slots: "_HostSlots", place: _HostPlace, rows: int):
+        place.written = False
+        self.memory, self.event = place.memory[:rows], place.event
+        self._free, self._places = slots.free, [place]
+
+    def let_go(self, written: bool = False) -> None:
+        """written: the event has been waited for."""
+        try:
+            place = self._places.pop()      # one thread gets it
+        except IndexError:
+            return
+        place.written = written
+        self._free.append(place)
+
+    def __del__(self):
+        self.let_go()
+
+
 class _HostSlots:
-    """Places in pinned host memory that sampling kernels write their tokens to, `SLOTS` of one row block each, and an event a place.  A
-    place is given out again once its holder has let go of it and its event has come; where none is, there is none (`take`
-    returns None) and the tokens are copied as any others.  Nothing here waits."""
+    """Up to `SLOTS` places for tokens, made as they are needed.  A place is given out again once its holder has let go of it and
+    its event has come; where there is none, `take` returns None and the tokens are copied as any others.  Nothing here waits.
+    (One block for all places, made by a sampler's first call: 64.3 us that call, 64 rows of 151,936 logits; a place at a time 62.5, and
+    61.7 with the copy, which costs every later call among others 40 instead of 34.)"""
 
     SLOTS = 256
 
-    def __init__(self, rows: int):
-        self.rows = rows
-        self.memory = torch.empty((self.SLOTS, rows), dtype=torch.int32, pin_memory=True)
-        self.places, self.events = [None] * self.SLOTS, [None] * self.SLOTS      # made as they are first taken
-        self.free = deque(range(self.SLOTS))      # the longest unused first (append and popleft are atomic)
+    def __init__(self):
+        self.free = deque()      # the longest unused first (append and popleft are atomic)
+        self._made, self._lock = 0, threading.Lock()
 
-    def take(self):
-        try:
-            i = self.free.popleft()
-        except IndexError:
-            return None
-        if self.events[i] is None:
-            self.places[i], self.events[i] = self.memory[i], torch.cuda.Event()
-        elif not self.events[i].query():
-            self.free.appendleft(i)
-            return None
-        return i
-
-    def __del__(self):
-        for event in self.events:      # the memory outlives the kernels that write to it
-            if event is not None:
-                event.synchronize()
+    def take(self, rows: int):
+        if torch.cuda.is_current_stream_capturing():
+            return None      # a replay would write where another call's tokens are by then
+        with self._lock:
+            if self.free and (self.free[0].written or self.free[0].event.query()):
+                return _HeldPlace(self, self.free.popleft(), rows)
+            if self._made == self.SLOTS:
+                return None
+            place = _HostPlace(ops.sample_host_rows())
+            self._made += 1
+            return _HeldPlace(self, place, rows)
 
 
 class Chosen:
     """The tokens that a step's sampling kernels chose, still on the GPU: handed to the next step as they are
-    (`feed`), and on their way into pinned host memory by a copy queued right behind the kernels, before anything
+    (`feed`), and on their way into pinned host memory, written there by the sampling kernel itself (a place of the sampler's, which
+    goes back to it once they are read) or by a copy queued right behind the kernels, before anything
     else is launched, so that reading them (`tokens`, `logprobs`) waits for the step that chose them and not for
-    the step launched after it.  (The reference reads its argmax back asynchronously into a ring of pinned
+    the step launched after it.  Any thread may read them.  (The reference reads its argmax back asynchronously into a ring of pinned
     buffers: infer/src/model/qwen3/batch_decode.rs:728-774.  A copy stream of its own was tried here and taken
     out: while its wait for the step sits in a second hardware queue, every kernel of the step takes 0.7 us longer
     to start, 0.23 ms a step of the Qwen3-4B shape.)"""
 
-    _slots = None
-
-    def __init__(self, token_tensor, logprob_tensor=None, read_back: bool = True, slots=None, slot=None):
-        """slots, slot: a place of a `_HostSlots` that the kernel which made the tokens writes them to; this object's from here on."""
+    def __init__(self, token_tensor, logprob_tensor=None, read_back: bool = True, held: _HeldPlace | None = None):
+        """held: the place that the kernel which made the tokens writes them to, its event recorded behind that kernel."""
+        self._slots = held      # until they are read
+        self._reading = threading.Lock()
         self.token_tensor = token_tensor       # int32 [rows]
         self.logprob_tensor = logprob_tensor   # float32 [rows] or None
         self._tokens = self._logprobs = self._arrived = None
         self._host = []
-        if slot is not None:
-            self._slots, self._slot = slots, slot
-            self._host.append(slots.places[slot][:token_tensor.shape[0]])
-            self._arrived = slots.events[slot]
+        copied = [logprob_tensor] if held is not None else [token_tensor, logprob_tensor]
+        if held is not None:
+            self._host.append(held.memory)
+            self._arrived = held.event
         if read_back and token_tensor.is_cuda:
-            for t in (token_tensor, logprob_tensor):
-                if t is not None and not (t is token_tensor and slot is not None):
+            for t in copied:
+                if t is not None:
                     self._host.append(torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t, non_blocking=True))
-            if slot is None:
+            if held is None:
                 self._arrived = torch.cuda.Event()
-            self._arrived.record()
-
-    def _let_go(self) -> None:
-        slots, self._slots = self._slots, None
-        if slots is not None:
-            slots.free.append(self._slot)
-
-    def __del__(self):
-        self._let_go()
+            if held is None or logprob_tensor is not None:
+                self._arrived.record()
 
     def feed(self, row: int) -> DeviceToken:
         return DeviceToken(self.token_tensor, row)
 
     def _read(self) -> None:
-        if self._tokens is not None:
-            return
-        if self._arrived is None:
-            self._tokens = self.token_tensor.tolist()
-            self._logprobs = None if self.logprob_tensor is None else self.logprob_tensor.tolist()
-            return
-        self._arrived.synchronize()
-        self._tokens = self._host[0].tolist()
-        self._logprobs = self._host[1].tolist() if len(self._host) > 1 else None
-        self._let_go()
+        with self._reading:
+            if self._tokens is not None:
+                return
+            if self._arrived is None:
+                tokens = self.token_tensor.tolist()
+                self._logprobs = None if self.logprob_tensor is None else self.logprob_tensor.tolist()
+            else:
+                self._arrived.synchronize()
+                tokens = self._host[0].tolist()
+                self._logprobs = self._host[1].tolist() if len(self._host) > 1 else None
+            self._tokens = tokens
+            held, self._slots, self._host = self._slots, None, []
+            if held is not None:
+                held.let_go(written=True)
 
     def tokens(self) -> list:
         self._read()
@@ -154,7 +184,7 @@ class Chosen:
 class Sampler:
     def __init__(self, device):
         self.device = device
-        self._slots = None
+        self._slots = _HostSlots()
 
     def sample(self, logits: torch.Tensor, rows) -> list:
         """rows: one (SamplingParams, seed, draw_index, generated_tokens) per row of `logits`."""
@@ -181,13 +211,13 @@ class Sampler:
         if any(p.has_penalties() for p in kinds) and any(p.has_penalties() and gen for p, _, _, gen in rows):
             logits = logits.clone()
             self._penalise(logits, rows)
-        chosen, *place = self._choose(logits, rows, kinds)
-        return Chosen(chosen, ops.token_logprobs(logits, chosen) if any(p.logprobs for p in kinds) else None, True, *place)
+        chosen, held = self._choose(logits, rows, kinds)
+        return Chosen(chosen, ops.token_logprobs(logits, chosen) if any(p.logprobs for p in kinds) else None, held=held)
 
     def _choose(self, logits: torch.Tensor, rows, kinds) -> tuple:
-        """(the tokens,) or (the tokens, a _HostSlots, the place in it that they are written to as well)"""
+        """(the tokens, the _HeldPlace that they are written to as well or None)"""
         if all(p.is_greedy() for p in kinds):
-            return ops.argmax_rows(logits),
+            return ops.argmax_rows(logits), None
         n, vocab, small = len(rows), logits.shape[1], ops.sample_small_k()
         params, seeds, indices, _ = zip(*rows)
         packed = np.empty((5, n), dtype=np.float32)       # top_k as the bits of an int32
@@ -202,19 +232,15 @@ class Sampler:
         promises = dict(use_top_k=any(0 < p.top_k < vocab for p in kinds), use_top_p=any(p.top_p < 1.0 for p in kinds),
                         small_k=all(0 < p.top_k <= small and p.top_k < vocab or p.is_greedy() for p in kinds))
         if promises["small_k"] and n <= ops.sample_host_rows() and vocab <= ops.SAMPLE_FINISH_VOCAB:
-            slots = self._slots
-            if slots is None:
-                slots = self._slots = _HostSlots(ops.sample_host_rows())
-            slot = slots.take()
-            if slot is None:
-                return ops.sample_rows(logits, packed, **promises),
-            try:     # the parameters travel with the launch
-                return ops.sample_rows(logits, packed, host_out=slots.places[slot][:n], **promises), slots, slot
-            except BaseException:
-                slots.free.append(slot)
-                raise
+            held = self._slots.take(n)      # the parameters travel with the launch
+            if held is None:
+                return ops.sample_rows(logits, packed, **promises), None
+            try:
+                return ops.sample_rows(logits, packed, host_out=held.memory, **promises), held
+            finally:
+                held.event.record()      # whatever fails from here on: the place is free when the kernel is done with it
         dev = upload(packed, self.device)      # one copy, queued: the host does not wait for the step that made the logits
-        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3], **promises),
+        return ops.sample_rows(logits, dev[0], dev[4].view(torch.int32), dev[1], dev[2], dev[3], **promises), None
 
     def _penalise(self, logits, rows) -> None:
         indptr, toks, counts = [0], [], []

@@ -63,14 +63,19 @@ struct RowsArgs {
 };
 constexpr int kSumsPitch = 256, kScaledRows = 8;
 
-// Every byte of W is read by one wave of the launch: it is loaded past the caches, where it would only displace what is read
-// again.  MI355X, cold weights, us, kept / past the caches: 19,456 x 2,560 with the activation at 9 rows 21.3 / 20.7, 2,560 x
-// 9,728 at 9 rows 11.2 / 10.6, 151,936 x 2,560 at 9 rows 142 / 125; decode steps of the Qwen3-4B shape at 1 and 8 requests
-// 2,440 / 2,381 and 2,837 / 2,756.  Not in gemm_stream_kernel, which
-// measured slower with it (2,560 x 4,096 at 9 and 16 rows 7.1 / 7.3 and 7.2 / 7.5).
+// Every byte of W is read by one wave of the launch.  As operand tiles, where a wave's load is whole lines, it is loaded past the
+// caches (ONCE), where it would only displace what is read again; as rows not: a step of a row is half a line, and the next step's load
+// finds the other half only if the line has stayed.  MI355X, cold weights, us, kept / past the caches:
+//   tiles: 19,456 x 2,560 with the activation at 9 rows 21.3 / 20.7, 2,560 x 9,728 at 9 rows 11.2 / 10.6, 151,936 x 2,560 at 9 rows
+//     142 / 125; decode steps of the Qwen3-4B shape at 1 and 8 requests 2,440 / 2,381 and 2,837 / 2,756.
+//   rows: 19,456 x 2,560 with the activation at 1 and 8 rows 24.2 / 29.1 and 32.5 / 38.2, 51,200 x 5,120 102 / 122 and 118 / 138,
+//     2,560 x 9,728 13.5 / 14.5 and 15.0 / 16.4; the same decode steps 2,669 / 2,934 and 3,349 / 3,709.
+// Not in gemm_stream_kernel, which measured slower with it (2,560 x 4,096 at 9 and 16 rows 7.1 / 7.3 and 7.2 / 7.5).
+template <bool ONCE>
 __device__ __forceinline__ bf16x8 load_w16(const uint16_t* p) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
+  if constexpr (ONCE) return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
 }
 
 // W as operand tiles: [ceil(N/16)][ceil(K/32)][64 lanes][8], tile (t, s) lane 16 g + i = W[16 t + i][32 s + 8 g .. +7],
@@ -88,7 +93,9 @@ __device__ __forceinline__ const uint16_t* tile_base(const RowsArgs& a, int n0, 
 //
 // SCALED (up to eight rows): every wave adds up the sums of one or two rows; they are asked for before W, so that they are there
 // when the staging of X, which waits for its own loads, is done.
-template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool ROUNDS = false, bool SCALED = false>
+//
+// TILED: RowsArgs::tiled, known here for the loads of W.
+template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool TILED, bool ROUNDS = false, bool SCALED = false>
 __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a) {
   constexpr int kThreads = WN * WK * 64;
   static_assert(PD % XD == 0, "the X ring must divide the W ring");
@@ -129,11 +136,11 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
     const int n_steps = max(0, min(w_begin + per, s_end) - w_begin);
 
     // rows: lane (i, g) reads 16 bytes of row n0 + i; tiles: the wave reads tile s of its column tile, lane by lane
-    const uint16_t* wrow = a.tiled ? tile_base(a, n0, lane) : a.w + static_cast<int64_t>(min(n0 + li, N - 1)) * a.ldw;
-    const int w_step = a.tiled ? 512 : 32, w_first = a.tiled ? 0 : 8 * g, w_last = a.tiled ? (steps_total - 1) * 512 : K - 8;
+    const uint16_t* wrow = TILED ? tile_base(a, n0, lane) : a.w + static_cast<int64_t>(min(n0 + li, N - 1)) * a.ldw;
+    const int w_step = TILED ? 512 : 32, w_first = TILED ? 0 : 8 * g, w_last = TILED ? (steps_total - 1) * 512 : K - 8;
     auto load_w = [&](int s) {
       const int e = min(w_step * s + w_first, w_last);  // clamped: always inside the row (the column tile)
-      return load_w16(wrow + e);
+      return load_w16<TILED>(wrow + e);
     };
 
     // the first PD steps of W are on their way before anything else happens; without a condition (a step past
@@ -448,11 +455,11 @@ inline size_t rows_lds_bytes(int M, int steps_per_split, int mt, int wn, int wk)
 }
 constexpr size_t kRowsLdsMax = 144 * 1024;  // of the 160 KB of a CU
 
-template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool SCALED = false>
-int launch_rows(const RowsArgs& a, int splits, hipStream_t s) {
+template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool TILED, bool SCALED>
+int launch_rows_as(const RowsArgs& a, int splits, hipStream_t s) {
   const size_t lds = rows_lds_bytes(a.M, a.steps_per_split, MT, WN, WK);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
-  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, EPI, TOut, false, SCALED>;
+  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, EPI, TOut, TILED, false, SCALED>;
   static OnceADevice asked;
   if (lds > 64 * 1024)
     if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
@@ -461,18 +468,29 @@ int launch_rows(const RowsArgs& a, int splits, hipStream_t s) {
   return launch_status();
 }
 
+template <int MT, int WN, int WK, int PD, int XD, int EPI, typename TOut, bool SCALED = false>
+int launch_rows(const RowsArgs& a, int splits, hipStream_t s) {
+  return a.tiled ? launch_rows_as<MT, WN, WK, PD, XD, EPI, TOut, true, SCALED>(a, splits, s)
+                 : launch_rows_as<MT, WN, WK, PD, XD, EPI, TOut, false, SCALED>(a, splits, s);
+}
+
 // The fused activation for more rows than LDS holds of all of K at once: one k slice, walked in rounds.
-template <int MT, int WN, int WK, int PD, int XD, typename TOut>
-int launch_rows_rounds(const RowsArgs& a, hipStream_t s) {
+template <int MT, int WN, int WK, int PD, int XD, typename TOut, bool TILED>
+int launch_rows_rounds_as(const RowsArgs& a, hipStream_t s) {
   const size_t lds = rows_lds_bytes(a.M, a.steps_per_round, MT, WN, WK);
   if (lds > kRowsLdsMax) return static_cast<int>(hipErrorInvalidValue);
-  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, kEpiSiluMul, TOut, true>;
+  auto kernel = gemm_rows_kernel<MT, WN, WK, PD, XD, kEpiSiluMul, TOut, TILED, true>;
   static OnceADevice asked;
   if (lds > 64 * 1024)
     if (const int e = ask_lds(asked, kRowsLdsMax, {reinterpret_cast<const void*>(kernel)})) return e;
   const int col_groups = (a.N + WN * 16 - 1) / (WN * 16);
   kernel<<<dim3(col_groups, 1), WN * WK * 64, lds, s>>>(a);
   return launch_status();
+}
+
+template <int MT, int WN, int WK, int PD, int XD, typename TOut>
+int launch_rows_rounds(const RowsArgs& a, hipStream_t s) {
+  return a.tiled ? launch_rows_rounds_as<MT, WN, WK, PD, XD, TOut, true>(a, s) : launch_rows_rounds_as<MT, WN, WK, PD, XD, TOut, false>(a, s);
 }
 
 template <int MT, int WN, int WK, int PD, int XD, int EPI>

@@ -34,6 +34,7 @@
 // runs an elementwise kernel for this, crates/cuda-kernels/csrc/misc/split_qkv.cu:35-52).  Plain product: the reference's
 // crates/cuda-kernels/csrc/gemm/gemv.cu:45-,240-330 and cuBLAS for more rows.
 #include "common.h"
+#include "scaled_rows.h"
 
 namespace arle {
 
@@ -56,12 +57,11 @@ struct RowsArgs {
   int tiled;             // w holds operand tiles (see below) instead of rows
   int steps_per_round;   // ROUNDS: k steps of 32 whose X rows are in LDS at one time (the slice is walked in rounds)
   // SCALED: the rows of X still have to be divided by their root mean square, which the sums of this product are instead:
-  // sums [M][kSumsPitch], the first sums_count of a row add up to the squares of its `1 / sums_inv` columns
+  // sums [M][kRowSums], the first sums_count of a row add up to the squares of its `1 / sums_inv` columns
   const float* sums = nullptr;
   int sums_count = 0;
   float sums_inv = 0.f, eps = 0.f;
 };
-constexpr int kSumsPitch = 256, kScaledRows = 8;
 
 // Every byte of W is read by one wave of the launch.  As operand tiles, where a wave's load is whole lines, it is loaded past the
 // caches (ONCE), where it would only displace what is read again; as rows not: a step of a row is half a line, and the next step's load
@@ -120,12 +120,13 @@ __global__ __launch_bounds__(WN* WK * 64) void gemm_rows_kernel(const RowsArgs a
   for (int b = 0; b < MT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   static_assert(!SCALED || (MT == 1 && !ROUNDS && 2 * WN * WK >= kScaledRows), "two rows a wave");
+  static_assert(kRowSums == 4 * kWave, "four sums of a row a lane");
   __shared__ float row_scale[SCALED ? kScaledRows : 1];
   [[maybe_unused]] float4 squares[2];
   if constexpr (SCALED) {
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      squares[u] = *reinterpret_cast<const float4*>(a.sums + min(wave + u * WN * WK, M - 1) * kSumsPitch + 4 * lane);
+      squares[u] = *reinterpret_cast<const float4*>(a.sums + min(wave + u * WN * WK, M - 1) * kRowSums + 4 * lane);
   }
 
   // one round: the steps [s_begin, s_end) of the slice, staged and multiplied (without ROUNDS: the whole slice)
@@ -577,7 +578,7 @@ extern "C" int arle_gemm_rows_scaled(const void* x, long long ldx, const void* w
   if (epilogue == kEpiSiluMul && (N % 32 != 0 || (arle_gemm_rows_geometry(variant) & 15) != 1))
     return static_cast<int>(hipErrorInvalidValue);
   if (epilogue != kEpiNone && epilogue != kEpiSiluMul) return static_cast<int>(hipErrorInvalidValue);
-  if (sums != nullptr && (M > kScaledRows || sums_count < 1 || sums_count > kSumsPitch || reinterpret_cast<uintptr_t>(sums) % 16 != 0))
+  if (sums != nullptr && (M > kScaledRows || sums_count < 1 || sums_count > kRowSums || reinterpret_cast<uintptr_t>(sums) % 16 != 0))
     return static_cast<int>(hipErrorInvalidValue);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RowsArgs a{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(w), ldw, out, ldo, M, N, K,

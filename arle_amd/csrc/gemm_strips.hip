@@ -22,6 +22,7 @@
 //   * Eight waves with four pairs of steps ahead each; sixteen waves with two measured within 4 % either way.
 #include "common.h"
 #include "lane_sums.h"
+#include "scaled_rows.h"
 
 namespace arle {
 
@@ -29,8 +30,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kStripRows = 8, kStripWaves = 8, kStripAhead = 4;   // rows; waves; pairs of steps that a wave has in flight
-constexpr int kStripMost = 256;                                   // strips, and sums a row in memory
+constexpr int kStripWaves = 8, kStripAhead = 4;   // waves; pairs of steps that a wave has in flight
 
 struct StripArgs {
   const uint16_t* x;
@@ -40,7 +40,7 @@ struct StripArgs {
   const void* weight;    // of the norm, [N]
   int weight_f32;
   uint16_t* rows;        // [M, N]
-  float* sums;           // [M, kStripMost]
+  float* sums;           // [M, kRowSums]
   int M, N, K, c;
 };
 
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kStripWaves* kWave) void gemm_strips_kernel(const S
 #pragma unroll
   for (int r = 0; r < 4; ++r) parts[(wave * 16 + i) * kPitch + 4 * g + r] = i < 8 ? even[r] : odd[r];
   __syncthreads();
-  if (tid >= kStripRows * 16) return;
+  if (tid >= kScaledRows * 16) return;
   float v = 0.f;
 #pragma unroll
   for (int k = 0; k < kStripWaves; ++k)
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kStripWaves* kWave) void gemm_strips_kernel(const S
     a.residual[at] = v;
     a.rows[at] = f32_to_bf16_bits(v * __uint_as_float(w_raw));
   }
-  if ((tid & 15) == 0 && row < M) a.sums[row * kStripMost + blockIdx.x] = square;
+  if ((tid & 15) == 0 && row < M) a.sums[row * kRowSums + blockIdx.x] = square;
 }
 
 }  // namespace arle
@@ -137,7 +137,7 @@ using namespace arle;
 extern "C" int arle_gemm_strips(const void* x, long long ldx, const void* w, void* residual, const void* weight, int weight_f32,
                                 void* rows, void* sums, int M, int N, int K, int c, void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > kStripRows || K < 64 || K % 64 != 0 || ldx % 8 != 0 || c < 1 || c > 16 || (N + c - 1) / c > kStripMost ||
+  if (M > kScaledRows || K < 64 || K % 64 != 0 || ldx % 8 != 0 || c < 1 || c > 16 || (N + c - 1) / c > kRowSums ||
       static_cast<long long>(c) * K > (1 << 26) || reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)
     return static_cast<int>(hipErrorInvalidValue);
   const StripArgs a{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(w), static_cast<float*>(residual), weight,
@@ -146,4 +146,4 @@ extern "C" int arle_gemm_strips(const void* x, long long ldx, const void* w, voi
   return launch_status();
 }
 
-extern "C" int arle_gemm_strips_most() { return kStripMost; }
+extern "C" int arle_gemm_strips_most() { return kRowSums; }

@@ -57,7 +57,7 @@ SOURCES = {
     "host": "host/runtime.cpp",
 }
 HEADERS = ("common.h", "once_a_device.h", "attention_static.h", "attention_args.h", "attention_stream.h", "attention_portions.h",
-           "attention_portions_dma.h", "lds_loads.h", "attention_softcap_portions.h", "addend.h", "chunks.h", "lane_sums.h")
+           "attention_portions_dma.h", "lds_loads.h", "attention_softcap_portions.h", "addend.h", "chunks.h", "lane_sums.h", "scaled_rows.h")
 HOST_LIBS = ("host",)   # plain C++: page pool, block tables, step packing
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared"]
 

@@ -957,6 +957,15 @@ def gemm_strips(x, strips, residual, weight, eps: float) -> ScaledRows:
     return ScaledRows(rows, sums, -(-N // c), N, float(eps))
 
 
+def _check_scaled(scaled: ScaledRows, x) -> None:
+    _need(scaled.rows is x and x.dim() == 2 and x.shape[0] <= STRIP_ROWS and x.shape[1] == scaled.width,
+          f"a divisor a row is for 1..{STRIP_ROWS} rows, those that the sums are of")
+    sums, most = scaled.sums, _strips_most()
+    _need(sums.dtype == torch.float32 and sums.shape == (x.shape[0], most) and sums.is_contiguous() and sums.device == x.device
+          and sums.data_ptr() % 16 == 0 and 1 <= scaled.count <= most,
+          f"the sums of scaled rows are contiguous float32 [rows, {most}], of which 1 to {most} count")
+
+
 def takes_scaled(rows: int, n: int, k: int, *, tiled: bool, fused: bool) -> bool:
     """Whether the product of these sizes runs in a kernel that can divide its sums (gemm_rows up to eight rows)."""
     return 1 <= rows <= STRIP_ROWS and choose_product(rows, n, k, k, tiled=tiled, fused=fused, partials_ok=not fused).kernel == "rows"
@@ -974,9 +983,10 @@ def gemm_rows(x, w, out_dtype=torch.bfloat16, epilogue: int = EPI_NONE, *, varia
     tiles: pack_weight_tiles(w); the kernel then streams these instead of the rows of w (same sums, bit for bit).
     scaled: x are its rows; the sums are divided by their root mean squares (before the activation).
     """
+    if scaled is not None:
+        _check_scaled(scaled, x)
     _gpu(x, w)
     _rows(x, "x")
-    _need(scaled is None or (scaled.rows is x and x.shape[0] <= STRIP_ROWS), f"a divisor a row is for 1..{STRIP_ROWS} rows")
     _need(w.dim() == 2 and w.is_contiguous(), "w must be contiguous [N, K]")
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_rows takes bfloat16 operands")
     M, K = x.shape

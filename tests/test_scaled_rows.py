@@ -1,0 +1,33 @@
+"""What comes with rows that a product still has to divide is looked at before anything is launched: the kernel reads whole rows of sums."""
+import pytest
+import torch
+
+from arle_amd.kernels import ops
+
+M, K = 3, 64
+
+
+def _scaled(sums, count=4, rows=None, width=K):
+    return ops.ScaledRows(torch.zeros(M, K, dtype=torch.bfloat16) if rows is None else rows, sums, count, width, 1e-6)
+
+
+@pytest.mark.parametrize("sums,count", [
+    (torch.zeros(M, 255), 4), (torch.zeros(M, 512), 4), (torch.zeros(M - 1, 256), 4), (torch.zeros(M * 256), 4),
+    (torch.zeros(M, 256, dtype=torch.float64), 4), (torch.zeros(M, 256, dtype=torch.bfloat16), 4), (torch.zeros(256, M).T, 4),
+    (torch.zeros(M, 512)[:, :256], 4), (torch.zeros(M * 256 + 1)[1:].view(M, 256), 4), (torch.zeros(M, 256), 0), (torch.zeros(M, 256), 257)])
+def test_sums_that_the_kernel_could_not_read_are_refused(sums, count):
+    scaled = _scaled(sums, count)
+    with pytest.raises(ops.ShapeError, match="the sums of scaled rows"):
+        ops.gemm_rows(scaled.rows, torch.zeros(16, K, dtype=torch.bfloat16), scaled=scaled)
+
+
+def test_sums_of_other_rows_are_refused():
+    w = torch.zeros(16, K, dtype=torch.bfloat16)
+    scaled = _scaled(torch.zeros(M, 256))
+    with pytest.raises(ops.ShapeError, match="those that the sums are of"):
+        ops.gemm_rows(scaled.rows.clone(), w, scaled=scaled)
+    for wrong in (_scaled(torch.zeros(M, 256), width=K - 1), _scaled(torch.zeros(9, 256), rows=torch.zeros(9, K, dtype=torch.bfloat16))):
+        with pytest.raises(ops.ShapeError, match="those that the sums are of"):
+            ops.gemm_rows(wrong.rows, w, scaled=wrong)
+    with pytest.raises(ops.ShapeError, match="GPU only"):      # whole ones go on to what every call needs
+        ops.gemm_rows(scaled.rows, w, scaled=scaled)

@@ -6,7 +6,7 @@
 // What that replaces in a decode step: a product that leaves a stack of partial sums and a kernel that adds them into the residual
 // and norms its rows, 4.6 us for a few kilobytes (a launch and three trips to memory one behind the other), twice a layer.
 // No stack may be left for that, so K is not cut over workgroups; what is cut evenly over the compute units instead is N: one
-// workgroup a strip of N / 256 columns (10 of 2,560, 16 of 4,096), whose waves share K and add through LDS in the order of K.
+// workgroup a strip of N / 256 columns (10 of 2,560, 16 of 4,096), whose waves share K and add through LDS, in the order of K and in pairs.
 // The bound is the weights from memory.  MI355X, cold weights, us at 1 / 4 / 8 rows, product and norm before -> here:
 //   2,560 x 4,096   9.0 / 9.4 / 9.8 ->  6.0 /  6.1 /  7.0      2,560 x 9,728   13.8 / 14.2 / 14.6 ->  9.9 / 10.1 / 11.7
 //   4,096 x 4,096  11.6 / 12.1 / 12.6 -> 7.7 / 7.9 /  8.0      4,096 x 12,288  22.5 / 23.1 / 24.4 -> 17.5 / 17.7 / 18.0
@@ -20,6 +20,10 @@
 //     is multiplied with both steps' weights, and what met the other step's falls in lanes that are dropped
 //     (2,560 x 9,728, 1 row: 12.9 -> 11.6 us).
 //   * Eight waves with four pairs of steps ahead each; sixteen waves with two measured within 4 % either way.
+//   * Whole sums mean long chains of additions: a wave keeps four sums (even and odd steps of even and odd pairs) and the waves' are added
+//     two by two.  The residual is then off by less than with the stack of partial sums (error against 64 bits, stack / one chain a
+//     step parity and the waves in a row / here: 2,560 x 9,728 7.7e-8 / 8.9e-8 / 6.9e-8; 2,560 x 4,096 5.6e-8 / 5.7e-8 / 4.9e-8;
+//     4,096 x 12,288 16.7e-8 / 9.9e-8 / 7.5e-8), in the same time.
 #include "common.h"
 #include "lane_sums.h"
 #include "scaled_rows.h"
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(kStripWaves* kWave) void gemm_strips_kernel(const S
   auto load_w = [&](int at) { return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w + at))); };
   auto load_x = [&](int pair) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x + pair * 64)); };
   bf16x8 wr[PD][2], xr[PD];
-  f32x4 even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+  f32x4 even[2] = {}, odd[2] = {};
   const int last = max(n - 1, 0);
 #pragma unroll
   for (int u = 0; u < PD; ++u) {
@@ -78,8 +82,8 @@ __global__ __launch_bounds__(kStripWaves* kWave) void gemm_strips_kernel(const S
   const uint32_t w_raw = a.weight_f32 ? static_cast<const uint32_t*>(a.weight)[col_in]
                                       : static_cast<uint32_t>(static_cast<const uint16_t*>(a.weight)[col_in]) << 16;
   auto multiply = [&](int u) {
-    even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][0], xr[u], even, 0, 0, 0);
-    odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][1], xr[u], odd, 0, 0, 0);
+    even[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][0], xr[u], even[u & 1], 0, 0, 0);
+    odd[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][1], xr[u], odd[u & 1], 0, 0, 0);
   };
   int base = 0;
   for (; base + 2 * PD <= n; base += PD) {
@@ -112,14 +116,17 @@ __global__ __launch_bounds__(kStripWaves* kWave) void gemm_strips_kernel(const S
 
   // lane (i, g), register r: column 4 g + r of the strip; row i and the even steps in lanes i < 8, row i - 8 and the odd ones behind
 #pragma unroll
-  for (int r = 0; r < 4; ++r) parts[(wave * 16 + i) * kPitch + 4 * g + r] = i < 8 ? even[r] : odd[r];
+  for (int r = 0; r < 4; ++r) parts[(wave * 16 + i) * kPitch + 4 * g + r] = i < 8 ? even[0][r] + even[1][r] : odd[0][r] + odd[1][r];
   __syncthreads();
   if (tid >= kScaledRows * 16) return;
-  float v = 0.f;
+  float sum[kStripWaves];
 #pragma unroll
-  for (int k = 0; k < kStripWaves; ++k)
-    v += parts[(k * 16 + row) * kPitch + (tid & 15)] + parts[(k * 16 + 8 + row) * kPitch + (tid & 15)];
-  v += before;
+  for (int k = 0; k < kStripWaves; ++k) sum[k] = parts[(k * 16 + row) * kPitch + (tid & 15)] + parts[(k * 16 + 8 + row) * kPitch + (tid & 15)];
+#pragma unroll
+  for (int half = kStripWaves / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int k = 0; k < half; ++k) sum[k] = sum[2 * k] + sum[2 * k + 1];
+  const float v = sum[0] + before;
   const float square = row_sum16(mine ? v * v : 0.f);
   if (mine) {
     a.residual[at] = v;

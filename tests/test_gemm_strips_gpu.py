@@ -43,6 +43,24 @@ def test_strips_add_into_the_residual_and_leave_the_rows_and_their_squares(N, K,
     assert (got.shape, got.dtype, got.count, got.width) == ((M, N), torch.bfloat16, -(-N // -(-N // 256)), N)
 
 
+@pytest.mark.parametrize("N,K", [(2560, 9728), (2560, 4096), (1024, 3072), (2048, 6144), (4096, 4096)])
+def test_the_residual_is_no_further_off_than_with_a_stack_of_partial_sums(N, K):
+    """Its additions in 32 bits are ordered so that whole sums cost no accuracy against the product in parts that the norm adds."""
+    whole, parts = 0.0, 0.0
+    for seed in range(6):
+        w = _made(N, K, seed=20 + seed, scale=0.02).bfloat16().to(DEV)
+        linear = Linear(w, tiles=True, strips=True)
+        for M in (1, 8):
+            x = _made(M, K, seed=40 + seed).bfloat16().to(DEV)
+            residual = _made(M, N, seed=60 + seed, scale=2.0).to(DEV)
+            want = residual.double() + x.double() @ w.double().T
+            by_parts, weight = residual.clone(), torch.ones(N, device=DEV)
+            ops.add_rmsnorm(by_parts, linear(x, partials_ok=True), weight, EPS, torch.bfloat16)
+            linear.late(x).norm(residual, weight, EPS)
+            whole, parts = whole + _rel(residual, want), parts + _rel(by_parts, want)
+    assert whole <= parts, (whole / 12, parts / 12)
+
+
 @pytest.mark.parametrize("M", [1, 3, 8])
 @pytest.mark.parametrize("variant,splits,fused", [(0, 1, False), (0, 3, False), (1, 2, False), (2, 1, False), (3, 1, False), (4, 2, False),
                                                   (0, 1, True), (1, 1, True), (3, 1, True), (4, 1, True)])

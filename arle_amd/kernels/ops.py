@@ -919,6 +919,22 @@ def strip_columns(n: int, k: int) -> int:
     return columns if _STRIP_COLUMNS[0] <= columns <= _STRIP_COLUMNS[1] and k >= 64 and k % 64 == 0 and columns * k <= 1 << 26 else 0
 
 
+# Strips of a few columns are a few hundred bytes a k step, and with a long K the steps cost more than the bytes.  MI355X, cold
+# weights, us at 1 / 8 rows, product and norm / strips:
+#   4 columns: 1,024 x 6,144 6.9 / 6.5 and 7.3 / 7.2, 1,024 x 8,192 8.0 / 7.6 and 8.5 / 8.2, 1,024 x 10,240 8.6 / 9.3 and 9.2 / 10.1
+#   5 to 7: 1,280 x 8,192 8.9 / 8.4 and 9.7 / 9.4, 1,280 x 10,240 9.2 / 8.5 and 10.3 / 10.0, 1,280 x 12,288 10.3 / 11.1 and 11.5 / 12.7,
+#     1,536 x 12,288 11.2 / 10.6 and 12.6 / 13.4, 1,792 x 10,240 11.0 / 9.7 and 11.8 / 10.7
+#   8 and more, ahead for every K: 2,048 x 24,576 22.7 / 20.5 and 27.6 / 24.5, 2,560 x 32,768 36.4 / 30.2 and 47.3 / 34.6; the
+#     worst of it is 4,096 x 32,768, 47.5 / 50.0 at one row and 64.9 / 46.4 at eight
+_STRIP_LONGEST_K = {4: 8192, 5: 10240, 6: 10240, 7: 10240}
+
+
+def strips_preferred(n: int, k: int) -> bool:
+    """Whether gemm_strips is ahead of the product by itself with the norm's kernel behind it."""
+    columns = strip_columns(n, k)
+    return columns > 0 and k <= _STRIP_LONGEST_K.get(columns, k)
+
+
 @functools.lru_cache(maxsize=None)
 def _strips_most() -> int:
     return lib.function("arle_gemm_strips_most")()

@@ -54,12 +54,9 @@ class Linear:
         if packed is None and tiles and weight.dtype == torch.bfloat16 and weight.is_cuda and self.in_features % 8 == 0:
             self.tiles = ops.pack_weight_tiles(weight)
         self.strips = None
-        if strips and weight.dtype == torch.bfloat16 and weight.is_cuda:
-            columns = ops.strip_columns(self.out_features, self.in_features)
-            if columns == 16 and self.tiles is not None:
-                self.strips = self.tiles
-            elif columns:
-                self.strips = ops.pack_weight_strips(weight)
+        if strips and weight.dtype == torch.bfloat16 and weight.is_cuda and ops.strips_preferred(self.out_features, self.in_features):
+            same = self.tiles is not None and ops.strip_columns(self.out_features, self.in_features) == 16
+            self.strips = self.tiles if same else ops.pack_weight_strips(weight)
 
     def takes_scaled(self, rows: int) -> bool:
         """Whether this projection of `rows` rows can read ops.ScaledRows."""

@@ -1,4 +1,5 @@
-"""What comes with rows that a product still has to divide is looked at before anything is launched: the kernel reads whole rows of sums."""
+"""What comes with rows that a product still has to divide is looked at before anything is launched: the kernel reads whole rows of sums;
+and which matrices leave such rows."""
 import pytest
 import torch
 
@@ -31,3 +32,13 @@ def test_sums_of_other_rows_are_refused():
             ops.gemm_rows(wrong.rows, w, scaled=wrong)
     with pytest.raises(ops.ShapeError, match="GPU only"):      # whole ones go on to what every call needs
         ops.gemm_rows(scaled.rows, w, scaled=scaled)
+
+
+@pytest.mark.parametrize("n,k,columns,preferred", [
+    (1024, 64, 4, True), (1024, 8192, 4, True), (1024, 8256, 4, False), (1024, 10240, 4, False), (1025, 8256, 5, True), (1280, 10240, 5, True),
+    (1280, 10304, 5, False), (1792, 10240, 7, True), (1792, 12288, 7, False), (1793, 12288, 8, True), (2048, 24576, 8, True),
+    (2560, 9728, 10, True), (2560, 32768, 10, True), (4096, 12288, 16, True), (4096, 32768, 16, True), (4097, 4096, 0, False),
+    (768, 4096, 0, False), (769, 4096, 4, True), (2560, 96, 0, False), (2560, 32, 0, False)])
+def test_which_matrices_are_cut_into_strips(n, k, columns, preferred):
+    """Narrow strips only up to the K that was measured ahead of the product with the norm behind it."""
+    assert (ops.strip_columns(n, k), ops.strips_preferred(n, k)) == (columns, preferred)

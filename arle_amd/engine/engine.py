@@ -86,9 +86,10 @@ class Engine:
             were measured at the Qwen3-4B, 8B and 32B widths decide.  The table is the process's, not this engine's.
         weight_tiles: hold every bfloat16 projection weight a second time in the layout that the few-rows
             kernels stream fastest (decode steps about a tenth faster, twice the weight memory), and the projections
-            whose results a norm takes up a third time where they have 1,024 to 4,096 columns, other than 16 a compute
-            unit (up to a sixth less a step of eight rows or fewer).  Default: yes if the weights and the first of these
-            copies together stay under a third of the GPU's memory.
+            that a norm and another projection stand behind (o and down, the last down not) a third time where they have 769 to
+            4,080 columns (up to a sixth less a step of eight rows or fewer, 2.5 GB of Qwen3-4B, which a cache sized by the
+            memory left holds 17,000 tokens less for; at 4,081 to 4,096 columns the second copy serves).  Default: yes if the weights
+            and the first of these copies together stay under a third of the GPU's memory.
         """
         self.device = _device(device)
         self.dtype = parse_dtype(dtype)

@@ -135,6 +135,9 @@ class DecoderModel:
             else:
                 self.blocks.append(lookup("block", layer.block)(mixer, ffn, norms))
         self.schedule = list(spec.schedule)
+        for entry, following in zip(self.schedule, self.schedule[1:]):
+            if hasattr(self.blocks[entry.layer], "followed_by"):
+                self.blocks[entry.layer].followed_by(self.blocks[following.layer])
         self.final_norm = build_part("norm", spec.final_norm, fetch, rt)
         self.head = build_part("head", spec.head, fetch, rt)
         parts = [self.embedding, self.final_norm, self.head, *self._extra_parts]

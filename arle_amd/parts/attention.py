@@ -76,8 +76,8 @@ class PagedAttention(Part):
         # for a layer that reads another layer's cache: the q rows of the fused matrix, no copy (head_dim is a
         # multiple of 16, so the q rows are whole operand tiles too)
         self.q_only = Linear(self.qkv.weight[: self.q_width], packed=self.qkv.tiles)
-        self.leaves_late = bool(rt.weight_tiles)
-        self.o = Linear(tensors["o"], rt.weight_tiles, strips=self.leaves_late)
+        self.leaves_late = False
+        self.o = Linear(tensors["o"], rt.weight_tiles)
         # steps of single decoded tokens run norm, rotation and cache write inside the attention's kernel where it
         # has that form (ops.attn_decode_prep_supported); params["fold_preparation"] = False keeps the two kernels
         self.folds_preparation = bool(params.get("fold_preparation", True))
@@ -109,6 +109,16 @@ class PagedAttention(Part):
 
     def decode_class_sizes(self):
         return self.rt.is_f32, self.D, self.nkv, self.window, self.folds_preparation
+
+    @property
+    def reads_scaled(self) -> bool:
+        return self.qkv.weight.dtype == torch.bfloat16
+
+    def leave_late(self) -> None:
+        """A norm that can run the output projection stands behind it, and a reader of ops.ScaledRows behind that."""
+        if self.rt.weight_tiles:
+            self.o.lay_strips()
+            self.leaves_late = self.o.strips is not None
 
     def takes_scaled(self, rows: int) -> bool:
         return self.qkv.takes_scaled(rows) and self.q_only.takes_scaled(rows)

@@ -27,7 +27,21 @@ class PreNormBlock:
         self.norms = norms
         self.norm_mixer = norms["mixer_in"]
         self.norm_ffn = norms["ffn_in"] if feed_forward is not None else None
-        self._late = [{"late": True} if getattr(part, "leaves_late", False) else {} for part in (mixer, feed_forward)]
+        self._late = [{}, {}]
+        if self.norm_ffn is not None:
+            self._leave_late(0, mixer, self.norm_ffn, feed_forward)
+
+    def followed_by(self, block) -> None:
+        """`block` may come next in the schedule: its first norm is what the last projection here can be left to."""
+        if getattr(block, "takes_late", False):
+            last = 0 if self.norm_ffn is None else 1
+            self._leave_late(last, (self.mixer, self.feed_forward)[last], block.norm_mixer, block.mixer)
+
+    def _leave_late(self, which: int, part, norm, reader) -> None:
+        if hasattr(part, "leave_late") and hasattr(norm, "add_late") and getattr(reader, "reads_scaled", False):
+            part.leave_late()
+            if part.leaves_late:
+                self._late[which] = {"late": True}
 
     @staticmethod
     def _add_norm(norm, residual, delta, reader):

@@ -49,12 +49,22 @@ class SwiGLU(Part):
         else:
             fused = torch.cat([gate, up], dim=0)
         self.gate_up = Linear(fused.contiguous(), rt.weight_tiles)
-        self.leaves_late = bool(rt.weight_tiles) and not self.float32_out
-        self.down = Linear(tensors["down"], rt.weight_tiles, strips=self.leaves_late)
+        self.leaves_late = False
+        self.down = Linear(tensors["down"], rt.weight_tiles)
+
+    @property
+    def reads_scaled(self) -> bool:
+        return bool(self.block) and self.act == 0
+
+    def leave_late(self) -> None:
+        """A norm that can run the down projection stands behind it, and a reader of ops.ScaledRows behind that."""
+        if self.rt.weight_tiles and not self.float32_out:
+            self.down.lay_strips()
+            self.leaves_late = self.down.strips is not None
 
     def takes_scaled(self, rows: int) -> bool:
-        return bool(self.block) and self.act == 0 and ops.takes_scaled(rows, self.gate_up.out_features, self.gate_up.in_features,
-                                                                       tiled=self.gate_up.tiles is not None, fused=True)
+        return self.reads_scaled and ops.takes_scaled(rows, self.gate_up.out_features, self.gate_up.in_features,
+                                                      tiled=self.gate_up.tiles is not None, fused=True)
 
     def products(self):
         if self.gate_up.weight.dtype != torch.bfloat16:

@@ -20,7 +20,7 @@ few-rows kernels then read one contiguous kilobyte a wave and k step instead of 
 which is worth a fifth of their time on MI355X.  The library needs the rows, so both copies stay.
 
 A projection whose result goes into the residual can be left to the norm behind it (`late`): for up to eight rows product, add
-and norm are then one kernel (ops.gemm_strips), for which `strips=True` holds the weight in that kernel's layout too where the
+and norm are then one kernel (ops.gemm_strips), for which `lay_strips` holds the weight in that kernel's layout too where the
 tiles are not that layout already.
 """
 from __future__ import annotations
@@ -54,9 +54,15 @@ class Linear:
         if packed is None and tiles and weight.dtype == torch.bfloat16 and weight.is_cuda and self.in_features % 8 == 0:
             self.tiles = ops.pack_weight_tiles(weight)
         self.strips = None
-        if strips and weight.dtype == torch.bfloat16 and weight.is_cuda and ops.strips_preferred(self.out_features, self.in_features):
+        if strips:
+            self.lay_strips()
+
+    def lay_strips(self) -> None:
+        """From here on `late` may leave the projection to the norm behind it."""
+        if (self.strips is None and self.weight.dtype == torch.bfloat16 and self.weight.is_cuda
+                and ops.strips_preferred(self.out_features, self.in_features)):
             same = self.tiles is not None and ops.strip_columns(self.out_features, self.in_features) == 16
-            self.strips = self.tiles if same else ops.pack_weight_strips(weight)
+            self.strips = self.tiles if same else ops.pack_weight_strips(self.weight)
 
     def takes_scaled(self, rows: int) -> bool:
         """Whether this projection of `rows` rows can read ops.ScaledRows."""

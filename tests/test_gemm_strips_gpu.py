@@ -98,3 +98,39 @@ def test_what_takes_no_strips_runs_as_before():
         ops.gemm_strips(rows, linear.strips, torch.zeros(9, 2560, device=DEV), torch.ones(2560, device=DEV), EPS)
     with pytest.raises(ops.ShapeError):
         ops.gemm_rows(rows, w, scaled=ops.ScaledRows(rows, torch.zeros(9, 256, device=DEV), 4, 640, EPS))
+
+
+def test_a_model_lays_strips_for_what_a_norm_runs_and_for_nothing_else():
+    """o and down of every layer but the last down, which the final norm reads whole; steps of one to nine rows against the same model
+    without copies of its weights."""
+    from arle_amd.config import Qwen3Config
+    from arle_amd.config.registry import detect_architecture
+    from arle_amd.engine import Engine, StepEntry
+
+    raw = dict(num_hidden_layers=3, hidden_size=1024, num_attention_heads=8, num_key_value_heads=2, head_dim=64, intermediate_size=1088,
+               vocab_size=512, rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=True, max_position_embeddings=256)
+    shapes = {"model.embed_tokens.weight": (512, 1024), "model.norm.weight": (1024,)}
+    for i in range(3):
+        p = f"model.layers.{i}."
+        shapes |= {p + f"self_attn.{n}_proj.weight": s for n, s in (("q", (512, 1024)), ("k", (128, 1024)), ("v", (128, 1024)), ("o", (1024, 512)))}
+        shapes |= {p + f"mlp.{n}_proj.weight": s for n, s in (("gate", (1088, 1024)), ("up", (1088, 1024)), ("down", (1024, 1088)))}
+        shapes |= {p + f"self_attn.{n}_norm.weight": (64,) for n in "qk"}
+        shapes |= {p + f"{n}_layernorm.weight": (1024,) for n in ("input", "post_attention")}
+    weights = {n: (_made(*s, seed=100 + i, scale=0.04) if len(s) == 2 else 1.0 + _made(*s, seed=100 + i, scale=0.1)).bfloat16().to(DEV)
+               for i, (n, s) in enumerate(sorted(shapes.items()))}
+    recipe = detect_architecture({"architectures": ["Qwen3ForCausalLM"]}).recipe(Qwen3Config.from_dict(raw), ())
+    engines = [Engine(recipe, dict(weights), dtype="bfloat16", max_slots=9, max_tokens=9 * 32, weight_tiles=tiles) for tiles in (True, False)]
+    blocks = engines[0].model.blocks
+    assert [b.mixer.o.strips is not None for b in blocks] == [True] * 3
+    assert [b.feed_forward.down.strips is not None for b in blocks] == [True, True, False]
+    assert all(b.mixer.o.strips is None and b.feed_forward.down.strips is None for b in engines[1].model.blocks)
+    for rows in (1, 2, 7, 8, 9):
+        logits = []
+        for eng in engines:
+            for r in range(rows):
+                eng.add_request(r)
+            eng.step([StepEntry(r, [5 + r, 6, 7], [2]) for r in range(rows)])
+            logits.append(eng.step([StepEntry(r, [11 * r + 3], [0]) for r in range(rows)]).clone())
+            for r in range(rows):
+                eng.end_request(r)
+        assert _rel(*logits) < 2e-2, rows      # three layers of bfloat16 rounding

@@ -120,8 +120,8 @@ class PagedAttention(Part):
             self.o.lay_strips()
             self.leaves_late = self.o.strips is not None
 
-    def takes_scaled(self, rows: int) -> bool:
-        return self.qkv.takes_scaled(rows) and self.q_only.takes_scaled(rows)
+    def takes_scaled(self, rows: int, cache=None) -> bool:
+        return (self.q_only if cache is not None and not cache.writes else self.qkv).takes_scaled(rows)
 
     def forward(self, x, batch, cache, late: bool = False):
         """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);

@@ -44,10 +44,10 @@ class PreNormBlock:
                 self._late[which] = {"late": True}
 
     @staticmethod
-    def _add_norm(norm, residual, delta, reader):
+    def _add_norm(norm, residual, delta, reader, cache_view=None):
         if isinstance(delta, LateProduct):
             takes = getattr(reader, "takes_scaled", None)
-            if takes is not None and hasattr(norm, "add_late") and takes(residual.shape[0]):
+            if takes is not None and hasattr(norm, "add_late") and takes(residual.shape[0], cache_view):
                 return norm.add_late(residual, delta)
             delta = delta.now()
         return norm.add_norm(residual, delta)
@@ -58,7 +58,7 @@ class PreNormBlock:
             if self.norm_ffn is None:
                 return residual, m
             return residual, self.feed_forward.forward(self.norm_ffn.add_norm(residual, m))
-        a = self._add_norm(self.norm_mixer, residual, delta, self.mixer)
+        a = self._add_norm(self.norm_mixer, residual, delta, self.mixer, cache_view)
         m = self.mixer.forward(a, batch, cache_view, **self._late[0])
         if self.norm_ffn is None:
             return residual, m

@@ -62,7 +62,7 @@ class SwiGLU(Part):
             self.down.lay_strips()
             self.leaves_late = self.down.strips is not None
 
-    def takes_scaled(self, rows: int) -> bool:
+    def takes_scaled(self, rows: int, cache=None) -> bool:
         return self.reads_scaled and ops.takes_scaled(rows, self.gate_up.out_features, self.gate_up.in_features,
                                                       tiled=self.gate_up.tiles is not None, fused=True)
 

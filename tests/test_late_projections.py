@@ -1,8 +1,11 @@
 """Which projections a pre_norm model leaves to the norm behind them (and lays out a further time for that): those with a norm behind
 them that can run them, and a reader of its rows behind that."""
+import types
+
 import pytest
 import torch
 
+from arle_amd.parts.attention import PagedAttention
 from arle_amd.parts.block import PreNormBlock
 
 
@@ -87,3 +90,12 @@ def test_without_a_feed_forward_the_mixer_is_left_to_the_next_layer():
     assert _left(block) == (None, "late")
     alone = PreNormBlock(Late(), None, {"mixer_in": Norm()})
     assert _left(alone) == (None, "whole")
+
+
+def test_a_layer_is_asked_about_the_product_that_it_runs():
+    """A table entry of the q rows alone says nothing about a layer that writes its own cache."""
+    part = PagedAttention.__new__(PagedAttention)
+    part.qkv = types.SimpleNamespace(takes_scaled=lambda rows: True)
+    part.q_only = types.SimpleNamespace(takes_scaled=lambda rows: False)
+    assert part.takes_scaled(1) and part.takes_scaled(1, types.SimpleNamespace(writes=True))
+    assert not part.takes_scaled(1, types.SimpleNamespace(writes=False))

@@ -346,7 +346,8 @@ class Engine:
             for name, n, k, fused, consumer in (part.products() if hasattr(part, "products") else []):
                 found.setdefault((n, k, fused), (name, n, k, fused, consumer))
         products = [p + ((tune.HEAD_ROWS,) if p[0] == "head" else ()) for p in found.values()]
-        table, _ = tune.tune_products(products, device=self.device, tiled=self.rt.weight_tiles, say=say, rows=rows)
+        table, _ = tune.tune_products(products, device=self.device, tiled=self.rt.weight_tiles, say=say, rows=rows,
+                                      behind=self.model.products_behind_strips())
         ops.load_product_table(table)
         if path:
             tune.write_table(path, table)

@@ -35,6 +35,11 @@ def model_products(hidden: int, q_width: int, kv_width: int, intermediate: int, 
     return found
 
 
+def model_strips(hidden: int, q_width: int, kv_width: int, intermediate: int, vocab: int = 0) -> dict:
+    """`behind` of tune_products for such a decoder: gate|up reads what o leaves, q|k|v what down leaves."""
+    return {(2 * intermediate, hidden, True): (hidden, q_width), (q_width + 2 * kv_width, hidden, False): (hidden, intermediate)}
+
+
 def _seconds(fn, iters: int, repeats: int = 3) -> float:
     """Seconds a call of fn takes on the GPU: `iters` calls are captured into one graph and the graph is replayed, so
     that the time is the kernels' and not the host's (a product of a few rows is shorter than its launch)."""
@@ -60,12 +65,41 @@ MIN_GAIN = 0.08     # a choice other than the rules' has to win by this much of 
 MIN_GAIN_US = 1.5   # (products timed alone gain a microsecond here and there that whole steps do not show)
 
 
-def tune_products(products, device="cuda:0", tiled: bool = True, iters: int = 20, say=None, rows=None) -> tuple:
+def pick(timed: dict, ruled, apart: float = 0.0):
+    """The choice of `timed` (seconds) that replaces `ruled`, or `ruled`.  apart: what the projection in front takes longer where the
+    product is none of gemm_rows, which alone divides its sums, so that the norm is a kernel of its own."""
+    whole = {c: t + (0.0 if c.kernel == "rows" else apart) for c, t in timed.items()}
+    best = min(whole, key=whole.get)
+    # what does not win clearly does not replace the rule
+    return ruled if whole[ruled] - whole[best] < max(MIN_GAIN * whole[ruled], MIN_GAIN_US * 1e-6) else best
+
+
+def _apart(m: int, n: int, k: int, device, iters: int) -> float:
+    """Seconds that m rows of a projection [n, k] with its norm take longer as a product and the norm's kernel than in gemm_strips."""
+    copies = max(2, -(-COLD_BYTES // (n * k * 2)))
+    weights = [torch.randn(n, k, device=device).mul_(0.02).to(torch.bfloat16) for _ in range(copies)]
+    tiles, strips = [ops.pack_weight_tiles(w) for w in weights], [ops.pack_weight_strips(w) for w in weights]
+    x, residual = torch.randn(m, k, device=device).to(torch.bfloat16), torch.zeros((m, n), dtype=torch.float32, device=device)
+    norm_weight, turn = torch.ones(n, dtype=torch.bfloat16, device=device), {"i": 0}
+
+    def next_copy():
+        turn["i"] = (turn["i"] + 1) % copies
+        return turn["i"]
+
+    def two_kernels():
+        i = next_copy()
+        ops.add_rmsnorm(residual, ops.gemm_bf16(x, weights[i], partials_ok=True, tiles=tiles[i]), norm_weight, 1e-6, torch.bfloat16)
+
+    return max(0.0, _seconds(two_kernels, iters) - _seconds(lambda: ops.gemm_strips(x, strips[next_copy()], residual, norm_weight, 1e-6), iters))
+
+
+def tune_products(products, device="cuda:0", tiled: bool = True, iters: int = 20, say=None, rows=None, behind: dict | None = None) -> tuple:
     """(table, report): table as `ops.load_product_table` reads it; report: one record a (product, row count) with
     the microseconds of every candidate, of the rules' choice and of the best.  products: (name, N, K, with the
     activation, consumer[, row counts]); rows: the row counts for all of them (default: each product's own, else
-    ROWS)."""
-    table, report = {}, []
+    ROWS).  behind: {(N, K, with the activation) -> (N, K) of the projection in front that leaves its norm to this product}: for the
+    rows that ops.gemm_strips takes, another kernel than gemm_rows pays for the norm's kernel in front as well."""
+    table, report, lost = {}, [], {}
     only = rows
     for name, n, k, fused, consumer, *own_rows in products:
         rows = only if only is not None else (own_rows[0] if own_rows else ROWS)
@@ -93,9 +127,14 @@ def tune_products(products, device="cuda:0", tiled: bool = True, iters: int = 20
                     timed[choice] = _seconds(lambda: run(choice), iters)
                 except (ops.ShapeError, RuntimeError):
                     continue        # a kernel that refuses this shape is no candidate
-            best = min(timed, key=timed.get)
-            if timed[ruled] - timed[best] < max(MIN_GAIN * timed[ruled], MIN_GAIN_US * 1e-6):
-                best = ruled        # what does not win clearly does not replace the rule
+            front = (behind or {}).get((n, k, bool(fused)))
+            if front is None or not tiled or not 1 <= m <= ops.STRIP_ROWS or not ops.strips_preferred(*front):
+                apart = 0.0
+            else:
+                if (m, front) not in lost:
+                    lost[m, front] = _apart(m, *front, device, iters)
+                apart = lost[m, front]
+            best = pick(timed, ruled, apart)
             entries.append([m, best.kernel, list(best.variant), best.splits])
             record = {"product": name, "rows": m, "rule": [ruled.kernel, list(ruled.variant), ruled.splits],
                       "rule_us": round(timed[ruled] * 1e6, 1), "best": [best.kernel, list(best.variant), best.splits],

@@ -169,6 +169,15 @@ class DecoderModel:
                     found.add((name, answer))
         return tuple(sorted(found, key=repr))
 
+    def products_behind_strips(self) -> dict:
+        """{(N, K, fused) of a product -> (N, K) of the projection in front that leaves its norm to it in steps of a few rows}"""
+        found = {}
+        for block in self.blocks:
+            for part, reader in getattr(block, "late_pairs", ()):
+                for key in reader.scaled_products():
+                    found[key] = (part.late_product.out_features, part.late_product.in_features)
+        return found
+
     def cache_needs(self):
         """(need of every schedule entry that owns a cache, {reader entry -> owner entry})."""
         needs, readers = [], {}

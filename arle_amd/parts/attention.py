@@ -123,6 +123,14 @@ class PagedAttention(Part):
     def takes_scaled(self, rows: int, cache=None) -> bool:
         return (self.q_only if cache is not None and not cache.writes else self.qkv).takes_scaled(rows)
 
+    @property
+    def late_product(self):
+        return self.o
+
+    def scaled_products(self) -> list:
+        """(N, K, fused) of the products that read what the norm in front leaves."""
+        return [(self.qkv.out_features, self.qkv.in_features, False)]
+
     def forward(self, x, batch, cache, late: bool = False):
         """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);
         late: possibly the output projection for the norm behind it to run."""

@@ -28,6 +28,7 @@ class PreNormBlock:
         self.norm_mixer = norms["mixer_in"]
         self.norm_ffn = norms["ffn_in"] if feed_forward is not None else None
         self._late = [{}, {}]
+        self.late_pairs = []      # (a part whose last projection is left to a norm, the part behind that norm)
         if self.norm_ffn is not None:
             self._leave_late(0, mixer, self.norm_ffn, feed_forward)
 
@@ -42,6 +43,7 @@ class PreNormBlock:
             part.leave_late()
             if part.leaves_late:
                 self._late[which] = {"late": True}
+                self.late_pairs.append((part, reader))
 
     @staticmethod
     def _add_norm(norm, residual, delta, reader, cache_view=None):

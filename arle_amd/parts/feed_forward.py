@@ -62,6 +62,14 @@ class SwiGLU(Part):
             self.down.lay_strips()
             self.leaves_late = self.down.strips is not None
 
+    @property
+    def late_product(self):
+        return self.down
+
+    def scaled_products(self) -> list:
+        """(N, K, fused) of the products that read what the norm in front leaves."""
+        return [(self.gate_up.out_features, self.gate_up.in_features, True)]
+
     def takes_scaled(self, rows: int, cache=None) -> bool:
         return self.reads_scaled and ops.takes_scaled(rows, self.gate_up.out_features, self.gate_up.in_features,
                                                       tiled=self.gate_up.tiles is not None, fused=True)

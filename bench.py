@@ -587,7 +587,8 @@ def tune_products(args) -> int:
         print(f"[tune] {rec['product']:8s} rows {rec['rows']:5d}: rule {rec['rule'][0]:13s} {rec['rule_us']:8.1f} us   "
               f"best {rec['best'][0]:13s} {rec['best_us']:8.1f} us", file=sys.stderr, flush=True)
 
-    table, report = tune.tune_products(tune.model_products(*widths), tiled=not args.no_weight_tiles, say=say)
+    table, report = tune.tune_products(tune.model_products(*widths), tiled=not args.no_weight_tiles, say=say,
+                                       behind=tune.model_strips(*widths) if not args.no_weight_tiles else None)
     path = args.out or f"product_table_{args.tune_products.replace(',', '_')}.json"
     if os.path.exists(path):       # a file may hold the tables of several runs (with and without operand tiles)
         with open(path, encoding="utf-8") as fh:

@@ -134,3 +134,20 @@ def test_a_model_lays_strips_for_what_a_norm_runs_and_for_nothing_else():
             for r in range(rows):
                 eng.end_request(r)
         assert _rel(*logits) < 2e-2, rows      # three layers of bfloat16 rounding
+
+
+def test_a_tuned_reader_is_charged_with_the_norm_in_front():
+    """The tuner runs with a projection in front, and takes one in front of few rows into account only."""
+    from arle_amd.kernels import tune
+
+    n, k, front = 1536, 1024, (1024, 512)
+    seen = []
+    real = tune.pick
+    try:
+        tune.pick = lambda timed, ruled, apart=0.0: seen.append(apart) or real(timed, ruled, apart)
+        table, report = tune.tune_products([("qkv", n, k, False, "norm")], device=DEV, rows=(1, 9), iters=4, behind={(n, k, False): front})
+    finally:
+        tune.pick = real
+    assert list(table) == ["1536,1024,0,1"] and [r["rows"] for r in report] == [1, 9]
+    assert seen[0] >= 0.0 and seen[1] == 0.0
+    assert tune._apart(8, *front, DEV, 20) >= 0.0

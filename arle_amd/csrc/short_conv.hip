@@ -104,12 +104,13 @@ __global__ void causal_conv_vec_kernel(const T* __restrict__ u, long long u_stri
                                          conv_out(acc[3], add_input)});
 }
 
-// The same for steps of many rows: a lane takes kConvRows rows of its four channels, whose inputs it slides over (each is
+// The same for steps of many rows whose segments are known: a lane takes kConvRows rows of its four channels, whose inputs it slides over (each is
 // fetched once, not once a tap), where they and the rows they look back on belong to one request; else row by row.
 //
-// UPDATE: the first TAPS - 1 rows of a segment, the only ones that look back on its state, are left to a workgroup of the segment's own
+// The first TAPS - 1 rows of a segment, the only ones that look back on its state, are left to a workgroup of the segment's own
 // behind those of the rows, which reads that state, makes those rows and writes the state moved on: the update is no kernel of its own
-// (4.9 us for a few kilobytes, twelve times in a prompt of eight Gufasun layers).
+// (4.9 us for a few kilobytes, twelve times in a prompt of eight Gufasun layers).  No other workgroup reads a state: with that branch
+// beside it, for steps without segments, the kernel took 9.9 / 15.6 us where it takes 8.7 / 14.7 (2,048 x 2,560 / 6,144, bfloat16).
 //
 // What bounds it is a chain of trips to memory, not its bytes (21 MB at 2,048 x 2,560, 3.7 us): all inputs and slots of a lane's rows are asked
 // for at once, before the weights and before anything is looked at, and SILU is known here, or every lane takes the exponential and the
@@ -117,7 +118,7 @@ __global__ void causal_conv_vec_kernel(const T* __restrict__ u, long long u_stri
 // 9.1 / 15.3; inputs and slots first 8.7 / 14.6 (four rows a lane 8.3 / 14.8, sixteen 11.5 / 18.3).
 constexpr int kConvRows = 8;
 
-template <typename T, int TAPS, bool UPDATE, bool SILU>
+template <typename T, int TAPS, bool SILU>
 __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_stride, const T* __restrict__ bias,
                                         const T* __restrict__ out_bias, const T* __restrict__ w, T* state,
                                         const int* __restrict__ slot_of_token, T* __restrict__ out, long long out_stride,
@@ -157,36 +158,34 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
     constexpr int kFlags = SILU ? kConvSilu : 0;
     st4<T>(out + t * out_stride + c, float4{conv_out(acc[0], kFlags), conv_out(acc[1], kFlags), conv_out(acc[2], kFlags), conv_out(acc[3], kFlags)});
   };
-  if constexpr (UPDATE) {
-    if (static_cast<int>(blockIdx.x) >= row_blocks) {
-      const int seg = static_cast<int>(blockIdx.x) - row_blocks;
-      const int row0 = seg_row0[seg], len = seg_row0[seg + 1] - row0;
-      T* mine = state + static_cast<int64_t>(seg_slot[seg]) * (TAPS - 1) * channels + c;
-      float4 old[TAPS - 1], first[TAPS - 1], fresh[TAPS - 1];
-      auto input = [&](int at) {     // row `at` of the segment, at a place that exists
-        const float4 v = ld4<T>(u + static_cast<int64_t>(min(max(row0 + at, 0), tokens - 1)) * u_stride + c);
-        return float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
-      };
+  if (static_cast<int>(blockIdx.x) >= row_blocks) {
+    const int seg = static_cast<int>(blockIdx.x) - row_blocks;
+    const int row0 = seg_row0[seg], len = seg_row0[seg + 1] - row0;
+    T* mine = state + static_cast<int64_t>(seg_slot[seg]) * (TAPS - 1) * channels + c;
+    float4 old[TAPS - 1], first[TAPS - 1], fresh[TAPS - 1];
+    auto input = [&](int at) {     // row `at` of the segment, at a place that exists
+      const float4 v = ld4<T>(u + static_cast<int64_t>(min(max(row0 + at, 0), tokens - 1)) * u_stride + c);
+      return float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
+    };
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) old[j] = ld4<T>(mine + static_cast<int64_t>(j) * channels), first[j] = input(j), fresh[j] = input(len - (TAPS - 1) + j);
+    for (int j = 0; j < TAPS - 1; ++j) old[j] = ld4<T>(mine + static_cast<int64_t>(j) * channels), first[j] = input(j), fresh[j] = input(len - (TAPS - 1) + j);
 #pragma unroll
-      for (int r = 0; r < TAPS - 1; ++r) {
-        float4 in[TAPS];
+    for (int r = 0; r < TAPS - 1; ++r) {
+      float4 in[TAPS];
 #pragma unroll
-        for (int back = 0; back < TAPS; ++back) in[back] = back <= r ? first[r - back] : old[TAPS - 1 - (back - r)];
-        if (r < len) row_out(row0 + r, in);
-      }
-#pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) {
-        const int at = len - (TAPS - 1) + j;      // place among the segment's rows; negative: still in the old state
-        float4 v = fresh[j];
-#pragma unroll
-        for (int back = 1; back < TAPS; ++back)
-          if (at == -back) v = old[TAPS - 1 - back];
-        st4<T>(mine + static_cast<int64_t>(j) * channels, v);
-      }
-      return;
+      for (int back = 0; back < TAPS; ++back) in[back] = back <= r ? first[r - back] : old[TAPS - 1 - (back - r)];
+      if (r < len) row_out(row0 + r, in);
     }
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int at = len - (TAPS - 1) + j;      // place among the segment's rows; negative: still in the old state
+      float4 v = fresh[j];
+#pragma unroll
+      for (int back = 1; back < TAPS; ++back)
+        if (at == -back) v = old[TAPS - 1 - back];
+      st4<T>(mine + static_cast<int64_t>(j) * channels, v);
+    }
+    return;
   }
   bool one = first_back >= 0;
 #pragma unroll
@@ -210,17 +209,12 @@ __global__ void causal_conv_rows_kernel(const T* __restrict__ u, long long u_str
     const int t = t0 + r, mine_slot = slot_of_token[t];
     int mine = 0;
     while (mine < TAPS - 1 && t - mine - 1 >= 0 && slot_of_token[t - mine - 1] == mine_slot) ++mine;
-    if (UPDATE && mine < TAPS - 1) continue;      // the segment's workgroup makes it
+    if (mine < TAPS - 1) continue;      // the segment's workgroup makes it
     float4 in[TAPS];
 #pragma unroll
     for (int back = 0; back < TAPS; ++back) {
-      if (back <= mine) {
-        const float4 v = ld4<T>(u + (t - back) * u_stride + c);
-        in[back] = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
-      } else {
-        const int64_t row = static_cast<int64_t>(mine_slot) * (TAPS - 1) + (TAPS - 1 - (back - mine));
-        in[back] = ld4<T>(state + row * channels + c);
-      }
+      const float4 v = ld4<T>(u + (t - back) * u_stride + c);
+      in[back] = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
     }
     row_out(t, in);
   }
@@ -416,22 +410,18 @@ extern "C" int arle_causal_conv(const void* u, long long u_stride, int u_dtype, 
   if (w && taps >= 2 && taps <= 4 && channels % 4 == 0 && u_stride % 4 == 0 && out_stride % 4 == 0 && at16(u) && at16(out) &&
       at16(state) && at16(w) && at16(bias) && at16(out_bias) && u_dtype == out_dtype && w_dtype == out_dtype && state_dtype == out_dtype &&
       (!bias || bias_dtype == out_dtype) && (!out_bias || ob_dtype == out_dtype)) {
-    if (tokens >= kConvManyRows) {
+    if (tokens >= kConvManyRows && moves) {
       const int row_blocks = (tokens + kConvRows - 1) / kConvRows;
-      const dim3 rgrid(static_cast<unsigned>(row_blocks + (moves ? segments : 0)), (channels / 4 + 255) / 256);
-#define ARLE_CONV_ROWS_AS(T, TAPS, UPDATE, SILU)                                                                    \
-  causal_conv_rows_kernel<T, TAPS, UPDATE, SILU><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
-                                                                       static_cast<const T*>(out_bias), static_cast<const T*>(w), \
-                                                                       static_cast<T*>(state), slot_of_token,       \
-                                                                       static_cast<T*>(out), out_stride, tokens, channels, add_input, \
-                                                                       seg_row0, seg_slot, row_blocks)
+      const dim3 rgrid(static_cast<unsigned>(row_blocks + segments), (channels / 4 + 255) / 256);
+#define ARLE_CONV_ROWS_AS(T, TAPS, SILU)                                                                            \
+  causal_conv_rows_kernel<T, TAPS, SILU><<<rgrid, 256, 0, s>>>(static_cast<const T*>(u), u_stride, static_cast<const T*>(bias), \
+                                                               static_cast<const T*>(out_bias), static_cast<const T*>(w), \
+                                                               static_cast<T*>(state), slot_of_token,               \
+                                                               static_cast<T*>(out), out_stride, tokens, channels, add_input, \
+                                                               seg_row0, seg_slot, row_blocks)
 #define ARLE_CONV_ROWS(T, TAPS)                                                                                     \
   do {                                                                                                              \
-    if (add_input & kConvSilu) {                                                                                    \
-      if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true, true); else ARLE_CONV_ROWS_AS(T, TAPS, false, true);              \
-    } else {                                                                                                        \
-      if (moves) ARLE_CONV_ROWS_AS(T, TAPS, true, false); else ARLE_CONV_ROWS_AS(T, TAPS, false, false);            \
-    }                                                                                                               \
+    if (add_input & kConvSilu) ARLE_CONV_ROWS_AS(T, TAPS, true); else ARLE_CONV_ROWS_AS(T, TAPS, false);            \
   } while (0)
       if (out_dtype == kF32) {
         if (taps == 2) ARLE_CONV_ROWS(float, 2); else if (taps == 3) ARLE_CONV_ROWS(float, 3); else ARLE_CONV_ROWS(float, 4);

@@ -454,6 +454,25 @@ static int compute_units() {
   return cus;
 }
 
+namespace arle {
+template <bool INWG, int D, bool WHOLE_IN>
+void launch_decode_prep_as(const AttnArgs& a, dim3 grid, int threads, hipStream_t s) {
+  if (a.P <= once_slots(INWG))
+    attn_mfma_kernel<1, D, true, true, INWG, WHOLE_IN, true><<<grid, threads, 0, s>>>(a);
+  else
+    attn_mfma_kernel<1, D, true, true, INWG, WHOLE_IN, false><<<grid, threads, 0, s>>>(a);
+}
+
+// head_dim 64 or 128
+template <bool INWG>
+void launch_decode_prep(const AttnArgs& a, bool whole_in, dim3 grid, int threads, hipStream_t s) {
+  if (a.D == 128)
+    whole_in ? launch_decode_prep_as<INWG, 128, true>(a, grid, threads, s) : launch_decode_prep_as<INWG, 128, false>(a, grid, threads, s);
+  else
+    whole_in ? launch_decode_prep_as<INWG, 64, true>(a, grid, threads, s) : launch_decode_prep_as<INWG, 64, false>(a, grid, threads, s);
+}
+}  // namespace arle
+
 // A step of single decoded tokens with the preparation of q, k and v folded into the attention: segment s is the
 // one token row s.  parts: the fused q|k|v projection of the step as n_parts float32 partial products
 // [token rows][(nq + 2 nkv) D] (part_stride elements apart, rows row_stride apart; both multiples of 8, parts
@@ -510,28 +529,14 @@ extern "C" int arle_attn_decode_prep(const void* parts, int parts_bf16, int n_pa
   if (!spread && splits > 1 && splits <= kInWgWavesMax && g_decode_inwg != 0 &&
       (g_decode_inwg > 0 || static_cast<long long>(segments) * nkv >= compute_units())) {
     const dim3 grid(1, nkv, static_cast<unsigned>(segments));
-    if (D == 128 && parts_bf16)
-      attn_mfma_kernel<1, 128, true, true, true, true><<<grid, splits * kWave, 0, s>>>(a);
-    else if (D == 128)
-      attn_mfma_kernel<1, 128, true, true, true, false><<<grid, splits * kWave, 0, s>>>(a);
-    else if (parts_bf16)
-      attn_mfma_kernel<1, 64, true, true, true, true><<<grid, splits * kWave, 0, s>>>(a);
-    else
-      attn_mfma_kernel<1, 64, true, true, true, false><<<grid, splits * kWave, 0, s>>>(a);
+    launch_decode_prep<true>(a, parts_bf16 != 0, grid, splits * kWave, s);
     return launch_status();
   }
   a.segments = segments;
   a.ws_plan = splits > 1 ? ws_plan : nullptr;
   a.plan_made = spread && plan_made;
   const dim3 grid(1, nkv, static_cast<unsigned>(z));
-  if (D == 128 && parts_bf16)
-    attn_mfma_kernel<1, 128, true, true, false, true><<<grid, kWave, 0, s>>>(a);
-  else if (D == 128)
-    attn_mfma_kernel<1, 128, true, true, false, false><<<grid, kWave, 0, s>>>(a);
-  else if (parts_bf16)
-    attn_mfma_kernel<1, 64, true, true, false, true><<<grid, kWave, 0, s>>>(a);
-  else
-    attn_mfma_kernel<1, 64, true, true, false, false><<<grid, kWave, 0, s>>>(a);
+  launch_decode_prep<false>(a, parts_bf16 != 0, grid, kWave, s);
   const int rc = launch_status();
   if (rc != 0 || splits == 1) return rc;
   attn_merge_kernel<<<dim3(segments * a.ws_rows, nq), kMergeWaves * kWave, 0, s>>>(

@@ -71,8 +71,9 @@ __global__ __launch_bounds__(GROUPS* kDmWaves* kWave, GROUPS == 1 ? 2 : 1) void 
     if (wg < first || wg >= first + wgs) {
       if (wg >= first) wg -= wgs;
       const int at = static_cast<int>(wg / nkv);
-      attn_mfma_body<1, kDmD, true, false, true, false>(a, at / beside_parts, static_cast<int>(wg % nkv), 0, kDmWaves, beside_parts,
-                                                        at % beside_parts, reinterpret_cast<float*>(lds_all));
+      static_assert(2 * once_slots(true) == kDmKeys, "without WHOLE, pages have up to that many slots");
+      attn_mfma_body<1, kDmD, true, false, true, false, !WHOLE>(a, at / beside_parts, static_cast<int>(wg % nkv), 0, kDmWaves, beside_parts,
+                                                                at % beside_parts, reinterpret_cast<float*>(lds_all));
       return;
     }
     wg -= first;

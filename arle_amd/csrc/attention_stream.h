@@ -25,12 +25,15 @@ namespace arle {
 // (many requests, few splits); with fewer, one-wave workgroups spread the same waves over more compute units.
 constexpr int kInWgWavesMax = 4;
 //
+// ONCE (pages of up to once_slots slots): the values are loaded past the caches, see load_v.
+constexpr int once_slots(bool inwg) { return inwg ? 32 : 16; }
+//
 // A workgroup's place in the launch is handed in: its segment, kv head and first row, and with INWG the number of its
 // waves, in how many parts the segment's keys are cut over workgroups (`parts`) and which of them this one takes;
 // without INWG, parts is the number of splits.  `handed`: LDS for what the waves of a workgroup hand to wave 0.
 constexpr int handed_pitch(int head_dim) { return 4 * (head_dim / 16) + 4; }   // floats a lane: its sums, m and l, and padding to 16 bytes
 constexpr int handed_floats(int head_dim) { return (kInWgWavesMax - 1) * kWave * handed_pitch(head_dim); }
-template <int NT, int DMAX, bool EXACT, bool PREP, bool INWG, bool WHOLE_IN>
+template <int NT, int DMAX, bool EXACT, bool PREP, bool INWG, bool WHOLE_IN, bool ONCE>
 __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const int kvh, const int row_begin, const int waves,
                                                const int parts, const int part, float* const handed) {
   static_assert(!PREP || (NT == 1 && EXACT), "the folded preparation is written for one row tile and a head_dim known here");
@@ -163,9 +166,13 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
     }
   };
 
-  // values of a block: for each 16-key tile the 4 keys 4g..4g+3, at d = 16*dt + li.  Nobody else reads them: past the caches, 64
-  // requests of the Qwen3-4B shape at 2,048 tokens 5,900 -> 5,743 us a step, 19 ragged ones 2,931 -> 2,908.  Keys as well
-  // gained nothing more there and cost 8 requests 1 to 2 %: a key's line is read by two loads, a half each.
+  // values of a block: for each 16-key tile the 4 keys 4g..4g+3, at d = 16*dt + li.  Nobody else reads them, and in pages of up to
+  // 16 slots a load takes whole lines: past the caches (ONCE).  In larger pages a line holds keys of the next tile too (32 slots) or of the
+  // next block (64), and has to stay.  Decode steps of the Qwen3-4B shape at 2,048 tokens, us, kept / past the caches: pages of 16
+  // slots, 64 requests (INWG) 5,930 / 5,750, 8 requests 2,570 / 2,540, 19 ragged ones 2,869 / 2,843; pages of 32 5,970 / 5,940, 2,640 / 2,660,
+  // 2,920 / 2,970; pages of 64 6,580 / 7,850, 2,790 / 2,910, 3,050 / 3,230.  Decoded rows beside portions likewise: four steps of Qwen3-8B
+  // with 32 requests, pages of 16 43,760 / 43,240, of 64 44,590 / 46,140.  Keys as well gained nothing more and cost 8 requests 1 to
+  // 2 %: a key's line is read by two loads, a half each.
   auto load_v = [&](int blk, u32x4 (&vreg)[DTL]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -176,7 +183,10 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt) {
         const int drow = EXACT ? 16 * dt + li : min(16 * dt + li, D - 1);  // a tile past head_dim reads its last row
-        const u32x2 four = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(vp + static_cast<int64_t>(drow) * P));
+        const u32x2* at = reinterpret_cast<const u32x2*>(vp + static_cast<int64_t>(drow) * P);
+        u32x2 four;
+        if constexpr (ONCE) four = __builtin_nontemporal_load(at);
+        else four = *at;
         vreg[dt][2 * t] = four[0];
         vreg[dt][2 * t + 1] = four[1];
       }
@@ -624,14 +634,14 @@ __device__ __forceinline__ void attn_mfma_body(const AttnArgs& a, int seg, const
   }
 }
 
-template <int NT, int DMAX, bool EXACT, bool PREP = false, bool INWG = false, bool WHOLE_IN = false>
+template <int NT, int DMAX, bool EXACT, bool PREP = false, bool INWG = false, bool WHOLE_IN = false, bool ONCE = false>
 __global__ __launch_bounds__(INWG ? kInWgWavesMax * kWave : kWave) void attn_mfma_kernel(const AttnArgs a) {
   const int z = static_cast<int>(blockIdx.z), row_begin = static_cast<int>(blockIdx.x) * (16 * NT);
   if constexpr (INWG) {
     __shared__ __align__(16) float handed[handed_floats(DMAX)];
-    attn_mfma_body<NT, DMAX, EXACT, PREP, true, WHOLE_IN>(a, z, blockIdx.y, row_begin, a.splits, 1, 0, handed);
+    attn_mfma_body<NT, DMAX, EXACT, PREP, true, WHOLE_IN, ONCE>(a, z, blockIdx.y, row_begin, a.splits, 1, 0, handed);
   } else {
-    attn_mfma_body<NT, DMAX, EXACT, PREP, false, WHOLE_IN>(a, z / a.splits, blockIdx.y, row_begin, 1, a.splits, z % a.splits, nullptr);
+    attn_mfma_body<NT, DMAX, EXACT, PREP, false, WHOLE_IN, ONCE>(a, z / a.splits, blockIdx.y, row_begin, 1, a.splits, z % a.splits, nullptr);
   }
 }
 

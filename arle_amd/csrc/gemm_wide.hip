@@ -16,8 +16,11 @@
 //     with two stages and lines touched ahead 32.7 (128 x 96, 97 rows: 30.6 / 34.9; 128 x 160, 160 rows 33.4 / 37.7); a sixth stage and
 //     more change nothing.  From operand tiles, whose kilobytes lie whole in memory where rows are 128 bytes each 5 KB apart,
 //     64 rows take 23.7 us for 26.8, 128 rows 29.5 for 32.7, 256 rows 35.0 for 38.7; from 544 rows on the two are level.
-//   * Weights that one row block reads (ONCE) are loaded past the caches: whole steps of the Qwen3-4B shape, 19 requests 2,908 ->
-//     2,856 us, 64 requests 5,743 -> 5,661, a prompt of 97 tokens 3,387 -> 3,194.
+//   * Weights that one row block reads (ONCE) are loaded past the caches, from tiles and from rows (a load takes whole lines of either).
+//     Cold, us, kept / past: 24,576 x 4,096 with the activation, 33 rows, 40.1 / 36.6 from tiles and 47.2 / 42.7 from rows; 4,096 x 12,288 in
+//     three parts 24.3 / 22.6 and 25.9 / 24.4; 128 rows level to 4 % ahead.  Whole steps of the Qwen3-4B shape, means of four to eight
+//     engines of each (which differ by 2 % among themselves): prompts of 33 and 64 tokens 2,686 / 2,587 and 2,998 / 2,891, 64 requests
+//     5,760 / 5,698; prompts of 97 and 120 tokens (3,357 / 3,319, 3,524 / 3,506) and 19 requests (2,906 / 2,895) within the spread.
 //   * Latency of what comes from memory in the large shapes: with two stages a fetch has one stage's time (1.2 to 1.8 us), which
 //     a miss of the L2 under load does not keep to.  There every wave touches, four stages ahead, a few of the 128-byte lines that its
 //     XCD's workgroups will fetch (a dword a line, into a corner of LDS that nobody reads): 2,048 rows 223 -> 186 us, 8,192

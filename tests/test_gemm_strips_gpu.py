@@ -37,7 +37,7 @@ def test_strips_add_into_the_residual_and_leave_the_rows_and_their_squares(N, K,
     assert _rel(residual, want) < 1e-5
     squares = got.sums[:, :got.count].double().sum(1)
     assert _rel(squares, (want * want).sum(1)) < 1e-5
-    # one rounding to bfloat16: 2^-9 of a value at most
+    # one rounding to bfloat16: half a unit of eight significant bits, 2^-8 of a value at most
     rows = want * weight.double()
     assert float(((got.rows.double() - rows).abs() - rows.abs() * 2.0 ** -8).max()) <= 1e-4
     assert (got.shape, got.dtype, got.count, got.width) == ((M, N), torch.bfloat16, -(-N // -(-N // 256)), N)

@@ -1732,7 +1732,8 @@ def run_product(choice: ProductChoice, x, w, tiles, out_dtype, partials_ok: bool
     """Launch what `choice` names.  Plain products come back as [M, N] in out_dtype, or, where the caller said
     partials_ok, possibly as a float32 stack [S, M, N]; fused ones as the activation [M, N/2]."""
     kernel = choice.kernel
-    _need(scaled is None or kernel == "rows", "only gemm_rows divides its sums (see takes_scaled)")
+    if scaled is not None:
+        _need(kernel == "rows", "only gemm_rows divides its sums (see takes_scaled)")
     if fused:
         if kernel == "rows":
             return gemm_rows(x, w, x.dtype, EPI_SILU_MUL, variant=choice.variant[0] if choice.variant else None,
@@ -1782,8 +1783,8 @@ def gate_up_act(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor | None = N
     rows, n, k = x.shape[0], w.shape[0], x.shape[1]
     if rows == 0:
         return torch.empty((0, n // 2), dtype=x.dtype, device=x.device)
-    _need(scaled is None or act == 0, "rows that are still to be divided need an activation that the product applies")
     if act != 0:     # the products that apply the activation themselves know silu only
+        _need(scaled is None, "rows that are still to be divided need an activation that the product applies")
         return act_mul_interleaved(gemm_bf16(x, w, x.dtype, tiles=tiles), act, 16)
     choice = choose_product(rows, n, k, x.stride(0), tiled=tiles is not None, fused=True, partials_ok=False,
                             aligned=x.data_ptr() % 16 == 0, w_aligned=w.is_contiguous() and w.data_ptr() % 16 == 0)

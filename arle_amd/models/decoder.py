@@ -204,7 +204,7 @@ class DecoderModel:
             debug_dump(residual, None, "embedding")
         for i, entry in enumerate(self.schedule):
             block = self.blocks[entry.layer]
-            if isinstance(delta, LateProduct) and not getattr(block, "takes_late", False):
+            if type(delta) is LateProduct and not getattr(block, "takes_late", False):
                 delta = delta.now()
             residual, delta = block.forward(residual, delta, batch, cache.view(i))
             if dump:

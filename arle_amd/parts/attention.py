@@ -134,11 +134,6 @@ class PagedAttention(Part):
     def forward(self, x, batch, cache, late: bool = False):
         """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);
         late: possibly the output projection for the norm behind it to run."""
-        out = self._mixed(x, batch, cache)
-        return self.o.late(out) if late and self.leaves_late else self.o(out, partials_ok=True)
-
-    def _mixed(self, x, batch, cache):
-        """x -> the heads' sums of values [T, Q], before the output projection."""
         Q, KV = self.q_width, self.kv_width
         self.position.ensure_positions(batch.max_position + 1)
         cos, sin, rot = self.position.fused_rotary()
@@ -163,7 +158,7 @@ class PagedAttention(Part):
                                  scale=self.scale, eps=self.eps, q_weight=self.q_norm, k_weight=self.k_norm, cos=cos,
                                  sin=sin, rotary_dim=rot, window=self.window or 0, splits=getattr(batch, "kv_splits", None),
                                  total_kv_len=getattr(batch, "total_context", 0) or None, carry=getattr(batch, "carry", None))
-            return out
+            return self.o.late(out) if late and self.leaves_late else self.o(out, partials_ok=True)
         if projected.dim() == 3:
             q = torch.empty((x.shape[0], Q), dtype=x.dtype, device=x.device)
             ops.qk_prep(q, None, None, q_weight=self.q_norm, k_weight=self.k_norm, cos=cos, sin=sin,
@@ -187,7 +182,7 @@ class PagedAttention(Part):
         out = torch.empty((x.shape[0], Q), dtype=q.dtype, device=q.device)
         paged_attention(q, out, cache, batch, num_q_heads=self.nq, num_kv_heads=self.nkv,
                         head_dim=self.D, scale=self.scale, window=self.window or 0)
-        return out
+        return self.o.late(out) if late and self.leaves_late else self.o(out, partials_ok=True)
 
 
 def paged_attention(q, out, cache, batch, *, num_q_heads, num_kv_heads, head_dim, scale, window):

@@ -83,7 +83,7 @@ class SwiGLU(Part):
     def forward(self, x, late: bool = False):
         """x [T, H] (or ops.ScaledRows, see takes_scaled) -> [T, H], or a float32 stack [S, T, H] to be added in order (see Linear);
         late: possibly the down projection for the norm behind it to run."""
-        if isinstance(x, ops.ScaledRows):
+        if type(x) is ops.ScaledRows:
             act = ops.gate_up_act(x.rows, self.gate_up.weight, self.gate_up.tiles, scaled=x)
         elif self.block:
             act = ops.gate_up_act(x, self.gate_up.weight, self.gate_up.tiles, self.act)   # one product with the activation, or two kernels
